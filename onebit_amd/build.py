@@ -3,8 +3,10 @@
 A library is one or more translation units (one hipcc process each, run in parallel; an object is rebuilt only when its
 source or one of the headers it includes -- transitively -- is newer), linked into one shared library:
   libonebit_hip.so      the 1-bit LLaMA path
-    onebit_hip.hip        layer, decode steps, prefill glue, train-mode layer
+    onebit_hip.hip        layer, decode steps, prefill glue
     onebit_mixed.hip      ragged attention / rope kernels, the split-KV decode attention, the mixed prefill + decode step
+    onebit_f32.hip        the float32 layer
+    onebit_train.hip      train-mode layer
   libonebit_hybrid.so   the hybrid decoders (dense weights, sigmoid attention, state-space layers)
     onebit_hybrid.hip
 A model family needs its own library only (``ensure``).
@@ -21,7 +23,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(CSRC, "build")
 LIB = os.path.join(CSRC, "libonebit_hip.so")
-SOURCES = ["onebit_hip.hip", "onebit_mixed.hip"]
+SOURCES = ["onebit_hip.hip", "onebit_mixed.hip", "onebit_f32.hip", "onebit_train.hip"]
 LIB_HYBRID = os.path.join(CSRC, "libonebit_hybrid.so")
 SOURCES_HYBRID = ["onebit_hybrid.hip"]
 # (packed FP32 instructions stay off: some of their forms have given wrong results on this hardware; hipcc makes them from ordinary

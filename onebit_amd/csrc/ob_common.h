@@ -12,6 +12,7 @@ typedef float ob_float2 __attribute__((ext_vector_type(2)));
 typedef uint32_t ob_u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t ob_u32x2 __attribute__((ext_vector_type(2)));
 typedef int32_t ob_i32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 ob_bf8 __attribute__((ext_vector_type(8)));
 
 #define OB_WAVE 64
 
@@ -75,6 +76,14 @@ __device__ __forceinline__ float ob_block_sum(float v, float *red)
     if (nw == 4) return (red[0] + red[1]) + (red[2] + red[3]);
     for (int i = 0; i < nw; ++i) s += red[i];
     return s;
+}
+
+// 1 KB from base + lane_off (16 bytes a lane) straight into LDS at lds_addr.  In flight until a vmcnt wait; M0 is as it was.
+__device__ __forceinline__ void ob_dma_1k(const char *base, uint32_t lane_off, uint32_t lds_addr)
+{
+    uint32_t keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3\n\ts_mov_b32 m0, %0"
+                 : "=&s"(keep) : "s"(lds_addr), "v"(lane_off), "s"(base) : "memory");
 }
 
 __device__ __forceinline__ float ob_round_h(float v) { return (float)(_Float16)v; }

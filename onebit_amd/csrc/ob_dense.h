@@ -11,7 +11,6 @@
 #pragma once
 #include "ob_common.h"
 
-typedef __bf16 ob_bf8 __attribute__((ext_vector_type(8)));
 typedef __bf16 ob_bf4 __attribute__((ext_vector_type(4)));
 
 template <typename E> struct ObElem;
@@ -344,13 +343,6 @@ __global__ __launch_bounds__(256, MT >= 4 ? 2 : 3) void ob_dense_skinny_kernel(c
 // Workgroup = NB n tiles x TB token tiles, waves WN x WT; NST stages of one k tile each in LDS, filled by 1 KB DMAs, ONE raw barrier
 // per k tile behind a counted vmcnt: at the top of step k the tile k has landed (at most the NST - 2 younger ones are outstanding),
 // the barrier tells everyone, and the buffer of tile k - 1 -- whose operand reads are complete -- takes tile k + NST - 1.
-__device__ __forceinline__ void ob_dma_1k(const char *base, uint32_t lane_off, uint32_t lds_addr)
-{
-    uint32_t keep;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3\n\ts_mov_b32 m0, %0"
-                 : "=&s"(keep) : "s"(lds_addr), "v"(lane_off), "s"(base) : "memory");
-}
-
 template <typename E, int EPI, int NB, int TB, int WN, int WT, int NST, int ROWS = OB_ROWS_ALL>
 __global__ __launch_bounds__(64 * WN * WT, 2) void ob_dense_tile_kernel(const typename ObDenseArgsOf<ROWS>::type A)
 {

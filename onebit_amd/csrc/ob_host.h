@@ -34,6 +34,13 @@ static inline void ob_set_max_lds_once(F kernel, bool (&done)[OB_MAX_DEVICES], i
     }
 }
 
+// ---- float32 layer on the matrix cores (onebit_f32.hip) -----------------------------------------------------------------
+// Workspace that the path needs (0: it does not take the shape), and the layer itself: false when it does not take the call (workspace, alignment,
+// N % 4 != 0) and nothing was launched.
+OB_HIDDEN size_t ob_f32_workspace(int64_t T, int64_t K, int64_t N);
+OB_HIDDEN bool ob_f32_forward(const void *packed, int64_t ldw_bytes, const float *x, const float *h, const float *g, const float *bias, float *y, float *u,
+                              void *workspace, size_t workspace_bytes, int64_t T, int64_t K, int64_t N, float eps, int skip, hipStream_t s);
+
 // ---- launchers of onebit_hip.hip that the mixed prefill + decode step (onebit_mixed.hip) drives directly ----------------
 // Row kernel of the batched / prefill glue (ob_b_norm_kernel) in every form the mixed step needs:
 //   embed != NULL:  r = embed[tokens[t]]                        (layer 0: modeling_bitllama.py:1275)
