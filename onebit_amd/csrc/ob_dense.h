@@ -9,7 +9,7 @@
 // fp32: four v_mfma_f32_16x16x4_f32 per tile pair; element j of every lane's four is one instruction's k, the same on both operands.
 // Products are computed transposed, D[n][t] = sum_k W[n][k] A[t][k]: a lane holds four consecutive output columns n of one token t.
 #pragma once
-#include "ob_common.h"
+#include "ob_mm.h"
 
 typedef __bf16 ob_bf4 __attribute__((ext_vector_type(4)));
 
@@ -107,7 +107,8 @@ enum ObDenseFn { OB_FN_ID = 0, OB_FN_XIELU = 1 };
 //   OB_ROWS_TABLE   few rows, formed here: gelu_tanh(sum of `n_pre` partial sums of another product) times the token's row of a table
 //   OB_ROWS_SEGS    rows of several requests' cache slots (fragment-major bands), output rows consecutive per request
 enum ObRowForm { OB_ROWS_ALL = 0, OB_ROWS_HEADS = 1, OB_ROWS_GATHER = 2, OB_ROWS_SORTED = 3, OB_ROWS_SEGS = 4, OB_ROWS_TABLE = 5 };
-struct ObRowBlock { int32_t group, row0, count, pad; };      // rows [row0, row0 + count) of weight group `group`; row0 a multiple of 16 at a group's start
+// rows [row0, row0 + count) of weight group `group`; row0 a multiple of 16 at a group's start.  n_used (of the table's first entry): the blocks with rows
+struct ObRowBlock { int32_t group, row0, count, n_used; };
 
 struct ObDenseArgs {
     const void *w, *a;             // fragment-major weights [n_tiles][nkt], activations [t tiles][nkt]
@@ -340,65 +341,105 @@ __global__ __launch_bounds__(256, MT >= 4 ? 2 : 3) void ob_dense_skinny_kernel(c
 }
 
 // ---- many rows: LDS-DMA tiles ------------------------------------------------------------------------------------------
-// Workgroup = NB n tiles x TB token tiles, waves WN x WT; NST stages of one k tile each in LDS, filled by 1 KB DMAs, ONE raw barrier
-// per k tile behind a counted vmcnt: at the top of step k the tile k has landed (at most the NST - 2 younger ones are outstanding),
-// the barrier tells everyone, and the buffer of tile k - 1 -- whose operand reads are complete -- takes tile k + NST - 1.
-template <typename E, int EPI, int NB, int TB, int WN, int WT, int NST, int ROWS = OB_ROWS_ALL>
-__global__ __launch_bounds__(64 * WN * WT, 2) void ob_dense_tile_kernel(const typename ObDenseArgsOf<ROWS>::type A)
+// Which rows and weights an output tile has: `rows` of them, activations from band `band0` on, outputs from row `out0` on, weight tiles from w0 on
+struct ObDenseRows { int band0, out0, rows; size_t w0; };
+template <int ROWS, int TB> __device__ __forceinline__ ObDenseRows ob_dense_rows(const typename ObDenseArgsOf<ROWS>::type &A, int tb)
 {
-    static_assert(ROWS != OB_ROWS_HEADS, "the block-diagonal form has few rows only");
-    typedef typename ObElem<E>::V16 V16;
-    constexpr int NW = WN * WT, TILES = NB + TB, PER = TILES / NW, MN = NB / WN, MT = TB / WT;
-    static_assert(TILES % NW == 0 && NB % WN == 0 && TB % WT == 0 && MN % 2 == 0, "tile shape");
-    extern __shared__ __attribute__((aligned(16))) char smem[];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wn = wave % WN, wt = wave / WN;
-    // XCD-aware numbering: workgroup ids are dealt round-robin to the 8 XCDs; give each a contiguous range of logical tiles, token
-    // blocks fastest, so that the tiles in flight on an XCD share weight bands and activation rows in its L2
-    const int ntb = (A.T + TB * 16 - 1) / (TB * 16);                   // (grouped forms: T = 16 TB times the number of blocks)
-    const int nwg = gridDim.x, orig = blockIdx.x, xcd = orig & 7, q8 = nwg >> 3, rem = nwg & 7;
-    const int bid = (xcd < rem ? xcd * (q8 + 1) : rem * (q8 + 1) + (xcd - rem) * q8) + (orig >> 3);
-    const int nb = bid / ntb, tb = bid - nb * ntb;
-    const int n0 = nb * NB, split = blockIdx.y;
-    // rows of this block: `rows` of them, activations from band `band0` on, outputs from row `out0` on
-    int band0 = tb * TB, out0 = tb * TB * 16, rows = A.T - out0;
-    size_t wg = 0;
+    ObDenseRows b = {tb * TB, tb * TB * 16, A.T - tb * TB * 16, 0};
     if constexpr (ROWS == OB_ROWS_GATHER || ROWS == OB_ROWS_SORTED) {
-        const ObRowBlock b = A.blk[tb];
-        if (b.count <= 0) return;                                     // (uniform)
-        band0 = b.row0 >> 4; out0 = b.row0; rows = b.count; wg = (size_t)b.group * A.w_group;
+        const ObRowBlock e = A.blk[tb];
+        b = {e.row0 >> 4, e.row0, e.count, (size_t)e.group * A.w_group};
     } else if constexpr (ROWS == OB_ROWS_SEGS) {
         int sg = 0;
         while (sg < A.nseg - 1 && tb >= A.blk_end[sg]) ++sg;
         const int loc = (tb - (sg ? A.blk_end[sg - 1] : 0)) * TB;
-        band0 = A.band0[sg] + loc; out0 = A.row0[sg] + loc * 16; rows = A.rows[sg] - loc * 16;
+        b.band0 = A.band0[sg] + loc; b.out0 = A.row0[sg] + loc * 16; b.rows = A.rows[sg] - loc * 16;
     }
-    const int k_lo = split * A.kt_split, k_hi = min(A.nkt, k_lo + A.kt_split), nk = k_hi - k_lo;
-    const int t_tiles = (rows + 15) >> 4;
-    const char *src[PER];
-    uint32_t loff[PER], kstep[PER];                                   // (two values, wave-uniform step: 1 KB tiles, or 64 bytes of a gathered row)
+    return b;
+}
+
+// Output tile of this workgroup.  Expert blocks: only those with rows are numbered -- the empty ones at the table's end would leave the last XCDs idle.
+template <int ROWS, int NB, int TB> __device__ __forceinline__ bool ob_dense_tile_of(const ObDenseArgs &A, int &nb, int &tb)
+{
+    int ntb = (A.T + TB * 16 - 1) / (TB * 16);                         // (grouped forms: T = 16 TB times the number of blocks)
+    if constexpr (ROWS == OB_ROWS_GATHER || ROWS == OB_ROWS_SORTED) ntb = A.blk[0].n_used;
+    return ob_tile_of(blockIdx.x, (A.n_tiles + NB - 1) / NB, ntb, nb, tb);
+}
+
+// One transfer of an output tile's k steps: tile j of the NB + TB of a step
+struct ObDenseSrc { const char *base; uint32_t lane_off; };
+template <typename E, int ROWS, int NB> __device__ __forceinline__ ObDenseSrc ob_dense_src(const ObDenseArgs &A, const ObDenseRows &b, int n0, int k_lo, int j, int lane)
+{
+    if (ROWS == OB_ROWS_GATHER && j >= NB)
+        return {(const char *)A.a + (size_t)k_lo * 64,
+                (uint32_t)A.gather[b.out0 + min((j - NB) * 16 + (lane & 15), b.rows - 1)] * (uint32_t)(A.lda * sizeof(E)) + (lane >> 4) * 16};
+    const size_t band = j < NB ? (size_t)min(n0 + j, A.n_tiles - 1) : (size_t)(b.band0 + min(j - NB, ((b.rows + 15) >> 4) - 1));
+    return {(const char *)(j < NB ? A.w : A.a) + ((j < NB ? b.w0 : 0) + band * A.nkt + k_lo) * 1024, (uint32_t)lane * 16};
+}
+
+// bf16: workgroup = 16 NB columns x 16 TB rows, four waves 2 x 2 (ob_mm.h has the loop).  NB = 16, TB = 8, three stages of 24 KB: 6016 x 2048 x 9728
+// 277 us with the tiles of 128 x 128 that stood here (8 KB of LDS reads per 16 MFMAs: LDS-bound) -> 224, 6016 x 17920 x 2048 532 -> 391,
+// 16384 x 11008 x 4096 1467 -> 1237 = 1194 TFLOP/s (fp32 sums written).  NB = TB = 8, four stages of 16 KB, where that leaves less than two
+// rounds of workgroups (1520 x 2048 x 9728: 80 us against 127).
+template <int EPI, int NB, int TB, int NST, int ROWS = OB_ROWS_ALL>
+__global__ __launch_bounds__(256, 2) void ob_dense_mm_kernel(const typename ObDenseArgsOf<ROWS>::type A)
+{
+    static_assert(ROWS != OB_ROWS_HEADS && ROWS != OB_ROWS_TABLE, "forms with few rows only");
+    constexpr int TILES = NB + TB, PER = TILES / 4, MN = NB / 2, MT = TB / 2;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wn = wave & 1, wt = wave >> 1;
+    int nb, tb;
+    if (!ob_dense_tile_of<ROWS, NB, TB>(A, nb, tb)) return;                         // (uniform)
+    const int n0 = nb * NB, split = blockIdx.y, k_lo = split * A.kt_split, nk = min(A.nkt - k_lo, A.kt_split);
+    const ObDenseRows b = ob_dense_rows<ROWS, TB>(A, tb);
+    if (b.rows <= 0) return;                                                         // (uniform)
+    ObDenseSrc src[PER];
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-        const int j = wave * PER + i;
-        const size_t band = j < NB ? (size_t)min(n0 + j, A.n_tiles - 1) : (size_t)(band0 + min(j - NB, t_tiles - 1));
-        src[i] = (const char *)(j < NB ? A.w : A.a) + ((j < NB ? wg : 0) + band * A.nkt + k_lo) * 1024;
-        loff[i] = lane * 16;
-        kstep[i] = 1024;
-        if constexpr (ROWS == OB_ROWS_GATHER) {
-            if (j >= NB) {
-                src[i] = (const char *)A.a + (size_t)k_lo * 64;
-                loff[i] = (uint32_t)A.gather[out0 + min((j - NB) * 16 + (lane & 15), rows - 1)] * (uint32_t)(A.lda * sizeof(E)) + (lane >> 4) * 16;
-                kstep[i] = 64;
-            }
-        }
-    }
+    for (int d = 0; d < PER; ++d) src[d] = ob_dense_src<__bf16, ROWS, NB>(A, b, n0, k_lo, wave * PER + d, lane);
     const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char *)smem;
-    auto dma = [&](int k, int buf) {
+    const auto dma = [&](int d, int k, int buf) {
+        const size_t kk = (size_t)min(k, nk - 1);
+        ob_dma_1k(src[d].base + kk * (ROWS == OB_ROWS_GATHER && wave * PER + d >= NB ? 64 : 1024), ROWS == OB_ROWS_GATHER ? src[d].lane_off : lane * 16,
+                  lds0 + (uint32_t)(buf * TILES + wave * PER + d) * 1024);
+    };
+    const auto tile = [&](int buf, int j) { return *reinterpret_cast<const ob_u32x4 *>(smem + (buf * TILES + j) * 1024 + lane * 16); };
+    ob_float4 acc[MN][MT];
+    ob_mm_loop<true, MN, MT, PER, NST>(acc, nk, [&](int buf, int i) { return tile(buf, wn * MN + i); }, [&](int buf, int j) { return tile(buf, NB + wt * MT + j); }, dma);
+    const int g = lane >> 4;
+#pragma unroll
+    for (int j = 0; j < MT; ++j) {
+        const int tl = (wt * MT + j) * 16 + (lane & 15);
+#pragma unroll
+        for (int i = 0; i < MN; i += 2) ob_dense_epilogue<__bf16, EPI>(A, n0 + wn * MN + i, b.out0 + tl, tl < b.rows, g, acc[i][j], acc[i + 1][j], split);
+    }
+}
+
+// fp32: workgroup = 8 n tiles x 8 token tiles, waves 2 x 2; four stages of one k tile each in LDS, ONE raw barrier per k tile behind a counted
+// vmcnt: at the top of step k the tile k has landed (at most the two younger ones are outstanding), the barrier tells everyone, and the buffer of
+// tile k - 1 -- whose operand reads are complete -- takes tile k + 3.  Bound by the fp32 matrix rate.
+template <int EPI, int ROWS = OB_ROWS_ALL>
+__global__ __launch_bounds__(256, 2) void ob_dense_tile_f32_kernel(const typename ObDenseArgsOf<ROWS>::type A)
+{
+    typedef float E;
+    typedef ObElem<E>::V16 V16;
+    constexpr int NB = 8, TB = 8, TILES = NB + TB, PER = TILES / 4, MN = NB / 2, MT = TB / 2, NST = 4;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wn = wave & 1, wt = wave >> 1;
+    int nb, tb;
+    if (!ob_dense_tile_of<ROWS, NB, TB>(A, nb, tb)) return;                         // (uniform)
+    const int n0 = nb * NB, split = blockIdx.y, k_lo = split * A.kt_split, nk = min(A.nkt - k_lo, A.kt_split);
+    const ObDenseRows b = ob_dense_rows<ROWS, TB>(A, tb);
+    if (b.rows <= 0) return;                                                         // (uniform)
+    ObDenseSrc src[PER];
+#pragma unroll
+    for (int d = 0; d < PER; ++d) src[d] = ob_dense_src<E, ROWS, NB>(A, b, n0, k_lo, wave * PER + d, lane);
+    const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char *)smem;
+    const auto dma = [&](int k, int buf) {
         const size_t kk = (size_t)min(k, nk - 1);
 #pragma unroll
-        for (int i = 0; i < PER; ++i)
-            ob_dma_1k(src[i] + kk * (ROWS == OB_ROWS_GATHER ? kstep[i] : 1024), ROWS == OB_ROWS_GATHER ? loff[i] : lane * 16,
-                      lds0 + (uint32_t)(buf * TILES + wave * PER + i) * 1024);
+        for (int d = 0; d < PER; ++d)
+            ob_dma_1k(src[d].base + kk * (ROWS == OB_ROWS_GATHER && wave * PER + d >= NB ? 64 : 1024), src[d].lane_off,
+                      lds0 + (uint32_t)(buf * TILES + wave * PER + d) * 1024);
     };
     ob_float4 acc[MN][MT];
 #pragma unroll
@@ -431,6 +472,6 @@ __global__ __launch_bounds__(64 * WN * WT, 2) void ob_dense_tile_kernel(const ty
     for (int j = 0; j < MT; ++j) {
         const int tl = (wt * MT + j) * 16 + (lane & 15);
 #pragma unroll
-        for (int i = 0; i < MN; i += 2) ob_dense_epilogue<E, EPI>(A, n0 + wn * MN + i, out0 + tl, tl < rows, g, acc[i][j], acc[i + 1][j], split);
+        for (int i = 0; i < MN; i += 2) ob_dense_epilogue<E, EPI>(A, n0 + wn * MN + i, b.out0 + tl, tl < b.rows, g, acc[i][j], acc[i + 1][j], split);
     }
 }

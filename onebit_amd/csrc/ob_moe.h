@@ -113,6 +113,8 @@ __device__ __forceinline__ void ob_route_offsets(const ObRouteArgs &A, int *cnt,
         }
     }
     for (int k = blk_base + tid; k < A.n_blk; k += 1024) A.blk[k] = {0, 0, 0, 0};
+    __syncthreads();                                                  // (the table's first entry is written)
+    if (tid == 0 && A.n_blk > 0) A.blk[0].n_used = min(blk_base, A.n_blk);
 }
 
 // first pass: choices, weights, and this workgroup's tokens per expert.  SINGLE: up to 64 tokens in one workgroup, everything in one launch.

@@ -72,6 +72,21 @@ static int gemm_splits(int n_tiles, int nkt, int T)
     return (int)std::max<int64_t>(1, s);
 }
 
+// the LDS-DMA tiles over `n_tb` blocks of 128 rows: 256 columns wide from two rounds of workgroups on (two per CU), else 128
+template <typename E, int EPI, int ROWS>
+static int tiles_launch(const typename ObDenseArgsOf<ROWS>::type &a, int64_t n_tb, int n_split, const char *what, hipStream_t s)
+{
+    const auto go = [&](auto k, int nb, int lds) {
+        if (!lds_ok((const void *)k, lds)) return hfail(ONEBIT_E_SHAPE, "%s: LDS", what);
+        hipLaunchKernelGGL(k, dim3((unsigned)(cdiv(a.n_tiles, nb) * n_tb), (unsigned)n_split), dim3(256), lds, s, a);
+        return hstatus(what);
+    };
+    if constexpr (sizeof(E) == 2) {
+        if (cdiv(a.n_tiles, 16) * n_tb * n_split >= 1024) return go(ob_dense_mm_kernel<EPI, 16, 8, 3, ROWS>, 16, 3 * 24 * 1024);
+        return go(ob_dense_mm_kernel<EPI, 8, 8, 4, ROWS>, 8, 4 * 16 * 1024);
+    } else return go(ob_dense_tile_f32_kernel<EPI, ROWS>, 8, 4 * 16 * 1024);
+}
+
 template <typename E, int EPI>
 static int dense_launch(ObDenseArgs a, int n_split, hipStream_t s)
 {
@@ -85,20 +100,7 @@ static int dense_launch(ObDenseArgs a, int n_split, hipStream_t s)
         else hipLaunchKernelGGL((ob_dense_skinny_kernel<E, EPI, 4>), grid, dim3(256), 0, s, a);
         return hstatus("dense product");
     }
-    if constexpr (sizeof(E) == 2) {
-        if (cdiv(a.n_tiles, 16) * cdiv(a.T, 256) * n_split >= 224) {
-            auto k = ob_dense_tile_kernel<E, EPI, 16, 16, 2, 4, 4>;
-            const int lds = 4 * 32 * 1024;
-            if (!lds_ok((const void *)k, lds)) return hfail(ONEBIT_E_SHAPE, "dense product: LDS");
-            hipLaunchKernelGGL(k, dim3((unsigned)(cdiv(a.n_tiles, 16) * cdiv(a.T, 256)), (unsigned)n_split), dim3(512), lds, s, a);
-            return hstatus("dense product");
-        }
-    }
-    auto k = ob_dense_tile_kernel<E, EPI, 8, 8, 2, 2, 4>;
-    const int lds = 4 * 16 * 1024;
-    if (!lds_ok((const void *)k, lds)) return hfail(ONEBIT_E_SHAPE, "dense product: LDS");
-    hipLaunchKernelGGL(k, dim3((unsigned)(cdiv(a.n_tiles, 8) * cdiv(a.T, 128)), (unsigned)n_split), dim3(256), lds, s, a);
-    return hstatus("dense product");
+    return tiles_launch<E, EPI, OB_ROWS_ALL>(a, cdiv(a.T, 128), n_split, "dense product", s);
 }
 
 // few rows, block-diagonal over heads (row-major activations), 64 rows at a time.  `out_step`: bytes of 64 output rows.
@@ -120,7 +122,7 @@ static int dense_heads_launch(ObDenseArgs a, size_t out_step, hipStream_t s)
     return hstatus("per-head product");
 }
 
-// the rows of experts: n_blk blocks of at most block_rows (64: few rows; 128 / 256: tiles)
+// the rows of experts: n_blk blocks of at most block_rows (64: few rows; 128: tiles)
 template <typename E, int EPI, int ROWS>
 static int dense_blocks_launch(ObDenseArgs a, int n_blk, int block_rows, int n_split, hipStream_t s)
 {
@@ -134,20 +136,7 @@ static int dense_blocks_launch(ObDenseArgs a, int n_blk, int block_rows, int n_s
         return hstatus("expert product");
     }
     a.T = n_blk * block_rows;
-    if constexpr (sizeof(E) == 2) {
-        if (block_rows == 256) {
-            auto k = ob_dense_tile_kernel<E, EPI, 16, 16, 2, 4, 4, ROWS>;
-            const int lds = 4 * 32 * 1024;
-            if (!lds_ok((const void *)k, lds)) return hfail(ONEBIT_E_SHAPE, "expert product: LDS");
-            hipLaunchKernelGGL(k, dim3((unsigned)(cdiv(a.n_tiles, 16) * n_blk), (unsigned)n_split), dim3(512), lds, s, a);
-            return hstatus("expert product");
-        }
-    }
-    auto k = ob_dense_tile_kernel<E, EPI, 8, 8, 2, 2, 4, ROWS>;
-    const int lds = 4 * 16 * 1024;
-    if (!lds_ok((const void *)k, lds)) return hfail(ONEBIT_E_SHAPE, "expert product: LDS");
-    hipLaunchKernelGGL(k, dim3((unsigned)(cdiv(a.n_tiles, 8) * n_blk), (unsigned)n_split), dim3(256), lds, s, a);
-    return hstatus("expert product");
+    return tiles_launch<E, EPI, ROWS>(a, n_blk, n_split, "expert product", s);
 }
 
 extern "C" int onebit_hybrid_gemm_splits(int32_t n_tiles, int32_t nkt, int32_t T) { return n_tiles > 0 && nkt > 0 && T > 0 ? gemm_splits(n_tiles, nkt, T) : 0; }
@@ -621,16 +610,12 @@ static int latent_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, con
             ObDenseSegArgs e = {};
             ObFlashSigArgs f = {};
             int64_t rows = 0, wgs = 0;
-            int64_t keys = 0;
-            for (int i = s0; i < st.n_seg && e.nseg < OB_DENSE_MAXSEG; ++i) keys += st.segs[i].past + st.segs[i].n;
-            const bool big = cdiv(2 * H * L.kp, 256) * cdiv(std::min(keys, P.kv_rows), 256) >= 224;
-            const int br = big ? 256 : 128;
             int blocks = 0, i = s0;
             for (; i < st.n_seg && e.nseg < OB_DENSE_MAXSEG; ++i) {
                 const onebit_hseg_t &g = st.segs[i];
                 const int len = g.past + g.n, n = e.nseg;
                 if (rows + rup(len, 16) > P.kv_rows) break;
-                blocks += (int)cdiv(len, br);
+                blocks += (int)cdiv(len, 128);
                 e.blk_end[n] = blocks; e.band0[n] = g.slot * bands; e.row0[n] = (int)rows; e.rows[n] = len;
                 wgs += (cdiv(g.n, OB_FL_BM) + 1) / 2 * H;
                 if (wgs > 0x3fffffffLL) return hfail(ONEBIT_E_ARG, "attention: too many workgroups");
@@ -640,16 +625,9 @@ static int latent_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, con
                 rows += rup(len, 16);
             }
             if (i == s0) return hfail(ONEBIT_E_SHAPE, "latent attention: chunk %d does not fit the expansion buffer", s0);
-            e.w = l.w_kv; e.a = run.s0; e.n_tiles = 2 * H * L.kp / 16; e.nkt = l.rp / KT; e.kt_split = e.nkt; e.T = blocks * br;
+            e.w = l.w_kv; e.a = run.s0; e.n_tiles = 2 * H * L.kp / 16; e.nkt = l.rp / KT; e.kt_split = e.nkt; e.T = blocks * 128;
             e.heads = ws + P.kv; e.d_shift = sh; e.head_rows = (int)P.kv_rows;
-            auto go = [&](auto kern, int nb, int thr, int lds) {
-                if (!lds_ok((const void *)kern, lds)) return hfail(ONEBIT_E_SHAPE, "expansion: LDS");
-                hipLaunchKernelGGL(kern, dim3((unsigned)(cdiv(e.n_tiles, nb) * blocks)), dim3(thr), lds, s, e);
-                return hstatus("expansion");
-            };
-            const int rc = big ? go(ob_dense_tile_kernel<E, OB_EPI_HEADS, 16, 16, 2, 4, 4, OB_ROWS_SEGS>, 16, 512, 128 * 1024)
-                               : go(ob_dense_tile_kernel<E, OB_EPI_HEADS, 8, 8, 2, 2, 4, OB_ROWS_SEGS>, 8, 256, 64 * 1024);
-            if (rc) return rc;
+            if (const int rc = tiles_launch<E, OB_EPI_HEADS, OB_ROWS_SEGS>(e, blocks, 1, "expansion", s)) return rc;
             f.a.q = (const _Float16 *)(ws + P.qu); f.a.k = (const _Float16 *)(ws + P.kv); f.a.v = f.a.k + (size_t)H * P.kv_rows * L.kp;     // (bf16 behind these pointers)
             f.a.H = f.a.Hkv = H; f.a.max_len = (int)P.kv_rows;
             f.a.scale_log2e = L.scale * OB_LOG2E;
@@ -692,8 +670,7 @@ static int ff_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, const o
     const int64_t TK = (int64_t)T * f.top, S = expert_rows(f, T);
     if ((int64_t)T * m.width_pad * (int)sizeof(E) > 0xffffffffLL || S > 0x7fffffff / 16) return hfail(ONEBIT_E_SHAPE, "experts: %d rows in one step", T);
     const int64_t live = std::min<int64_t>(f.experts, TK);
-    int br = OB_SKINNY_T;
-    if (T > OB_SKINNY_T) br = sizeof(E) == 2 && TK / f.experts >= 384 ? 256 : 128;
+    const int br = T > OB_SKINNY_T ? 128 : OB_SKINNY_T;
     const int n_blk = (int)(live + (br == OB_SKINNY_T ? 0 : TK / br));
     ObRouteArgs r = {};
     int32_t *at = (int32_t *)(ws + P.route);
