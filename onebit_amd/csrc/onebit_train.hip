@@ -3,31 +3,125 @@
 #include <type_traits>
 #include "ob_host.h"
 #include "ob_train.h"
+#include "ob_train16.h"
 
 // onebit_train_forward / onebit_train_backward: bitnet.py:14-28 (SignSTE) and :58-68 (BitLinear.forward)
 template <typename TI, bool RCA, bool RCB, int TXA, int TXB, int EPI>
 static void ob_launch_tgemm(const ObTGemmArgs &a, hipStream_t s)
 {
-    if constexpr (std::is_same<TI, _Float16>::value) {      // gfx950 tiling for fp16 (ob_train.h); fp32 keeps the 64 x 64 form
-        static const bool legacy = getenv("OB_TRAIN_GEMM64") != nullptr;
-        if (!legacy) {
-            const dim3 grid((unsigned)((a.N + OB_TG2_B - 1) / OB_TG2_B), (unsigned)((a.M + OB_TG2_B - 1) / OB_TG2_B));
-            static bool attr_set[OB_MAX_DEVICES] = {};
-            ob_set_max_lds_once(ob_tgemm128_f16_kernel<RCA, RCB, TXA, TXB, EPI>, attr_set, OB_TG2_LDS);
-            hipLaunchKernelGGL((ob_tgemm128_f16_kernel<RCA, RCB, TXA, TXB, EPI>), grid, dim3(OB_TG_THREADS), OB_TG2_LDS, s, a);
-            return;
-        }
-    }
     const dim3 grid((unsigned)((a.N + OB_TG_BN - 1) / OB_TG_BN), (unsigned)((a.M + OB_TG_BM - 1) / OB_TG_BM));
     hipLaunchKernelGGL((ob_tgemm_kernel<TI, RCA, RCB, TXA, TXB, EPI>), grid, dim3(OB_TG_THREADS), 0, s, a);
 }
 
 static size_t ob_train_align(size_t b) { return (b + 255) & ~(size_t)255; }
 
+// ---- float16 (ob_train16.h) ---------------------------------------------------------------------------------------------
+static int64_t ob_t16_up32(int64_t n) { return (n + 31) / 32 * 32; }
+static size_t ob_t16_bytes(int64_t rows, int64_t cols) { return (size_t)ob_t16_up32(rows) * ob_t16_up32(cols) * 2; }
+// band slices of the column sums, and the sums' bytes ([slices][2][N]; the input gradient's: two per block of 128 rows, [..][K])
+static int ob_t16_slices(int64_t T) { const int64_t bands = ob_t16_up32(T) / 16; return (int)(bands < OB_TC_SLICES ? bands : OB_TC_SLICES); }
+static size_t ob_t16_part_bytes(int64_t T, int64_t K, int64_t N)
+{
+    const size_t a = (size_t)ob_t16_slices(T) * 2 * N * 4, b = (size_t)((T + 127) / 128) * 2 * K * 4;
+    return ob_train_align(a > b ? a : b);
+}
+
+static void ob_t16_tiles(bool sign, const void *p, const void *vec, char *out, int64_t rows, int64_t cols, hipStream_t s)
+{
+    ObT16Tiles a = {(const _Float16 *)p, (const _Float16 *)vec, out, (int)rows, (int)cols, (int)(ob_t16_up32(rows) / 16), (int)(ob_t16_up32(cols) / 32)};
+    const unsigned grid = (unsigned)(((int64_t)a.bands * ((a.ct + 3) / 4) + 3) / 4);
+    if (sign) hipLaunchKernelGGL(ob_t16_tiles_kernel<OB_T16_SIGN>, dim3(grid), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL(ob_t16_tiles_kernel<OB_T16_SCALE>, dim3(grid), dim3(256), 0, s, a);
+}
+
+// 256 x 128 outputs a workgroup from two rounds of them on (two per CU), else 128 x 128
+template <int EPI, bool TRW, bool TRA>
+static void ob_t16_mm(const ObT16Mm &a, hipStream_t s)
+{
+    const int64_t tb = (a.na + 7) / 8, nb = (a.nw + 15) / 16;
+    if (nb * tb >= 4 * (int64_t)ob_cu_count()) {
+        static bool attr_set[OB_MAX_DEVICES] = {};
+        ob_set_max_lds_once(ob_t16_mm_kernel<EPI, TRW, TRA, 16, 8, 3>, attr_set, 3 * 24 * 1024);
+        hipLaunchKernelGGL((ob_t16_mm_kernel<EPI, TRW, TRA, 16, 8, 3>), dim3((unsigned)(nb * tb)), dim3(256), 3 * 24 * 1024, s, a);
+    } else {
+        static bool attr_set[OB_MAX_DEVICES] = {};
+        ob_set_max_lds_once(ob_t16_mm_kernel<EPI, TRW, TRA, 8, 8, 4>, attr_set, 4 * 16 * 1024);
+        hipLaunchKernelGGL((ob_t16_mm_kernel<EPI, TRW, TRA, 8, 8, 4>), dim3((unsigned)((a.nw + 7) / 8 * tb)), dim3(256), 4 * 16 * 1024, s, a);
+    }
+}
+
+// rows in registers where their width and alignment allow, else ob_train_ln_fwd_kernel
+static void ob_t16_layernorm(const void *z, const void *g, const void *bias, void *y, float *stats, int64_t T, int64_t N, float eps, hipStream_t s)
+{
+#define OB_T16_LN(NV_) hipLaunchKernelGGL(ob_t16_ln_kernel<NV_>, dim3((unsigned)T), dim3(256), 0, s, (const _Float16 *)z, (const _Float16 *)g, \
+                                          (const _Float16 *)bias, (_Float16 *)y, stats, (int)N, eps)
+    if (N % 8 != 0 || N > 16384 || !ob_aligned(z, 16) || !ob_aligned(g, 16) || !ob_aligned(y, 16) || (bias && !ob_aligned(bias, 16)))
+        hipLaunchKernelGGL((ob_train_ln_fwd_kernel<_Float16>), dim3((unsigned)T), dim3(256), 0, s, (const _Float16 *)z, (const _Float16 *)g,
+                           (const _Float16 *)bias, (_Float16 *)y, stats, (int)N, eps);
+    else if (N <= 2048) OB_T16_LN(1);
+    else if (N <= 4096) OB_T16_LN(2);
+    else if (N <= 8192) OB_T16_LN(4);
+    else if (N <= 12288) OB_T16_LN(6);
+    else OB_T16_LN(8);
+#undef OB_T16_LN
+}
+
+static int ob_t16_forward(const void *x, const void *w, const void *h, const void *g, const void *bias, void *y, void *z, float *stats, char *ws,
+                          int64_t T, int64_t K, int64_t N, float eps, hipStream_t s)
+{
+    char *a = ws, *sg = ws + ob_t16_bytes(T, K);
+    ob_t16_tiles(false, x, h, a, T, K, s);
+    ob_t16_tiles(true, w, nullptr, sg, N, K, s);
+    const int kt = (int)(ob_t16_up32(K) / 32);
+    ObT16Mm m = {sg, a, (int)((N + 15) / 16), (int)((T + 15) / 16), kt, kt, kt, (_Float16 *)z, (int)T, (int)N};
+    m.vec4 = N % 4 == 0 && ob_aligned(z, 8);
+    ob_t16_mm<OB_T16_Z, false, false>(m, s);
+    int rc = ob_launch_status("train_forward(product)");
+    if (rc) return rc;
+    ob_t16_layernorm(z, g, bias, y, stats, T, N, eps, s);
+    return ob_launch_status("train_forward(layernorm)");
+}
+
+static int ob_t16_backward(const void *gy, const void *x, const void *w, const void *h, const void *g, const void *z, const float *stats, void *gx, void *gw,
+                           void *gh, void *gg, void *gbias, char *ws, int64_t T, int64_t K, int64_t N, hipStream_t s)
+{
+    char *a = ws, *sg = a + ob_t16_bytes(T, K), *gz = sg + ob_t16_bytes(N, K);
+    float *part = (float *)(gz + ob_t16_bytes(T, N)), *rowc = (float *)((char *)part + ob_t16_part_bytes(T, K, N));
+    const int kt = (int)(ob_t16_up32(K) / 32), nt = (int)(ob_t16_up32(N) / 32), tt = (int)(ob_t16_up32(T) / 32), slices = ob_t16_slices(T);
+    ObT16Gz q = {(const _Float16 *)gy, (const _Float16 *)z, (const _Float16 *)g, stats, rowc, part, gz, (int)T, (int)N, 2 * tt, nt, (2 * tt + slices - 1) / slices};
+    int rc;
+    hipLaunchKernelGGL(ob_t16_rowc_kernel, dim3((unsigned)T), dim3(256), 0, s, q);
+    hipLaunchKernelGGL(ob_t16_gz_kernel, dim3((unsigned)((nt + 3) / 4), (unsigned)slices), dim3(256), 0, s, q);
+    hipLaunchKernelGGL(ob_t16_cols_kernel<2>, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, s, (const float *)part, (_Float16 *)gg, (_Float16 *)gbias, (int)N, slices);
+    ob_t16_tiles(false, x, h, a, T, K, s);
+    ob_t16_tiles(true, w, nullptr, sg, N, K, s);
+    if ((rc = ob_launch_status("train_backward(layernorm)"))) return rc;
+    // gx [T, K] = fp16(gz S) h;  gh = sum_t fp16(gz S) x
+    ObT16Mm m = {sg, gz, (int)((K + 15) / 16), (int)((T + 15) / 16), kt, nt, nt, (_Float16 *)gx, (int)T, (int)K, (const _Float16 *)h, (const _Float16 *)x, part};
+    m.vec4 = K % 4 == 0 && ob_aligned(gx, 8) && ob_aligned(x, 8);
+    ob_t16_mm<OB_T16_GX, true, false>(m, s);
+    hipLaunchKernelGGL(ob_t16_cols_kernel<1>, dim3((unsigned)((K + 255) / 256)), dim3(256), 0, s, (const float *)part, (_Float16 *)gh, (_Float16 *)nullptr, (int)K,
+                       2 * (int)((T + 127) / 128));
+    if ((rc = ob_launch_status("train_backward(grad input)"))) return rc;
+    // gW [N, K] = (gz^T a) (1.001 - tanh(W)^2)
+    ObT16Mm v = {a, gz, (int)((K + 15) / 16), (int)((N + 15) / 16), kt, nt, tt, (_Float16 *)gw, (int)N, (int)K, (const _Float16 *)w};
+    v.vec4 = K % 4 == 0 && ob_aligned(gw, 8) && ob_aligned(w, 8);
+    ob_t16_mm<OB_T16_GW, true, true>(v, s);
+    return ob_launch_status("train_backward(grad weight)");
+}
+
+// Workspace of the forward pass: a smaller or absent one takes the kernels that transform operands on their way into LDS
+extern "C" size_t onebit_train_forward_workspace_bytes(int64_t T, int64_t K, int64_t N, int dtype)
+{
+    if (T <= 0 || K <= 0 || N <= 0 || dtype != ONEBIT_F16) return 0;
+    return ob_t16_bytes(T, K) + ob_t16_bytes(N, K);
+}
+
 extern "C" size_t onebit_train_workspace_bytes(int64_t T, int64_t K, int64_t N, int dtype)
 {
     if (T <= 0 || K <= 0 || N <= 0) return 0;
-    const size_t sz = dtype == ONEBIT_F32 ? 4 : 2;
+    if (dtype != ONEBIT_F32) return ob_t16_bytes(T, K) + ob_t16_bytes(N, K) + ob_t16_bytes(T, N) + ob_t16_part_bytes(T, K, N) + ob_train_align((size_t)T * 8);
+    const size_t sz = 4;
     return ob_train_align((size_t)T * N * sz) + ob_train_align((size_t)T * K * sz) + ob_train_align((size_t)T * 2 * sizeof(float)) +
            ob_train_align((size_t)OB_TC_SLICES * (2 * (size_t)N > (size_t)K ? 2 * (size_t)N : (size_t)K) * sizeof(float));     // column-sum partials
 }
@@ -48,7 +142,12 @@ static int ob_train_forward_t(const void *x, const void *w, const void *h, const
     a.A = x; a.lda = K; a.va = h;            // A(t, k) = x[t, k] * h[k]
     a.B = w; a.ldb = K;                      // B(n, k) = sign(W[n, k])
     a.C = z; a.ldc = N; a.M = (int)T; a.N = (int)N; a.R = (int)K;
-    ob_launch_tgemm<TI, true, true, OB_TX_SCALE_R, OB_TX_SIGN, OB_TE_PLAIN>(a, s);
+    if constexpr (std::is_same<TI, _Float16>::value) {
+        static bool attr_set[OB_MAX_DEVICES] = {};
+        ob_set_max_lds_once(ob_tgemm128_f16_kernel, attr_set, OB_TG2_LDS);
+        hipLaunchKernelGGL(ob_tgemm128_f16_kernel, dim3((unsigned)((N + OB_TG2_B - 1) / OB_TG2_B), (unsigned)((T + OB_TG2_B - 1) / OB_TG2_B)), dim3(OB_TG_THREADS),
+                           OB_TG2_LDS, s, a);
+    } else ob_launch_tgemm<TI, true, true, OB_TX_SCALE_R, OB_TX_SIGN, OB_TE_PLAIN>(a, s);
     int rc = ob_launch_status("train_forward(gemm)");
     if (rc) return rc;
     hipLaunchKernelGGL((ob_train_ln_fwd_kernel<TI>), dim3((unsigned)T), dim3(256), 0, s, (const TI *)z, (const TI *)g, (const TI *)bias,
@@ -56,9 +155,9 @@ static int ob_train_forward_t(const void *x, const void *w, const void *h, const
     return ob_launch_status("train_forward(layernorm)");
 }
 
-extern "C" int onebit_train_forward(const void *x, const void *w_latent, const void *h, const void *g, const void *bias_or_null,
-                                    void *y, void *z_save, float *ln_stats, int64_t T, int64_t K, int64_t N, int dtype,
-                                    float ln_eps, void *stream)
+extern "C" int onebit_train_forward_ws(const void *x, const void *w_latent, const void *h, const void *g, const void *bias_or_null,
+                                       void *y, void *z_save, float *ln_stats, void *workspace, size_t workspace_bytes, int64_t T, int64_t K, int64_t N,
+                                       int dtype, float ln_eps, void *stream)
 {
     int rc = ob_train_check("train_forward", T, K, N, dtype);
     if (rc) return rc;
@@ -66,8 +165,17 @@ extern "C" int onebit_train_forward(const void *x, const void *w_latent, const v
     if (K == 0) return ob_fail(ONEBIT_E_SHAPE, "train_forward: in_features = 0");
     if (!x || !w_latent || !h || !g || !y || !z_save || !ln_stats) return ob_fail(ONEBIT_E_ARG, "train_forward: null pointer");
     hipStream_t s = (hipStream_t)stream;
+    if (dtype == ONEBIT_F16 && workspace && ob_aligned(workspace, 16) && workspace_bytes >= onebit_train_forward_workspace_bytes(T, K, N, dtype))
+        return ob_t16_forward(x, w_latent, h, g, bias_or_null, y, z_save, ln_stats, (char *)workspace, T, K, N, ln_eps, s);
     return dtype == ONEBIT_F16 ? ob_train_forward_t<_Float16>(x, w_latent, h, g, bias_or_null, y, z_save, ln_stats, T, K, N, ln_eps, s)
                                : ob_train_forward_t<float>(x, w_latent, h, g, bias_or_null, y, z_save, ln_stats, T, K, N, ln_eps, s);
+}
+
+extern "C" int onebit_train_forward(const void *x, const void *w_latent, const void *h, const void *g, const void *bias_or_null,
+                                    void *y, void *z_save, float *ln_stats, int64_t T, int64_t K, int64_t N, int dtype,
+                                    float ln_eps, void *stream)
+{
+    return onebit_train_forward_ws(x, w_latent, h, g, bias_or_null, y, z_save, ln_stats, nullptr, 0, T, K, N, dtype, ln_eps, stream);
 }
 
 template <typename TI>
@@ -124,7 +232,7 @@ extern "C" int onebit_train_backward(const void *gy, const void *x, const void *
     if (!workspace || workspace_bytes < onebit_train_workspace_bytes(T, K, N, dtype) || !ob_aligned(workspace, 16))
         return ob_fail(ONEBIT_E_WSPACE, "train_backward: needs %zu bytes of 16-byte aligned workspace", onebit_train_workspace_bytes(T, K, N, dtype));
     hipStream_t s = (hipStream_t)stream;
-    return dtype == ONEBIT_F16 ? ob_train_backward_t<_Float16>(gy, x, w_latent, h, g, z_save, ln_stats, gx, gw, gh, gg, gbias_or_null, (char *)workspace, T, K, N, s)
+    return dtype == ONEBIT_F16 ? ob_t16_backward(gy, x, w_latent, h, g, z_save, ln_stats, gx, gw, gh, gg, gbias_or_null, (char *)workspace, T, K, N, s)
                                : ob_train_backward_t<float>(gy, x, w_latent, h, g, z_save, ln_stats, gx, gw, gh, gg, gbias_or_null, (char *)workspace, T, K, N, s);
 }
 

@@ -4,9 +4,8 @@
 constructor, parameter names (``weight`` latent full precision ``[out, in]``, ``weight_scale``, ``input_factor``,
 optional ``bias``) and state-dict keys, so a training checkpoint of the reference loads unchanged and
 ``checkpoint.convert_train_state_dict`` turns it into the packed inference layout.  Forward and backward run
-hand-written HIP kernels through the C ABI (``onebit_train_forward`` / ``onebit_train_backward``,
-``csrc/ob_train.h``): the sign is taken while the latent weights are staged for the MFMA GEMM (no dense +-1
-matrix in HBM), the backward pass applies the reference's straight-through estimator
+hand-written HIP kernels through the C ABI (``onebit_train_forward_ws`` / ``onebit_train_backward``,
+``csrc/ob_train.h``, float16 ``csrc/ob_train16.h``): the backward pass applies the reference's straight-through estimator
 ``grad * (1.001 - tanh(w)^2)`` (``SignSTEFunc.backward``, ``:21-23``) in the weight-gradient GEMM's epilogue.
 There is no CPU fallback: CPU tensors raise.  (The torch-ops restatement used to check this lives in
 ``oracle/train_ref.py``, test infrastructure.)
@@ -48,9 +47,12 @@ class _BitLinearFn(torch.autograd.Function):
         z = torch.empty((T, N), dtype=dt, device=x.device)
         stats = torch.empty((T, 2), dtype=torch.float32, device=x.device)
         lib = _lib.load()
+        nws = lib.onebit_train_forward_workspace_bytes(T, K, N, code)
+        ws = torch.empty(nws, dtype=torch.uint8, device=x.device) if nws else None
         with torch.cuda.device(x.device):
-            rc = lib.onebit_train_forward(x2.data_ptr(), w.data_ptr(), h.data_ptr(), g.data_ptr(), None if b is None else b.data_ptr(),
-                                          y.data_ptr(), z.data_ptr(), stats.data_ptr(), T, K, N, code, eps, _stream_ptr(x.device))
+            rc = lib.onebit_train_forward_ws(x2.data_ptr(), w.data_ptr(), h.data_ptr(), g.data_ptr(), None if b is None else b.data_ptr(),
+                                             y.data_ptr(), z.data_ptr(), stats.data_ptr(), None if ws is None else ws.data_ptr(), nws, T, K, N, code,
+                                             eps, _stream_ptr(x.device))
         _lib.check(rc, "onebit_train_forward")
         ctx.save_for_backward(x2, w, g, h, z, stats)
         ctx.has_bias, ctx.code, ctx.lead = b is not None, code, x.shape[:-1]
