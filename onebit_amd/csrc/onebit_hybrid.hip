@@ -58,6 +58,7 @@ static bool lds_ok(const void *f, int bytes)
 
 // ------------------------------------------------------------------------------------------------------ dense products --
 #define OB_SKINNY_T 64
+#define OB_DEEP_KT 61            // k tiles of a split from which every wave has 16 (the last one 13)
 #define OB_ZROWS 2048           // fp32 rows the partial-sum buffer holds at least: splits * T <= max(OB_ZROWS, T)
 
 // K splits of an output product: enough workgroups to fill the chip, each with a worthwhile share of k tiles
@@ -95,7 +96,8 @@ static int dense_launch(ObDenseArgs a, int n_split, hipStream_t s)
     n_split = (int)cdiv(a.nkt, a.kt_split);               // (no empty split)
     if (a.T <= OB_SKINNY_T) {
         const dim3 grid((unsigned)cdiv(a.n_tiles, 2), (unsigned)n_split);
-        if (a.T <= 16) hipLaunchKernelGGL((ob_dense_skinny_kernel<E, EPI, 1>), grid, dim3(256), 0, s, a);
+        if (a.T <= 16 && a.kt_split >= OB_DEEP_KT) hipLaunchKernelGGL((ob_dense_skinny_kernel<E, EPI, 1, OB_ROWS_ALL, true>), grid, dim3(256), 0, s, a);
+        else if (a.T <= 16) hipLaunchKernelGGL((ob_dense_skinny_kernel<E, EPI, 1>), grid, dim3(256), 0, s, a);
         else if (a.T <= 32) hipLaunchKernelGGL((ob_dense_skinny_kernel<E, EPI, 2>), grid, dim3(256), 0, s, a);
         else hipLaunchKernelGGL((ob_dense_skinny_kernel<E, EPI, 4>), grid, dim3(256), 0, s, a);
         return hstatus("dense product");
@@ -130,7 +132,8 @@ static int dense_blocks_launch(ObDenseArgs a, int n_blk, int block_rows, int n_s
     n_split = (int)cdiv(a.nkt, a.kt_split);
     if (block_rows <= OB_SKINNY_T) {
         const dim3 grid((unsigned)cdiv(a.n_tiles, 2), (unsigned)n_split, (unsigned)n_blk);
-        if (a.T <= 16) hipLaunchKernelGGL((ob_dense_skinny_kernel<E, EPI, 1, ROWS>), grid, dim3(256), 0, s, a);
+        if (a.T <= 16 && a.kt_split >= OB_DEEP_KT) hipLaunchKernelGGL((ob_dense_skinny_kernel<E, EPI, 1, ROWS, true>), grid, dim3(256), 0, s, a);
+        else if (a.T <= 16) hipLaunchKernelGGL((ob_dense_skinny_kernel<E, EPI, 1, ROWS>), grid, dim3(256), 0, s, a);
         else if (a.T <= 32) hipLaunchKernelGGL((ob_dense_skinny_kernel<E, EPI, 2, ROWS>), grid, dim3(256), 0, s, a);
         else hipLaunchKernelGGL((ob_dense_skinny_kernel<E, EPI, 4, ROWS>), grid, dim3(256), 0, s, a);
         return hstatus("expert product");
