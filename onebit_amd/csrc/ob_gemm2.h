@@ -262,19 +262,23 @@ __device__ __forceinline__ int ob_g3_bid()
     return (xcd < rem ? xcd * (q8 + 1) : rem * (q8 + 1) + (xcd - rem) * q8) + (orig >> 3);
 }
 
-template <bool PARTIAL, int WT>
+#undef RT
+// RT = 16-token tiles of a wave: 8, or 7 / 6 where that leaves less of the last round of workgroups empty (ob_gemm3_rt); the staging stays that of 8,
+// rows beyond the tile are fetched and not multiplied.
+template <bool PARTIAL, int WT, int RT>
 __device__ __forceinline__ void ob_gemm3_body(
     const uint32_t *__restrict__ W, int64_t ldw_words, const _Float16 *__restrict__ a, int64_t lda,
     const _Float16 *__restrict__ g, _Float16 *__restrict__ u, float *__restrict__ zp, int T, int K, int N, int nbn, const int bid)
 {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    constexpr int TTILE = 128 * WT;              // tokens per workgroup tile
+    static_assert(RT == 8 || WT == 1, "narrow tiles: the 4-wave form");
+    constexpr int TTILE = 128 * WT;              // token rows staged per workgroup
     _Float16 (*As)[TTILE][OB_G2_PITCH] = reinterpret_cast<_Float16 (*)[TTILE][OB_G2_PITCH]>(smem);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wn = wave & 3, wt = wave >> 2;
     const int r = lane & 15, gq = lane >> 4;
     const int tt = bid / nbn, tn = bid - tt * nbn;
-    const int n0 = tn * OB_G2_N, t0 = tt * TTILE;
+    const int n0 = tn * OB_G2_N, t0 = tt * 16 * RT * WT;
     const int nk = K / OB_G2_K;                 // K % 256 == 0 here (host-checked): whole quads of steps
 
     // DMA source of this lane for each of the wave's 4 instructions per tile, as a 32-bit BYTE offset from
@@ -493,7 +497,7 @@ __device__ __forceinline__ void ob_gemm3_body(
         const int64_t ntile64 = N >> 6;
         const int tile_idx = (n0 + wn * 64) >> 6;
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
+        for (int j = 0; j < 2 * RT; ++j) {
             const int row = j * 8 + (lane >> 3), ch = lane & 7;
             const ob_half8 v = *reinterpret_cast<const ob_half8 *>(ep + row * EP + ch * 16);
             if (row < trows) *reinterpret_cast<ob_half8 *>(ub + (int64_t)row * N + ch * 8) = v;
@@ -552,12 +556,12 @@ __device__ __forceinline__ void ob_gemm3_body(
     }
 }
 
-template <bool PARTIAL, int WT = 2>
+template <bool PARTIAL, int WT = 2, int RT = 8>
 __global__ __launch_bounds__(256 * WT, 2) void ob_gemm3_f16_kernel(
     const uint32_t *__restrict__ W, int64_t ldw_words, const _Float16 *__restrict__ a, int64_t lda,
     const _Float16 *__restrict__ g, _Float16 *__restrict__ u, float *__restrict__ zp, int T, int K, int N, int nbn)
 {
-    ob_gemm3_body<PARTIAL, WT>(W, ldw_words, a, lda, g, u, zp, T, K, N, nbn, ob_g3_bid());
+    ob_gemm3_body<PARTIAL, WT, RT>(W, ldw_words, a, lda, g, u, zp, T, K, N, nbn, ob_g3_bid());
 }
 
 // GROUPED form (round 6): up to three projections that share T, K and the row pitches -- q | k | v or gate | up of a decoder layer on the
@@ -570,7 +574,7 @@ struct ObG3Group {
     long long ldw_words, lda;
     int T, K;
 };
-template <int WT>
+template <int WT, int RT = 8>
 __global__ __launch_bounds__(256 * WT, 2) void ob_gemm3g_f16_kernel(const ObG3Group G)
 {
     const int bid = ob_g3_bid();
@@ -582,7 +586,7 @@ __global__ __launch_bounds__(256 * WT, 2) void ob_gemm3g_f16_kernel(const ObG3Gr
     _Float16 *u = p == 0 ? G.u[0] : (p == 1 ? G.u[1] : G.u[2]);
     const int N = p == 0 ? G.N[0] : (p == 1 ? G.N[1] : G.N[2]);
     const int nbn = p == 0 ? G.nbn[0] : (p == 1 ? G.nbn[1] : G.nbn[2]);
-    ob_gemm3_body<false, WT>(W, G.ldw_words, a, G.lda, g, u, nullptr, G.T, G.K, N, nbn, bid - b0);
+    ob_gemm3_body<false, WT, RT>(W, G.ldw_words, a, G.lda, g, u, nullptr, G.T, G.K, N, nbn, bid - b0);
 }
 
 // K-SLICED form (round 6): ONE projection whose 256 x 128 tiles alone leave most of the chip idle (hidden-width outputs at a few hundred
@@ -596,7 +600,7 @@ struct ObG3Slices {
     long long ldw_words, lda;
     int T, N, nbn, tiles, ns, quads;
 };
-template <int WT>
+template <int WT, int RT = 8>
 __global__ __launch_bounds__(256 * WT, 2) void ob_gemm3ks_f16_kernel(const ObG3Slices G)
 {
     const int bid = ob_g3_bid();
@@ -604,8 +608,7 @@ __global__ __launch_bounds__(256 * WT, 2) void ob_gemm3ks_f16_kernel(const ObG3S
     const int qb = G.quads / G.ns, qr = G.quads - qb * G.ns;
     const int q0 = j * qb + min(j, qr), nq = qb + (j < qr ? 1 : 0);
     float *zp = j == 0 ? G.z[0] : (j == 1 ? G.z[1] : (j == 2 ? G.z[2] : G.z[3]));
-    ob_gemm3_body<true, WT>(G.W + q0 * (4 * OB_G2_K / 32), G.ldw_words, G.a + q0 * (4 * OB_G2_K), G.lda, nullptr, nullptr, zp, G.T,
+    ob_gemm3_body<true, WT, RT>(G.W + q0 * (4 * OB_G2_K / 32), G.ldw_words, G.a + q0 * (4 * OB_G2_K), G.lda, nullptr, nullptr, zp, G.T,
                             nq * (4 * OB_G2_K), G.N, G.nbn, bid - j * G.tiles);
 }
 #undef RN
-#undef RT

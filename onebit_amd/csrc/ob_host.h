@@ -78,6 +78,8 @@ OB_HIDDEN bool ob_gemm3_group_ok(const onebit_proj_t *const *ps, int np, int64_t
 // 256 x 128 tiles of that launch (sum over the members) and the workgroup slots of one round (two workgroups per CU)
 OB_HIDDEN int64_t ob_gemm3_group_tiles(const onebit_proj_t *const *ps, int np, int64_t T);
 OB_HIDDEN int ob_gemm3_slots();
+// what a launch over `nb` 256-row blocks and T tokens costs with the tile it takes, in 1 / 8.4 of a full round of 128-token tiles (105 us at K = 4096)
+OB_HIDDEN double ob_gemm3_cost(int64_t nb, int64_t T);
 // ONE projection on its pre-scaled rows a [T, K] as two to four K-slices in one launch of the LDS-DMA GEMM (fp32 sums z[i] [T, N], added and
 // scaled by the consuming row kernel): a hidden-width projection at a few hundred rows has too few 256 x 128 tiles for the chip (13B, 543 rows:
 // 100), its slices have that many times more.  ob_gemm3_ksplit_n: 0 when the projection alone is eligible for the LDS-DMA GEMM or no

@@ -317,6 +317,25 @@ static bool ob_gemm3_ok(int64_t T, int64_t K, int64_t N)
     return 3 * tiles >= 2 * (int64_t)ob_cu_count() || env == 2;
 }
 
+// 16-token tiles per workgroup of the 4-wave form (8 = 128 tokens, 7, 6) for `nb` 256-row blocks (times K slices): rounds of two workgroups per CU
+// times the tile's size, a round of at most one per CU taking 0.55 of one of two (473 / 559 tiles of 4096 -> 11008: 107 / 153 us).  1540 rows: 12 x 86
+// tiles of 128 tokens for gate | up are 2.02 rounds, 16 x 86 of 96 are 2.69 three-quarter ones; 192 tiles of a hidden-width projection leave a quarter
+// of the CUs idle, 256 of 96 tokens none.
+static double ob_gemm3_tiles_cost(int64_t nb, int64_t T, int rt)
+{
+    const int64_t cus = ob_cu_count(), slots = 2 * cus, t = nb * ((T + 16 * rt - 1) / (16 * rt)), rem = t % slots;
+    return ((double)(t / slots) + (rem == 0 ? 0.0 : rem <= cus ? 0.55 : 1.0)) * (rt + 0.4);
+}
+static int ob_gemm3_rt(int64_t nb, int64_t T)
+{
+    static const int env = getenv("OB_GEMM3_RT") ? atoi(getenv("OB_GEMM3_RT")) : 0;        // A/B: 6, 7, 8
+    if (env >= 6 && env <= 8) return env;
+    int best = 8;
+    for (int rt = 7; rt >= 6; --rt) if (ob_gemm3_tiles_cost(nb, T, rt) < 0.97 * ob_gemm3_tiles_cost(nb, T, best)) best = rt;
+    return best;
+}
+double ob_gemm3_cost(int64_t nb, int64_t T) { return ob_gemm3_tiles_cost(nb, T, ob_gemm3_rt(nb, T)); }
+
 // The LDS-DMA GEMM in its 8-wave (256 x 256 tile, one workgroup per CU) or 4-wave (256 rows x 128 tokens, two workgroups per
 // CU) form; OB_GEMM3_WT=1 / 2 selects (A/B), default below.
 #ifndef OB_GEMM4_DEFAULT
@@ -336,11 +355,16 @@ static void ob_launch_gemm3(const uint32_t *W, int64_t ldw_words, const _Float16
         hipLaunchKernelGGL((ob_gemm4_f16_kernel<PARTIAL>), dim3((unsigned)(nbn * nbt)), dim3(256), OB_G4_LDS, s,
                            W, ldw_words, a, lda, g, u, zp, (int)T, (int)K, (int)N, nbn);
     } else if (wt_env == 1) {
-        static bool attr_set[OB_MAX_DEVICES] = {};
-        ob_set_max_lds_once(ob_gemm3_f16_kernel<PARTIAL, 1>, attr_set, OB_G3_LDS_W(1));
-        const int nbt = (int)((T + 127) / 128);
-        hipLaunchKernelGGL((ob_gemm3_f16_kernel<PARTIAL, 1>), dim3((unsigned)(nbn * nbt)), dim3(256), OB_G3_LDS_W(1), s,
-                           W, ldw_words, a, lda, g, u, zp, (int)T, (int)K, (int)N, nbn);
+        const int rt = ob_gemm3_rt(nbn, T);
+        const auto go = [&](auto kern, bool (&attr_set)[OB_MAX_DEVICES]) {
+            ob_set_max_lds_once(kern, attr_set, OB_G3_LDS_W(1));
+            hipLaunchKernelGGL(kern, dim3((unsigned)(nbn * ((T + 16 * rt - 1) / (16 * rt)))), dim3(256), OB_G3_LDS_W(1), s,
+                               W, ldw_words, a, lda, g, u, zp, (int)T, (int)K, (int)N, nbn);
+        };
+        static bool attr_set[3][OB_MAX_DEVICES] = {};
+        if (rt == 6) go(ob_gemm3_f16_kernel<PARTIAL, 1, 6>, attr_set[0]);
+        else if (rt == 7) go(ob_gemm3_f16_kernel<PARTIAL, 1, 7>, attr_set[1]);
+        else go(ob_gemm3_f16_kernel<PARTIAL, 1>, attr_set[2]);
     } else {
         static bool attr_set[OB_MAX_DEVICES] = {};
         ob_set_max_lds_once(ob_gemm3_f16_kernel<PARTIAL, 2>, attr_set, OB_G3_LDS);
@@ -1684,9 +1708,17 @@ int ob_gemm3_grouped(const onebit_proj_t *const *ps, void *const *us, const void
         hipLaunchKernelGGL(ob_gemm4g_f16_kernel, dim3((unsigned)tiles), dim3(256), OB_G4_LDS, s, G);
         return ob_launch_status("gemm4_grouped");
     }
-    static bool attr_set[OB_MAX_DEVICES] = {};
-    ob_set_max_lds_once(ob_gemm3g_f16_kernel<1>, attr_set, OB_G3_LDS_W(1));
-    hipLaunchKernelGGL((ob_gemm3g_f16_kernel<1>), dim3((unsigned)tiles), dim3(256), OB_G3_LDS_W(1), s, G);
+    const int64_t nb = tiles / nbt;
+    const int rt = ob_gemm3_rt(nb, T);
+    for (int i = 0; i < 3; ++i) G.tile_end[i] = (int)(G.tile_end[i] / nbt * ((T + 16 * rt - 1) / (16 * rt)));
+    const auto go = [&](auto kern, bool (&attr_set)[OB_MAX_DEVICES]) {
+        ob_set_max_lds_once(kern, attr_set, OB_G3_LDS_W(1));
+        hipLaunchKernelGGL(kern, dim3((unsigned)G.tile_end[2]), dim3(256), OB_G3_LDS_W(1), s, G);
+    };
+    static bool attr_set[3][OB_MAX_DEVICES] = {};
+    if (rt == 6) go(ob_gemm3g_f16_kernel<1, 6>, attr_set[0]);
+    else if (rt == 7) go(ob_gemm3g_f16_kernel<1, 7>, attr_set[1]);
+    else go(ob_gemm3g_f16_kernel<1>, attr_set[2]);
     return ob_launch_status("gemm3_grouped");
 }
 
@@ -1719,10 +1751,17 @@ int ob_gemm3_ksplit(const onebit_proj_t &p, const void *a, float *const *z, int 
         if (!G.z[i] || !ob_aligned(G.z[i], 16)) return ob_fail(ONEBIT_E_ALIGN, "gemm3_ksplit: partial sums must be 16-byte aligned");
     }
     G.W = (const uint32_t *)p.weight; G.a = (const _Float16 *)a; G.ldw_words = p.ldw_bytes / 4; G.lda = p.K; G.T = (int)T; G.N = (int)p.N;
-    G.nbn = (int)((p.N + OB_G2_N - 1) / OB_G2_N); G.tiles = G.nbn * (int)((T + 127) / 128); G.ns = ns; G.quads = (int)(p.K / (4 * OB_G2_K));
-    static bool attr_set[OB_MAX_DEVICES] = {};
-    ob_set_max_lds_once(ob_gemm3ks_f16_kernel<1>, attr_set, OB_G3_LDS_W(1));
-    hipLaunchKernelGGL((ob_gemm3ks_f16_kernel<1>), dim3((unsigned)(ns * G.tiles)), dim3(256), OB_G3_LDS_W(1), s, G);
+    G.nbn = (int)((p.N + OB_G2_N - 1) / OB_G2_N); G.ns = ns; G.quads = (int)(p.K / (4 * OB_G2_K));
+    const int rt = ob_gemm3_rt((int64_t)G.nbn * ns, T);
+    G.tiles = G.nbn * (int)((T + 16 * rt - 1) / (16 * rt));
+    const auto go = [&](auto kern, bool (&attr_set)[OB_MAX_DEVICES]) {
+        ob_set_max_lds_once(kern, attr_set, OB_G3_LDS_W(1));
+        hipLaunchKernelGGL(kern, dim3((unsigned)(ns * G.tiles)), dim3(256), OB_G3_LDS_W(1), s, G);
+    };
+    static bool attr_set[3][OB_MAX_DEVICES] = {};
+    if (rt == 6) go(ob_gemm3ks_f16_kernel<1, 6>, attr_set[0]);
+    else if (rt == 7) go(ob_gemm3ks_f16_kernel<1, 7>, attr_set[1]);
+    else go(ob_gemm3ks_f16_kernel<1>, attr_set[2]);
     return ob_launch_status("gemm3_ksplit");
 }
 

@@ -315,7 +315,9 @@ extern "C" int onebit_mixed_step(const onebit_model_t *m, const onebit_mixed_sta
             if (tail_env > 0 && tail >= 2 && tail <= tail_env && Tm >= 192 && ob_gemm3_group_ok(ps, np, Tm)) {
                 const int64_t slots = ob_gemm3_slots();
                 const int64_t r_all = (ob_gemm3_group_tiles(ps, np, T) + slots - 1) / slots, r_main = (ob_gemm3_group_tiles(ps, np, Tm) + slots - 1) / slots;
-                bool sk_ok = r_main < r_all;
+                // (a pass of the skinny GEMM: 30 us next to a round's 105 at K = 4096, 2.4 in ob_gemm3_cost's unit)
+                const int64_t nb = ob_gemm3_group_tiles(ps, np, T) / nbt;
+                bool sk_ok = r_main < r_all && ob_gemm3_cost(nb, Tm) + 2.4 * ((tail + 63) / 64) < ob_gemm3_cost(nb, T);
                 for (int i = 0; sk_ok && i < np; ++i) sk_ok = ob_sk3_proj_ok(*ps[i]);
                 if (sk_ok && ob_gemm3_grouped(ps, us, av, np, Tm, s) == 0) {
                     const int nblk = (tail + 63) / 64, rows = (tail + nblk - 1) / nblk;

@@ -1,0 +1,59 @@
+"""The 1-bit LDS-DMA products at row counts around every tile they choose from (96, 112, 128 tokens): unsliced, K-sliced and grouped launches.
+
+Bound: u = fp16(fp16(z) g): two roundings of 2^-11, and the float32 sum of z behind them: K / 32 additions, 2^-24 sqrt(K) |a|_2 with a factor 4."""
+import ctypes
+
+import pytest
+import torch
+from torch import nn
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _layer(K, N, g):
+    from onebit_amd import BitLinearInf
+    m = BitLinearInf(K, N, device=DEV, dtype=torch.float16)
+    m.weight.data = torch.randint(0, 256, (N, K // 8), generator=g, device=DEV, dtype=torch.uint8).view(torch.int8)
+    m.input_factor.data = (0.05 + 0.1 * torch.rand(K, generator=g, device=DEV)).half()
+    m.weight_scale.data = (0.05 + 0.1 * torch.rand(N, generator=g, device=DEV)).half()
+    return m
+
+
+def _check(m, a, u):
+    s = 1.0 - 2.0 * ((m.weight.view(torch.uint8)[:, :, None] >> torch.arange(8, device=DEV, dtype=torch.uint8)) & 1).reshape(m.out_features, -1).double()
+    ref = (a.double() @ s.T) * m.weight_scale.double()
+    bound = 1.1 * 2.0 ** -10 * ref.abs() + 4 * 2.0 ** -24 * a.shape[1] ** 0.5 * a.double().norm(dim=1, keepdim=True) * m.weight_scale.double() + 2.0 ** -24
+    assert ((u.double() - ref).abs() <= bound).all(), float(((u.double() - ref).abs() / bound).max())
+
+
+@pytest.mark.parametrize("K,N", [(4096, 4096), (2048, 11008), (1024, 4100)])
+@pytest.mark.parametrize("T", [97, 130, 192, 193, 224, 225, 337, 389, 449, 575, 577, 673, 701, 897, 1153, 1300, 1537, 1540, 2100])
+def test_one_projection(T, K, N):
+    g = torch.Generator(device=DEV).manual_seed(T + K)
+    m = _layer(K, N, g)
+    m.layernorm = nn.Identity()
+    x = torch.randn(T, K, generator=g, device=DEV).half()
+    _check(m, x * m.input_factor, m(x))
+
+
+@pytest.mark.parametrize("Ns", [(4096, 4096, 4096), (11008, 11008), (5120, 1028, 260)])
+@pytest.mark.parametrize("T", [192, 577, 673, 897, 1025, 1153, 1540])
+def test_grouped_projections(T, Ns):
+    from onebit_amd import _lib
+    from onebit_amd.bitnet import _stream_ptr
+    from onebit_amd.engine import _Proj, _proj
+    K, lib = 1024, _lib.load()
+    g = torch.Generator(device=DEV).manual_seed(T)
+    ms = [_layer(K, N, g) for N in Ns]
+    xs = [torch.randn(T, K, generator=g, device=DEV).half() for _ in ms]
+    us = [torch.full((T + 1, N), 7.0, dtype=torch.float16, device=DEV) for N in Ns]
+    arr = (_Proj * len(ms))(*[_proj(m) for m in ms])
+    up, ap = ((ctypes.c_void_p * 3)(*[t.data_ptr() for t in ts]) for ts in (us, xs))
+    rc = lib.onebit_linear_group_prescaled(ctypes.cast(arr, ctypes.c_void_p), up, ap, len(ms), T, _stream_ptr(xs[0].device))
+    if rc == -2:
+        pytest.skip("too few tiles for one launch")
+    assert rc == 0
+    for m, x, u in zip(ms, xs, us):
+        _check(m, x, u[:T])
+        assert (u[T] == 7.0).all()                 # nothing behind the last row
