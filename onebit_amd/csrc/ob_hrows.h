@@ -92,6 +92,52 @@ __global__ __launch_bounds__(1024) void ob_hnorm_kernel(const ObHNormArgs A)
     }
 }
 
+// ... of many rows: four rows a workgroup, four waves each (1024 NV columns, W % 4 == 0, no embedding row), the row in registers.  The four rows' pieces
+// of the fragment-major output lie next to each other and leave as whole sectors from one L2 (ob_gated_norm_rows_kernel):
+// 6100 rows of 2048 columns 46 -> 42 us.
+template <typename E, int NV>
+__global__ __launch_bounds__(1024) void ob_hnorm_rows_kernel(const ObHNormArgs A, int n_rows)
+{
+    __shared__ float red[16];
+    const int tid = threadIdx.x & 255, q = threadIdx.x >> 8, t = min((int)blockIdx.x * 4 + q, n_rows - 1);
+    const bool live = (int)blockIdx.x * 4 + q < n_rows;                // (a row beyond the last: read again, not written)
+    const int src = A.rows ? A.rows[t] : t;
+    float *xr = A.x + (size_t)src * A.W;
+    ob_float4 r[NV];
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const int c = (i * 256 + tid) * 4;
+        if (c < A.W) {
+            r[i] = *reinterpret_cast<const ob_float4 *>(xr + c);
+            float s[4] = {0.f, 0.f, 0.f, 0.f};
+            ob_sum_splits<4>(s, A.z + (size_t)src * A.ldz + c, A.z_split, A.n_split);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) r[i][e] += A.mult * (A.bias ? s[e] + A.bias[c + e] : s[e]);
+            if (A.emb_add) r[i] += *reinterpret_cast<const ob_float4 *>(A.emb_add + (size_t)src * A.W + c);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) ss = __builtin_fmaf(r[i][e], r[i][e], ss);
+        }
+    }
+    ss = ob_wave_sum(ss);
+    if ((tid & 63) == 0) red[threadIdx.x >> 6] = ss;
+    __syncthreads();                                                   // (every read of the residual row is done)
+    const float *rq = red + 4 * q;
+    const float rs = 1.0f / sqrtf(((rq[0] + rq[1]) + (rq[2] + rq[3])) / (float)A.W + A.eps);
+    if (!live) return;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const int c = (i * 256 + tid) * 4;
+        if (c >= A.W) break;
+        if (!A.rows) *reinterpret_cast<ob_float4 *>(xr + c) = r[i];
+        const ob_float4 w = *reinterpret_cast<const ob_float4 *>(A.w + c);
+        ob_float4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = r[i][e] * rs * (A.off + w[e]);
+        *reinterpret_cast<typename ObElem<E>::V4 *>((E *)A.out + ob_frag<E>(t, c, A.out_nkt)) = ob_to_v4<E>(v);
+    }
+}
+
 // The same row with everything a sequential layer adds to it:
 //   s = sum of the splits (+ bias) + sum_k tok_w[k] ez[tok_row[k]] (experts; eo: their outputs in the work type) + id_w h (identity experts; h = idh or the residual itself)
 //   r = x + mult * (post_w ? s / sqrt(mean s^2 + eps) * post_w : s) (+ emb_add)
@@ -313,6 +359,46 @@ __global__ __launch_bounds__(256) void ob_gated_norm_kernel(const ObGatedNormArg
         for (int e = 0; e < VEC; ++e) v[e] = (E)(sm[c + e] * rs * A.w[c0 + c + e]);
         if constexpr (VEC > 1) *reinterpret_cast<V16 *>(out + ob_frag<E>(t, c0 + c, A.out_nkt)) = v;       // (16 bytes of a row are contiguous)
         else out[ob_frag<E>(t, c0 + c, A.out_nkt)] = v[0];
+    }
+}
+
+// ... of many rows: a wave per row, four rows a workgroup.  A row's 16-byte pieces of the fragment-major output then leave as whole 64-byte sectors (four
+// rows of a tile lie next to each other) from one L2: 6100 rows of 4096 columns 62 us one row a workgroup,
+// partial sectors from four XCDs -> 48.
+// The row stays in registers (NV 16-byte pieces per lane); groups of up to 512 NV columns, whole pieces.
+template <typename E, int NV>
+__global__ __launch_bounds__(256) void ob_gated_norm_rows_kernel(const ObGatedNormArgs A, int rows)
+{
+    typedef typename ObElem<E>::V16 V16;
+    constexpr int VEC = ObElem<E>::EPL;
+    const int lane = threadIdx.x & 63, t = blockIdx.y * 4 + (threadIdx.x >> 6), c0 = blockIdx.x * A.gsize;
+    if (t >= rows) return;
+    const E *y = (const E *)A.y + (size_t)t * A.ldy + c0, *z = (const E *)A.gate + (size_t)t * A.ldg + c0;
+    V16 yv[NV], zv[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const int c = (i * 64 + lane) * VEC;
+        if (c < A.gsize) { yv[i] = *reinterpret_cast<const V16 *>(y + c); zv[i] = *reinterpret_cast<const V16 *>(z + c); }
+    }
+    float v[NV][VEC], ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+        if ((i * 64 + lane) * VEC < A.gsize) {
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) {
+                v[i][e] = (float)yv[i][e] * ob_silu<E>((float)zv[i][e]);
+                ss = __builtin_fmaf(v[i][e], v[i][e], ss);
+            }
+        }
+    const float rs = 1.0f / sqrtf(ob_wave_sum(ss) / (float)A.gsize + A.eps);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const int c = (i * 64 + lane) * VEC;
+        if (c >= A.gsize) break;
+        V16 o;
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) o[e] = (E)(v[i][e] * rs * A.w[c0 + c + e]);
+        *reinterpret_cast<V16 *>((E *)A.out + ob_frag<E>(t, c0 + c, A.out_nkt)) = o;
     }
 }
 

@@ -344,6 +344,7 @@ extern "C" size_t onebit_hybrid_workspace_bytes(const onebit_hmodel_t *m, int64_
 }
 
 // ---------------------------------------------------------------------------------------------------------------- step --
+#define OB_MANY_ROWS 1024       // rows from which a row kernel's workgroup takes four (the chip stays full)
 // the row kernel between two products; the wider form only where a layer needs it
 template <typename E>
 static int row_launch(const ObXRowArgs &a, int rows, hipStream_t s)
@@ -364,6 +365,13 @@ static int row_launch(const ObXRowArgs &a, int rows, hipStream_t s)
 #undef OB_XROW
     }
     const ObHNormArgs &n = a;
+    if (rows >= OB_MANY_ROWS && !a.embed && !a.emb_save && a.W % 4 == 0 && a.W <= 4096) {
+        const auto four = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3((unsigned)cdiv(rows, 4)), dim3(1024), 0, s, n, rows);
+            return hstatus("row kernel");
+        };
+        return a.W <= 1024 ? four(ob_hnorm_rows_kernel<E, 1>) : a.W <= 2048 ? four(ob_hnorm_rows_kernel<E, 2>) : four(ob_hnorm_rows_kernel<E, 4>);
+    }
     return a.W % 4 == 0 ? go(ob_hnorm_kernel<E, 4>, n) : go(ob_hnorm_kernel<E, 1>, n);
 }
 
@@ -500,7 +508,13 @@ static int ssm_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, const 
         n.out = (char *)act + (size_t)(r0 / 16) * act_nkt * 1024;
         const dim3 grid((unsigned)L.norm_groups, (unsigned)std::min(st.n_rows - r0, 32768));
         const unsigned thr = (unsigned)std::min<int64_t>(256, std::max<int64_t>(64, rup(cdiv(n.gsize, VEC), 64)));
-        if (n.gsize % VEC == 0) hipLaunchKernelGGL(k4, grid, dim3(thr), lds, s, n);
+        const int pieces = (int)cdiv(n.gsize, 64 * VEC);
+        if (st.n_rows >= OB_MANY_ROWS && n.gsize % VEC == 0 && pieces <= 8) {
+            const dim3 wgrid(grid.x, (unsigned)cdiv(grid.y, 4));
+            if (pieces <= 1) hipLaunchKernelGGL((ob_gated_norm_rows_kernel<E, 1>), wgrid, dim3(256), 0, s, n, (int)grid.y);
+            else if (pieces <= 4) hipLaunchKernelGGL((ob_gated_norm_rows_kernel<E, 4>), wgrid, dim3(256), 0, s, n, (int)grid.y);
+            else hipLaunchKernelGGL((ob_gated_norm_rows_kernel<E, 8>), wgrid, dim3(256), 0, s, n, (int)grid.y);
+        } else if (n.gsize % VEC == 0) hipLaunchKernelGGL(k4, grid, dim3(thr), lds, s, n);
         else hipLaunchKernelGGL(k1, grid, dim3(256), lds, s, n);
     }
     return hstatus("gated norm");
