@@ -43,6 +43,7 @@
 // this kernel with the two query tiles of a wave taken in turn, one tile's exponentials interleaved with the other's MFMAs
 // (577; ob_flash_split_experiment.h).
 #pragma once
+#include <algorithm>
 #include <type_traits>
 #include "ob_common.h"
 
@@ -62,13 +63,15 @@ struct ObFlashArgs {
 // RAGGED form (round 6, the mixed prefill + decode step of continuous batching): the queries are the token rows of SEVERAL
 // sequences, concatenated; segment i = rows [row0, row0 + n) of the request in KV-cache slot `slot`, first new token at position
 // `past` (its keys 0 .. past + n - 1 are in the cache).  The segment table travels in the kernel arguments (<= 64 segments per
-// launch: no device-side table to upload, graph-capture safe); wg_end[i] = workgroups of segments 0 .. i (n_heads * ceil(query
-// blocks / 2) each).  Everything else is the kernel above with (b, S, past) read per segment.
+// launch: no device-side table to upload, graph-capture safe); wg_end[i] = workgroups of segments 0 .. i (n_heads * query
+// blocks each, or half as many pairs of blocks: ob_fl_number).  Everything else is the kernel above with (b, S, past) read per segment.
 #define OB_FL_MAXSEG 64
 struct ObFlashSeg { int row0, n, slot, past; };
 struct ObFlashRaggedArgs {
     ObFlashArgs a;            // q / o [rows, H, D]; k / v [slots][Hkv][max_len][D]; S, past, nmb unused
     int nseg;
+    int hg;                   // 0: pairs of query blocks; else single blocks, numbered over groups of hg heads (set by ob_fl_number)
+    int snake;                // single blocks, all resident at once: the lighter half comes lightest first
     int wg_end[OB_FL_MAXSEG];
     ObFlashSeg seg[OB_FL_MAXSEG];
 };
@@ -112,6 +115,37 @@ struct ObFlSoftmaxBf16 : ObFlSigmoidBf16 {
 #define OB_FL_BM 128
 #define OB_FL_BN 64
 #define OB_FL_THREADS 256
+#define OB_FL_SLOTS 512         // resident workgroups of the chip: two to each of 256 CUs
+
+// Workgroups of a ragged launch: sets wg_end, hg and snake from the segments' row counts; 0 = too many.
+// Pairs of query blocks are the same work each, but a workgroup is as long as two blocks: where the pairs do not take every slot, some CUs
+// run one workgroup (4 waves, the latencies of a block's barriers bare) while others run two, or all run one.  Then the blocks go one by
+// one, heaviest first over the heads that one XCD's share of the launch covers (their keys and values stay in its L2); if all are resident
+// at once nothing is dealt later, and the lighter half comes lightest first, so that a heavy and a light block share a CU.  Measured, pairs
+// -> single blocks: 4 x 500 rows x 32 heads of width 128 (256 pairs, 512 blocks) 33.7 -> 27.3 us; a bf16 launch of 384 pairs 124.6 -> 120.0 us
+// with sigmoid weights, 100.0 -> 98.4 us with softmax ones.  From OB_FL_SLOTS pairs on they fill the chip.
+inline int64_t ob_fl_number(ObFlashRaggedArgs &f)
+{
+    const int H = f.a.H;
+    int64_t pairs = 0, single = 0;
+    for (int i = 0; i < f.nseg; ++i) {
+        const int64_t nmb = ((int64_t)f.seg[i].n + OB_FL_BM - 1) / OB_FL_BM;
+        pairs += (nmb + 1) / 2 * H;
+        single += nmb * H;
+        if (pairs > 0x3fffffffLL) return 0;
+    }
+    const bool one = pairs < OB_FL_SLOTS;
+    f.hg = 0;
+    f.snake = one && single <= OB_FL_SLOTS;
+    if (one) for (f.hg = (int)std::min<int64_t>(H, std::max<int64_t>(1, (int64_t)H * f.nseg / 8)); H % f.hg; --f.hg) ;
+    int64_t end = 0;
+    for (int i = 0; i < f.nseg; ++i) {
+        const int64_t nmb = ((int64_t)f.seg[i].n + OB_FL_BM - 1) / OB_FL_BM;
+        f.wg_end[i] = (int)(end += (one ? nmb : (nmb + 1) / 2) * H);
+    }
+    return end;
+}
+
 #ifdef OB_FL_TRACE
 #define OB_FL_T(i) do { if (tr) tr[(pass * 32 + kb) * 8 + (i)] = __builtin_amdgcn_s_memtime(); } while (0)
 #define OB_FL_TP(i) do { if (tr) tr[(64 + pass) * 8 + (i)] = __builtin_amdgcn_s_memtime(); } while (0)
@@ -189,7 +223,13 @@ __global__ __launch_bounds__(256, 2) void ob_flash_fwd_kernel(const std::conditi
         nmb = (S + OB_FL_BM - 1) / OB_FL_BM;
         npair = (nmb + 1) >> 1;
         const int loc = bid - wg0;
-        pj = loc % npair; head = loc / npair;
+        if (AA.hg) {
+            const int per = nmb * AA.hg, grp = loc / per, r = loc - grp * per;
+            pj = r / AA.hg; head = grp * AA.hg + r - pj * AA.hg;
+            if (AA.snake && pj >= npair) pj = nmb - 1 - (pj - npair);
+        } else {
+            pj = loc % npair; head = loc / npair;
+        }
     } else {
         S = A.S; past = A.past; nmb = A.nmb;
         npair = (nmb + 1) >> 1;
@@ -220,6 +260,7 @@ __global__ __launch_bounds__(256, 2) void ob_flash_fwd_kernel(const std::conditi
     OB_FL_TP(0);
     const int mb = pass == 0 ? nmb - 1 - pj : pj;
     if (pass == 1 && mb == nmb - 1 - pj) break;                 // odd count: the middle block has no partner
+    if constexpr (RAGGED) { if (pass == 1 && AA.hg) break; }    // the workgroup has a single block
     const int m0 = mb * OB_FL_BM;
     // Q^T fragments of the wave's two query tiles: lane (query = lr, d = 32 ds + 8 g .. + 7)
     V8 qf[2][DK];

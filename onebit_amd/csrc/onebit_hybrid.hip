@@ -426,15 +426,12 @@ static int attention_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, 
         a.a.scale_log2e = -L.scale * OB_LOG2E;
         a.r1 = L.r1; a.r2 = L.r2; a.pb = L.pb; a.out = act; a.out_nkt = act_nkt; a.vdim = L.vdim;
         a.nseg = ns;
-        int64_t wgs = 0;
         for (int i = 0; i < ns; ++i) {
             const onebit_hseg_t &g = st.segs[s0 + i];
-            const int64_t nmb = cdiv(g.n, OB_FL_BM);
-            wgs += (nmb + 1) / 2 * L.heads;
-            if (wgs > 0x3fffffffLL) return hfail(ONEBIT_E_ARG, "attention: too many workgroups");
-            a.wg_end[i] = (int)wgs;
             a.seg[i] = {g.row0, g.n, g.slot, g.past};
         }
+        const int64_t wgs = ob_fl_number(a);
+        if (!wgs) return hfail(ONEBIT_E_ARG, "attention: too many workgroups");
         if (L.kp == 128) hipLaunchKernelGGL((ob_flash_fwd_kernel<128, true, ObFlSigmoidBf16>), dim3((unsigned)wgs), dim3(256), 0, s, a);
         else hipLaunchKernelGGL((ob_flash_fwd_kernel<64, true, ObFlSigmoidBf16>), dim3((unsigned)wgs), dim3(256), 0, s, a);
     }
@@ -626,7 +623,7 @@ static int latent_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, con
         for (int s0 = first; s0 < st.n_seg;) {
             ObDenseSegArgs e = {};
             ObFlashSigArgs f = {};
-            int64_t rows = 0, wgs = 0;
+            int64_t rows = 0;
             int blocks = 0, i = s0;
             for (; i < st.n_seg && e.nseg < OB_DENSE_MAXSEG; ++i) {
                 const onebit_hseg_t &g = st.segs[i];
@@ -634,9 +631,6 @@ static int latent_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, con
                 if (rows + rup(len, 16) > P.kv_rows) break;
                 blocks += (int)cdiv(len, 128);
                 e.blk_end[n] = blocks; e.band0[n] = g.slot * bands; e.row0[n] = (int)rows; e.rows[n] = len;
-                wgs += (cdiv(g.n, OB_FL_BM) + 1) / 2 * H;
-                if (wgs > 0x3fffffffLL) return hfail(ONEBIT_E_ARG, "attention: too many workgroups");
-                f.wg_end[n] = (int)wgs;
                 f.seg[n] = {g.row0, g.n, (int)rows, g.past};
                 f.nseg = ++e.nseg;
                 rows += rup(len, 16);
@@ -649,6 +643,8 @@ static int latent_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, con
             f.a.H = f.a.Hkv = H; f.a.max_len = (int)P.kv_rows;
             f.a.scale_log2e = L.scale * OB_LOG2E;
             f.out = act; f.out_nkt = act_nkt; f.vdim = l.vdp;
+            const int64_t wgs = ob_fl_number(f);
+            if (!wgs) return hfail(ONEBIT_E_ARG, "attention: too many workgroups");
             if (L.kp == 128) hipLaunchKernelGGL((ob_flash_fwd_kernel<128, true, ObFlSoftmaxBf16>), dim3((unsigned)wgs), dim3(256), 0, s, f);
             else hipLaunchKernelGGL((ob_flash_fwd_kernel<64, true, ObFlSoftmaxBf16>), dim3((unsigned)wgs), dim3(256), 0, s, f);
             if (int rc2 = hstatus("prompt attention")) return rc2;

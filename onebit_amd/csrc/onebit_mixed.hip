@@ -53,15 +53,12 @@ extern "C" int onebit_attention_ragged(const void *q, const void *k_cache, const
         a.a.h_next = (const _Float16 *)h_next; a.a.H = n_heads; a.a.Hkv = n_kv_heads; a.a.max_len = (int)max_len;
         a.a.scale_log2e = 1.4426950408889634f / sqrtf((float)head_dim);
         a.nseg = ns;
-        int64_t wgs = 0;
         for (int i = 0; i < ns; ++i) {
             const onebit_seg_t &g = segs[s0 + i];
-            const int nmb = (g.n + OB_FL_BM - 1) / OB_FL_BM;
-            wgs += (int64_t)((nmb + 1) / 2) * n_heads;
-            if (wgs > 0x3fffffffLL) return ob_fail(ONEBIT_E_ARG, "attention_ragged: too many workgroups");
-            a.wg_end[i] = (int)wgs;
             a.seg[i] = {g.row0, g.n, g.slot, g.past};
         }
+        const int64_t wgs = ob_fl_number(a);
+        if (!wgs) return ob_fail(ONEBIT_E_ARG, "attention_ragged: too many workgroups");
         if (head_dim == 128) hipLaunchKernelGGL((ob_flash_fwd_kernel<128, true>), dim3((unsigned)wgs), dim3(256), 0, (hipStream_t)stream, a);
         else hipLaunchKernelGGL((ob_flash_fwd_kernel<64, true>), dim3((unsigned)wgs), dim3(256), 0, (hipStream_t)stream, a);
         const int rc = ob_launch_status("attention_ragged");
