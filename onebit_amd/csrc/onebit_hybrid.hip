@@ -358,6 +358,16 @@ static int row_launch(const ObXRowArgs &a, int rows, hipStream_t s)
         hipLaunchKernelGGL(kern, dim3((unsigned)rows), dim3(thr), lds, s, args);
         return hstatus("row kernel");
     };
+    const bool many = rows >= OB_MANY_ROWS && !a.embed && !a.emb_save && a.W % 4 == 0 && a.W <= 4096;
+    const auto four = [&](auto kern, const auto &args) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)cdiv(rows, 4)), dim3(1024), 0, s, args, rows);
+        return hstatus("row kernel");
+    };
+    if (ext && many && (!a.top || a.eo) && a.ld_ez % 4 == 0 && (!a.out_rm || a.ld_rm % 4 == 0)) {
+#define OB_XROWS(K) (a.W <= 1024 ? four(ob_xrow_rows_kernel<E, 1, K>, a) : a.W <= 2048 ? four(ob_xrow_rows_kernel<E, 2, K>, a) : four(ob_xrow_rows_kernel<E, 4, K>, a))
+        return a.top && a.hist ? OB_XROWS(OB_X_BOTH) : a.top ? OB_XROWS(OB_X_EXPERTS) : a.hist ? OB_XROWS(OB_X_DEPTH) : OB_XROWS(OB_X_PLAIN);
+#undef OB_XROWS
+    }
     if (ext) {
         const bool one = a.W <= 4 * (int)thr;
 #define OB_XROW(K) (a.W % 4 == 0 ? one ? go(ob_xrow_kernel<E, 4, true, K>, a) : go(ob_xrow_kernel<E, 4, false, K>, a) : go(ob_xrow_kernel<E, 1, false, K>, a))
@@ -365,13 +375,7 @@ static int row_launch(const ObXRowArgs &a, int rows, hipStream_t s)
 #undef OB_XROW
     }
     const ObHNormArgs &n = a;
-    if (rows >= OB_MANY_ROWS && !a.embed && !a.emb_save && a.W % 4 == 0 && a.W <= 4096) {
-        const auto four = [&](auto kern) {
-            hipLaunchKernelGGL(kern, dim3((unsigned)cdiv(rows, 4)), dim3(1024), 0, s, n, rows);
-            return hstatus("row kernel");
-        };
-        return a.W <= 1024 ? four(ob_hnorm_rows_kernel<E, 1>) : a.W <= 2048 ? four(ob_hnorm_rows_kernel<E, 2>) : four(ob_hnorm_rows_kernel<E, 4>);
-    }
+    if (many) return a.W <= 1024 ? four(ob_hnorm_rows_kernel<E, 1>, n) : a.W <= 2048 ? four(ob_hnorm_rows_kernel<E, 2>, n) : four(ob_hnorm_rows_kernel<E, 4>, n);
     return a.W % 4 == 0 ? go(ob_hnorm_kernel<E, 4>, n) : go(ob_hnorm_kernel<E, 1>, n);
 }
 

@@ -30,3 +30,26 @@ def test_many_rows_equal_few(width, heads, vdim, groups, dtype):
         few, many = eng.logits[:len(p)], whole[row:row + len(p)]
         assert float(((many - few).norm(dim=1) / few.norm(dim=1)).max()) < (1e-2 if dtype == torch.bfloat16 else 1e-4), i
         row += len(p)
+
+
+# the same widths; experts all chosen (no choice can flip), six a token = one and a half rounds of four; identity expert, shared expert, none; depth
+# averages over up to five results, token input.  (bf16, 2e-2: where few rows keep the experts' outputs in 32 bits, many rows round each to 2^-9)
+@pytest.mark.parametrize("width,dtype", [(80, torch.bfloat16), (1028, torch.bfloat16), (2056, torch.bfloat16), (4100, torch.bfloat16), (1100, torch.float32)])
+def test_many_sequential_rows_equal_few(width, dtype):
+    from onebit_amd.serotar import SerotarConfig, build_synthetic_model
+    mixer = dict(heads=2, dim=32, vdim=32, q_rank=32, kv_rank=32, scale=0.2)
+    moe = lambda n, identity: {"kind": "moe", "expert": {"ff": 24}, "router": dict(experts=n, top=n + identity, identity=identity)}
+    cfg = SerotarConfig(vocab_size=96, width=width, norm_eps=1e-5, embed_scale=2.0, bigram={"buckets": 64, "mul_prev": 7, "mul_cur": 5}, side_dim=16, layers=[
+        {"type": "latent_attention", "mixer": mixer, "mlp": mlp} for mlp in ({"kind": "dense", "ff": 64}, dict(moe(5, 1), shared={"ff": 24}), None, moe(2, 0))])
+    model = build_synthetic_model(cfg, seed=4, device="cuda", dtype=dtype)
+    g = torch.Generator().manual_seed(width)
+    prompts = [torch.randint(0, 96, (n,), generator=g).tolist() for n in (350, 349, 217, 111)]        # 1027 rows
+    eng = model.step_engine(4, 352, max_rows=1027)
+    eng.launch([(i, 0, p, len(p)) for i, p in enumerate(prompts)])
+    whole = eng.logits[:1027].clone()
+    row = 0
+    for i, p in enumerate(prompts):
+        eng.launch([(i, 0, p, len(p))])
+        few, many = eng.logits[:len(p)], whole[row:row + len(p)]
+        assert float(((many - few).norm(dim=1) / few.norm(dim=1)).max()) < (2e-2 if dtype == torch.bfloat16 else 1e-4), i
+        row += len(p)
