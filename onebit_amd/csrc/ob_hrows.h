@@ -92,19 +92,38 @@ __global__ __launch_bounds__(1024) void ob_hnorm_kernel(const ObHNormArgs A)
     }
 }
 
+// Sum of a row that four of the workgroup's waves share (row q of four, thread tid of its 256), in the order of ob_block_sum over 256 NS threads: v[i] is
+// what thread 256 i + tid would have.  `red`: 16 NS floats of its own.
+template <int NS> __device__ __forceinline__ float ob_rows4_sum(const float (&v)[NS], float *red, int q, int tid)
+{
+    float *rq = red + 4 * NS * q;
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+        const float w = ob_wave_sum(v[i]);
+        if ((tid & 63) == 0) rq[4 * i + (tid >> 6)] = w;
+    }
+    __syncthreads();
+    if (NS == 1) return (rq[0] + rq[1]) + (rq[2] + rq[3]);
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4 * NS; ++i) s += rq[i];
+    return s;
+}
+
 // ... of many rows: four rows a workgroup, four waves each (1024 NV columns, W % 4 == 0, no embedding row), the row in registers.  The four rows' pieces
 // of the fragment-major output lie next to each other and leave as whole sectors from one L2 (ob_gated_norm_rows_kernel):
-// 6100 rows of 2048 columns 46 -> 42 us.
+// 6100 rows of 2048 columns 46 -> 42 us.  A row's squares are added in ob_hnorm_kernel's order: a row's result does not depend on the others' number.
 template <typename E, int NV>
 __global__ __launch_bounds__(1024) void ob_hnorm_rows_kernel(const ObHNormArgs A, int n_rows)
 {
-    __shared__ float red[16];
+    constexpr int NS = NV < 2 ? NV : 2;                                // (ob_hnorm_kernel has 512 threads here: pieces i and i + 2 are one thread's)
+    __shared__ float red[16 * NS];
     const int tid = threadIdx.x & 255, q = threadIdx.x >> 8, t = min((int)blockIdx.x * 4 + q, n_rows - 1);
     const bool live = (int)blockIdx.x * 4 + q < n_rows;                // (a row beyond the last: read again, not written)
     const int src = A.rows ? A.rows[t] : t;
     float *xr = A.x + (size_t)src * A.W;
     ob_float4 r[NV];
-    float ss = 0.f;
+    float ss[NS] = {};
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
         const int c = (i * 256 + tid) * 4;
@@ -116,14 +135,10 @@ __global__ __launch_bounds__(1024) void ob_hnorm_rows_kernel(const ObHNormArgs A
             for (int e = 0; e < 4; ++e) r[i][e] += A.mult * (A.bias ? s[e] + A.bias[c + e] : s[e]);
             if (A.emb_add) r[i] += *reinterpret_cast<const ob_float4 *>(A.emb_add + (size_t)src * A.W + c);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) ss = __builtin_fmaf(r[i][e], r[i][e], ss);
+            for (int e = 0; e < 4; ++e) ss[i % NS] = __builtin_fmaf(r[i][e], r[i][e], ss[i % NS]);
         }
     }
-    ss = ob_wave_sum(ss);
-    if ((tid & 63) == 0) red[threadIdx.x >> 6] = ss;
-    __syncthreads();                                                   // (every read of the residual row is done)
-    const float *rq = red + 4 * q;
-    const float rs = 1.0f / sqrtf(((rq[0] + rq[1]) + (rq[2] + rq[3])) / (float)A.W + A.eps);
+    const float rs = 1.0f / sqrtf(ob_rows4_sum<NS>(ss, red, q, tid) / (float)A.W + A.eps);      // (every read of the residual row is done)
     if (!live) return;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
@@ -335,13 +350,13 @@ __global__ __launch_bounds__(1024) void ob_xrow_rows_kernel(const ObXRowArgs A, 
     constexpr int NH = 8;
     constexpr bool EXP = (KIND & 1) != 0, DEP = (KIND & 2) != 0;
     typedef typename ObElem<E>::V4 V4;
-    __shared__ float red[2][16];
+    __shared__ float red[2][16 * NV];
     const int tid = threadIdx.x & 255, q = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), t = min((int)blockIdx.x * 4 + q, n_rows - 1);
     const bool live = (int)blockIdx.x * 4 + q < n_rows;                // (a row beyond the last: read again, not written)
     const int src = A.rows ? A.rows[t] : t;
     float *xr = A.x + (size_t)src * A.W, *hr = A.hist + (size_t)src * A.W;
     ob_float4 x[NV], s[NV];
-    float ss = 0.f;
+    float ss[NV] = {};                                                 // (ob_xrow_kernel has a thread for every piece)
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
         const int c = (i * 256 + tid) * 4;
@@ -395,20 +410,15 @@ __global__ __launch_bounds__(1024) void ob_xrow_rows_kernel(const ObXRowArgs A, 
             }
         }
     }
-    const auto row_sum = [&](float v, float (&r)[16]) {
-        v = ob_wave_sum(v);
-        if ((tid & 63) == 0) r[threadIdx.x >> 6] = v;
-        __syncthreads();
-        return (r[4 * q] + r[4 * q + 1]) + (r[4 * q + 2] + r[4 * q + 3]);
-    };
     float rp = 1.f;
     if (A.post_w) {                                                    // (uniform)
 #pragma unroll
         for (int i = 0; i < NV; ++i)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) ss = __builtin_fmaf(s[i][e], s[i][e], ss);
-        rp = 1.0f / sqrtf(row_sum(ss, red[0]) / (float)A.W + A.eps);
-        ss = 0.f;
+            for (int e = 0; e < 4; ++e) ss[i] = __builtin_fmaf(s[i][e], s[i][e], ss[i]);
+        rp = 1.0f / sqrtf(ob_rows4_sum<NV>(ss, red[0], q, tid) / (float)A.W + A.eps);
+#pragma unroll
+        for (int i = 0; i < NV; ++i) ss[i] = 0.f;
     }
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
@@ -440,12 +450,12 @@ __global__ __launch_bounds__(1024) void ob_xrow_rows_kernel(const ObXRowArgs A, 
             }
             if (!A.rows && live) *reinterpret_cast<ob_float4 *>(xr + c) = r;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) ss = __builtin_fmaf(r[e], r[e], ss);
+            for (int e = 0; e < 4; ++e) ss[i] = __builtin_fmaf(r[e], r[e], ss[i]);
             s[i] = r;
         }
     }
     float rs = 1.f;
-    if (A.w) rs = 1.0f / sqrtf(row_sum(ss, red[1]) / (float)A.W + A.eps);                 // (uniform)
+    if (A.w) rs = 1.0f / sqrtf(ob_rows4_sum<NV>(ss, red[1], q, tid) / (float)A.W + A.eps);       // (uniform)
     if (!live) return;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
@@ -519,17 +529,20 @@ __global__ __launch_bounds__(256) void ob_gated_norm_rows_kernel(const ObGatedNo
         const int c = (i * 64 + lane) * VEC;
         if (c < A.gsize) { yv[i] = *reinterpret_cast<const V16 *>(y + c); zv[i] = *reinterpret_cast<const V16 *>(z + c); }
     }
-    float v[NV][VEC], ss = 0.f;
+    constexpr int NS = NV < 4 ? NV : 4;                                // (added in ob_gated_norm_kernel's order: 256 threads, pieces i and i + 4 are one's)
+    float v[NV][VEC], ss[NS] = {};
 #pragma unroll
     for (int i = 0; i < NV; ++i)
         if ((i * 64 + lane) * VEC < A.gsize) {
 #pragma unroll
             for (int e = 0; e < VEC; ++e) {
                 v[i][e] = (float)yv[i][e] * ob_silu<E>((float)zv[i][e]);
-                ss = __builtin_fmaf(v[i][e], v[i][e], ss);
+                ss[i % NS] = __builtin_fmaf(v[i][e], v[i][e], ss[i % NS]);
             }
         }
-    const float rs = 1.0f / sqrtf(ob_wave_sum(ss) / (float)A.gsize + A.eps);
+#pragma unroll
+    for (int i = 0; i < NS; ++i) ss[i] = ob_wave_sum(ss[i]);
+    const float rs = 1.0f / sqrtf((NS == 1 ? ss[0] : (ss[0] + ss[1 % NS]) + (ss[2 % NS] + ss[3 % NS])) / (float)A.gsize + A.eps);
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
         const int c = (i * 64 + lane) * VEC;

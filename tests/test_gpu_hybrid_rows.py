@@ -1,12 +1,25 @@
 """The hybrid decoders' row kernels of many rows (four rows a workgroup, from 1024 rows on) against the kernels of few rows: the same prompts as one
 step of more than 1024 rows, and one request at a time.
 
-Only the order in which a row's squares are added differs: one float32 ulp of a norm, which moves single bf16 roundings (2^-9) of what follows; 1 % of
-the logits' norm is asserted of every row (a row, or a quarter of one, that is wrong shows as 10 % and more)."""
+A row's squares are added in the same order whatever the number of rows, so a step of 1024 rows equals, bit for bit, the same step without its last row
+(everything else, the number of K splits among it, is the same in both).  One request at a time the products are split otherwise: float32 ulps that move
+single bf16 roundings (2^-9) of what follows; 1 % of the logits' norm is asserted of every row (a row, or a quarter of one, that is wrong shows as 10 %
+and more)."""
 import pytest
 import torch
 
 pytestmark = pytest.mark.gpu
+
+
+def _equal_without_last_row(model, prompts):
+    """Every row's logits of a step of 1024 rows are those of the same step of 1023."""
+    eng = model.step_engine(4, 352, max_rows=1024)
+    assert sum(len(p) for p in prompts) == 1024
+    eng.launch([(i, 0, p, len(p)) for i, p in enumerate(prompts)])
+    whole = eng.logits[:1024].clone()
+    eng.launch([(i, 0, p[:len(p) - (i == 3)], len(p) - (i == 3)) for i, p in enumerate(prompts)])
+    wrong = (whole[:1023] != eng.logits[:1023]).any(1).nonzero()
+    assert not len(wrong), wrong[:8].flatten().tolist()
 
 
 # widths of one, two and four pieces per thread and beyond (4100: the general kernel); groups of 24, 2048 and 4096 columns; not a whole piece (20)
@@ -30,6 +43,7 @@ def test_many_rows_equal_few(width, heads, vdim, groups, dtype):
         few, many = eng.logits[:len(p)], whole[row:row + len(p)]
         assert float(((many - few).norm(dim=1) / few.norm(dim=1)).max()) < (1e-2 if dtype == torch.bfloat16 else 1e-4), i
         row += len(p)
+    _equal_without_last_row(model, prompts[:3] + [prompts[3][:108]])
 
 
 # the same widths; experts all chosen (no choice can flip), six a token = one and a half rounds of four; identity expert, shared expert, none; depth
@@ -53,3 +67,4 @@ def test_many_sequential_rows_equal_few(width, dtype):
         few, many = eng.logits[:len(p)], whole[row:row + len(p)]
         assert float(((many - few).norm(dim=1) / few.norm(dim=1)).max()) < (2e-2 if dtype == torch.bfloat16 else 1e-4), i
         row += len(p)
+    _equal_without_last_row(model, prompts[:3] + [prompts[3][:108]])
