@@ -87,12 +87,6 @@ static int ob_fdec_launch(const void *q, const void *k_cache, const void *v_cach
 {
     ObFdecArgs a = {};
     if (fu) a = *fu;
-    // (row, head) pairs that fill the chip by themselves: neighbouring splits become one, up to 512 positions from one pair per CU on, 1024 from two --
-    // a split ends in a ticket and the last one's combination, 2 us that no load hides (29 rows of 32 heads, 225-450 positions, 4 layers: chunks of
-    // 128 / 256 / 512 positions 460 / 440 / 419 us a step; 4 rows 285 / 284 / 289).  Scratch is laid out for the caller's splits: fewer fit.
-    const int64_t pairs = rows * n_heads, cus = ob_cu_count();
-    const int merge = std::min(n_splits, (pairs >= 2 * cus ? 1024 : pairs >= cus ? 512 : 0) / chunk);
-    if (merge > 1) { n_splits = (n_splits + merge - 1) / merge; chunk *= merge; }
     a.q = (const _Float16 *)q; a.k = (const _Float16 *)k_cache; a.v = (const _Float16 *)v_cache; a.o = (_Float16 *)o;
     a.h_next = (const _Float16 *)h_next; a.row_slot = row_slot; a.row_pos = row_pos;
     a.H = n_heads; a.Hkv = n_kv_heads; a.D = head_dim; a.max_len = (int)max_len; a.n_slots = (int)n_slots; a.chunk = chunk; a.nsplit = n_splits;
