@@ -115,34 +115,42 @@ struct ObFlSoftmaxBf16 : ObFlSigmoidBf16 {
 #define OB_FL_BM 128
 #define OB_FL_BN 64
 #define OB_FL_THREADS 256
-#define OB_FL_SLOTS 512         // resident workgroups of the chip: two to each of 256 CUs
 
-// Workgroups of a ragged launch: sets wg_end, hg and snake from the segments' row counts; 0 = too many.
-// Pairs of query blocks are the same work each, but a workgroup is as long as two blocks: where the pairs do not take every slot, some CUs
-// run one workgroup (4 waves, the latencies of a block's barriers bare) while others run two, or all run one.  Then the blocks go one by
+// Workgroups of a ragged launch on a chip of `cus` CUs: sets wg_end, hg and snake from the segments' row counts; 0 = too many.
+// Pairs of query blocks are the same work each, but a workgroup is as long as two blocks: where the pairs do not take every slot (two workgroups per
+// CU), some CUs run one (4 waves, the latencies of a block's barriers bare) while others run two, or all run one.  Then the blocks go one by
 // one, heaviest first over the heads that one XCD's share of the launch covers (their keys and values stay in its L2); if all are resident
-// at once nothing is dealt later, and the lighter half comes lightest first, so that a heavy and a light block share a CU.  Measured, pairs
-// -> single blocks: 4 x 500 rows x 32 heads of width 128 (256 pairs, 512 blocks) 33.7 -> 27.3 us; a bf16 launch of 384 pairs 124.6 -> 120.0 us
-// with sigmoid weights, 100.0 -> 98.4 us with softmax ones.  From OB_FL_SLOTS pairs on they fill the chip.
-inline int64_t ob_fl_number(ObFlashRaggedArgs &f)
+// at once nothing is dealt later, and the lighter half comes lightest first, so that a heavy and a light block share a CU.  Where the line lies (420 random
+// launches of 1-8 segments, pairs -> single blocks):
+//   * every XCD's share is one group of heads with all its blocks (segments of equally many blocks): never slower, 1.24x on average; 4 x 500 rows x 32
+//     heads of width 128 (256 pairs, 512 blocks) 33.7 -> 27.3 us; a bf16 launch of 384 pairs 124.6 -> 120.0 us with sigmoid weights, 100.0 -> 98.4 with softmax
+//   * else some XCDs get the heavy blocks and others the light ones.  All resident, that is still faster where a pair is a tenth longer than the longest
+//     single block (1.10-1.6x), not where one block far back in its cache is the longest workgroup either way (6 segments x 40 heads: 35 against 45 us)
+//   * not all resident: 3 x 1000 rows x 40 heads 53 against 62 us, half of such launches slower
+inline int64_t ob_fl_number(ObFlashRaggedArgs &f, int cus)
 {
     const int H = f.a.H;
-    int64_t pairs = 0, single = 0;
+    int64_t pairs = 0, single = 0, len1 = 0, len2 = 0;                 // longest single block and pair, in blocks of keys
+    bool equal = true;
+    const auto blocks = [&](int i) { return ((int64_t)f.seg[i].n + OB_FL_BM - 1) / OB_FL_BM; };
     for (int i = 0; i < f.nseg; ++i) {
-        const int64_t nmb = ((int64_t)f.seg[i].n + OB_FL_BM - 1) / OB_FL_BM;
+        const int64_t nmb = blocks(i), keys = (int64_t)f.seg[i].past + f.seg[i].n, first = f.seg[i].past + std::min(f.seg[i].n, OB_FL_BM);
         pairs += (nmb + 1) / 2 * H;
         single += nmb * H;
+        equal = equal && nmb == blocks(0);
+        const int64_t top = (keys + OB_FL_BN - 1) / OB_FL_BN;
+        len1 = std::max(len1, top);
+        len2 = std::max(len2, top + (nmb > 1 ? (first + OB_FL_BN - 1) / OB_FL_BN : 0));
         if (pairs > 0x3fffffffLL) return 0;
     }
-    const bool one = pairs < OB_FL_SLOTS;
+    const int64_t per_xcd = (int64_t)H * f.nseg / 8;
+    const bool whole = equal && (int64_t)H * f.nseg % 8 == 0 && H % per_xcd == 0;
+    const bool one = pairs < 2 * cus && (whole || (single <= 2 * cus && 10 * len2 >= 11 * len1));
     f.hg = 0;
-    f.snake = one && single <= OB_FL_SLOTS;
-    if (one) for (f.hg = (int)std::min<int64_t>(H, std::max<int64_t>(1, (int64_t)H * f.nseg / 8)); H % f.hg; --f.hg) ;
+    f.snake = one && single <= 2 * cus;
+    if (one) for (f.hg = (int)std::min<int64_t>(H, std::max<int64_t>(1, per_xcd)); H % f.hg; --f.hg) ;
     int64_t end = 0;
-    for (int i = 0; i < f.nseg; ++i) {
-        const int64_t nmb = ((int64_t)f.seg[i].n + OB_FL_BM - 1) / OB_FL_BM;
-        f.wg_end[i] = (int)(end += (one ? nmb : (nmb + 1) / 2) * H);
-    }
+    for (int i = 0; i < f.nseg; ++i) f.wg_end[i] = (int)(end += (one ? blocks(i) : (blocks(i) + 1) / 2) * H);
     return end;
 }
 

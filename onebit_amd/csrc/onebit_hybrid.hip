@@ -5,6 +5,7 @@
 // before it (sums, output norm, residual, depth average) and forms the input of the next.
 #include <hip/hip_runtime.h>
 #include <algorithm>
+#include <atomic>
 #include <mutex>
 #include <set>
 #include <utility>
@@ -40,6 +41,16 @@ extern "C" const char *onebit_hybrid_last_error(void) { return g_err; }
 
 static inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 static inline int64_t rup(int64_t a, int64_t b) { return cdiv(a, b) * b; }
+static int cu_count()
+{
+    static std::atomic<int> cached[64];
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
+    if ((n = cached[dev].load(std::memory_order_relaxed)) > 0) return n;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return 256;
+    cached[dev].store(n, std::memory_order_relaxed);
+    return n;
+}
 // more than 64 KB of LDS: allowed once per (device, kernel), up to the 160 KB of a CU
 static bool lds_ok(const void *f, int bytes)
 {
@@ -434,7 +445,7 @@ static int attention_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, 
             const onebit_hseg_t &g = st.segs[s0 + i];
             a.seg[i] = {g.row0, g.n, g.slot, g.past};
         }
-        const int64_t wgs = ob_fl_number(a);
+        const int64_t wgs = ob_fl_number(a, cu_count());
         if (!wgs) return hfail(ONEBIT_E_ARG, "attention: too many workgroups");
         if (L.kp == 128) hipLaunchKernelGGL((ob_flash_fwd_kernel<128, true, ObFlSigmoidBf16>), dim3((unsigned)wgs), dim3(256), 0, s, a);
         else hipLaunchKernelGGL((ob_flash_fwd_kernel<64, true, ObFlSigmoidBf16>), dim3((unsigned)wgs), dim3(256), 0, s, a);
@@ -647,7 +658,7 @@ static int latent_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, con
             f.a.H = f.a.Hkv = H; f.a.max_len = (int)P.kv_rows;
             f.a.scale_log2e = L.scale * OB_LOG2E;
             f.out = act; f.out_nkt = act_nkt; f.vdim = l.vdp;
-            const int64_t wgs = ob_fl_number(f);
+            const int64_t wgs = ob_fl_number(f, cu_count());
             if (!wgs) return hfail(ONEBIT_E_ARG, "attention: too many workgroups");
             if (L.kp == 128) hipLaunchKernelGGL((ob_flash_fwd_kernel<128, true, ObFlSoftmaxBf16>), dim3((unsigned)wgs), dim3(256), 0, s, f);
             else hipLaunchKernelGGL((ob_flash_fwd_kernel<64, true, ObFlSoftmaxBf16>), dim3((unsigned)wgs), dim3(256), 0, s, f);

@@ -57,7 +57,7 @@ extern "C" int onebit_attention_ragged(const void *q, const void *k_cache, const
             const onebit_seg_t &g = segs[s0 + i];
             a.seg[i] = {g.row0, g.n, g.slot, g.past};
         }
-        const int64_t wgs = ob_fl_number(a);
+        const int64_t wgs = ob_fl_number(a, ob_cu_count());
         if (!wgs) return ob_fail(ONEBIT_E_ARG, "attention_ragged: too many workgroups");
         if (head_dim == 128) hipLaunchKernelGGL((ob_flash_fwd_kernel<128, true>), dim3((unsigned)wgs), dim3(256), 0, (hipStream_t)stream, a);
         else hipLaunchKernelGGL((ob_flash_fwd_kernel<64, true>), dim3((unsigned)wgs), dim3(256), 0, (hipStream_t)stream, a);

@@ -1,4 +1,5 @@
-"""Prompt attention of several sequences: query blocks taken one by one where their pairs leave slots of the chip free, in pairs from 512 pairs on.
+"""Prompt attention of several sequences: query blocks taken one by one where their pairs leave slots of the chip free and the XCDs' shares stay even,
+in pairs elsewhere and from 512 pairs on.
 Which workgroup sweeps a block does not enter its arithmetic: every segment's rows are, bit for bit, the single-sequence kernel's (always pairs)."""
 import ctypes
 
@@ -9,11 +10,13 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-# (rows, past) of the segments; H x blocks: all resident (<= 512 blocks), dealt in rounds (<= 511 pairs), pairs; odd block counts, heads the groups do
-# not divide evenly, one head, a segment of one row, a segment past a full cache
+# (rows, past) of the segments; H x blocks: all resident (<= 512 blocks), dealt in rounds (equal segments, <= 511 pairs), pairs (from 512 on; unequal
+# segments of more than 512 blocks; a block far back in its cache the longest either way); odd block counts, heads the groups do not divide evenly,
+# one head, a segment of one row, a segment past a full cache
 @pytest.mark.parametrize("spec,H,Hkv,D", [
     ([(1, 0)], 1, 1, 64), ([(700, 0)], 5, 1, 128), ([(129, 70), (1, 130), (640, 0), (385, 315)], 12, 4, 64), ([(512, 0)] * 4, 32, 8, 128),
-    ([(513, 0), (700, 0), (127, 5)], 40, 40, 64), ([(640, 60), (640, 0), (256, 3)], 73, 73, 64), ([(700, 0)] * 6, 28, 28, 64), ([(257, 0)] * 8, 32, 4, 128)])
+    ([(513, 0), (700, 0), (127, 5)], 40, 40, 64), ([(640, 60), (640, 0), (256, 3)], 73, 73, 64), ([(700, 0)] * 6, 28, 28, 64), ([(257, 0)] * 8, 32, 4, 128),
+    ([(640, 0)] * 4, 32, 8, 128), ([(300, 0), (600, 0)], 60, 12, 128), ([(256, 0), (106, 590), (31, 600)], 40, 8, 128)])
 def test_blocks_and_pairs(spec, H, Hkv, D):
     from onebit_amd import _lib
     from onebit_amd.bitnet import _stream_ptr
