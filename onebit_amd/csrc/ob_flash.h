@@ -184,14 +184,15 @@ __device__ __forceinline__ float ob_fl_col_sum(float v)
 #define OB_FL_DEFER_THR 8.0f    // log2 units: the running maximum is kept while the new tile's maximum exceeds it by less (P <= 2^8)
 #endif
 
-template <int D, bool RAGGED = false, class POL = ObFlSoftmaxF16>
+// SINGLE: a workgroup has one query block (ObFlashRaggedArgs::hg), no pair -- a kernel of its own: the pairs' loop is 1-4 % slower with the choice in it
+template <int D, bool RAGGED = false, class POL = ObFlSoftmaxF16, bool SINGLE = false>
 __global__ __launch_bounds__(256, 2) void ob_flash_fwd_kernel(const std::conditional_t<RAGGED, typename POL::RaggedArgs, ObFlashArgs> AA)
 {
     typedef typename POL::H H16;
     typedef typename POL::V8 V8;
     constexpr bool SM = POL::SOFTMAX;
     constexpr bool B16 = POL::BF16;
-    static_assert(!B16 || RAGGED, "the bf16 forms have ragged rows only");
+    static_assert(RAGGED || !(B16 || SINGLE), "the bf16 forms and single blocks have ragged rows only");
     const ObFlashArgs &A = [&]() -> const ObFlashArgs & { if constexpr (RAGGED) return AA.a; else return AA; }();
     constexpr int DT = D / 16, DK = D / 32;
     constexpr int NPC = D / 8;                  // 16-byte pieces per K / V row
@@ -231,7 +232,7 @@ __global__ __launch_bounds__(256, 2) void ob_flash_fwd_kernel(const std::conditi
         nmb = (S + OB_FL_BM - 1) / OB_FL_BM;
         npair = (nmb + 1) >> 1;
         const int loc = bid - wg0;
-        if (AA.hg) {
+        if constexpr (SINGLE) {
             const int per = nmb * AA.hg, grp = loc / per, r = loc - grp * per;
             pj = r / AA.hg; head = grp * AA.hg + r - pj * AA.hg;
             if (AA.snake && pj >= npair) pj = nmb - 1 - (pj - npair);
@@ -264,11 +265,10 @@ __global__ __launch_bounds__(256, 2) void ob_flash_fwd_kernel(const std::conditi
     unsigned long long *tr = nullptr;
     if (A.trace && (orig == 0 || orig == nwg / 2) && lane == 0) tr = A.trace + ((orig ? 1 : 0) * (OB_FL_THREADS / 64) + wave) * 66 * 8;
 #endif
-    for (int pass = 0; pass < 2; ++pass) {
+    for (int pass = 0; pass < (SINGLE ? 1 : 2); ++pass) {
     OB_FL_TP(0);
     const int mb = pass == 0 ? nmb - 1 - pj : pj;
     if (pass == 1 && mb == nmb - 1 - pj) break;                 // odd count: the middle block has no partner
-    if constexpr (RAGGED) { if (pass == 1 && AA.hg) break; }    // the workgroup has a single block
     const int m0 = mb * OB_FL_BM;
     // Q^T fragments of the wave's two query tiles: lane (query = lr, d = 32 ds + 8 g .. + 7)
     V8 qf[2][DK];
@@ -605,4 +605,12 @@ __global__ __launch_bounds__(256, 2) void ob_flash_fwd_kernel(const std::conditi
     }
     OB_FL_TP(3);
     }
+}
+
+// a numbered ragged launch
+template <int D, class POL = ObFlSoftmaxF16>
+inline void ob_fl_launch(const typename POL::RaggedArgs &a, int64_t wgs, hipStream_t s)
+{
+    if (a.hg) hipLaunchKernelGGL((ob_flash_fwd_kernel<D, true, POL, true>), dim3((unsigned)wgs), dim3(OB_FL_THREADS), 0, s, a);
+    else hipLaunchKernelGGL((ob_flash_fwd_kernel<D, true, POL>), dim3((unsigned)wgs), dim3(OB_FL_THREADS), 0, s, a);
 }

@@ -447,8 +447,8 @@ static int attention_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, 
         }
         const int64_t wgs = ob_fl_number(a, cu_count());
         if (!wgs) return hfail(ONEBIT_E_ARG, "attention: too many workgroups");
-        if (L.kp == 128) hipLaunchKernelGGL((ob_flash_fwd_kernel<128, true, ObFlSigmoidBf16>), dim3((unsigned)wgs), dim3(256), 0, s, a);
-        else hipLaunchKernelGGL((ob_flash_fwd_kernel<64, true, ObFlSigmoidBf16>), dim3((unsigned)wgs), dim3(256), 0, s, a);
+        if (L.kp == 128) ob_fl_launch<128, ObFlSigmoidBf16>(a, wgs, s);
+        else ob_fl_launch<64, ObFlSigmoidBf16>(a, wgs, s);
     }
     return hstatus("prompt attention");
 }
@@ -660,8 +660,8 @@ static int latent_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, con
             f.out = act; f.out_nkt = act_nkt; f.vdim = l.vdp;
             const int64_t wgs = ob_fl_number(f, cu_count());
             if (!wgs) return hfail(ONEBIT_E_ARG, "attention: too many workgroups");
-            if (L.kp == 128) hipLaunchKernelGGL((ob_flash_fwd_kernel<128, true, ObFlSoftmaxBf16>), dim3((unsigned)wgs), dim3(256), 0, s, f);
-            else hipLaunchKernelGGL((ob_flash_fwd_kernel<64, true, ObFlSoftmaxBf16>), dim3((unsigned)wgs), dim3(256), 0, s, f);
+            if (L.kp == 128) ob_fl_launch<128, ObFlSoftmaxBf16>(f, wgs, s);
+            else ob_fl_launch<64, ObFlSoftmaxBf16>(f, wgs, s);
             if (int rc2 = hstatus("prompt attention")) return rc2;
             s0 = i;
         }

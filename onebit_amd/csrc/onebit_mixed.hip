@@ -59,8 +59,8 @@ extern "C" int onebit_attention_ragged(const void *q, const void *k_cache, const
         }
         const int64_t wgs = ob_fl_number(a, ob_cu_count());
         if (!wgs) return ob_fail(ONEBIT_E_ARG, "attention_ragged: too many workgroups");
-        if (head_dim == 128) hipLaunchKernelGGL((ob_flash_fwd_kernel<128, true>), dim3((unsigned)wgs), dim3(256), 0, (hipStream_t)stream, a);
-        else hipLaunchKernelGGL((ob_flash_fwd_kernel<64, true>), dim3((unsigned)wgs), dim3(256), 0, (hipStream_t)stream, a);
+        if (head_dim == 128) ob_fl_launch<128>(a, wgs, (hipStream_t)stream);
+        else ob_fl_launch<64>(a, wgs, (hipStream_t)stream);
         const int rc = ob_launch_status("attention_ragged");
         if (rc) return rc;
     }
