@@ -394,11 +394,11 @@ template <int ROWS, int TB> __device__ __forceinline__ ObDenseRows ob_dense_rows
 }
 
 // Output tile of this workgroup.  Expert blocks: only those with rows are numbered -- the empty ones at the table's end would leave the last XCDs idle.
-template <int ROWS, int NB, int TB> __device__ __forceinline__ bool ob_dense_tile_of(const ObDenseArgs &A, int &nb, int &tb)
+template <int ROWS, int NB, int TB, int BAND = 8> __device__ __forceinline__ bool ob_dense_tile_of(const ObDenseArgs &A, int &nb, int &tb)
 {
     int ntb = (A.T + TB * 16 - 1) / (TB * 16);                         // (grouped forms: T = 16 TB times the number of blocks)
     if constexpr (ROWS == OB_ROWS_GATHER || ROWS == OB_ROWS_SORTED) ntb = A.blk[0].n_used;
-    return ob_tile_of(blockIdx.x, (A.n_tiles + NB - 1) / NB, ntb, nb, tb);
+    return ob_tile_of(blockIdx.x, (A.n_tiles + NB - 1) / NB, ntb, nb, tb, BAND);
 }
 
 // One transfer of an output tile's k steps: tile j of the NB + TB of a step
@@ -412,10 +412,9 @@ template <typename E, int ROWS, int NB> __device__ __forceinline__ ObDenseSrc ob
     return {(const char *)(j < NB ? A.w : A.a) + ((j < NB ? b.w0 : 0) + band * A.nkt + k_lo) * 1024, (uint32_t)lane * 16};
 }
 
-// bf16: workgroup = 16 NB columns x 16 TB rows, four waves 2 x 2 (ob_mm.h has the loop).  NB = 16, TB = 8, three stages of 24 KB: 6016 x 2048 x 9728
-// 277 us with the tiles of 128 x 128 that stood here (8 KB of LDS reads per 16 MFMAs: LDS-bound) -> 224, 6016 x 17920 x 2048 532 -> 391,
-// 16384 x 11008 x 4096 1467 -> 1237 = 1194 TFLOP/s (fp32 sums written).  NB = TB = 8, four stages of 16 KB, where that leaves less than two
-// rounds of workgroups (1520 x 2048 x 9728: 80 us against 127).
+// bf16: workgroup = 16 NB columns x 16 TB rows, four waves 2 x 2 (ob_mm.h has the loop).  NB = 16, TB = 8, three stages of 24 KB (6016 x 2048 x 9728:
+// 227 us with NB = 8, 208 with 16; 16384 x 11008 x 4096 1237 = 1194 TFLOP/s, fp32 sums written); NB = TB = 8, four stages of 16 KB, where 256-column
+// tiles fill their last round of workgroups worse (tiles_launch; 1520 x 2048 x 4096: 35 us against 57).
 template <int EPI, int NB, int TB, int NST, int ROWS = OB_ROWS_ALL>
 __global__ __launch_bounds__(256, 2) void ob_dense_mm_kernel(const typename ObDenseArgsOf<ROWS>::type A)
 {
@@ -449,19 +448,22 @@ __global__ __launch_bounds__(256, 2) void ob_dense_mm_kernel(const typename ObDe
     }
 }
 
-// fp32: workgroup = 8 n tiles x 8 token tiles, waves 2 x 2; four stages of one k tile each in LDS, ONE raw barrier per k tile behind a counted
-// vmcnt: at the top of step k the tile k has landed (at most the two younger ones are outstanding), the barrier tells everyone, and the buffer of
-// tile k - 1 -- whose operand reads are complete -- takes tile k + 3.  Bound by the fp32 matrix rate.
-template <int EPI, int ROWS = OB_ROWS_ALL>
-__global__ __launch_bounds__(256, 2) void ob_dense_tile_f32_kernel(const typename ObDenseArgsOf<ROWS>::type A)
+// fp32, and bf16 where all workgroups are resident, two to a CU: workgroup = 8 n tiles x 8 token tiles, waves 2 x 2; four stages of one k tile each in LDS,
+// ONE raw barrier per k tile behind a counted vmcnt: at the top of step k the tile k has landed (at most the two younger ones are outstanding), the
+// barrier tells everyone, and the buffer of tile k - 1 -- whose operand reads are complete -- takes tile k + 3.  fp32: bound by the fp32 matrix rate.
+// bf16: one workgroup reads its operands while the other multiplies; 352 workgroups of 11008 k columns 121 us against 133 with ob_mm.h's loop, whose
+// one workgroup per CU is the faster (256 workgroups: 110 against 88), and so are many rounds of them (1024: 412 against 308).  Bands of 4 token blocks:
+// 2300-3300 rows of 9728 -> 2048, weights from HBM, 105-118 us; bands of 8 103-152, all token blocks in one 103-128.
+template <typename E, int EPI, int ROWS = OB_ROWS_ALL>
+__global__ __launch_bounds__(256, 2) void ob_dense_tile_kernel(const typename ObDenseArgsOf<ROWS>::type A)
 {
-    typedef float E;
-    typedef ObElem<E>::V16 V16;
+    static_assert(ROWS != OB_ROWS_HEADS && ROWS != OB_ROWS_TABLE, "forms with few rows only");
+    typedef typename ObElem<E>::V16 V16;
     constexpr int NB = 8, TB = 8, TILES = NB + TB, PER = TILES / 4, MN = NB / 2, MT = TB / 2, NST = 4;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wn = wave & 1, wt = wave >> 1;
     int nb, tb;
-    if (!ob_dense_tile_of<ROWS, NB, TB>(A, nb, tb)) return;                         // (uniform)
+    if (!ob_dense_tile_of<ROWS, NB, TB, 4>(A, nb, tb)) return;                         // (uniform)
     const int n0 = nb * NB, split = blockIdx.y, k_lo = split * A.kt_split, nk = min(A.nkt - k_lo, A.kt_split);
     const ObDenseRows b = ob_dense_rows<ROWS, TB>(A, tb);
     if (b.rows <= 0) return;                                                         // (uniform)

@@ -16,14 +16,14 @@
 // every XCD takes a contiguous range of tiles numbered in bands of 8 token blocks, token block fastest: the 32-64 tiles in flight on it are about
 // as many token blocks as weight blocks.  (Token blocks fastest over ALL token blocks, one weight block at a time, reads 3 times as much past the
 // L2: 6016 x 2048 x 9728 270 -> 213 us, 16384 x 11008 x 4096 1465 -> 1177 with the same kernel; bands of 4, 5, 6, 12 are within 2 % of 8.)
-__device__ __forceinline__ bool ob_tile_of(int orig, int nnb, int ntb, int &nb, int &tb)
+__device__ __forceinline__ bool ob_tile_of(int orig, int nnb, int ntb, int &nb, int &tb, int band_of = 8)
 {
     const int nwg = nnb * ntb, xcd = orig & 7, j = orig >> 3, q8 = nwg >> 3, rem = nwg & 7;
     if (j >= q8 + (xcd < rem ? 1 : 0)) return false;
     const int id = (xcd < rem ? xcd * (q8 + 1) : rem * (q8 + 1) + (xcd - rem) * q8) + j;
-    const int band = id / (8 * nnb), r = id - band * 8 * nnb, w = min(8, ntb - band * 8);
+    const int band = id / (band_of * nnb), r = id - band * band_of * nnb, w = min(band_of, ntb - band * band_of);
     nb = r / w;
-    tb = band * 8 + r - nb * w;
+    tb = band * band_of + r - nb * w;
     return true;
 }
 

@@ -84,7 +84,20 @@ static int gemm_splits(int n_tiles, int nkt, int T)
     return (int)std::max<int64_t>(1, s);
 }
 
-// the LDS-DMA tiles over `n_tb` blocks of 128 rows: 256 columns wide from two rounds of workgroups on (two per CU), else 128
+// Time of `x` equal workgroups, two resident per CU, in full rounds of them: half a round of one per CU takes 0.57 (0.42 behind full rounds, whose
+// end it overlaps), more of a round 0.6 + 0.4 of its fill.  (4096 k columns, 128 x 128 tiles: 256 / 320 / 384 / 512 / 752 / 946 / 1024 workgroups 37 / 52 / 55 /
+// 63 / 94 / 118 / 121 us.)
+static double round_cost(int64_t x)
+{
+    const int64_t cus = cu_count(), full = x / (2 * cus), rem = x - full * 2 * cus;
+    return (double)full + (rem == 0 ? 0.0 : rem <= cus ? (full ? 0.42 : 0.57) : 0.6 + 0.2 * (double)rem / (double)cus);
+}
+// the LDS-DMA tiles over `n_tb` blocks of 128 rows.  A round of 256 columns takes 1.8 of one of 128 columns: the wider tiles where they cost less so.
+// (170 products of 128-8192 rows, 1536-11008 columns either way, against the better of the two: 0.999 on average, worst 0.93; 1520 rows of 2048 -> 9728, 912 or 456
+// workgroups, 67 us with 128 columns, 60 with 256; 1800 rows, 1140 or 570, 83 and 89.)  128-column tiles that are all resident, some CUs with two, take
+// ob_dense_tile_kernel up to 7/4 per CU; above, one 256-column tile a CU (weights from HBM, 9728 -> 2048: 384 tiles 111 us against 133, 464 151 against 135;
+// ob_dense_mm_kernel's 128 columns 122-150).  Experts' blocks, of which some are empty and whose rows are gathered: 256 columns from two
+// rounds on (7600 rows, six of 32 experts each, 1408 columns of gate and up: 214 us, 274 with 128)
 template <typename E, int EPI, int ROWS>
 static int tiles_launch(const typename ObDenseArgsOf<ROWS>::type &a, int64_t n_tb, int n_split, const char *what, hipStream_t s)
 {
@@ -94,9 +107,14 @@ static int tiles_launch(const typename ObDenseArgsOf<ROWS>::type &a, int64_t n_t
         return hstatus(what);
     };
     if constexpr (sizeof(E) == 2) {
-        if (cdiv(a.n_tiles, 16) * n_tb * n_split >= 1024) return go(ob_dense_mm_kernel<EPI, 16, 8, 3, ROWS>, 16, 3 * 24 * 1024);
-        return go(ob_dense_mm_kernel<EPI, 8, 8, 4, ROWS>, 8, 4 * 16 * 1024);
-    } else return go(ob_dense_tile_f32_kernel<EPI, ROWS>, 8, 4 * 16 * 1024);
+        constexpr bool EXPERTS = ROWS == OB_ROWS_GATHER || ROWS == OB_ROWS_SORTED;
+        const int64_t cus = cu_count(), wide = cdiv(a.n_tiles, 16) * n_tb * n_split, narrow = cdiv(a.n_tiles, 8) * n_tb * n_split;
+        const bool two = !EXPERTS && narrow > cus && narrow <= 2 * cus;
+        if (EXPERTS ? wide >= 4 * cus : two ? 4 * narrow > 7 * cus && wide <= cus : 1.8 * round_cost(wide) < round_cost(narrow))
+            return go(ob_dense_mm_kernel<EPI, 16, 8, 3, ROWS>, 16, 3 * 24 * 1024);
+        if (!two) return go(ob_dense_mm_kernel<EPI, 8, 8, 4, ROWS>, 8, 4 * 16 * 1024);
+    }
+    return go(ob_dense_tile_kernel<E, EPI, ROWS>, 8, 4 * 16 * 1024);
 }
 
 template <typename E, int EPI>
