@@ -542,7 +542,8 @@ int onebit_fused_gemv(const onebit_proj_t *projs, void *const *outs, int nproj, 
  *             backward pass reads instead of recomputing the GEMM.
  *   backward  from gy [T,N]: gx [T,K], gw [N,K] = (gz^T . (x*h)) * (1.001 - tanh(W)^2) (the STE, :21-23), gh [K],
  *             gg [N], gbias [N] (optional).  workspace: onebit_train_workspace_bytes(T,K,N,dtype), 16-byte aligned.
- *             forward_ws: the same with scratch memory, onebit_train_forward_workspace_bytes(T,K,N,dtype) of it 16-byte aligned (0 for fp32;
+ *             forward_ws: the same with scratch memory, onebit_train_forward_workspace_bytes(T,K,N,dtype) of it 16-byte aligned (0 for fp32 and
+ *             for products too small to gain;
  *             less or NULL takes the form of onebit_train_forward, half as fast in fp16 at T = 4096, 4096 -> 11008).
  * fp16: MFMA 16x16x32 f16 with fp32 accumulation, every tensor-level op of the reference rounded once to fp16;
  * fp32: MFMA 16x16x4 f32.  Deterministic (no atomics: column sums have a fixed order).                          */

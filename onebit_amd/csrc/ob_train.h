@@ -197,8 +197,11 @@ __global__ __launch_bounds__(OB_TG_THREADS, 2) void ob_tgemm128_f16_kernel(const
     auto put = [&](int buf, int r0) {
         const int gr = r0 + (tid & 3) * 8;
         ob_half8 f;
+        if (gr + 8 <= a.R && ((uintptr_t)(h + gr) % 16) == 0) f = *reinterpret_cast<const ob_half8 *>(h + gr);
+        else {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) f[e] = gr + e < a.R ? h[gr + e] : (_Float16)0;
+            for (int e = 0; e < 8; ++e) f[e] = gr + e < a.R ? h[gr + e] : (_Float16)0;
+        }
 #pragma unroll
         for (int hf = 0; hf < 2; ++hf) {
             const int o = buf * OB_TG2_TILE + (64 * hf + (tid >> 2)) * OB_TG2_PITCH + (tid & 3) * 8;

@@ -80,6 +80,13 @@ def test_forward_without_workspace_is_the_same_layer():
     assert _off(y, m(x).detach().double()) <= 2e-3
 
 
+def test_small_products_ask_for_no_workspace():
+    from onebit_amd import _lib
+    ws = lambda *s: _lib.load().onebit_train_forward_workspace_bytes(*s, _lib.ONEBIT_F16)
+    assert not any((ws(1, 64, 64), ws(2048, 64, 64), ws(64, 128, 128), ws(4096, 256, 64), ws(1, 255, 4096)))
+    assert all((ws(1, 256, 128), ws(1, 512, 32), ws(8192, 128, 128), ws(4096, 4096, 11008)))
+
+
 def test_sign_and_straight_through_factor_at_special_weights():
     """sign(0) = sign(-0) = 0, NaN has no sign; the factor 1.001 - tanh(w)^2 from tiny to saturated weights, with its float16 roundings."""
     from onebit_amd.train import BitLinear
