@@ -274,7 +274,12 @@ class BitLinearInf(nn.Module):
                     if len(cache) > 256:
                         cache.clear()
                     ws_bytes = cache[key] = int(lib.onebit_linear_workspace_bytes(T, K, N, code))
-            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
+            try:
+                ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
+            except torch.OutOfMemoryError:
+                if cdt != torch.float32:
+                    raise
+                ws, ws_bytes = None, 0                         # float32: the general kernel needs none
             rc = lib.onebit_linear_forward(
                 w.data_ptr(), w.stride(0), x.data_ptr(), h.data_ptr(), g.data_ptr(),
                 None if b is None else b.data_ptr(), y.data_ptr(), None,

@@ -1,4 +1,5 @@
 // float32 1-bit layer of libonebit_hip.so: launches of ob_f32.h.
+#include <algorithm>
 #include "ob_host.h"
 #include "ob_ln.h"
 #include "ob_f32.h"
@@ -9,11 +10,25 @@
 // Products below 24 M (36 M where the packed rows are copied first) stay with ob_simple_kernel: three or four launches and their host work cost more
 // than they save there (1 row of 4096 -> 4096: 18.2 us a call against 19.8; 2 rows: 21.3 / 20.4; 4 rows of 4064 -> 1000: 16.8 / 23.0, 16 rows:
 // 22.8 / 22.6).  Larger ones: 16 rows of 4096 -> 11008 188 us -> 26, 731 rows 7371 -> 165 (1.2 PFLOP/s of bf16 products), 2048 rows 20.6 ms -> 483 us.
-struct ObF32Plan { int bt, tb, quads, nb, nb_full, S, ld_t; size_t planes, rows, zt; };
-static bool ob_f32_plan(int64_t T, int64_t K, int64_t N, ObF32Plan &p)
+static bool ob_f32_takes(int64_t T, int64_t K, int64_t N)
 {
-    if (T < 1 || K < 8 || N < 4 || N % 4 != 0 || T > (1 << 24) || K > (1 << 24) || N > (1 << 24)) return false;
-    if (T * N < (K % 256 == 0 ? 24000000 : 36000000) / K) return false;
+    return T >= 1 && K >= 8 && N >= 4 && N % 4 == 0 && T <= (1 << 24) && K <= (1 << 24) && N <= (1 << 24) && T * N >= (K % 256 == 0 ? 24000000 : 36000000) / K &&
+           (size_t)N * ((K + 255) / 256) * 32 < ((size_t)1 << 32);
+}
+// Rows whose parts the scratch memory holds at once (6 bytes per activation, at most OB_F32_PLANES of them): all, or as few equal portions as fit.
+// (16384 rows of 4096 columns fit; 30000 in two portions 9.64 ms to 11008 columns, at once 9.51.)
+#define OB_F32_PLANES ((size_t)512 << 20)
+static int64_t ob_f32_portion(int64_t T, int64_t K)
+{
+    const size_t band = (size_t)((K + 255) / 256) * (8 * 3072);
+    const int64_t fit = (int64_t)std::max<size_t>(1, OB_F32_PLANES / band) * 16;
+    if (T <= fit) return T;
+    const int64_t n = (T + fit - 1) / fit, even = (T + n - 1) / n, up = (even + 127) / 128 * 128;
+    return up <= fit ? up : fit >= 128 ? fit / 128 * 128 : fit;
+}
+struct ObF32Plan { int bt, tb, quads, nb, nb_full, S, ld_t; size_t planes, rows, zt; };
+static void ob_f32_plan(int64_t T, int64_t K, int64_t N, ObF32Plan &p)
+{
     const auto align = [](size_t b) { return (b + 255) & ~(size_t)255; };
     p.quads = (int)((K + 255) / 256);
     const int64_t t64 = (T + 63) / 64 * 64, t128 = (T + 127) / 128 * 128;
@@ -21,7 +36,6 @@ static bool ob_f32_plan(int64_t T, int64_t K, int64_t N, ObF32Plan &p)
     p.tb = (int)((T + p.bt - 1) / p.bt);
     p.nb = (int)((N + 127) / 128);
     const int64_t slots = 2 * (int64_t)ob_cu_count(), tiles = (int64_t)p.nb * p.tb;
-    if (tiles > 0x7fffffff) return false;
     p.nb_full = (int)(tiles / slots * slots / p.tb);
     const int64_t left = (int64_t)(p.nb - p.nb_full) * p.tb;
     p.S = left > 0 ? (int)(slots / left) : 1;
@@ -32,12 +46,15 @@ static bool ob_f32_plan(int64_t T, int64_t K, int64_t N, ObF32Plan &p)
     p.planes = align((size_t)((T + 15) / 16) * p.quads * (8 * 3072));
     p.rows = K % 256 == 0 ? 0 : align((size_t)N * p.quads * 32);
     p.zt = (size_t)p.S * T * p.ld_t * 4;
-    return (size_t)N * p.quads * 32 < ((size_t)1 << 32);
 }
 size_t ob_f32_workspace(int64_t T, int64_t K, int64_t N)
 {
-    ObF32Plan p;
-    return ob_f32_plan(T, K, N, p) ? p.planes + p.rows + p.zt : 0;
+    if (!ob_f32_takes(T, K, N)) return 0;
+    const int64_t Tp = ob_f32_portion(T, K), rest = T % Tp;            // (the last portion, if shorter, may split K further)
+    ObF32Plan p, q;
+    ob_f32_plan(Tp, K, N, p);
+    ob_f32_plan(rest ? rest : Tp, K, N, q);
+    return p.rows + std::max(p.planes + p.zt, q.planes + q.zt);
 }
 
 template <int WN, int WT, int NW, int TW, int KS, int NST>
@@ -50,27 +67,16 @@ static void ob_launch_f32_gemm(const ObF32Gemm &a, hipStream_t s)
     hipLaunchKernelGGL((ob_f32_gemm_kernel<WN, WT, NW, TW, KS, NST>), dim3((unsigned)grid), dim3(256), lds, s, a);
 }
 
-bool ob_f32_forward(const void *packed, int64_t ldw_bytes, const float *x, const float *h, const float *g, const float *bias, float *y, float *u,
-                    void *workspace, size_t workspace_bytes, int64_t T, int64_t K, int64_t N, float eps, int skip, hipStream_t s)
+// the rows of one portion
+static void ob_f32_rows(const ObF32Plan &p, const void *packed, int64_t ldw_bytes, const float *x, const float *h, const float *g, const float *bias, float *y,
+                        float *u, char *planes, int64_t T, int64_t K, int64_t N, float eps, int skip, hipStream_t s)
 {
-    ObF32Plan p;
-    if (!ob_f32_plan(T, K, N, p) || !workspace || !ob_aligned(workspace, 256) || workspace_bytes < p.planes + p.rows + p.zt) return false;
-    // packed rows that are not whole 16-byte pieces of whole quads are copied so first
-    if (!p.rows && (ldw_bytes % 16 != 0 || !ob_aligned(packed, 16) || N * ldw_bytes >= ((int64_t)1 << 32))) return false;
-    if (!ob_aligned(g, 16) || (bias && !ob_aligned(bias, 16)) || (u && !ob_aligned(u, 16))) return false;
-    char *planes = (char *)workspace, *rows = planes + p.planes;
-    float *zt = (float *)(rows + p.rows);
+    float *zt = (float *)(planes + p.planes);
     ObF32Split sp = {x, K, h, planes, (int)T, (int)K, p.quads};
     const int64_t units = (T + 15) / 16 * p.quads;
     hipLaunchKernelGGL(ob_f32_split_kernel, dim3((unsigned)((units + 3) / 4)), dim3(256), 0, s, sp);
     ObF32Gemm a = {};
     a.W = (const char *)packed; a.ldw = ldw_bytes;
-    if (p.rows) {
-        const int64_t words = N * p.quads * 8;
-        hipLaunchKernelGGL(ob_f32_rows_kernel, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, s, (const uint8_t *)packed, (long long)ldw_bytes,
-                           (uint32_t *)rows, (int)N, (int)(K / 8), p.quads);
-        a.W = rows; a.ldw = p.quads * 32;
-    }
     a.planes = planes; a.z = y; a.zt = zt; a.zt_split = (long long)T * p.ld_t; a.ld_t = p.ld_t;
     a.T = (int)T; a.N = (int)N; a.quads = p.quads; a.tb = p.tb; a.nb_full = p.nb_full; a.nb_all = p.nb; a.S = p.S;
     if (p.bt == 16) ob_launch_f32_gemm<4, 1, 2, 1, 4, 4>(a, s);
@@ -80,7 +86,7 @@ bool ob_f32_forward(const void *packed, int64_t ldw_bytes, const float *x, const
     if (N > 16384) {
         hipLaunchKernelGGL((ob_layernorm_kernel<float, true>), dim3((unsigned)T), dim3(256), 0, s, (const float *)y, (const float *)nullptr, g, bias, y, u,
                            (int)N, eps, skip);
-        return true;
+        return;
     }
     ObF32Ln l = {y, zt, a.zt_split, p.ld_t, p.S, p.nb_full * 128, g, bias, y, u, (int)N, skip, eps};
 #define OB_F32_LN(NV_, TH_) hipLaunchKernelGGL((ob_f32_ln_kernel<NV_, TH_>), dim3((unsigned)T), dim3(TH_), 0, s, l)
@@ -91,5 +97,29 @@ bool ob_f32_forward(const void *packed, int64_t ldw_bytes, const float *x, const
     else if (N <= 12288) OB_F32_LN(6, 512);
     else OB_F32_LN(8, 512);
 #undef OB_F32_LN
+}
+
+bool ob_f32_forward(const void *packed, int64_t ldw_bytes, const float *x, const float *h, const float *g, const float *bias, float *y, float *u,
+                    void *workspace, size_t workspace_bytes, int64_t T, int64_t K, int64_t N, float eps, int skip, hipStream_t s)
+{
+    if (!ob_f32_takes(T, K, N) || !workspace || !ob_aligned(workspace, 256) || workspace_bytes < ob_f32_workspace(T, K, N)) return false;
+    const int64_t Tp = ob_f32_portion(T, K);
+    ObF32Plan p;
+    ob_f32_plan(Tp, K, N, p);
+    // packed rows that are not whole 16-byte pieces of whole quads are copied so first
+    if (!p.rows && (ldw_bytes % 16 != 0 || !ob_aligned(packed, 16) || N * ldw_bytes >= ((int64_t)1 << 32))) return false;
+    if (!ob_aligned(g, 16) || (bias && !ob_aligned(bias, 16)) || (u && !ob_aligned(u, 16))) return false;
+    char *planes = (char *)workspace + p.rows;
+    if (p.rows) {
+        const int64_t words = N * p.quads * 8;
+        hipLaunchKernelGGL(ob_f32_rows_kernel, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, s, (const uint8_t *)packed, (long long)ldw_bytes,
+                           (uint32_t *)workspace, (int)N, (int)(K / 8), p.quads);
+        packed = workspace; ldw_bytes = p.quads * 32;
+    }
+    for (int64_t t0 = 0; t0 < T; t0 += Tp) {
+        const int64_t n = std::min(Tp, T - t0);
+        ob_f32_plan(n, K, N, p);
+        ob_f32_rows(p, packed, ldw_bytes, x + t0 * K, h, g, bias, y + t0 * N, u ? u + t0 * N : nullptr, planes, n, K, N, eps, skip, s);
+    }
     return true;
 }

@@ -86,6 +86,32 @@ def test_magnitudes_and_non_finite():
     assert torch.isfinite(u[keep]).all()
 
 
+@pytest.mark.parametrize("T,K,N", [(11000, 8200, 132), (22500, 4096, 260), (48, 1900000, 20)])
+def test_portions_of_bounded_scratch(T, K, N):
+    """Scratch memory does not grow with the rows beyond 512 MB of parts; portions of rows, the last one shorter and split otherwise, are the same layer."""
+    from onebit_amd import _lib
+    ws = lambda t: _lib.load().onebit_linear_workspace_bytes(t, K, N, _lib.ONEBIT_F32)
+    rest = 40 * 2 ** 20 + N * (K + 256) // 8             # sums of split K, packed rows with columns left over
+    assert T * K * 6 > 2 ** 29 and 0 < ws(T) <= 2 ** 29 + rest and ws(20 * T) <= 2 ** 29 + rest
+    m, g = _layer(K, N, T, True)
+    _check(m, torch.randn(T, K, generator=g, device="cuda"))
+
+
+def test_without_memory_for_scratch(monkeypatch):
+    """No room for the scratch memory: the general kernel, which needs none, as before there was any."""
+    T, K, N = 70, 1376, 4100
+    m, g = _layer(K, N, 2, True)
+    x = torch.randn(T, K, generator=g, device="cuda")
+    y, empty = m(x), torch.empty
+
+    def full(*a, dtype=None, **k):
+        if dtype == torch.uint8:
+            raise torch.OutOfMemoryError("full")
+        return empty(*a, dtype=dtype, **k)
+    monkeypatch.setattr(torch, "empty", full)
+    np.testing.assert_allclose(m(x).cpu().numpy(), y.cpu().numpy(), rtol=0, atol=2e-5)
+
+
 def test_small_workspace_keeps_the_general_path():
     """A caller without the workspace is served as before, by the same numbers up to the order of additions."""
     from onebit_amd import _lib
