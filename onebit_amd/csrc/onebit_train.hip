@@ -1,5 +1,5 @@
 // Train-mode 1-bit linear layer of libonebit_hip.so (include/onebit.h): launches of ob_train.h.
-#include <stdlib.h>
+#include <algorithm>
 #include <type_traits>
 #include "ob_host.h"
 #include "ob_train.h"
@@ -66,18 +66,30 @@ static void ob_t16_layernorm(const void *z, const void *g, const void *bias, voi
 #undef OB_T16_LN
 }
 
+// rows of x whose tiles the forward's scratch memory holds at once: all up to 512 MB of them, else equal portions
+static int64_t ob_t16_portion(int64_t T, int64_t K)
+{
+    const int64_t fit = std::max<int64_t>(1, (int64_t)(((size_t)512 << 20) / ((size_t)ob_t16_up32(K) * 256))) * 128;
+    if (T <= fit) return T;
+    const int64_t n = (T + fit - 1) / fit;
+    return ((T + n - 1) / n + 127) / 128 * 128;
+}
+
 static int ob_t16_forward(const void *x, const void *w, const void *h, const void *g, const void *bias, void *y, void *z, float *stats, char *ws,
                           int64_t T, int64_t K, int64_t N, float eps, hipStream_t s)
 {
-    char *a = ws, *sg = ws + ob_t16_bytes(T, K);
-    ob_t16_tiles(false, x, h, a, T, K, s);
+    char *sg = ws, *a = ws + ob_t16_bytes(N, K);
     ob_t16_tiles(true, w, nullptr, sg, N, K, s);
     const int kt = (int)(ob_t16_up32(K) / 32);
-    ObT16Mm m = {sg, a, (int)((N + 15) / 16), (int)((T + 15) / 16), kt, kt, kt, (_Float16 *)z, (int)T, (int)N};
-    m.vec4 = N % 4 == 0 && ob_aligned(z, 8);
-    ob_t16_mm<OB_T16_Z, false, false>(m, s);
-    int rc = ob_launch_status("train_forward(product)");
-    if (rc) return rc;
+    const int64_t Tp = ob_t16_portion(T, K);
+    for (int64_t t0 = 0; t0 < T; t0 += Tp) {
+        const int64_t n = std::min(Tp, T - t0);
+        ob_t16_tiles(false, (const _Float16 *)x + t0 * K, h, a, n, K, s);
+        ObT16Mm m = {sg, a, (int)((N + 15) / 16), (int)((n + 15) / 16), kt, kt, kt, (_Float16 *)z + t0 * N, (int)n, (int)N};
+        m.vec4 = N % 4 == 0 && ob_aligned(z, 8);
+        ob_t16_mm<OB_T16_Z, false, false>(m, s);
+        if (const int rc = ob_launch_status("train_forward(product)")) return rc;
+    }
     ob_t16_layernorm(z, g, bias, y, stats, T, N, eps, s);
     return ob_launch_status("train_forward(layernorm)");
 }
@@ -85,7 +97,8 @@ static int ob_t16_forward(const void *x, const void *w, const void *h, const voi
 static int ob_t16_backward(const void *gy, const void *x, const void *w, const void *h, const void *g, const void *z, const float *stats, void *gx, void *gw,
                            void *gh, void *gg, void *gbias, char *ws, int64_t T, int64_t K, int64_t N, hipStream_t s)
 {
-    char *a = ws, *sg = a + ob_t16_bytes(T, K), *gz = sg + ob_t16_bytes(N, K);
+    // (the sign matrix and, once the input gradient is formed, x h in one place)
+    char *sg = ws, *a = ws, *gz = ws + std::max(ob_t16_bytes(T, K), ob_t16_bytes(N, K));
     float *part = (float *)(gz + ob_t16_bytes(T, N)), *rowc = (float *)((char *)part + ob_t16_part_bytes(T, K, N));
     const int kt = (int)(ob_t16_up32(K) / 32), nt = (int)(ob_t16_up32(N) / 32), tt = (int)(ob_t16_up32(T) / 32), slices = ob_t16_slices(T);
     ObT16Gz q = {(const _Float16 *)gy, (const _Float16 *)z, (const _Float16 *)g, stats, rowc, part, gz, (int)T, (int)N, 2 * tt, nt, (2 * tt + slices - 1) / slices};
@@ -93,7 +106,6 @@ static int ob_t16_backward(const void *gy, const void *x, const void *w, const v
     hipLaunchKernelGGL(ob_t16_rowc_kernel, dim3((unsigned)T), dim3(256), 0, s, q);
     hipLaunchKernelGGL(ob_t16_gz_kernel, dim3((unsigned)((nt + 3) / 4), (unsigned)slices), dim3(256), 0, s, q);
     hipLaunchKernelGGL(ob_t16_cols_kernel<2>, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, s, (const float *)part, (_Float16 *)gg, (_Float16 *)gbias, (int)N, slices);
-    ob_t16_tiles(false, x, h, a, T, K, s);
     ob_t16_tiles(true, w, nullptr, sg, N, K, s);
     if ((rc = ob_launch_status("train_backward(layernorm)"))) return rc;
     // gx [T, K] = fp16(gz S) h;  gh = sum_t fp16(gz S) x
@@ -104,6 +116,7 @@ static int ob_t16_backward(const void *gy, const void *x, const void *w, const v
                        2 * (int)((T + 127) / 128));
     if ((rc = ob_launch_status("train_backward(grad input)"))) return rc;
     // gW [N, K] = (gz^T a) (1.001 - tanh(W)^2)
+    ob_t16_tiles(false, x, h, a, T, K, s);
     ObT16Mm v = {a, gz, (int)((K + 15) / 16), (int)((N + 15) / 16), kt, nt, tt, (_Float16 *)gw, (int)N, (int)K, (const _Float16 *)w};
     v.vec4 = K % 4 == 0 && ob_aligned(gw, 8) && ob_aligned(w, 8);
     ob_t16_mm<OB_T16_GW, true, true>(v, s);
@@ -116,13 +129,13 @@ extern "C" size_t onebit_train_forward_workspace_bytes(int64_t T, int64_t K, int
 {
     if (T <= 0 || K <= 0 || N <= 0 || dtype != ONEBIT_F16) return 0;
     if (K < 512 && (N < 128 || (K < 256 && T < 100000000 / (K * N)))) return 0;
-    return ob_t16_bytes(T, K) + ob_t16_bytes(N, K);
+    return ob_t16_bytes(ob_t16_portion(T, K), K) + ob_t16_bytes(N, K);
 }
 
 extern "C" size_t onebit_train_workspace_bytes(int64_t T, int64_t K, int64_t N, int dtype)
 {
     if (T <= 0 || K <= 0 || N <= 0) return 0;
-    if (dtype != ONEBIT_F32) return ob_t16_bytes(T, K) + ob_t16_bytes(N, K) + ob_t16_bytes(T, N) + ob_t16_part_bytes(T, K, N) + ob_train_align((size_t)T * 8);
+    if (dtype != ONEBIT_F32) return std::max(ob_t16_bytes(T, K), ob_t16_bytes(N, K)) + ob_t16_bytes(T, N) + ob_t16_part_bytes(T, K, N) + ob_train_align((size_t)T * 8);
     const size_t sz = 4;
     return ob_train_align((size_t)T * N * sz) + ob_train_align((size_t)T * K * sz) + ob_train_align((size_t)T * 2 * sizeof(float)) +
            ob_train_align((size_t)OB_TC_SLICES * (2 * (size_t)N > (size_t)K ? 2 * (size_t)N : (size_t)K) * sizeof(float));     // column-sum partials

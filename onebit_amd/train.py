@@ -48,7 +48,10 @@ class _BitLinearFn(torch.autograd.Function):
         stats = torch.empty((T, 2), dtype=torch.float32, device=x.device)
         lib = _lib.load()
         nws = lib.onebit_train_forward_workspace_bytes(T, K, N, code)
-        ws = torch.empty(nws, dtype=torch.uint8, device=x.device) if nws else None
+        try:
+            ws = torch.empty(nws, dtype=torch.uint8, device=x.device) if nws else None
+        except torch.OutOfMemoryError:
+            ws, nws = None, 0                          # the kernel that needs none
         with torch.cuda.device(x.device):
             rc = lib.onebit_train_forward_ws(x2.data_ptr(), w.data_ptr(), h.data_ptr(), g.data_ptr(), None if b is None else b.data_ptr(),
                                              y.data_ptr(), z.data_ptr(), stats.data_ptr(), None if ws is None else ws.data_ptr(), nws, T, K, N, code,

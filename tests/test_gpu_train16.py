@@ -80,6 +80,33 @@ def test_forward_without_workspace_is_the_same_layer():
     assert _off(y, m(x).detach().double()) <= 2e-3
 
 
+def test_scratch_memory_is_bounded_and_optional(monkeypatch):
+    """The forward's scratch does not grow with the rows beyond 512 MB of them (portions are the same layer); the backward's holds one matrix of the layer
+    beside the output's gradient; without memory the forward runs without."""
+    from onebit_amd import _lib
+    T, K, N = 35000, 8200, 136
+    lib = _lib.load()
+    fw, bw = lib.onebit_train_forward_workspace_bytes, lib.onebit_train_workspace_bytes
+    assert T * K * 2 > 2 ** 29 and fw(T, K, N, _lib.ONEBIT_F16) <= 2 ** 29 + 2 * 160 * 8224 and fw(9 * T, K, N, _lib.ONEBIT_F16) <= 2 ** 29 + 2 * 160 * 8224
+    assert bw(4096, 4096, 11008, _lib.ONEBIT_F16) < 1.05 * 2 * 11008 * (4096 + 4096)
+    m, x, _ = _case(T, K, N, 3)
+    y = m(x.detach())
+    s, a = torch.sign(m.weight.detach()).float(), (x.detach() * m.input_factor.detach()).float()
+    u = (a @ s.T).half() * m.weight_scale.detach()
+    ref = torch.nn.functional.layer_norm(u.double(), (N,)) + m.bias.detach().double()
+    assert _off(y, ref) <= 4e-3
+    T, K, N = 300, 520, 264
+    m, x, gy = _case(T, K, N, 4)
+    full, empty = m(x.detach()), torch.empty
+
+    def none_left(*a, dtype=None, **k):
+        if dtype == torch.uint8:
+            raise torch.OutOfMemoryError("full")
+        return empty(*a, dtype=dtype, **k)
+    monkeypatch.setattr(torch, "empty", none_left)
+    assert _off(m(x.detach()), full.detach().double()) <= 2e-3
+
+
 def test_small_products_ask_for_no_workspace():
     from onebit_amd import _lib
     ws = lambda *s: _lib.load().onebit_train_forward_workspace_bytes(*s, _lib.ONEBIT_F16)
