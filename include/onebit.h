@@ -105,8 +105,8 @@ int onebit_linear_forward(const void *packed, int64_t ldw_bytes, const void *x, 
 int onebit_matmul_partial(const void *packed, int64_t ldw_bytes, const void *x, int64_t ldx,
                           const void *h, float *zp, int64_t T, int64_t K, int64_t N, int dtype,
                           void *stream);
-/* The same with a caller workspace: onebit_linear_workspace_bytes(T, K, N, dtype) bytes let large
- * calls run the LDS-DMA GEMM on the pre-scaled K slice (a smaller or NULL workspace is accepted). */
+/* The same with a caller workspace: onebit_linear_workspace_bytes(T, K, N, ONEBIT_F16) bytes, 16-byte aligned, let large
+ * float16 calls run the LDS-DMA GEMM on the pre-scaled K slice (a smaller or NULL workspace is accepted; float32 uses none). */
 int onebit_matmul_partial_ws(const void *packed, int64_t ldw_bytes, const void *x, int64_t ldx,
                              const void *h, float *zp, void *workspace, size_t workspace_bytes,
                              int64_t T, int64_t K, int64_t N, int dtype, void *stream);

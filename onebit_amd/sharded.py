@@ -74,9 +74,11 @@ def hip_partial(shard: KShard, x_slice: torch.Tensor) -> torch.Tensor:
     zp = torch.empty((T, shard.out_features), dtype=torch.float32, device=x_slice.device)
     w = shard.weight
     code = _dtype_code(x_slice.dtype)
-    # room for the pre-scaled slice: large calls then take the LDS-DMA GEMM
-    with torch.cuda.device(x_slice.device):         # the eligibility query depends on the CURRENT device's CU count
-        ws_bytes = lib.onebit_linear_workspace_bytes(T, Ks, shard.out_features, code)
+    # room for the pre-scaled slice: large float16 calls then take the LDS-DMA GEMM (float32 partial sums need none)
+    ws_bytes = 0
+    if x_slice.dtype == torch.float16:
+        with torch.cuda.device(x_slice.device):     # the eligibility query depends on the CURRENT device's CU count
+            ws_bytes = lib.onebit_linear_workspace_bytes(T, Ks, shard.out_features, code)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x_slice.device) if ws_bytes else None
     with torch.cuda.device(x_slice.device):
         rc = lib.onebit_matmul_partial_ws(w.data_ptr(), w.stride(0), x_slice.data_ptr(), x_slice.stride(0),

@@ -97,6 +97,26 @@ def test_portions_of_bounded_scratch(T, K, N):
     _check(m, torch.randn(T, K, generator=g, device="cuda"))
 
 
+def test_partial_sums_of_a_k_shard_take_no_scratch(monkeypatch):
+    from onebit_amd.sharded import hip_partial, shard_k
+    T, K, N = 64, 1024, 1000
+    m, g = _layer(K, N, 4, False)
+    x = torch.randn(T, K, generator=g, device="cuda")
+    parts, empty, asked = [], torch.empty, []
+
+    def count(*a, dtype=None, **k):
+        if dtype == torch.uint8:
+            asked.append(a)
+        return empty(*a, dtype=dtype, **k)
+    monkeypatch.setattr(torch, "empty", count)
+    for r in range(2):
+        sh = shard_k(m.weight.data, m.input_factor.data, m.weight_scale.data, None, r, 2)
+        parts.append(hip_partial(sh, x[:, sh.k0:sh.k1]))
+    assert not asked
+    z = (x * m.input_factor).double() @ _signs(m).T
+    assert float((sum(parts).double() - z).norm() / z.norm()) < 1e-6
+
+
 def test_without_memory_for_scratch(monkeypatch):
     """No room for the scratch memory: the general kernel, which needs none, as before there was any."""
     T, K, N = 70, 1376, 4100
