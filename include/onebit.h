@@ -82,11 +82,18 @@ int onebit_unpack_signs(const void *packed, void *out, int dtype, int64_t N, int
  *   K % 32 == 0 with 4-byte aligned packed rows (every LLaMA shape; 16-byte
  *   aligned rows get the widest loads); other shapes run a generic kernel.
  *   x, y rows contiguous; x/h/y 16-byte aligned.  u_or_null, if given,
- *   receives the pre-LayerNorm u [T,N].  workspace: caller-owned, 16-byte
- *   aligned scratch of onebit_linear_workspace_bytes() bytes: required only
- *   for K % 32 != 0 (fp32 z); for large prefill calls it holds the pre-scaled
- *   activations fp16(x*h) of the LDS-DMA GEMM -- without it (NULL / smaller)
- *   the register-staged GEMM runs instead, same results.
+ *   receives the pre-LayerNorm u [T,N].  workspace: caller-owned scratch of
+ *   onebit_linear_workspace_bytes() bytes, 16-byte aligned.  Required only for
+ *   F16 with K % 32 != 0 (fp32 z).  Otherwise optional; smaller or NULL selects
+ *   a slower kernel, with the same results up to the order of fp32 sums:
+ *     F16, large calls: the pre-scaled activations fp16(x*h) of the LDS-DMA GEMM;
+ *     F16, a few hundred rows: those and the fp32 sums of K slices (256-byte
+ *       aligned; 16 bytes selects the register-staged GEMM);
+ *     F32, T*K*N from 24 million on (36 if K % 256 != 0), N % 4 == 0, g / bias /
+ *       u (with K % 256 == 0 the packed rows, too) 16-byte aligned: the
+ *       activations' three bf16 parts and the sums of split K for the matrix
+ *       cores (731 rows, 4096 -> 11008: 0.16 ms, without 7.4 ms); at most 512 MB
+ *       of parts, larger calls take the rows in portions.
  */
 size_t onebit_linear_workspace_bytes(int64_t T, int64_t K, int64_t N, int dtype);
 int onebit_linear_forward(const void *packed, int64_t ldw_bytes, const void *x, const void *h,

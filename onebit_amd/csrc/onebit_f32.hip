@@ -102,7 +102,7 @@ static void ob_f32_rows(const ObF32Plan &p, const void *packed, int64_t ldw_byte
 bool ob_f32_forward(const void *packed, int64_t ldw_bytes, const float *x, const float *h, const float *g, const float *bias, float *y, float *u,
                     void *workspace, size_t workspace_bytes, int64_t T, int64_t K, int64_t N, float eps, int skip, hipStream_t s)
 {
-    if (!ob_f32_takes(T, K, N) || !workspace || !ob_aligned(workspace, 256) || workspace_bytes < ob_f32_workspace(T, K, N)) return false;
+    if (!ob_f32_takes(T, K, N) || !workspace || !ob_aligned(workspace, 16) || workspace_bytes < ob_f32_workspace(T, K, N)) return false;
     const int64_t Tp = ob_f32_portion(T, K);
     ObF32Plan p;
     ob_f32_plan(Tp, K, N, p);

@@ -132,6 +132,21 @@ def test_without_memory_for_scratch(monkeypatch):
     np.testing.assert_allclose(m(x).cpu().numpy(), y.cpu().numpy(), rtol=0, atol=2e-5)
 
 
+def test_workspace_of_the_promised_alignment():
+    """16 bytes, as the header promises: the same kernels (bit for bit) as with the module's."""
+    from onebit_amd import _lib
+    from onebit_amd.bitnet import _stream_ptr
+    for T, K, N in ((64, 1024, 1000), (20, 1376, 4100)):
+        m, g = _layer(K, N, 1, True)
+        x = torch.randn(T, K, generator=g, device="cuda")
+        y, n = torch.empty(T, N, device="cuda"), _lib.load().onebit_linear_workspace_bytes(T, K, N, _lib.ONEBIT_F32)
+        ws = torch.empty(n + 16, dtype=torch.uint8, device="cuda")
+        assert _lib.load().onebit_linear_forward(m.weight.data_ptr(), m.weight.stride(0), x.data_ptr(), m.input_factor.data_ptr(), m.weight_scale.data_ptr(),
+                                                 m.bias.data_ptr(), y.data_ptr(), None, ws.data_ptr() + 16, n, T, K, N, _lib.ONEBIT_F32, 1e-5, 0,
+                                                 _stream_ptr(x.device)) == 0
+        assert torch.equal(y, m(x))
+
+
 def test_small_workspace_keeps_the_general_path():
     """A caller without the workspace is served as before, by the same numbers up to the order of additions."""
     from onebit_amd import _lib
