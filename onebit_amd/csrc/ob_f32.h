@@ -5,7 +5,8 @@
 // product multiplies, at a third of the bf16 rate instead of the vector units': nothing of the inputs is rounded away.  The upper parts add
 // up in accumulators of their own: 8-bit addends against a 24-bit sum leave almost no rounding error there, and the error of the two
 // lower parts is 2^-8 smaller, so the sum is closer to the 64-bit one than 64 lanes' float32 chains are (731 rows, 4096 -> 11008: the layer's
-// output is 9.6e-8 off instead of 1.8e-7).  Infinities stay infinite (lower parts zero), NaN stays NaN.
+// output is 9.6e-8 off instead of 1.8e-7).  Infinities stay infinite (lower parts zero), NaN stays NaN.  Exact down to |x h| = 2^-110: smaller
+// ones lose what lies below the smallest bf16, 2^-133 (2e-6 of an activation of 2^-115), which a LayerNorm with eps 1e-5 takes away anyway.
 //
 // What bounds it: the matrix cores, three products for one (whole call at 731 rows, 4096 -> 11008: 7371 us with ob_simple_kernel, 165 now; alone in
 // a trace the product takes 159 us = 1.24 PFLOP/s, the split 8, the row pass 13).
@@ -63,7 +64,7 @@ __global__ __launch_bounds__(256) void ob_f32_split_kernel(const ObF32Split A)
     }
 }
 
-// packed rows with K % 256 columns left over, an odd pitch or an odd address: rows of `quads` x 32 bytes, zeros behind K (their planes are zero)
+// packed rows with K % 256 columns left over (of any pitch and address): rows of `quads` x 32 bytes, zeros behind K (their planes are zero)
 __global__ __launch_bounds__(256) void ob_f32_rows_kernel(const uint8_t *__restrict__ W, long long ldw, uint32_t *__restrict__ out, int N, int kb, int quads)
 {
     const long long i = (long long)blockIdx.x * 256 + threadIdx.x;

@@ -1,4 +1,4 @@
-// Inner loop of the LDS-staged 16-bit matrix products (ob_dense.h, ob_train.h) and their numbering of output tiles.
+// Inner loop of the LDS-staged 16-bit matrix products (ob_dense.h, ob_train16.h) and their numbering of output tiles.
 //
 // What bounds such a product here is the LDS (128 bytes a clock and CU) as soon as a wave's tile is small: 64 x 64 per wave asks for 12 KB of
 // operands per 16 MFMA issue slots of its SIMD, 128 x 64 for 18 per 32.  A wave therefore keeps up to 128 x 64 sums, two workgroups share a CU,

@@ -1,4 +1,4 @@
-// Train-mode 1-bit linear layer (SURVEY.md section 8 rows a8 / f4): forward and backward of the reference's
+// Train-mode 1-bit linear layer: forward and backward of the reference's
 // BitLinear + SignSTE (transformers/src/transformers/models/bitnet.py:14-28, 58-68) on LATENT full-precision
 // weights, for knowledge-distillation training on MI355X.
 //
@@ -25,7 +25,7 @@ enum { OB_TE_PLAIN = 0, OB_TE_GX = 1, OB_TE_STE = 2 };
 struct ObTGemmArgs {
     const void *A, *B;        // C[m, n] = sum_r A(m, r) * B(n, r)
     long long lda, ldb;       // leading dimension of the operand's storage (elements)
-    const void *va, *vb;      // transform vectors (same dtype), or null
+    const void *va, *vb;      // transform vectors, or null
     void *C;                  // [M, N] row-major, pitch ldc
     void *C2;                 // OB_TE_GX: C2 = C * vc[n]
     const void *vc;           // OB_TE_GX: vector [N];  OB_TE_STE: latent W [M, N] (pitch ldc)
@@ -33,9 +33,7 @@ struct ObTGemmArgs {
     int M, N, R;
 };
 
-template <typename TI> struct ObTgT;
-template <> struct ObTgT<_Float16> { static constexpr int PITCH = OB_TG_BR + 8; };     // 80-byte rows
-template <> struct ObTgT<float> { static constexpr int PITCH = OB_TG_BR + 4; };        // 144-byte rows
+#define OB_TG_PITCH (OB_TG_BR + 4)        // 144-byte rows
 
 template <typename TI>
 __device__ __forceinline__ TI ob_tg_sign(TI v)
@@ -45,55 +43,49 @@ __device__ __forceinline__ TI ob_tg_sign(TI v)
 
 // One 64 x 32 operand tile into LDS as S[i][r].  RC: the reduction index r is the contiguous one in memory
 // (element (i, r) at P[i * ld + r]); otherwise the output index i is (element at P[r * ld + i]) and the tile is
-// transposed on its way in.  8 contiguous elements per thread, one 16-byte (fp16) or two 16-byte (fp32) loads
-// when the run is inside the matrix and aligned.
-template <typename TI, bool RC, int TX>
-__device__ __forceinline__ void ob_tg_load(TI (*S)[ObTgT<TI>::PITCH], const TI *__restrict__ P, long long ld,
-                                           const TI *__restrict__ vec, int i0, int r0, int I, int R, int tid)
+// transposed on its way in.  8 contiguous elements per thread, two 16-byte loads when the run is inside the matrix and aligned.
+template <bool RC, int TX>
+__device__ __forceinline__ void ob_tg_load(float (*S)[OB_TG_PITCH], const float *__restrict__ P, long long ld, const float *__restrict__ vec,
+                                           int i0, int r0, int I, int R, int tid)
 {
-    TI v[8];
+    float v[8];
     int gi, gr;
     if (RC) { gi = i0 + (tid >> 2); gr = r0 + (tid & 3) * 8; }
     else { gr = r0 + (tid >> 3); gi = i0 + (tid & 7) * 8; }
-    const TI *p = RC ? P + (long long)gi * ld + gr : P + (long long)gr * ld + gi;
+    const float *p = RC ? P + (long long)gi * ld + gr : P + (long long)gr * ld + gi;
     const bool inside = RC ? (gi < I && gr + 8 <= R) : (gr < R && gi + 8 <= I);
     if (inside && ((uintptr_t)p % 16) == 0) {
-        if (sizeof(TI) == 2) {
-            *reinterpret_cast<ob_u32x4 *>(v) = *reinterpret_cast<const ob_u32x4 *>(p);
-        } else {
-            reinterpret_cast<ob_u32x4 *>(v)[0] = reinterpret_cast<const ob_u32x4 *>(p)[0];
-            reinterpret_cast<ob_u32x4 *>(v)[1] = reinterpret_cast<const ob_u32x4 *>(p)[1];
-        }
+        reinterpret_cast<ob_u32x4 *>(v)[0] = reinterpret_cast<const ob_u32x4 *>(p)[0];
+        reinterpret_cast<ob_u32x4 *>(v)[1] = reinterpret_cast<const ob_u32x4 *>(p)[1];
     } else {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             const bool ok = RC ? (gi < I && gr + e < R) : (gr < R && gi + e < I);
-            v[e] = ok ? p[e] : (TI)0;
+            v[e] = ok ? p[e] : 0.f;
         }
     }
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
         const int ei = RC ? gi : gi + e, er = RC ? gr + e : gr;
-        if (TX == OB_TX_SIGN) v[e] = ob_tg_sign<TI>(v[e]);
-        if (TX == OB_TX_SCALE_R) v[e] = (ei < I && er < R) ? (TI)(v[e] * vec[er]) : (TI)0;
-        if (TX == OB_TX_SCALE_I) v[e] = (ei < I && er < R) ? (TI)(v[e] * vec[ei]) : (TI)0;
+        if (TX == OB_TX_SIGN) v[e] = ob_tg_sign<float>(v[e]);
+        if (TX == OB_TX_SCALE_R) v[e] = (ei < I && er < R) ? v[e] * vec[er] : 0.f;
+        if (TX == OB_TX_SCALE_I) v[e] = (ei < I && er < R) ? v[e] * vec[ei] : 0.f;
     }
     if (RC) {
-        TI *d = &S[tid >> 2][(tid & 3) * 8];
-        if (sizeof(TI) == 2) *reinterpret_cast<ob_u32x4 *>(d) = *reinterpret_cast<ob_u32x4 *>(v);
-        else { reinterpret_cast<ob_u32x4 *>(d)[0] = reinterpret_cast<ob_u32x4 *>(v)[0]; reinterpret_cast<ob_u32x4 *>(d)[1] = reinterpret_cast<ob_u32x4 *>(v)[1]; }
+        float *d = &S[tid >> 2][(tid & 3) * 8];
+        reinterpret_cast<ob_u32x4 *>(d)[0] = reinterpret_cast<ob_u32x4 *>(v)[0];
+        reinterpret_cast<ob_u32x4 *>(d)[1] = reinterpret_cast<ob_u32x4 *>(v)[1];
     } else {
 #pragma unroll
         for (int e = 0; e < 8; ++e) S[(tid & 7) * 8 + e][tid >> 3] = v[e];
     }
 }
 
-template <typename TI, bool RCA, bool RCB, int TXA, int TXB, int EPI>
+template <bool RCA, bool RCB, int TXA, int TXB, int EPI>
 __global__ __launch_bounds__(OB_TG_THREADS) void ob_tgemm_kernel(const ObTGemmArgs a)
 {
-    constexpr int PITCH = ObTgT<TI>::PITCH;
-    __shared__ __attribute__((aligned(16))) TI As[OB_TG_BM][PITCH];
-    __shared__ __attribute__((aligned(16))) TI Bs[OB_TG_BN][PITCH];
+    __shared__ __attribute__((aligned(16))) float As[OB_TG_BM][OB_TG_PITCH];
+    __shared__ __attribute__((aligned(16))) float Bs[OB_TG_BN][OB_TG_PITCH];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave & 1, wn = wave >> 1;
     const int i0 = blockIdx.y * OB_TG_BM, j0 = blockIdx.x * OB_TG_BN;
@@ -103,18 +95,18 @@ __global__ __launch_bounds__(OB_TG_THREADS) void ob_tgemm_kernel(const ObTGemmAr
     for (int x = 0; x < 2; ++x)
 #pragma unroll
         for (int y = 0; y < 2; ++y) acc[x][y] = (ob_float4){0.f, 0.f, 0.f, 0.f};
-    const TI *A = (const TI *)a.A, *B = (const TI *)a.B;
+    const float *A = (const float *)a.A, *B = (const float *)a.B;
     for (int r0 = 0; r0 < a.R; r0 += OB_TG_BR) {
-        ob_tg_load<TI, RCA, TXA>(As, A, a.lda, (const TI *)a.va, i0, r0, a.M, a.R, tid);
-        ob_tg_load<TI, RCB, TXB>(Bs, B, a.ldb, (const TI *)a.vb, j0, r0, a.N, a.R, tid);
+        ob_tg_load<RCA, TXA>(As, A, a.lda, (const float *)a.va, i0, r0, a.M, a.R, tid);
+        ob_tg_load<RCB, TXB>(Bs, B, a.ldb, (const float *)a.vb, j0, r0, a.N, a.R, tid);
         __syncthreads();
 #pragma unroll
         for (int kk = 0; kk < OB_TG_BR; kk += 4) {
             float fa[2], fb[2];
 #pragma unroll
             for (int x = 0; x < 2; ++x) {
-                fa[x] = (float)As[wm * 32 + x * 16 + lr][kk + lg];
-                fb[x] = (float)Bs[wn * 32 + x * 16 + lr][kk + lg];
+                fa[x] = As[wm * 32 + x * 16 + lr][kk + lg];
+                fb[x] = Bs[wn * 32 + x * 16 + lr][kk + lg];
             }
 #pragma unroll
             for (int x = 0; x < 2; ++x)
@@ -123,8 +115,8 @@ __global__ __launch_bounds__(OB_TG_THREADS) void ob_tgemm_kernel(const ObTGemmAr
         }
         __syncthreads();
     }
-    TI *C = (TI *)a.C, *C2 = (TI *)a.C2;
-    const TI *vc = (const TI *)a.vc;
+    float *C = (float *)a.C, *C2 = (float *)a.C2;
+    const float *vc = (const float *)a.vc;
 #pragma unroll
     for (int x = 0; x < 2; ++x) {
         const int m = i0 + wm * 32 + x * 16 + lr;
@@ -136,17 +128,12 @@ __global__ __launch_bounds__(OB_TG_THREADS) void ob_tgemm_kernel(const ObTGemmAr
             for (int e = 0; e < 4; ++e) {
                 if (n + e >= a.N) continue;
                 const long long o = (long long)m * a.ldc + n + e;
-                const TI c = (TI)acc[x][y][e];
+                const float c = acc[x][y][e];
                 if (EPI == OB_TE_PLAIN) C[o] = c;
-                if (EPI == OB_TE_GX) { C[o] = c; C2[o] = (TI)(c * vc[n + e]); }
-                if (EPI == OB_TE_STE) {
-                    // SignSTEFunc.backward (bitnet.py:22-23): grad * (1.001 - tanh(w) ** 2) as TENSOR ops in the tensor
-                    // dtype -- tanh, the square, the subtraction (the scalar 1.001 becomes TI: 1.000977 in fp16) and the
-                    // product each round once to TI
-                    const TI t = (TI)tanhf((float)vc[o]);
-                    const TI t2 = (TI)((float)t * (float)t);
-                    const TI f = (TI)((float)(TI)1.001f - (float)t2);
-                    C[o] = (TI)((float)c * (float)f);
+                if (EPI == OB_TE_GX) { C[o] = c; C2[o] = c * vc[n + e]; }
+                if (EPI == OB_TE_STE) {                                // SignSTEFunc.backward (bitnet.py:22-23): grad * (1.001 - tanh(w) ** 2)
+                    const float w = tanhf(vc[o]);
+                    C[o] = c * (1.001f - w * w);
                 }
             }
         }
@@ -275,37 +262,35 @@ __global__ __launch_bounds__(256) void ob_train_ln_fwd_kernel(const TI *__restri
 // backward through the LayerNorm and the * g: with uh = (u - mean) * rstd,
 //   gu = rstd * (gy - mean_n(gy) - uh * mean_n(gy * uh));   gz = gu * g
 // rowc[t] = {mean_n(gy), mean_n(gy * uh)} is kept for the column reductions (gg needs gu again).
-template <typename TI>
-__global__ __launch_bounds__(256) void ob_train_ln_bwd_kernel(const TI *__restrict__ gy, const TI *__restrict__ z, const TI *__restrict__ g,
-                                                              const float *__restrict__ stats, TI *__restrict__ gz, float *__restrict__ rowc, int N)
+__global__ __launch_bounds__(256) void ob_train_ln_bwd_kernel(const float *__restrict__ gy, const float *__restrict__ z, const float *__restrict__ g,
+                                                              const float *__restrict__ stats, float *__restrict__ gz, float *__restrict__ rowc, int N)
 {
     __shared__ float red[8];
     const int t = blockIdx.x;
-    const TI *zr = z + (long long)t * N, *gr = gy + (long long)t * N;
+    const float *zr = z + (long long)t * N, *gr = gy + (long long)t * N;
     const float mean = stats[2 * t], rstd = stats[2 * t + 1];
     float s1 = 0.f, s2 = 0.f;
     for (int n = threadIdx.x; n < N; n += 256) {
-        const float uh = ((float)(TI)(zr[n] * g[n]) - mean) * rstd, d = (float)gr[n];
+        const float uh = (zr[n] * g[n] - mean) * rstd, d = gr[n];
         s1 += d; s2 += d * uh;
     }
     const float c1 = ob_block_sum(s1, red) / (float)N;
     const float c2 = ob_block_sum(s2, red) / (float)N;
     for (int n = threadIdx.x; n < N; n += 256) {
-        const float uh = ((float)(TI)(zr[n] * g[n]) - mean) * rstd;
-        const TI gu = (TI)(rstd * ((float)gr[n] - c1 - uh * c2));
-        gz[(long long)t * N + n] = (TI)(gu * g[n]);
+        const float uh = (zr[n] * g[n] - mean) * rstd;
+        const float gu = rstd * (gr[n] - c1 - uh * c2);
+        gz[(long long)t * N + n] = gu * g[n];
     }
     if (threadIdx.x == 0) { rowc[2 * t] = c1; rowc[2 * t + 1] = c2; }
 }
 
-// Column sums over the tokens, in two deterministic stages (round 4; one 64-column block walking all T rows took 0.45 / 0.30 ms of a
+// Column sums over the tokens, in two deterministic stages (one 64-column block walking all T rows took 0.45 / 0.30 ms of a
 // 3.3 ms layer step): stage 1 -- block (column block, token slice s of OB_TC_SLICES) accumulates its rows in fp32 and writes
-// part[s][column]; stage 2 -- one thread per column adds the slices in order and rounds once to the tensor dtype.
+// part[s][column]; stage 2 -- one thread per column adds the slices in order.
 //   gg[n] = sum_t gu[t, n] * z[t, n], gbias[n] = sum_t gy[t, n]      (gu: the LayerNorm backward of ob_train_ln_bwd_kernel, recomputed)
 //   gh[k] = sum_t ga[t, k] * x[t, k]
 #define OB_TC_SLICES 32
-template <typename TI>
-__global__ __launch_bounds__(256) void ob_train_cols_ln_kernel(const TI *__restrict__ gy, const TI *__restrict__ z, const TI *__restrict__ g,
+__global__ __launch_bounds__(256) void ob_train_cols_ln_kernel(const float *__restrict__ gy, const float *__restrict__ z, const float *__restrict__ g,
                                                                const float *__restrict__ stats, const float *__restrict__ rowc,
                                                                float *__restrict__ part, int T, int N)
 {
@@ -314,13 +299,13 @@ __global__ __launch_bounds__(256) void ob_train_cols_ln_kernel(const TI *__restr
     const int per = (T + OB_TC_SLICES - 1) / OB_TC_SLICES, t0 = blockIdx.y * per, t1 = min(T, t0 + per);
     float a0 = 0.f, a1 = 0.f;
     if (n < N) {
-        const float gn = (float)g[n];
+        const float gn = g[n];
         for (int t = t0 + rl; t < t1; t += 4) {
             const float mean = stats[2 * t], rstd = stats[2 * t + 1], c1 = rowc[2 * t], c2 = rowc[2 * t + 1];
-            const TI zz = z[(long long)t * N + n];
-            const float uh = ((float)(TI)(zz * (TI)gn) - mean) * rstd, d = (float)gy[(long long)t * N + n];
-            const TI gu = (TI)(rstd * (d - c1 - uh * c2));
-            a0 += (float)gu * (float)zz;
+            const float zz = z[(long long)t * N + n];
+            const float uh = (zz * gn - mean) * rstd, d = gy[(long long)t * N + n];
+            const float gu = rstd * (d - c1 - uh * c2);
+            a0 += gu * zz;
             a1 += d;
         }
     }
@@ -332,23 +317,22 @@ __global__ __launch_bounds__(256) void ob_train_cols_ln_kernel(const TI *__restr
     }
 }
 
-template <typename TI>
-__global__ __launch_bounds__(256) void ob_train_cols_gh_kernel(const TI *__restrict__ ga, const TI *__restrict__ x, float *__restrict__ part, int T, int K)
+__global__ __launch_bounds__(256) void ob_train_cols_gh_kernel(const float *__restrict__ ga, const float *__restrict__ x, float *__restrict__ part, int T, int K)
 {
     __shared__ float sm[4][64];
     const int c = threadIdx.x & 63, rl = threadIdx.x >> 6, k = blockIdx.x * 64 + c;
     const int per = (T + OB_TC_SLICES - 1) / OB_TC_SLICES, t0 = blockIdx.y * per, t1 = min(T, t0 + per);
     float a0 = 0.f;
     if (k < K)
-        for (int t = t0 + rl; t < t1; t += 4) a0 += (float)(TI)(ga[(long long)t * K + k] * x[(long long)t * K + k]);
+        for (int t = t0 + rl; t < t1; t += 4) a0 += ga[(long long)t * K + k] * x[(long long)t * K + k];
     sm[rl][c] = a0;
     __syncthreads();
     if (rl == 0 && k < K) part[(size_t)blockIdx.y * K + k] = (sm[0][c] + sm[1][c]) + (sm[2][c] + sm[3][c]);
 }
 
-// stage 2: out_j[c] = TI(sum over slices of part[s][j][c]), j < NOUT (out_1 may be null)
-template <typename TI, int NOUT>
-__global__ __launch_bounds__(256) void ob_train_cols_finish_kernel(const float *__restrict__ part, TI *__restrict__ out0, TI *__restrict__ out1, int C)
+// stage 2: out_j[c] = sum over slices of part[s][j][c], j < NOUT (out_1 may be null)
+template <int NOUT>
+__global__ __launch_bounds__(256) void ob_train_cols_finish_kernel(const float *__restrict__ part, float *__restrict__ out0, float *__restrict__ out1, int C)
 {
     const int c = blockIdx.x * 256 + threadIdx.x;
     if (c >= C) return;
@@ -356,7 +340,7 @@ __global__ __launch_bounds__(256) void ob_train_cols_finish_kernel(const float *
     for (int j = 0; j < NOUT; ++j) {
         float a = 0.f;
         for (int sl = 0; sl < OB_TC_SLICES; ++sl) a += part[((size_t)sl * NOUT + j) * C + c];
-        TI *o = j == 0 ? out0 : out1;
-        if (o) o[c] = (TI)a;
+        float *o = j == 0 ? out0 : out1;
+        if (o) o[c] = a;
     }
 }

@@ -6,11 +6,11 @@
 #include "ob_train16.h"
 
 // onebit_train_forward / onebit_train_backward: bitnet.py:14-28 (SignSTE) and :58-68 (BitLinear.forward)
-template <typename TI, bool RCA, bool RCB, int TXA, int TXB, int EPI>
+template <bool RCA, bool RCB, int TXA, int TXB, int EPI>
 static void ob_launch_tgemm(const ObTGemmArgs &a, hipStream_t s)
 {
     const dim3 grid((unsigned)((a.N + OB_TG_BN - 1) / OB_TG_BN), (unsigned)((a.M + OB_TG_BM - 1) / OB_TG_BM));
-    hipLaunchKernelGGL((ob_tgemm_kernel<TI, RCA, RCB, TXA, TXB, EPI>), grid, dim3(OB_TG_THREADS), 0, s, a);
+    hipLaunchKernelGGL((ob_tgemm_kernel<RCA, RCB, TXA, TXB, EPI>), grid, dim3(OB_TG_THREADS), 0, s, a);
 }
 
 static size_t ob_train_align(size_t b) { return (b + 255) & ~(size_t)255; }
@@ -162,7 +162,7 @@ static int ob_train_forward_t(const void *x, const void *w, const void *h, const
         ob_set_max_lds_once(ob_tgemm128_f16_kernel, attr_set, OB_TG2_LDS);
         hipLaunchKernelGGL(ob_tgemm128_f16_kernel, dim3((unsigned)((N + OB_TG2_B - 1) / OB_TG2_B), (unsigned)((T + OB_TG2_B - 1) / OB_TG2_B)), dim3(OB_TG_THREADS),
                            OB_TG2_LDS, s, a);
-    } else ob_launch_tgemm<TI, true, true, OB_TX_SCALE_R, OB_TX_SIGN, OB_TE_PLAIN>(a, s);
+    } else ob_launch_tgemm<true, true, OB_TX_SCALE_R, OB_TX_SIGN, OB_TE_PLAIN>(a, s);
     int rc = ob_launch_status("train_forward(gemm)");
     if (rc) return rc;
     hipLaunchKernelGGL((ob_train_ln_fwd_kernel<TI>), dim3((unsigned)T), dim3(256), 0, s, (const TI *)z, (const TI *)g, (const TI *)bias,
@@ -194,22 +194,21 @@ extern "C" int onebit_train_forward(const void *x, const void *w_latent, const v
     return onebit_train_forward_ws(x, w_latent, h, g, bias_or_null, y, z_save, ln_stats, nullptr, 0, T, K, N, dtype, ln_eps, stream);
 }
 
-template <typename TI>
-static int ob_train_backward_t(const void *gy, const void *x, const void *w, const void *h, const void *g, const void *z,
-                               const float *stats, void *gx, void *gw, void *gh, void *gg, void *gbias, char *ws,
-                               int64_t T, int64_t K, int64_t N, hipStream_t s)
+static int ob_train_backward_f32(const void *gy, const void *x, const void *w, const void *h, const void *g, const void *z,
+                                 const float *stats, void *gx, void *gw, void *gh, void *gg, void *gbias, char *ws,
+                                 int64_t T, int64_t K, int64_t N, hipStream_t s)
 {
-    TI *gz = (TI *)ws;
-    TI *ga = (TI *)(ws + ob_train_align((size_t)T * N * sizeof(TI)));
-    float *rowc = (float *)(ws + ob_train_align((size_t)T * N * sizeof(TI)) + ob_train_align((size_t)T * K * sizeof(TI)));
+    float *gz = (float *)ws;
+    float *ga = (float *)(ws + ob_train_align((size_t)T * N * sizeof(float)));
+    float *rowc = (float *)(ws + ob_train_align((size_t)T * N * sizeof(float)) + ob_train_align((size_t)T * K * sizeof(float)));
     float *part = (float *)((char *)rowc + ob_train_align((size_t)T * 2 * sizeof(float)));     // [OB_TC_SLICES][2 N | K] column-sum partials
     int rc;
     // 1. through the LayerNorm and * g: gz [T, N]; column sums gg, gbias
-    hipLaunchKernelGGL((ob_train_ln_bwd_kernel<TI>), dim3((unsigned)T), dim3(256), 0, s, (const TI *)gy, (const TI *)z, (const TI *)g, stats, gz, rowc, (int)N);
+    hipLaunchKernelGGL(ob_train_ln_bwd_kernel, dim3((unsigned)T), dim3(256), 0, s, (const float *)gy, (const float *)z, (const float *)g, stats, gz, rowc, (int)N);
     if ((rc = ob_launch_status("train_backward(layernorm)"))) return rc;
-    hipLaunchKernelGGL((ob_train_cols_ln_kernel<TI>), dim3((unsigned)((N + 63) / 64), OB_TC_SLICES), dim3(256), 0, s, (const TI *)gy, (const TI *)z, (const TI *)g, stats,
+    hipLaunchKernelGGL(ob_train_cols_ln_kernel, dim3((unsigned)((N + 63) / 64), OB_TC_SLICES), dim3(256), 0, s, (const float *)gy, (const float *)z, (const float *)g, stats,
                        (const float *)rowc, part, (int)T, (int)N);
-    hipLaunchKernelGGL((ob_train_cols_finish_kernel<TI, 2>), dim3((unsigned)((N + 255) / 256)), dim3(256), 0, s, (const float *)part, (TI *)gg, (TI *)gbias, (int)N);
+    hipLaunchKernelGGL(ob_train_cols_finish_kernel<2>, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, s, (const float *)part, (float *)gg, (float *)gbias, (int)N);
     if ((rc = ob_launch_status("train_backward(gg)"))) return rc;
     // 2. ga [T, K] = gz . sign(W);  gx = ga * h;  gh = sum_t ga * x
     {
@@ -217,10 +216,10 @@ static int ob_train_backward_t(const void *gy, const void *x, const void *w, con
         a.A = gz; a.lda = N;                 // A(t, n) = gz[t, n]            (n contiguous)
         a.B = w; a.ldb = K;                  // B(k, n) = sign(W[n, k])        (k = output index, contiguous)
         a.C = ga; a.C2 = gx; a.vc = h; a.ldc = K; a.M = (int)T; a.N = (int)K; a.R = (int)N;
-        ob_launch_tgemm<TI, true, false, OB_TX_NONE, OB_TX_SIGN, OB_TE_GX>(a, s);
+        ob_launch_tgemm<true, false, OB_TX_NONE, OB_TX_SIGN, OB_TE_GX>(a, s);
         if ((rc = ob_launch_status("train_backward(grad input)"))) return rc;
-        hipLaunchKernelGGL((ob_train_cols_gh_kernel<TI>), dim3((unsigned)((K + 63) / 64), OB_TC_SLICES), dim3(256), 0, s, (const TI *)ga, (const TI *)x, part, (int)T, (int)K);
-        hipLaunchKernelGGL((ob_train_cols_finish_kernel<TI, 1>), dim3((unsigned)((K + 255) / 256)), dim3(256), 0, s, (const float *)part, (TI *)gh, (TI *)nullptr, (int)K);
+        hipLaunchKernelGGL(ob_train_cols_gh_kernel, dim3((unsigned)((K + 63) / 64), OB_TC_SLICES), dim3(256), 0, s, (const float *)ga, (const float *)x, part, (int)T, (int)K);
+        hipLaunchKernelGGL(ob_train_cols_finish_kernel<1>, dim3((unsigned)((K + 255) / 256)), dim3(256), 0, s, (const float *)part, (float *)gh, (float *)nullptr, (int)K);
         if ((rc = ob_launch_status("train_backward(gh)"))) return rc;
     }
     // 3. gW [N, K] = (gz^T . (x * h)) * (1.001 - tanh(W)^2)
@@ -229,7 +228,7 @@ static int ob_train_backward_t(const void *gy, const void *x, const void *w, con
         a.A = gz; a.lda = N;                 // A(n, t) = gz[t, n]            (n = output index, contiguous)
         a.B = x; a.ldb = K; a.vb = h;        // B(k, t) = x[t, k] * h[k]      (k = output index, contiguous)
         a.C = gw; a.vc = w; a.ldc = K; a.M = (int)N; a.N = (int)K; a.R = (int)T;
-        ob_launch_tgemm<TI, false, false, OB_TX_NONE, OB_TX_SCALE_I, OB_TE_STE>(a, s);
+        ob_launch_tgemm<false, false, OB_TX_NONE, OB_TX_SCALE_I, OB_TE_STE>(a, s);
         if ((rc = ob_launch_status("train_backward(grad weight)"))) return rc;
     }
     return 0;
@@ -249,6 +248,6 @@ extern "C" int onebit_train_backward(const void *gy, const void *x, const void *
         return ob_fail(ONEBIT_E_WSPACE, "train_backward: needs %zu bytes of 16-byte aligned workspace", onebit_train_workspace_bytes(T, K, N, dtype));
     hipStream_t s = (hipStream_t)stream;
     return dtype == ONEBIT_F16 ? ob_t16_backward(gy, x, w_latent, h, g, z_save, ln_stats, gx, gw, gh, gg, gbias_or_null, (char *)workspace, T, K, N, s)
-                               : ob_train_backward_t<float>(gy, x, w_latent, h, g, z_save, ln_stats, gx, gw, gh, gg, gbias_or_null, (char *)workspace, T, K, N, s);
+                               : ob_train_backward_f32(gy, x, w_latent, h, g, z_save, ln_stats, gx, gw, gh, gg, gbias_or_null, (char *)workspace, T, K, N, s);
 }
 
