@@ -51,8 +51,10 @@ def test_rows_against_64_bits(T, K, N):
     _check(m, torch.randn(T, K, generator=g, device="cuda"))
 
 
-# K in and out of whole quads of 256 columns, N at and off the 128-column blocks, odd pitches, wide rows (row pass of its own beyond 16384)
-@pytest.mark.parametrize("K,N,pitch", [(8, 4, 0), (248, 124, 0), (264, 132, 0), (1376, 4100, 0), (512, 128, 16), (512, 128, 3), (520, 12292, 1), (256, 16384, 0), (256, 16388, 0), (13824, 5120, 0)])
+# K in and out of whole quads of 256 columns, N at and off the 128-column blocks, other pitches (odd ones with columns left over), wide rows (row pass of
+# its own beyond 16384); at the largest T all of them take the matrix cores, whole quads with an odd pitch the general kernel
+@pytest.mark.parametrize("K,N,pitch", [(8, 4372, 0), (248, 1004, 0), (264, 2052, 0), (1376, 4100, 0), (512, 128, 16), (512, 128, 3), (1000, 3004, 3), (520, 12292, 1),
+                                       (256, 16384, 0), (256, 16388, 0), (13824, 5120, 0)])
 @pytest.mark.parametrize("T", [3, 70, 1030])
 def test_columns_against_64_bits(T, K, N, pitch):
     m, g = _layer(K, N, K + N, True, pitch)

@@ -76,20 +76,54 @@ def test_dense_product(T, dtype):
             assert float((z.double().sum(0) - ref).abs().max()) < 1e-5 * K, (N, nkt, s)
 
 
-def test_dense_product_large_tiles():
-    """The 256 x 256 tiles (enough of them to fill the chip), a ragged last row block and the fp32 accumulation over a long K."""
+# forms of many rows: 256-column tiles (rounds of them, split K, few and many k tiles), one a CU, 128-column tiles resident two to a CU, one round and several
+# (N, T, k tiles, splits); the last columns' and rows' tiles are partly filled
+@pytest.mark.parametrize("N,T,nkt,splits", [(8224, 4001, 49, 1), (8224, 4001, 1, 1), (8224, 4001, 2, 1), (2064, 1999, 49, 7), (4112, 1900, 49, 1), (4112, 1900, 1, 1),
+                                            (4112, 1300, 49, 1), (4112, 1300, 3, 1), (2064, 300, 64, 4), (4112, 3599, 49, 1), (1040, 5000, 10, 1)])
+def test_dense_product_large_tiles(N, T, nkt, splits):
     from onebit_amd import _lib
     from onebit_amd.hybrid import pack_fragments
-    lib = _lib.load_hybrid()
-    N, T, K = 4112, 3599, 1568
-    w, a = torch.randn(N, K, device="cuda").to(BF), torch.randn(T, K, device="cuda").to(BF)
-    wp, ap = pack_fragments(w, BF), torch.zeros(3840 // 16, K // 32, 64, 8, dtype=BF, device="cuda")
+    lib, K = _lib.load_hybrid(), 32 * nkt
+    g = torch.Generator(device="cuda").manual_seed(N + T + nkt)
+    w, a = torch.randn(N, K, generator=g, device="cuda").to(BF), torch.randn(T, K, generator=g, device="cuda").to(BF)
+    wp, ap = pack_fragments(w, BF), torch.zeros(-(-T // 256) * 16, nkt, 64, 8, dtype=BF, device="cuda")
     ap[:-(-T // 16)] = pack_fragments(a, BF)
-    z = torch.full((T, N), float("nan"), device="cuda")
-    _lib.check_hybrid(lib.onebit_hybrid_gemm(wp.data_ptr(), ap.data_ptr(), z.data_ptr(), 2, N // 16, K // 32, T, 1, torch.cuda.current_stream().cuda_stream), "gemm")
+    z = torch.full((splits, T, N), float("nan"), device="cuda")
+    _lib.check_hybrid(lib.onebit_hybrid_gemm(wp.data_ptr(), ap.data_ptr(), z.data_ptr(), 2, N // 16, nkt, T, splits, torch.cuda.current_stream().cuda_stream), "gemm")
     torch.cuda.synchronize()
     ref = a.float() @ w.float().t()
-    assert float((z - ref).abs().max()) < 1e-4 * K ** 0.5
+    assert float((z.sum(0) - ref).abs().max()) < 1e-4 * K ** 0.5
+
+
+# few rows with eight k tiles in flight per wave (from 61 k tiles a split on), every remainder of a wave's share; the others beside them
+@pytest.mark.parametrize("T", [1, 7, 16, 17])
+@DTYPES
+def test_dense_product_long_sums(T, dtype):
+    from onebit_amd import _lib
+    from onebit_amd.hybrid import k_tile, pack_fragments
+    lib, g = _lib.load_hybrid(), torch.Generator(device="cuda").manual_seed(T)
+    for nkt, splits in ((60, 1), (61, 1), (62, 1), (63, 1), (64, 1), (65, 1), (66, 1), (67, 1), (68, 1), (93, 1), (122, 2), (127, 1), (195, 3), (200, 1), (244, 4)):
+        N, K = 80, nkt * k_tile(dtype)
+        w, a = torch.randn(N, K, generator=g, device="cuda").to(dtype), torch.randn(T, K, generator=g, device="cuda").to(dtype)
+        wp, ap = pack_fragments(w, dtype), pack_fragments(a, dtype)
+        z = torch.full((splits, T, N), float("nan"), device="cuda")
+        _lib.check_hybrid(lib.onebit_hybrid_gemm(wp.data_ptr(), ap.data_ptr(), z.data_ptr(), 2 if dtype == BF else 1, N // 16, nkt, T, splits,
+                                                 torch.cuda.current_stream().cuda_stream), "gemm")
+        torch.cuda.synchronize()
+        # (fp32 sums of K products of unit variance: half an ulp of a running sum of sqrt(K) per addition, sqrt(K) of them)
+        assert float((z.double().sum(0) - a.double() @ w.double().t()).abs().max()) < 2 ** -22 * K, (nkt, splits)
+
+
+@DTYPES
+def test_few_rows_with_a_shorter_last_split(dtype):
+    """An output product of 8 K splits of 62 k tiles, the last one of fewer (narrow model, wide feed-forward)."""
+    per = 32 if dtype == BF else 16
+    raw = raw_config([att(heads=2, kv_heads=2, dim=16, vdim=16, scale=0.3, ff=per * 490)], width=80, vocab=61, max_positions=64)
+    m, w = build(raw, dtype)
+    eng = m.step_engine(2, 64)
+    for T in (1, 7, 16):
+        toks = tokens(T, 61, T)
+        assert err(run(eng, 0, 0, toks), R.forward(raw, w, toks)) < TOL[dtype], T
 
 
 ATTENTION_SIZES = [dict(heads=4, kv_heads=4, dim=64, vdim=64, scale=0.125), dict(heads=6, kv_heads=2, dim=24, vdim=40, scale=0.4),

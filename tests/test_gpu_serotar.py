@@ -157,7 +157,7 @@ def test_expert_mixture_alone(name, dtype):
 
 
 def test_expert_mixture_in_large_blocks():
-    """Enough rows per expert for the 256-row tiles, more than one split of the output product for few rows."""
+    """Enough rows per expert for several 128-row blocks each, more than one split of the output product for few rows."""
     raw = raw_config([layer(moe(3, 2, 1, (2, 2), 600, 0))], width=512, side=0, vocab=300)
     m, w = build(raw, BF, edit=only("mlp"))
     eng = m.step_engine(1, 1000)
@@ -165,6 +165,43 @@ def test_expert_mixture_in_large_blocks():
         toks = tokens(T, 300, T)
         ref, ok = clear_choices(raw, w, toks)
         assert err(run(eng, 0, 0, toks), ref, ok) < TOL[BF]
+
+
+def test_experts_in_wide_tiles():
+    """Enough blocks of rows that both expert products take 256-column tiles (four per CU and more), partly filled and empty blocks among them.  Only the
+    feed-forward speaks, so a row's logits follow from its token and the one before: a period of tokens stands for all of them."""
+    raw = raw_config([layer(moe(5, 4, 1, None, 920, 0))], width=1848, side=0, vocab=300)
+    m, w = build(raw, BF, edit=only("mlp"))
+    T, P = 4300, 48
+    toks = tokens(P, 300) * (T // P + 1)
+    ref, ok = clear_choices(raw, w, toks[:2 * P])
+    assert float(ok[P:].double().mean()) > 0.3
+    at = torch.tensor([P + t % P for t in range(1, T)])
+    assert err(run(m.step_engine(1, T + 1), 0, 0, toks[:T])[1:], ref[at], ok[at]) < TOL[BF]
+
+
+def test_experts_few_rows_of_long_sums():
+    """From 61 k tiles on a wave of the few-row products keeps eight in flight: both expert products."""
+    raw = raw_config([layer(moe(10, 2, 1, None, 2000, 0))], width=1980, side=0, vocab=300)
+    m, w = build(raw, BF, edit=only("mlp"))
+    eng = m.step_engine(1, 64)
+    for T in (1, 12, 16):
+        toks = tokens(T, 300, T)
+        ref, ok = clear_choices(raw, w, toks)
+        assert ok.any() and err(run(eng, 0, 0, toks), ref, ok) < TOL[BF], T
+
+
+def test_latent_expansion_in_wide_tiles():
+    """Keys and values of several requests expanded in one product of 256-column tiles (31 blocks of 128 positions x 4096 columns)."""
+    raw = raw_config([layer(heads=16, dim=128, vdim=128, q_rank=72, kv_rank=112, scale=0.1)], width=72, side=0)
+    m, w = build(raw, BF, edit=only("mix"))
+    prompts = [tokens(n, 61, n) for n in (1000, 900, 1024, 777)]
+    eng = m.step_engine(4, 1100)
+    eng.launch([(i, 0, p, list(range(len(p)))) for i, p in enumerate(prompts)])
+    row = 0
+    for p in prompts:
+        assert err(eng.logits[row:row + len(p)], R.forward(raw, w, p)) < TOL[BF], len(p)
+        row += len(p)
 
 
 @DTYPES

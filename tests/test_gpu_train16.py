@@ -1,5 +1,6 @@
 """The float16 train-mode layer (csrc/ob_train16.h) against the same formulas in 64 bits, at the edges of its 16- and 32-element tiles, 128-row and
-128- / 256-column blocks, with rows that are not 16-byte aligned.
+128- / 256-column blocks (the wide ones from four per CU on: all three products at 4100 x 8200 x 8216, one each at the sizes after it), with rows
+that are not 16-byte aligned.
 
 Bound: every tensor-level result is rounded to float16 (2^-11 relative) once per operation, at most five of them in a row (x h, z, u, gz, ga,
 gx); roundings of a sum's addends are independent.  A row or column of a result may therefore be off by about 5 x 2^-11 = 2.4e-3 of its 2-norm at the
@@ -52,7 +53,9 @@ def _case(T, K, N, seed, shift=0):
 
 @pytest.mark.parametrize("T,K,N,shift", [
     (1, 32, 64, 0), (31, 33, 32, 0), (32, 64, 31, 0), (33, 31, 130, 0), (127, 160, 129, 0), (128, 256, 256, 0), (129, 257, 255, 0),
-    (200, 1376, 1000, 0), (65, 2050, 1028, 3), (300, 264, 520, 1), (4100, 512, 2056, 0), (1030, 4096, 4160, 0), (96, 1024, 16392, 0)])
+    (200, 1376, 1000, 0), (65, 2050, 1028, 3), (300, 264, 520, 1), (4100, 512, 2056, 0), (1030, 4096, 4160, 0), (96, 1024, 16392, 0),
+    (1, 256, 130, 0), (33, 259, 129, 1), (129, 513, 33, 0),                                              # (smaller ones: the forward of two launches)
+    (4100, 8200, 8216, 0), (8200, 200, 8216, 0), (8216, 8200, 40, 0), (40, 8216, 8200, 1)])              # 256-column blocks, sums of 2-7 steps of 32
 def test_rows_and_columns_against_64_bits(T, K, N, shift):
     m, x, gy = _case(T, K, N, T + K + N, shift)
     y = m(x)
