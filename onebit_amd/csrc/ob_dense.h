@@ -412,9 +412,9 @@ template <typename E, int ROWS, int NB> __device__ __forceinline__ ObDenseSrc ob
     return {(const char *)(j < NB ? A.w : A.a) + ((j < NB ? b.w0 : 0) + band * A.nkt + k_lo) * 1024, (uint32_t)lane * 16};
 }
 
-// bf16: workgroup = 16 NB columns x 16 TB rows, four waves 2 x 2 (ob_mm.h has the loop).  NB = 16, TB = 8, three stages of 24 KB (6016 x 2048 x 9728:
-// 227 us with NB = 8, 208 with 16; 16384 x 11008 x 4096 1237 = 1194 TFLOP/s, fp32 sums written); NB = TB = 8, four stages of 16 KB, where 256-column
-// tiles fill their last round of workgroups worse (tiles_launch; 1520 x 2048 x 4096: 35 us against 57).
+// bf16: workgroup = 16 NB columns x 16 TB rows, four waves 2 x 2 (ob_mm.h has the loop).  NB = 16, TB = 8, three stages of 24 KB (rows x k columns x columns,
+// fp32 sums written: 6016 x 2048 x 9728 231 us with NB = 8, 208 with 16; 16384 x 4096 x 11008 1446 and 1202 = 1229 TFLOP/s); NB = TB = 8, four stages of
+// 16 KB, where 256-column tiles fill their last round of workgroups worse (tiles_launch; 1520 x 4096 x 2048: 36 us against 57).
 template <int EPI, int NB, int TB, int NST, int ROWS = OB_ROWS_ALL>
 __global__ __launch_bounds__(256, 2) void ob_dense_mm_kernel(const typename ObDenseArgsOf<ROWS>::type A)
 {

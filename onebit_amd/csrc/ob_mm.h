@@ -8,14 +8,14 @@
 //   * one barrier a step, between the halves: there every wave has read its last operand of tile k (lgkmcnt 0; the reads were issued half a step
 //     ago) and tile k + 1 has landed (counted vmcnt), so tile k's buffer takes tile k + NST
 //   * the MFMAs accumulate in place in AGPRs by inline assembly: with the builtin hipcc (ROCm 7.2) rotates accumulators between registers, 150
-//     copies a step of 64 MFMAs (16384 x 11008 x 4096: 1571 us against 1242)
+//     copies a step of 64 MFMAs, a quarter of the time
 #pragma once
 #include "ob_common.h"
 
 // Output tile of workgroup `orig` (of at least nnb * ntb; false: none).  Workgroup ids are dealt round-robin to the 8 XCDs, each with its own L2;
 // every XCD takes a contiguous range of tiles numbered in bands of 8 token blocks, token block fastest: the 32-64 tiles in flight on it are about
-// as many token blocks as weight blocks.  (Token blocks fastest over ALL token blocks, one weight block at a time, reads 3 times as much past the
-// L2: 6016 x 2048 x 9728 270 -> 213 us, 16384 x 11008 x 4096 1465 -> 1177 with the same kernel; bands of 4, 5, 6, 12 are within 2 % of 8.)
+// as many token blocks as weight blocks.  (Rows x k columns x columns, token blocks fastest over ALL token blocks -> in bands of 8, the same kernel: 6016 x
+// 2048 x 9728 224 -> 208 us, 6016 x 2048 x 17920 418 -> 381, 16384 x 4096 x 11008 1229 -> 1202; bands of 4, 5, 6, 12 are within 2 % of 8.)
 __device__ __forceinline__ bool ob_tile_of(int orig, int nnb, int ntb, int &nb, int &tb, int band_of = 8)
 {
     const int nwg = nnb * ntb, xcd = orig & 7, j = orig >> 3, q8 = nwg >> 3, rem = nwg & 7;
