@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """profiles/pmc_traffic.json from a `rocprofv3 --pmc FETCH_SIZE` summary (tools/pmc_summary.py output),
 stamped with the hash of the kernel sources so bench.py only reports it for the code it was taken on.
-Usage: python tools/make_pmc_traffic.py gpurun_out/.../pmc_FETCH_SIZE.txt"""
+Usage: python tools/make_pmc_traffic.py gpurun_out/.../pmc_FETCH_SIZE.txt [what was run, if not bench.py]"""
 import json, os, re, sys
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 sys.path.insert(0, ROOT)
@@ -21,8 +21,8 @@ for line in open(sys.argv[1]):
             out[nm] = int(float(m.group(1)) * 1024 * 2)
     if "ob_dec_lmhead_kernel" in line:
         out["lm_head"] = int(float(m.group(1)) * 1024 * 2)
-json.dump({"source": "rocprofv3 --pmc FETCH_SIZE (own pass) -- python bench.py --steps 8 --warmup 2 --no-cpu-baseline --no-prefill "
-                     "--no-serve --no-roofline; per-kernel averages via tools/pmc_summary.py",
+run = sys.argv[2] if len(sys.argv) > 2 else "rocprofv3 --pmc FETCH_SIZE (own pass) -- python bench.py --steps 8 --warmup 2 --no-cpu-baseline --no-prefill --no-serve --no-roofline"
+json.dump({"source": run + "; per-kernel averages via tools/pmc_summary.py",
            "units": "FETCH_SIZE is reported in KiB; on gfx950 it counts 128-B fabric requests as 64 B for wide coalesced streams "
                     "(MI355X_MICROARCH.md, HBM section), so bytes = FETCH_SIZE * 1024 * 2",
            "csrc_sha": csrc_sha(), "bytes_per_launch": out}, open(os.path.join(ROOT, "profiles", "pmc_traffic.json"), "w"), indent=1)
