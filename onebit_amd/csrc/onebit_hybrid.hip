@@ -106,15 +106,16 @@ static int tiles_launch(const typename ObDenseArgsOf<ROWS>::type &a, int64_t n_t
         hipLaunchKernelGGL(k, dim3((unsigned)(cdiv(a.n_tiles, nb) * n_tb), (unsigned)n_split), dim3(256), lds, s, a);
         return hstatus(what);
     };
-    if constexpr (sizeof(E) == 2) {
-        constexpr bool EXPERTS = ROWS == OB_ROWS_GATHER || ROWS == OB_ROWS_SORTED;
+    constexpr bool EXPERTS = ROWS == OB_ROWS_GATHER || ROWS == OB_ROWS_SORTED;
+    if constexpr (sizeof(E) == 4) return go(ob_dense_tile_kernel<E, EPI, ROWS>, 8, 4 * 16 * 1024);
+    else {
         const int64_t cus = cu_count(), wide = cdiv(a.n_tiles, 16) * n_tb * n_split, narrow = cdiv(a.n_tiles, 8) * n_tb * n_split;
         const bool two = !EXPERTS && narrow > cus && narrow <= 2 * cus;
         if (EXPERTS ? wide >= 4 * cus : two ? 4 * narrow > 7 * cus && wide <= cus : 1.8 * round_cost(wide) < round_cost(narrow))
             return go(ob_dense_mm_kernel<EPI, 16, 8, 3, ROWS>, 16, 3 * 24 * 1024);
-        if (!two) return go(ob_dense_mm_kernel<EPI, 8, 8, 4, ROWS>, 8, 4 * 16 * 1024);
+        if constexpr (!EXPERTS) if (two) return go(ob_dense_tile_kernel<E, EPI, ROWS>, 8, 4 * 16 * 1024);
+        return go(ob_dense_mm_kernel<EPI, 8, 8, 4, ROWS>, 8, 4 * 16 * 1024);
     }
-    return go(ob_dense_tile_kernel<E, EPI, ROWS>, 8, 4 * 16 * 1024);
 }
 
 template <typename E, int EPI>
