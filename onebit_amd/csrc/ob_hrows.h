@@ -3,9 +3,35 @@
 #pragma once
 #include "ob_dense.h"
 
-// s += sum of n partial sums `stride` apart: four in flight, added in order
+// s += sum of n partial sums `stride` apart, added in order, up to eight in flight.  (Splits there are not are fetched again and added as zeros: with a branch
+// around each addition, as below, the compiler fetches the last ones behind it, a second trip to memory.  12 rows of 2048 columns: a decode step's norms
+// 4.7 -> 4.4 us.)
+template <int VEC, int U>
+__device__ __forceinline__ void ob_sum_splits_u(float (&s)[VEC], const float *p, size_t stride, int k, int n)
+{
+    float zv[U][VEC];
+#pragma unroll
+    for (int j = 0; j < U; ++j)
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) zv[j][e] = p[(size_t)min(k + j, n - 1) * stride + e];
+#pragma unroll
+    for (int j = 0; j < U; ++j)
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) s[e] += k + j < n ? zv[j][e] : 0.f;
+}
 template <int VEC>
 __device__ __forceinline__ void ob_sum_splits(float (&s)[VEC], const float *p, size_t stride, int n)
+{
+    if (n == 1) {                                                     // (uniform)
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) s[e] += p[e];
+    } else if (n > 4) {
+        for (int k = 0; k < n; k += 8) ob_sum_splits_u<VEC, 8>(s, p, stride, k, n);
+    } else if (n > 0) ob_sum_splits_u<VEC, 4>(s, p, stride, 0, n);
+}
+// ... of many rows: mostly one split, and other rows fill the waits
+template <int VEC>
+__device__ __forceinline__ void ob_sum_splits_rows(float (&s)[VEC], const float *p, size_t stride, int n)
 {
     for (int k = 0; k < n; k += 4) {
         float zv[4][VEC];
@@ -130,7 +156,7 @@ __global__ __launch_bounds__(1024) void ob_hnorm_rows_kernel(const ObHNormArgs A
         if (c < A.W) {
             r[i] = *reinterpret_cast<const ob_float4 *>(xr + c);
             float s[4] = {0.f, 0.f, 0.f, 0.f};
-            ob_sum_splits<4>(s, A.z + (size_t)src * A.ldz + c, A.z_split, A.n_split);
+            ob_sum_splits_rows<4>(s, A.z + (size_t)src * A.ldz + c, A.z_split, A.n_split);
 #pragma unroll
             for (int e = 0; e < 4; ++e) r[i][e] += A.mult * (A.bias ? s[e] + A.bias[c + e] : s[e]);
             if (A.emb_add) r[i] += *reinterpret_cast<const ob_float4 *>(A.emb_add + (size_t)src * A.W + c);
@@ -364,7 +390,7 @@ __global__ __launch_bounds__(1024) void ob_xrow_rows_kernel(const ObXRowArgs A, 
         if (c < A.W) {
             x[i] = *reinterpret_cast<const ob_float4 *>(xr + c);
             float z[4] = {0.f, 0.f, 0.f, 0.f};
-            if (A.z) ob_sum_splits<4>(z, A.z + (size_t)src * A.ldz + c, A.z_split, A.n_split);
+            if (A.z) ob_sum_splits_rows<4>(z, A.z + (size_t)src * A.ldz + c, A.z_split, A.n_split);
             if (A.bias) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) z[e] += A.bias[c + e];
