@@ -243,54 +243,15 @@ template <typename E> __global__ __launch_bounds__(256) void ob_table_rows_kerne
     if (i < (int64_t)A.T * nv) ob_table_piece<E>(A, (E *)A.act, (int)(i / nv), 4 * (int)(i % nv));
 }
 
-// ---- few rows (T <= 64): weights from HBM straight into the operand registers ------------------------------------------
-// Workgroup = 2 n tiles (32 output columns; a gate / up pair) x all token tiles x one K split; its four waves take a quarter of the
-// split's k tiles each and add up through LDS.  Activations come from L2 (1 KB linear loads).  Bound by the weights' way from HBM.  The next U k tiles
-// (2 KB of weights each) are requested before the current U are multiplied.  DEEP, from 16 k tiles per wave and up to 16 rows on: eight tiles are in
-// flight at every moment, a tile's registers take the eighth next one as soon as it is multiplied (12 rows, 2048 columns: 71 MB of input product
-// 16.7 -> 16.1 us, the router's 5.6 -> 5.1; with 5-8 tiles per wave it is 2-4 % slower).
-// Row-major activations (OB_ROWS_HEADS, OB_ROWS_GATHER): a lane's 16 bytes come from its own row, 64 bytes per row and k tile.
-// Expert blocks: grid.z = entries of the block table (count 0: nothing to do).
-template <typename E, int EPI, int MT, int ROWS = OB_ROWS_ALL, bool DEEP = false>
-__global__ __launch_bounds__(256, MT >= 4 ? 2 : 3) void ob_dense_skinny_kernel(const ObDenseArgs A)
+// Sums of two n tiles over k tiles [k0, k1) of one wave: weights (1 KB tiles from w0, w1 on) straight into the operand registers, activations from ap[m],
+// KSTEP 16-byte pieces from one k tile to the next.
+template <typename E, int MT, int KSTEP, bool DEEP>
+__device__ __forceinline__ void ob_skinny_stream(const typename ObElem<E>::V16 *w0, const typename ObElem<E>::V16 *w1, const typename ObElem<E>::V16 *const (&ap)[MT], int k0, int k1,
+                                                 ob_float4 (&acc)[2][MT])
 {
     typedef typename ObElem<E>::V16 V16;
     constexpr int U = DEEP ? 8 : MT >= 4 ? 2 : 4;
     static_assert(!DEEP || MT == 1, "eight tiles in flight: one token tile");
-    __shared__ ob_float4 red[4][2][MT][64];
-    extern __shared__ __attribute__((aligned(16))) char formed[];      // OB_ROWS_TABLE: [MT][nkt] tiles
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int nt = blockIdx.x * 2, split = blockIdx.y;
-    const int k_lo = split * A.kt_split, k_hi = min(A.nkt, k_lo + A.kt_split);
-    const int per = (k_hi - k_lo + 3) >> 2;
-    const int k0 = k_lo + wave * per, k1 = min(k0 + per, k_hi);
-    int t0 = 0, rows = A.T;
-    size_t wg = 0;
-    if constexpr (ROWS == OB_ROWS_GATHER || ROWS == OB_ROWS_SORTED) {
-        const ObRowBlock b = A.blk[blockIdx.z];
-        if (b.count <= 0) return;                        // (uniform)
-        t0 = b.row0; rows = b.count; wg = (size_t)b.group * A.w_group;
-    }
-    const V16 *w0 = (const V16 *)A.w + (wg + (size_t)nt * A.nkt) * 64 + lane;
-    const V16 *w1 = (const V16 *)A.w + (wg + (size_t)min(nt + 1, A.n_tiles - 1) * A.nkt) * 64 + lane;
-    if constexpr (ROWS == OB_ROWS_TABLE) {
-        const int nv = A.nkt * ObElem<E>::KT / 4;
-        for (int i = tid; i < A.T * nv; i += 256) ob_table_piece<E>(A, (E *)formed, i / nv, 4 * (i % nv));
-        __syncthreads();
-    }
-    // this lane's piece of k tile 0 of every token tile, and the step (in 16 bytes) to the next k tile
-    const V16 *ap[MT];
-    constexpr int KSTEP = ROWS == OB_ROWS_HEADS || ROWS == OB_ROWS_GATHER ? 4 : 64;
-#pragma unroll
-    for (int m = 0; m < MT; ++m) {
-        if constexpr (ROWS == OB_ROWS_HEADS)
-            ap[m] = (const V16 *)((const E *)A.a + (size_t)min(m * 16 + (lane & 15), rows - 1) * A.lda + nt / A.tile_group * A.act_cols) + (lane >> 4);
-        else if constexpr (ROWS == OB_ROWS_GATHER)
-            ap[m] = (const V16 *)((const E *)A.a + (size_t)A.gather[t0 + min(m * 16 + (lane & 15), rows - 1)] * A.lda) + (lane >> 4);
-        else if constexpr (ROWS == OB_ROWS_TABLE) ap[m] = (const V16 *)formed + lane + (size_t)m * A.nkt * 64;
-        else ap[m] = (const V16 *)A.a + lane + (size_t)((t0 >> 4) + m) * A.nkt * 64;
-    }
-    ob_float4 acc[2][MT];
 #pragma unroll
     for (int m = 0; m < MT; ++m) acc[0][m] = acc[1][m] = (ob_float4){0.f, 0.f, 0.f, 0.f};
     if constexpr (DEEP) {
@@ -361,6 +322,55 @@ __global__ __launch_bounds__(256, MT >= 4 ? 2 : 3) void ob_dense_skinny_kernel(c
             }
         }
     }
+}
+
+// ---- few rows (T <= 64): weights from HBM straight into the operand registers ------------------------------------------
+// Workgroup = 2 n tiles (32 output columns; a gate / up pair) x all token tiles x one K split; its four waves take a quarter of the
+// split's k tiles each and add up through LDS.  Activations come from L2 (1 KB linear loads).  Bound by the weights' way from HBM.  The next U k tiles
+// (2 KB of weights each) are requested before the current U are multiplied.  DEEP, from 16 k tiles per wave and up to 16 rows on: eight tiles are in
+// flight at every moment, a tile's registers take the eighth next one as soon as it is multiplied (12 rows, 2048 columns: 71 MB of input product
+// 16.7 -> 16.1 us, the router's 5.6 -> 5.1; with 5-8 tiles per wave it is 2-4 % slower).
+// Row-major activations (OB_ROWS_HEADS, OB_ROWS_GATHER): a lane's 16 bytes come from its own row, 64 bytes per row and k tile.
+// Expert blocks: grid.z = entries of the block table (count 0: nothing to do).
+template <typename E, int EPI, int MT, int ROWS = OB_ROWS_ALL, bool DEEP = false>
+__global__ __launch_bounds__(256, MT >= 4 ? 2 : 3) void ob_dense_skinny_kernel(const ObDenseArgs A)
+{
+    typedef typename ObElem<E>::V16 V16;
+    __shared__ ob_float4 red[4][2][MT][64];
+    extern __shared__ __attribute__((aligned(16))) char formed[];      // OB_ROWS_TABLE: [MT][nkt] tiles
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nt = blockIdx.x * 2, split = blockIdx.y;
+    const int k_lo = split * A.kt_split, k_hi = min(A.nkt, k_lo + A.kt_split);
+    const int per = (k_hi - k_lo + 3) >> 2;
+    const int k0 = k_lo + wave * per, k1 = min(k0 + per, k_hi);
+    int t0 = 0, rows = A.T;
+    size_t wg = 0;
+    if constexpr (ROWS == OB_ROWS_GATHER || ROWS == OB_ROWS_SORTED) {
+        const ObRowBlock b = A.blk[blockIdx.z];
+        if (b.count <= 0) return;                        // (uniform)
+        t0 = b.row0; rows = b.count; wg = (size_t)b.group * A.w_group;
+    }
+    const V16 *w0 = (const V16 *)A.w + (wg + (size_t)nt * A.nkt) * 64 + lane;
+    const V16 *w1 = (const V16 *)A.w + (wg + (size_t)min(nt + 1, A.n_tiles - 1) * A.nkt) * 64 + lane;
+    if constexpr (ROWS == OB_ROWS_TABLE) {
+        const int nv = A.nkt * ObElem<E>::KT / 4;
+        for (int i = tid; i < A.T * nv; i += 256) ob_table_piece<E>(A, (E *)formed, i / nv, 4 * (i % nv));
+        __syncthreads();
+    }
+    // this lane's piece of k tile 0 of every token tile, and the step (in 16 bytes) to the next k tile
+    const V16 *ap[MT];
+    constexpr int KSTEP = ROWS == OB_ROWS_HEADS || ROWS == OB_ROWS_GATHER ? 4 : 64;
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        if constexpr (ROWS == OB_ROWS_HEADS)
+            ap[m] = (const V16 *)((const E *)A.a + (size_t)min(m * 16 + (lane & 15), rows - 1) * A.lda + nt / A.tile_group * A.act_cols) + (lane >> 4);
+        else if constexpr (ROWS == OB_ROWS_GATHER)
+            ap[m] = (const V16 *)((const E *)A.a + (size_t)A.gather[t0 + min(m * 16 + (lane & 15), rows - 1)] * A.lda) + (lane >> 4);
+        else if constexpr (ROWS == OB_ROWS_TABLE) ap[m] = (const V16 *)formed + lane + (size_t)m * A.nkt * 64;
+        else ap[m] = (const V16 *)A.a + lane + (size_t)((t0 >> 4) + m) * A.nkt * 64;
+    }
+    ob_float4 acc[2][MT];
+    ob_skinny_stream<E, MT, KSTEP, DEEP>(w0, w1, ap, k0, k1, acc);
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll

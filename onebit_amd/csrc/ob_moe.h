@@ -54,6 +54,7 @@ __device__ __forceinline__ void ob_route_token(const ObRouteArgs &A, int t, cons
             const int g = group(j);
             const uint32_t mine = gs[g];
             int r = 0;
+#pragma unroll 8
             for (int o = 0; o < A.groups; ++o) r += gs[o] > mine || (gs[o] == mine && o < g);
             if (r >= A.keep) c[j] = -INFINITY;
         }

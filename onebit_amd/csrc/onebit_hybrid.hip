@@ -21,6 +21,7 @@
 #include "ob_ssm.h"
 #include "ob_latent.h"
 #include "ob_moe.h"
+#include "ob_few.h"
 
 static thread_local char g_err[512];
 static int hfail(int code, const char *fmt, ...)
@@ -198,6 +199,8 @@ static int act_index(const HPlan &P, const onebit_hlayer_t &L)
 }
 #define OB_LAT_PARTS 1024       // (row, split) pairs of the latent decode attention with more than one split
 #define OB_SIDE_SPLITS 4        // K splits of a token input's gate product
+#define OB_FEW_SIDE_KT 64       // ... of a layer's end, which has two products
+#define OB_FEW_KT 128           // k tiles of a product in a row kernel (of up to 64 columns)
 #define OB_EZ_ROWS 4096         // fp32 rows of the experts' partial sums at least
 // rows of the experts' sorted space: every (token, choice), each expert's first row at a multiple of 16
 static int64_t expert_rows(const onebit_hff_t &f, int64_t T) { return T * f.top + 16 * std::min<int64_t>(f.experts, T * f.top); }
@@ -688,6 +691,103 @@ static int latent_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, con
     return 0;
 }
 
+// ---- mixtures of experts with few rows (ob_few.h): bf16, up to 64 rows (the skinny products' range), router entries that fit a wave, choices that a wave scans
+// in four rounds of loads, rows that a workgroup holds.  OB_FEW_KT: at 4096 columns (128 k tiles, two rounds of weights) still 1.03 of the separate launches
+static bool few_experts(const onebit_hmodel_t &m, const onebit_hlayer_t &L, int T)
+{
+    const onebit_hff_t &f = L.ff;
+    const int nkt = m.width_pad / 32;
+    return m.dtype == ONEBIT_HYB_BF16 && f.experts && T <= OB_SKINNY_T && m.width % 4 == 0 && m.width <= 4096 && f.experts + f.identity <= 64 && nkt <= OB_FEW_KT &&
+           T * f.top <= 1024;
+}
+// K splits of a few-row product whose launch has `wgs` workgroups of one split
+static int few_splits(int64_t wgs, int nkt, int64_t most)
+{
+    const int64_t s = std::max<int64_t>(1, std::min<int64_t>({cdiv(512, wgs), nkt / 8, most, 8}));
+    return (int)cdiv(nkt, cdiv(nkt, s));
+}
+// the row kernel before them, `a`, with the router; then both products.  What the next row kernel adds goes into `pend`.
+static int few_experts_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, const onebit_hstate_t &st, const HPlan &P, char *ws, const ObXRowArgs &a, ObXRowArgs &pend, hipStream_t s)
+{
+    const onebit_hff_t &f = L.ff;
+    const int T = st.n_rows, w_nkt = m.width_pad / 32, wt = (int)cdiv(m.width, 16);
+    const int64_t TK = (int64_t)T * f.top, live = std::min<int64_t>(f.experts, TK);
+    int32_t *at = (int32_t *)(ws + P.route);
+    ObFewRowArgs r = {};
+    static_cast<ObXRowArgs &>(r) = a;
+    r.p = {f.w_gated_in, w_nkt};                // (the router's rows are the matrix's first)
+    r.route.correction = f.correction;
+    r.route.T = T; r.route.experts = f.experts; r.route.identity = f.identity; r.route.top = f.top; r.route.groups = f.groups; r.route.keep = f.keep;
+    r.route.tok_row = at; at += TK;
+    r.route.tok_w = (float *)at; at += TK;
+    r.route.id_w = (float *)at; at += T;
+    r.sel = at;
+    const int lds = ob_few_row_lds(r);
+    const int n_router = (int)cdiv(f.experts + f.identity, 16);
+    if (n_router == 1) hipLaunchKernelGGL(ob_few_route_kernel<1>, dim3((unsigned)T), dim3(1024), lds, s, r);
+    else if (n_router == 2) hipLaunchKernelGGL(ob_few_route_kernel<2>, dim3((unsigned)T), dim3(1024), lds, s, r);
+    else if (n_router == 3) hipLaunchKernelGGL(ob_few_route_kernel<3>, dim3((unsigned)T), dim3(1024), lds, s, r);
+    else hipLaunchKernelGGL(ob_few_route_kernel<4>, dim3((unsigned)T), dim3(1024), lds, s, r);
+    if (int rc = hstatus("router")) return rc;
+    const int ff = 8 * f.nt_expert, sf = 8 * f.nt_gated;
+    ObFewExpertArgs e = {};
+    e.sel = r.sel; e.T = T; e.top = f.top; e.by_choice = f.experts > TK; e.ldz = 16 * wt;
+    const auto go = [&](auto up, int kt) {
+        constexpr bool UP = decltype(up)::value;
+        const dim3 grid((unsigned)(cdiv(e.s.n_tiles, 2) * e.s.n_split + live * cdiv(e.e.n_tiles, 2) * e.e.n_split));
+        if (T <= 16 && kt >= OB_DEEP_KT) hipLaunchKernelGGL((ob_few_expert_kernel<1, UP, true>), grid, dim3(256), 0, s, e);
+        else if (T <= 16) hipLaunchKernelGGL((ob_few_expert_kernel<1, UP, false>), grid, dim3(256), 0, s, e);
+        else if (T <= 32) hipLaunchKernelGGL((ob_few_expert_kernel<2, UP, false>), grid, dim3(256), 0, s, e);
+        else hipLaunchKernelGGL((ob_few_expert_kernel<4, UP, false>), grid, dim3(256), 0, s, e);
+        return hstatus("expert product");
+    };
+    e.w_group = (size_t)f.nt_expert * w_nkt;
+    e.e = {f.w_expert_in, f.nt_expert, w_nkt, w_nkt, 1, ws + P.hrm, m.width_pad, ws + P.acte, ff, nullptr, 0};
+    e.s = {(const char *)f.w_gated_in + (size_t)f.nt_aux * w_nkt * 1024, f.nt_gated, w_nkt, w_nkt, 1, ws + P.hrm, m.width_pad, ws + P.actf, sf, nullptr, 0};
+    if (int rc = go(std::true_type(), w_nkt)) return rc;
+    const int64_t wgs = (int64_t)cdiv(wt, 2);
+    const int ke = ff / 32, ks = sf / 32, ne = few_splits(wgs * live, ke, OB_EZ_ROWS / TK), per_e = (int)cdiv(ke, ne);
+    const int per_s = std::max(1, (int)cdiv(ks, std::max<int64_t>(1, std::min<int64_t>({cdiv(ks, per_e), 8, OB_ZROWS / T}))));      // (workgroups of a length)
+    e.w_group = (size_t)wt * ke;
+    e.e = {f.w_expert_out, wt, ke, per_e, ne, ws + P.acte, ff, nullptr, 0, (float *)(ws + P.ez), (size_t)TK * e.ldz};
+    e.s = {f.w_gated_out, ks ? wt : 0, ks, per_s, (int)cdiv(ks, per_s), ws + P.actf, sf, nullptr, 0, (float *)(ws + P.z), (size_t)T * e.ldz};
+    if (int rc = go(std::false_type(), e.e.kt_split)) return rc;
+    if (ks) { pend.z = e.s.z; pend.ldz = e.ldz; pend.z_split = e.s.z_split; pend.n_split = e.s.n_split; }
+    pend.ez = e.e.z; pend.ez_split = e.e.z_split; pend.ez_n = ne; pend.ld_ez = e.ldz; pend.top = f.top; pend.tok_row = r.route.tok_row; pend.tok_w = r.route.tok_w;
+    if (f.identity) {
+        pend.id_w = r.route.id_w;
+        if (L.pre2_w) { pend.idh = ws + P.hrm; pend.ld_idh = m.width_pad; }
+    }
+    return 0;
+}
+
+// The end of a sequential layer with few rows, from its feed-forward's products (`a`) to the next layer's operand: ob_few_side_kernel.  Up to 2048 columns and
+// 64 of the token input: every row's workgroup reads both weights whole (512 KB, 3.4 us; 2 MB at 4096 x 128 would be 14, the separate launches take 21)
+static bool few_side(const onebit_hmodel_t &m, const onebit_hlayer_t &L, const onebit_hstate_t &st, const ObXRowArgs &a)
+{
+    return m.dtype == ONEBIT_HYB_BF16 && st.n_rows <= OB_SKINNY_T && m.width % 4 == 0 && m.width <= 4096 && m.width_pad / 32 <= OB_FEW_SIDE_KT &&
+           (L.side.nt == 2 || L.side.nt == 4) && !a.embed && !a.emb_save && !a.emb_add && !a.bias && !a.eo && (!a.top || (a.ez && few_experts(m, L, st.n_rows)));
+}
+static int few_side_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, const onebit_hstate_t &st, const ObXRowArgs &a, const float *next_w, void *out, hipStream_t s)
+{
+    ObFewSideArgs f = {};
+    static_cast<ObXRowArgs &>(f) = a;
+    f.w = next_w; f.out = out;
+    f.p = {L.side.w_gate, m.width_pad / 32};
+    f.q = {L.side.w_proj, L.side.nt / 2};
+    f.table = L.side.table; f.ld_table = m.side_cols; f.dim = L.side.dim; f.side_w = L.side.norm_w;
+    const int lds = ob_few_side_lds(f);
+    const dim3 grid((unsigned)st.n_rows);
+    if (L.side.nt == 2) {
+        if (a.top) hipLaunchKernelGGL((ob_few_side_kernel<OB_X_EXPERTS, 2>), grid, dim3(1024), lds, s, f);
+        else hipLaunchKernelGGL((ob_few_side_kernel<OB_X_PLAIN, 2>), grid, dim3(1024), lds, s, f);
+    } else {
+        if (a.top) hipLaunchKernelGGL((ob_few_side_kernel<OB_X_EXPERTS, 4>), grid, dim3(1024), lds, s, f);
+        else hipLaunchKernelGGL((ob_few_side_kernel<OB_X_PLAIN, 4>), grid, dim3(1024), lds, s, f);
+    }
+    return hstatus("token input");
+}
+
 // the feed-forward of a sequential layer; what the next row kernel adds goes into `pend`
 template <typename E>
 static int ff_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, const onebit_hstate_t &st, const HPlan &P, char *ws, ObXRowArgs &pend, hipStream_t s)
@@ -838,6 +938,7 @@ static int step_impl(const onebit_hmodel_t &m, const onebit_hstate_t &st, const 
         a.emb_save = nullptr;
         return row_launch<E>(a, T, s);
     };
+    bool formed = false;                                              // the layer's operand: by the launch that ended the layer before
     for (int r = 0; r < m.n_runs; ++r) {
         const onebit_hrun_t &run = m.runs[r];
         const onebit_hlayer_t &L = m.layers[run.layer];
@@ -847,7 +948,8 @@ static int step_impl(const onebit_hmodel_t &m, const onebit_hstate_t &st, const 
         ObXRowArgs a = pend;
         a.w = L.norm_w; a.out = ws + P.h;
         if (run.add_embedding) a.emb_add = (const float *)(ws + P.emb0);
-        if (int rc = row_launch<E>(a, T, s)) return rc;
+        if (!formed) if (int rc = row_launch<E>(a, T, s)) return rc;
+        formed = false;
         if (latent) {
             if (int rc = latent_launch<E>(m, L, run, st, P, ws, act, act_nkt, s)) return rc;
         } else {
@@ -871,10 +973,22 @@ static int step_impl(const onebit_hmodel_t &m, const onebit_hstate_t &st, const 
                 a = pend;
                 a.w = L.pre2_w; a.out = ws + P.h;
                 if (f.experts) a.out_rm = ws + P.hrm;
-                if (int rc = row_launch<E>(a, T, s)) return rc;
                 pend = nb;
                 pend.post_w = L.post2_w;
-                if (int rc = ff_launch<E>(m, L, st, P, ws, pend, s)) return rc;
+                if (few_experts(m, L, T)) {
+                    if (int rc = few_experts_launch(m, L, st, P, ws, a, pend, s)) return rc;
+                } else {
+                    if (int rc = row_launch<E>(a, T, s)) return rc;
+                    if (int rc = ff_launch<E>(m, L, st, P, ws, pend, s)) return rc;
+                }
+            }
+            const bool last = r + 1 == m.n_runs;
+            if (L.side.nt && !st.residuals && (last || !m.runs[r + 1].add_embedding) && few_side(m, L, st, pend)) {
+                keep_result(r + 1, L.dwa);
+                if (int rc = few_side_launch(m, L, st, pend, last ? nullptr : m.layers[m.runs[r + 1].layer].norm_w, last ? nullptr : ws + P.h, s)) return rc;
+                pend = nb;                                            // (the row is in x, nothing is pending, the next layer's operand is there)
+                formed = true;
+                continue;
             }
             if (L.side.nt) {
                 a = pend;

@@ -1,0 +1,64 @@
+"""Steps of up to 64 rows of a sequential hybrid decoder (bf16): the row kernels that carry the router's or the token input's products, and the expert
+products that find their rows in the choices, against the plain restatement (oracle/serotar_ref.py, float64).
+
+``TOL``: bf16 activations (2^-9 relative each) through the two layers' dozen products, as in test_gpu_serotar.py; positions at which a choice of experts is
+close are left out (``clear_choices``)."""
+import pytest
+import torch
+
+from oracle import serotar_ref as R
+from test_gpu_serotar import BF, TOL, build, clear_choices, err, rows_err, run, tokens
+from test_serotar_cpu import dense, layer, moe, raw_config
+
+pytestmark = pytest.mark.gpu
+
+# width, mixture, columns of the token input: one and several waves of columns, a last wave that is not full, padded k tiles; router of 1 .. 4 column tiles, the
+# largest (64 entries); more experts than choices; no shared expert; the longest sums of a row kernel's products (64 and 128 k tiles) and one beyond
+FORMS = {"one wave": (64, moe(6, 2, 2, (4, 2), 24, 32), 10), "four tiles": (260, moe(60, 5, 4, (8, 3), 40, 100), 33), "two tiles, no shared": (300, moe(20, 3, 0, None, 72, 0), 32),
+         "full": (2048, moe(32, 6, 8, (8, 4), 64, 128), 64), "router only": (2052, moe(12, 2, 4, (4, 2), 40, 24), 20), "wide router": (4096, moe(30, 4, 2, None, 32, 64), 40),
+         "wider than any": (4100, moe(10, 2, 0, None, 32, 0), 12)}
+
+
+@pytest.mark.parametrize("name", FORMS)
+def test_rows_of_a_step(name):
+    width, mlp, side = FORMS[name]
+    raw = raw_config([layer(mlp), layer(dense(40)), layer(mlp)], width=width, side=side, vocab=130)
+    m, w = build(raw, BF)
+    eng = m.step_engine(2, 80)
+    for T in (1, 2, 16, 17, 33, 64):
+        toks = tokens(T, 130, T)
+        ref, ok = clear_choices(raw, w, toks, 0.04)
+        if bool(ok.any()):
+            assert err(run(eng, 0, 0, toks), ref, ok) < TOL[BF], T
+
+
+def test_decoded_rows_with_idle_ones():
+    """17 requests in a bucket of 20 rows: the idle rows choose no expert and change nothing."""
+    raw = raw_config([layer(moe(12, 3, 4, (4, 2), 40, 64)), layer(moe(12, 3, 4, (4, 2), 40, 64))], width=192, vocab=140)
+    m, w = build(raw, BF)
+    eng = m.step_engine(20, 40)
+    prompts = [tokens(5 + i % 9, 140, i) for i in range(17)]
+    eng.launch([(i, 0, p[:-1]) for i, p in enumerate(prompts)])
+    eng.launch([(i, len(p) - 1, p[-1:]) for i, p in enumerate(prompts)])
+    got, seen = eng.logits[:17].clone(), 0
+    for i, p in enumerate(prompts):
+        ref, ok = clear_choices(raw, w, p, 0.04)
+        if bool(ok[-1]):
+            seen += 1
+            assert float(rows_err(got[i:i + 1], ref[-1:])) < 2 * TOL[BF], i       # (one row against its own rms instead of the whole reference's)
+    assert seen > 4
+
+
+def test_rows_do_not_change_each_other():
+    """A row of a step is the same bits alone, among 15 others and in a step of other order: sums run over a row, whatever its neighbours."""
+    raw = raw_config([layer(moe(12, 3, 4, (4, 2), 40, 64))], width=192, vocab=140)
+    m, _ = build(raw, BF)
+    eng = m.step_engine(16, 40)
+    prompts = [tokens(6, 140, i) for i in range(16)]
+    eng.launch([(i, 0, p) for i, p in enumerate(prompts)])
+    eng.launch([(i, 6, [i + 3]) for i in range(16)])
+    together = eng.logits[:16].clone()
+    eng.launch([(i, 6, [i + 3]) for i in reversed(range(16))])
+    assert torch.equal(eng.logits[:16].flip(0), together)
+    eng.launch([(9, 6, [12])])
+    assert float((eng.logits[0] - together[9]).abs().max()) <= 1e-2 * float(together[9].abs().max())      # (splits of the sums follow the number of rows)
