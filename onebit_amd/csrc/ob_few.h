@@ -3,9 +3,12 @@
 //   ob_few_side_kernel   the row kernel behind its feed-forward, the token input's two products and the row kernel that ends the layer
 //   ob_few_expert_kernel expert products, gate / up or down, of the routed experts and the shared one in one launch; a workgroup finds its expert's
 //                        rows in the choices by itself (no row lists, no block table, no launch that makes them)
+//   ob_few_query_kernel  latent attention from its input product to the absorbed queries: both norms, the cache's new entry, query product, absorbing product
+//   ob_few_value_kernel  the splits of its context together, and the product that makes the heads' outputs of them
 // Rows of the experts' space here are the choices themselves: row t * top + k is choice k of token t.
 #pragma once
 #include "ob_hrows.h"
+#include "ob_latent.h"
 #include "ob_moe.h"
 
 // A row's product with NT n tiles (16 NT <= 64 columns).  The weights depend on nothing: a wave requests its k tiles (nkt / 16 of them, four at a time) before
@@ -407,5 +410,261 @@ __global__ __launch_bounds__(256, MT >= 4 ? 2 : MT == 1 && !DEEP ? 4 : 3) void o
             *reinterpret_cast<ob_float4 *>(z) = v[0];
             if (nt + 1 < P.n_tiles) *reinterpret_cast<ob_float4 *>(z + 16) = v[1];
         }
+    }
+}
+
+// Up to 32 rows of latent attention.  Workgroups [0, 4 H): head b % H, a quarter of its absorbed columns (a head's four on one XCD where H % 8 == 0: they read
+// the same rows of W_uq, and q is computed in all of them: less of a CU's work than two launches); then one per row: the cache's new entry.
+// Eight waves; a wave takes the n tiles wave, wave + 8 .. of the query product and requests its first 24 k tiles before the normalised row is there.
+// 12 rows, 16 heads of 128, ranks 768 and 256: 7.6 us behind an input product of one split (9.9 behind four: every workgroup adds them), for launches of
+// 4.5 (norms) + 4.7 + 4.7.  A head's weights of 384 KB (rank 1536) take longer than the launches: 0.97 of a step.
+struct ObFewQueryArgs : ObLatPrepArgs {
+    int T, H;
+    const void *w_uq, *w_uk;           // [H][kp / 16][cq_nkt] and [H][rp / 16][kp / 32] tiles
+    int kp;
+    void *heads; int d_shift, head_rows;
+};
+static inline int ob_few_query_ld(int cols) { return (cols + 31) / 32 * 32 + 8; }       // elements of a row in LDS: rows in different banks
+static inline int ob_few_query_lds(const ObFewQueryArgs &A, int mt) { return 16 * mt * (ob_few_query_ld(A.q_rank) + ob_few_query_ld(A.kp)) * 2; }
+template <int MT>
+__global__ __launch_bounds__(512) void ob_few_query_kernel(const ObFewQueryArgs A, int ldc, int ldq)
+{
+    constexpr int U = 12;
+    extern __shared__ __attribute__((aligned(16))) char smem[];        // c_q [16 MT][ldc] | q [16 MT][ldq], bf16
+    __bf16 *cq = reinterpret_cast<__bf16 *>(smem), *qs = cq + 16 * MT * ldc;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, g = lane >> 4;
+    // norm of `cols` columns (a multiple of 4) from column c0 of a row, by one wave; the first 1024 columns wait in registers: request, then finish with
+    // piece(column, four values)
+    struct Row { ob_float4 v[4]; };
+    const auto at = [&](int t, int c) {
+        float s[4] = {0.f, 0.f, 0.f, 0.f};
+        ob_sum_splits<4>(s, A.z + (size_t)t * A.ldz + c, A.z_split, A.n_split);
+        return (ob_float4){s[0], s[1], s[2], s[3]};
+    };
+    const auto request = [&](Row &x, int t, int c0, int cols) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int c = (i * 64 + lane) * 4;
+            x.v[i] = (ob_float4){0.f, 0.f, 0.f, 0.f};
+            if (i * 256 < cols) {                                      // (uniform)
+                if (A.n_split == 1) x.v[i] = *reinterpret_cast<const ob_float4 *>(A.z + (size_t)t * A.ldz + c0 + min(c, cols - 4));
+                else x.v[i] = at(t, c0 + min(c, cols - 4));
+            }
+        }
+    };
+    const auto finish = [&](const Row &x, int t, int c0, int cols, const float *w, auto piece) {
+        float ss = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if ((i * 64 + lane) * 4 < cols) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) ss = __builtin_fmaf(x.v[i][e], x.v[i][e], ss);
+            }
+        for (int c = 1024 + lane * 4; c < cols; c += 256) {
+            const ob_float4 u = at(t, c0 + c);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) ss = __builtin_fmaf(u[e], u[e], ss);
+        }
+        const float r = 1.0f / sqrtf(ob_wave_sum(ss) / (float)cols + A.eps);
+        const auto out = [&](int c, ob_float4 u) {
+            const ob_float4 wv = *reinterpret_cast<const ob_float4 *>(w + c);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) u[e] = u[e] * r * wv[e];
+            piece(c, ob_to_v4<__bf16>(u));
+        };
+#pragma unroll
+        for (int i = 0; i < 4; ++i) if ((i * 64 + lane) * 4 < cols) out((i * 64 + lane) * 4, x.v[i]);
+        for (int c = 1024 + lane * 4; c < cols; c += 256) out(c, at(t, c0 + c));
+    };
+    if ((int)blockIdx.x >= 4 * A.H) {                                  // the cache's new entry, columns beyond kv_rank zero
+        const int t = blockIdx.x - 4 * A.H;
+        if (wave) return;
+        const int slot = A.row_slot[t], pos = A.row_pos[t];
+        if (slot < 0 || slot >= A.n_slots || pos < 0 || pos >= A.max_len) return;      // idle row
+        const int nkt = A.rp / 32;
+        __bf16 *dst = (__bf16 *)A.cache + (size_t)slot * A.bands * nkt * 512;
+        Row x;
+        request(x, t, A.c0, A.kv_rank);
+        finish(x, t, A.c0, A.kv_rank, A.kvn_w, [&](int c, ob_bf4 v) { *reinterpret_cast<ob_bf4 *>(dst + ob_frag<__bf16>(pos, c, nkt)) = v; });
+        for (int c = A.kv_rank + lane * 4; c < A.rp; c += 256) *reinterpret_cast<ob_bf4 *>(dst + ob_frag<__bf16>(pos, c, nkt)) = (ob_bf4)(__bf16)0.f;
+        return;
+    }
+    const int h = blockIdx.x % A.H, part = blockIdx.x / A.H, nt = A.kp >> 4, kts = A.kp >> 5, rt = A.rp >> 6;      // n tiles, k tiles of the absorbing product, its n tiles here
+    const ob_bf8 *wq = (const ob_bf8 *)A.w_uq + (size_t)h * nt * A.cq_nkt * 64 + lane;
+    ob_bf8 w[2 * U];
+    const auto fetch = [&](int b, int n, int k0) {                     // (tiles there are not: the last one again)
+#pragma unroll
+        for (int u = 0; u < U; ++u) w[b * U + u] = wq[((size_t)n * A.cq_nkt + min(k0 + u, A.cq_nkt - 1)) * 64];
+    };
+    Row x[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) if (wave + 8 * q < A.T) request(x[q], wave + 8 * q, 0, A.q_rank);
+    // (the weights behind the rows, those of all waves: a CU's requests are served in order, the head's part of W_uq takes 1.3 us)
+    asm volatile("s_barrier" ::: "memory");
+    if (wave < nt) { fetch(0, wave, 0); fetch(1, wave, U); }
+#pragma unroll
+    for (int q = 0; q < 2 * MT; ++q) {
+        const int t = wave + 8 * q;
+        if (t >= A.T) break;
+        if (q >= 2) request(x[q & 1], t, 0, A.q_rank);
+        finish(x[q & 1], t, 0, A.q_rank, A.qn_w, [&](int c, ob_bf4 v) { *reinterpret_cast<ob_bf4 *>(cq + t * ldc + c) = v; });
+        for (int c = A.q_rank + lane * 4; c < A.cq_nkt * 32; c += 256) *reinterpret_cast<ob_bf4 *>(cq + t * ldc + c) = (ob_bf4)(__bf16)0.f;
+    }
+    __syncthreads();
+    int row[MT];                                                       // (rows beyond the last: the last one again, not written)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) row[m] = min(m * 16 + lr, A.T - 1);
+    for (int n = wave; n < nt; n += 8) {                               // (wave-uniform)
+        if (n != wave) { fetch(0, n, 0); fetch(1, n, U); }
+        ob_float4 acc[MT];
+#pragma unroll
+        for (int m = 0; m < MT; ++m) acc[m] = (ob_float4){0.f, 0.f, 0.f, 0.f};
+        for (int k0 = 0; k0 < A.cq_nkt; k0 += 2 * U) {
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const int k = k0 + b * U + u;
+                    if (k < A.cq_nkt) {                                // (uniform)
+#pragma unroll
+                        for (int m = 0; m < MT; ++m) acc[m] = ObElem<__bf16>::mma(w[b * U + u], *reinterpret_cast<const ob_bf8 *>(cq + row[m] * ldc + k * 32 + g * 8), acc[m]);
+                    }
+                }
+                if (k0 + 2 * U + b * U < A.cq_nkt) fetch(b, n, k0 + 2 * U + b * U);
+            }
+        }
+#pragma unroll
+        for (int m = 0; m < MT; ++m) if (m * 16 + lr < A.T) *reinterpret_cast<ob_bf4 *>(qs + (m * 16 + lr) * ldq + n * 16 + 4 * g) = ob_to_v4<__bf16>(acc[m]);
+    }
+    // this quarter's tiles of the absorbing product: wave, wave + 8 ..
+    const ob_bf8 *wk = (const ob_bf8 *)A.w_uk + ((size_t)h * (A.rp >> 4) + part * rt) * kts * 64 + lane;
+    ob_bf8 wa[4];
+    const auto absorb = [&](int n, int k0) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) wa[k] = wk[(size_t)(n * kts + min(k0 + k, kts - 1)) * 64];
+    };
+    if (wave < rt) absorb(wave, 0);
+    __syncthreads();
+    for (int n = wave; n < rt; n += 8) {
+        if (n != wave) absorb(n, 0);
+        ob_float4 acc[MT];
+#pragma unroll
+        for (int m = 0; m < MT; ++m) acc[m] = (ob_float4){0.f, 0.f, 0.f, 0.f};
+        for (int k0 = 0; k0 < kts; k0 += 4) {
+            if (k0) absorb(n, k0);
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (k0 + k < kts) {                                    // (uniform)
+#pragma unroll
+                    for (int m = 0; m < MT; ++m) acc[m] = ObElem<__bf16>::mma(wa[k], *reinterpret_cast<const ob_bf8 *>(qs + row[m] * ldq + (k0 + k) * 32 + g * 8), acc[m]);
+                }
+        }
+        const int r = (part * rt + n) * 16 + 4 * g;
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            const int t = m * 16 + lr;
+            if (t < A.T) *reinterpret_cast<ob_bf4 *>((__bf16 *)A.heads + ((((size_t)t * A.head_rows + (h >> 4)) << (A.d_shift + 4)) + ob_frag<__bf16>(h & 15, r, 0))) = ob_to_v4<__bf16>(acc[m]);
+        }
+    }
+}
+
+// Up to 32 rows.  Workgroup = (head, four n tiles of its outputs), eight waves: the splits of all rows' contexts of this head together (as
+// ob_lat_combine_kernel, every workgroup of the head again: 18 KB at 12 rows of three live splits), in LDS, then the product with W_uv: a wave takes one n tile
+// and every other k tile, its first four requested before the splits are there.  12 rows, 16 heads of 128, rank 256: 4.8 us for launches of 4.7 + 4.7.
+struct ObFewValueArgs : ObLatArgs {
+    int T;
+    const void *w; int nt, nkt;        // [H][nt][nkt] tiles
+    void *act; int act_nkt;
+};
+static inline int ob_few_value_lds(const ObFewValueArgs &A, int mt) { return 16 * mt * (A.rp + 8) * 2; }
+template <int MT>
+__global__ __launch_bounds__(512) void ob_few_value_kernel(const ObFewValueArgs A)
+{
+    extern __shared__ __attribute__((aligned(16))) char smem[];        // [16 MT][rp + 8] bf16
+    __shared__ ob_float4 red[4][MT][64];
+    __bf16 *ctx = reinterpret_cast<__bf16 *>(smem);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, g = lane >> 4, ld = A.rp + 8, pieces = A.rp >> 3;
+    const int h = blockIdx.x, n = blockIdx.y * 4 + (wave & 3), k0 = wave >> 2;
+    const ob_bf8 *wp = (const ob_bf8 *)A.w + ((size_t)h * A.nt + min(n, A.nt - 1)) * A.nkt * 64 + lane;
+    ob_bf8 w[4];
+    const auto fetch = [&](int k) {                                    // (tiles there are not: the last one again)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) w[u] = wp[(size_t)min(k + 2 * u, A.nkt - 1) * 64];
+    };
+    fetch(k0);
+    for (int i = tid; i < A.T * pieces; i += 512) {
+        const int t = i / pieces, d = (i - t * pieces) * 8, slot = A.row_slot[t], pos = A.row_pos[t];
+        float o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        if (slot >= 0 && slot < A.n_slots && pos >= 0 && pos < A.max_len) {
+            const int nlive = (pos + A.chunk) / A.chunk;
+            if (nlive == 1) {                                          // (written by the attention itself)
+                const ob_bf8 v = *reinterpret_cast<const ob_bf8 *>((const __bf16 *)A.ctx + (size_t)t * A.ldq + (size_t)h * A.rp + d);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) o[e] = (float)v[e];
+            } else {
+                const size_t at = (size_t)t * A.nsplit * A.H + h;
+                const float *ml = A.ml + 2 * at;
+                const __bf16 *part = (const __bf16 *)A.part + at * A.rp + d;
+                float m = -INFINITY, l = 0.f;                          // four splits in flight
+                for (int s0 = 0; s0 < nlive; s0 += 4) {
+                    ob_bf8 v[4];
+                    float ms[4], ls[4];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const size_t sp = (size_t)min(s0 + j, nlive - 1) * A.H;
+                        v[j] = *reinterpret_cast<const ob_bf8 *>(part + sp * A.rp);
+                        ms[j] = ml[2 * sp]; ls[j] = ml[2 * sp + 1];
+                    }
+                    float mx = fmaxf(fmaxf(m, fmaxf(ms[0], ms[1])), fmaxf(ms[2], ms[3]));
+                    const float keep = __builtin_amdgcn_exp2f(m - mx);         // (a split's maximum is finite)
+                    l *= keep;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) o[e] *= keep;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const float f = s0 + j < nlive ? ls[j] * __builtin_amdgcn_exp2f(ms[j] - mx) : 0.f;
+                        l += f;
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) o[e] = __builtin_fmaf(f, (float)v[j][e], o[e]);
+                    }
+                    m = mx;
+                }
+                const float inv = 1.0f / l;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) o[e] *= inv;
+            }
+        }
+        ob_bf8 r;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) r[e] = (__bf16)o[e];
+        *reinterpret_cast<ob_bf8 *>(ctx + t * ld + d) = r;
+    }
+    __syncthreads();
+    ob_float4 acc[MT];
+    const __bf16 *xr[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        acc[m] = (ob_float4){0.f, 0.f, 0.f, 0.f};
+        xr[m] = ctx + min(m * 16 + lr, A.T - 1) * ld + g * 8;
+    }
+    for (int k = k0; k < A.nkt; k += 8) {
+        if (k != k0) fetch(k);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (k + 2 * u < A.nkt) {                                   // (wave-uniform)
+#pragma unroll
+                for (int m = 0; m < MT; ++m) acc[m] = ObElem<__bf16>::mma(w[u], *reinterpret_cast<const ob_bf8 *>(xr[m] + (k + 2 * u) * 32), acc[m]);
+            }
+    }
+    if (k0) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m) red[wave & 3][m][lane] = acc[m];
+    }
+    __syncthreads();
+    if (k0 || n >= A.nt) return;
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        const int t = m * 16 + lr;
+        if (t < A.T) *reinterpret_cast<ob_bf4 *>((__bf16 *)A.act + ob_frag<__bf16>(t, (h * A.nt + n) * 16 + 4 * g, A.act_nkt)) = ob_to_v4<__bf16>(acc[m] + red[wave & 3][m][lane]);
     }
 }

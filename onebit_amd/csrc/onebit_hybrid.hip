@@ -199,6 +199,8 @@ static int act_index(const HPlan &P, const onebit_hlayer_t &L)
 }
 #define OB_LAT_PARTS 1024       // (row, split) pairs of the latent decode attention with more than one split
 #define OB_SIDE_SPLITS 4        // K splits of a token input's gate product
+#define OB_FEW_LATENT 32        // rows of the merged launches of latent attention
+#define OB_FEW_QUERY 200        // weight tiles of a head's query product that four workgroups read each (half of them for more than 16 rows)
 #define OB_FEW_SIDE_KT 64       // ... of a layer's end, which has two products
 #define OB_FEW_KT 128           // k tiles of a product in a row kernel (of up to 64 columns)
 #define OB_EZ_ROWS 4096         // fp32 rows of the experts' partial sums at least
@@ -556,10 +558,10 @@ static int ssm_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, const 
 
 // plain product into fp32 partial sums: returns the number of splits through n_split
 template <typename E>
-static int part_launch(ObDenseArgs d, float *z, int &n_split, hipStream_t s)
+static int part_launch(ObDenseArgs d, float *z, int &n_split, hipStream_t s, int most = 8)
 {
     d.z = z; d.ldz = 16 * d.n_tiles; d.z_split = (size_t)d.T * d.ldz;
-    n_split = gemm_splits(d.n_tiles, d.nkt, d.T);
+    n_split = std::min(most, gemm_splits(d.n_tiles, d.nkt, d.T));
     n_split = (int)cdiv(d.nkt, cdiv(d.nkt, n_split));
     return dense_launch<E, OB_EPI_PART>(d, n_split, s);
 }
@@ -572,36 +574,54 @@ static int latent_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, con
     constexpr int KT = ObElem<E>::KT;
     const onebit_hlatent_t &l = L.latent;
     const int T = st.n_rows, H = L.heads, bands = (int)cdiv(m.max_len, 16), cq_nkt = (int)cdiv(l.q_rank, KT);
-    float *z = (float *)(ws + P.z);
-    int n_split;
-    ObDenseArgs d = {};
-    d.w = L.w_in; d.a = ws + P.h; d.n_tiles = L.nt_in; d.nkt = m.width_pad / KT; d.T = T;
-    if (int rc = part_launch<E>(d, z, n_split, s)) return rc;
-    ObLatPrepArgs p = {z, (size_t)T * 16 * L.nt_in, n_split, 16 * L.nt_in, l.q_rank, 16 * l.nt_q, l.kv_rank, l.qn_w, l.kvn_w, m.eps, ws + P.cq, cq_nkt, run.s0, l.rp, bands,
-                       st.row_slot, st.row_pos, m.n_slots, m.max_len};
-    const int n_in = l.q_rank + l.kv_rank, plds = (((n_in + 3) & ~3) + 16) * 4;
     const bool vec = l.q_rank % 4 == 0 && l.kv_rank % 4 == 0;
-    auto pgo = [&](auto pk) {
-        if (!lds_ok((const void *)pk, plds)) return hfail(ONEBIT_E_SHAPE, "latent norms: LDS");
-        hipLaunchKernelGGL(pk, dim3((unsigned)T), dim3((unsigned)std::min<int64_t>(T <= 256 ? 1024 : 512, rup(cdiv(n_in, vec ? 4 : 1), 64))), plds, s, p);
-        return hstatus("latent norms");
-    };
-    if (int rc = vec ? pgo(ob_lat_prep_kernel<E, 4>) : pgo(ob_lat_prep_kernel<E, 1>)) return rc;
-    // queries, row-major [T][H kp]
-    ObDenseArgs q = {};
-    q.w = l.w_uq; q.a = ws + P.cq; q.n_tiles = q.nt_mix = H * L.kp / 16; q.nkt = cq_nkt; q.T = T; q.u = ws + P.qu;
-    if (int rc = dense_launch<E, OB_EPI_IN>(q, 1, s)) return rc;
     int n_abs = T;
     int first = st.n_seg;
     if (l.tiled && l.flash) {
         n_abs = st.n_dec;
         for (first = 0; first < st.n_short; ++first) n_abs += st.segs[first].n;
     }
+    // few rows, all of the absorbed form: norms and both products of the queries in one launch; the splits' outputs together within the value product
+    const bool few = l.tiled && n_abs == T && T <= OB_FEW_LATENT, few_q = few && vec && L.kp / 16 * cq_nkt <= (T <= 16 ? OB_FEW_QUERY : OB_FEW_QUERY / 2)
+                       && 64 * (ob_few_query_ld(l.q_rank) + ob_few_query_ld(L.kp)) <= 150 * 1024;      // (LDS at 32 rows)
+    float *z = (float *)(ws + P.z);
+    int n_split;
+    ObDenseArgs d = {};
+    d.w = L.w_in; d.a = ws + P.h; d.n_tiles = L.nt_in; d.nkt = m.width_pad / KT; d.T = T;
+    if (int rc = part_launch<E>(d, z, n_split, s, few_q && T > 8 ? 1 : 8)) return rc;
+    ObLatPrepArgs p = {z, (size_t)T * 16 * L.nt_in, n_split, 16 * L.nt_in, l.q_rank, 16 * l.nt_q, l.kv_rank, l.qn_w, l.kvn_w, m.eps, ws + P.cq, cq_nkt, run.s0, l.rp, bands,
+                       st.row_slot, st.row_pos, m.n_slots, m.max_len};
+    if constexpr (sizeof(E) == 2) if (few_q) {
+        ObFewQueryArgs f = {};
+        static_cast<ObLatPrepArgs &>(f) = p;
+        f.T = T; f.H = H; f.w_uq = l.w_uq; f.w_uk = l.w_uk; f.kp = L.kp; f.heads = ws + P.qa; f.head_rows = (int)cdiv(H, 16);
+        for (f.d_shift = 6; (1 << f.d_shift) < l.rp; ++f.d_shift) {}
+        const int mt = T <= 16 ? 1 : 2, lds = ob_few_query_lds(f, mt);
+        auto go = [&](auto k) {
+            if (!lds_ok((const void *)k, lds)) return hfail(ONEBIT_E_SHAPE, "latent queries: LDS");
+            hipLaunchKernelGGL(k, dim3((unsigned)(4 * H + T)), dim3(512), lds, s, f, ob_few_query_ld(l.q_rank), ob_few_query_ld(L.kp));
+            return hstatus("latent queries");
+        };
+        if (int rc = mt == 1 ? go(ob_few_query_kernel<1>) : go(ob_few_query_kernel<2>)) return rc;
+    }
+    if (!few_q) {
+        const int n_in = l.q_rank + l.kv_rank, plds = (((n_in + 3) & ~3) + 16) * 4;
+        auto pgo = [&](auto pk) {
+            if (!lds_ok((const void *)pk, plds)) return hfail(ONEBIT_E_SHAPE, "latent norms: LDS");
+            hipLaunchKernelGGL(pk, dim3((unsigned)T), dim3((unsigned)std::min<int64_t>(T <= 256 ? 1024 : 512, rup(cdiv(n_in, vec ? 4 : 1), 64))), plds, s, p);
+            return hstatus("latent norms");
+        };
+        if (int rc = vec ? pgo(ob_lat_prep_kernel<E, 4>) : pgo(ob_lat_prep_kernel<E, 1>)) return rc;
+        // queries, row-major [T][H kp]
+        ObDenseArgs q = {};
+        q.w = l.w_uq; q.a = ws + P.cq; q.n_tiles = q.nt_mix = H * L.kp / 16; q.nkt = cq_nkt; q.T = T; q.u = ws + P.qu;
+        if (int rc = dense_launch<E, OB_EPI_IN>(q, 1, s)) return rc;
+    }
     if (n_abs) {
         ObDenseArgs k = {};
         k.w = l.w_uk; k.a = ws + P.qu; k.lda = H * L.kp; k.tile_group = l.rp / 16; k.act_cols = L.kp; k.n_tiles = k.nt_mix = H * l.rp / 16; k.nkt = L.kp / KT; k.T = n_abs; k.u = ws + P.qa;
         if constexpr (sizeof(E) == 2) {
-            if (l.tiled) {
+            if (l.tiled && !few_q) {
                 k.heads = ws + P.qa; k.head_rows = (int)cdiv(H, 16);
                 for (k.d_shift = 6; (1 << k.d_shift) < l.rp; ++k.d_shift) {}
                 if (int rc = dense_heads_launch<E, OB_EPI_QFRAG>(k, (size_t)OB_SKINNY_T * rup(H, 16) * l.rp * sizeof(E), s)) return rc;
@@ -645,6 +665,16 @@ static int latent_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, con
                             : l.rp == 256 ? go(ob_lat_dec_kernel<256, 1>, 256) : go(ob_lat_dec_kernel<512, 1>, 512);
                 } else rc = hfail(ONEBIT_E_DTYPE, "latent attention: tiled form in fp32");
                 if (rc) return rc;
+                if constexpr (sizeof(E) == 2) if (few && a.nsplit > 1) {
+                    ObFewValueArgs f = {};
+                    static_cast<ObLatArgs &>(f) = a;
+                    f.T = T; f.w = l.w_uv; f.nt = l.vdp / 16; f.nkt = l.rp / KT; f.act = act; f.act_nkt = act_nkt;
+                    const int mt = T <= 16 ? 1 : 2, lds = ob_few_value_lds(f, mt);       // (at most 33 KB)
+                    const dim3 vgrid((unsigned)H, (unsigned)cdiv(f.nt, 4));
+                    if (mt == 1) hipLaunchKernelGGL(ob_few_value_kernel<1>, vgrid, dim3(512), lds, s, f);
+                    else hipLaunchKernelGGL(ob_few_value_kernel<2>, vgrid, dim3(512), lds, s, f);
+                    return hstatus("latent attention outputs");        // (no rows of the expanded form)
+                }
                 if (a.nsplit > 1) hipLaunchKernelGGL(ob_lat_combine_kernel, dim3((unsigned)H, grid.y), dim3((unsigned)std::min<int64_t>(256, rup(l.rp / 8, 64))), 0, s, a);
             }
         }

@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from oracle import serotar_ref as R
-from test_gpu_serotar import BF, TOL, build, clear_choices, err, rows_err, run, tokens
+from test_gpu_serotar import BF, TOL, build, clear_choices, err, only, rows_err, run, tokens
 from test_serotar_cpu import dense, layer, moe, raw_config
 
 pytestmark = pytest.mark.gpu
@@ -62,3 +62,26 @@ def test_rows_do_not_change_each_other():
     assert torch.equal(eng.logits[:16].flip(0), together)
     eng.launch([(9, 6, [12])])
     assert float((eng.logits[0] - together[9]).abs().max()) <= 1e-2 * float(together[9].abs().max())      # (splits of the sums follow the number of rows)
+
+
+# heads, sizes and ranks: rp 64 .. 512, padded columns everywhere, heads beyond a group of 16, more n tiles than waves, absorbing products of 1, 4 and 5 k tiles,
+# a rank beyond the registers' 1024 columns, ranks that are no multiple of 4 (the launches by themselves)
+LATENTS = {"rp 64": dict(heads=3, dim=24, vdim=40, q_rank=20, kv_rank=36, scale=0.4), "rp 128": dict(heads=17, dim=64, vdim=56, q_rank=100, kv_rank=112, scale=0.1),
+           "rp 256": dict(heads=16, dim=128, vdim=128, q_rank=768, kv_rank=256, scale=0.08), "rp 512": dict(heads=20, dim=128, vdim=64, q_rank=96, kv_rank=500, scale=0.09),
+           "wide heads": dict(heads=2, dim=144, vdim=136, q_rank=64, kv_rank=300, scale=0.08), "long rank": dict(heads=2, dim=32, vdim=32, q_rank=1236, kv_rank=64, scale=0.2),
+           "odd ranks": dict(heads=5, dim=32, vdim=32, q_rank=39, kv_rank=61, scale=0.2)}
+
+
+@pytest.mark.parametrize("name", LATENTS)
+def test_decoded_rows_of_latent_attention(name):
+    """1 .. 33 requests at contexts from one key to many splits, one token each."""
+    raw = raw_config([layer(**LATENTS[name])], width=96, side=0)
+    m, w = build(raw, BF, edit=only("mix"))
+    toks = tokens(720, 61)
+    ref = R.forward(raw, w, toks)
+    for n in (1, 2, 9, 16, 17, 32, 33):
+        at = [int(round(x)) for x in torch.linspace(719 if n == 1 else 1, 719, n).tolist()]
+        eng = m.step_engine(n, 768, max_rows=sum(at))
+        eng.launch([(i, 0, toks[:p]) for i, p in enumerate(at)])
+        eng.launch([(i, p, toks[p:p + 1]) for i, p in enumerate(at)])
+        assert err(eng.logits[:n], ref[at]) < TOL[BF], n
