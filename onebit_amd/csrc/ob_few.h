@@ -568,9 +568,9 @@ __global__ __launch_bounds__(512) void ob_few_query_kernel(const ObFewQueryArgs 
     }
 }
 
-// Up to 32 rows.  Workgroup = (head, four n tiles of its outputs), eight waves: the splits of all rows' contexts of this head together (as
+// Up to 32 rows.  Workgroup = (head, two n tiles of its outputs), eight waves: the splits of all rows' contexts of this head together (as
 // ob_lat_combine_kernel, every workgroup of the head again: 18 KB at 12 rows of three live splits), in LDS, then the product with W_uv: a wave takes one n tile
-// and every other k tile, its first four requested before the splits are there.  12 rows, 16 heads of 128, rank 256: 4.8 us for launches of 4.7 + 4.7.
+// and every fourth k tile, all requested before the splits are there.  12 rows, 16 heads of 128, rank 256: 4.8 us for launches of 4.7 + 4.7.
 struct ObFewValueArgs : ObLatArgs {
     int T;
     const void *w; int nt, nkt;        // [H][nt][nkt] tiles
@@ -581,15 +581,15 @@ template <int MT>
 __global__ __launch_bounds__(512) void ob_few_value_kernel(const ObFewValueArgs A)
 {
     extern __shared__ __attribute__((aligned(16))) char smem[];        // [16 MT][rp + 8] bf16
-    __shared__ ob_float4 red[4][MT][64];
+    __shared__ ob_float4 red[6][MT][64];
     __bf16 *ctx = reinterpret_cast<__bf16 *>(smem);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, g = lane >> 4, ld = A.rp + 8, pieces = A.rp >> 3;
-    const int h = blockIdx.x, n = blockIdx.y * 4 + (wave & 3), k0 = wave >> 2;
+    const int h = blockIdx.x, n = blockIdx.y * 2 + (wave & 1), k0 = wave >> 1;
     const ob_bf8 *wp = (const ob_bf8 *)A.w + ((size_t)h * A.nt + min(n, A.nt - 1)) * A.nkt * 64 + lane;
-    ob_bf8 w[4];
+    ob_bf8 w[4];                                                       // (rank 512: 16 k tiles)
     const auto fetch = [&](int k) {                                    // (tiles there are not: the last one again)
 #pragma unroll
-        for (int u = 0; u < 4; ++u) w[u] = wp[(size_t)min(k + 2 * u, A.nkt - 1) * 64];
+        for (int u = 0; u < 4; ++u) w[u] = wp[(size_t)min(k + 4 * u, A.nkt - 1) * 64];
     };
     fetch(k0);
     for (int i = tid; i < A.T * pieces; i += 512) {
@@ -647,24 +647,24 @@ __global__ __launch_bounds__(512) void ob_few_value_kernel(const ObFewValueArgs 
         acc[m] = (ob_float4){0.f, 0.f, 0.f, 0.f};
         xr[m] = ctx + min(m * 16 + lr, A.T - 1) * ld + g * 8;
     }
-    for (int k = k0; k < A.nkt; k += 8) {
+    for (int k = k0; k < A.nkt; k += 16) {
         if (k != k0) fetch(k);
 #pragma unroll
         for (int u = 0; u < 4; ++u)
-            if (k + 2 * u < A.nkt) {                                   // (wave-uniform)
+            if (k + 4 * u < A.nkt) {                                   // (wave-uniform)
 #pragma unroll
-                for (int m = 0; m < MT; ++m) acc[m] = ObElem<__bf16>::mma(w[u], *reinterpret_cast<const ob_bf8 *>(xr[m] + (k + 2 * u) * 32), acc[m]);
+                for (int m = 0; m < MT; ++m) acc[m] = ObElem<__bf16>::mma(w[u], *reinterpret_cast<const ob_bf8 *>(xr[m] + (k + 4 * u) * 32), acc[m]);
             }
     }
     if (k0) {
 #pragma unroll
-        for (int m = 0; m < MT; ++m) red[wave & 3][m][lane] = acc[m];
+        for (int m = 0; m < MT; ++m) red[wave - 2][m][lane] = acc[m];
     }
     __syncthreads();
     if (k0 || n >= A.nt) return;
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
         const int t = m * 16 + lr;
-        if (t < A.T) *reinterpret_cast<ob_bf4 *>((__bf16 *)A.act + ob_frag<__bf16>(t, (h * A.nt + n) * 16 + 4 * g, A.act_nkt)) = ob_to_v4<__bf16>(acc[m] + red[wave & 3][m][lane]);
+        if (t < A.T) *reinterpret_cast<ob_bf4 *>((__bf16 *)A.act + ob_frag<__bf16>(t, (h * A.nt + n) * 16 + 4 * g, A.act_nkt)) = ob_to_v4<__bf16>((acc[m] + red[wave][m][lane]) + (red[wave + 2][m][lane] + red[wave + 4][m][lane]));
     }
 }

@@ -670,7 +670,7 @@ static int latent_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, con
                     static_cast<ObLatArgs &>(f) = a;
                     f.T = T; f.w = l.w_uv; f.nt = l.vdp / 16; f.nkt = l.rp / KT; f.act = act; f.act_nkt = act_nkt;
                     const int mt = T <= 16 ? 1 : 2, lds = ob_few_value_lds(f, mt);       // (at most 33 KB)
-                    const dim3 vgrid((unsigned)H, (unsigned)cdiv(f.nt, 4));
+                    const dim3 vgrid((unsigned)H, (unsigned)cdiv(f.nt, 2));
                     if (mt == 1) hipLaunchKernelGGL(ob_few_value_kernel<1>, vgrid, dim3(512), lds, s, f);
                     else hipLaunchKernelGGL(ob_few_value_kernel<2>, vgrid, dim3(512), lds, s, f);
                     return hstatus("latent attention outputs");        // (no rows of the expanded form)
