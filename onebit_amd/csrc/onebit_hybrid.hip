@@ -22,6 +22,7 @@
 #include "ob_latent.h"
 #include "ob_moe.h"
 #include "ob_few.h"
+#include "ob_side.h"
 
 static thread_local char g_err[512];
 static int hfail(int code, const char *fmt, ...)
@@ -791,12 +792,14 @@ static int few_experts_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L
     return 0;
 }
 
-// The end of a sequential layer with few rows, from its feed-forward's products (`a`) to the next layer's operand: ob_few_side_kernel.  Up to 2048 columns and
-// 64 of the token input: every row's workgroup reads both weights whole (512 KB, 3.4 us; 2 MB at 4096 x 128 would be 14, the separate launches take 21)
+// The end of a sequential layer, from its feed-forward's products (`a`) to the next layer's operand, in one launch: up to 64 rows ob_few_side_kernel, more
+// ob_side_rows_kernel.  Up to 2048 columns and 64 of the token input: every workgroup reads both weights whole (512 KB, 3.4 us; 2 MB at 4096 x 128 would be
+// 14, a few rows' separate launches take 21; a prompt's row of 4096 columns does not fit the registers).  Many rows: whole k tiles (the others' separate launches)
 static bool few_side(const onebit_hmodel_t &m, const onebit_hlayer_t &L, const onebit_hstate_t &st, const ObXRowArgs &a)
 {
-    return m.dtype == ONEBIT_HYB_BF16 && st.n_rows <= OB_SKINNY_T && m.width % 4 == 0 && m.width <= 4096 && m.width_pad / 32 <= OB_FEW_SIDE_KT &&
-           (L.side.nt == 2 || L.side.nt == 4) && !a.embed && !a.emb_save && !a.emb_add && !a.bias && !a.eo && (!a.top || (a.ez && few_experts(m, L, st.n_rows)));
+    if (m.dtype != ONEBIT_HYB_BF16 || m.width > 32 * OB_FEW_SIDE_KT || (L.side.nt != 2 && L.side.nt != 4) || a.embed || a.emb_save || a.emb_add || a.bias) return false;
+    if (st.n_rows > OB_SKINNY_T) return m.width % 32 == 0 && m.width_pad == m.width && (!a.top || a.eo);      // ob_side_rows_kernel: whole k tiles
+    return m.width % 4 == 0 && !a.eo && (!a.top || (a.ez && few_experts(m, L, st.n_rows)));
 }
 static int few_side_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, const onebit_hstate_t &st, const ObXRowArgs &a, const float *next_w, void *out, hipStream_t s)
 {
@@ -806,6 +809,19 @@ static int few_side_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, c
     f.p = {L.side.w_gate, m.width_pad / 32};
     f.q = {L.side.w_proj, L.side.nt / 2};
     f.table = L.side.table; f.ld_table = m.side_cols; f.dim = L.side.dim; f.side_w = L.side.norm_w;
+    if (st.n_rows > OB_SKINNY_T) {
+        const int lds = ob_side_rows_lds(L.side.nt), wg_rows = ob_side_rows_of(st.n_rows, cu_count());
+        const auto go = [&](auto k) {
+            if (!lds_ok((const void *)k, lds)) return hfail(ONEBIT_E_SHAPE, "token input: LDS");
+            hipLaunchKernelGGL(k, dim3((unsigned)cdiv(st.n_rows, wg_rows)), dim3(1024), lds, s, f, st.n_rows, wg_rows);
+            return hstatus("token input");
+        };
+        const bool narrow = m.width <= 1024;
+        if (L.side.nt == 2) return a.top ? narrow ? go(ob_side_rows_kernel<OB_X_EXPERTS, 2, 2>) : go(ob_side_rows_kernel<OB_X_EXPERTS, 2, 4>)
+                                         : narrow ? go(ob_side_rows_kernel<OB_X_PLAIN, 2, 2>) : go(ob_side_rows_kernel<OB_X_PLAIN, 2, 4>);
+        return a.top ? narrow ? go(ob_side_rows_kernel<OB_X_EXPERTS, 4, 2>) : go(ob_side_rows_kernel<OB_X_EXPERTS, 4, 4>)
+                     : narrow ? go(ob_side_rows_kernel<OB_X_PLAIN, 4, 2>) : go(ob_side_rows_kernel<OB_X_PLAIN, 4, 4>);
+    }
     const int lds = ob_few_side_lds(f);
     const dim3 grid((unsigned)st.n_rows);
     if (L.side.nt == 2) {
