@@ -527,32 +527,39 @@ __global__ __launch_bounds__(512) void ob_b_lmhead_kernel(const ObBHeadArgs A)
 
     // staging: thread -> (token st_b + 16 i, halves st_k .. st_k + 7) of a [TT*16, 256] chunk
     const int st_b = tid >> 5, st_k = (tid & 31) * 8;
-    auto stage = [&](int kc, int buf) {
+    ob_half8 xv[TT];
+    auto fetch = [&](int kc) {
 #pragma unroll
         for (int i = 0; i < TT; ++i) {
             const int b = st_b + 16 * i, k = kc * OB_BH_K + st_k;
-            ob_half8 v = (ob_half8)(_Float16)0;
-            if (b < B && k < H) v = *reinterpret_cast<const ob_half8 *>(A.x + (int64_t)b * H + k);
-            *reinterpret_cast<ob_half8 *>(&xs[buf][b][st_k]) = v;
+            xv[i] = (ob_half8)(_Float16)0;
+            if (b < B && k < H) xv[i] = *reinterpret_cast<const ob_half8 *>(A.x + (int64_t)b * H + k);
+        }
+    };
+    auto stage = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < TT; ++i) *reinterpret_cast<ob_half8 *>(&xs[buf][st_b + 16 * i][st_k]) = xv[i];
+    };
+    // this lane's 8 x 16 bytes of its row for a chunk (non-temporal: read exactly once per step), requested while the chunk before is multiplied and behind
+    // that chunk's activations, so that nothing waits for them early: 29 rows, 262 MB of weights 68 -> 64 us (whole 64-byte pieces an instruction: 62.5, the same step)
+    auto weights = [&](ob_half8 (&wf)[8], int kc) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int kk = min(kc * OB_BH_K + q * 64, H - 64);       // H % 64 == 0 (host-checked); clamp the tail chunk
+            wf[2 * q] = __builtin_nontemporal_load(reinterpret_cast<const ob_half8 *>(wrow + kk));
+            wf[2 * q + 1] = __builtin_nontemporal_load(reinterpret_cast<const ob_half8 *>(wrow + kk + 8));
         }
     };
     ob_float4 acc[TT];
 #pragma unroll
     for (int t = 0; t < TT; ++t) acc[t] = (ob_float4){0.f, 0.f, 0.f, 0.f};
-    stage(0, 0);
-    __syncthreads();
-    for (int kc = 0; kc < nkc; ++kc) {
+    ob_half8 w0[8], w1[8];
+    auto chunk = [&](ob_half8 (&wf)[8], ob_half8 (&next)[8], int kc) {
         const int buf = kc & 1;
-        // this lane's 8 x 16 bytes of its row for the chunk (non-temporal: read exactly once per step)
-        ob_half8 wf[8];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int k = kc * OB_BH_K + q * 64;
-            const int kk = min(k, H - 64);                       // H % 64 == 0 (host-checked); clamp the tail chunk
-            wf[2 * q] = __builtin_nontemporal_load(reinterpret_cast<const ob_half8 *>(wrow + kk));
-            wf[2 * q + 1] = __builtin_nontemporal_load(reinterpret_cast<const ob_half8 *>(wrow + kk + 8));
+        if (kc + 1 < nkc) {
+            fetch(kc + 1);
+            weights(next, kc + 1);
         }
-        if (kc + 1 < nkc) stage(kc + 1, buf ^ 1);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             if (kc * OB_BH_K + q * 64 < H) {
@@ -566,7 +573,16 @@ __global__ __launch_bounds__(512) void ob_b_lmhead_kernel(const ObBHeadArgs A)
                 }
             }
         }
+        if (kc + 1 < nkc) stage(buf ^ 1);
         __syncthreads();
+    };
+    fetch(0);
+    weights(w0, 0);
+    stage(0);
+    __syncthreads();
+    for (int kc = 0; kc < nkc; kc += 2) {
+        chunk(w0, w1, kc);
+        if (kc + 1 < nkc) chunk(w1, w0, kc + 1);
     }
     // D[v][b]: lane holds v = v0 + 4 gq + i (i = 0..3), b = t * 16 + r
 #pragma unroll
