@@ -612,7 +612,12 @@ static int latent_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, con
             hipLaunchKernelGGL(pk, dim3((unsigned)T), dim3((unsigned)std::min<int64_t>(T <= 256 ? 1024 : 512, rup(cdiv(n_in, vec ? 4 : 1), 64))), plds, s, p);
             return hstatus("latent norms");
         };
-        if (int rc = vec ? pgo(ob_lat_prep_kernel<E, 4>) : pgo(ob_lat_prep_kernel<E, 1>)) return rc;
+        if (vec && T > OB_SKINNY_T && n_in <= 2048) {                 // many rows: a wave each
+            const dim3 rgrid((unsigned)cdiv(T, 4));
+            if (n_in <= 1024) hipLaunchKernelGGL((ob_lat_prep_rows_kernel<E, 4>), rgrid, dim3(256), 0, s, p, T);
+            else hipLaunchKernelGGL((ob_lat_prep_rows_kernel<E, 8>), rgrid, dim3(256), 0, s, p, T);
+            if (int rc = hstatus("latent norms")) return rc;
+        } else if (int rc = vec ? pgo(ob_lat_prep_kernel<E, 4>) : pgo(ob_lat_prep_kernel<E, 1>)) return rc;
         // queries, row-major [T][H kp]
         ObDenseArgs q = {};
         q.w = l.w_uq; q.a = ws + P.cq; q.n_tiles = q.nt_mix = H * L.kp / 16; q.nkt = cq_nkt; q.T = T; q.u = ws + P.qu;
