@@ -471,3 +471,25 @@ def test_large_tile_kernels_forced_on_ragged_shapes(dev, env):
     child = os.path.join(os.path.dirname(os.path.abspath(__file__)), "forced_route_child.py")
     r = subprocess.run([sys.executable, child], env=dict(os.environ, **env), capture_output=True, text=True, timeout=600)
     assert r.returncode == 0 and "forced-route ok" in r.stdout, (r.stdout[-2000:], r.stderr[-2000:])
+
+
+def test_leading_dimensions_and_strides_are_the_same_rows(dev):
+    """Rows as a vector, a matrix, a batch, every other row, a transposed batch and none: the same bits, the input's leading dimensions, contiguous."""
+    from onebit_amd import BitLinearInf
+    K, N = 256, 96
+    g = torch.Generator(device=dev).manual_seed(3)
+    m = BitLinearInf(K, N, dtype=torch.float16).to(dev)
+    m.weight.data = torch.randint(-128, 128, (N, K // 8), generator=g, device=dev, dtype=torch.int8)
+    x = torch.randn(6, K, generator=g, device=dev).half()
+    ref = m(x)
+    assert ref.shape == (6, N)
+    wide, both = torch.empty(12, K + 8, dtype=torch.float16, device=dev), x.view(2, 3, K).transpose(0, 1).contiguous().transpose(0, 1)
+    wide[::2, :K] = x
+    for rows, want in ((x.view(2, 3, K), ref.view(2, 3, N)), (wide[::2, :K], ref), (both, ref.view(2, 3, N)), (x.view(1, 6, K), ref.view(1, 6, N))):
+        y = m(rows)
+        assert y.shape == want.shape and y.is_contiguous() and torch.equal(y, want)
+    one = m(x[4])
+    assert one.shape == (N,) and torch.equal(one, m(x[4:5])[0])
+    assert m(x[:0].view(0, 3, K)).shape == (0, 3, N)
+    with pytest.raises(RuntimeError):
+        BitLinearInf(0, N, dtype=torch.float16).to(dev)(torch.empty(2, 0, dtype=torch.float16, device=dev))
