@@ -8,17 +8,19 @@
 #pragma once
 #include "ob_dense.h"
 
-#define OB_MOE_TOKENS 64              // tokens per workgroup
+#define OB_MOE_TOKENS 64              // tokens per workgroup at most
+#define OB_MOE_FEW 16                 // ... one a wave, where their counts are few
 struct ObRouteArgs {
     const float *z; int ldz;                   // router logits [T][experts + identity]
     const float *correction;
     int T, experts, identity, top, groups, keep;
+    int tokens;                                // per workgroup of the first pass
     int32_t *tok_row; float *tok_w, *id_w;     // (tok_row holds the expert between the two passes)
-    int32_t *hist;                             // [workgroups][experts]
+    int32_t *hist;                             // [workgroups of the first pass][experts]
     int32_t *gather; ObRowBlock *blk; int block_rows, n_blk;
 };
-// LDS of the first pass: per wave [groups] group maxima; [experts] counts; [64 top] experts of the workgroup's tokens
-static inline size_t ob_route_lds(const ObRouteArgs &A) { return (16 * (size_t)A.groups + A.experts + (size_t)OB_MOE_TOKENS * A.top) * 4; }
+// LDS of the first pass: per wave [groups] group maxima; [experts] counts; [tokens top] experts of the workgroup's tokens
+static inline size_t ob_route_lds(const ObRouteArgs &A) { return (16 * (size_t)A.groups + A.experts + (size_t)A.tokens * A.top) * 4; }
 #define OB_MOE_MAX 1024               // experts + identity experts
 
 // order-preserving integers: the largest of a group through an LDS atomic
@@ -85,8 +87,8 @@ __device__ __forceinline__ void ob_route_token(const ObRouteArgs &A, int t, cons
     if (lane == 0) A.id_w[t] = idw;
 }
 
-// offsets of the experts' rows and the block table from counts in LDS; 1024 threads.  cnt[e] -> first row of e.
-__device__ __forceinline__ void ob_route_offsets(const ObRouteArgs &A, int *cnt, int *scan, int tid)
+// offsets of the experts' rows and (one workgroup) the block table from counts in LDS; 1024 threads.  cnt[e] -> first row of e.
+__device__ __forceinline__ void ob_route_offsets(const ObRouteArgs &A, int *cnt, int *scan, int tid, bool table)
 {
     // scan[2 w], scan[2 w + 1]: rows / blocks of the waves before; experts in runs of 1024
     int row_base = 0, blk_base = 0;
@@ -110,9 +112,10 @@ __device__ __forceinline__ void ob_route_offsets(const ObRouteArgs &A, int *cnt,
         r0 += r - rows; b0 += b - nb;
         if (e < A.experts) {
             cnt[e] = r0;
-            for (int k = 0; k < nb && b0 + k < A.n_blk; ++k) A.blk[b0 + k] = {e, r0 + k * A.block_rows, min(A.block_rows, c - k * A.block_rows), 0};
+            if (table) for (int k = 0; k < nb && b0 + k < A.n_blk; ++k) A.blk[b0 + k] = {e, r0 + k * A.block_rows, min(A.block_rows, c - k * A.block_rows), 0};
         }
     }
+    if (!table) return;                                               // (uniform)
     for (int k = blk_base + tid; k < A.n_blk; k += 1024) A.blk[k] = {0, 0, 0, 0};
     __syncthreads();                                                  // (the table's first entry is written)
     if (tid == 0 && A.n_blk > 0) A.blk[0].n_used = min(blk_base, A.n_blk);
@@ -129,7 +132,7 @@ __global__ __launch_bounds__(1024) void ob_route_kernel(const ObRouteArgs A)
     uint32_t *gs = reinterpret_cast<uint32_t *>(sm) + wave * A.groups;
     int *cnt = reinterpret_cast<int *>(sm) + 16 * A.groups, *slots = cnt + A.experts;
     for (int e = tid; e < A.experts; e += 1024) cnt[e] = 0;
-    const int t0 = blockIdx.x * OB_MOE_TOKENS, t1 = min(A.T, t0 + OB_MOE_TOKENS), n = (t1 - t0) * A.top;
+    const int t0 = blockIdx.x * A.tokens, t1 = min(A.T, t0 + A.tokens), n = (t1 - t0) * A.top;
     float corr[NJ];
 #pragma unroll
     for (int j = 0; j < NJ; ++j) corr[j] = lane + 64 * j < N ? A.correction[lane + 64 * j] : 0.f;
@@ -158,7 +161,7 @@ __global__ __launch_bounds__(1024) void ob_route_kernel(const ObRouteArgs A)
         for (int e = tid; e < A.experts; e += 1024) A.hist[(size_t)blockIdx.x * A.experts + e] = cnt[e];
         for (int i = tid; i < n; i += 1024) A.tok_row[(size_t)t0 * A.top + i] = slots[i];
     } else {
-        ob_route_offsets(A, cnt, scan, tid);
+        ob_route_offsets(A, cnt, scan, tid, true);
         __syncthreads();
         for (int i = tid; i < n; i += 1024) {
             int r = -1;
@@ -171,53 +174,44 @@ __global__ __launch_bounds__(1024) void ob_route_kernel(const ObRouteArgs A)
     }
 }
 
-// second pass, one workgroup: counts of all workgroups -> where each workgroup's tokens of an expert start; row and block tables.  An expert's
-// workgroups are shared by `runs` threads (runs * experts <= 1024, or one run).
-__global__ __launch_bounds__(1024) void ob_route_scan_kernel(const ObRouteArgs A, int n_wg, int runs)
+// second pass, 64 tokens a workgroup: every one adds up the counts of all workgroups of the first by itself (what an expert has in all, and before its own
+// tokens; `runs` threads an expert, runs * experts <= 1024, or one), the first one writes the block table, each its tokens' rows.  (A launch of one workgroup for
+// the offsets and one for the rows: 8.5 + 4.8 us of 6095 tokens and 32 experts, now 9.6; the first pass with 16 tokens a workgroup 13.2 -> 7.8 us.)
+static inline size_t ob_route_place_lds(const ObRouteArgs &A, int runs) { return (size_t)A.experts * (2 + 2 * runs) * 4; }
+__global__ __launch_bounds__(1024) void ob_route_place_kernel(const ObRouteArgs A, int n_wg, int runs)
 {
-    extern __shared__ int icnt[];                                     // [experts] | [runs][experts]
+    extern __shared__ int icnt[];                                     // [experts] counts, first rows | [experts] counts before | [2][runs][experts]
     __shared__ int scan[32];
-    int *part = icnt + A.experts;
-    const int tid = threadIdx.x, per = (n_wg + runs - 1) / runs;
+    int *before = icnt + A.experts, *part = before + A.experts;
+    const int tid = threadIdx.x, per = (n_wg + runs - 1) / runs, t0 = blockIdx.x * OB_MOE_TOKENS, t1 = min(A.T, t0 + OB_MOE_TOKENS), own = t0 / A.tokens;
     for (int i = tid; i < runs * A.experts; i += 1024) {
         const int q = i / A.experts, e = i - q * A.experts, b1 = min(n_wg, (q + 1) * per);
-        int c = 0;
-#pragma unroll 4
-        for (int b = q * per; b < b1; ++b) c += A.hist[(size_t)b * A.experts + e];
-        part[i] = c;
+        int all = 0, mine = 0;
+#pragma unroll 8
+        for (int b = q * per; b < b1; ++b) {
+            const int v = A.hist[(size_t)b * A.experts + e];
+            all += v;
+            mine += b < own ? v : 0;
+        }
+        part[i] = all;
+        part[runs * A.experts + i] = mine;
     }
     __syncthreads();
     for (int e = tid; e < A.experts; e += 1024) {
-        int c = 0;
-        for (int q = 0; q < runs; ++q) { const int v = part[q * A.experts + e]; part[q * A.experts + e] = c; c += v; }
-        icnt[e] = c;
+        int all = 0, mine = 0;
+        for (int q = 0; q < runs; ++q) { all += part[q * A.experts + e]; mine += part[(runs + q) * A.experts + e]; }
+        icnt[e] = all;
+        before[e] = mine;
     }
     __syncthreads();
-    ob_route_offsets(A, icnt, scan, tid);
+    ob_route_offsets(A, icnt, scan, tid, blockIdx.x == 0);
     __syncthreads();
-    for (int i = tid; i < runs * A.experts; i += 1024) {
-        const int q = i / A.experts, e = i - q * A.experts, b1 = min(n_wg, (q + 1) * per);
-        int c = icnt[e] + part[i];
-        for (int b = q * per; b < b1; ++b) {
-            int *h = A.hist + (size_t)b * A.experts + e;
-            const int v = *h;
-            *h = c;
-            c += v;
-        }
-    }
-}
-
-// third pass: every token's row
-__global__ __launch_bounds__(256) void ob_route_rows_kernel(const ObRouteArgs A)
-{
-    extern __shared__ int icnt[];                                     // [experts]
-    const int tid = threadIdx.x, t0 = blockIdx.x * OB_MOE_TOKENS, t1 = min(A.T, t0 + OB_MOE_TOKENS);
-    for (int e = tid; e < A.experts; e += 256) icnt[e] = A.hist[(size_t)blockIdx.x * A.experts + e];
+    for (int e = tid; e < A.experts; e += 1024) icnt[e] += before[e];
     __syncthreads();
-    for (int i = t0 * A.top + tid; i < t1 * A.top; i += 256) {
+    for (int i = t0 * A.top + tid; i < t1 * A.top; i += 1024) {
         const int e = A.tok_row[i];
         if (e < 0) continue;
-        const int r = atomicAdd(&icnt[e], 1);
+        const int r = atomicAdd(&icnt[e], 1);                         // (the order within an expert is free: every row is computed alone)
         A.gather[r] = i / A.top;
         A.tok_row[i] = r;
     }

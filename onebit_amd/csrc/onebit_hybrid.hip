@@ -237,7 +237,7 @@ static int make_plan(const onebit_hmodel_t &m, int64_t rows, int64_t n_out, int 
                 P.ez_rows = std::max<int64_t>({P.ez_rows, S, OB_EZ_ROWS});
                 ae = std::max<int64_t>(ae, S * 8 * f.nt_expert);
                 // tok_row, tok_w, gather | id_w | hist | blocks
-                rt = std::max<int64_t>(rt, 2 * R * f.top + S + R + cdiv(R, OB_MOE_TOKENS) * f.experts + 4 * (std::min<int64_t>(f.experts, R * f.top) + R * f.top / 64 + 2));
+                rt = std::max<int64_t>(rt, 2 * R * f.top + S + R + cdiv(R, OB_MOE_FEW) * f.experts + 4 * (std::min<int64_t>(f.experts, R * f.top) + R * f.top / 64 + 2));
             }
             as = std::max<int64_t>(as, R * 16 * L.side.nt);
         }
@@ -328,7 +328,7 @@ static int check_model(const onebit_hmodel_t *m)
                     return hfail(ONEBIT_E_SHAPE, "hybrid: layer %d: router sizes", i);
                 ObRouteArgs ra = {};
                 ra.experts = f.experts; ra.identity = f.identity; ra.groups = f.groups;
-                ra.top = f.top;
+                ra.top = f.top; ra.tokens = OB_MOE_TOKENS;
                 if (n > OB_MOE_MAX || ob_route_lds(ra) > 150 * 1024) return hfail(ONEBIT_E_SHAPE, "hybrid: layer %d: too many experts", i);
             }
             if (L.side.nt < 0 || (L.side.nt & 1) || (L.side.nt && (!L.side.w_gate || !L.side.w_proj || !L.side.norm_w || !L.side.table || L.side.dim <= 0 ||
@@ -874,7 +874,9 @@ static int ff_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, const o
     int32_t *at = (int32_t *)(ws + P.route);
     r.z = (const float *)(ws + P.aux); r.ldz = 16 * f.nt_aux; r.correction = f.correction;
     r.T = T; r.experts = f.experts; r.identity = f.identity; r.top = f.top; r.groups = f.groups; r.keep = f.keep;
-    const int n_wg = (int)cdiv(T, OB_MOE_TOKENS);
+    // one token a wave, unless their counts would keep a workgroup of the second pass (1024 threads) longer than that gains
+    r.tokens = T > OB_MOE_TOKENS && cdiv(T, OB_MOE_FEW) * f.experts <= 16 * 1024 ? OB_MOE_FEW : OB_MOE_TOKENS;
+    const int n_wg = (int)cdiv(T, r.tokens);
     r.blk = (ObRowBlock *)at; at += 4 * n_blk;
     r.tok_row = at; at += TK;
     r.tok_w = (float *)at; at += TK;
@@ -893,8 +895,7 @@ static int ff_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, const o
 #undef OB_ROUTE
     if (n_wg > 1) {
         const int runs = std::max(1, 1024 / f.experts);
-        hipLaunchKernelGGL(ob_route_scan_kernel, dim3(1), dim3(1024), f.experts * 4 * (runs + 1), s, r, n_wg, runs);
-        hipLaunchKernelGGL(ob_route_rows_kernel, dim3((unsigned)n_wg), dim3(256), f.experts * 4, s, r);
+        hipLaunchKernelGGL(ob_route_place_kernel, dim3((unsigned)cdiv(T, OB_MOE_TOKENS)), dim3(1024), ob_route_place_lds(r, runs), s, r, n_wg, runs);
     }
     if (int rc = hstatus("router")) return rc;
     ObDenseArgs u = {};
