@@ -26,6 +26,9 @@ struct ObSsmArgs {
     const int32_t *row_slot, *row_pos;
     int row0;                                  // runs: row0 + blockIdx.y (single tokens) or the segment table
     int heads, groups, N, P, sp, taps, ch, n_slots, max_len;
+    // decode steps whose output product applies the norm (ob_few_gated_out_kernel; columns P in whole slices of 32): y silu(gate) norm weight leaves as that product's
+    // operand, its squares' sums before the weight as [rows][workgroups of a row]; y then stays NULL
+    const float *gnorm_w; void *act; int act_nkt; float *sq;
 };
 
 #define OB_SSM_MAXSEG 64
@@ -151,6 +154,11 @@ __global__ __launch_bounds__(256) void ob_ssm_step_kernel(const ObSsmArgs A, con
     for (int t = 0; t < sg.n; ++t) {
         const int row = sg.row0 + t, pos = sg.past + t;
         if (t == 0 && npx < 32) for (int i = tid; i < 32; i += 256) xs[i] = 0.f;
+        float gate = 0.f, gw = 0.f;
+        if (A.sq && tid < npx) {                                       // (the gate: the leading columns of the input product)
+            gate = (float)((const E *)A.u)[(size_t)row * A.ldu + h * A.P + p0 + tid];
+            gw = A.gnorm_w[h * A.P + p0 + tid];
+        }
         if (t > 0 || npx < 32) __syncthreads();
         for (int i = tid; i < nch; i += 256) {
             const int c = chan(i);
@@ -190,7 +198,18 @@ __global__ __launch_bounds__(256) void ob_ssm_step_kernel(const ObSsmArgs A, con
             float s[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int k = 0; k < 32; ++k) s[k & 3] += yc[32 * k];
-            ((E *)A.y)[(size_t)row * A.ldy + h * A.P + p0 + tid] = (E)__builtin_fmaf(Dh, xs[tid], (s[0] + s[1]) + (s[2] + s[3]));
+            const float yv = __builtin_fmaf(Dh, xs[tid], (s[0] + s[1]) + (s[2] + s[3]));
+            if (A.sq) {                                                // (uniform; 32 lanes of the first wave)
+                const float v = yv * ob_silu<E>(gate);
+                ((E *)A.act)[ob_frag<E>(row, h * A.P + p0 + tid, A.act_nkt)] = (E)(v * gw);
+                float ss = v * v;
+                ss += OB_DPP_F(ss, 0xB1, 0xF);
+                ss += OB_DPP_F(ss, 0x4E, 0xF);
+                ss += OB_DPP_F(ss, 0x141, 0xF);
+                ss += OB_DPP_F(ss, 0x140, 0xF);                        // (every lane of 16 holds their sum)
+                ss += __shfl_xor(ss, 16);
+                if (tid == 0) A.sq[(size_t)row * gridDim.x + blockIdx.x] = ss;
+            } else ((E *)A.y)[(size_t)row * A.ldy + h * A.P + p0 + tid] = (E)yv;
         }
     }
 #pragma unroll

@@ -478,6 +478,15 @@ static int attention_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, 
     return hstatus("prompt attention");
 }
 
+// Decode steps whose output product applies the state-space mixer's norm (ob_few_gated_out_kernel): bf16, up to 64 rows (the skinny products' range), one group
+// of whole slices without padded columns, as many square sums as 16-byte pieces.  (Groups of their own, 8 of them at 4096 columns, keep the norm's launch: a
+// wave's k tiles would be cut at every group.)
+static bool few_gated(const onebit_hmodel_t &m, const onebit_hlayer_t &L, const onebit_hstate_t &st)
+{
+    return m.dtype == ONEBIT_HYB_BF16 && L.kind == ONEBIT_MIX_SSM && st.n_rows <= OB_SKINNY_T && st.n_dec == st.n_rows && L.norm_groups == 1 &&
+           L.vdim % 32 == 0 && L.heads * (L.vdim / 32) % 4 == 0 && L.heads * L.vdim == L.mix_k;
+}
+
 template <typename E>
 static int ssm_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, const onebit_hrun_t &run, const onebit_hstate_t &st, const HPlan &P, char *ws,
                       void *act, int act_nkt, hipStream_t s)
@@ -493,9 +502,12 @@ static int ssm_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, const 
         else if (L.state <= 256) hipLaunchKernelGGL((ob_ssm_step_kernel<E, 8>), grid, dim3(256), 0, s, aa, sg);
         else hipLaunchKernelGGL((ob_ssm_step_kernel<E, 16>), grid, dim3(256), 0, s, aa, sg);
     };
+    const bool gated = few_gated(m, L, st);
     if (st.n_dec) {
+        if (gated) { a.gnorm_w = L.gnorm_w; a.act = act; a.act_nkt = act_nkt; a.sq = (float *)(ws + P.y); a.y = nullptr; }      // (1 / 16 of y's room)
         step(a, ObSsmSegs{}, st.n_dec);
         if (int rc = hstatus("state-space decode")) return rc;
+        if (gated) return 0;
     }
     if (st.n_seg) {
         const int rest = st.n_rows - st.n_dec;
@@ -1018,7 +1030,19 @@ static int step_impl(const onebit_hmodel_t &m, const onebit_hstate_t &st, const 
         o.w = L.w_out; o.a = act; o.n_tiles = ldz / 16; o.nkt = act_nkt; o.T = T;
         pend = nb;
         pend.z = (float *)(ws + P.z); pend.z_split = (size_t)T * ldz; pend.bias = L.b_out; pend.post_w = L.post1_w;
-        if (int rc = part_launch<E>(o, (float *)(ws + P.z), pend.n_split, s)) return rc;
+        if (few_gated(m, L, st)) {
+            ObFewGatedOutArgs f = {};
+            static_cast<ObDenseArgs &>(f) = o;
+            f.z = (float *)(ws + P.z); f.ldz = 16 * o.n_tiles; f.z_split = (size_t)T * f.ldz;
+            f.kt_split = (int)cdiv(o.nkt, gemm_splits(o.n_tiles, o.nkt, T));
+            pend.n_split = (int)cdiv(o.nkt, f.kt_split);
+            f.sq = (const float *)(ws + P.y); f.n_sq = L.heads * (L.vdim / 32); f.mix_nkt = L.mix_k / KT; f.inner = (float)(L.heads * L.vdim); f.eps = m.eps;
+            const dim3 grid((unsigned)cdiv(o.n_tiles, 2), (unsigned)pend.n_split);
+            if (T <= 16) hipLaunchKernelGGL(ob_few_gated_out_kernel<1>, grid, dim3(256), 0, s, f);
+            else if (T <= 32) hipLaunchKernelGGL(ob_few_gated_out_kernel<2>, grid, dim3(256), 0, s, f);
+            else hipLaunchKernelGGL(ob_few_gated_out_kernel<4>, grid, dim3(256), 0, s, f);
+            if (int rc = hstatus("output product")) return rc;
+        } else if (int rc = part_launch<E>(o, (float *)(ws + P.z), pend.n_split, s)) return rc;
         if (L.form == ONEBIT_LAYER_SEQUENTIAL) {
             const onebit_hff_t &f = L.ff;
             if (f.nt_plain || f.nt_gated || f.experts) {
