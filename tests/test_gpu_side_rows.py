@@ -25,6 +25,26 @@ def test_rows_of_a_prompt(name):
     raw = raw_config([layer(mlp), layer(dense(40)), layer(mlp)], width=width, side=side, vocab=130)
     m, w = build(raw, BF)
     eng = m.step_engine(2, 160)
-    for T in (65, 80, 97, 144):                                        # (five workgroups of 16 rows, the last with one; whole ones)
+    for T in (65, 80, 97, 144):                                        # (one row a workgroup; the last band of 16 with one row, whole)
         toks = tokens(T, 130, T)
         assert err(run(eng, 0, 0, toks), R.forward(raw, w, toks)) < (TOL[BF] if width > 32 else 0.047), T
+
+
+@pytest.mark.parametrize("name", ["half a wave", "one more", "full"])
+def test_rows_of_a_workgroup(name):
+    """Steps of 4096 rows (16 a workgroup on 256 CUs), 4100 (nine, two rounds; the last workgroup with five) and 700 (three) against the same prompts one at a
+    time, one to six rows a workgroup.  Products split otherwise move single bf16 roundings (2^-9) of what follows: 2 % of a row's norm, as in
+    test_gpu_hybrid_rows.py; a row in another's place shows as 100 %."""
+    width, mlp, side = FORMS[name]
+    m, _ = build(raw_config([layer(mlp), layer(dense(40))], width=width, side=side, vocab=130), BF)
+    eng = m.step_engine(4, 1408, max_rows=4100)
+    prompts = [tokens(n, 130, n) for n in (1404, 1300, 1000, 396)]
+    for lens in ((1400, 1300, 1000, 396), (1404, 1300, 1000, 396), (240, 222, 170, 68)):
+        batch = [p[:n] for p, n in zip(prompts, lens)]
+        eng.launch([(i, 0, p, len(p)) for i, p in enumerate(batch)])
+        whole, row = eng.logits[:sum(map(len, batch))].clone(), 0
+        for i, p in enumerate(batch):
+            eng.launch([(i, 0, p, len(p))])
+            few, many = eng.logits[:len(p)], whole[row:row + len(p)]
+            assert float(((many - few).norm(dim=1) / few.norm(dim=1)).max()) < 2e-2, (lens, i)
+            row += len(p)
