@@ -156,7 +156,7 @@ __global__ __launch_bounds__(1024) void ob_few_route_kernel(const ObFewRowArgs A
 #pragma unroll
         for (int e = 0; e < 4; ++e) x[e] = x[e] * r * (A.off + nw[e]);
     }
-    if (c < A.p.nkt * 32) {                                            // (nkt 32 - W < 32: no wave without columns of the row)
+    if (c < A.p.nkt * 32) {                                            // (zeros behind the row, by waves without columns of it too)
         const ob_bf4 h = on ? ob_to_v4<__bf16>(x) : (ob_bf4)(__bf16)0.f;
         *reinterpret_cast<ob_bf4 *>(row + c) = h;
         if (on) *reinterpret_cast<ob_bf4 *>((__bf16 *)A.out_rm + (size_t)t * A.ld_rm + c) = h;

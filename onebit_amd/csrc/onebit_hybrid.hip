@@ -816,7 +816,8 @@ static bool few_side(const onebit_hmodel_t &m, const onebit_hlayer_t &L, const o
 {
     if (m.dtype != ONEBIT_HYB_BF16 || m.width > 32 * OB_FEW_SIDE_KT || (L.side.nt != 2 && L.side.nt != 4) || a.embed || a.emb_save || a.emb_add || a.bias) return false;
     if (st.n_rows > OB_SKINNY_T) return m.width % 32 == 0 && m.width_pad == m.width && (!a.top || a.eo);      // ob_side_rows_kernel: whole k tiles
-    return m.width % 4 == 0 && !a.eo && (!a.top || (a.ez && few_experts(m, L, st.n_rows)));
+    // (no k tile without columns of the row: the kernel's waves write the columns they have, their last tile's padding included)
+    return m.width % 4 == 0 && m.width_pad - m.width < 32 && !a.eo && (!a.top || (a.ez && few_experts(m, L, st.n_rows)));
 }
 static int few_side_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, const onebit_hstate_t &st, const ObXRowArgs &a, const float *next_w, void *out, hipStream_t s)
 {

@@ -6,6 +6,7 @@ close are left out (``clear_choices``)."""
 import pytest
 import torch
 
+from onebit_amd import hybrid
 from oracle import serotar_ref as R
 from test_gpu_serotar import BF, TOL, build, clear_choices, err, only, rows_err, run, tokens
 from test_serotar_cpu import dense, layer, moe, raw_config
@@ -85,3 +86,21 @@ def test_decoded_rows_of_latent_attention(name):
         eng.launch([(i, 0, toks[:p]) for i, p in enumerate(at)])
         eng.launch([(i, p, toks[p:p + 1]) for i, p in enumerate(at)])
         assert err(eng.logits[:n], ref[at]) < TOL[BF], n
+
+
+@pytest.mark.parametrize("pad", [512, 33024])
+def test_more_padding_than_the_width_needs(pad, monkeypatch):
+    """A model whose rows are padded by whole waves of columns, and beyond what a workgroup's default LDS holds: both are the C interface's to accept."""
+    true_up = hybrid._up
+    monkeypatch.setattr(hybrid, "_up", lambda n, m: pad if (n, m) == (68, 32) else true_up(n, m))
+    raw = raw_config([layer(moe(4, 4, 2, None, 24, 32)), layer(dense(40)), layer(moe(4, 4, 2, None, 24, 32))], width=68, vocab=130)
+    m, w = build(raw, BF)
+    assert m.width_pad == pad
+    eng = m.step_engine(2, 80)
+    for T in (1, 16, 64, 70):
+        toks = tokens(T, 130, T)
+        ref, ok = clear_choices(raw, w, toks, 0.04)
+        got = run(eng, 0, 0, toks)
+        assert bool(torch.isfinite(got).all()), T
+        if bool(ok.any()):
+            assert err(got, ref, ok) < TOL[BF], T
