@@ -624,7 +624,10 @@ static int latent_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, con
             hipLaunchKernelGGL(pk, dim3((unsigned)T), dim3((unsigned)std::min<int64_t>(T <= 256 ? 1024 : 512, rup(cdiv(n_in, vec ? 4 : 1), 64))), plds, s, p);
             return hstatus("latent norms");
         };
-        if (vec && T > OB_SKINNY_T && n_in <= 2048) {                 // many rows: a wave each
+        // many rows: a wave each.  Fewer leave a CU one or two waves, which then wait for a whole row's splits (512, 1024 and 2048 columns, a workgroup a
+        // row / a wave: 200 rows 3.4 / 4.5, 4.2 / 6.5 and 6.5 / 16.4 us; 900 rows 4.7 / 4.7, 6.4 / 6.4, 9.2 / 11.8; 1300 rows 4.8 / 4.8, 7.0 / 6.1, 10.7 / 10.8;
+        // 2000 rows 5.8 / 4.9, 7.9 / 6.8, 13.2 / 11.4)
+        if (vec && n_in <= 2048 && T >= (n_in <= 1024 ? OB_MANY_ROWS : OB_MANY_ROWS * 3 / 2)) {
             const dim3 rgrid((unsigned)cdiv(T, 4));
             if (n_in <= 1024) hipLaunchKernelGGL((ob_lat_prep_rows_kernel<E, 4>), rgrid, dim3(256), 0, s, p, T);
             else hipLaunchKernelGGL((ob_lat_prep_rows_kernel<E, 8>), rgrid, dim3(256), 0, s, p, T);
