@@ -62,9 +62,11 @@ struct ObHNormArgs {
     int W;
 };
 
-// (the workgroup is as wide as the row allows, up to 1024 threads: at one to 64 rows its few dependent passes ARE the launch's time)
+// (the workgroup is as wide as the row allows, up to 1024 threads: at one to 64 rows its few dependent passes ARE the launch's time.  Eight waves a SIMD, that
+// is two workgroups a CU, here and in ob_xrow_kernel's plain form: with a scalar register too many there is room for seven, one workgroup at a time.  Plain form
+// of 4096 columns, 300 / 500 / 900 rows: 11.9 / 14.3 / 20.0 -> 9.9 / 11.5 / 16.9 us; here 900 rows of 2048 columns 9.7 -> 8.6)
 template <typename E, int VEC>
-__global__ __launch_bounds__(1024) void ob_hnorm_kernel(const ObHNormArgs A)
+__global__ __launch_bounds__(1024, 8) void ob_hnorm_kernel(const ObHNormArgs A)
 {
     extern __shared__ __attribute__((aligned(16))) float sm[];        // [W] row | [16] reduction
     float *red = sm + ((A.W + 3) & ~3);
@@ -198,7 +200,7 @@ struct ObXRowArgs : ObHNormArgs {
 // KIND: what can be there besides the sum of splits (smaller code: at a few rows a launch's time is its chain of fetches, instructions included)
 enum ObXKind { OB_X_PLAIN = 0, OB_X_EXPERTS = 1, OB_X_DEPTH = 2, OB_X_BOTH = 3, OB_X_EMBED = 4 };
 template <typename E, int VEC, bool ONE, int KIND>
-__global__ __launch_bounds__(1024) void ob_xrow_kernel(const ObXRowArgs A)
+__global__ __launch_bounds__(1024, KIND == OB_X_PLAIN ? 8 : 4) void ob_xrow_kernel(const ObXRowArgs A)
 {
     constexpr int NH = 8;
     constexpr bool EMB = KIND == OB_X_EMBED, EXP = (KIND & 1) != 0, DEP = (KIND & 2) != 0;
