@@ -700,7 +700,7 @@ __global__ __launch_bounds__(256, MT >= 2 ? 2 : 3) void ob_few_gated_out_kernel(
             if (part == 0) {                                           // 1 / rms of row lane & 15 of the token tile
                 const float *p = A.sq + (size_t)min(m * 16 + (lane & 15), A.T - 1) * A.n_sq;
                 ob_float4 q = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll (MT == 1 ? 8 : 2)
+#pragma unroll(MT == 1 ? 8 : 2)
                 for (int j = 4 * (lane >> 4); j < A.n_sq; j += 16) q += *reinterpret_cast<const ob_float4 *>(p + j);
                 float v = (q[0] + q[1]) + (q[2] + q[3]);
                 v += __shfl_xor(v, 16);

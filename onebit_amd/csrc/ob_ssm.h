@@ -124,8 +124,8 @@ __global__ __launch_bounds__(256) void ob_conv_rows_kernel(const ObSsmArgs A, co
     }
 }
 
-// ---- token by token.  Thread = (4 state columns, every 32nd state row): NI rows in registers
-template <typename E, int NI>
+// ---- token by token.  Thread = (4 state columns, every 32nd state row): NI rows in registers.  GATED: the form whose output product applies the norm
+template <typename E, int NI, bool GATED>
 __global__ __launch_bounds__(256) void ob_ssm_step_kernel(const ObSsmArgs A, const ObSsmSegs SG)
 {
     constexpr int NMAX = NI * 32;
@@ -155,7 +155,7 @@ __global__ __launch_bounds__(256) void ob_ssm_step_kernel(const ObSsmArgs A, con
         const int row = sg.row0 + t, pos = sg.past + t;
         if (t == 0 && npx < 32) for (int i = tid; i < 32; i += 256) xs[i] = 0.f;
         float gate = 0.f, gw = 0.f;
-        if (A.sq && tid < npx) {                                       // (the gate: the leading columns of the input product)
+        if (GATED && tid < npx) {                                      // (the gate: the leading columns of the input product)
             gate = (float)((const E *)A.u)[(size_t)row * A.ldu + h * A.P + p0 + tid];
             gw = A.gnorm_w[h * A.P + p0 + tid];
         }
@@ -199,7 +199,7 @@ __global__ __launch_bounds__(256) void ob_ssm_step_kernel(const ObSsmArgs A, con
 #pragma unroll
             for (int k = 0; k < 32; ++k) s[k & 3] += yc[32 * k];
             const float yv = __builtin_fmaf(Dh, xs[tid], (s[0] + s[1]) + (s[2] + s[3]));
-            if (A.sq) {                                                // (uniform; 32 lanes of the first wave)
+            if constexpr (GATED) {                                     // (32 lanes of the first wave)
                 const float v = yv * ob_silu<E>(gate);
                 ((E *)A.act)[ob_frag<E>(row, h * A.P + p0 + tid, A.act_nkt)] = (E)(v * gw);
                 float ss = v * v;

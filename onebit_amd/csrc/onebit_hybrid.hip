@@ -201,6 +201,7 @@ static int act_index(const HPlan &P, const onebit_hlayer_t &L)
 #define OB_LAT_PARTS 1024       // (row, split) pairs of the latent decode attention with more than one split
 #define OB_SIDE_SPLITS 4        // K splits of a token input's gate product
 #define OB_FEW_LATENT 32        // rows of the merged launches of latent attention
+#define OB_FEW_GATED 32         // rows of a state-space layer's output product with the norm in it
 #define OB_FEW_QUERY 200        // weight tiles of a head's query product that four workgroups read each (half of them for more than 16 rows)
 #define OB_FEW_SIDE_KT 64       // ... of a layer's end, which has two products
 #define OB_FEW_KT 128           // k tiles of a product in a row kernel (of up to 64 columns)
@@ -478,12 +479,14 @@ static int attention_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, 
     return hstatus("prompt attention");
 }
 
-// Decode steps whose output product applies the state-space mixer's norm (ob_few_gated_out_kernel): bf16, up to 64 rows (the skinny products' range), one group
-// of whole slices without padded columns, as many square sums as 16-byte pieces.  (Groups of their own, 8 of them at 4096 columns, keep the norm's launch: a
-// wave's k tiles would be cut at every group.)
+// Decode steps whose output product applies the state-space mixer's norm (ob_few_gated_out_kernel): bf16, up to OB_FEW_GATED rows, one group of whole slices
+// without padded columns, as many square sums as 16-byte pieces.  (Groups of their own, 8 of them at 4096 columns, keep the norm's launch: a wave's k tiles
+// would be cut at every group.)  More rows: every wave adds up all rows' square sums, which then takes what the launch did.  A step of four layers, two of them
+// state-space, with the launch / without: 2048 columns, 1 / 16 / 32 / 48 / 64 rows 184 / 224 / 278 / 349 / 382 and 179 / 217 / 277 / 351 / 384 us; 1024 columns,
+// 1 / 32 / 33 / 64 rows 115 / 157 / 168.5 / 197 and 112 / 154 / 168.8 / 199
 static bool few_gated(const onebit_hmodel_t &m, const onebit_hlayer_t &L, const onebit_hstate_t &st)
 {
-    return m.dtype == ONEBIT_HYB_BF16 && L.kind == ONEBIT_MIX_SSM && st.n_rows <= OB_SKINNY_T && st.n_dec == st.n_rows && L.norm_groups == 1 &&
+    return m.dtype == ONEBIT_HYB_BF16 && L.kind == ONEBIT_MIX_SSM && st.n_rows <= OB_FEW_GATED && st.n_dec == st.n_rows && L.norm_groups == 1 &&
            L.vdim % 32 == 0 && L.heads * (L.vdim / 32) % 4 == 0 && L.heads * L.vdim == L.mix_k;
 }
 
@@ -495,19 +498,23 @@ static int ssm_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, const 
     const int inner = L.heads * L.vdim, ch = inner + 2 * L.groups * L.state, ldy = (int)rup(inner, 8), ldx = (int)rup(ch, 8), nsl = (int)cdiv(L.vdim, 32);
     ObSsmArgs a = {ws + P.u, 16 * L.nt_mix, inner, nullptr, ldx, (const float *)(ws + P.aux), 16 * L.nt_aux, L.conv_w, L.conv_b, L.dt_bias, L.A_log, L.D,
                    (float *)run.s0, run.s1, ws + P.y, ldy, st.row_slot, st.row_pos, 0, L.heads, L.groups, L.state, L.vdim, L.sp, L.taps, ch, m.n_slots, m.max_len};
-    auto step = [&](const ObSsmArgs &aa, const ObSsmSegs &sg, int n) {
+    auto launch = [&](auto form, const ObSsmArgs &aa, const ObSsmSegs &sg, int n) {
+        constexpr bool G = decltype(form)::value;
         const dim3 grid((unsigned)(L.heads * nsl), (unsigned)n);
-        if (L.state <= 64) hipLaunchKernelGGL((ob_ssm_step_kernel<E, 2>), grid, dim3(256), 0, s, aa, sg);
-        else if (L.state <= 128) hipLaunchKernelGGL((ob_ssm_step_kernel<E, 4>), grid, dim3(256), 0, s, aa, sg);
-        else if (L.state <= 256) hipLaunchKernelGGL((ob_ssm_step_kernel<E, 8>), grid, dim3(256), 0, s, aa, sg);
-        else hipLaunchKernelGGL((ob_ssm_step_kernel<E, 16>), grid, dim3(256), 0, s, aa, sg);
+        if (L.state <= 64) hipLaunchKernelGGL((ob_ssm_step_kernel<E, 2, G>), grid, dim3(256), 0, s, aa, sg);
+        else if (L.state <= 128) hipLaunchKernelGGL((ob_ssm_step_kernel<E, 4, G>), grid, dim3(256), 0, s, aa, sg);
+        else if (L.state <= 256) hipLaunchKernelGGL((ob_ssm_step_kernel<E, 8, G>), grid, dim3(256), 0, s, aa, sg);
+        else hipLaunchKernelGGL((ob_ssm_step_kernel<E, 16, G>), grid, dim3(256), 0, s, aa, sg);
     };
-    const bool gated = few_gated(m, L, st);
+    auto step = [&](const ObSsmArgs &aa, const ObSsmSegs &sg, int n) { launch(std::false_type(), aa, sg, n); };
+    if constexpr (sizeof(E) == 2) if (few_gated(m, L, st)) {
+        a.gnorm_w = L.gnorm_w; a.act = act; a.act_nkt = act_nkt; a.sq = (float *)(ws + P.y); a.y = nullptr;      // (1 / 16 of y's room)
+        launch(std::true_type(), a, ObSsmSegs{}, st.n_dec);
+        return hstatus("state-space decode");
+    }
     if (st.n_dec) {
-        if (gated) { a.gnorm_w = L.gnorm_w; a.act = act; a.act_nkt = act_nkt; a.sq = (float *)(ws + P.y); a.y = nullptr; }      // (1 / 16 of y's room)
         step(a, ObSsmSegs{}, st.n_dec);
         if (int rc = hstatus("state-space decode")) return rc;
-        if (gated) return 0;
     }
     if (st.n_seg) {
         const int rest = st.n_rows - st.n_dec;
@@ -1043,8 +1050,7 @@ static int step_impl(const onebit_hmodel_t &m, const onebit_hstate_t &st, const 
             f.sq = (const float *)(ws + P.y); f.n_sq = L.heads * (L.vdim / 32); f.mix_nkt = L.mix_k / KT; f.inner = (float)(L.heads * L.vdim); f.eps = m.eps;
             const dim3 grid((unsigned)cdiv(o.n_tiles, 2), (unsigned)pend.n_split);
             if (T <= 16) hipLaunchKernelGGL(ob_few_gated_out_kernel<1>, grid, dim3(256), 0, s, f);
-            else if (T <= 32) hipLaunchKernelGGL(ob_few_gated_out_kernel<2>, grid, dim3(256), 0, s, f);
-            else hipLaunchKernelGGL(ob_few_gated_out_kernel<4>, grid, dim3(256), 0, s, f);
+            else hipLaunchKernelGGL(ob_few_gated_out_kernel<2>, grid, dim3(256), 0, s, f);
             if (int rc = hstatus("output product")) return rc;
         } else if (int rc = part_launch<E>(o, (float *)(ws + P.z), pend.n_split, s)) return rc;
         if (L.form == ONEBIT_LAYER_SEQUENTIAL) {

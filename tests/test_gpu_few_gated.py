@@ -1,4 +1,4 @@
-"""Decode steps of a state-space layer whose output product applies the mixer's norm (bf16, up to 64 rows), against the plain restatement
+"""Decode steps of a state-space layer whose output product applies the mixer's norm (bf16, up to 32 rows), against the plain restatement
 (oracle/lebepel_ref.py, float64).
 
 ``TOL`` (test_gpu_hybrid.py): bf16 activations, 2^-9 relative each; the product's operand is rounded before the row's factor 1 / rms instead of after it, once
