@@ -825,7 +825,10 @@ static int few_experts_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L
 static bool few_side(const onebit_hmodel_t &m, const onebit_hlayer_t &L, const onebit_hstate_t &st, const ObXRowArgs &a)
 {
     if (m.dtype != ONEBIT_HYB_BF16 || m.width > 32 * OB_FEW_SIDE_KT || (L.side.nt != 2 && L.side.nt != 4) || a.embed || a.emb_save || a.emb_add || a.bias) return false;
-    if (st.n_rows > OB_SKINNY_T) return m.width % 32 == 0 && m.width_pad == m.width && (!a.top || a.eo);      // ob_side_rows_kernel: whole k tiles
+    // ob_side_rows_kernel: whole k tiles.  Without experts fewer of the separate launches' bytes stay away, and up to 1024 columns a launch is short (a step of
+    // four layers, separate / one launch, 65 / 96 / 128 / 200 / 320 rows: no experts, 2048 columns 478 / 497 / 524 / 541 / 612 and 489 / 501 / 525 / 539 / 597 us,
+    // 1024 columns 424 / 429 / 440 / 461 / 476 and 375 / 378 / 392 / 410 / 424; experts, 2048 columns 838 / 875 / 939 / 954 / 1011 and 801 / 837 / 895 / 910 / 964)
+    if (st.n_rows > OB_SKINNY_T) return m.width % 32 == 0 && m.width_pad == m.width && (a.top ? a.eo != nullptr : m.width <= 1024 || st.n_rows >= 128);
     // (no k tile without columns of the row: the kernel's waves write the columns they have, their last tile's padding included)
     return m.width % 4 == 0 && m.width_pad - m.width < 32 && !a.eo && (!a.top || (a.ez && few_experts(m, L, st.n_rows)));
 }
