@@ -181,7 +181,7 @@ struct ObFewSideArgs : ObXRowArgs {
     const void *table; int ld_table, dim;          // entry (tokens[t], n), n < dim
     const float *side_w;
 };
-// grid (rows), 1024 threads; W <= 4096, W % 4 == 0.  The row kernel behind a feed-forward (KIND: with experts or not), the token's own input (gate product,
+// grid (rows), 1024 threads; W <= 2048 (eight n tiles of the output product a wave), W % 4 == 0, top <= 64.  The row kernel behind a feed-forward (KIND: with experts or not), the token's own input (gate product,
 // gelu times the token's table row, output product, its norm, residual) and the row kernel behind that (depth average, next norm): what the row leaves for
 // the next layer, in one launch.  12 rows of 2048 columns, 64 of the token input (256 KB of weights for either product, a CU takes them at 64 bytes a clock):
 // 11.4 us, for launches of 6.6 + 4.6 + 4.7 + 5.0.
@@ -227,10 +227,7 @@ __global__ __launch_bounds__(1024) void ob_few_side_kernel(const ObFewSideArgs A
 #pragma unroll
                 for (int e = 0; e < 4; ++e) s[e] = __builtin_fmaf(wj, v[e], s[e]);
             };
-            const auto weight = [&](int k) {
-                if (k < 64) return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, tw), k));
-                return A.tok_row[t * A.top + k] >= 0 ? A.tok_w[t * A.top + k] : 0.f;
-            };
+            const auto weight = [&](int k) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, tw), k)); };
 #pragma unroll
             for (int j = 0; j < 8; ++j) if (j < A.top) add(weight(j), y[j]);
             for (int sp = 0; sp < A.ez_n; ++sp)
@@ -259,29 +256,23 @@ __global__ __launch_bounds__(1024) void ob_few_side_kernel(const ObFewSideArgs A
     }
     __syncthreads();
     const float pre = ob_few_multiply(w, A.p, row, part, tid);
-    // the output product's tiles: n tiles wave, wave + 16, .. of this wave, eight (and all their k tiles) at a time
+    // the output product's tiles: n tiles wave, wave + 16, .. of this wave and all their k tiles (n tiles there are not: the last one again)
     ob_bf8 wq[8 * KQ];
-    const auto fetch = [&](int n0) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
+    for (int i = 0; i < 8; ++i)
 #pragma unroll
-            for (int k = 0; k < KQ; ++k) wq[i * KQ + k] = *reinterpret_cast<const ob_bf8 *>((const char *)A.q.w + (size_t)(uint32_t)(min(n0 + 16 * i, nq - 1) * KQ + k) * 1024 + lane * 16);
-    };
-    fetch(wave);
+        for (int k = 0; k < KQ; ++k) wq[i * KQ + k] = *reinterpret_cast<const ob_bf8 *>((const char *)A.q.w + (size_t)(uint32_t)(min(wave + 16 * i, nq - 1) * KQ + k) * 1024 + lane * 16);
     if (wave == 0) formed[lane] = (__bf16)(lane < A.dim ? ob_gelu_tanh<__bf16>(pre) * entry : 0.f);
     __syncthreads();
     ob_bf8 f[KQ];
 #pragma unroll
     for (int k = 0; k < KQ; ++k) f[k] = *reinterpret_cast<const ob_bf8 *>(formed + k * 32 + (lane >> 4) * 8);
-    for (int n0 = wave; n0 < nq; n0 += 128) {                          // (wave-uniform)
-        if (n0 != wave) fetch(n0);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            ob_float4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < 8; ++i) {
+        ob_float4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int k = 0; k < KQ; ++k) acc = ObElem<__bf16>::mma(wq[i * KQ + k], f[k], acc);
-            if (n0 + 16 * i < nq && (lane & 15) == 0) *reinterpret_cast<ob_float4 *>(out + (n0 + 16 * i) * 16 + (lane >> 4) * 4) = acc;
-        }
+        for (int k = 0; k < KQ; ++k) acc = ObElem<__bf16>::mma(wq[i * KQ + k], f[k], acc);
+        if (wave + 16 * i < nq && (lane & 15) == 0) *reinterpret_cast<ob_float4 *>(out + (wave + 16 * i) * 16 + (lane >> 4) * 4) = acc;
     }
     const bool depth = A.hist && A.dwa;                                // (uniform)
     ob_float4 sw, nw, h[NH];
@@ -587,12 +578,9 @@ __global__ __launch_bounds__(512) void ob_few_value_kernel(const ObFewValueArgs 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, g = lane >> 4, ld = A.rp + 8, pieces = A.rp >> 3;
     const int h = blockIdx.x, n = blockIdx.y * 2 + (wave & 1), k0 = wave >> 1;
     const ob_bf8 *wp = (const ob_bf8 *)A.w + ((size_t)h * A.nt + min(n, A.nt - 1)) * A.nkt * 64 + lane;
-    ob_bf8 w[4];                                                       // (rank 512: 16 k tiles)
-    const auto fetch = [&](int k) {                                    // (tiles there are not: the last one again)
+    ob_bf8 w[4];                                                       // (at most rank 512: 16 k tiles; tiles there are not: the last one again)
 #pragma unroll
-        for (int u = 0; u < 4; ++u) w[u] = wp[(size_t)min(k + 4 * u, A.nkt - 1) * 64];
-    };
-    fetch(k0);
+    for (int u = 0; u < 4; ++u) w[u] = wp[(size_t)min(k0 + 4 * u, A.nkt - 1) * 64];
     for (int i = tid; i < A.T * pieces; i += 512) {
         const int t = i / pieces, d = (i - t * pieces) * 8, slot = A.row_slot[t], pos = A.row_pos[t];
         float o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -648,15 +636,12 @@ __global__ __launch_bounds__(512) void ob_few_value_kernel(const ObFewValueArgs 
         acc[m] = (ob_float4){0.f, 0.f, 0.f, 0.f};
         xr[m] = ctx + min(m * 16 + lr, A.T - 1) * ld + g * 8;
     }
-    for (int k = k0; k < A.nkt; k += 16) {
-        if (k != k0) fetch(k);
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-            if (k + 4 * u < A.nkt) {                                   // (wave-uniform)
+    for (int u = 0; u < 4; ++u)
+        if (k0 + 4 * u < A.nkt) {                                      // (wave-uniform)
 #pragma unroll
-                for (int m = 0; m < MT; ++m) acc[m] = ObElem<__bf16>::mma(w[u], *reinterpret_cast<const ob_bf8 *>(xr[m] + (k + 4 * u) * 32), acc[m]);
-            }
-    }
+            for (int m = 0; m < MT; ++m) acc[m] = ObElem<__bf16>::mma(w[u], *reinterpret_cast<const ob_bf8 *>(xr[m] + (k0 + 4 * u) * 32), acc[m]);
+        }
     if (k0) {
 #pragma unroll
         for (int m = 0; m < MT; ++m) red[wave - 2][m][lane] = acc[m];
@@ -689,6 +674,7 @@ __global__ __launch_bounds__(256, MT >= 2 ? 2 : 3) void ob_few_gated_out_kernel(
 #pragma unroll
     for (int m = 0; m < MT; ++m) acc[0][m] = acc[1][m] = (ob_float4){0.f, 0.f, 0.f, 0.f};
     const int mid = max(k0, min(k1, A.mix_nkt));
+    constexpr int SU = MT == 1 ? 8 : 2;
 #pragma unroll 1
     for (int part = 0; part < 2; ++part) {                             // the mixer's k tiles, the others (a wave mostly has one of them)
         const int a = part ? mid : k0, b = part ? k1 : mid;
@@ -700,7 +686,7 @@ __global__ __launch_bounds__(256, MT >= 2 ? 2 : 3) void ob_few_gated_out_kernel(
             if (part == 0) {                                           // 1 / rms of row lane & 15 of the token tile
                 const float *p = A.sq + (size_t)min(m * 16 + (lane & 15), A.T - 1) * A.n_sq;
                 ob_float4 q = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll(MT == 1 ? 8 : 2)
+#pragma unroll SU
                 for (int j = 4 * (lane >> 4); j < A.n_sq; j += 16) q += *reinterpret_cast<const ob_float4 *>(p + j);
                 float v = (q[0] + q[1]) + (q[2] + q[3]);
                 v += __shfl_xor(v, 16);

@@ -203,8 +203,8 @@ static int act_index(const HPlan &P, const onebit_hlayer_t &L)
 #define OB_FEW_LATENT 32        // rows of the merged launches of latent attention
 #define OB_FEW_GATED 32         // rows of a state-space layer's output product with the norm in it
 #define OB_FEW_QUERY 200        // weight tiles of a head's query product that four workgroups read each (half of them for more than 16 rows)
-#define OB_FEW_SIDE_KT 64       // ... of a layer's end, which has two products
 #define OB_FEW_KT 128           // k tiles of a product in a row kernel (of up to 64 columns)
+#define OB_FEW_SIDE_KT 64       // ... of a layer's end, which has two products
 #define OB_EZ_ROWS 4096         // fp32 rows of the experts' partial sums at least
 // rows of the experts' sorted space: every (token, choice), each expert's first row at a multiple of 16
 static int64_t expert_rows(const onebit_hff_t &f, int64_t T) { return T * f.top + 16 * std::min<int64_t>(f.experts, T * f.top); }
@@ -601,7 +601,10 @@ static int latent_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, con
         n_abs = st.n_dec;
         for (first = 0; first < st.n_short; ++first) n_abs += st.segs[first].n;
     }
-    // few rows, all of the absorbed form: norms and both products of the queries in one launch; the splits' outputs together within the value product
+    // few rows, all of the absorbed form: norms and both products of the queries in one launch; the splits' outputs together within the value product.  A head's
+    // weights are read by four workgroups, with more than 16 rows' norms and products on top (two layers of 2048 columns, separate / one launch: 256 tiles
+    // 1 / 8 / 16 rows 166 / 215 / 239 and 167 / 214 / 240 us, 384 tiles 168 / 219 / 247 and 175 / 222 / 252; four layers, 192 tiles, 17 / 24 / 32 rows 438 / 458 / 473
+    // and 446 / 468 / 488)
     const bool few = l.tiled && n_abs == T && T <= OB_FEW_LATENT, few_q = few && vec && L.kp / 16 * cq_nkt <= (T <= 16 ? OB_FEW_QUERY : OB_FEW_QUERY / 2)
                        && 64 * (ob_few_query_ld(l.q_rank) + ob_few_query_ld(L.kp)) <= 150 * 1024;      // (LDS at 32 rows)
     float *z = (float *)(ws + P.z);
@@ -820,8 +823,10 @@ static int few_experts_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L
 }
 
 // The end of a sequential layer, from its feed-forward's products (`a`) to the next layer's operand, in one launch: up to 64 rows ob_few_side_kernel, more
-// ob_side_rows_kernel.  Up to 2048 columns and 64 of the token input: every workgroup reads both weights whole (512 KB, 3.4 us; 2 MB at 4096 x 128 would be
-// 14, a few rows' separate launches take 21; a prompt's row of 4096 columns does not fit the registers).  Many rows: whole k tiles (the others' separate launches)
+// ob_side_rows_kernel.  Up to 64 columns of the token input: eight n tiles' weights do not fit the 128 registers of a thread of 1024 beside the rest.  Up to 2048
+// columns: a prompt's row of more does not fit the registers, and a few rows' workgroup has eight n tiles of the output product a wave.  (Few rows with rounds of
+// eight, two layers with experts, separate / one launch, 1 / 8 / 16 / 32 / 64 rows: 2560 columns 189 / 249 / 272 / 326 / 389 and 186 / 242 / 269 / 314 / 369 us, 4096
+// columns 265 / 425 / 520 / 599 / 711 and 254 / 417 / 523 / 585 / 689, 12 rows 501 and 507.)
 static bool few_side(const onebit_hmodel_t &m, const onebit_hlayer_t &L, const onebit_hstate_t &st, const ObXRowArgs &a)
 {
     if (m.dtype != ONEBIT_HYB_BF16 || m.width > 32 * OB_FEW_SIDE_KT || (L.side.nt != 2 && L.side.nt != 4) || a.embed || a.emb_save || a.emb_add || a.bias) return false;
