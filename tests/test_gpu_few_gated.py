@@ -22,16 +22,21 @@ FORMS = {"small": (dict(heads=2, groups=1, state=16, vdim=64, norm_groups=1), 40
 
 @pytest.mark.parametrize("name", FORMS)
 def test_decoded_rows(name):
-    """1 .. 64 requests, one token each at positions from the first on; 17 and 33 in buckets with idle rows."""
+    """1 .. 64 requests, one token each at positions from the first on, in engines of as many slots and of more: then rows without a request, behind which the
+    prompts' operands and square sums lie, share a token tile with live ones."""
     mix, width = FORMS[name]
     raw = raw_config([ssm(**mix), att(heads=2, kv_heads=2), ssm(**mix)], width=width, max_positions=64)
     m, w = build(raw, BF)
     toks = tokens(60, 61)
     ref = R.forward(raw, w, toks)
-    for n in (1, 2, 16, 17, 32, 33, 64):
+    for n, slots in ((1, 1), (1, 16), (2, 2), (2, 16), (16, 16), (17, 17), (17, 20), (17, 32), (32, 32), (33, 33), (33, 48), (64, 64)):
         at = [int(round(x)) for x in torch.linspace(59 if n == 1 else 0, 59, n).tolist()]
-        eng = m.step_engine(n, 64, max_rows=max(n, sum(at)))
+        eng = m.step_engine(slots, 64, max_rows=max(slots, sum(at)))
         if any(at):
             eng.launch([(i, 0, toks[:p]) for i, p in enumerate(at) if p])
+        if slots > n:                                                  # (and a step of every row)
+            eng.launch([(i, at[i] if i < n else 0, toks[at[i]:at[i] + 1] if i < n else toks[:1]) for i in range(slots)])
+            for i, p in enumerate(at):
+                eng.launch([(i, 0, toks[:p])] if p else [(i, 0, toks[:1])])
         eng.launch([(i, p, toks[p:p + 1]) for i, p in enumerate(at)])
-        assert err(eng.logits[:n], ref[at]) < TOL[BF], n
+        assert err(eng.logits[:n], ref[at]) < TOL[BF], (n, slots)

@@ -20,6 +20,17 @@ FORMS = {"one wave": (64, moe(6, 2, 2, (4, 2), 24, 32), 10), "four tiles": (260,
          "wider than any": (4100, moe(10, 2, 0, None, 32, 0), 12)}
 
 
+def clear_tokens(raw, w, T):
+    """T tokens, their logits, and at which of them no choice of experts is close: more than a third of the positions (the first seed with one)."""
+    for seed in (T, T + 1000, T + 2000):
+        toks = tokens(T, 130, seed)
+        ref, ok = clear_choices(raw, w, toks, 0.04)
+        if bool(ok.any()):
+            break
+    assert int(ok.sum()) > T // 3
+    return toks, ref, ok
+
+
 @pytest.mark.parametrize("name", FORMS)
 def test_rows_of_a_step(name):
     width, mlp, side = FORMS[name]
@@ -27,10 +38,8 @@ def test_rows_of_a_step(name):
     m, w = build(raw, BF)
     eng = m.step_engine(2, 80)
     for T in (1, 2, 16, 17, 33, 64):
-        toks = tokens(T, 130, T)
-        ref, ok = clear_choices(raw, w, toks, 0.04)
-        if bool(ok.any()):
-            assert err(run(eng, 0, 0, toks), ref, ok) < TOL[BF], T
+        toks, ref, ok = clear_tokens(raw, w, T)
+        assert err(run(eng, 0, 0, toks), ref, ok) < TOL[BF], T
 
 
 def test_decoded_rows_with_idle_ones():
@@ -51,7 +60,8 @@ def test_decoded_rows_with_idle_ones():
 
 
 def test_rows_do_not_change_each_other():
-    """A row of a step is the same bits alone, among 15 others and in a step of other order: sums run over a row, whatever its neighbours."""
+    """A row of a step is the same bits alone (with rows without a request beside it, and as an engine's only row), among 15 others and in a step of other
+    order: sums run over a row, whatever its neighbours.  (Sums of six k tiles at most: none is split here, however many rows there are.)"""
     raw = raw_config([layer(moe(12, 3, 4, (4, 2), 40, 64))], width=192, vocab=140)
     m, _ = build(raw, BF)
     eng = m.step_engine(16, 40)
@@ -62,7 +72,11 @@ def test_rows_do_not_change_each_other():
     eng.launch([(i, 6, [i + 3]) for i in reversed(range(16))])
     assert torch.equal(eng.logits[:16].flip(0), together)
     eng.launch([(9, 6, [12])])
-    assert float((eng.logits[0] - together[9]).abs().max()) <= 1e-2 * float(together[9].abs().max())      # (splits of the sums follow the number of rows)
+    assert torch.equal(eng.logits[0], together[9])
+    one = m.step_engine(1, 40)
+    one.launch([(0, 0, prompts[9])])
+    one.launch([(0, 6, [12])])
+    assert torch.equal(one.logits[0], together[9])
 
 
 # heads, sizes and ranks: rp 64 .. 512, padded columns everywhere, heads beyond a group of 16, more n tiles than waves, absorbing products of 1, 4 and 5 k tiles,
@@ -98,9 +112,7 @@ def test_more_padding_than_the_width_needs(pad, monkeypatch):
     assert m.width_pad == pad
     eng = m.step_engine(2, 80)
     for T in (1, 16, 64, 70):
-        toks = tokens(T, 130, T)
-        ref, ok = clear_choices(raw, w, toks, 0.04)
+        toks, ref, ok = clear_tokens(raw, w, T)
         got = run(eng, 0, 0, toks)
         assert bool(torch.isfinite(got).all()), T
-        if bool(ok.any()):
-            assert err(got, ref, ok) < TOL[BF], T
+        assert err(got, ref, ok) < TOL[BF], T

@@ -70,16 +70,17 @@ def test_native_batched_step_on_7b_shaped_layers():
             assert abs(float(lg[got[j]] - lg[ref[j]])) < 2e-2 * float(lg.abs().max()), (rid, j)
 
 
-@pytest.mark.parametrize("batch,vocab", [(5, 1000), (32, 32000), (48, 4099)])
-def test_batched_lm_head_and_argmax_inside_the_step(batch, vocab):
+# (hidden sizes in chunks of 256 columns: two; an odd number; the last one part-filled behind others, of an odd and an even number)
+@pytest.mark.parametrize("batch,vocab,hidden", [(5, 1000, 512), (32, 32000, 512), (48, 4099, 512), (29, 4099, 768), (48, 1000, 704), (5, 1000, 832), (20, 1000, 1216)])
+def test_batched_lm_head_and_argmax_inside_the_step(batch, vocab, hidden):
     """onebit_decode_step_batched with next_tokens: the fp16 logits of every slot against the dense
     product of the step's own final-norm output with lm_head (fp32 accumulate -> fp16, as
     modeling_bitllama.py:1610 computes them), and the greedy token = argmax (first index on ties)."""
     from onebit_amd.engine import BatchedDecodeStep
     from onebit_amd.llama import OneBitLlamaConfig, build_synthetic_model
     dev = torch.device("cuda:0")
-    cfg = OneBitLlamaConfig(vocab_size=vocab, hidden_size=512, intermediate_size=1408, num_hidden_layers=1,
-                            num_attention_heads=8, max_position_embeddings=32)
+    cfg = OneBitLlamaConfig(vocab_size=vocab, hidden_size=hidden, intermediate_size=1408, num_hidden_layers=1,
+                            num_attention_heads=hidden // 64, max_position_embeddings=32)
     model = build_synthetic_model(cfg, seed=21, device=dev)
     shape = (batch, cfg.num_key_value_heads, 16, cfg.head_dim)
     caches = [(torch.zeros(shape, device=dev, dtype=torch.float16), torch.zeros(shape, device=dev, dtype=torch.float16))]
