@@ -244,7 +244,9 @@ template <typename E> __global__ __launch_bounds__(256) void ob_table_rows_kerne
 }
 
 // The sums of ob_skinny_stream without DEEP, into acc[2][MT]: U k tiles on the way while U are multiplied.  Text, because the compiler orders it otherwise when it
-// comes out of a function (decode steps of 17-64 rows then take 0.3-0.6 % longer: 4096 columns, two layers, 17 / 48 rows 309.5 / 429.5 us, 310.6 / 430.7).
+// comes out of a function.  bf16 is faster as text (hybrid decode steps of 17-64 rows 0.3-0.6 %: 4096 columns, two layers, 17 / 48 rows 309.5 / 429.5 us, 310.6 /
+// 430.7 as a function), float32 of more than 16 rows as a function (1024 columns, two layers, 17 / 32 rows
+// 384 / 413 us as text, 371 / 401; 4 / 12 rows 260 / 304 as text, 261 / 305).
 #define OB_SKINNY_LOOP \
     V16 wc[2][U], ac[MT][U], wn[2][U], an[MT][U];                                                              \
     auto fetch = [&](V16 (&wd)[2][U], V16 (&ad)[MT][U], int k) {                                               \
@@ -375,7 +377,7 @@ __global__ __launch_bounds__(256, MT >= 4 ? 2 : 3) void ob_dense_skinny_kernel(c
         else ap[m] = (const V16 *)A.a + lane + (size_t)((t0 >> 4) + m) * A.nkt * 64;
     }
     ob_float4 acc[2][MT];
-    if constexpr (DEEP) ob_skinny_stream<E, MT, KSTEP, true>(w0, w1, ap, k0, k1, acc);
+    if constexpr (DEEP || (sizeof(E) == 4 && MT > 1)) ob_skinny_stream<E, MT, KSTEP, DEEP>(w0, w1, ap, k0, k1, acc);
     else {
         constexpr int U = MT >= 4 ? 2 : 4;
 #pragma unroll

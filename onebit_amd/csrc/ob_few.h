@@ -5,7 +5,7 @@
 //                        rows in the choices by itself (no row lists, no block table, no launch that makes them)
 //   ob_few_query_kernel  latent attention from its input product to the absorbed queries: both norms, the cache's new entry, query product, absorbing product
 //   ob_few_value_kernel  the splits of its context together, and the product that makes the heads' outputs of them
-//   ob_few_gated_out_kernel  a parallel layer's output product behind a state-space mixer, with the mixer's norm
+//   ob_few_gated_out_kernel  the output product behind a state-space mixer, with the mixer's norm
 // Rows of the experts' space here are the choices themselves: row t * top + k is choice k of token t.
 #pragma once
 #include "ob_hrows.h"
@@ -655,10 +655,10 @@ __global__ __launch_bounds__(512) void ob_few_value_kernel(const ObFewValueArgs 
     }
 }
 
-// The output product of a parallel layer with a state-space mixer, the mixer's norm (one group) in it: its columns, the first mix_nkt k tiles, come as
+// Up to 32 rows.  The output product of a layer with a state-space mixer, the mixer's norm (one group) in it: its columns, the first mix_nkt k tiles, come as
 // y silu(gate) w without the factor 1 / rms, which a row's sums take after them (the rounding to bf16 is relative: of either product the same).  Else as
-// ob_dense_skinny_kernel.  Takes the norm's launch of 4.6 us off a
-// decode step's layer; 12 rows, 2048 columns of 4096 + 5632: 9.4 us for 8.4 of the product alone, the state-space step 13.0 for 12.2.
+// ob_dense_skinny_kernel.  Takes the norm's launch of 4.6 us off a decode step's layer; 12 rows, 2048 columns of 4096 + 5632: 9.4 us for 8.4 of the product
+// alone, the state-space step 13.0 for 12.2; 24 rows 12.4 for 9.7 and 24.8 for 23.1.
 struct ObFewGatedOutArgs : ObDenseArgs { const float *sq; int n_sq, mix_nkt; float inner, eps; };
 template <int MT>
 __global__ __launch_bounds__(256, MT >= 2 ? 2 : 3) void ob_few_gated_out_kernel(const ObFewGatedOutArgs A)
