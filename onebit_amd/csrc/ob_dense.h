@@ -245,8 +245,8 @@ template <typename E> __global__ __launch_bounds__(256) void ob_table_rows_kerne
 
 // The sums of ob_skinny_stream without DEEP, into acc[2][MT]: U k tiles on the way while U are multiplied.  Text, because the compiler orders it otherwise when it
 // comes out of a function.  bf16 is faster as text (hybrid decode steps of 17-64 rows 0.3-0.6 %: 4096 columns, two layers, 17 / 48 rows 309.5 / 429.5 us, 310.6 /
-// 430.7 as a function), float32 of more than 16 rows as a function (1024 columns, two layers, 17 / 32 rows
-// 384 / 413 us as text, 371 / 401; 4 / 12 rows 260 / 304 as text, 261 / 305).
+// 430.7 as a function), float32 of more than 16 rows as a function (1024 columns, two layers, 17 / 32 rows 384 / 413 us as text, 371 / 401; 4 / 12 rows 260 / 304
+// as text, 261 / 305).
 #define OB_SKINNY_LOOP \
     V16 wc[2][U], ac[MT][U], wn[2][U], an[MT][U];                                                              \
     auto fetch = [&](V16 (&wd)[2][U], V16 (&ad)[MT][U], int k) {                                               \

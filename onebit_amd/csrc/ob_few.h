@@ -181,10 +181,10 @@ struct ObFewSideArgs : ObXRowArgs {
     const void *table; int ld_table, dim;          // entry (tokens[t], n), n < dim
     const float *side_w;
 };
-// grid (rows), 1024 threads; W <= 2048 (eight n tiles of the output product a wave), W % 4 == 0, top <= 64.  The row kernel behind a feed-forward (KIND: with experts or not), the token's own input (gate product,
-// gelu times the token's table row, output product, its norm, residual) and the row kernel behind that (depth average, next norm): what the row leaves for
-// the next layer, in one launch.  12 rows of 2048 columns, 64 of the token input (256 KB of weights for either product, a CU takes them at 64 bytes a clock):
-// 11.4 us, for launches of 6.6 + 4.6 + 4.7 + 5.0.
+// grid (rows), 1024 threads; W <= 2048 (eight n tiles of the output product a wave), W % 4 == 0, top <= 64.  The row kernel behind a feed-forward (KIND: with
+// experts or not), the token's own input (gate product, gelu times the token's table row, output product, its norm, residual) and the row kernel behind that
+// (depth average, next norm): what the row leaves for the next layer, in one launch.  12 rows of 2048 columns, 64 of the token input (256 KB of weights for
+// either product, a CU takes them at 64 bytes a clock): 11.4 us, for launches of 6.6 + 4.6 + 4.7 + 5.0.
 static inline int ob_few_side_lds(const ObFewSideArgs &A) { return A.p.nkt * 64 + 128 + (16 * 64 + 3 * 16 + 16 * ((A.W + 15) / 16)) * 4; }
 template <int KIND, int NT>
 __global__ __launch_bounds__(1024) void ob_few_side_kernel(const ObFewSideArgs A)

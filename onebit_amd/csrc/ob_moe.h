@@ -176,8 +176,8 @@ __global__ __launch_bounds__(1024) void ob_route_kernel(const ObRouteArgs A)
 
 // second pass, 64 tokens a workgroup: every one adds up the counts of all workgroups of the first by itself (what an expert has in all, and before its own
 // tokens; `runs` threads an expert, runs * experts <= 1024, or one), the first one writes the block table, each its tokens' rows.  (A launch of one workgroup for
-// the offsets and one for the rows: 8.5 + 4.8 us of 6095 tokens and 32 experts, now 9.6; the first pass with 16 tokens a workgroup 13.2 -> 7.8 us.  The sums grow with the square of
-// the tokens, but slowly: 512 experts, 2000 / 16000 / 32000 tokens 12.4 / 35 / 60 us in two launches, 6.4 / 14.6 / 38 here.)
+// the offsets and one for the rows: 8.5 + 4.8 us of 6095 tokens and 32 experts, now 9.6; the first pass with 16 tokens a workgroup 13.2 -> 7.8 us.
+// The sums grow with the square of the tokens, but slowly: 512 experts, 2000 / 16000 / 32000 tokens 12.4 / 35 / 60 us in two launches, 6.4 / 14.6 / 38 here.)
 static inline size_t ob_route_place_lds(const ObRouteArgs &A, int runs) { return (size_t)A.experts * (2 + 2 * runs) * 4; }
 __global__ __launch_bounds__(1024) void ob_route_place_kernel(const ObRouteArgs A, int n_wg, int runs)
 {
