@@ -86,37 +86,67 @@ static int gemm_splits(int n_tiles, int nkt, int T)
     return (int)std::max<int64_t>(1, s);
 }
 
-// Time of `x` equal workgroups, two resident per CU, in full rounds of them: half a round of one per CU takes 0.57 (0.42 behind full rounds, whose
-// end it overlaps), more of a round 0.6 + 0.4 of its fill.  (4096 k columns, 128 x 128 tiles: 256 / 320 / 384 / 512 / 752 / 946 / 1024 workgroups 37 / 52 / 55 /
-// 63 / 94 / 118 / 121 us.)
-static double round_cost(int64_t x)
+// Rows of a tile of ob_dense_wr_kernel in 16s, `most` at most, where tiles of mt x 16 rows are tiles_of(mt); 0: ob_dense_mm_kernel's 128 x 128 tiles.
+// The latter where they leave CUs idle: they have twice the column blocks, and a CU takes 49 GB/s of weights from HBM, no more (up to 1900 rows of 9728 ->
+// 2048 76-85 us, 98-104 with 256 columns, whatever their rows; 1000 x 19200 x 4096 172 and 196).  Else by rounds of workgroups, two to a CU up to 128 rows,
+// one from 160 on: a tile's time grows with its rows and a constant, half a round of tiles takes about as long as half their work (1.1), more of one 1.5-2.
+// 152 products of 300-7600 rows, 1024-19200 k columns and 1024-18592 columns, weights from HBM, fp32 sums: 0.3 % above the best rows of each on average
+// (6.8 % at most), 1.18 times as fast as 128 x 128 and 256 x 128 tiles with both operands in LDS (0.97-1.5): 4600 x 9728 x 2048 201 -> 139 us (160 rows),
+// 6016 x 7680 x 2048 178 -> 133 (192), 2300 x 19200 x 4096 406 -> 271 (160), 1500 x 2048 x 18592 119 -> 107 (112), 2600 x 2048 x 2048 29.5 -> 23.7 (96).
+template <typename F> static int wr_rows(int64_t narrow, int most, F tiles_of)
 {
-    const int64_t cus = cu_count(), full = x / (2 * cus), rem = x - full * 2 * cus;
-    return (double)full + (rem == 0 ? 0.0 : rem <= cus ? (full ? 0.42 : 0.57) : 0.6 + 0.2 * (double)rem / (double)cus);
+    const int64_t cus = cu_count();
+    if (narrow <= cus) return 0;
+    int best = 0;
+    double least = 0;
+    for (const int mt : {4, 5, 6, 7, 8, 10, 12, 14, 16}) {
+        if (mt > most) break;
+        const int64_t t = tiles_of(mt), full = t / (2 * cus), rem = t - full * 2 * cus;
+        double c;
+        if (mt > 8) c = 1.05 * (double)cdiv(t, cus) * (mt + 5.6);
+        else if (t <= cus) c = mt + 4.5;
+        else c = 1.04 * (mt + 4.5) * (2.0 * full + (rem == 0 ? 0.0 : rem <= cus ? (full ? 1.1 : 1.0) : 1.0 + 0.5 * (double)rem / (double)cus));
+        if (!best || c < least) { best = mt; least = c; }
+    }
+    return best;
 }
-// the LDS-DMA tiles over `n_tb` blocks of 128 rows.  A round of 256 columns takes 1.8 of one of 128 columns: the wider tiles where they cost less so.
-// (170 products of 128-8192 rows, 1536-11008 columns either way, against the better of the two: 0.999 on average, worst 0.93; 1520 rows of 2048 -> 9728, 912 or 456
-// workgroups, 67 us with 128 columns, 60 with 256; 1800 rows, 1140 or 570, 83 and 89.)  128-column tiles that are all resident, some CUs with two, take
-// ob_dense_tile_kernel up to 7/4 per CU; above, one 256-column tile a CU (weights from HBM, 9728 -> 2048: 384 tiles 111 us against 133, 464 151 against 135;
-// ob_dense_mm_kernel's 128 columns 122-150).  Experts' blocks, of which some are empty and whose rows are gathered: 256 columns from two
-// rounds on (7600 rows, six of 32 experts each, 1408 columns of gate and up: 214 us, 274 with 128)
+// fp32 sums are written while the next tile's products run or not at all; what else a product's output becomes takes a CU's only workgroup 5 us a tile (8
+// prompts' layers of 2048 columns, 9728-19776 columns written: 128 rows 5873 us, 192 6180)
+template <int EPI> constexpr int wr_most() { return EPI == OB_EPI_PART ? 16 : 8; }
+// the LDS-DMA tiles over `n_tb` blocks of 16 mt rows (wr_rows), of 128 with mt = 0.  Experts' blocks have 128 rows; weights to registers from two rounds of them
+// on (12 prompts of 150 rows, 32 experts: 14041 us for them and 16 tokens each, 14069 always, 14186 never)
 template <typename E, int EPI, int ROWS>
-static int tiles_launch(const typename ObDenseArgsOf<ROWS>::type &a, int64_t n_tb, int n_split, const char *what, hipStream_t s)
+static int tiles_launch(const typename ObDenseArgsOf<ROWS>::type &a, int64_t n_tb, int n_split, int mt, const char *what, hipStream_t s)
 {
     const auto go = [&](auto k, int nb, int lds) {
         if (!lds_ok((const void *)k, lds)) return hfail(ONEBIT_E_SHAPE, "%s: LDS", what);
         hipLaunchKernelGGL(k, dim3((unsigned)(cdiv(a.n_tiles, nb) * n_tb), (unsigned)n_split), dim3(256), lds, s, a);
         return hstatus(what);
     };
-    constexpr bool EXPERTS = ROWS == OB_ROWS_GATHER || ROWS == OB_ROWS_SORTED;
-    if constexpr (sizeof(E) == 4) return go(ob_dense_tile_kernel<E, EPI, ROWS>, 8, 4 * 16 * 1024);
+    if constexpr (sizeof(E) == 4) return go(ob_dense_tile_kernel<EPI, ROWS>, 8, 4 * 16 * 1024);
     else {
-        const int64_t cus = cu_count(), wide = cdiv(a.n_tiles, 16) * n_tb * n_split, narrow = cdiv(a.n_tiles, 8) * n_tb * n_split;
-        const bool two = !EXPERTS && narrow > cus && narrow <= 2 * cus;
-        if (EXPERTS ? wide >= 4 * cus : two ? 4 * narrow > 7 * cus && wide <= cus : 1.8 * round_cost(wide) < round_cost(narrow))
-            return go(ob_dense_mm_kernel<EPI, 16, 8, 3, ROWS>, 16, 3 * 24 * 1024);
-        if constexpr (!EXPERTS) if (two) return go(ob_dense_tile_kernel<E, EPI, ROWS>, 8, 4 * 16 * 1024);
-        return go(ob_dense_mm_kernel<EPI, 8, 8, 4, ROWS>, 8, 4 * 16 * 1024);
+        const auto wr = [&]<int MT>() {
+            constexpr int NST = ob_wr_steps(MT);
+            return go(ob_dense_wr_kernel<EPI, MT, NST, ROWS>, 16, NST * MT * 1024);
+        };
+        if constexpr (ROWS == OB_ROWS_GATHER || ROWS == OB_ROWS_SORTED) {
+            if (cdiv(a.n_tiles, 16) * n_tb * n_split >= 2 * (int64_t)cu_count()) return wr.template operator()<8>();
+        } else {
+            switch (mt) {
+            case 4: return wr.template operator()<4>();
+            case 5: return wr.template operator()<5>();
+            case 6: return wr.template operator()<6>();
+            case 7: return wr.template operator()<7>();
+            case 8: return wr.template operator()<8>();
+            }
+            if constexpr (wr_most<EPI>() > 8) switch (mt) {
+            case 10: return wr.template operator()<10>();
+            case 12: return wr.template operator()<12>();
+            case 14: return wr.template operator()<14>();
+            case 16: return wr.template operator()<16>();
+            }
+        }
+        return go(ob_dense_mm_kernel<EPI, ROWS>, 8, 4 * 16 * 1024);
     }
 }
 
@@ -134,7 +164,9 @@ static int dense_launch(ObDenseArgs a, int n_split, hipStream_t s)
         else hipLaunchKernelGGL((ob_dense_skinny_kernel<E, EPI, 4>), grid, dim3(256), 0, s, a);
         return hstatus("dense product");
     }
-    return tiles_launch<E, EPI, OB_ROWS_ALL>(a, cdiv(a.T, 128), n_split, "dense product", s);
+    const int64_t narrow = cdiv(a.n_tiles, 8) * cdiv(a.T, 128) * n_split;
+    const int mt = sizeof(E) == 4 ? 0 : wr_rows(narrow, wr_most<EPI>(), [&](int m) { return cdiv(a.n_tiles, 16) * cdiv(a.T, 16 * m) * n_split; });
+    return tiles_launch<E, EPI, OB_ROWS_ALL>(a, cdiv(a.T, mt ? 16 * mt : 128), n_split, mt, "dense product", s);
 }
 
 // few rows, block-diagonal over heads (row-major activations), 64 rows at a time.  `out_step`: bytes of 64 output rows.
@@ -171,7 +203,7 @@ static int dense_blocks_launch(ObDenseArgs a, int n_blk, int block_rows, int n_s
         return hstatus("expert product");
     }
     a.T = n_blk * block_rows;
-    return tiles_launch<E, EPI, ROWS>(a, n_blk, n_split, "expert product", s);
+    return tiles_launch<E, EPI, ROWS>(a, n_blk, n_split, 0, "expert product", s);
 }
 
 extern "C" int onebit_hybrid_gemm_splits(int32_t n_tiles, int32_t nkt, int32_t T) { return n_tiles > 0 && nkt > 0 && T > 0 ? gemm_splits(n_tiles, nkt, T) : 0; }
@@ -722,21 +754,25 @@ static int latent_launch(const onebit_hmodel_t &m, const onebit_hlayer_t &L, con
             ObDenseSegArgs e = {};
             ObFlashSigArgs f = {};
             int64_t rows = 0;
-            int blocks = 0, i = s0;
+            int i = s0;
             for (; i < st.n_seg && e.nseg < OB_DENSE_MAXSEG; ++i) {
                 const onebit_hseg_t &g = st.segs[i];
                 const int len = g.past + g.n, n = e.nseg;
                 if (rows + rup(len, 16) > P.kv_rows) break;
-                blocks += (int)cdiv(len, 128);
-                e.blk_end[n] = blocks; e.band0[n] = g.slot * bands; e.row0[n] = (int)rows; e.rows[n] = len;
+                e.band0[n] = g.slot * bands; e.row0[n] = (int)rows; e.rows[n] = len;
                 f.seg[n] = {g.row0, g.n, (int)rows, g.past};
                 f.nseg = ++e.nseg;
                 rows += rup(len, 16);
             }
             if (i == s0) return hfail(ONEBIT_E_SHAPE, "latent attention: chunk %d does not fit the expansion buffer", s0);
-            e.w = l.w_kv; e.a = run.s0; e.n_tiles = 2 * H * L.kp / 16; e.nkt = l.rp / KT; e.kt_split = e.nkt; e.T = blocks * 128;
+            e.w = l.w_kv; e.a = run.s0; e.n_tiles = 2 * H * L.kp / 16; e.nkt = l.rp / KT; e.kt_split = e.nkt;
+            const auto blocks_of = [&](int m) { int64_t b = 0; for (int q = 0; q < e.nseg; ++q) b += cdiv(e.rows[q], 16 * m); return b; };
+            const int mt = wr_rows(cdiv(e.n_tiles, 8) * blocks_of(8), wr_most<OB_EPI_HEADS>(), [&](int m) { return cdiv(e.n_tiles, 16) * blocks_of(m); }), br = mt ? 16 * mt : 128;
+            const int64_t blocks = blocks_of(br / 16);
+            for (int q = 0; q < e.nseg; ++q) e.blk_end[q] = (q ? e.blk_end[q - 1] : 0) + (int)cdiv(e.rows[q], br);
+            e.T = (int)blocks * br;
             e.heads = ws + P.kv; e.d_shift = sh; e.head_rows = (int)P.kv_rows;
-            if (const int rc = tiles_launch<E, OB_EPI_HEADS, OB_ROWS_SEGS>(e, blocks, 1, "expansion", s)) return rc;
+            if (const int rc = tiles_launch<E, OB_EPI_HEADS, OB_ROWS_SEGS>(e, blocks, 1, mt, "expansion", s)) return rc;
             f.a.q = (const _Float16 *)(ws + P.qu); f.a.k = (const _Float16 *)(ws + P.kv); f.a.v = f.a.k + (size_t)H * P.kv_rows * L.kp;     // (bf16 behind these pointers)
             f.a.H = f.a.Hkv = H; f.a.max_len = (int)P.kv_rows;
             f.a.scale_log2e = L.scale * OB_LOG2E;

@@ -95,6 +95,25 @@ def test_dense_product_large_tiles(N, T, nkt, splits):
     assert float((z.sum(0) - ref).abs().max()) < 1e-4 * K ** 0.5
 
 
+# weights straight to registers: each number of rows a tile may have (4-8, 10, 12, 14, 16 tiles of 16 at these T), its last tile of rows and the last 256 columns
+# partly filled; k tiles fewer than a turn of 4 or 5 steps, one or two turns and every remainder, split K
+@pytest.mark.parametrize("T", [431, 449, 547, 600, 700, 800, 1001, 1130, 1400, 1601])
+def test_dense_product_tile_heights(T):
+    from onebit_amd import _lib
+    from onebit_amd.hybrid import pack_fragments
+    lib, g, N = _lib.load_hybrid(), torch.Generator(device="cuda").manual_seed(T), 8224
+    for nkt, splits in ((1, 1), (2, 1), (3, 1), (4, 1), (5, 1), (6, 1), (7, 1), (8, 1), (9, 1), (10, 1), (11, 1), (12, 1), (14, 1), (18, 2), (23, 1)):
+        K = 32 * nkt
+        w, a = torch.randn(N, K, generator=g, device="cuda").to(BF), torch.randn(T, K, generator=g, device="cuda").to(BF)
+        wp, ap = pack_fragments(w, BF), torch.zeros(-(-T // 256) * 16, nkt, 64, 8, dtype=BF, device="cuda")
+        ap[:-(-T // 16)] = pack_fragments(a, BF)
+        z = torch.full((splits, T, N), float("nan"), device="cuda")
+        _lib.check_hybrid(lib.onebit_hybrid_gemm(wp.data_ptr(), ap.data_ptr(), z.data_ptr(), 2, N // 16, nkt, T, splits, torch.cuda.current_stream().cuda_stream), "gemm")
+        torch.cuda.synchronize()
+        # (as test_dense_product_long_sums)
+        assert float((z.double().sum(0) - a.double() @ w.double().t()).abs().max()) < 2 ** -22 * K + 2 ** -21, (nkt, splits)
+
+
 # few rows with eight k tiles in flight per wave (from 61 k tiles a split on), every remainder of a wave's share; the others beside them
 @pytest.mark.parametrize("T", [1, 7, 16, 17])
 @DTYPES
