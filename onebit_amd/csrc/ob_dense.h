@@ -10,7 +10,6 @@
 // Products are computed transposed, D[n][t] = sum_k W[n][k] A[t][k]: a lane holds four consecutive output columns n of one token t.
 #pragma once
 #include "ob_mm.h"
-#include <utility>
 
 typedef __bf16 ob_bf4 __attribute__((ext_vector_type(4)));
 
@@ -471,23 +470,12 @@ __global__ __launch_bounds__(256, 2) void ob_dense_mm_kernel(const typename ObDe
     }
 }
 
-// bf16, weights straight into the operand registers: workgroup = 256 columns x 16 MT rows, a wave 64 columns x all rows.  A weight tile then belongs to one
-// wave and LDS carries the activations only: with MT = 8 8 KB written and 32 read for 128 MFMA, where both operands through the LDS take 24 and 48 of the 64 KB
-// that it moves meanwhile.  Up to MT = 8 two workgroups share a CU; above, one has it, all 512 registers, and asks for 32 instead of 48 bytes a clock
-// (MT = 16), which is what bounds the smaller ones (8192^3: MFMA 77 % of the cycles with MT = 16, 70 % with 8, 64 % with both operands in LDS).
-//   * NST steps of weights (16 registers each, refilled behind a step's last MFMA with them) and of activations (LDS) are on the way
-//   * a step runs in two halves with its one barrier between them: there everyone has read all of tile k, and tile k + 1 has landed (counted vmcnt); the
-//     first half's activations of step k + 1 are read in the second half of step k, the second half's in the first
-//   * one load, transfer or LDS read behind an MFMA, never two: an MFMA hides what issues in its 16 cycles
-//   * whole turns of NST steps without a way out between them: where paths meet hipcc waits for every load
-// hipcc does not know that the assembly is an MFMA: an operand it copies (a spill, a full register file) right in front of one is read too early, wrong by whole
-// tiles.  No copy is left with these steps (ob_wr_steps); the sums are those of both operands through LDS, bit for bit, which is how the tests see it.
-constexpr int ob_wr_steps(int mt) { return mt < 8 ? 5 : 4; }
+// bf16, weights straight into the operand registers (ob_mm.h, ob_wr_loop): workgroup = 256 columns x 16 MT rows, a wave 64 columns x all rows.
 template <int EPI, int MT, int NST, int ROWS = OB_ROWS_ALL>
 __global__ __launch_bounds__(256, MT > 8 ? 1 : 2) void ob_dense_wr_kernel(const typename ObDenseArgsOf<ROWS>::type A)
 {
     static_assert(ROWS != OB_ROWS_HEADS && ROWS != OB_ROWS_TABLE, "forms with few rows only");
-    constexpr int NB = 16, MN = 4, PER = (MT + 3) / 4, H = MT / 2;
+    constexpr int NB = 16, MN = 4, PER = (MT + 3) / 4, AK = ROWS == OB_ROWS_GATHER ? 64 : 1024;      // (AK: bytes from k tile to k tile of the rows)
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int nb, tb;
@@ -495,100 +483,26 @@ __global__ __launch_bounds__(256, MT > 8 ? 1 : 2) void ob_dense_wr_kernel(const 
     const int n0 = nb * NB + wave * MN, split = blockIdx.y, k_lo = split * A.kt_split, nk = min(A.nkt - k_lo, A.kt_split);
     const ObDenseRows b = ob_dense_rows<ROWS, MT>(A, tb);
     if (b.rows <= 0) return;                                                         // (uniform)
-    // transfer d of a step moves tile j of the rows (a wave without PER tiles of its own: the last one again)
-    constexpr int AK = ROWS == OB_ROWS_GATHER ? 64 : 1024, C = NST / 2;              // bytes from k tile to k tile; a turn's weights at immediate offsets around the C-th
-    const char *ab[PER];
-    uint32_t aoff[PER];
+    // transfer d of a step moves tile wave PER + d of the rows (a wave without PER tiles of its own: the last one again)
+    const char *ab[PER], *wb[MN];
+    uint32_t aoff[PER], ldst[PER], aof[PER];
+    const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char *)smem;
 #pragma unroll
     for (int d = 0; d < PER; ++d) {
         const ObDenseSrc src = ob_dense_src<__bf16, ROWS, NB>(A, b, n0, k_lo, NB + min(wave * PER + d, MT - 1), lane);
         ab[d] = src.base; aoff[d] = src.lane_off;
+        aof[d] = aoff[d] + (NST - 1) * AK;
+        ldst[d] = lds0 + (uint32_t)min(wave * PER + d, MT - 1) * 1024;
     }
-    const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char *)smem;
-    uint32_t ldst[PER];
-#pragma unroll
-    for (int d = 0; d < PER; ++d) ldst[d] = lds0 + (uint32_t)min(wave * PER + d, MT - 1) * 1024;
-    const char *wb[MN];
 #pragma unroll
     for (int i = 0; i < MN; ++i) wb[i] = (const char *)A.w + (b.w0 + (size_t)min(n0 + i, A.n_tiles - 1) * A.nkt + k_lo) * 1024;
-    ob_u32x4 w[NST][MN], a[MT];
-    // step k's weights / activations, clamped (past the end: the last ones again, nobody uses them); "fast": at a constant distance from k0
-    const auto wload = [&](int i, int k, int u) { w[u][i] = *reinterpret_cast<const ob_u32x4 *>(wb[i] + (size_t)((uint32_t)min(k, nk - 1) * 1024u + (uint32_t)lane * 16u)); };
-    const auto dma = [&](int d, int k, int buf) { ob_dma_1k(ab[d], aoff[d] + (uint32_t)min(k, nk - 1) * AK, ldst[d] + buf * MT * 1024); };
-    const auto ra = [&](int buf, int j) { return *reinterpret_cast<const ob_u32x4 *>(smem + (buf * MT + j) * 1024 + lane * 16); };
     ob_float4 acc[MN][MT];
-#pragma unroll
-    for (int s = 0; s < NST; ++s) {
-#pragma unroll
-        for (int d = 0; d < PER; ++d) if (s < NST - 1) dma(d, s, s);
-#pragma unroll
-        for (int i = 0; i < MN; ++i) wload(i, s, s);
-    }
-#pragma unroll
-    for (int i = 0; i < MN; ++i)
-#pragma unroll
-        for (int j = 0; j < MT; ++j) {
-            acc[i][j] = (ob_float4){0.f, 0.f, 0.f, 0.f};
-            asm volatile("" : "+a"(acc[i][j]));
-        }
-    __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" :: "n"((NST - 2) * (PER + MN) + 2 * MN) : "memory");       // (the zeros above are long written)
-#pragma unroll
-    for (int j = 0; j < H; ++j) a[j] = ra(0, j);
-    const auto step = [&]<bool FAST, int u>(int k0, uint32_t woff, const uint32_t (&aof)[PER]) __attribute__((always_inline)) {
-        // younger than tile k + 1's transfers: weights and activations of NST - 2 steps; lgkmcnt(0)
-        constexpr int VM = (NST - 2) * (PER + MN), WAIT = (VM & 15) | 0x70 | (VM >> 4 << 14), G = MT - H;
-        static_assert(VM + 2 * MN < 64, "vmcnt");
-        constexpr int nu = (u + 1) % NST, pu = (u + NST - 1) % NST;
-#pragma unroll
-        for (int j = 0; j < H; ++j)
-#pragma unroll
-            for (int i = 0; i < MN; ++i) {
-                const int m = j * MN + i;
-                ob_mma_acc<true>(acc[i][j], w[u][i], a[j]);
-                __builtin_amdgcn_sched_barrier(0);
-                if (m % 2 == 0 && m / 2 < G) a[H + m / 2] = ra(u, H + m / 2);
-                if (m % 2 == 1 && m / 2 < PER) {
-                    if constexpr (FAST) ob_dma_1k(ab[m / 2], aof[m / 2] + u * AK, ldst[m / 2] + pu * MT * 1024); else dma(m / 2, k0 + u + NST - 1, pu);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        __builtin_amdgcn_s_waitcnt(WAIT);
-        asm volatile("s_barrier" ::: "memory");
-#pragma unroll
-        for (int i = 0; i < MN; ++i)
-#pragma unroll
-            for (int j = 0; j < G; ++j) {
-                const int m = i * G + j;
-                ob_mma_acc<true>(acc[i][H + j], w[u][i], a[H + j]);
-                __builtin_amdgcn_sched_barrier(0);
-                if (m % 2 == 0 && m / 2 < H) a[m / 2] = ra(nu, m / 2);
-                if (j == G - 1) {
-                    if constexpr (FAST) w[u][i] = *reinterpret_cast<const ob_u32x4 *>(wb[i] + (size_t)woff + (u - C) * 1024); else wload(i, k0 + u + NST, u);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-    };
-    int k = 0;
-    uint32_t woff = (uint32_t)lane * 16u + (NST + C) * 1024, aof[PER];
-#pragma unroll
-    for (int d = 0; d < PER; ++d) aof[d] = aoff[d] + (NST - 1) * AK;
-    const auto turn = [&]<bool FAST, int... U>(std::integer_sequence<int, U...>) __attribute__((always_inline)) { (step.template operator()<FAST, U>(k, woff, aof), ...); };
-    for (; k + 2 * NST <= nk; k += NST) {                                            // (loops without a way out of the middle: hipcc would wait for all loads there)
-        turn.template operator()<true>(std::make_integer_sequence<int, NST>{});
-        woff += NST * 1024;
-#pragma unroll
-        for (int d = 0; d < PER; ++d) aof[d] += NST * AK;
-    }
-    for (; k + NST <= nk; k += NST) turn.template operator()<false>(std::make_integer_sequence<int, NST>{});
-    const auto rest = [&]<int... U>(std::integer_sequence<int, U...>) __attribute__((always_inline)) { ((k + U < nk ? step.template operator()<false, U>(k, woff, aof) : (void)0), ...); };
-    rest(std::make_integer_sequence<int, NST - 1>{});
-    // No transfer may land after the workgroup's LDS is released; the last sums leave the matrix pipe before anything reads them.
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");
-#pragma unroll
-    for (int i = 0; i < MN; ++i)
-#pragma unroll
-        for (int j = 0; j < MT; ++j) asm volatile("" : "+a"(acc[i][j]));
+    ob_wr_loop<true, false, MT, PER, NST>(acc, nk, wb, lane * 16, [&](int buf, int j) { return *reinterpret_cast<const ob_u32x4 *>(smem + (buf * MT + j) * 1024 + lane * 16); },
+        [&](int d, int k, int buf) { ob_dma_1k(ab[d], aoff[d] + (uint32_t)k * AK, ldst[d] + buf * MT * 1024); },
+        [&](int d, int u, int buf) {
+            ob_dma_1k(ab[d], aof[d] + u * AK, ldst[d] + buf * MT * 1024);
+            if (u == NST - 1) aof[d] += NST * AK;
+        });
     const int g = lane >> 4;
 #pragma unroll
     for (int j = 0; j < MT; ++j) {

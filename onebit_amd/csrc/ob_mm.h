@@ -11,6 +11,7 @@
 //     copies a step of 64 MFMAs, a quarter of the time
 #pragma once
 #include "ob_common.h"
+#include <utility>
 
 // Output tile of workgroup `orig` (of at least nnb * ntb; false: none).  Workgroup ids are dealt round-robin to the 8 XCDs, each with its own L2;
 // every XCD takes a contiguous range of tiles numbered in bands of 8 token blocks, token block fastest: the 32-64 tiles in flight on it are about
@@ -85,6 +86,111 @@ __device__ __forceinline__ void ob_mm_loop(ob_float4 (&acc)[MN][MT], int nk, RW 
         }
         buf = nbuf;
     }
+    // No transfer may land after the workgroup's LDS is released; the last sums leave the matrix pipe before anything reads them.
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < MN; ++i)
+#pragma unroll
+        for (int j = 0; j < MT; ++j) asm volatile("" : "+a"(acc[i][j]));
+}
+
+// ---- one operand straight into registers --------------------------------------------------------------------------------------------------------
+// Workgroup = 16 MT x 256 outputs: a wave has 64 of the "direct" operand's, whose tiles go from memory to its registers, times all 16 MT of the other's, which the
+// four waves share through the LDS.  A direct tile belongs to one wave: with MT = 8 the LDS takes 8 KB and gives 32 for 128 MFMA, where both operands through it
+// take 24 and 48 of the 64 KB that it moves meanwhile.  Up to MT = 8 two workgroups share a CU; above, one has it, all 512 registers, and asks for 32 instead
+// of 48 bytes a clock (MT = 16), which is what bounds the smaller ones (8192^3 bf16: MFMA 77 % of the cycles with MT = 16, 70 % with 8, 64 % with both operands in
+// the LDS).
+//   * NST steps of the direct operand (16 registers each, refilled behind a step's last MFMA with them) and of the other (LDS) are on the way
+//   * a step runs in two halves with its one barrier between them: there everyone has read all of tile k, and tile k + 1 has landed (counted vmcnt); the
+//     first half's shared operands of step k + 1 are read in the second half of step k, the second half's in the first
+//   * one load, transfer or LDS read behind an MFMA: an MFMA hides what issues in its 16 cycles
+//   * whole turns of NST steps without a way out between them: where paths meet hipcc waits for every load
+// hipcc does not know that the assembly is an MFMA: an operand that it copies (a spill, a full register file) right in front of one is read too early, wrong by whole
+// tiles.  No copy is left with these numbers of steps; the sums are those of ob_mm_loop, bit for bit.
+constexpr int ob_wr_steps(int mt) { return mt < 8 ? 5 : 4; }
+
+// What a launch of t such workgroups costs by its rounds of them: a tile's time grows with its rows and a constant; half a round of two to a CU takes about as long
+// as half their work (1.1 of it), more of one 1.5-2 tiles' time.  (Fitted to 152 products of the hybrid decoders, onebit_hybrid.hip.)
+static inline double ob_wr_cost(int64_t t, int mt, int64_t cus)
+{
+    if (mt > 8) return 1.05 * (double)((t + cus - 1) / cus) * (mt + 5.6);
+    if (t <= cus) return mt + 4.5;
+    const int64_t full = t / (2 * cus), rem = t - full * 2 * cus;
+    return 1.04 * (mt + 4.5) * (2.0 * (double)full + (rem == 0 ? 0.0 : rem <= cus ? (full ? 1.1 : 1.0) : 1.0 + 0.5 * (double)rem / (double)cus));
+}
+
+// acc[i][j] = sum over nk k steps of direct_i other_j (SWAP: the direct operand is the MFMA's second).  Direct tile i of step k: 16 bytes at wb[i] + 1024 k + wlane.
+// ra(buf, j): operand j of the step in LDS buffer `buf`; dma(d, k, buf): transfer d of this wave's PER of step k < nk into `buf`; dma_next(d, u, buf): the
+// same of step u + NST - 1 behind the turn's first one, in turns one behind the other from the first on.  All waves of the workgroup.
+template <bool BF16, bool SWAP, int MT, int PER, int NST, typename RA, typename DMA, typename DMAN>
+__device__ __forceinline__ void ob_wr_loop(ob_float4 (&acc)[4][MT], int nk, const char *const (&wb)[4], uint32_t wlane, RA ra, DMA dma, DMAN dma_next)
+{
+    constexpr int MN = 4, H = MT / 2, G = MT - H, C = NST / 2, VM = (NST - 2) * (PER + MN), WAIT = (VM & 15) | 0x70 | (VM >> 4 << 14);
+    static_assert(VM + 2 * MN < 64 && 2 * PER <= H * MN && 2 * G <= H * MN + 1 && 2 * H <= G * MN + 1, "vmcnt; places behind MFMAs");
+    ob_u32x4 w[NST][MN], a[MT];
+    // (past the end: the last step's again, nobody uses them)
+    const auto wload = [&](int i, int k, int u) { w[u][i] = *reinterpret_cast<const ob_u32x4 *>(wb[i] + (size_t)((uint32_t)min(k, nk - 1) * 1024u + wlane)); };
+    const auto mma = [&](ob_float4 &c, ob_u32x4 x, ob_u32x4 y) { if constexpr (SWAP) ob_mma_acc<BF16>(c, y, x); else ob_mma_acc<BF16>(c, x, y); };
+#pragma unroll
+    for (int s = 0; s < NST; ++s) {
+#pragma unroll
+        for (int d = 0; d < PER; ++d) if (s < NST - 1) dma(d, min(s, nk - 1), s);
+#pragma unroll
+        for (int i = 0; i < MN; ++i) wload(i, s, s);
+    }
+#pragma unroll
+    for (int i = 0; i < MN; ++i)
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+            acc[i][j] = (ob_float4){0.f, 0.f, 0.f, 0.f};
+            asm volatile("" : "+a"(acc[i][j]));
+        }
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" :: "n"(VM + 2 * MN) : "memory");                       // (the zeros above are long written)
+#pragma unroll
+    for (int j = 0; j < H; ++j) a[j] = ra(0, j);
+    int k = 0;
+    uint32_t woff = wlane + (NST + C) * 1024;                                        // (immediate offsets reach 4 KB either way)
+    const auto step = [&]<bool FAST, int u>() __attribute__((always_inline)) {
+        constexpr int nu = (u + 1) % NST, pu = (u + NST - 1) % NST;
+#pragma unroll
+        for (int j = 0; j < H; ++j)
+#pragma unroll
+            for (int i = 0; i < MN; ++i) {
+                const int m = j * MN + i;
+                mma(acc[i][j], w[u][i], a[j]);
+                __builtin_amdgcn_sched_barrier(0);
+                if (m % 2 == 0 && m / 2 < G) a[H + m / 2] = ra(u, H + m / 2);
+                if (m % 2 == 1 && m / 2 < PER) {
+                    if constexpr (FAST) dma_next(m / 2, u, pu); else dma(m / 2, min(k + u + NST - 1, nk - 1), pu);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        // younger than tile k + 1's transfers: NST - 2 steps' loads of both; lgkmcnt(0)
+        __builtin_amdgcn_s_waitcnt(WAIT);
+        asm volatile("s_barrier" ::: "memory");
+#pragma unroll
+        for (int i = 0; i < MN; ++i)
+#pragma unroll
+            for (int j = 0; j < G; ++j) {
+                const int m = i * G + j;
+                mma(acc[i][H + j], w[u][i], a[H + j]);
+                __builtin_amdgcn_sched_barrier(0);
+                if (m % 2 == 0 && m / 2 < H) a[m / 2] = ra(nu, m / 2);
+                if (j == G - 1) {
+                    if constexpr (FAST) w[u][i] = *reinterpret_cast<const ob_u32x4 *>(wb[i] + (size_t)woff + (u - C) * 1024); else wload(i, k + u + NST, u);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+    };
+    const auto turn = [&]<bool FAST, int... U>(std::integer_sequence<int, U...>) __attribute__((always_inline)) { (step.template operator()<FAST, U>(), ...); };
+    for (; k + 2 * NST <= nk; k += NST) {
+        turn.template operator()<true>(std::make_integer_sequence<int, NST>{});
+        woff += NST * 1024;
+    }
+    for (; k + NST <= nk; k += NST) turn.template operator()<false>(std::make_integer_sequence<int, NST>{});
+    const auto rest = [&]<int... U>(std::integer_sequence<int, U...>) __attribute__((always_inline)) { ((k + U < nk ? step.template operator()<false, U>() : (void)0), ...); };
+    rest(std::make_integer_sequence<int, NST - 1>{});
     // No transfer may land after the workgroup's LDS is released; the last sums leave the matrix pipe before anything reads them.
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");
 #pragma unroll

@@ -5,12 +5,13 @@
 //   S = sign(W)   [N][K]     z = a S^T                       ga = gz S   (reduced over N)
 //   gz            [T][N]     ga = gz S                       gS = gz^T a
 // stored as 1 KB tiles of 16 rows x 32 columns, [16-row band][column tile], zero beyond the matrix up to 32 rows and columns.  Reduced over its
-// columns, a tile is an MFMA operand as it lies (one ds_read_b128); reduced over its rows, two tiles are two operands through the transposing
+// columns, a tile is an MFMA operand as it lies (16 bytes a lane); reduced over its rows, two tiles are two operands through the transposing
 // read (ds_read_b64_tr_b16).  The 16-byte piece (row, g = column / 8) sits at place 16 g + (row ^ 4 (g & 1)): both reads are free of bank
-// conflicts.  Loop, tile shapes and numbering: ob_mm.h.
-// What bounds it: the matrix cores for the products (the kernel that transformed operands on their way from registers to LDS reached 430-510
-// TFLOP/s), memory for the passes.  T = 4096, 4096 -> 11008, forward + backward: 2496 us before, 1227 now; in a trace the products 309-342 (z), 376-410
-// (ga) and 406-446 us (gS) = 1.2 / 0.98 / 0.91 PFLOP/s at best, the passes 215 us at 4-5 TB/s.  64 rows: 811 us before, 320 now.
+// conflicts.  Every product has one operand that lies as it is reduced, and goes straight to registers with it: S for z, gz for ga, and for gS a^T, whose tiles
+// their pass turns.  Loops, tile shapes and numbering: ob_mm.h.
+// What bounds it: the matrix cores and their power for the products, memory for the passes.  T = 4096, 4096 -> 11008, forward + backward: 1217 us with both
+// operands through the LDS, 1037 now; in a trace the products 343 -> 316 (z), 408 -> 282 (ga) and 441 -> 376 us (gS) = 1.17, 1.31 and 0.98 PFLOP/s, the passes
+// 205 us at 4-5 TB/s.
 #pragma once
 #include "ob_mm.h"
 
@@ -27,6 +28,21 @@ __device__ __forceinline__ ob_half8 ob_t16_load(const _Float16 *p, int n)
     return v;
 }
 __device__ __forceinline__ int ob_t16_place(int row, int g) { return (16 * g + (row ^ ((g & 1) << 2))) * 16; }
+
+// MFMA operand i (of two) of a pair of tiles (32 rows x 32 columns at p) reduced over its rows, through the transposing read: this lane's 8 of the rows,
+// column 16 i + lr
+__device__ __forceinline__ ob_u32x4 ob_t16_turned(const char *p, int i, int lr, int lg)
+{
+    typedef short v4s __attribute__((ext_vector_type(4)));
+    typedef short v8s __attribute__((ext_vector_type(8)));
+    typedef __attribute__((address_space(3))) v4s lds_v4s;
+    // rows 8 lg .. + 7 of the 32 (two bands), columns 16 i ..: this lane's piece of a 4-row x 16-column block
+    const int g = 2 * i + ((lr & 3) >> 1), row = 8 * (lg & 1) + (lr >> 2);
+    p += (lg >> 1) * 1024 + 8 * (lr & 1);
+    const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s *)(p + ob_t16_place(row, g)));
+    const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s *)(p + ob_t16_place(row + 4, g)));
+    return __builtin_bit_cast(ob_u32x4, (v8s){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
+}
 
 // x -> a, W -> S: a wave takes four column tiles of a band (256 bytes of each of its 16 rows)
 template <int TX>
@@ -54,6 +70,41 @@ __global__ __launch_bounds__(256) void ob_t16_tiles_kernel(const ObT16Tiles A)
     }
 }
 
+// x -> (x h)^T: tiles of 16 columns x 32 rows of x, [16-column band][32-row tile], the operand's transposing read done here once.  A wave takes 32 rows x four
+// column tiles (256 bytes of each row), lays them into the LDS as the pass above lays them into memory and reads them back turned.
+struct ObT16Turn { const _Float16 *p, *vec; char *out; int rows, cols, rt, ct; };      // rt, ct: tiles of 32 rows / columns
+__global__ __launch_bounds__(256) void ob_t16_turn_kernel(const ObT16Turn A)
+{
+    __shared__ __attribute__((aligned(16))) char smem[4][8 * 1024];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4, cg = (A.ct + 3) >> 2;
+    const int unit = blockIdx.x * 4 + wave, tt = unit % A.rt, c0 = unit / A.rt * 4;
+    if (c0 >= 4 * cg) return;                                          // (wave-uniform; no barrier below)
+    ob_half8 v[2][4], h[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const int col = (c0 + c) * 32 + 8 * g;
+        h[c] = ob_t16_load(A.vec + col, A.cols - col);
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            const int row = tt * 32 + b * 16 + r;
+            v[b][c] = ob_t16_load(A.p + (size_t)row * A.cols + col, row < A.rows ? A.cols - col : 0);
+        }
+    }
+    char *base = smem[wave];
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) *reinterpret_cast<ob_half8 *>(base + (2 * c + b) * 1024 + ob_t16_place(r, g)) = v[b][c] * h[c];
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        if (c0 + c >= A.ct) return;                                    // (wave-uniform)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            *reinterpret_cast<ob_u32x4 *>(A.out + ((size_t)(2 * (c0 + c) + i) * A.rt + tt) * 1024 + ob_t16_place(r, g)) = ob_t16_turned(base + 2 * c * 1024, i, r, g);
+    }
+}
+
 // C[t][n] = sum_r a(t, r) w(n, r).  TRW / TRA: the operand's tiles are reduced over their rows (nw / na count its 16-element groups either way).
 enum { OB_T16_Z = 0, OB_T16_GX = 1, OB_T16_GW = 2 };
 struct ObT16Mm {
@@ -74,10 +125,87 @@ __device__ __forceinline__ float ob_t16_ste(float w)
     return ob_round_h((float)(_Float16)1.001f - t2);
 }
 
-template <int EPI, bool TRW, bool TRA, int NB, int TB, int NST>
+// MN x MT tiles of outputs from column n0, row t0 on: a lane has four columns n0 + 16 i + 4 lg .. of row t0 + 16 j + lr.  `half`: the rows' place in A.part.
+// x / W beside an output are requested 16 tiles ahead: stores lie between the loads, and hipcc leaves them in order (one at a time, the weight gradient's
+// epilogue took 38 us a 256 x 256 tile).
+template <int EPI, int MN, int MT, typename ACC>
+__device__ __forceinline__ void ob_t16_epilogue(const ObT16Mm &A, int n0, int t0, int half, int lane, ACC acc)
+{
+    constexpr int IB = MT >= 16 ? 1 : 16 / MT < MN ? 16 / MT : MN;     // column tiles of a batch
+    const int lr = lane & 15, lg = lane >> 4;
+    const _Float16 *q = EPI == OB_T16_GX ? A.x : A.vec;
+    ob_half4 p[2][IB][MT];
+    const auto fetch = [&](int b) __attribute__((always_inline)) {
+#pragma unroll
+        for (int ii = 0; ii < IB; ++ii)
+#pragma unroll
+            for (int j = 0; j < MT; ++j) {
+                const int n = n0 + (b * IB + ii) * 16 + 4 * lg, left = A.cols - n, t = t0 + j * 16 + lr;
+                ob_half4 v = (ob_half4)(_Float16)0;
+                if (t < A.rows && left > 0) {
+                    if (A.vec4 && left >= 4) v = *reinterpret_cast<const ob_half4 *>(q + (size_t)t * A.cols + n);
+                    else {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) if (e < left) v[e] = q[(size_t)t * A.cols + n + e];
+                    }
+                }
+                p[b & 1][ii][j] = v;
+            }
+    };
+    if (EPI != OB_T16_Z) fetch(0);
+#pragma unroll
+    for (int i = 0; i < MN; ++i) {
+        if (EPI != OB_T16_Z && i % IB == 0 && i + IB < MN) fetch(i / IB + 1);
+        const int n = n0 + i * 16 + 4 * lg, left = A.cols - n;         // four columns, `left` of them inside
+        const bool v4 = A.vec4 && left >= 4;
+        ob_half4 h4 = (ob_half4)(_Float16)0;
+        float sum[4] = {0.f, 0.f, 0.f, 0.f};                           // (scalars: OB_DPP_F of a vector's element reads element 0)
+        if (EPI == OB_T16_GX) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) if (e < left) h4[e] = A.vec[n + e];
+        }
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+            const int t = t0 + j * 16 + lr;
+            if (t >= A.rows || left <= 0) continue;
+            const size_t o = (size_t)t * A.cols + n;
+            ob_half4 c;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) c[e] = (_Float16)acc(i, j)[e];
+            const ob_half4 b = p[i / IB & 1][i % IB][j];
+            if (EPI == OB_T16_GX) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sum[e] += (float)(_Float16)(c[e] * b[e]);
+                c = c * h4;
+            }
+            if (EPI == OB_T16_GW) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) c[e] = (_Float16)((float)c[e] * ob_t16_ste((float)b[e]));
+            }
+            if (v4) *reinterpret_cast<ob_half4 *>(A.C + o) = c;
+            else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) if (e < left) A.C[o + e] = c[e];
+            }
+        }
+        if (EPI == OB_T16_GX) {                                        // over the 16 rows of the lane group
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                sum[e] += OB_DPP_F(sum[e], 0xB1, 0xF);
+                sum[e] += OB_DPP_F(sum[e], 0x4E, 0xF);
+                sum[e] += OB_DPP_F(sum[e], 0x141, 0xF);
+                sum[e] += OB_DPP_F(sum[e], 0x140, 0xF);
+                if (lr == 0 && e < left && half < 2 * ((A.rows + 127) >> 7)) A.part[(size_t)half * A.cols + n + e] = sum[e];
+            }
+        }
+    }
+}
+
+// both operands through the LDS (ob_mm_loop), 128 x 128 outputs: few tiles
+template <int EPI, bool TRW, bool TRA>
 __global__ __launch_bounds__(256, 2) void ob_t16_mm_kernel(const ObT16Mm A)
 {
-    constexpr int TILES = NB + TB, PER = TILES / 4, MN = NB / 2, MT = TB / 2;
+    constexpr int NB = 8, TB = 8, NST = 4, TILES = NB + TB, PER = TILES / 4, MN = NB / 2, MT = TB / 2;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wn = wave & 1, wt = wave >> 1, lr = lane & 15, lg = lane >> 4;
     int nb, tb;
@@ -102,71 +230,52 @@ __global__ __launch_bounds__(256, 2) void ob_t16_mm_kernel(const ObT16Mm A)
     const auto frag = [&](bool tr, int buf, int t0, int i) -> ob_u32x4 {
         const char *base = smem + (buf * TILES + t0) * 1024;
         if (!tr) return *reinterpret_cast<const ob_u32x4 *>(base + i * 1024 + plain);
-        typedef short v4s __attribute__((ext_vector_type(4)));
-        typedef short v8s __attribute__((ext_vector_type(8)));
-        typedef __attribute__((address_space(3))) v4s lds_v4s;
-        // rows 8 lg .. + 7 of the 32 (two bands), columns 16 (i & 1) .. of the 32-column tile i / 2: this lane's piece of a 4-row x 16-column block
-        const int g = 2 * (i & 1) + ((lr & 3) >> 1), row = 8 * (lg & 1) + (lr >> 2);
-        const char *p = base + ((i >> 1) * 2 + (lg >> 1)) * 1024 + 8 * (lr & 1);
-        const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s *)(p + ob_t16_place(row, g)));
-        const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s *)(p + ob_t16_place(row + 4, g)));
-        return __builtin_bit_cast(ob_u32x4, (v8s){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
+        return ob_t16_turned(base + (i >> 1) * 2048, i & 1, lr, lg);
     };
     ob_float4 acc[MN][MT];
     ob_mm_loop<false, MN, MT, PER, NST>(acc, A.nk, [&](int buf, int i) { return frag(TRW, buf, 0, wn * MN + i); },
                                         [&](int buf, int j) { return frag(TRA, buf, NB, wt * MT + j); }, dma);
+    ob_t16_epilogue<EPI, MN, MT>(A, (nb * NB + wn * MN) * 16, (tb * TB + wt * MT) * 16, tb * 2 + wt, lane, [&](int i, int j) -> const ob_float4 & { return acc[i][j]; });
+}
+
+// ... with one operand straight into registers (ob_mm.h, ob_wr_loop): the one that lies as it is reduced, gz for the input gradient (SWAP: it is the MFMA's
+// second operand, so that a lane still has four columns of a row), S and (x h)^T for the others.  TRL: the other one's tiles are reduced over their rows.
+template <int EPI, bool TRL, bool SWAP, int MT>
+__global__ __launch_bounds__(256, MT > 8 ? 1 : 2) void ob_t16_wr_kernel(const ObT16Mm A)
+{
+    constexpr int MN = 4, PER = MT / 4, NST = ob_wr_steps(MT);
+    static_assert(MT % 4 == 0, "pairs of tiles, as many transfers in every wave");
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lr = lane & 15, lg = lane >> 4;
+    const char *dm = SWAP ? A.a : A.w, *lm = SWAP ? A.w : A.a;
+    const int nd = SWAP ? A.na : A.nw, dld = SWAP ? A.ald : A.wld, nl = SWAP ? A.nw : A.na, lld = SWAP ? A.wld : A.ald;
+    int nb, tb;
+    if (!ob_tile_of(blockIdx.x, SWAP ? (nl + MT - 1) / MT : (nd + 15) / 16, SWAP ? (nd + 15) / 16 : (nl + MT - 1) / MT, nb, tb)) return;      // (uniform)
+    const int d0 = (SWAP ? tb : nb) * 16 + wave * MN, l0 = (SWAP ? nb : tb) * MT;
+    const char *src[PER], *nxt[PER], *wb[MN];
+    uint32_t ldst[PER];
+    const size_t step = TRL ? (size_t)lld * 2048 : 1024;
+    const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char *)smem;
 #pragma unroll
-    for (int i = 0; i < MN; ++i) {
-        const int n = (nb * NB + wn * MN + i) * 16 + 4 * lg, left = A.cols - n;      // four columns, `left` of them inside
-        const bool v4 = A.vec4 && left >= 4;
-        ob_half4 h4 = (ob_half4)(_Float16)0;
-        float sum[4] = {0.f, 0.f, 0.f, 0.f};                           // (scalars: OB_DPP_F of a vector's element reads element 0)
-        if (EPI == OB_T16_GX) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) if (e < left) h4[e] = A.vec[n + e];
-        }
-#pragma unroll
-        for (int j = 0; j < MT; ++j) {
-            const int t = (tb * TB + wt * MT + j) * 16 + lr;
-            if (t >= A.rows || left <= 0) continue;
-            const size_t o = (size_t)t * A.cols + n;
-            ob_half4 c, p = (ob_half4)(_Float16)0;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) c[e] = (_Float16)acc[i][j][e];
-            const _Float16 *q = EPI == OB_T16_GX ? A.x : A.vec;
-            if (EPI != OB_T16_Z) {
-                if (v4) p = *reinterpret_cast<const ob_half4 *>(q + o);
-                else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) if (e < left) p[e] = q[o + e];
-                }
-            }
-            if (EPI == OB_T16_GX) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) sum[e] += (float)(_Float16)(c[e] * p[e]);
-                c = c * h4;
-            }
-            if (EPI == OB_T16_GW) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) c[e] = (_Float16)((float)c[e] * ob_t16_ste((float)p[e]));
-            }
-            if (v4) *reinterpret_cast<ob_half4 *>(A.C + o) = c;
-            else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) if (e < left) A.C[o + e] = c[e];
-            }
-        }
-        if (EPI == OB_T16_GX) {                                        // over the 16 rows of the lane group
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                sum[e] += OB_DPP_F(sum[e], 0xB1, 0xF);
-                sum[e] += OB_DPP_F(sum[e], 0x4E, 0xF);
-                sum[e] += OB_DPP_F(sum[e], 0x141, 0xF);
-                sum[e] += OB_DPP_F(sum[e], 0x140, 0xF);
-                if (lr == 0 && e < left) A.part[(size_t)(tb * 2 + wt) * A.cols + n + e] = sum[e];
-            }
-        }
+    for (int d = 0; d < PER; ++d) {
+        const int o = wave * PER + d;
+        src[d] = lm + (TRL ? (size_t)(o & 1) * lld + min(l0 / 2 + (o >> 1), lld - 1) : (size_t)min(l0 + o, nl - 1) * lld) * 1024;
+        nxt[d] = src[d] + (NST - 1) * step;
+        ldst[d] = lds0 + (uint32_t)o * 1024;
     }
+#pragma unroll
+    for (int i = 0; i < MN; ++i) wb[i] = dm + (size_t)min(d0 + i, nd - 1) * dld * 1024;
+    const int plain = ob_t16_place(lr, lg);
+    ob_float4 acc[MN][MT];
+    ob_wr_loop<false, SWAP, MT, PER, NST>(acc, A.nk, wb, plain,
+        [&](int buf, int j) -> ob_u32x4 {
+            if constexpr (TRL) return ob_t16_turned(smem + (buf * MT + (j & ~1)) * 1024, j & 1, lr, lg);
+            else return *reinterpret_cast<const ob_u32x4 *>(smem + (buf * MT + j) * 1024 + plain);
+        },
+        [&](int d, int k, int buf) { ob_dma_1k(src[d] + (size_t)k * step, lane * 16, ldst[d] + buf * MT * 1024); },
+        [&](int d, int, int buf) { ob_dma_1k(nxt[d], lane * 16, ldst[d] + buf * MT * 1024); nxt[d] += step; });
+    if constexpr (SWAP) ob_t16_epilogue<EPI, MT, MN>(A, l0 * 16, d0 * 16, tb * 4 + wave, lane, [&](int i, int j) -> const ob_float4 & { return acc[j][i]; });
+    else ob_t16_epilogue<EPI, MN, MT>(A, d0 * 16, l0 * 16, 0, lane, [&](int i, int j) -> const ob_float4 & { return acc[i][j]; });
 }
 
 // LayerNorm of z g, rows up to 16384 wide in registers (N % 8 == 0, 16-byte aligned): ob_train_ln_fwd_kernel's arithmetic, z read once

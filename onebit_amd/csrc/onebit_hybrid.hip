@@ -88,8 +88,8 @@ static int gemm_splits(int n_tiles, int nkt, int T)
 
 // Rows of a tile of ob_dense_wr_kernel in 16s, `most` at most, where tiles of mt x 16 rows are tiles_of(mt); 0: ob_dense_mm_kernel's 128 x 128 tiles.
 // The latter where they leave CUs idle: they have twice the column blocks, and a CU takes 49 GB/s of weights from HBM, no more (up to 1900 rows of 9728 ->
-// 2048 76-85 us, 98-104 with 256 columns, whatever their rows; 1000 x 19200 x 4096 172 and 196).  Else by rounds of workgroups, two to a CU up to 128 rows,
-// one from 160 on: a tile's time grows with its rows and a constant, half a round of tiles takes about as long as half their work (1.1), more of one 1.5-2.
+// 2048 76-85 us, 98-104 with 256 columns, whatever their rows; 1000 x 19200 x 4096 172 and 196).  Else by rounds of workgroups (ob_wr_cost), two to a CU up
+// to 128 rows, one from 160 on.
 // 152 products of 300-7600 rows, 1024-19200 k columns and 1024-18592 columns, weights from HBM, fp32 sums: 0.3 % above the best rows of each on average
 // (6.8 % at most), 1.18 times as fast as 128 x 128 and 256 x 128 tiles with both operands in LDS (0.97-1.5): 4600 x 9728 x 2048 201 -> 139 us (160 rows),
 // 6016 x 7680 x 2048 178 -> 133 (192), 2300 x 19200 x 4096 406 -> 271 (160), 1500 x 2048 x 18592 119 -> 107 (112), 2600 x 2048 x 2048 29.5 -> 23.7 (96).
@@ -101,11 +101,7 @@ template <typename F> static int wr_rows(int64_t narrow, int most, F tiles_of)
     double least = 0;
     for (const int mt : {4, 5, 6, 7, 8, 10, 12, 14, 16}) {
         if (mt > most) break;
-        const int64_t t = tiles_of(mt), full = t / (2 * cus), rem = t - full * 2 * cus;
-        double c;
-        if (mt > 8) c = 1.05 * (double)cdiv(t, cus) * (mt + 5.6);
-        else if (t <= cus) c = mt + 4.5;
-        else c = 1.04 * (mt + 4.5) * (2.0 * full + (rem == 0 ? 0.0 : rem <= cus ? (full ? 1.1 : 1.0) : 1.0 + 0.5 * (double)rem / (double)cus));
+        const double c = ob_wr_cost(tiles_of(mt), mt, cus);
         if (!best || c < least) { best = mt; least = c; }
     }
     return best;

@@ -34,20 +34,36 @@ static void ob_t16_tiles(bool sign, const void *p, const void *vec, char *out, i
     else hipLaunchKernelGGL(ob_t16_tiles_kernel<OB_T16_SCALE>, dim3(grid), dim3(256), 0, s, a);
 }
 
-// 256 x 128 outputs a workgroup from two rounds of them on (two per CU), else 128 x 128
+static void ob_t16_turn(const void *p, const void *vec, char *out, int64_t rows, int64_t cols, hipStream_t s)
+{
+    ObT16Turn a = {(const _Float16 *)p, (const _Float16 *)vec, out, (int)rows, (int)cols, (int)(ob_t16_up32(rows) / 32), (int)(ob_t16_up32(cols) / 32)};
+    hipLaunchKernelGGL(ob_t16_turn_kernel, dim3((unsigned)(((int64_t)a.rt * ((a.ct + 3) / 4) + 3) / 4)), dim3(256), 0, s, a);
+}
+
+// One operand straight into registers from more 128 x 128 outputs than CUs on, with 128 or 256 of the other operand's, whichever costs less by its rounds.  The
+// weight gradient's epilogue reads W: with 128, whose second workgroup's products run meanwhile (4096 rows, 4096 -> 11008 376 us, 394 with 256), or with 64
+// where it is most of the work, up to 1280 rows (whole step of that layer, 64 / 128: 512 rows 346 / 368 us, 1024 rows 433 / 450, 1500 rows 569 / 563).
+// Both operands through the LDS -> now, 4096 and 1024 rows: z 343 -> 316, 95 -> 89 us, input gradient 408 -> 282, 131 -> 130 (few tiles: as before), weight
+// gradient 441 -> 376, 163 -> 130.
 template <int EPI, bool TRW, bool TRA>
 static void ob_t16_mm(const ObT16Mm &a, hipStream_t s)
 {
-    const int64_t tb = (a.na + 7) / 8, nb = (a.nw + 15) / 16;
-    if (nb * tb >= 4 * (int64_t)ob_cu_count()) {
-        static bool attr_set[OB_MAX_DEVICES] = {};
-        ob_set_max_lds_once(ob_t16_mm_kernel<EPI, TRW, TRA, 16, 8, 3>, attr_set, 3 * 24 * 1024);
-        hipLaunchKernelGGL((ob_t16_mm_kernel<EPI, TRW, TRA, 16, 8, 3>), dim3((unsigned)(nb * tb)), dim3(256), 3 * 24 * 1024, s, a);
-    } else {
-        static bool attr_set[OB_MAX_DEVICES] = {};
-        ob_set_max_lds_once(ob_t16_mm_kernel<EPI, TRW, TRA, 8, 8, 4>, attr_set, 4 * 16 * 1024);
-        hipLaunchKernelGGL((ob_t16_mm_kernel<EPI, TRW, TRA, 8, 8, 4>), dim3((unsigned)((a.nw + 7) / 8 * tb)), dim3(256), 4 * 16 * 1024, s, a);
+    constexpr bool SWAP = TRW, TRL = TRW || TRA;
+    static_assert(!(TRW && TRA), "one operand lies as it is reduced");
+    const int64_t cus = ob_cu_count(), narrow = (int64_t)((a.nw + 7) / 8) * ((a.na + 7) / 8), nd = ((SWAP ? a.na : a.nw) + 15) / 16, nl = SWAP ? a.nw : a.na;
+    const auto go = [&](auto kern, int64_t grid, int lds, bool (&attr_set)[OB_MAX_DEVICES]) {
+        ob_set_max_lds_once(kern, attr_set, lds);
+        hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), lds, s, a);
+    };
+    static bool attr_set[4][OB_MAX_DEVICES] = {};
+    const int64_t t8 = nd * ((nl + 7) / 8), t16 = nd * ((nl + 15) / 16);
+    if (narrow <= cus) go(ob_t16_mm_kernel<EPI, TRW, TRA>, narrow, 4 * 16 * 1024, attr_set[0]);
+    else if constexpr (EPI == OB_T16_GW) {
+        if (a.nk <= 40) go(ob_t16_wr_kernel<EPI, TRL, SWAP, 4>, nd * ((nl + 3) / 4), ob_wr_steps(4) * 4 * 1024, attr_set[3]);
+        else go(ob_t16_wr_kernel<EPI, TRL, SWAP, 8>, t8, ob_wr_steps(8) * 8 * 1024, attr_set[1]);
     }
+    else if (ob_wr_cost(t8, 8, cus) <= ob_wr_cost(t16, 16, cus)) go(ob_t16_wr_kernel<EPI, TRL, SWAP, 8>, t8, ob_wr_steps(8) * 8 * 1024, attr_set[1]);
+    else go(ob_t16_wr_kernel<EPI, TRL, SWAP, 16>, t16, ob_wr_steps(16) * 16 * 1024, attr_set[2]);
 }
 
 // rows in registers where their width and alignment allow, else ob_train_ln_fwd_kernel
@@ -116,10 +132,10 @@ static int ob_t16_backward(const void *gy, const void *x, const void *w, const v
                        2 * (int)((T + 127) / 128));
     if ((rc = ob_launch_status("train_backward(grad input)"))) return rc;
     // gW [N, K] = (gz^T a) (1.001 - tanh(W)^2)
-    ob_t16_tiles(false, x, h, a, T, K, s);
-    ObT16Mm v = {a, gz, (int)((K + 15) / 16), (int)((N + 15) / 16), kt, nt, tt, (_Float16 *)gw, (int)N, (int)K, (const _Float16 *)w};
+    ob_t16_turn(x, h, a, T, K, s);
+    ObT16Mm v = {a, gz, (int)((K + 15) / 16), (int)((N + 15) / 16), tt, nt, tt, (_Float16 *)gw, (int)N, (int)K, (const _Float16 *)w};
     v.vec4 = K % 4 == 0 && ob_aligned(gw, 8) && ob_aligned(w, 8);
-    ob_t16_mm<OB_T16_GW, true, true>(v, s);
+    ob_t16_mm<OB_T16_GW, false, true>(v, s);
     return ob_launch_status("train_backward(grad weight)");
 }
 

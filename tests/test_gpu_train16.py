@@ -1,5 +1,5 @@
 """The float16 train-mode layer (csrc/ob_train16.h) against the same formulas in 64 bits, at the edges of its 16- and 32-element tiles, 128-row and
-128- / 256-column blocks (the wide ones from four per CU on: all three products at 4100 x 8200 x 8216, one each at the sizes after it), with rows
+128- / 256-column blocks (64 to 256 x 256 where they are more than the CUs: all three products at 4100 x 8200 x 8216, one or two each at the sizes after it), with rows
 that are not 16-byte aligned.
 
 Bound: every tensor-level result is rounded to float16 (2^-11 relative) once per operation, at most five of them in a row (x h, z, u, gz, ga,
@@ -55,7 +55,10 @@ def _case(T, K, N, seed, shift=0):
     (1, 32, 64, 0), (31, 33, 32, 0), (32, 64, 31, 0), (33, 31, 130, 0), (127, 160, 129, 0), (128, 256, 256, 0), (129, 257, 255, 0),
     (200, 1376, 1000, 0), (65, 2050, 1028, 3), (300, 264, 520, 1), (4100, 512, 2056, 0), (1030, 4096, 4160, 0), (96, 1024, 16392, 0),
     (1, 256, 130, 0), (33, 259, 129, 1), (129, 513, 33, 0),                                              # (smaller ones: the forward of two launches)
-    (4100, 8200, 8216, 0), (8200, 200, 8216, 0), (8216, 8200, 40, 0), (40, 8216, 8200, 1)])              # 256-column blocks, sums of 2-7 steps of 32
+    (4100, 8200, 8216, 0), (8200, 200, 8216, 0), (8216, 8200, 40, 0), (40, 8216, 8200, 1),              # 256-column blocks, sums of 2-7 steps of 32
+    # one operand straight to registers, 64 / 128 / 256 of the other's: last blocks part-filled, sums of 1 to 4 turns of steps and every remainder
+    (1300, 4100, 2300, 0), (2056, 2056, 4104, 1), (1930, 2081, 3000, 3), (31, 4104, 4200, 0), (4500, 33, 2500, 0), (4500, 96, 2500, 0), (4500, 130, 2056, 0),
+    (4500, 260, 2056, 1), (3000, 4096, 300, 0), (5000, 4096, 33, 0), (1281, 5000, 1500, 0)])
 def test_rows_and_columns_against_64_bits(T, K, N, shift):
     m, x, gy = _case(T, K, N, T + K + N, shift)
     y = m(x)
