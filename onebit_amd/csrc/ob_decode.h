@@ -92,6 +92,78 @@ struct ObGemvArgs {
     int zout;                      // host-side selector of the ZOUT instances (fp32 partial sums of a K slice to ObProj.u); PLAIN only
 };
 
+// TAIL (a single layer's call, onebit_linear_forward of one token): the workgroup that finishes last takes the LayerNorm of the row too, so that the call is ONE
+// launch -- at one token a call's time is the host's, 3.5 us a launch (4096 -> 4096, calls one behind the other: 7.9 -> 4.1 us at the C entry, 12.4 -> 9.6 us a module's call).  u goes to memory
+// write-through (workgroups sit on XCDs with an L2 each), every wave drains its stores, one ticket a workgroup; whoever draws the last one reads the row back
+// with agent-scope loads.  Tickets: four counters per stream, a call takes them in turn and clears the other three: calls of a stream run one behind the other, so
+// nobody else is using them, and a call finds its own at zero whatever became of the three before it.
+#define OB_TAIL_STREAMS 32
+static __device__ uint32_t ob_tail_counters[OB_TAIL_STREAMS * 4][32];        // (a counter a 128-byte line)
+struct ObGemvTailArgs : ObGemvArgs {
+    _Float16 *tail_y;
+    const _Float16 *tail_bias;     // or NULL
+    float tail_eps;
+    int tail_at;                   // the call's counter
+};
+template <bool TAIL> struct ObGemvArgsOf { typedef ObGemvArgs type; };
+template <> struct ObGemvArgsOf<true> { typedef ObGemvTailArgs type; };
+
+// ob_layernorm_rows_kernel's arithmetic (its 256 threads, its order of additions) on one row of N % 8 == 0, N <= 16384, by OB_DEC_THREADS threads.  red: 8 floats
+__device__ __forceinline__ void ob_tail_layernorm(const _Float16 *uin, const _Float16 *bias, _Float16 *y, int N, float eps, float *red, int tid)
+{
+    const int lane = tid & 63, wave = tid >> 6;
+    const auto sum = [&](float v, float *r) {
+        v = ob_wave_sum(v);
+        if (lane == 0 && wave < 4) r[wave] = v;
+        __syncthreads();
+        return (r[0] + r[1]) + (r[2] + r[3]);
+    };
+    uint64_t raw[8][2];
+    bool ok[8];
+#pragma unroll
+    for (int v = 0; v < 8; ++v) {
+        const int base = (v * 256 + tid) * 8;
+        ok[v] = wave < 4 && base < N;
+        if (ok[v]) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) raw[v][i] = __hip_atomic_load((const uint64_t *)(uin + base) + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+    const auto u = [&](int v, int i) { return (float)__builtin_bit_cast(ob_half4, raw[v][i >> 2])[i & 3]; };
+    float s = 0.f, q = 0.f;
+#pragma unroll
+    for (int v = 0; v < 8; ++v)
+        if (ok[v]) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) s += u(v, i);
+        }
+    const float mean = sum(s, red) / (float)N;
+#pragma unroll
+    for (int v = 0; v < 8; ++v)
+        if (ok[v]) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) { const float d = u(v, i) - mean; q = fmaf(d, d, q); }
+        }
+    const float rstd = 1.0f / sqrtf(sum(q, red + 4) / (float)N + eps);
+#pragma unroll
+    for (int v = 0; v < 8; ++v)
+        if (ok[v]) {
+            const int base = (v * 256 + tid) * 8;
+            ob_half8 o, bv = (ob_half8)(_Float16)0;
+            if (bias) bv = *reinterpret_cast<const ob_half8 *>(bias + base);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                // one rounding, as ob_layernorm_rows_kernel's code rounds it; left to itself the compiler packs half of these as a product and a conversion,
+                // two roundings, and a replayed call differs from an eager one where the product lies at a tie
+                uint32_t r;
+                asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(r) : "v"(u(v, i) - mean), "v"(rstd));
+                o[i] = __builtin_bit_cast(_Float16, (uint16_t)r);
+                if (bias) o[i] = (_Float16)((float)o[i] + (float)bv[i]);
+            }
+            *reinterpret_cast<ob_half8 *>(y + base) = o;
+        }
+}
+
 // Block-wide sums of NV values through LDS.  `red` must be a slot (16*NV floats, 16-byte aligned)
 // not used by any other reduction still in flight, so a single barrier suffices.  NW (waves per
 // workgroup) is a compile-time constant: the partials of one value are two ds_read_b128, not a
@@ -443,9 +515,10 @@ __device__ __forceinline__ void ob_st8(_Float16 *p, const ob_half8 v)
 // and xin already offset to the slice, K = its width, ldw the full row pitch) and stores the fp32 partial sum z of every row to
 // ObProj.u (as float *) -- no rounding, no weight_scale, no LayerNorm partials: the caller all-reduces z across the K shards
 // and the consumer applies fp16(fp16(z) * g) (bitnet.py:115-116) to the complete sum.
-template <int KV, int MS, bool ALIGNED, int PRO, int MATH, int NPROJ, bool PST, bool WGP = false, bool BIAS = false, bool ZOUT = false>
-__global__ __launch_bounds__(OB_DEC_THREADS) void ob_dec_gemv_kernel(const ObGemvArgs A)
+template <int KV, int MS, bool ALIGNED, int PRO, int MATH, int NPROJ, bool PST, bool WGP = false, bool BIAS = false, bool ZOUT = false, bool TAIL = false>
+__global__ __launch_bounds__(OB_DEC_THREADS) void ob_dec_gemv_kernel(const typename ObGemvArgsOf<TAIL>::type A)
 {
+    static_assert(!TAIL || (MATH == 1 && ALIGNED && PRO == OB_P_PLAIN && NPROJ == 1 && !WGP && !ZOUT), "the tail is a single layer's");
     static_assert(!WGP || NPROJ == 1, "WGP kernels are instantiated with NPROJ = 1");
     static_assert(!BIAS || PRO == OB_P_RES_LN_RMS, "only the residual prologue adds the producer's bias");
     constexpr int MT = MS * NPROJ;
@@ -1111,7 +1184,8 @@ __global__ __launch_bounds__(OB_DEC_THREADS) void ob_dec_gemv_kernel(const ObGem
                 reinterpret_cast<float *>(u_out)[n_out] = z;             // fp32 partial sum of this K slice (rounded by the consumer)
             } else {
                 const _Float16 uh = (_Float16)(ob_round_h(z) * (float)g_h);   // fp16(z) (bitnet.py:115), * g -> fp16 (:116)
-                u_out[n_out] = uh;
+                if constexpr (TAIL) __hip_atomic_store((uint16_t *)u_out + n_out, __builtin_bit_cast(uint16_t, uh), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                else u_out[n_out] = uh;
                 uval = (float)uh;
             }
         }
@@ -1135,6 +1209,20 @@ __global__ __launch_bounds__(OB_DEC_THREADS) void ob_dec_gemv_kernel(const ObGem
 #undef OB_STAMP
 #undef OB_STAMP_FLUSH
 #undef OB_ISSUE
+    if constexpr (TAIL) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");              // every wave: its part of u has left
+        __syncthreads();
+        int *last = reinterpret_cast<int *>(red);
+        if (tid == 0) {
+            if (blockIdx.x == 0) {
+#pragma unroll
+                for (int i = 1; i < 4; ++i) __hip_atomic_store(&ob_tail_counters[(A.tail_at & ~3) | ((A.tail_at + i) & 3)][0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            *last = __hip_atomic_fetch_add(&ob_tail_counters[A.tail_at][0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+        }
+        __syncthreads();
+        if (*last) ob_tail_layernorm(PP[0].u, A.tail_bias, A.tail_y, PP[0].N, A.tail_eps, red + 4, tid);
+    }
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -298,9 +298,11 @@ template <bool PARTIAL> static bool ob_launch_skinny3(const ObSk3Args &a, int gr
 static bool ob_skinny3_shape_ok(const void *packed, int64_t ldw_bytes, const void *a, int64_t lda, int64_t T, int64_t K, int64_t N);
 static int ob_skinny3_rnt(int64_t N);
 static int ob_skinny3_pick_rnt(const int64_t *N, int np, int copies);
-static int ob_launch_dec_gemv(const ObGemvArgs &a_in, hipStream_t s);
+// the LayerNorm that a one-token launch finishes with (ob_decode.h, TAIL); done: it did
+struct ObTail { void *y; const void *bias; float eps; bool done; };
+static int ob_launch_dec_gemv(const ObGemvArgs &a_in, hipStream_t s, ObTail *tail = nullptr);
 static int ob_single_token_gemv(const void *packed, int64_t ldw_bytes, const void *x, const void *h, const void *g,
-                                void *u, int64_t K, int64_t N, hipStream_t s);
+                                void *u, int64_t K, int64_t N, hipStream_t s, ObTail *tail);
 
 // The LDS-DMA prefill GEMM (ob_gemm3_f16_kernel) consumes pre-scaled activations from the caller's
 // workspace (or the producer's rows).  OB_GEMM3=0 disables it (A/B), =2 forces it on any eligible shape.
@@ -455,8 +457,10 @@ extern "C" int onebit_linear_forward(const void *packed, int64_t ldw_bytes, cons
             (void)hipMemsetAsync(ubuf, 0, (size_t)T * N * 2, s);
         } else if (T == 1 && K % 128 == 0 && ldw_bytes % 16 == 0 && ob_aligned(packed, 16) && K <= 16384) {
             // one token: the persistent decode GEMV (plain prologue) instead of the 16-token tile kernel
-            rc = ob_single_token_gemv(packed, ldw_bytes, x, h, g, ubuf, K, N, s);
-            if (rc) return rc;
+            ObTail tail = {y, bias, ln_eps, false};
+            const bool row = !skip && N % 8 == 0 && N <= 16384 && ob_aligned(ubuf, 16) && (!bias || ob_aligned(bias, 16));
+            rc = ob_single_token_gemv(packed, ldw_bytes, x, h, g, ubuf, K, N, s, row ? &tail : nullptr);
+            if (rc || tail.done) return rc;
         } else if (prescaled && !ob_gemm3_ok(T, K, N)) {
             // 2 <= T <= 64 on producer-scaled rows: the LDS-DMA skinny GEMM (ob_skinny3.h)
             if (!ob_skinny3_shape_ok(packed, ldw_bytes, x, K, T, K, N))
@@ -866,7 +870,47 @@ static bool ob_launch_dec_gemv_wgp(const ObGemvArgs &a, int G, size_t lds, hipSt
     return true;
 }
 
-static int ob_launch_dec_gemv(const ObGemvArgs &a_in, hipStream_t s)
+// A stream's four counters (ob_decode.h, TAIL), the first OB_TAIL_STREAMS streams of a device to ask.  A capture gets none, because a graph's launch would run
+// beside the stream's own calls, nor does hipStreamPerThread, one handle for many streams.  `held` keeps a stream's calls in the order of their numbers.
+struct ObTailStream { hipStream_t s; uint32_t calls; std::mutex mu; };
+struct ObTailStreams { std::mutex mu; int n; ObTailStream of[OB_TAIL_STREAMS]; };
+static int ob_tail_slot(hipStream_t s, ObTailStream *&q, std::unique_lock<std::mutex> &held)
+{
+    static ObTailStreams all[OB_MAX_DEVICES];
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (s == hipStreamPerThread) return -1;
+    if (hipStreamIsCapturing(s, &cap) != hipSuccess) { (void)hipGetLastError(); return -1; }
+    if (cap != hipStreamCaptureStatusNone) return -1;
+    ObTailStreams &d = all[ob_device_index()];
+    int i = 0;
+    {
+        std::lock_guard<std::mutex> g(d.mu);
+        while (i < d.n && d.of[i].s != s) ++i;
+        if (i == OB_TAIL_STREAMS) return -1;
+        if (i == d.n) { d.of[i].s = s; ++d.n; }
+    }
+    q = &d.of[i];
+    held = std::unique_lock<std::mutex>(q->mu);
+    return i;
+}
+template <int KV, int MS>
+static bool ob_launch_dec_gemv_tail(const ObGemvArgs &a, int G, size_t lds, hipStream_t s, ObTail &tail)
+{
+    ObTailStream *q = nullptr;
+    std::unique_lock<std::mutex> held;
+    const int slot = ob_tail_slot(s, q, held);
+    if (slot < 0) return false;
+    ObGemvTailArgs t;
+    static_cast<ObGemvArgs &>(t) = a;
+    t.tail_y = (_Float16 *)tail.y; t.tail_bias = (const _Float16 *)tail.bias; t.tail_eps = tail.eps;
+    t.tail_at = slot * 4 + (int)(q->calls++ & 3);
+    static bool attr_set[OB_MAX_DEVICES] = {};
+    ob_set_max_lds_once(ob_dec_gemv_kernel<KV, MS, true, OB_P_PLAIN, 1, 1, false, false, false, false, true>, attr_set, 160 * 1024);
+    hipLaunchKernelGGL((ob_dec_gemv_kernel<KV, MS, true, OB_P_PLAIN, 1, 1, false, false, false, false, true>), dim3(G), dim3(OB_DEC_THREADS), lds, s, t);
+    return tail.done = true;
+}
+
+static int ob_launch_dec_gemv(const ObGemvArgs &a_in, hipStream_t s, ObTail *tail)
 {
     ObGemvArgs a = a_in;
     a.ablate = ob_ablate_mode();
@@ -916,7 +960,7 @@ static int ob_launch_dec_gemv(const ObGemvArgs &a_in, hipStream_t s)
 #define OB_CASE(P, M)                                                              \
     if (!hit && aligned && KV == P && MS == M) {                                   \
         hit = true;                                                                \
-        ok = use_i8 ? ob_launch_dec_gemv_p<P, M, true, 1>(a, G, lds, s)            \
+        ok = use_i8 ? (tail && ob_launch_dec_gemv_tail<P, M>(a, G, lds, s, *tail)) || ob_launch_dec_gemv_p<P, M, true, 1>(a, G, lds, s) \
                     : ob_launch_dec_gemv_p<P, M, true, 0>(a, G, lds, s);           \
     }
 #define OB_CASE_U(M)                                                               \
@@ -942,7 +986,7 @@ static int ob_launch_dec_gemv(const ObGemvArgs &a_in, hipStream_t s)
 }
 
 static int ob_single_token_gemv(const void *packed, int64_t ldw_bytes, const void *x, const void *h, const void *g,
-                                void *u, int64_t K, int64_t N, hipStream_t s)
+                                void *u, int64_t K, int64_t N, hipStream_t s, ObTail *tail)
 {
     ObGemvArgs a = {};
     a.nproj = 1; a.K = (int)K; a.prologue = OB_P_PLAIN;
@@ -950,7 +994,7 @@ static int ob_single_token_gemv(const void *packed, int64_t ldw_bytes, const voi
     a.p[0].u = (_Float16 *)u; a.p[0].N = (int)N; a.p[0].K = (int)K; a.p[0].ldw = (int)(ldw_bytes / 4);
     a.xin = (const _Float16 *)x;
     a.rms_eps = 1e-6f; a.ln_eps = 1e-5f;
-    return ob_launch_dec_gemv(a, s);
+    return ob_launch_dec_gemv(a, s, tail);
 }
 
 extern "C" int onebit_rows_res_ln_rms_bias(const void *hres_in, const void *u_prev, const void *bias_prev, const void *rms_w, void *hres_out,
