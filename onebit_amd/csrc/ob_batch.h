@@ -525,65 +525,84 @@ __global__ __launch_bounds__(512) void ob_b_lmhead_kernel(const ObBHeadArgs A)
     const _Float16 *wrow = A.lm_w + (int64_t)min(v0 + r, V - 1) * H + gq * 16;       // lane: 16 consecutive k per 64-k block
     const int nkc = (H + OB_BH_K - 1) / OB_BH_K;
 
-    // staging: thread -> (token st_b + 16 i, halves st_k .. st_k + 7) of a [TT*16, 256] chunk
+    // A chunk: this thread's share of the activations (token st_b + 16 i, halves st_k .. st_k + 7) and this lane's 8 x 16 bytes of its row, non-temporal (read
+    // exactly once per step).  Requested together and three chunks before their use, activations first: loads return in order, so that staging a chunk's activations
+    // waits for no younger weights and a CU keeps 192 KB on their way across the barriers.  29 rows, 262 MB of weights: 62.5 us with one chunk ahead, 58 with three.
+    // Workgroups begin at different chunks (`turn`) and go round: side by side they all read the same few hundred bytes of every 8 KB row at a time, which is a
+    // few of the memory's channels: 58 -> 53.5 us (4.9 TB/s); 8 rows 62 -> 52.  (A last chunk that is not whole stays last: its columns beyond H are not multiplied.)
     const int st_b = tid >> 5, st_k = (tid & 31) * 8;
-    ob_half8 xv[TT];
-    auto fetch = [&](int kc) {
+    struct Chunk { ob_half8 x[TT], w[8]; };
+    const int turn = H % OB_BH_K == 0 ? (int)((blockIdx.x + blockIdx.x / 8) % nkc) : 0;
+    auto fetch = [&](Chunk &c, int kc) {
+        kc = kc + turn < nkc ? kc + turn : kc + turn - nkc;
 #pragma unroll
-        for (int i = 0; i < TT; ++i) {
-            const int b = st_b + 16 * i, k = kc * OB_BH_K + st_k;
-            xv[i] = (ob_half8)(_Float16)0;
-            if (b < B && k < H) xv[i] = *reinterpret_cast<const ob_half8 *>(A.x + (int64_t)b * H + k);
+        for (int i = 0; i < TT; ++i) {                               // (rows and columns beyond the input: any inside, zeroed when staged)
+            const int b = min(st_b + 16 * i, B - 1), k = min(kc * OB_BH_K + st_k, H - 8);
+            c.x[i] = *reinterpret_cast<const ob_half8 *>(A.x + (int64_t)b * H + k);
         }
-    };
-    auto stage = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < TT; ++i) *reinterpret_cast<ob_half8 *>(&xs[buf][st_b + 16 * i][st_k]) = xv[i];
-    };
-    // this lane's 8 x 16 bytes of its row for a chunk (non-temporal: read exactly once per step), requested while the chunk before is multiplied and behind
-    // that chunk's activations, so that nothing waits for them early: 29 rows, 262 MB of weights 68 -> 64 us (whole 64-byte pieces an instruction: 62.5, the same step)
-    auto weights = [&](ob_half8 (&wf)[8], int kc) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const int kk = min(kc * OB_BH_K + q * 64, H - 64);       // H % 64 == 0 (host-checked); clamp the tail chunk
-            wf[2 * q] = __builtin_nontemporal_load(reinterpret_cast<const ob_half8 *>(wrow + kk));
-            wf[2 * q + 1] = __builtin_nontemporal_load(reinterpret_cast<const ob_half8 *>(wrow + kk + 8));
+            c.w[2 * q] = __builtin_nontemporal_load(reinterpret_cast<const ob_half8 *>(wrow + kk));
+            c.w[2 * q + 1] = __builtin_nontemporal_load(reinterpret_cast<const ob_half8 *>(wrow + kk + 8));
         }
+    };
+    auto stage = [&](const Chunk &c, int kc) {
+#pragma unroll
+        for (int i = 0; i < TT; ++i)
+            *reinterpret_cast<ob_half8 *>(&xs[kc & 1][st_b + 16 * i][st_k]) = st_b + 16 * i < B && kc * OB_BH_K + st_k < H ? c.x[i] : (ob_half8)(_Float16)0;
     };
     ob_float4 acc[TT];
 #pragma unroll
     for (int t = 0; t < TT; ++t) acc[t] = (ob_float4){0.f, 0.f, 0.f, 0.f};
-    ob_half8 w0[8], w1[8];
-    auto chunk = [&](ob_half8 (&wf)[8], ob_half8 (&next)[8], int kc) {
-        const int buf = kc & 1;
-        if (kc + 1 < nkc) {
-            fetch(kc + 1);
-            weights(next, kc + 1);
-        }
+    auto mul = [&](const Chunk &c, int kc, bool whole) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            if (kc * OB_BH_K + q * 64 < H) {
+            if (whole || kc * OB_BH_K + q * 64 < H) {
 #pragma unroll
                 for (int s = 0; s < 2; ++s) {
 #pragma unroll
                     for (int t = 0; t < TT; ++t) {
-                        const ob_half8 bx = *reinterpret_cast<const ob_half8 *>(&xs[buf][t * 16 + r][q * 64 + gq * 16 + 8 * s]);
-                        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf[2 * q + s], bx, acc[t], 0, 0, 0);
+                        const ob_half8 bx = *reinterpret_cast<const ob_half8 *>(&xs[kc & 1][t * 16 + r][q * 64 + gq * 16 + 8 * s]);
+                        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(c.w[2 * q + s], bx, acc[t], 0, 0, 0);
                     }
                 }
             }
         }
-        if (kc + 1 < nkc) stage(buf ^ 1);
-        __syncthreads();
     };
-    fetch(0);
-    weights(w0, 0);
-    stage(0);
-    __syncthreads();
-    for (int kc = 0; kc < nkc; kc += 2) {
-        chunk(w0, w1, kc);
-        if (kc + 1 < nkc) chunk(w1, w0, kc + 1);
+    // (the barrier waits for LDS alone: __syncthreads would drain the loads)
+#define OB_BH_SYNC() do { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); __builtin_amdgcn_s_barrier(); asm volatile("" ::: "memory"); } while (0)
+    Chunk c0, c1, c2, c3;
+    fetch(c0, 0);
+    fetch(c1, 1);                                                    // (beyond the last: its addresses are clamped)
+    fetch(c2, 2);
+    stage(c0, 0);
+    OB_BH_SYNC();
+    int kc = 0;
+#define OB_BH_CHUNK(C0, C1, C3, J)                                                                                                            \
+    { fetch(C3, kc + (J) + 3); __builtin_amdgcn_sched_barrier(0); mul(C0, kc + (J), true); stage(C1, kc + (J) + 1); OB_BH_SYNC(); }
+    for (; kc + 6 < nkc; kc += 4) {
+        OB_BH_CHUNK(c0, c1, c3, 0)
+        OB_BH_CHUNK(c1, c2, c0, 1)
+        OB_BH_CHUNK(c2, c3, c1, 2)
+        OB_BH_CHUNK(c3, c0, c2, 3)
     }
+#define OB_BH_LAST(C0, C1, C3, J)                                                                                                             \
+    if (kc + (J) < nkc) {                                                                                                                     \
+        if (kc + (J) + 3 < nkc) fetch(C3, kc + (J) + 3);                                                                                      \
+        mul(C0, kc + (J), false);                                                                                                             \
+        if (kc + (J) + 1 < nkc) stage(C1, kc + (J) + 1);                                                                                      \
+        OB_BH_SYNC();                                                                                                                         \
+    }
+    OB_BH_LAST(c0, c1, c3, 0)                                        // 6 at most
+    OB_BH_LAST(c1, c2, c0, 1)
+    OB_BH_LAST(c2, c3, c1, 2)
+    OB_BH_LAST(c3, c0, c2, 3)
+    OB_BH_LAST(c0, c1, c3, 4)
+    OB_BH_LAST(c1, c2, c0, 5)
+#undef OB_BH_LAST
+#undef OB_BH_CHUNK
+#undef OB_BH_SYNC
     // D[v][b]: lane holds v = v0 + 4 gq + i (i = 0..3), b = t * 16 + r
 #pragma unroll
     for (int t = 0; t < TT; ++t) {

@@ -101,6 +101,12 @@ def test_batched_lm_head_and_argmax_inside_the_step(batch, vocab, hidden):
         float(got[b, tok[b]]) == float(got[b].max()) and int(tok[b]) == int((got[b] == got[b].max()).nonzero()[0]) for b in range(batch))
 
 
+# (seven chunks of 256 columns and more, where whole chunks are requested three ahead and workgroups begin at different ones: 7, 8, 10 and 11 of which the last is part-filled)
+@pytest.mark.parametrize("batch,vocab,hidden", [(5, 4099, 1792), (29, 1000, 2048), (48, 4100, 2560), (20, 1000, 2752)])
+def test_batched_lm_head_of_many_chunks(batch, vocab, hidden):
+    test_batched_lm_head_and_argmax_inside_the_step(batch, vocab, hidden)
+
+
 @pytest.mark.parametrize("native", [False, True])
 def test_chunked_prefill_produces_the_same_tokens(golden_dir, native):
     """prefill_chunk = 4: prompts enter the cache in chunks while other requests decode (chunks with a non-empty
