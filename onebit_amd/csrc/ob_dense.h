@@ -243,16 +243,28 @@ template <typename E> __global__ __launch_bounds__(256) void ob_table_rows_kerne
     if (i < (int64_t)A.T * nv) ob_table_piece<E>(A, (E *)A.act, (int)(i / nv), 4 * (int)(i % nv));
 }
 
+// Where a wave begins in its k tiles [k0, k1); it goes round.  Workgroups that all begin at their first tile read, side by side, addresses whole powers of two apart
+// (64 KB an n tile of 2048 columns, 16 KB a wave), which are a few of the memory's channels.  12 rows, a decode step's weights from HBM: input product of 71 MB
+// 15.7 -> 15.2 us, lm_head of 131 MB 22.7 -> 22.3, one of 33 MB 7.4 -> 6.6.  Chats of 12 requests at 4096 columns, two layers: 4768 -> 4600 us (state space), 7170 ->
+// 6915 (experts); of 20 at 2048 columns, eight layers: 7746 -> 7636 and 14354 -> 14257; at 1024 columns equal.  It costs nothing where it gains nothing (one
+// token tile, few k tiles a wave: 9.4 -> 9.5 and 7.5 -> 7.4 us).
+__device__ __forceinline__ int ob_skinny_turn(int k0, int k1)
+{
+    return k0 < k1 ? (int)((blockIdx.x + (blockIdx.x >> 3) + blockIdx.y) % (uint32_t)(k1 - k0)) : 0;
+}
+
 // The sums of ob_skinny_stream without DEEP, into acc[2][MT]: U k tiles on the way while U are multiplied.  Text, because the compiler orders it otherwise when it
 // comes out of a function.  bf16 is faster as text (hybrid decode steps of 17-64 rows 0.3-0.6 %: 4096 columns, two layers, 17 / 48 rows 309.5 / 429.5 us, 310.6 /
 // 430.7 as a function), float32 of more than 16 rows as a function (1024 columns, two layers, 17 / 32 rows 384 / 413 us as text, 371 / 401; 4 / 12 rows 260 / 304
 // as text, 261 / 305).
 #define OB_SKINNY_LOOP \
+    const int turn = ob_skinny_turn(k0, k1);                                                                   \
     V16 wc[2][U], ac[MT][U], wn[2][U], an[MT][U];                                                              \
     auto fetch = [&](V16 (&wd)[2][U], V16 (&ad)[MT][U], int k) {                                               \
         _Pragma("unroll")                                                                                      \
         for (int u = 0; u < U; ++u) {                                                                          \
-            const int kk = min(k + u, k1 - 1);                                                                 \
+            int kk = min(k + u, k1 - 1);                                                                       \
+            kk += kk + turn < k1 ? turn : turn - (k1 - k0);                                                    \
             wd[0][u] = __builtin_nontemporal_load(w0 + (size_t)kk * 64);                                       \
             wd[1][u] = __builtin_nontemporal_load(w1 + (size_t)kk * 64);                                       \
             _Pragma("unroll")                                                                                  \
@@ -298,7 +310,9 @@ __device__ __forceinline__ void ob_skinny_stream(const typename ObElem<E>::V16 *
     for (int m = 0; m < MT; ++m) acc[0][m] = acc[1][m] = (ob_float4){0.f, 0.f, 0.f, 0.f};
     if constexpr (DEEP) {
         V16 w[2][U], x[MT][U];
+        const int turn = ob_skinny_turn(k0, k1);
         const auto fetch = [&](int u, int k) {
+            k += k + turn < k1 ? turn : turn - (k1 - k0);
             w[0][u] = __builtin_nontemporal_load(w0 + (size_t)k * 64);
             w[1][u] = __builtin_nontemporal_load(w1 + (size_t)k * 64);
 #pragma unroll
