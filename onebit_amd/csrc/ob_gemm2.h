@@ -233,8 +233,14 @@ __global__ __launch_bounds__(OB_G2_THREADS, 2) void ob_gemm2_f16_kernel(
 // ablations of the register-staged kernel said it costs (957 -> 1372 TFLOP/s without staging).
 // The DMA writes wave-uniform base + 16 * lane: lane l of DMA i of wave w fills row (4w + i) * 8 +
 // (l >> 3), position l & 7, and FETCHES chunk (l & 7) ^ f(row) -- the XOR swizzle lives in the source
-// address.  Three LDS buffers, one __syncthreads per step (hipcc drains vmcnt before it: the tile
-// of step ks + 2 has the whole MFMA block of step ks to land).
+// address.  Four LDS buffers, one raw barrier a step behind a counted wait.
+// Workgroup = 256 rows x 16 RT tokens, 4 waves of 64 rows (80 KB: TWO workgroups per CU, each with its own barrier -- while one
+// waits the other multiplies).
+// Bound by the matrix cores' issue and, where the grid is several rounds, by power.  Everything a wave does beside its products is placed by hand behind one of
+// them (ob_gemm3_body): left to the compiler, an operand's four words were made in front of its RT products and the matrix pipe waited for them, which a second
+// workgroup on the CU hides in part and a launch of at most one a CU not at all.  Layer calls, LayerNorm and scale pass included, before -> with the placement:
+// 389 rows 11008 -> 4096 (four K slices, one workgroup a CU) 53.1 -> 46.3 us; 2020 rows 169.8 -> 145.0, 4096 -> 4096 72.9 -> 63.6; 1000 rows 4096 -> 11008
+// 87.0 -> 82.5; 16384 rows 1133 -> 1095.  Same products in the same order: the same bits.
 // ---------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void ob_scale_rows_kernel(const _Float16 *__restrict__ x, int64_t ldx, const _Float16 *__restrict__ h,
                                                             _Float16 *__restrict__ a, int64_t T, int K)
@@ -249,11 +255,8 @@ __global__ __launch_bounds__(256) void ob_scale_rows_kernel(const _Float16 *__re
 }
 
 #define OB_G3_BUFS 4
-#define OB_G3_LDS (OB_G3_BUFS * OB_G2_T * OB_G2_PITCH * 2 + 2 * 8192)      // 4 activation tiles + 2 weight quads
-#define OB_G3_LDS_W(WT_) (OB_G3_BUFS * 128 * (WT_) * OB_G2_PITCH * 2 + 2 * 8192)
-// WT = token-side waves: 2 = the 256 x 256 / 8-wave workgroup described above (one per CU: 147 KB of LDS); 1 = 256 rows x
-// 128 tokens / 4 waves (80 KB: TWO workgroups per CU, each with its own barrier -- while one waits the other multiplies;
-// the same wave tile, the same activation traffic per flop, twice the (tiny) weight traffic).
+#define OB_G3_T 128                          // token rows staged per tile
+#define OB_G3_LDS (OB_G3_BUFS * OB_G3_T * OB_G2_PITCH * 2 + 2 * 8192)      // 4 activation tiles + 2 weight quads
 // logical tile id of this workgroup: consecutive ids on one XCD (see ob_flash.h)
 __device__ __forceinline__ int ob_g3_bid()
 {
@@ -265,20 +268,20 @@ __device__ __forceinline__ int ob_g3_bid()
 #undef RT
 // RT = 16-token tiles of a wave: 8, or 7 / 6 where that leaves less of the last round of workgroups empty (ob_gemm3_rt); the staging stays that of 8,
 // rows beyond the tile are fetched and not multiplied.
-template <bool PARTIAL, int WT, int RT>
+template <bool PARTIAL, int RT>
 __device__ __forceinline__ void ob_gemm3_body(
     const uint32_t *__restrict__ W, int64_t ldw_words, const _Float16 *__restrict__ a, int64_t lda,
     const _Float16 *__restrict__ g, _Float16 *__restrict__ u, float *__restrict__ zp, int T, int K, int N, int nbn, const int bid)
 {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    static_assert(RT == 8 || WT == 1, "narrow tiles: the 4-wave form");
-    constexpr int TTILE = 128 * WT;              // token rows staged per workgroup
+    static_assert(RT >= 6 && RT <= 8, "six slots behind an operand's products");
+    constexpr int TTILE = OB_G3_T;
     _Float16 (*As)[TTILE][OB_G2_PITCH] = reinterpret_cast<_Float16 (*)[TTILE][OB_G2_PITCH]>(smem);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wn = wave & 3, wt = wave >> 2;
+    const int wn = wave;
     const int r = lane & 15, gq = lane >> 4;
     const int tt = bid / nbn, tn = bid - tt * nbn;
-    const int n0 = tn * OB_G2_N, t0 = tt * 16 * RT * WT;
+    const int n0 = tn * OB_G2_N, t0 = tt * 16 * RT;
     const int nk = K / OB_G2_K;                 // K % 256 == 0 here (host-checked): whole quads of steps
 
     // DMA source of this lane for each of the wave's 4 instructions per tile, as a 32-bit BYTE offset from
@@ -308,12 +311,9 @@ __device__ __forceinline__ void ob_gemm3_body(
         asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3\n\ts_mov_b32 m0, %0"
                      : "=&s"(m0_keep) : "s"(lds_addr), "v"(voff), "s"(base) : "memory");
     };
-    auto dma = [&](int tile) {
-        const uint32_t buf = (uint32_t)tile & (OB_G3_BUFS - 1);
-        const uint32_t kofs = (uint32_t)((tile >> 1) * 128 + (tile & 1) * 32) * 2u;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            dma16(abase, src[i] + kofs, lds0 + (buf * TTILE + (wave_u * 4 + i) * 8) * (OB_G2_PITCH * 2));
+    // piece i of tile `tile` into buffer tile % 4; half h of quad `quad` of the weights
+    auto dma = [&](int tile, int i) __attribute__((always_inline)) {
+        dma16(abase + ((tile >> 1) * 128 + (tile & 1) * 32) * 2, src[i], lds0 + (((uint32_t)tile & (OB_G3_BUFS - 1)) * TTILE + (wave_u * 4 + i) * 8) * (OB_G2_PITCH * 2));
     };
     // Weights go through LDS as well: while LDS-DMA transfers are pending hipcc turns EVERY wait for an
     // ordinary global load into vmcnt(0) (and an asm load's destination registers are fair game for its
@@ -326,13 +326,11 @@ __device__ __forceinline__ void ob_gemm3_body(
     // the two halves of a lane group pair broadcast).
     const char *wbase = reinterpret_cast<const char *>(W);
     const uint32_t wsrc = (uint32_t)((int64_t)min(n0 + 32 * wave + (lane & 31), N - 1) * ldw_words * 4 + 16 * (lane >> 5));
-    // (4-wave form: a wave fetches two 32-row blocks per quad, its own and the one 4 waves up)
+    // (a wave fetches two 32-row blocks per quad, its own and the one 4 waves up)
     const uint32_t wsrc2 = (uint32_t)((int64_t)min(n0 + 32 * (wave + 4) + (lane & 31), N - 1) * ldw_words * 4 + 16 * (lane >> 5));
     char *wlds = smem + OB_G3_BUFS * TTILE * OB_G2_PITCH * 2;
-    auto wdma = [&](int quad) {
-        dma16(wbase, wsrc + 32u * (uint32_t)quad, lds0 + OB_G3_BUFS * TTILE * OB_G2_PITCH * 2 + ((uint32_t)quad & 1) * 8192 + wave_u * 1024);
-        if (WT == 1)
-            dma16(wbase, wsrc2 + 32u * (uint32_t)quad, lds0 + OB_G3_BUFS * TTILE * OB_G2_PITCH * 2 + ((uint32_t)quad & 1) * 8192 + (wave_u + 4) * 1024);
+    auto wdma = [&](int quad, int h) __attribute__((always_inline)) {
+        dma16(wbase + 32 * quad, h ? wsrc2 : wsrc, lds0 + OB_G3_BUFS * TTILE * OB_G2_PITCH * 2 + ((uint32_t)quad & 1) * 8192 + (wave_u + 4 * h) * 1024);
     };
     // row wn * 64 + rn * 16 + r: block (row >> 5) = 2 wn + (rn >> 1), row-in-block (rn & 1) * 16 + r
     const char *wrd = wlds + wn * 2048 + r * 16 + 8 * (gq >> 1);
@@ -343,134 +341,82 @@ __device__ __forceinline__ void ob_gemm3_body(
     for (int x_ = 0; x_ < RN; ++x_)
 #pragma unroll
         for (int y_ = 0; y_ < RT; ++y_) acc[x_][y_] = (ob_float4){0.f, 0.f, 0.f, 0.f};
-    // the weight quad and all four tile buffers in flight before the first MFMA
-    wdma(0);
-    dma(0);
-    dma(1);
-    dma(2);
-    dma(3);                                     // nk % 4 == 0, nk >= 4 (host-checked)
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");     // (drains everything once)
-    ob_u32x2 wc[RN], wnx[RN];                   // packed words of the current / next pair of steps
+    // the weight quad and all four tile buffers in flight before the first MFMA (nk % 4 == 0, nk >= 4: host-checked)
 #pragma unroll
-    for (int rn = 0; rn < RN; ++rn) {
-        wc[rn] = *reinterpret_cast<const ob_u32x2 *>(wrd + (rn >> 1) * 1024 + (rn & 1) * 256);
-        wnx[rn] = wc[rn];
-    }
-    // operand reads are software-pipelined one half-step ahead of the MFMAs that consume them (two register
-    // sets): after a barrier all 8 waves would otherwise ask the LDS for 8 KB each at once and the matrix
-    // pipe idles until the first answers arrive -- 40 % of the kernel without any staging, by ablation
-    ob_half8 bopA[RT], bopB[RT];
-    // s_setprio(1) around the MFMA clusters (two 4-wave workgroups share a CU: the wave that is multiplying keeps the issue
-    // port against the other workgroup's staging / expansion instructions): +1.5 % on all three 7B shapes at T = 16384
-    // (1359 / 1402 / 1258 -> 1380 / 1419 / 1270 TFLOP/s, same box, alternating runs); -DOB_G3_PRIO=0: A/B build.
-    // Measured and dropped: expanding the next row tile's operand into a second register quad between the current
-    // tile's MFMAs (hipcc forms every operand in ONE quad: 8 MFMAs, 8 VALU, hazard nop) -- the kernel sits at 256 VGPRs,
-    // the second quad spills (1321 vs 1370 TFLOP/s).
-#ifndef OB_G3_PRIO
-#define OB_G3_PRIO 1
-#endif
-#ifndef OB_G3_ABL
-#define OB_G3_ABL 0                             // timing experiments only (tools/prefill_probe.py): 1 no operand reads,
-#endif                                          // 2 no sign expansion, 4 no DMA, 8 no wait / barrier -- results are wrong
-#define OB_G3_READ(DST, BUF, S)                                                                                          \
-    _Pragma("unroll") for (int rt = 0; rt < RT; ++rt)                                                                    \
-        if (!(OB_G3_ABL & 1) || ks < 0)                                                                                  \
-            DST[rt] = *reinterpret_cast<const ob_half8 *>(&As[BUF][wt * 128 + rt * 16 + r][ob_g2_swz(r, gq * 2 + (S)) * 8]);
-    // sign expansion (ob_expand16's arithmetic) done PER operand, right before its 8 MFMAs: 4 live registers
-    // instead of 32 for the whole step
-#define OB_G3_MMA(SRC, S)                                                                                                \
-    _Pragma("unroll") for (int rn = 0; rn < RN; ++rn) {                                                                  \
-        ob_u32x4 av;                                                                                                     \
-        _Pragma("unroll") for (int p = 0; p < 4; ++p)                                                                    \
-            av[p] = (OB_G3_ABL & 2) ? cw[rn] + p : ((cw[rn] << (15 - 2 * (4 * (S) + p))) & mask) | (0x3C003C00u & ~mask);  \
-        const ob_half8 aop = __builtin_bit_cast(ob_half8, av);                                                           \
-        _Pragma("unroll") for (int rt = 0; rt < RT; ++rt)                                                                \
-            acc[rn][rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aop, SRC[rt], acc[rn][rt], 0, 0, 0);                    \
-    }
-    int ks = -1;
-    OB_G3_READ(bopA, 0, 0)
-    if (OB_G3_ABL & 1) { OB_G3_READ(bopB, 0, 1) }
+    for (int h = 0; h < 2; ++h) wdma(0, h);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) dma(i >> 2, i & 3);
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");     // (drains everything once)
+    ob_u32x2 wp[RN];                            // packed words of a pair of steps
+    ob_half8 bopA[RT], bopB[RT];                // activations of a step's first half (k sub-step 0) and second
+    // One sign operand = four 32-bit words (ob_expand16's arithmetic); jn = 4 * sub-step + row tile counts a step's eight
+    uint32_t cw[RN], mask = 0x80008000u, one = 0x3C003C00u;
+    asm("" : "+s"(mask));
+    asm("" : "+v"(one));                        // (registers of the two kinds: one v_and_or_b32)
+    const auto bits = [&](int rn, int par) {
+        const uint32_t b16 = (wp[rn][par] >> wsh) & 0xffffu;
+        return (b16 & 0x5555u) | ((b16 & 0xAAAAu) << 15);
+    };
+    const auto word = [&](int jn, int p) { return ((cw[jn & 3] << (15 - 2 * (4 * (jn >> 2) + p))) & mask) | one; };
+    const auto rd = [&](int buf, int rt, int S) { return *reinterpret_cast<const ob_half8 *>(&As[buf][rt * 16 + r][ob_g2_swz(r, gq * 2 + S) * 8]); };
+    const auto rw = [&](int rn, int pm) { return *reinterpret_cast<const ob_u32x2 *>(wrd + ((pm >> 1) & 1) * 8192 + (pm & 1) * 512 + (rn >> 1) * 1024 + (rn & 1) * 256); };
+    ob_u32x4 cur, nxt;
+#pragma unroll
+    for (int rn = 0; rn < RN; ++rn) wp[rn] = rw(rn, 0);
+#pragma unroll
+    for (int rn = 0; rn < RN; ++rn) cw[rn] = bits(rn, 0);
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) bopA[rt] = rd(0, rt, 0);
+#pragma unroll
+    for (int p = 0; p < 4; ++p) cur[p] = word(0, p);
 
-    // One K step as a macro: Q (the step within its quad) and STEADY are literals, so the steady-state loop
-    // has NO branch in it.  Step kc:
-    //   read the second half's operands | 32 MFMAs of the first half | COUNTED wait + raw barrier (tile
-    //   kc + 1 has landed for everyone, every read of tile kc is complete; a __syncthreads would drain the
-    //   younger transfers) | [Q == 0: weights of the next quad] DMA of tile kc + 4 into tile kc's buffer |
-    //   [Q odd: ds_read the next pair's packed words] read the FIRST half of step kc + 1 | 32 MFMAs of the
-    //   second half.
-    // In-order completion: tile kc + 1 (requested in step kc - 3) has landed once at most the transfers of
-    // steps kc - 2 and kc - 1 are outstanding: 4 + 4 + one weight DMA if either opens a quad (Q = 1, 2) --
-    // and everything older, including the next quad's weights (step 4j, first read in step 4j + 3), with it.
-#define OB_G3_STEP(Q, STEADY)                                                                                            \
-    {                                                                                                                    \
-        const int kc = ks + (Q), cur = kc & (OB_G3_BUFS - 1);                                                            \
-        uint32_t cw[RN];                                                                                                 \
-        _Pragma("unroll") for (int rn = 0; rn < RN; ++rn) {                                                              \
-            const uint32_t b16 = (wc[rn][(Q) & 1] >> wsh) & 0xffffu;                                                     \
-            cw[rn] = (b16 & 0x5555u) | ((b16 & 0xAAAAu) << 15);                                                          \
-        }                                                                                                                \
-        uint32_t mask = 0x80008000u;                                                                                     \
-        asm("" : "+s"(mask));                                                                                            \
-        OB_G3_READ(bopB, cur, 1)                                                                                         \
-        __builtin_amdgcn_sched_barrier(0);                                                                               \
-        if (OB_G3_PRIO) __builtin_amdgcn_s_setprio(1);                                                                   \
-        OB_G3_MMA(bopA, 0)                                                                                               \
-        if (OB_G3_PRIO) __builtin_amdgcn_s_setprio(0);                                                                   \
-        __builtin_amdgcn_sched_barrier(0);                                                                               \
-        if (OB_G3_ABL & 8) {                                                                                             \
-        } else if (STEADY) {                                                                                             \
-            if (((Q) == 1 || (Q) == 2) && WT == 1) asm volatile("s_waitcnt vmcnt(10) lgkmcnt(0)\n\ts_barrier" ::: "memory");  \
-            else if ((Q) == 1 || (Q) == 2) asm volatile("s_waitcnt vmcnt(9) lgkmcnt(0)\n\ts_barrier" ::: "memory");      \
-            else asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");                                \
-        } else {                                                                                                         \
-            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");                                     \
-        }                                                                                                                \
-        if ((STEADY) && !(OB_G3_ABL & 4)) {                                                                              \
-            if ((Q) == 0) wdma((kc >> 2) + 1);                                                                           \
-            dma(kc + 4);                                                                                                 \
-        }                                                                                                                \
-        if (((Q) & 1) && ((STEADY) || kc + 1 < nk)) {                                                                    \
-            const int pm = (kc + 1) >> 1;                                                                                \
-            const char *wq = wrd + ((pm >> 1) & 1) * 8192 + (pm & 1) * 512;                                              \
-            _Pragma("unroll") for (int rn = 0; rn < RN; ++rn)                                                            \
-                wnx[rn] = *reinterpret_cast<const ob_u32x2 *>(wq + (rn >> 1) * 1024 + (rn & 1) * 256);                   \
-        }                                                                                                                \
-        if ((STEADY) || kc + 1 < nk) { OB_G3_READ(bopA, (kc + 1) & (OB_G3_BUFS - 1), 0) }                                \
-        __builtin_amdgcn_sched_barrier(0);                                                                               \
-        if (OB_G3_PRIO) __builtin_amdgcn_s_setprio(1);                                                                   \
-        OB_G3_MMA(bopB, 1)                                                                                               \
-        if (OB_G3_PRIO) __builtin_amdgcn_s_setprio(0);                                                                   \
-        __builtin_amdgcn_sched_barrier(0);                                                                               \
-        if ((Q) & 1) {                                                                                                   \
-            /* consume the packed words HERE (32 MFMAs after their ds_read): left pending over the step boundary */     \
-            /* hipcc waits for them with lgkmcnt(0) at the top of the next step, which also drains the operand */       \
-            /* reads just issued for the second half */                                                                  \
-            asm volatile("" : "+v"(wnx[0]), "+v"(wnx[1]), "+v"(wnx[2]), "+v"(wnx[3]));                                   \
-            _Pragma("unroll") for (int rn = 0; rn < RN; ++rn) wc[rn] = wnx[rn];                                          \
-        }                                                                                                                \
+    // One K step kc, the Q-th of its quad (Q, steady: literals): operands j = 0 .. 7, RT products each, and behind a product one of
+    //   every j      a word of operand j + 1 (the next step's first behind j = 7)
+    //   j = 0        the second half's activations
+    //   j = 4        [the wait and barrier in front: tile kc + 1 has landed for everyone, every read of tile kc is complete; a __syncthreads would drain the
+    //                younger transfers] the first half's activations of step kc + 1; Q odd: the next pair's packed words
+    //   j = 5        the transfers of tile kc + 4 into tile kc's buffer; Q == 0: the weights of the next quad
+    //   j = 6, 7     the next step's sign bits out of the packed words
+    // In-order completion: tile kc + 1 (requested in step kc - 3) has landed once at most the transfers of steps kc - 2 and kc - 1 are outstanding: 4 + 4 + two
+    // weight transfers if either opens a quad (Q = 1, 2) -- and everything older, including the next quad's weights (step 4j, first read in step 4j + 3), with it.
+    const auto step = [&](int kc, int Q, bool steady) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            if (j == 4) {
+                if (!steady) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                else if (Q == 1 || Q == 2) asm volatile("s_waitcnt vmcnt(10) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                else asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            }
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                acc[j & 3][rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(ob_half8, cur), j < 4 ? bopA[rt] : bopB[rt], acc[j & 3][rt], 0, 0, 0);
+                if (rt < 4) nxt[rt] = word((j + 1) & 7, rt);
+                if (j >= 6 && (rt == 4 || rt == 5)) cw[2 * (j - 6) + rt - 4] = bits(2 * (j - 6) + rt - 4, (Q + 1) & 1);
+                if (j == 0) bopB[rt] = rd(Q, rt, 1);
+                if (j == 4 && (steady || Q < 3)) {
+                    bopA[rt] = rd((Q + 1) & 3, rt, 0);
+                    if ((Q & 1) && rt < 4) wp[rt] = rw(rt, (kc + 1) >> 1);
+                }
+                if (j == 5 && steady) {
+                    if (rt < 4) dma(kc + 4, rt);
+                    else if (Q == 0 && rt < 6) wdma((kc >> 2) + 1, rt - 4);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            cur = nxt;
+        }
+    };
+    int kc = 0;
+    for (; kc + 4 < nk; kc += 4) {              // every quad but the last
+        step(kc, 0, true); step(kc + 1, 1, true); step(kc + 2, 2, true); step(kc + 3, 3, true);
     }
-    ks = 0;
-    for (; ks + 4 < nk; ks += 4) {              // steady state (every quad but the last): all conditions true
-        OB_G3_STEP(0, true)
-        OB_G3_STEP(1, true)
-        OB_G3_STEP(2, true)
-        OB_G3_STEP(3, true)
-    }
-    {                                           // the last quad: its tiles are all requested; drain
-        OB_G3_STEP(0, false)
-        OB_G3_STEP(1, false)
-        OB_G3_STEP(2, false)
-        OB_G3_STEP(3, false)
-    }
-#undef OB_G3_STEP
-#undef OB_G3_MMA
-#undef OB_G3_READ
+    step(kc, 0, false); step(kc + 1, 1, false); step(kc + 2, 2, false); step(kc + 3, 3, false);      // its tiles are all requested: drain
 
     // Epilogue through LDS (fp16 outputs, wave's 64 rows inside N): a lane's accumulators are 4 consecutive rows
     // of one token -- stored directly that is 8 bytes per lane and 32 contiguous bytes per token row and instruction.
     // Each wave transposes its 64 x 128 tile in its own 18 KB of the (now idle: every read finished before the
     // last barrier) staging memory and writes whole 128-byte row segments, 8 token rows per instruction.
-    if (!PARTIAL && n0 + wn * 64 + 64 <= N && (N & 7) == 0 && (reinterpret_cast<size_t>(u) & 15) == 0 && !(OB_G3_ABL & 32)) {
+    if (!PARTIAL && n0 + wn * 64 + 64 <= N && (N & 7) == 0 && (reinterpret_cast<size_t>(u) & 15) == 0) {
         constexpr int EP = 144;                                // bytes per token row: 128 + 16 (rows shift by 4 banks)
         char *ep = smem + (size_t)wave * 128 * EP;
 #pragma unroll
@@ -486,8 +432,8 @@ __device__ __forceinline__ void ob_gemm3_body(
             }
         }
         // (same wave wrote what it reads: no barrier, the compiler orders the LDS accesses with lgkmcnt)
-        _Float16 *ub = u + (int64_t)(t0 + wt * 128) * N + n0 + wn * 64;
-        const int trows = T - (t0 + wt * 128);
+        _Float16 *ub = u + (int64_t)t0 * N + n0 + wn * 64;
+        const int trows = T - t0;
         // Optional (ONEBIT_FLAG_TILE_STATS; `zp` is the output, N % 64 == 0 host-checked): LayerNorm partials of the rows
         // just formed -- per token and 64-row block (sum, sum of squared deviations from the block mean) of the fp16 values
         // being stored.  The 8 lanes that write a token's 128-byte segment hold its 64 values: two 8-lane DPP reductions.
@@ -516,7 +462,7 @@ __device__ __forceinline__ void ob_gemm3_body(
                 m2 += OB_DPP_F(m2, 0x4E, 0xF);
                 m2 += OB_DPP_F(m2, 0x141, 0xF);
                 if (ch == 0 && row < trows)
-                    *reinterpret_cast<ob_float2 *>(tsp + ((int64_t)(t0 + wt * 128 + row) * ntile64 + tile_idx) * 2) = (ob_float2){sm, m2};
+                    *reinterpret_cast<ob_float2 *>(tsp + ((int64_t)(t0 + row) * ntile64 + tile_idx) * 2) = (ob_float2){sm, m2};
             }
         }
         return;
@@ -529,7 +475,7 @@ __device__ __forceinline__ void ob_gemm3_body(
         for (int i = 0; i < 4; ++i) gn[i] = PARTIAL ? 1.0f : (float)g[min(nb + i, N - 1)];
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
-            const int t = t0 + wt * 128 + rt * 16 + r;
+            const int t = t0 + rt * 16 + r;
             if (t >= T) continue;
             if (PARTIAL) {
                 if (nb + 3 < N) {
@@ -556,12 +502,12 @@ __device__ __forceinline__ void ob_gemm3_body(
     }
 }
 
-template <bool PARTIAL, int WT = 2, int RT = 8>
-__global__ __launch_bounds__(256 * WT, 2) void ob_gemm3_f16_kernel(
+template <bool PARTIAL, int RT>
+__global__ __launch_bounds__(256, 2) void ob_gemm3_f16_kernel(
     const uint32_t *__restrict__ W, int64_t ldw_words, const _Float16 *__restrict__ a, int64_t lda,
     const _Float16 *__restrict__ g, _Float16 *__restrict__ u, float *__restrict__ zp, int T, int K, int N, int nbn)
 {
-    ob_gemm3_body<PARTIAL, WT, RT>(W, ldw_words, a, lda, g, u, zp, T, K, N, nbn, ob_g3_bid());
+    ob_gemm3_body<PARTIAL, RT>(W, ldw_words, a, lda, g, u, zp, T, K, N, nbn, ob_g3_bid());
 }
 
 // GROUPED form (round 6): up to three projections that share T, K and the row pitches -- q | k | v or gate | up of a decoder layer on the
@@ -574,8 +520,8 @@ struct ObG3Group {
     long long ldw_words, lda;
     int T, K;
 };
-template <int WT, int RT = 8>
-__global__ __launch_bounds__(256 * WT, 2) void ob_gemm3g_f16_kernel(const ObG3Group G)
+template <int RT>
+__global__ __launch_bounds__(256, 2) void ob_gemm3g_f16_kernel(const ObG3Group G)
 {
     const int bid = ob_g3_bid();
     const int p = (bid >= G.tile_end[0] ? 1 : 0) + (bid >= G.tile_end[1] ? 1 : 0);
@@ -586,7 +532,7 @@ __global__ __launch_bounds__(256 * WT, 2) void ob_gemm3g_f16_kernel(const ObG3Gr
     _Float16 *u = p == 0 ? G.u[0] : (p == 1 ? G.u[1] : G.u[2]);
     const int N = p == 0 ? G.N[0] : (p == 1 ? G.N[1] : G.N[2]);
     const int nbn = p == 0 ? G.nbn[0] : (p == 1 ? G.nbn[1] : G.nbn[2]);
-    ob_gemm3_body<false, WT, RT>(W, G.ldw_words, a, G.lda, g, u, nullptr, G.T, G.K, N, nbn, bid - b0);
+    ob_gemm3_body<false, RT>(W, G.ldw_words, a, G.lda, g, u, nullptr, G.T, G.K, N, nbn, bid - b0);
 }
 
 // K-SLICED form (round 6): ONE projection whose 256 x 128 tiles alone leave most of the chip idle (hidden-width outputs at a few hundred
@@ -600,15 +546,15 @@ struct ObG3Slices {
     long long ldw_words, lda;
     int T, N, nbn, tiles, ns, quads;
 };
-template <int WT, int RT = 8>
-__global__ __launch_bounds__(256 * WT, 2) void ob_gemm3ks_f16_kernel(const ObG3Slices G)
+template <int RT>
+__global__ __launch_bounds__(256, 2) void ob_gemm3ks_f16_kernel(const ObG3Slices G)
 {
     const int bid = ob_g3_bid();
     const int j = bid / G.tiles;
     const int qb = G.quads / G.ns, qr = G.quads - qb * G.ns;
     const int q0 = j * qb + min(j, qr), nq = qb + (j < qr ? 1 : 0);
     float *zp = j == 0 ? G.z[0] : (j == 1 ? G.z[1] : (j == 2 ? G.z[2] : G.z[3]));
-    ob_gemm3_body<true, WT, RT>(G.W + q0 * (4 * OB_G2_K / 32), G.ldw_words, G.a + q0 * (4 * OB_G2_K), G.lda, nullptr, nullptr, zp, G.T,
+    ob_gemm3_body<true, RT>(G.W + q0 * (4 * OB_G2_K / 32), G.ldw_words, G.a + q0 * (4 * OB_G2_K), G.lda, nullptr, nullptr, zp, G.T,
                             nq * (4 * OB_G2_K), G.N, G.nbn, bid - j * G.tiles);
 }
 #undef RN

@@ -338,8 +338,7 @@ static int ob_gemm3_rt(int64_t nb, int64_t T)
 }
 double ob_gemm3_cost(int64_t nb, int64_t T) { return ob_gemm3_tiles_cost(nb, T, ob_gemm3_rt(nb, T)); }
 
-// The LDS-DMA GEMM in its 8-wave (256 x 256 tile, one workgroup per CU) or 4-wave (256 rows x 128 tokens, two workgroups per
-// CU) form; OB_GEMM3_WT=1 / 2 selects (A/B), default below.
+// The LDS-DMA GEMM (ob_gemm2.h)
 #ifndef OB_GEMM4_DEFAULT
 #define OB_GEMM4_DEFAULT 0
 #endif
@@ -347,7 +346,6 @@ template <bool PARTIAL>
 static void ob_launch_gemm3(const uint32_t *W, int64_t ldw_words, const _Float16 *a, int64_t lda, const _Float16 *g, _Float16 *u,
                             float *zp, int64_t T, int64_t K, int64_t N, hipStream_t s)
 {
-    static const int wt_env = getenv("OB_GEMM3_WT") ? atoi(getenv("OB_GEMM3_WT")) : 1;    // 4-wave form: +3-4 % (1286 -> 1335 TFLOP/s on 4096 -> 11008), bit-identical
     static const int g4_env = getenv("OB_GEMM4") ? atoi(getenv("OB_GEMM4")) : OB_GEMM4_DEFAULT;   // the 32x32x16-MFMA form of the same tiling (ob_gemm4.h)
     const int nbn = (int)((N + OB_G2_N - 1) / OB_G2_N);
     if (g4_env) {
@@ -356,23 +354,17 @@ static void ob_launch_gemm3(const uint32_t *W, int64_t ldw_words, const _Float16
         const int nbt = (int)((T + 127) / 128);
         hipLaunchKernelGGL((ob_gemm4_f16_kernel<PARTIAL>), dim3((unsigned)(nbn * nbt)), dim3(256), OB_G4_LDS, s,
                            W, ldw_words, a, lda, g, u, zp, (int)T, (int)K, (int)N, nbn);
-    } else if (wt_env == 1) {
+    } else {
         const int rt = ob_gemm3_rt(nbn, T);
         const auto go = [&](auto kern, bool (&attr_set)[OB_MAX_DEVICES]) {
-            ob_set_max_lds_once(kern, attr_set, OB_G3_LDS_W(1));
-            hipLaunchKernelGGL(kern, dim3((unsigned)(nbn * ((T + 16 * rt - 1) / (16 * rt)))), dim3(256), OB_G3_LDS_W(1), s,
+            ob_set_max_lds_once(kern, attr_set, OB_G3_LDS);
+            hipLaunchKernelGGL(kern, dim3((unsigned)(nbn * ((T + 16 * rt - 1) / (16 * rt)))), dim3(256), OB_G3_LDS, s,
                                W, ldw_words, a, lda, g, u, zp, (int)T, (int)K, (int)N, nbn);
         };
         static bool attr_set[3][OB_MAX_DEVICES] = {};
-        if (rt == 6) go(ob_gemm3_f16_kernel<PARTIAL, 1, 6>, attr_set[0]);
-        else if (rt == 7) go(ob_gemm3_f16_kernel<PARTIAL, 1, 7>, attr_set[1]);
-        else go(ob_gemm3_f16_kernel<PARTIAL, 1>, attr_set[2]);
-    } else {
-        static bool attr_set[OB_MAX_DEVICES] = {};
-        ob_set_max_lds_once(ob_gemm3_f16_kernel<PARTIAL, 2>, attr_set, OB_G3_LDS);
-        const int nbt = (int)((T + OB_G2_T - 1) / OB_G2_T);
-        hipLaunchKernelGGL((ob_gemm3_f16_kernel<PARTIAL, 2>), dim3((unsigned)(nbn * nbt)), dim3(OB_G2_THREADS), OB_G3_LDS, s,
-                           W, ldw_words, a, lda, g, u, zp, (int)T, (int)K, (int)N, nbn);
+        if (rt == 6) go(ob_gemm3_f16_kernel<PARTIAL, 6>, attr_set[0]);
+        else if (rt == 7) go(ob_gemm3_f16_kernel<PARTIAL, 7>, attr_set[1]);
+        else go(ob_gemm3_f16_kernel<PARTIAL, 8>, attr_set[2]);
     }
 }
 
@@ -1756,13 +1748,13 @@ int ob_gemm3_grouped(const onebit_proj_t *const *ps, void *const *us, const void
     const int rt = ob_gemm3_rt(nb, T);
     for (int i = 0; i < 3; ++i) G.tile_end[i] = (int)(G.tile_end[i] / nbt * ((T + 16 * rt - 1) / (16 * rt)));
     const auto go = [&](auto kern, bool (&attr_set)[OB_MAX_DEVICES]) {
-        ob_set_max_lds_once(kern, attr_set, OB_G3_LDS_W(1));
-        hipLaunchKernelGGL(kern, dim3((unsigned)G.tile_end[2]), dim3(256), OB_G3_LDS_W(1), s, G);
+        ob_set_max_lds_once(kern, attr_set, OB_G3_LDS);
+        hipLaunchKernelGGL(kern, dim3((unsigned)G.tile_end[2]), dim3(256), OB_G3_LDS, s, G);
     };
     static bool attr_set[3][OB_MAX_DEVICES] = {};
-    if (rt == 6) go(ob_gemm3g_f16_kernel<1, 6>, attr_set[0]);
-    else if (rt == 7) go(ob_gemm3g_f16_kernel<1, 7>, attr_set[1]);
-    else go(ob_gemm3g_f16_kernel<1>, attr_set[2]);
+    if (rt == 6) go(ob_gemm3g_f16_kernel<6>, attr_set[0]);
+    else if (rt == 7) go(ob_gemm3g_f16_kernel<7>, attr_set[1]);
+    else go(ob_gemm3g_f16_kernel<8>, attr_set[2]);
     return ob_launch_status("gemm3_grouped");
 }
 
@@ -1799,13 +1791,13 @@ int ob_gemm3_ksplit(const onebit_proj_t &p, const void *a, float *const *z, int 
     const int rt = ob_gemm3_rt((int64_t)G.nbn * ns, T);
     G.tiles = G.nbn * (int)((T + 16 * rt - 1) / (16 * rt));
     const auto go = [&](auto kern, bool (&attr_set)[OB_MAX_DEVICES]) {
-        ob_set_max_lds_once(kern, attr_set, OB_G3_LDS_W(1));
-        hipLaunchKernelGGL(kern, dim3((unsigned)(ns * G.tiles)), dim3(256), OB_G3_LDS_W(1), s, G);
+        ob_set_max_lds_once(kern, attr_set, OB_G3_LDS);
+        hipLaunchKernelGGL(kern, dim3((unsigned)(ns * G.tiles)), dim3(256), OB_G3_LDS, s, G);
     };
     static bool attr_set[3][OB_MAX_DEVICES] = {};
-    if (rt == 6) go(ob_gemm3ks_f16_kernel<1, 6>, attr_set[0]);
-    else if (rt == 7) go(ob_gemm3ks_f16_kernel<1, 7>, attr_set[1]);
-    else go(ob_gemm3ks_f16_kernel<1>, attr_set[2]);
+    if (rt == 6) go(ob_gemm3ks_f16_kernel<6>, attr_set[0]);
+    else if (rt == 7) go(ob_gemm3ks_f16_kernel<7>, attr_set[1]);
+    else go(ob_gemm3ks_f16_kernel<8>, attr_set[2]);
     return ob_launch_status("gemm3_ksplit");
 }
 

@@ -1,6 +1,5 @@
-"""TFLOP/s of the LDS-DMA prefill GEMM (pre-scaling pass included, module path) on the three 7B shapes at T = 16384, for the
-current OB_GEMM3_WT setting; bit-identity of the two workgroup forms is checked by comparing against a saved reference run
-(pass a file name to save / compare).  Usage: [OB_GEMM3_WT=1|2] python tools/gemm3_cmp.py [ref.pt]"""
+"""TFLOP/s of the LDS-DMA prefill GEMM (pre-scaling pass included, module path) on the three 7B shapes at T = 16384; bit-identity of two builds is
+checked by comparing against a saved reference run (pass a file name to save / compare).  Usage: python tools/gemm3_cmp.py [ref.pt]"""
 import os, sys, torch
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 from onebit_amd import BitLinearInf
@@ -22,7 +21,7 @@ for K, N in ((4096, 11008), (11008, 4096), (4096, 4096)):
     for _ in range(20): u = m.pre_layernorm_prescaled(a)
     e1.record(); torch.cuda.synchronize()
     ms = e0.elapsed_time(e1) / 20
-    print("WT=%s  %5d -> %5d  T=%d: %.3f ms = %.0f TFLOP/s (GEMM kernel alone, pre-scaled rows)" % (os.environ.get("OB_GEMM3_WT", "2"), K, N, T, ms, 2.0 * T * K * N / ms / 1e9), flush=True)
+    print("%5d -> %5d  T=%d: %.3f ms = %.0f TFLOP/s (GEMM kernel alone, pre-scaled rows)" % (K, N, T, ms, 2.0 * T * K * N / ms / 1e9), flush=True)
     outs["%d_%d" % (K, N)] = u[::997].cpu()
     del m, x, a, u
 if len(sys.argv) > 1:
