@@ -8,17 +8,19 @@
 // output is 9.6e-8 off instead of 1.8e-7).  Infinities stay infinite (lower parts zero), NaN stays NaN.  Exact down to |x h| = 2^-110: smaller
 // ones lose what lies below the smallest bf16, 2^-133 (2e-6 of an activation of 2^-115), which a LayerNorm with eps 1e-5 takes away anyway.
 //
-// What bounds it: the matrix cores, three products for one (whole call at 731 rows, 4096 -> 11008: 7371 us with ob_simple_kernel, 165 now; alone in
-// a trace the product takes 159 us = 1.24 PFLOP/s, the split 8, the row pass 13).
+// What bounds it: the matrix cores, three products for one (whole call at 731 rows, 4096 -> 11008: 7371 us with ob_simple_kernel, 162 with a stage's operands read
+// in front of its products, 154 with everything placed behind single products, as below; 2000 rows 460 -> 445, 1300 rows 4096 -> 4096 151 -> 141, 300 rows
+// 11008 -> 4096 83.5 -> 79, 50 rows 22.4 -> 21.6; the same bits).  In a trace the split takes 8 and the row pass 13.
 //
 //   ob_f32_split_kernel    x, h -> planes: 1 KB tiles [16-row band][k step][part], a tile in MFMA operand order (one wave, 16 bytes a lane).
 //                          Step s of the 256-column quad q holds, for lane group gq, columns 256 q + 64 gq + 8 s ..: a lane's sign bytes of
 //                          the quad's eight steps are then 8 ADJACENT bytes of its packed row, one ds_read_b64 per row tile and quad
 //   ob_f32_gemm_kernel     128 output columns x 16 TB rows per workgroup, four waves; planes and packed rows through LDS by 1 KB DMAs, NST
-//                          stages of 12 or 24 KB, one raw barrier per stage behind a counted wait (as ob_dense_tile_kernel)
+//                          stages of 12 or 24 KB, one raw barrier per stage behind a counted wait
 //   ob_f32_ln_kernel       one workgroup per row: sums of the K splits, * g, LayerNorm, bias; the row stays in registers
 #pragma once
 #include "ob_common.h"
+#include <type_traits>
 
 struct ObF32Split { const float *x; long long ldx; const float *h; char *planes; int T, K, quads; };
 
@@ -86,7 +88,6 @@ struct ObF32Gemm {
     int T, N, quads, tb, nb_full, nb_all, S;
 };
 
-// (as ob_dense_tile_kernel's: M0 kept, destination = the wave's 1 KB)
 template <int WN, int WT, int NW, int TW, int KS, int NST>
 __global__ __launch_bounds__(256, 2) void ob_f32_gemm_kernel(const ObF32Gemm A)
 {
@@ -134,6 +135,73 @@ __global__ __launch_bounds__(256, 2) void ob_f32_gemm_kernel(const ObF32Gemm A)
     for (int i = 0; i < NW; ++i)
 #pragma unroll
         for (int j = 0; j < TW; ++j) hi[i][j] = lo[i][j] = (ob_float4){0.f, 0.f, 0.f, 0.f};
+    if constexpr (KS == 1) {
+        // A step's products by part (upper, middle, lower), each part's operands read while the part before is multiplied, a sign operand's words, the reads and the
+        // transfers one behind each product (sched_barrier keeps them there).  The wait and barrier stand behind the upper part: stage st + 1 has landed for everyone,
+        // and everyone has read stage st, whose buffer takes stage st + NST.
+        ob_bf8 a[TW][3];
+        ob_u32x4 w[NW];
+        ob_u32x2 wq[NW];
+        uint32_t c = 0, mask = 0x80008000u, one = 0x3F803F80u;
+        asm("" : "+s"(mask));
+        asm("" : "+v"(one));
+        const char *lane0 = smem + lane * 16 + wt * (TW * 3072), *wrow = smem + WBUF + (wn * NW * 16 + r) * 32 + gq * 8;
+        const auto rd = [&](int b, int j, int p) { return *reinterpret_cast<const ob_bf8 *>(lane0 + b * (TILES * 1024) + (j * 3 + p) * 1024); };
+        // words 4 j / TW .. of row tile i's sign operand in step st of its quad, behind product j of another row tile
+        const auto make = [&](int i, int st, int j) __attribute__((always_inline)) {
+            if (j == 0) { const uint32_t b = wq[i][st >> 2] >> (8 * (st & 3)); c = (b & 0x55u) | ((b & 0xAAu) << 15); }
+#pragma unroll
+            for (int p = 4 * j / TW; p < 4 * (j + 1) / TW; ++p) w[i][p] = ((c << (15 - 2 * p)) & mask) | one;
+        };
+        wdma(0);
+#pragma unroll
+        for (int s = 0; s < NST; ++s) dma(s, s);
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+        for (int i = 0; i < NW; ++i) wq[i] = *reinterpret_cast<const ob_u32x2 *>(wrow + i * 512);
+#pragma unroll
+        for (int i = 0; i < (NW - 1) * TW; ++i) make(i / TW, 0, i % TW);
+#pragma unroll
+        for (int j = 0; j < TW; ++j) { a[j][0] = rd(0, j, 0); a[j][1] = rd(0, j, 1); }
+        int buf = 0;
+        const auto step = [&](auto sqc, int q) __attribute__((always_inline)) {
+            constexpr int sq = decltype(sqc)::value, PN = NW * TW;
+            static_assert(PN >= 5 + PER && NW >= 2, "room behind the products");
+            const int next = buf + 1 == NST ? 0 : buf + 1;
+#pragma unroll
+            for (int p = 0; p < 3; ++p) {
+                // (the younger stages may be outstanding, and the next quad's packed rows where they were requested behind stage st + 1)
+                if (p == 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"((NST - 2) * PER + (sq >= 1 && sq <= NST - 1 ? 1 : 0)) : "memory");
+#pragma unroll
+                for (int m = 0; m < PN; ++m) {
+                    const int i = m / TW, j = m % TW;
+                    ob_float4 &z = p ? lo[i][j] : hi[i][j];
+                    z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(ob_bf8, w[i]), a[j][p], z, 0, 0, 0);
+                    if (p == 0 && m < TW) a[m][2] = rd(buf, m, 2);
+                    if (p == 1) {
+                        if (m < TW) a[m][0] = rd(next, m, 0);
+                        if (sq == 7 && m < NW) wq[m] = *reinterpret_cast<const ob_u32x2 *>(wrow + ((q + 1) & 1) * 4096 + m * 512);
+                        if (m >= 4 && m < 4 + PER) {
+                            const int d = m - 4;
+                            ob_dma_1k(src[d] + (size_t)min(q * 8 + sq + NST, nst - 1) * 3072, lane * 16, lds0 + (uint32_t)(buf * TILES + wave * PER + d) * 1024);
+                        }
+                        if (sq == 0 && m == 4 + PER) wdma(q + 1);
+                    }
+                    if (p == 2 && m < TW) a[m][1] = rd(next, m, 1);
+                    // a row tile's operand makes room for the next step's when its last product has it; the last one's is made in that step
+                    if (p == 0 && i == 0) make(NW - 1, sq, j);
+                    if (p == 2 && i > 0) make(i - 1, (sq + 1) & 7, j);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            buf = next;
+        };
+        for (int q = 0; q < nq; ++q) {
+            step(std::integral_constant<int, 0>(), q); step(std::integral_constant<int, 1>(), q); step(std::integral_constant<int, 2>(), q);
+            step(std::integral_constant<int, 3>(), q); step(std::integral_constant<int, 4>(), q); step(std::integral_constant<int, 5>(), q);
+            step(std::integral_constant<int, 6>(), q); step(std::integral_constant<int, 7>(), q);
+        }
+    } else {
     wdma(0);
 #pragma unroll
     for (int s = 0; s < NST - 1; ++s) dma(s, s);
@@ -183,6 +251,7 @@ __global__ __launch_bounds__(256, 2) void ob_f32_gemm_kernel(const ObF32Gemm A)
             }
             buf = buf + 1 == NST ? 0 : buf + 1;
         }
+    }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                   // no transfer may land after the workgroup's LDS is released
     float *out = tail ? A.zt + (size_t)split * A.zt_split - A.nb_full * 128 : A.z;
