@@ -864,6 +864,7 @@ static bool ob_launch_dec_gemv_wgp(const ObGemvArgs &a, int G, size_t lds, hipSt
 
 // A stream's four counters (ob_decode.h, TAIL), the first OB_TAIL_STREAMS streams of a device to ask.  A capture gets none, because a graph's launch would run
 // beside the stream's own calls, nor does hipStreamPerThread, one handle for many streams.  `held` keeps a stream's calls in the order of their numbers.
+// (A destroyed stream's queue outlives the work on it, so a handle that comes back finds its counters unused.)
 struct ObTailStream { hipStream_t s; uint32_t calls; std::mutex mu; };
 struct ObTailStreams { std::mutex mu; int n; ObTailStream of[OB_TAIL_STREAMS]; };
 static int ob_tail_slot(hipStream_t s, ObTailStream *&q, std::unique_lock<std::mutex> &held)
