@@ -105,8 +105,10 @@ __device__ __forceinline__ void ob_mm_loop(ob_float4 (&acc)[MN][MT], int nk, RW 
 //     first half's shared operands of step k + 1 are read in the second half of step k, the second half's in the first
 //   * one load, transfer or LDS read behind an MFMA: an MFMA hides what issues in its 16 cycles
 //   * whole turns of NST steps without a way out between them: where paths meet hipcc waits for every load
+//   * the last steps, fewer than a turn, request nothing and wait for everything: hipcc leaves out loads whose result nobody uses, and a count with them in it would
+//     let the barrier pass before the tile has landed
 // hipcc does not know that the assembly is an MFMA: an operand that it copies (a spill, a full register file) right in front of one is read too early, wrong by whole
-// tiles.  No copy is left with these numbers of steps; the sums are those of ob_mm_loop, bit for bit.
+// tiles.  No copy is left with these numbers of steps, and a test of the compiled code holds the waits; the sums are those of ob_mm_loop, bit for bit.
 constexpr int ob_wr_steps(int mt) { return mt < 8 ? 5 : 4; }
 
 // What a launch of t such workgroups costs by its rounds of them: a tile's time grows with its rows and a constant; half a round of two to a CU takes about as long
@@ -151,7 +153,8 @@ __device__ __forceinline__ void ob_wr_loop(ob_float4 (&acc)[4][MT], int nk, cons
     for (int j = 0; j < H; ++j) a[j] = ra(0, j);
     int k = 0;
     uint32_t woff = wlane + (NST + C) * 1024;                                        // (immediate offsets reach 4 KB either way)
-    const auto step = [&]<bool FAST, int u>() __attribute__((always_inline)) {
+    enum { MORE, TURN, REST };                                                       // another turn behind this one; the last whole turn; the steps behind it
+    const auto step = [&]<int KIND, int u>() __attribute__((always_inline)) {
         constexpr int nu = (u + 1) % NST, pu = (u + NST - 1) % NST;
 #pragma unroll
         for (int j = 0; j < H; ++j)
@@ -162,12 +165,12 @@ __device__ __forceinline__ void ob_wr_loop(ob_float4 (&acc)[4][MT], int nk, cons
                 __builtin_amdgcn_sched_barrier(0);
                 if (m % 2 == 0 && m / 2 < G) a[H + m / 2] = ra(u, H + m / 2);
                 if (m % 2 == 1 && m / 2 < PER) {
-                    if constexpr (FAST) dma_next(m / 2, u, pu); else dma(m / 2, min(k + u + NST - 1, nk - 1), pu);
+                    if constexpr (KIND == MORE) dma_next(m / 2, u, pu); else if constexpr (KIND == TURN) dma(m / 2, min(k + u + NST - 1, nk - 1), pu);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
-        // younger than tile k + 1's transfers: NST - 2 steps' loads of both; lgkmcnt(0)
-        __builtin_amdgcn_s_waitcnt(WAIT);
+        // younger than tile k + 1's transfers: NST - 2 steps' loads of both (REST: not counted); lgkmcnt(0)
+        __builtin_amdgcn_s_waitcnt(KIND == REST ? 0x70 : WAIT);
         asm volatile("s_barrier" ::: "memory");
 #pragma unroll
         for (int i = 0; i < MN; ++i)
@@ -178,18 +181,19 @@ __device__ __forceinline__ void ob_wr_loop(ob_float4 (&acc)[4][MT], int nk, cons
                 __builtin_amdgcn_sched_barrier(0);
                 if (m % 2 == 0 && m / 2 < H) a[m / 2] = ra(nu, m / 2);
                 if (j == G - 1) {
-                    if constexpr (FAST) w[u][i] = *reinterpret_cast<const ob_u32x4 *>(wb[i] + (size_t)woff + (u - C) * 1024); else wload(i, k + u + NST, u);
+                    if constexpr (KIND == MORE) w[u][i] = *reinterpret_cast<const ob_u32x4 *>(wb[i] + (size_t)woff + (u - C) * 1024);
+                    else if constexpr (KIND == TURN) wload(i, k + u + NST, u);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
     };
-    const auto turn = [&]<bool FAST, int... U>(std::integer_sequence<int, U...>) __attribute__((always_inline)) { (step.template operator()<FAST, U>(), ...); };
+    const auto turn = [&]<int KIND, int... U>(std::integer_sequence<int, U...>) __attribute__((always_inline)) { (step.template operator()<KIND, U>(), ...); };
     for (; k + 2 * NST <= nk; k += NST) {
-        turn.template operator()<true>(std::make_integer_sequence<int, NST>{});
+        turn.template operator()<MORE>(std::make_integer_sequence<int, NST>{});
         woff += NST * 1024;
     }
-    for (; k + NST <= nk; k += NST) turn.template operator()<false>(std::make_integer_sequence<int, NST>{});
-    const auto rest = [&]<int... U>(std::integer_sequence<int, U...>) __attribute__((always_inline)) { ((k + U < nk ? step.template operator()<false, U>() : (void)0), ...); };
+    for (; k + NST <= nk; k += NST) turn.template operator()<TURN>(std::make_integer_sequence<int, NST>{});
+    const auto rest = [&]<int... U>(std::integer_sequence<int, U...>) __attribute__((always_inline)) { ((k + U < nk ? step.template operator()<REST, U>() : (void)0), ...); };
     rest(std::make_integer_sequence<int, NST - 1>{});
     // No transfer may land after the workgroup's LDS is released; the last sums leave the matrix pipe before anything reads them.
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");

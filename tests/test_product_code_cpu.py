@@ -1,0 +1,128 @@
+"""The compiled code of the matrix products whose loops count on instructions that hipcc does not know or may leave out (csrc/ob_mm.h): every
+``ob_dense_wr / mm`` and ``ob_t16_wr / mm`` kernel of the built objects, disassembled.
+
+``ob_wr_loop``'s waits in front of its barriers count the loads of later steps.  hipcc drops a load whose result is never used, and a count that includes it lets the
+barrier pass before a tile has landed.  Along every path through the kernel the waits in front of barriers alone, without the others that hipcc happens to
+place, must leave at most the transfers of NST - 2 steps on their way."""
+import os
+import re
+import shutil
+import struct
+import subprocess
+
+import pytest
+
+from onebit_amd import build as B
+
+LIBS = {"onebit_hybrid.hip": (B.LIB_HYBRID, B.SOURCES_HYBRID), "onebit_train.hip": (B.LIB, B.SOURCES)}
+KERNEL = re.compile(r"ob_(dense|t16)_(wr|mm)_kernel")
+
+
+def _objdump():
+    tool = shutil.which("llvm-objdump", path=os.path.join(os.path.dirname(os.path.realpath(B._hipcc())), "..", "lib", "llvm", "bin") + ":/opt/rocm/llvm/bin")
+    return tool or pytest.skip("no llvm-objdump")
+
+
+class Kernel:
+    """Instructions of one function: ``text[i]`` = (mnemonic, operands), ``target[i]`` = index a branch goes to or None."""
+
+    def __init__(self, name, base, lines):
+        self.name, self.text, self.target, at, to = name, [], [], {}, []
+        for addr, line, dest in lines:
+            at[addr - base] = len(self.text)
+            op, _, rest = line.partition(" ")
+            self.text.append((op, rest.strip()))
+            to.append(dest)
+        self.target = [at.get(d) if d is not None else None for d in to]
+
+    def args(self):
+        return [int(v) for v in re.findall(r"L[ib](\d+)E", self.name)]
+
+
+def _kernels(src, tmp):
+    lib, sources = LIBS[src]
+    if not os.path.exists(B._obj(src)):
+        B.build(lib=lib, sources=sources)
+    data = open(B._obj(src), "rb").read()
+    at = data.index(b"__CLANG_OFFLOAD_BUNDLE__")
+    (n,), p = struct.unpack_from("<Q", data, at + 24), at + 32
+    for _ in range(n):
+        off, size, idlen = struct.unpack_from("<QQQ", data, p)
+        if b"gfx950" in data[p + 24:p + 24 + idlen]:
+            break
+        p += 24 + idlen
+    co = os.path.join(str(tmp), src + ".co")
+    open(co, "wb").write(data[at + off:at + off + size])
+    out, name = [], None
+    proc = subprocess.Popen([_objdump(), "-d", "--no-show-raw-insn", co], stdout=subprocess.PIPE, text=True)
+    for line in proc.stdout:
+        m = re.match(r"([0-9a-f]+) <(\S+)>:", line)
+        if m:
+            base, name = int(m[1], 16), m[2] if KERNEL.search(m[2]) else None
+            if name:
+                out.append((name, base, []))
+            continue
+        m = name and re.match(r"\s+(\S.*?)\s*// ([0-9A-F]+):(?:.*<[^>]*?(?:\+0x([0-9a-f]+))?>)?", line)
+        if m:
+            dest = (int(m[3], 16) if m[3] else 0) if m[1].startswith(("s_cbranch", "s_branch")) else None
+            out[-1][2].append((int(m[2], 16), m[1], dest))
+    assert proc.wait() == 0
+    return [Kernel(*k) for k in out]
+
+
+@pytest.fixture(scope="module")
+def kernels(tmp_path_factory):
+    tmp = tmp_path_factory.mktemp("code")
+    return [k for src in LIBS for k in _kernels(src, tmp)]
+
+
+def _vmcnt(ops):
+    m = re.search(r"vmcnt\((\d+)\)", ops)
+    return int(m[1]) if m else None
+
+
+def _late_transfers(k, most):
+    """Largest number of transfers to the LDS that may still be on their way behind a barrier, by the waits directly in front of barriers.  ``most``: those allowed;
+    paths end where the loop drains everything, or at the first barrier with more."""
+    worst, seen, todo = 0, set(), [(0, ())]
+    while todo:
+        i, queue = todo.pop()
+        while (i, queue) not in seen:
+            seen.add((i, queue))
+            op, ops = k.text[i]
+            if op == "s_endpgm":
+                break
+            if op.startswith("global_load_lds"):
+                queue = (queue + ("T",))[-64:]
+            elif re.match(r"(global|flat|buffer|scratch)_(load|store|atomic)", op):
+                queue = (queue + ("L",))[-64:]
+            elif op == "s_waitcnt" and _vmcnt(ops) is not None:
+                if k.text[i + 1][0] == "s_barrier":
+                    queue = queue[-_vmcnt(ops):] if _vmcnt(ops) else ()
+                    worst = max(worst, queue.count("T"))
+                    if worst > most:
+                        return worst
+                elif _vmcnt(ops) == 0 and k.text[i + 1] == ("s_nop", "15"):
+                    break                                                # the end of the loop: everything has landed
+            if k.target[i] is not None:
+                if op == "s_branch":
+                    i = k.target[i]
+                    continue
+                todo.append((k.target[i], queue))
+            i += 1
+    return worst
+
+
+def test_barriers_wait_for_the_tile_they_publish(kernels):
+    checked = 0
+    for k in kernels:
+        if "_wr_" not in k.name:
+            continue
+        a = k.args()
+        mt = a[1] if "dense" in k.name else a[-1]
+        nst, per = (a[2], (mt + 3) // 4) if "dense" in k.name else (5 if mt < 8 else 4, mt // 4)
+        late = _late_transfers(k, (nst - 2) * per)
+        assert late <= (nst - 2) * per, f"{k.name}: {late} transfers on their way behind a barrier, {(nst - 2) * per} are of later steps"
+        assert late == (nst - 2) * per, f"{k.name}: the steady step waits for more than it has to"
+        checked += 1
+    assert checked >= 30
