@@ -108,7 +108,7 @@ __device__ __forceinline__ void ob_mm_loop(ob_float4 (&acc)[MN][MT], int nk, RW 
 //   * the last steps, fewer than a turn, request nothing and wait for everything: hipcc leaves out loads whose result nobody uses, and a count with them in it would
 //     let the barrier pass before the tile has landed
 // hipcc does not know that the assembly is an MFMA: an operand that it copies (a spill, a full register file) right in front of one is read too early, wrong by whole
-// tiles.  No copy is left with these numbers of steps, and a test of the compiled code holds the waits; the sums are those of ob_mm_loop, bit for bit.
+// tiles.  No copy is left with these numbers of steps, and a test of the compiled code holds both, this and the waits; the sums are those of ob_mm_loop, bit for bit.
 constexpr int ob_wr_steps(int mt) { return mt < 8 ? 5 : 4; }
 
 // What a launch of t such workgroups costs by its rounds of them: a tile's time grows with its rows and a constant; half a round of two to a CU takes about as long

@@ -1,9 +1,11 @@
 """The compiled code of the matrix products whose loops count on instructions that hipcc does not know or may leave out (csrc/ob_mm.h): every
 ``ob_dense_wr / mm`` and ``ob_t16_wr / mm`` kernel of the built objects, disassembled.
 
-``ob_wr_loop``'s waits in front of its barriers count the loads of later steps.  hipcc drops a load whose result is never used, and a count that includes it lets the
-barrier pass before a tile has landed.  Along every path through the kernel the waits in front of barriers alone, without the others that hipcc happens to
-place, must leave at most the transfers of NST - 2 steps on their way."""
+- ``ob_wr_loop``'s waits in front of its barriers count the loads of later steps.  hipcc drops a load whose result is never used, and a count that includes it lets the
+  barrier pass before a tile has landed.  Along every path through the kernel the waits in front of barriers alone, without the others that hipcc happens to
+  place, must leave at most the transfers of NST - 2 steps on their way.
+- The MFMAs are inline assembly, so hipcc does not keep the two wait states that an operand written by the vector unit needs before an MFMA reads it, and a register
+  kept in scratch would be fetched in front of one."""
 import os
 import re
 import shutil
@@ -126,3 +128,30 @@ def test_barriers_wait_for_the_tile_they_publish(kernels):
         assert late == (nst - 2) * per, f"{k.name}: the steady step waits for more than it has to"
         checked += 1
     assert checked >= 30
+
+
+def _regs(ops, kind="v"):
+    out = set()
+    for m in re.finditer(rf"\b{kind}(?:(\d+)|\[(\d+):(\d+)\])", ops):
+        out |= {int(m[1])} if m[1] else set(range(int(m[2]), int(m[3]) + 1))
+    return out
+
+
+def test_operands_are_not_written_in_front_of_their_products(kernels):
+    products = 0
+    for k in kernels:
+        mf = [i for i, (op, _) in enumerate(k.text) if op.startswith("v_mfma")]
+        products += len(mf)
+        assert not any(op.startswith("scratch_") for op, _ in k.text[mf[0]:mf[-1]]), f"{k.name}: a register in scratch between products"
+        for i in mf:
+            parts = re.findall(r"[va]\[\d+:\d+\]", k.text[i][1])
+            assert len(parts) == 4 and parts[0] == parts[3] and parts[0][0] == "a" and parts[1][0] == parts[2][0] == "v", (k.name, k.text[i])
+            operands, sums, states, j = _regs(parts[1]) | _regs(parts[2]), _regs(parts[0], "a"), 0, i - 1
+            while states < 2 and j >= 0:                                 # (an operand may also come from in front of a branch: the loop's first product)
+                op, ops = k.text[j]
+                if op.startswith("v_") and not op.startswith(("v_mfma", "v_cmp", "v_readfirstlane")):
+                    to = ops.split(",")[0]
+                    assert not _regs(to) & operands and not _regs(to, "a") & sums, f"{k.name}: {op} {ops} in front of {k.text[i]}"
+                states += 1 + (int(ops) if op == "s_nop" else 0)
+                j -= 1
+    assert products > 5000
