@@ -167,6 +167,8 @@ __global__ __launch_bounds__(256, 2) void ob_f32_gemm_kernel(const ObF32Gemm A)
         const auto step = [&](auto sqc, int q) __attribute__((always_inline)) {
             constexpr int sq = decltype(sqc)::value, PN = NW * TW;
             static_assert(PN >= 5 + PER && NW >= 2, "room behind the products");
+            // (step 7 reads the next quad's packed rows, requested in step 0: six stages of transfers are younger by then, of which the wait may leave NST - 2)
+            static_assert(NST >= 2 && NST <= 7, "the next quad's packed rows have landed");
             const int next = buf + 1 == NST ? 0 : buf + 1;
 #pragma unroll
             for (int p = 0; p < 3; ++p) {
