@@ -71,8 +71,16 @@ __device__ __forceinline__ float ob_fd_rows_max(float v)
 #define OB_FD_THREADS 256
 #define OB_FD_PG 16               // position groups per workgroup
 
-template <int NI, bool FUSED = false>   // NI: keys per thread in flight (16 * NI positions per sweep of the workgroup)
-__global__ __launch_bounds__(OB_FD_THREADS) void ob_fdec_kernel(const ObFdecArgs A)
+// NI: keys per thread and sweep (16 * NI positions per sweep of the workgroup).  A row's running maximum moves once a sweep, so NI decides the last bits of its sums:
+// it follows from the caller's chunk alone, never from how many rows or splits a launch has, and a row's output does not depend on the rows beside it.
+// FUSED: a register that has been used takes its next sweep's key or value at once, so that one set of 2 NI loads is on the way, four workgroups fit a CU
+// (127 registers) and hide each other's serial head and tail (statistics, query, merge, ticket).  Two sets, the next sweep's requested in front of this one's
+// arithmetic, hold 201 registers, two workgroups.  Steps of 32 heads, 8 layers, us, two sets -> one: 2 / 4 / 8 rows of 450, 450, 300 tokens 463 / 474 / 494 ->
+// 457 / 465 / 487; 12 rows of 700 616 -> 591; 16 / 29 / 48 rows of 450 603 / 785 / 1088 -> 587 / 740 / 1047; 29 / 48 rows of 1400 1226 / 1814 -> 1204 / 1792; 4 of
+// 1400 516 -> 523; one row 278.  One set without the bound on registers (149, three a CU): 747 and 1054 at 29 and 48 rows of 450, 1194 and 1778 at 1400.
+// Not fused: two sets (152 registers; a workgroup has no head of its own to hide).
+template <int NI, bool FUSED = false>
+__global__ __launch_bounds__(OB_FD_THREADS, FUSED ? 4 : 1) void ob_fdec_kernel(const ObFdecArgs A)
 {
     __shared__ __attribute__((aligned(16))) float sm[4 * 128 + 16 + (FUSED ? 3 * 64 : 0)];      // po[4 waves][128] | red[16] | q, k, v (ONE LDS object)
     float *po = sm, *red = sm + 4 * 128;
@@ -94,16 +102,13 @@ __global__ __launch_bounds__(OB_FD_THREADS) void ob_fdec_kernel(const ObFdecArgs
     const int dcl = dok ? 8 * ds : 0;
     const _Float16 *kb = A.k + (((int64_t)slot * A.Hkv + kvh) * A.max_len) * D + dcl;
     const _Float16 *vb = A.v + (((int64_t)slot * A.Hkv + kvh) * A.max_len) * D + dcl;
-    // the next sweep's rows are requested before the current sweep's arithmetic (two register sets): a split of several sweeps
-    // keeps 2 * NI loads per thread in flight instead of draining between sweeps
-    ob_half8 k8[NI], v8[NI], kn[NI], vn[NI];
-    auto fetch = [&](ob_half8 (&kd)[NI], ob_half8 (&vd)[NI], int base) {
+    ob_half8 k8[NI], v8[NI], kn[NI], vn[NI];                                         // (kn, vn: the second set, not FUSED)
+    const auto row8 = [&](const _Float16 *b, int base, int i) {                      // key / value i of the sweep at `base`, the row's last beyond its end
+        return __builtin_nontemporal_load(reinterpret_cast<const ob_half8 *>(b + (int64_t)min(base + pg + OB_FD_PG * i, L - 1) * D));
+    };
+    const auto fetch = [&](ob_half8 (&kd)[NI], ob_half8 (&vd)[NI], int base) {
 #pragma unroll
-        for (int i = 0; i < NI; ++i) {
-            const int64_t off = (int64_t)min(base + pg + OB_FD_PG * i, L - 1) * D;
-            kd[i] = __builtin_nontemporal_load(reinterpret_cast<const ob_half8 *>(kb + off));
-            vd[i] = __builtin_nontemporal_load(reinterpret_cast<const ob_half8 *>(vb + off));
-        }
+        for (int i = 0; i < NI; ++i) { kd[i] = row8(kb, base, i); vd[i] = row8(vb, base, i); }
     };
     fetch(k8, v8, p_lo);                                                             // in flight under the query's formation (FUSED)
     ob_half8 q8, kn8 = (ob_half8)(_Float16)0, vn8 = (ob_half8)(_Float16)0;
@@ -166,9 +171,9 @@ __global__ __launch_bounds__(OB_FD_THREADS) void ob_fdec_kernel(const ObFdecArgs
     };
     float m = -INFINITY, l = 0.f;
     float o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    for (int base = p_lo; base < p_hi; base += OB_FD_PG * NI) {
-        const bool more = base + OB_FD_PG * NI < p_hi;                               // (uniform)
-        if (more) fetch(kn, vn, base + OB_FD_PG * NI);
+    const auto sweep = [&](int base, bool more) __attribute__((always_inline)) {
+        const int next = base + OB_FD_PG * NI;
+        if (!FUSED && more) fetch(kn, vn, next);
         float sc[NI];
         float mx = -INFINITY;
 #pragma unroll
@@ -181,6 +186,7 @@ __global__ __launch_bounds__(OB_FD_THREADS) void ob_fdec_kernel(const ObFdecArgs
             const float sv = ob_round_h(ob_round_h(dot) * A.inv_sqrt_d);         // :546, fp16 matmul output, / sqrt(D) -> fp16
             sc[i] = p < p_hi ? sv : -INFINITY;
             mx = fmaxf(mx, sc[i]);
+            if (FUSED && more) k8[i] = row8(kb, next, i);
         }
         if (mx > m) {                                    // (uniform within a 16-lane row; -inf > -inf is false)
             const float f = __expf(m - mx);              // m = -inf: 0
@@ -195,11 +201,19 @@ __global__ __launch_bounds__(OB_FD_THREADS) void ob_fdec_kernel(const ObFdecArgs
             l += pe;
 #pragma unroll
             for (int e = 0; e < 8; ++e) o[e] = __builtin_fmaf(pe, (float)v8[i][e], o[e]);
+            if (FUSED && more) v8[i] = row8(vb, next, i);
         }
-        if (more) {
+        if (!FUSED && more) {
 #pragma unroll
             for (int i = 0; i < NI; ++i) { k8[i] = kn[i]; v8[i] = vn[i]; }
         }
+    };
+    if constexpr (FUSED) {
+        int base = p_lo;
+        for (; base + OB_FD_PG * NI < p_hi; base += OB_FD_PG * NI) sweep(base, true);
+        sweep(base, false);
+    } else {
+        for (int base = p_lo; base < p_hi; base += OB_FD_PG * NI) sweep(base, base + OB_FD_PG * NI < p_hi);
     }
     // ---- merge the workgroup's 16 rows: maximum, rescale, sums
     const float mw = ob_fd_rows_max(m);

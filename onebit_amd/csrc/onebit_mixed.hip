@@ -99,14 +99,9 @@ static int ob_fdec_launch(const void *q, const void *k_cache, const void *v_cach
         a.part_o = (float *)p;
     }
     const dim3 grid((unsigned)n_heads, (unsigned)rows, (unsigned)n_splits);
-    // keys per thread in flight: 8 where the chunk is whole sweeps of 8 * 16 positions (one round trip per 128 positions), else 4.  The fused form takes 4 also
-    // where it has more workgroups than the chip holds of its form with 8 (218 registers, two a CU): then what counts is how many are resident, four at 121.
-    // 32 heads, 8 layers, a step of 29 / 48 rows of 450 / 1400 tokens: 785 / 1824 -> 744 / 1783 us (38 -> 33 us a launch of 29 rows, 5.1 TB/s); 8 rows of 300
-    // equal; 2 and 4 rows of 450: 8 is the better by 1 % (466 and 475 us against 471 and 480).  2 in flight: 753 us; refilling one register set in
-    // place (104 registers): 744.  Not fused, 8 has 158 registers and 4 no gain.
-    const int64_t grids = (int64_t)n_heads * rows * n_splits;
+    // keys per thread and sweep (ob_fdec.h): 8 where the chunk is whole sweeps of 8 * 16 positions (one round trip per 128 positions), else 4
     if (fu) {
-        if (chunk % 128 == 0 && grids <= 2 * (int64_t)ob_cu_count()) hipLaunchKernelGGL((ob_fdec_kernel<8, true>), grid, dim3(OB_FD_THREADS), 0, stream, a);
+        if (chunk % 128 == 0) hipLaunchKernelGGL((ob_fdec_kernel<8, true>), grid, dim3(OB_FD_THREADS), 0, stream, a);
         else hipLaunchKernelGGL((ob_fdec_kernel<4, true>), grid, dim3(OB_FD_THREADS), 0, stream, a);
     } else if (chunk % 128 == 0) hipLaunchKernelGGL((ob_fdec_kernel<8>), grid, dim3(OB_FD_THREADS), 0, stream, a);
     else hipLaunchKernelGGL((ob_fdec_kernel<4>), grid, dim3(OB_FD_THREADS), 0, stream, a);

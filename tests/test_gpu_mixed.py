@@ -434,6 +434,40 @@ def test_fused_decode_rows_equals_rope_launch_plus_attention(H, Hkv, D, chunk, b
     assert changed == (rows - 1) * Hkv
 
 
+@pytest.mark.parametrize("rows,nsplit", [(5, 4), (17, 2), (29, 6), (48, 12)])
+@pytest.mark.parametrize("chunk", [64, 128, 192, 256])
+def test_fused_decode_rows_do_not_depend_on_the_batch(rows, nsplit, chunk):
+    """A row's output bits are those of the row alone: with many rows beside it and in a launch of more splits (a longer conversation beside it), at contexts of
+    one key, around the ends of sweeps of 64 and 128 positions and of chunks."""
+    L, lib = _lib()
+    dev, H, D = torch.device(DEV), 32, 128
+    g = torch.Generator(device="cpu").manual_seed(rows + chunk)
+    max_len, NQ = nsplit * chunk, H * D
+    ends = [1, 63, 64, 65, 127, 128, 129, 191, 192, 193, 255, 256, 257, chunk, chunk + 1, max_len - 1, max_len]
+    ctx = [min(ends[r % len(ends)], max_len) for r in range(rows)]
+    u = [(torch.randn(rows, NQ, generator=g) * 2 + 0.3).half().to(dev) for _ in range(3)]
+    st = [_tile_partials(t) for t in u]
+    cos, sin = _rope_tables(D, max_len, dev)
+    base_k, base_v = [(torch.randn(rows, H, max_len, D, generator=g) * f).half().to(dev) for f in (0.7, 1.0)]
+
+    def run(sel, n):
+        k, v = base_k.clone(), base_v.clone()
+        uu, ss = [t[sel].contiguous() for t in u], [t[sel].contiguous() for t in st]
+        slot = torch.tensor(sel, dtype=torch.int32, device=dev)
+        pos = torch.tensor([ctx[r] - 1 for r in sel], dtype=torch.int32, device=dev)
+        o = torch.zeros(len(sel), NQ, dtype=torch.float16, device=dev)
+        scratch = torch.zeros(max(int(lib.onebit_attention_decode_scratch_bytes(len(sel), H, n)), 16), dtype=torch.uint8, device=dev)
+        L.check(lib.onebit_attention_decode_rows_fused(*[t.data_ptr() for t in uu + ss], None, None, None, cos.data_ptr(), sin.data_ptr(), k.data_ptr(), v.data_ptr(),
+                                                       o.data_ptr(), None, slot.data_ptr(), pos.data_ptr(), len(sel), H, H, D, rows, max_len, max_len, chunk, n, 1e-5,
+                                                       scratch.data_ptr(), scratch.numel(), _sp()), "fused")
+        return o
+    o = run(list(range(rows)), nsplit)
+    assert torch.isfinite(o.float()).all()
+    for r in range(min(rows, len(ends))):
+        alone = run([r], -(-ctx[r] // chunk))
+        assert torch.equal(o[r:r + 1], alone), (r, ctx[r])
+
+
 def test_mixed_step_full_size_properties():
     """BASELINE config 5's step at its real width and row count (LLaMA2-13B widths, 2 layers; 8 x 512 prompt tokens + 24 decode rows = 4120
     rows) through size-independent properties: (1) the step is deterministic and idempotent (the same items twice: bit-identical logits --
