@@ -11,7 +11,9 @@
  *
  * Conventions
  *  - All pointers are DEVICE pointers owned by the caller (torch tensors in
- *    practice).  The library never allocates, frees or retains them.
+ *    practice).  The library never allocates, frees or retains them.  Of its own it
+ *    keeps, per device, the tickets of one-token onebit_linear_forward calls (a call
+ *    in flight owns some of them and gives them back when it ends).
  *  - `stream` is a hipStream_t passed as void* (NULL = default stream).  Calls
  *    only enqueue work; they never synchronise and are graph-capture safe.
  *  - `dtype` selects the floating type of x / h / g / bias / y: ONEBIT_F16 or

@@ -93,17 +93,21 @@ struct ObGemvArgs {
 };
 
 // TAIL (a single layer's call, onebit_linear_forward of one token): the workgroup that finishes last takes the LayerNorm of the row too, so that the call is ONE
-// launch -- at one token a call's time is the host's, 3.5 us a launch (4096 -> 4096, calls one behind the other: 7.9 -> 4.1 us at the C entry, 12.4 -> 9.6 us a module's call).  u goes to memory
-// write-through (workgroups sit on XCDs with an L2 each), every wave drains its stores, one ticket a workgroup; whoever draws the last one reads the row back
-// with agent-scope loads.  Tickets: four counters per stream, a call takes them in turn and clears the other three: calls of a stream run one behind the other, so
-// nobody else is using them, and a call finds its own at zero whatever became of the three before it.
-#define OB_TAIL_STREAMS 32
-static __device__ uint32_t ob_tail_counters[OB_TAIL_STREAMS * 4][32];        // (a counter a 128-byte line)
+// launch.  u goes to memory write-through (workgroups sit on XCDs with an L2 each), every wave drains its stores, one ticket a workgroup; whoever draws the last one
+// reads the row back with agent-scope loads.
+// A call owns a slot of tickets until its last workgroup writes the call's number to the host's word (ObTailPool): every ticket has been drawn by then.  Slots have two
+// counters, taken in turn; workgroup 0 clears the other one in front of its own ticket.
+// Us a call, two launches / one, 4096 -> 4096, 4096 -> 11008 and 11008 -> 4096: on the device 7.0 / 8.9, 10.0 / 11.5, 8.7 / 10.5; the host's share of a call from C 6.8 / 4.1; a
+// module's calls of the first shape, where Python is the slower side, 13.3 / 10.4.
+#define OB_TAIL_SLOTS 32
+static __device__ uint32_t ob_tail_tickets[OB_TAIL_SLOTS][2][32];
 struct ObGemvTailArgs : ObGemvArgs {
     _Float16 *tail_y;
     const _Float16 *tail_bias;     // or NULL
+    uint32_t *tail_done;           // the slot's word in host memory
+    uint32_t tail_call;            // what the last workgroup writes there; its last bit chooses the counter
     float tail_eps;
-    int tail_at;                   // the call's counter
+    int tail_slot;
 };
 template <bool TAIL> struct ObGemvArgsOf { typedef ObGemvArgs type; };
 template <> struct ObGemvArgsOf<true> { typedef ObGemvTailArgs type; };
@@ -1210,15 +1214,15 @@ __global__ __launch_bounds__(OB_DEC_THREADS) void ob_dec_gemv_kernel(const typen
 #undef OB_STAMP_FLUSH
 #undef OB_ISSUE
     if constexpr (TAIL) {
+        if (blockIdx.x == 0 && tid == 0)
+            __hip_atomic_store(&ob_tail_tickets[A.tail_slot][~A.tail_call & 1][0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");              // every wave: its part of u has left
         __syncthreads();
         int *last = reinterpret_cast<int *>(red);
         if (tid == 0) {
-            if (blockIdx.x == 0) {
-#pragma unroll
-                for (int i = 1; i < 4; ++i) __hip_atomic_store(&ob_tail_counters[(A.tail_at & ~3) | ((A.tail_at + i) & 3)][0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-            *last = __hip_atomic_fetch_add(&ob_tail_counters[A.tail_at][0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+            const bool mine = __hip_atomic_fetch_add(&ob_tail_tickets[A.tail_slot][A.tail_call & 1][0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+            if (mine) __hip_atomic_store(A.tail_done, A.tail_call, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            *last = mine;
         }
         __syncthreads();
         if (*last) ob_tail_layernorm(PP[0].u, A.tail_bias, A.tail_y, PP[0].N, A.tail_eps, red + 4, tid);

@@ -862,45 +862,69 @@ static bool ob_launch_dec_gemv_wgp(const ObGemvArgs &a, int G, size_t lds, hipSt
     return true;
 }
 
-// A stream's four counters (ob_decode.h, TAIL), the first OB_TAIL_STREAMS streams of a device to ask.  A capture gets none, because a graph's launch would run
-// beside the stream's own calls, nor does hipStreamPerThread, one handle for many streams.  `held` keeps a stream's calls in the order of their numbers.
-// (A destroyed stream's queue outlives the work on it, so a handle that comes back finds its counters unused.)
-struct ObTailStream { hipStream_t s; uint32_t calls; std::mutex mu; };
-struct ObTailStreams { std::mutex mu; int n; ObTailStream of[OB_TAIL_STREAMS]; };
-static int ob_tail_slot(hipStream_t s, ObTailStream *&q, std::unique_lock<std::mutex> &held)
+// A device's slots of tickets (ob_decode.h, TAIL).  A call takes any free one and has it until its last workgroup writes the call's number to the slot's word of
+// pinned memory, so a slot belongs to no stream or thread, comes back by itself, and is never used by two calls in flight.  Where all are out (a caller far ahead of
+// the device) a call is two launches, and so is a captured one, whose number would be replayed, and one on a stream of another device than the current one.
+struct ObTailPool {
+    static_assert(OB_TAIL_SLOTS == 32, "a bit each");
+    std::mutex mu;
+    uint32_t *done = nullptr, call[OB_TAIL_SLOTS] = {};              // the words; each slot's last call
+    uint32_t free = 0;                                                // slots known to be free: the words are read when none is (a read misses the caches)
+    bool refused = false;
+};
+static ObTailPool *ob_tail_take(hipStream_t s, int &slot)
 {
-    static ObTailStreams all[OB_MAX_DEVICES];
+    static ObTailPool pools[OB_MAX_DEVICES];
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (s == hipStreamPerThread) return -1;
-    if (hipStreamIsCapturing(s, &cap) != hipSuccess) { (void)hipGetLastError(); return -1; }
-    if (cap != hipStreamCaptureStatusNone) return -1;
-    ObTailStreams &d = all[ob_device_index()];
-    int i = 0;
-    {
-        std::lock_guard<std::mutex> g(d.mu);
-        while (i < d.n && d.of[i].s != s) ++i;
-        if (i == OB_TAIL_STREAMS) return -1;
-        if (i == d.n) { d.of[i].s = s; ++d.n; }
+    int dev = -1;
+    if (hipStreamIsCapturing(s, &cap) != hipSuccess || hipGetDevice(&dev) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
+    if (cap != hipStreamCaptureStatusNone || dev < 0 || dev >= OB_MAX_DEVICES) return nullptr;
+    if (s && s != hipStreamLegacy && s != hipStreamPerThread) {       // (those are the current device's)
+        hipDevice_t d;
+        if (hipStreamGetDevice(s, &d) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
+        if (d != dev) return nullptr;
     }
-    q = &d.of[i];
-    held = std::unique_lock<std::mutex>(q->mu);
-    return i;
+    ObTailPool &p = pools[dev];
+    std::lock_guard<std::mutex> g(p.mu);
+    if (!p.done) {
+        if (p.refused) return nullptr;
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;      // (another thread may be capturing: allocations end a capture in the other modes)
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+        void *m = nullptr;
+        const hipError_t e = hipHostMalloc(&m, OB_TAIL_SLOTS * 4, hipHostMallocPortable | hipHostMallocMapped);
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+        if (e != hipSuccess) { (void)hipGetLastError(); p.refused = true; return nullptr; }
+        p.done = (uint32_t *)m;
+        for (int i = 0; i < OB_TAIL_SLOTS; ++i) p.done[i] = 0;
+    }
+    if (!p.free)
+        for (int i = 0; i < OB_TAIL_SLOTS; ++i) p.free |= (uint32_t)(__atomic_load_n(p.done + i, __ATOMIC_ACQUIRE) == p.call[i]) << i;
+    if (!p.free) return nullptr;
+    slot = __builtin_ctz(p.free);
+    p.free &= p.free - 1;
+    ++p.call[slot];
+    return &p;
 }
 template <int KV, int MS>
 static bool ob_launch_dec_gemv_tail(const ObGemvArgs &a, int G, size_t lds, hipStream_t s, ObTail &tail)
 {
-    ObTailStream *q = nullptr;
-    std::unique_lock<std::mutex> held;
-    const int slot = ob_tail_slot(s, q, held);
-    if (slot < 0) return false;
+    int slot;
+    ObTailPool *p = ob_tail_take(s, slot);
+    if (!p) return false;
+    const auto kern = ob_dec_gemv_kernel<KV, MS, true, OB_P_PLAIN, 1, 1, false, false, false, false, true>;
     ObGemvTailArgs t;
     static_cast<ObGemvArgs &>(t) = a;
     t.tail_y = (_Float16 *)tail.y; t.tail_bias = (const _Float16 *)tail.bias; t.tail_eps = tail.eps;
-    t.tail_at = slot * 4 + (int)(q->calls++ & 3);
+    t.tail_done = p->done + slot; t.tail_call = p->call[slot]; t.tail_slot = slot;
     static bool attr_set[OB_MAX_DEVICES] = {};
-    ob_set_max_lds_once(ob_dec_gemv_kernel<KV, MS, true, OB_P_PLAIN, 1, 1, false, false, false, false, true>, attr_set, 160 * 1024);
-    hipLaunchKernelGGL((ob_dec_gemv_kernel<KV, MS, true, OB_P_PLAIN, 1, 1, false, false, false, false, true>), dim3(G), dim3(OB_DEC_THREADS), lds, s, t);
-    return tail.done = true;
+    ob_set_max_lds_once(kern, attr_set, 160 * 1024);
+    void *args[] = {&t};
+    if (hipLaunchKernel((const void *)kern, dim3(G), dim3(OB_DEC_THREADS), args, lds, s) == hipSuccess) return tail.done = true;
+    (void)hipGetLastError();
+    std::lock_guard<std::mutex> g(p->mu);
+    --p->call[slot];                                                  // (no call is behind this number: the slot is free)
+    p->free |= 1u << slot;
+    return false;
 }
 
 static int ob_launch_dec_gemv(const ObGemvArgs &a_in, hipStream_t s, ObTail *tail)

@@ -38,14 +38,14 @@ def test_one_launch_equals_two(K, N):
     for bias in (False, True):
         m, x = _layer(K, N, K + N, bias)
         ref = _captured(m, x)
-        for _ in range(9):                                            # (each of the stream's four counters, twice)
+        for _ in range(9):                                            # (slots of tickets, taken in turn)
             assert torch.equal(m(x), ref)
         x[0, K // 2] = float("nan")                                   # ... and the NaN of the whole row
         assert bool(torch.isnan(m(x)).all())
 
 
 def test_streams_beside_each_other():
-    """More streams than have counters, calls of different layers in flight on all of them, eager and replayed ones on the same stream."""
+    """Calls of different layers in flight on many streams, eager and replayed ones on the same stream."""
     layers = [_layer(K, N, i, bool(i & 1)) for i, (K, N) in enumerate([(4096, 4096), (4096, 11008), (11008, 4096), (512, 16), (2048, 5632)])]
     refs = [_captured(m, x) for m, x in layers]
     streams = [torch.cuda.Stream() for _ in range(40)]
@@ -87,3 +87,53 @@ def test_threads_of_one_stream_and_of_their_own():
         for t in ts:
             t.join()
     assert not bad
+
+
+def _launches(f):
+    """Kernels that ``f`` launches."""
+    from torch.profiler import ProfilerActivity, profile
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        f()
+        torch.cuda.synchronize()
+    return sum(e.count for e in prof.key_averages() if "ob_" in e.key)
+
+
+def test_one_launch_on_the_fiftieth_stream():
+    """What a call took is given back when it ends, whatever becomes of its stream."""
+    import ctypes
+    hip, streams = ctypes.CDLL("libamdhip64.so"), []
+    m, x = _layer(4096, 4096, 1)
+    ref = _captured(m, x)
+    assert _launches(lambda: m(x)) == 1
+    for i in range(50):
+        h = ctypes.c_void_p()
+        assert hip.hipStreamCreateWithFlags(ctypes.byref(h), 1) == 0              # (non-blocking)
+        streams.append(h)
+        with torch.cuda.stream(torch.cuda.ExternalStream(h.value)):
+            y = m(x)
+            if i == 49:
+                assert _launches(lambda: m(x)) == 1
+        torch.cuda.synchronize()
+        assert torch.equal(y, ref)
+    for h in streams:
+        assert hip.hipStreamDestroy(h) == 0
+
+
+def test_far_ahead_of_the_device():
+    """More calls waiting on a stream than there are slots, and calls on another stream beside them: all right, and the slots are back afterwards."""
+    layers = [_layer(K, N, i, bool(i & 1)) for i, (K, N) in enumerate([(4096, 4096), (8192, 16384), (16384, 16384), (512, 16), (4096, 520)])]
+    refs = [_captured(m, x) for m, x in layers]
+    other = torch.cuda.Stream()
+    for _ in range(3):
+        torch.cuda._sleep(20_000_000)
+        out = []
+        for i in range(90):
+            m, x = layers[i % 5]
+            out.append((i % 5, m(x)))
+        with torch.cuda.stream(other):
+            for i in range(90):
+                m, x = layers[i % 5]
+                out.append((i % 5, m(x)))
+        torch.cuda.synchronize()
+        assert all(torch.equal(y, refs[i]) for i, y in out)
+    assert [_launches(lambda: m(x)) for m, x in layers] == [1] * 5
