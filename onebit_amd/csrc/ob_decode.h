@@ -93,21 +93,25 @@ struct ObGemvArgs {
 };
 
 // TAIL (a single layer's call, onebit_linear_forward of one token): the workgroup that finishes last takes the LayerNorm of the row too, so that the call is ONE
-// launch.  u goes to memory write-through (workgroups sit on XCDs with an L2 each), every wave drains its stores, one ticket a workgroup; whoever draws the last one
-// reads the row back with agent-scope loads.
+// launch.  u goes to memory write-through (workgroups sit on XCDs with an L2 each), every wave drains its stores, then tickets; whoever draws the last one reads the
+// row back with agent-scope loads.  256 tickets of one counter are drawn one behind the other (10 ns each, 2.5 us a call): from OB_TAIL_FLAT workgroups on, groups of
+// 16 or more draw theirs side by side and the last of each group draws one for the group.  Groups' tickets and the final one lie a line each.
 // A call owns a slot of tickets until its last workgroup writes the call's number to the host's word (ObTailPool): every ticket has been drawn by then.  Slots have two
-// counters, taken in turn; workgroup 0 clears the other one in front of its own ticket.
-// Us a call, two launches / one, 4096 -> 4096, 4096 -> 11008 and 11008 -> 4096: on the device 7.0 / 8.9, 10.0 / 11.5, 8.7 / 10.5; the host's share of a call from C 6.8 / 4.1; a
-// module's calls of the first shape, where Python is the slower side, 13.3 / 10.4.
+// sets, taken in turn; workgroup 0 clears the other one in front of its own ticket.
+// Us a call, two launches / one, 4096 -> 4096, 4096 -> 11008 and 11008 -> 4096: on the device 7.0 / 6.9, 10.0 / 9.7, 8.7 / 8.5 (one counter: 8.9, 11.5, 10.5); from C, a
+// thousand calls waited for together 7.1 / 6.3, 9.1 / 9.2, 8.1 / 8.0 a call (the host's share of one is 6.8 / 4.1), one by one 18.5 / 18.3, 20.8 / 20.8, 20.0 / 19.7;
+// 16384 -> 16384 19.2 / 19.2.  A module's calls of the first shape, where Python is the slower side: 13.3 / 10.4.
 #define OB_TAIL_SLOTS 32
-static __device__ uint32_t ob_tail_tickets[OB_TAIL_SLOTS][2][32];
+#define OB_TAIL_GROUPS 32
+#define OB_TAIL_FLAT 32
+static __device__ uint32_t ob_tail_tickets[OB_TAIL_SLOTS][2][OB_TAIL_GROUPS + 1][32];
 struct ObGemvTailArgs : ObGemvArgs {
     _Float16 *tail_y;
     const _Float16 *tail_bias;     // or NULL
     uint32_t *tail_done;           // the slot's word in host memory
-    uint32_t tail_call;            // what the last workgroup writes there; its last bit chooses the counter
+    uint32_t tail_call;            // what the last workgroup writes there; its last bit chooses the set
     float tail_eps;
-    int tail_slot;
+    int tail_slot, tail_shift;     // 1 << tail_shift workgroups a group
 };
 template <bool TAIL> struct ObGemvArgsOf { typedef ObGemvArgs type; };
 template <> struct ObGemvArgsOf<true> { typedef ObGemvTailArgs type; };
@@ -1214,13 +1218,17 @@ __global__ __launch_bounds__(OB_DEC_THREADS) void ob_dec_gemv_kernel(const typen
 #undef OB_STAMP_FLUSH
 #undef OB_ISSUE
     if constexpr (TAIL) {
-        if (blockIdx.x == 0 && tid == 0)
-            __hip_atomic_store(&ob_tail_tickets[A.tail_slot][~A.tail_call & 1][0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        uint32_t (*const set)[32] = ob_tail_tickets[A.tail_slot][A.tail_call & 1];
+        if (blockIdx.x == 0 && tid <= OB_TAIL_GROUPS)
+            __hip_atomic_store(&ob_tail_tickets[A.tail_slot][~A.tail_call & 1][tid][0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");              // every wave: its part of u has left
         __syncthreads();
         int *last = reinterpret_cast<int *>(red);
         if (tid == 0) {
-            const bool mine = __hip_atomic_fetch_add(&ob_tail_tickets[A.tail_slot][A.tail_call & 1][0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+            const uint32_t group = blockIdx.x >> A.tail_shift, groups = ((gridDim.x - 1) >> A.tail_shift) + 1;
+            const uint32_t of = min(1u << A.tail_shift, gridDim.x - (group << A.tail_shift));
+            bool mine = __hip_atomic_fetch_add(&set[group][0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == of - 1;
+            if (mine && groups > 1) mine = __hip_atomic_fetch_add(&set[OB_TAIL_GROUPS][0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == groups - 1;
             if (mine) __hip_atomic_store(A.tail_done, A.tail_call, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             *last = mine;
         }

@@ -908,14 +908,15 @@ static ObTailPool *ob_tail_take(hipStream_t s, int &slot)
 template <int KV, int MS>
 static bool ob_launch_dec_gemv_tail(const ObGemvArgs &a, int G, size_t lds, hipStream_t s, ObTail &tail)
 {
-    int slot;
+    int slot, shift = G <= OB_TAIL_FLAT ? 5 : 4;
+    while (((G - 1) >> shift) + 1 > OB_TAIL_GROUPS) ++shift;
     ObTailPool *p = ob_tail_take(s, slot);
     if (!p) return false;
     const auto kern = ob_dec_gemv_kernel<KV, MS, true, OB_P_PLAIN, 1, 1, false, false, false, false, true>;
     ObGemvTailArgs t;
     static_cast<ObGemvArgs &>(t) = a;
     t.tail_y = (_Float16 *)tail.y; t.tail_bias = (const _Float16 *)tail.bias; t.tail_eps = tail.eps;
-    t.tail_done = p->done + slot; t.tail_call = p->call[slot]; t.tail_slot = slot;
+    t.tail_done = p->done + slot; t.tail_call = p->call[slot]; t.tail_slot = slot; t.tail_shift = shift;
     static bool attr_set[OB_MAX_DEVICES] = {};
     ob_set_max_lds_once(kern, attr_set, 160 * 1024);
     void *args[] = {&t};

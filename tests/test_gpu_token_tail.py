@@ -89,6 +89,16 @@ def test_threads_of_one_stream_and_of_their_own():
     assert not bad
 
 
+# workgroups that draw from one counter (32 at most), one more, a last group of one and of all, and where groups grow (512 workgroups, 528, 1024)
+@pytest.mark.parametrize("K,N", [(512, 512), (512, 528), (4096, 16 * 48), (4096, 16 * 49), (4096, 4080), (8192, 16384), (11008, 16 * 513), (11008, 16 * 528), (16384, 16384)])
+def test_groups_of_tickets(K, N):
+    m, x = _layer(K, N, K + N)
+    ref = _captured(m, x)
+    ys = [m(x) for _ in range(70)]                                    # (every slot, both of its sets)
+    torch.cuda.synchronize()
+    assert all(torch.equal(y, ref) for y in ys)
+
+
 def _launches(f):
     """Kernels that ``f`` launches."""
     from torch.profiler import ProfilerActivity, profile
