@@ -105,8 +105,8 @@ __device__ __forceinline__ void ob_mm_loop(ob_float4 (&acc)[MN][MT], int nk, RW 
 //     first half's shared operands of step k + 1 are read in the second half of step k, the second half's in the first
 //   * one load, transfer or LDS read behind an MFMA: an MFMA hides what issues in its 16 cycles
 //   * whole turns of NST steps without a way out between them: where paths meet hipcc waits for every load
-//   * the last steps, fewer than a turn, request nothing and wait for everything: hipcc leaves out loads whose result nobody uses, and a count with them in it would
-//     let the barrier pass before the tile has landed
+//   * the last steps, fewer than a turn, request nothing, and their waits count transfers alone: hipcc leaves out loads whose result nobody uses, and a count with
+//     them in it would let the barrier pass before the tile has landed
 // hipcc does not know that the assembly is an MFMA: an operand that it copies (a spill, a full register file) right in front of one is read too early, wrong by whole
 // tiles.  No copy is left with these numbers of steps, and a test of the compiled code holds both, this and the waits; the sums are those of ob_mm_loop, bit for bit.
 constexpr int ob_wr_steps(int mt) { return mt < 8 ? 5 : 4; }
@@ -169,8 +169,9 @@ __device__ __forceinline__ void ob_wr_loop(ob_float4 (&acc)[4][MT], int nk, cons
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
-        // younger than tile k + 1's transfers: NST - 2 steps' loads of both (REST: not counted); lgkmcnt(0)
-        __builtin_amdgcn_s_waitcnt(KIND == REST ? 0x70 : WAIT);
+        // younger than tile k + 1's transfers: NST - 2 steps' loads of both (REST: the transfers of the tiles behind it, NST - 3 - u at most); lgkmcnt(0)
+        constexpr int VR = u < NST - 3 ? (NST - 3 - u) * PER : 0;
+        __builtin_amdgcn_s_waitcnt(KIND == REST ? (VR & 15) | 0x70 | (VR >> 4 << 14) : WAIT);
         asm volatile("s_barrier" ::: "memory");
 #pragma unroll
         for (int i = 0; i < MN; ++i)
