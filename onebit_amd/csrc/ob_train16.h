@@ -1,6 +1,7 @@
 // The float16 train-mode layer on LDS-DMA matrix products (arithmetic and rounding points: ob_train.h).
 //
-// The three products read three matrices, each formed once by an elementwise pass, both ways:
+// The three products read three matrices that elementwise passes form, each both ways (S and x h by the forward and again by the backward, which is handed no
+// tiles: 32 and 14 us at the size below):
 //   a = fp16(x h) [T][K]     z = a S^T (reduced over K)      gS = gz^T a (reduced over T)
 //   S = sign(W)   [N][K]     z = a S^T                       ga = gz S   (reduced over N)
 //   gz            [T][N]     ga = gz S                       gS = gz^T a
@@ -9,9 +10,10 @@
 // read (ds_read_b64_tr_b16).  The 16-byte piece (row, g = column / 8) sits at place 16 g + (row ^ 4 (g & 1)): both reads are free of bank
 // conflicts.  Every product has one operand that lies as it is reduced, and goes straight to registers with it: S for z, gz for ga, and for gS a^T, whose tiles
 // their pass turns.  Loops, tile shapes and numbering: ob_mm.h.
-// What bounds it: the matrix cores and their power for the products, memory for the passes.  T = 4096, 4096 -> 11008, forward + backward: 1217 us with both
-// operands through the LDS, 1037 now; in a trace the products 343 -> 316 (z), 408 -> 282 (ga) and 441 -> 376 us (gS) = 1.17, 1.31 and 0.98 PFLOP/s, the passes
-// 205 us at 4-5 TB/s.
+// What bounds it: the chip's power for the products, memory for the passes.  T = 4096, 4096 -> 11008, forward + backward: 1217 us with both operands through the
+// LDS, 1037 now; in a trace the products 343 -> 316 (z), 408 -> 282 (ga) and 441 -> 376 us (gS) = 1.17, 1.31 and 0.98 PFLOP/s, the passes 205 us at 4-5 TB/s.  Each
+// product alone in a loop, at 1.39 kW of the 1.4 that the chip is given: 251 us at 2.08 GHz, 222 at 2.19 and 338 at 1.61 (gS multiplies full-range values by full-range
+// values, the others by signs).
 #pragma once
 #include "ob_mm.h"
 
