@@ -97,16 +97,25 @@ __global__ __launch_bounds__(256, 2) void ob_f32_gemm_kernel(const ObF32Gemm A)
     constexpr int WBUF = NST * TILES * 1024;                                            // two 4 KB buffers of packed rows behind the stages
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wn = wave % WN, wt = wave / WN, r = lane & 15, gq = lane >> 4;
-    // whole tiles first, then the splits; each part dealt to the 8 XCDs in contiguous ranges, token blocks fastest
+    // whole tiles first, then the splits; each part dealt to the 8 XCDs in contiguous ranges.  A column block's packed rows are 1/48 of a token block's parts: the
+    // tiles in flight on an XCD are all the columns of a token block or two.  Up to 8 token blocks (whose parts its range needs anyway), and among
+    // the splits, it is the token blocks that come first, so that an XCD reads its own columns' packed rows alone.  Token blocks first -> as it is, whole call: 5500 rows 4096 -> 4096 750 -> 452 us (2.9 GB
+    // of parts through the L2s, 0.13 now), 16000 rows 1024 -> 2816 453 -> 312, 2000 rows 4096 -> 11008 446 -> 413, 1300 rows 4096 -> 4096 (11 blocks) 141 -> 136;
+    // 731 rows 4096 -> 11008 (6) 152.4 either way, 130 rows (3) 74.0 -> 75.3; splits alone, 1100 rows 1024 -> 2816, 40.4 -> 41.3.
     const int nfull = A.nb_full * A.tb;
     const bool tail = (int)blockIdx.x >= nfull;
     const int nwg = tail ? (int)gridDim.x - nfull : nfull, orig = (int)blockIdx.x - (tail ? nfull : 0);
     const int xcd = orig & 7, q8 = nwg >> 3, rem = nwg & 7;
     int bid = (xcd < rem ? xcd * (q8 + 1) : rem * (q8 + 1) + (xcd - rem) * q8) + (orig >> 3);
-    const int tblk = bid % A.tb;
-    bid /= A.tb;
-    const int ntail = A.nb_all - A.nb_full;
-    const int split = tail ? bid / ntail : 0, nblk = tail ? A.nb_full + bid % ntail : bid;
+    int tblk, nblk, split = 0;
+    if (!tail && A.tb > 8) { nblk = bid % A.nb_full; tblk = bid / A.nb_full; }
+    else {
+        tblk = bid % A.tb;
+        bid /= A.tb;
+        const int ntail = A.nb_all - A.nb_full;
+        split = tail ? bid / ntail : 0;
+        nblk = tail ? A.nb_full + bid % ntail : bid;
+    }
     const int n0 = nblk * 128, band0 = tblk * TB, bands = (A.T + 15) >> 4;
     int q_lo = 0, nq = A.quads;
     if (tail) {

@@ -51,6 +51,14 @@ def test_rows_against_64_bits(T, K, N):
     _check(m, torch.randn(T, K, generator=g, device="cuda"))
 
 
+# both numberings of the tiles: up to 8 blocks of 128 rows the token blocks come first, beyond it the columns; with and without whole rounds, a split rest in both
+@pytest.mark.parametrize("T", [1024, 1025, 1409, 2100])
+@pytest.mark.parametrize("K,N", [(264, 4100), (512, 9000), (256, 16388)])
+def test_many_token_blocks_against_64_bits(T, K, N):
+    m, g = _layer(K, N, T + N, False)
+    _check(m, torch.randn(T, K, generator=g, device="cuda"))
+
+
 # K in and out of whole quads of 256 columns, N at and off the 128-column blocks, other pitches (odd ones with columns left over), wide rows (row pass of
 # its own beyond 16384); at the largest T all of them take the matrix cores, whole quads with an odd pitch the general kernel
 @pytest.mark.parametrize("K,N,pitch", [(8, 4372, 0), (248, 1004, 0), (264, 2052, 0), (1376, 4100, 0), (512, 128, 16), (512, 128, 3), (1000, 3004, 3), (520, 12292, 1),
