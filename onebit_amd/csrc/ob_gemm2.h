@@ -17,7 +17,7 @@
 // 16-byte chunks XOR-swizzled: operand reads and staging stores are both bank-conflict free.
 // Workgroups are renumbered so that consecutive ids on one XCD share the token tile (L2 reuse).
 #pragma once
-#include "ob_common.h"
+#include "ob_mm.h"
 
 #define OB_G2_N 256
 #define OB_G2_T 256
@@ -241,6 +241,9 @@ __global__ __launch_bounds__(OB_G2_THREADS, 2) void ob_gemm2_f16_kernel(
 // workgroup on the CU hides in part and a launch of at most one a CU not at all.  Layer calls, LayerNorm and scale pass included, before -> with the placement:
 // 389 rows 11008 -> 4096 (four K slices, one workgroup a CU) 53.1 -> 46.3 us; 2020 rows 169.8 -> 145.0, 4096 -> 4096 72.9 -> 63.6; 1000 rows 4096 -> 11008
 // 87.0 -> 82.5; 16384 rows 1133 -> 1095.  Same products in the same order: the same bits.
+// Products as assembly, sums in place in AGPRs, and what stands behind them evened out to three instructions (a lone wave issues one in four cycles, a product takes
+// sixteen): a step of 112 tokens 1265 -> 1175 cycles, 896 of them products (32 workgroups on the chip); layer calls, this tiling either way: 16384 rows
+// 4096 -> 11008 1107 -> 1086 us, 1600 rows 4096 -> 4096 the product alone 49.2 -> 46.6, 1000 rows 4096 -> 11008 76.4 -> 71.8.
 // ---------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void ob_scale_rows_kernel(const _Float16 *__restrict__ x, int64_t ldx, const _Float16 *__restrict__ h,
                                                             _Float16 *__restrict__ a, int64_t T, int K)
@@ -255,8 +258,13 @@ __global__ __launch_bounds__(256) void ob_scale_rows_kernel(const _Float16 *__re
 }
 
 #define OB_G3_BUFS 4
-#define OB_G3_T 128                          // token rows staged per tile
-#define OB_G3_LDS (OB_G3_BUFS * OB_G3_T * OB_G2_PITCH * 2 + 2 * 8192)      // 4 activation tiles + 2 weight quads
+// A workgroup's tile: WN waves of 64 rows side by side times 4 / WN groups of 16 RT tokens
+__host__ __device__ constexpr int ob_g3_rows(int wn) { return 64 * wn; }
+__host__ __device__ constexpr int ob_g3_tokens(int wn, int rt) { return 64 / wn * rt; }
+__host__ __device__ constexpr int ob_g3_staged(int wn, int rt) { return wn == 4 ? 128 : 32 * rt; }                     // token rows staged per step
+__host__ __device__ constexpr int ob_g3_lds(int wn, int rt) { return OB_G3_BUFS * ob_g3_staged(wn, rt) * OB_G2_PITCH * 2 + 2 * 2048 * wn; }      // 4 activation tiles + 2 weight quads
+struct ObG3Form { int wn, rt; int tokens() const { return ob_g3_tokens(wn, rt); } };
+struct ObG3Plan { ObG3Form f; int ns; double us; };                     // tile, K slices, estimated time
 // logical tile id of this workgroup: consecutive ids on one XCD (see ob_flash.h)
 __device__ __forceinline__ int ob_g3_bid()
 {
@@ -266,31 +274,33 @@ __device__ __forceinline__ int ob_g3_bid()
 }
 
 #undef RT
-// RT = 16-token tiles of a wave: 8, or 7 / 6 where that leaves less of the last round of workgroups empty (ob_gemm3_rt); the staging stays that of 8,
+// WN = 4: RT = 16-token tiles of a wave: 8, or 7 / 6 where that leaves less of the last round of workgroups empty (ob_g3_plan); the staging stays that of 8,
 // rows beyond the tile are fetched and not multiplied.
-template <bool PARTIAL, int RT>
+// WN = 2: 128 rows x 128 or 96 tokens (RT = 4, 3), half the work a workgroup: for grids that the larger tiles leave uneven or too small.  A sign operand is made
+// for half as many products, and an activation tile goes through the L2 twice as often.
+template <bool PARTIAL, int RT, int WN>
 __device__ __forceinline__ void ob_gemm3_body(
     const uint32_t *__restrict__ W, int64_t ldw_words, const _Float16 *__restrict__ a, int64_t lda,
     const _Float16 *__restrict__ g, _Float16 *__restrict__ u, float *__restrict__ zp, int T, int K, int N, int nbn, const int bid)
 {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    static_assert(RT >= 6 && RT <= 8, "six slots behind an operand's products");
-    constexpr int TTILE = OB_G3_T;
+    static_assert(WN == 4 ? RT >= 6 && RT <= 8 : WN == 2 && (RT == 3 || RT == 4), "slots behind an operand's products");
+    constexpr int TTILE = ob_g3_staged(WN, RT), PER = TTILE / 32, WPER = WN / 2, WQUAD = 2048 * WN;      // transfers of a wave: a tile's, a weight quad's; bytes of a quad
     _Float16 (*As)[TTILE][OB_G2_PITCH] = reinterpret_cast<_Float16 (*)[TTILE][OB_G2_PITCH]>(smem);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wn = wave;
+    const int wn = wave % WN, wt = wave / WN;
     const int r = lane & 15, gq = lane >> 4;
     const int tt = bid / nbn, tn = bid - tt * nbn;
-    const int n0 = tn * OB_G2_N, t0 = tt * 16 * RT;
+    const int n0 = tn * ob_g3_rows(WN), t0 = tt * ob_g3_tokens(WN, RT);
     const int nk = K / OB_G2_K;                 // K % 256 == 0 here (host-checked): whole quads of steps
 
     // DMA source of this lane for each of the wave's 4 instructions per tile, as a 32-bit BYTE offset from
     // the (scalar) base pointer: global_load_lds v_off, s[base:base+1] -- half the address registers of
     // 64-bit per-lane pointers (the host checks T * lda * 2 < 4 GB)
-    uint32_t src[4];
+    uint32_t src[PER];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int row = (wave * 4 + i) * 8 + (lane >> 3);
+    for (int i = 0; i < PER; ++i) {
+        const int row = (wave * PER + i) * 8 + (lane >> 3);
         // k order of a step: chunk c (= 2 * k-group + sub-step) of step 2m + par covers
         // k = 128 m + 64 (c >> 2) + 32 par + 8 (c & 3) .. + 7 -- so that a lane's packed words of the two steps
         // of a pair are ADJACENT (words 4m + 2 (gq >> 1) + par): one 8-byte load per row tile and pair
@@ -313,7 +323,7 @@ __device__ __forceinline__ void ob_gemm3_body(
     };
     // piece i of tile `tile` into buffer tile % 4; half h of quad `quad` of the weights
     auto dma = [&](int tile, int i) __attribute__((always_inline)) {
-        dma16(abase + ((tile >> 1) * 128 + (tile & 1) * 32) * 2, src[i], lds0 + (((uint32_t)tile & (OB_G3_BUFS - 1)) * TTILE + (wave_u * 4 + i) * 8) * (OB_G2_PITCH * 2));
+        dma16(abase + ((tile >> 1) * 128 + (tile & 1) * 32) * 2, src[i], lds0 + (((uint32_t)tile & (OB_G3_BUFS - 1)) * TTILE + (wave_u * PER + i) * 8) * (OB_G2_PITCH * 2));
     };
     // Weights go through LDS as well: while LDS-DMA transfers are pending hipcc turns EVERY wait for an
     // ordinary global load into vmcnt(0) (and an asm load's destination registers are fair game for its
@@ -321,16 +331,16 @@ __device__ __forceinline__ void ob_gemm3_body(
     // has no register-destination global load at all.  One DMA instruction per wave and QUAD of steps
     // (256 k = 32 bytes of a packed row): lane l of wave w fetches row 32 w + (l & 31), 16-byte half l >> 5
     // (= pair of steps 2 q + (l >> 5)), landing at w * 1024 + (l >> 5) * 512 + (l & 31) * 16 of the quad's
-    // 8 KB buffer (two buffers).  A lane's 16 sign bits of a step sit in word 2 (gq >> 1) + par of the pair's
+    // buffer (two, 2 KB a 64 rows).  A lane's 16 sign bits of a step sit in word 2 (gq >> 1) + par of the pair's
     // 16 bytes (k order above): one ds_read_b64 per row tile and PAIR of steps, conflict-free (16 rows x 16 B,
     // the two halves of a lane group pair broadcast).
     const char *wbase = reinterpret_cast<const char *>(W);
     const uint32_t wsrc = (uint32_t)((int64_t)min(n0 + 32 * wave + (lane & 31), N - 1) * ldw_words * 4 + 16 * (lane >> 5));
-    // (a wave fetches two 32-row blocks per quad, its own and the one 4 waves up)
+    // (of 256 rows a wave fetches two 32-row blocks per quad, its own and the one 4 waves up)
     const uint32_t wsrc2 = (uint32_t)((int64_t)min(n0 + 32 * (wave + 4) + (lane & 31), N - 1) * ldw_words * 4 + 16 * (lane >> 5));
     char *wlds = smem + OB_G3_BUFS * TTILE * OB_G2_PITCH * 2;
     auto wdma = [&](int quad, int h) __attribute__((always_inline)) {
-        dma16(wbase + 32 * quad, h ? wsrc2 : wsrc, lds0 + OB_G3_BUFS * TTILE * OB_G2_PITCH * 2 + ((uint32_t)quad & 1) * 8192 + (wave_u + 4 * h) * 1024);
+        dma16(wbase + 32 * quad, h ? wsrc2 : wsrc, lds0 + OB_G3_BUFS * TTILE * OB_G2_PITCH * 2 + ((uint32_t)quad & 1) * WQUAD + (wave_u + 4 * h) * 1024);
     };
     // row wn * 64 + rn * 16 + r: block (row >> 5) = 2 wn + (rn >> 1), row-in-block (rn & 1) * 16 + r
     const char *wrd = wlds + wn * 2048 + r * 16 + 8 * (gq >> 1);
@@ -340,12 +350,15 @@ __device__ __forceinline__ void ob_gemm3_body(
 #pragma unroll
     for (int x_ = 0; x_ < RN; ++x_)
 #pragma unroll
-        for (int y_ = 0; y_ < RT; ++y_) acc[x_][y_] = (ob_float4){0.f, 0.f, 0.f, 0.f};
+        for (int y_ = 0; y_ < RT; ++y_) {
+            acc[x_][y_] = (ob_float4){0.f, 0.f, 0.f, 0.f};
+            asm volatile("" : "+a"(acc[x_][y_]));
+        }
     // the weight quad and all four tile buffers in flight before the first MFMA (nk % 4 == 0, nk >= 4: host-checked)
 #pragma unroll
-    for (int h = 0; h < 2; ++h) wdma(0, h);
+    for (int h = 0; h < WPER; ++h) wdma(0, h);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) dma(i >> 2, i & 3);
+    for (int i = 0; i < 4 * PER; ++i) dma(i / PER, i % PER);
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");     // (drains everything once)
     ob_u32x2 wp[RN];                            // packed words of a pair of steps
     ob_half8 bopA[RT], bopB[RT];                // activations of a step's first half (k sub-step 0) and second
@@ -358,8 +371,8 @@ __device__ __forceinline__ void ob_gemm3_body(
         return (b16 & 0x5555u) | ((b16 & 0xAAAAu) << 15);
     };
     const auto word = [&](int jn, int p) { return ((cw[jn & 3] << (15 - 2 * (4 * (jn >> 2) + p))) & mask) | one; };
-    const auto rd = [&](int buf, int rt, int S) { return *reinterpret_cast<const ob_half8 *>(&As[buf][rt * 16 + r][ob_g2_swz(r, gq * 2 + S) * 8]); };
-    const auto rw = [&](int rn, int pm) { return *reinterpret_cast<const ob_u32x2 *>(wrd + ((pm >> 1) & 1) * 8192 + (pm & 1) * 512 + (rn >> 1) * 1024 + (rn & 1) * 256); };
+    const auto rd = [&](int buf, int rt, int S) { return *reinterpret_cast<const ob_half8 *>(&As[buf][(wt * RT + rt) * 16 + r][ob_g2_swz(r, gq * 2 + S) * 8]); };
+    const auto rw = [&](int rn, int pm) { return *reinterpret_cast<const ob_u32x2 *>(wrd + ((pm >> 1) & 1) * WQUAD + (pm & 1) * 512 + (rn >> 1) * 1024 + (rn & 1) * 256); };
     ob_u32x4 cur, nxt;
 #pragma unroll
     for (int rn = 0; rn < RN; ++rn) wp[rn] = rw(rn, 0);
@@ -370,36 +383,57 @@ __device__ __forceinline__ void ob_gemm3_body(
 #pragma unroll
     for (int p = 0; p < 4; ++p) cur[p] = word(0, p);
 
-    // One K step kc, the Q-th of its quad (Q, steady: literals): operands j = 0 .. 7, RT products each, and behind a product one of
-    //   every j      a word of operand j + 1 (the next step's first behind j = 7)
+    // One K step kc, the Q-th of its quad (Q, steady: literals): operands j = 0 .. 7, RT products each, and behind a product at most three instructions, which is
+    // what issues while the matrix pipe has it (a transfer's five apart):
+    //   every j      the words of operand j + 1 (the next step's first behind j = 7)
     //   j = 0        the second half's activations
-    //   j = 4        [the wait and barrier in front: tile kc + 1 has landed for everyone, every read of tile kc is complete; a __syncthreads would drain the
-    //                younger transfers] the first half's activations of step kc + 1; Q odd: the next pair's packed words
-    //   j = 5        the transfers of tile kc + 4 into tile kc's buffer; Q == 0: the weights of the next quad
-    //   j = 6, 7     the next step's sign bits out of the packed words
-    // In-order completion: tile kc + 1 (requested in step kc - 3) has landed once at most the transfers of steps kc - 2 and kc - 1 are outstanding: 4 + 4 + two
-    // weight transfers if either opens a quad (Q = 1, 2) -- and everything older, including the next quad's weights (step 4j, first read in step 4j + 3), with it.
+    //   j = 0, 1     the sign bits of row tiles 2, 3;  j = 5, 6: of the next step's 0, 1 (their places are free by then)
+    //   j = 2        [the wait and barrier in front: tile kc + 1 has landed for everyone, every read of tile kc is complete; a __syncthreads would drain the
+    //                younger transfers]
+    //   j = 2 .. 5   the transfers of tile kc + 4 into tile kc's buffer, one an operand;  j = 6, 7, Q == 0: the weights of the next quad
+    //   j = 3        Q odd: the next pair's packed words
+    //   j = 4, 5     the first half's activations of step kc + 1
+    // In-order completion: tile kc + 1 (requested in step kc - 3) has landed once at most the transfers of steps kc - 2 and kc - 1 are outstanding: PER + PER +
+    // WPER weight transfers if either opens a quad (Q = 1, 2) -- and everything older, including the next quad's weights (step 4j, first read in step 4j + 3), with it.
     const auto step = [&](int kc, int Q, bool steady) __attribute__((always_inline)) {
+        uint32_t bw = 0, be = 0;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            if (j == 4) {
+            if (j == 2) {
                 if (!steady) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-                else if (Q == 1 || Q == 2) asm volatile("s_waitcnt vmcnt(10) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-                else asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                else if (Q == 1 || Q == 2) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(2 * PER + WPER) : "memory");
+                else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(2 * PER) : "memory");
             }
 #pragma unroll
             for (int rt = 0; rt < RT; ++rt) {
-                acc[j & 3][rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(ob_half8, cur), j < 4 ? bopA[rt] : bopB[rt], acc[j & 3][rt], 0, 0, 0);
-                if (rt < 4) nxt[rt] = word((j + 1) & 7, rt);
-                if (j >= 6 && (rt == 4 || rt == 5)) cw[2 * (j - 6) + rt - 4] = bits(2 * (j - 6) + rt - 4, (Q + 1) & 1);
-                if (j == 0) bopB[rt] = rd(Q, rt, 1);
-                if (j == 4 && (steady || Q < 3)) {
-                    bopA[rt] = rd((Q + 1) & 3, rt, 0);
-                    if ((Q & 1) && rt < 4) wp[rt] = rw(rt, (kc + 1) >> 1);
+                ob_mma_acc<false>(acc[j & 3][rt], cur, __builtin_bit_cast(ob_u32x4, j < 4 ? bopA[rt] : bopB[rt]));
+                __builtin_amdgcn_sched_barrier(0);
+                // (a word's two wait states before a product reads it: two instructions, as hipcc does not know that the assembly is one)
+                if (RT >= 6 && rt < 4) nxt[rt] = word((j + 1) & 7, rt);
+                if (RT < 6 && rt < 2) {
+                    nxt[2 * rt] = word((j + 1) & 7, 2 * rt);
+                    nxt[2 * rt + 1] = word((j + 1) & 7, 2 * rt + 1);
+                    if (RT == 3 && rt == 1) asm volatile("s_nop 0");
                 }
-                if (j == 5 && steady) {
-                    if (rt < 4) dma(kc + 4, rt);
-                    else if (Q == 0 && rt < 6) wdma((kc >> 2) + 1, rt - 4);
+                if (j == 0) bopB[rt] = rd(Q, rt, 1);
+                constexpr int B0 = RT - 3 + (RT == 3);                          // sign bits in two halves, behind products that make no word
+                if (j < 2 || j == 5 || j == 6) {
+                    const int rn = j < 2 ? j + 2 : j - 5, par = (j < 2 ? Q : Q + 1) & 1;
+                    if (rt == B0) { bw = wp[rn][par] >> wsh; be = bw & 0x5555u; }
+                    if (rt == B0 + 1) cw[rn] = ((bw << 15) & 0x55550000u) | be;
+                }
+                if (steady) {
+                    if (rt == RT - 1 && j >= 2 && j < 2 + PER) dma(kc + 4, j - 2);
+                    if (rt == RT - 1 && Q == 0 && j >= 6 && j < 6 + WPER) wdma((kc >> 2) + 1, j - 6);
+                }
+                if (steady || Q < 3) {
+                    constexpr int HALF = RT < 4 ? RT : 4;
+                    if (j == 3 && (Q & 1)) {
+                        if (rt < 4) wp[rt] = rw(rt, (kc + 1) >> 1);
+                        if (RT == 3 && rt == 2) wp[3] = rw(3, (kc + 1) >> 1);
+                    }
+                    if (j == 4 && rt < HALF) bopA[rt] = rd((Q + 1) & 3, rt, 0);
+                    if (j == 5 && rt < RT - HALF) bopA[HALF + rt] = rd((Q + 1) & 3, HALF + rt, 0);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -411,6 +445,11 @@ __device__ __forceinline__ void ob_gemm3_body(
         step(kc, 0, true); step(kc + 1, 1, true); step(kc + 2, 2, true); step(kc + 3, 3, true);
     }
     step(kc, 0, false); step(kc + 1, 1, false); step(kc + 2, 2, false); step(kc + 3, 3, false);      // its tiles are all requested: drain
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");            // the last sums leave the matrix pipe before anything reads them
+#pragma unroll
+    for (int x_ = 0; x_ < RN; ++x_)
+#pragma unroll
+        for (int y_ = 0; y_ < RT; ++y_) asm volatile("" : "+a"(acc[x_][y_]));
 
     // Epilogue through LDS (fp16 outputs, wave's 64 rows inside N): a lane's accumulators are 4 consecutive rows
     // of one token -- stored directly that is 8 bytes per lane and 32 contiguous bytes per token row and instruction.
@@ -418,7 +457,7 @@ __device__ __forceinline__ void ob_gemm3_body(
     // last barrier) staging memory and writes whole 128-byte row segments, 8 token rows per instruction.
     if (!PARTIAL && n0 + wn * 64 + 64 <= N && (N & 7) == 0 && (reinterpret_cast<size_t>(u) & 15) == 0) {
         constexpr int EP = 144;                                // bytes per token row: 128 + 16 (rows shift by 4 banks)
-        char *ep = smem + (size_t)wave * 128 * EP;
+        char *ep = smem + (size_t)wave * (16 * RT) * EP;
 #pragma unroll
         for (int rn = 0; rn < RN; ++rn) {
             const int nb = n0 + wn * 64 + rn * 16 + 4 * gq;
@@ -432,8 +471,9 @@ __device__ __forceinline__ void ob_gemm3_body(
             }
         }
         // (same wave wrote what it reads: no barrier, the compiler orders the LDS accesses with lgkmcnt)
-        _Float16 *ub = u + (int64_t)t0 * N + n0 + wn * 64;
-        const int trows = T - t0;
+        const int tw = t0 + wt * 16 * RT;
+        _Float16 *ub = u + (int64_t)tw * N + n0 + wn * 64;
+        const int trows = T - tw;
         // Optional (ONEBIT_FLAG_TILE_STATS; `zp` is the output, N % 64 == 0 host-checked): LayerNorm partials of the rows
         // just formed -- per token and 64-row block (sum, sum of squared deviations from the block mean) of the fp16 values
         // being stored.  The 8 lanes that write a token's 128-byte segment hold its 64 values: two 8-lane DPP reductions.
@@ -462,7 +502,7 @@ __device__ __forceinline__ void ob_gemm3_body(
                 m2 += OB_DPP_F(m2, 0x4E, 0xF);
                 m2 += OB_DPP_F(m2, 0x141, 0xF);
                 if (ch == 0 && row < trows)
-                    *reinterpret_cast<ob_float2 *>(tsp + ((int64_t)(t0 + row) * ntile64 + tile_idx) * 2) = (ob_float2){sm, m2};
+                    *reinterpret_cast<ob_float2 *>(tsp + ((int64_t)(tw + row) * ntile64 + tile_idx) * 2) = (ob_float2){sm, m2};
             }
         }
         return;
@@ -475,7 +515,7 @@ __device__ __forceinline__ void ob_gemm3_body(
         for (int i = 0; i < 4; ++i) gn[i] = PARTIAL ? 1.0f : (float)g[min(nb + i, N - 1)];
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
-            const int t = t0 + rt * 16 + r;
+            const int t = t0 + (wt * RT + rt) * 16 + r;
             if (t >= T) continue;
             if (PARTIAL) {
                 if (nb + 3 < N) {
@@ -502,12 +542,12 @@ __device__ __forceinline__ void ob_gemm3_body(
     }
 }
 
-template <bool PARTIAL, int RT>
+template <bool PARTIAL, int RT, int WN>
 __global__ __launch_bounds__(256, 2) void ob_gemm3_f16_kernel(
     const uint32_t *__restrict__ W, int64_t ldw_words, const _Float16 *__restrict__ a, int64_t lda,
     const _Float16 *__restrict__ g, _Float16 *__restrict__ u, float *__restrict__ zp, int T, int K, int N, int nbn)
 {
-    ob_gemm3_body<PARTIAL, RT>(W, ldw_words, a, lda, g, u, zp, T, K, N, nbn, ob_g3_bid());
+    ob_gemm3_body<PARTIAL, RT, WN>(W, ldw_words, a, lda, g, u, zp, T, K, N, nbn, ob_g3_bid());
 }
 
 // GROUPED form (round 6): up to three projections that share T, K and the row pitches -- q | k | v or gate | up of a decoder layer on the
@@ -520,7 +560,7 @@ struct ObG3Group {
     long long ldw_words, lda;
     int T, K;
 };
-template <int RT>
+template <int RT, int WN>
 __global__ __launch_bounds__(256, 2) void ob_gemm3g_f16_kernel(const ObG3Group G)
 {
     const int bid = ob_g3_bid();
@@ -532,7 +572,7 @@ __global__ __launch_bounds__(256, 2) void ob_gemm3g_f16_kernel(const ObG3Group G
     _Float16 *u = p == 0 ? G.u[0] : (p == 1 ? G.u[1] : G.u[2]);
     const int N = p == 0 ? G.N[0] : (p == 1 ? G.N[1] : G.N[2]);
     const int nbn = p == 0 ? G.nbn[0] : (p == 1 ? G.nbn[1] : G.nbn[2]);
-    ob_gemm3_body<false, RT>(W, G.ldw_words, a, G.lda, g, u, nullptr, G.T, G.K, N, nbn, bid - b0);
+    ob_gemm3_body<false, RT, WN>(W, G.ldw_words, a, G.lda, g, u, nullptr, G.T, G.K, N, nbn, bid - b0);
 }
 
 // K-SLICED form (round 6): ONE projection whose 256 x 128 tiles alone leave most of the chip idle (hidden-width outputs at a few hundred
@@ -546,7 +586,7 @@ struct ObG3Slices {
     long long ldw_words, lda;
     int T, N, nbn, tiles, ns, quads;
 };
-template <int RT>
+template <int RT, int WN>
 __global__ __launch_bounds__(256, 2) void ob_gemm3ks_f16_kernel(const ObG3Slices G)
 {
     const int bid = ob_g3_bid();
@@ -554,7 +594,7 @@ __global__ __launch_bounds__(256, 2) void ob_gemm3ks_f16_kernel(const ObG3Slices
     const int qb = G.quads / G.ns, qr = G.quads - qb * G.ns;
     const int q0 = j * qb + min(j, qr), nq = qb + (j < qr ? 1 : 0);
     float *zp = j == 0 ? G.z[0] : (j == 1 ? G.z[1] : (j == 2 ? G.z[2] : G.z[3]));
-    ob_gemm3_body<true, RT>(G.W + q0 * (4 * OB_G2_K / 32), G.ldw_words, G.a + q0 * (4 * OB_G2_K), G.lda, nullptr, nullptr, zp, G.T,
+    ob_gemm3_body<true, RT, WN>(G.W + q0 * (4 * OB_G2_K / 32), G.ldw_words, G.a + q0 * (4 * OB_G2_K), G.lda, nullptr, nullptr, zp, G.T,
                             nq * (4 * OB_G2_K), G.N, G.nbn, bid - j * G.tiles);
 }
 #undef RN

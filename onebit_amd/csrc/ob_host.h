@@ -68,21 +68,16 @@ OB_HIDDEN int ob_lm_head_argmax(const void *x, const void *lm_head, void *logits
 OB_HIDDEN int ob_sk3_multi(const onebit_proj_t *const *ps, void *const *us, const void *const *as, int np, int64_t T, hipStream_t s);
 // the projection's part of that eligibility (shape, pitch, the weights' alignment; rows assumed 16-byte aligned, 2 <= T <= 64)
 OB_HIDDEN bool ob_sk3_proj_ok(const onebit_proj_t &p);
-// up to three projections sharing T, K and the packed row pitch in ONE launch of the LDS-DMA prefill GEMM (ob_gemm3g_f16_kernel) on
+// one to three projections sharing T, K and the packed row pitch in ONE launch of the LDS-DMA prefill GEMM (ob_gemm3g_f16_kernel) on
 // their pre-scaled rows a[i] [T, K]: u[i] = fp16(fp16(W_i . a_i) * g_i).  ONEBIT_E_SHAPE when the group is not eligible (the caller
 // falls back to onebit_linear_forward per projection).
 OB_HIDDEN int ob_gemm3_grouped(const onebit_proj_t *const *ps, void *const *us, const void *const *as, int np, int64_t T, hipStream_t s);
-// the eligibility test of ob_gemm3_grouped alone (shapes, pitches, the weights' alignment, the GROUP's tile count against the CU count;
-// rows / outputs assumed 16-byte aligned): a caller that is about to choose between pre-scaled rows for the group and plain rows asks first
+// the eligibility test of ob_gemm3_grouped alone (shapes, pitches, the weights' alignment; rows / outputs assumed 16-byte aligned): a caller that is about to choose between pre-scaled rows for the group and plain rows asks first
 OB_HIDDEN bool ob_gemm3_group_ok(const onebit_proj_t *const *ps, int np, int64_t T);
-// 256 x 128 tiles of that launch (sum over the members) and the workgroup slots of one round (two workgroups per CU)
-OB_HIDDEN int64_t ob_gemm3_group_tiles(const onebit_proj_t *const *ps, int np, int64_t T);
-OB_HIDDEN int ob_gemm3_slots();
-// what a launch over `nb` 256-row blocks and T tokens costs with the tile it takes, in 1 / 8.4 of a full round of 128-token tiles (105 us at K = 4096)
-OB_HIDDEN double ob_gemm3_cost(int64_t nb, int64_t T);
+// what that launch takes by the estimate that its tile is chosen by, us
+OB_HIDDEN double ob_gemm3_group_us(const onebit_proj_t *const *ps, int np, int64_t T);
 // ONE projection on its pre-scaled rows a [T, K] as two to four K-slices in one launch of the LDS-DMA GEMM (fp32 sums z[i] [T, N], added and
 // scaled by the consuming row kernel): a hidden-width projection at a few hundred rows has too few 256 x 128 tiles for the chip (13B, 543 rows:
-// 100), its slices have that many times more.  ob_gemm3_ksplit_n: 0 when the projection alone is eligible for the LDS-DMA GEMM or no
-// slicing fills two thirds of the CUs, else the number of slices (the fewest that do).
+// 100), its slices have that many times more.  ob_gemm3_ksplit_n: the number of slices, 0 where none are the faster or the projection is not eligible.
 OB_HIDDEN int ob_gemm3_ksplit_n(const onebit_proj_t &p, int64_t T);
 OB_HIDDEN int ob_gemm3_ksplit(const onebit_proj_t &p, const void *a, float *const *z, int ns, int64_t T, hipStream_t s);

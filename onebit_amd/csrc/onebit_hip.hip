@@ -3,6 +3,7 @@
 // the caller's stream.
 #include <hip/hip_runtime.h>
 #include <algorithm>
+#include <math.h>
 #include <mutex>
 #include <stdarg.h>
 #include <stdio.h>
@@ -319,24 +320,66 @@ static bool ob_gemm3_ok(int64_t T, int64_t K, int64_t N)
     return 3 * tiles >= 2 * (int64_t)ob_cu_count() || env == 2;
 }
 
-// 16-token tiles per workgroup of the 4-wave form (8 = 128 tokens, 7, 6) for `nb` 256-row blocks (times K slices): rounds of two workgroups per CU
-// times the tile's size, a round of at most one per CU taking 0.55 of one of two (473 / 559 tiles of 4096 -> 11008: 107 / 153 us).  1540 rows: 12 x 86
-// tiles of 128 tokens for gate | up are 2.02 rounds, 16 x 86 of 96 are 2.69 three-quarter ones; 192 tiles of a hidden-width projection leave a quarter
-// of the CUs idle, 256 of 96 tokens none.
-static double ob_gemm3_tiles_cost(int64_t nb, int64_t T, int rt)
+// Which tile (WN waves of 64 rows x 64 / WN * RT tokens) and how many K slices a product of the LDS-DMA GEMM takes: the cheapest by an estimate of its time.  A launch
+// costs F us, and a K step of a CU's workgroups a + b t / 256 us while t <= 256 workgroups are in flight (one a CU at most), A + B (t / 256 - 1) up to two a CU,
+// whole rounds of two beyond; slices add their fp32 sums' way out and back in, 0.26 us a MB.  Fitted to 900 launches (K 1024 .. 13824, 70 .. 2000 rows, 2048 .. 13824
+// columns, 1 .. 4 slices; 5 % rms); its choices cost 0.4 % more than the best of those measured, the row pass included.  With 256 x 128 .. 96 tiles alone and slices
+// wherever they leave a third of the CUs idle -> as it is, the product: 100 rows 11008 -> 4096 29.6 -> 23.0 us, 250 rows 2048 -> 5632 18.2 -> 15.5, 1000 rows
+// 2048 -> 2048 20.9 -> 16.7, 250 rows 4096 -> 4096 20.8 -> 18.6.
+struct ObG3Cost { ObG3Form f; double F, a, b, A, B; };
+static double ob_g3_us(const ObG3Cost &c, const int64_t *N, int np, int64_t K, int64_t T, int ns)
 {
-    const int64_t cus = ob_cu_count(), slots = 2 * cus, t = nb * ((T + 16 * rt - 1) / (16 * rt)), rem = t % slots;
-    return ((double)(t / slots) + (rem == 0 ? 0.0 : rem <= cus ? 0.55 : 1.0)) * (rt + 0.4);
+    int64_t t = 0, z = 0;
+    for (int i = 0; i < np; ++i) { t += (N[i] + ob_g3_rows(c.f.wn) - 1) / ob_g3_rows(c.f.wn); z += N[i]; }
+    t *= (T + c.f.tokens() - 1) / c.f.tokens() * ns;
+    const int64_t quads = K / (4 * OB_G2_K);
+    const double L = (double)t / ob_cu_count(), full = floor(0.5 * L), rem = L - 2 * full;
+    const double step = full * (c.A + c.B) + (rem <= 0 ? 0.0 : rem <= 1 ? c.a + c.b * rem : c.A + c.B * (rem - 1));
+    return c.F + 4.0 * (double)((quads + ns - 1) / ns) * step + 1e-6 * (double)T * (double)z * (ns > 1 ? 0.26 * 4 * ns : 0.05 * 2);
 }
-static int ob_gemm3_rt(int64_t nb, int64_t T)
+// np projections of N[i] columns in one launch (one: in up to max_ns slices, of 512 columns of K at least)
+ObG3Plan ob_g3_plan(const int64_t *N, int np, int64_t K, int64_t T, int max_ns)
 {
-    static const int env = getenv("OB_GEMM3_RT") ? atoi(getenv("OB_GEMM3_RT")) : 0;        // A/B: 6, 7, 8
-    if (env >= 6 && env <= 8) return env;
-    int best = 8;
-    for (int rt = 7; rt >= 6; --rt) if (ob_gemm3_tiles_cost(nb, T, rt) < 0.97 * ob_gemm3_tiles_cost(nb, T, best)) best = rt;
+    static const ObG3Cost forms[] = {{{4, 8}, 7.5, 0.48, 0.24, 1.11, 0.19}, {{4, 7}, 7.3, 0.42, 0.23, 0.97, 0.21}, {{4, 6}, 7.0, 0.37, 0.22, 0.86, 0.18},
+                                     {{2, 4}, 5.4, 0.30, 0.17, 0.71, 0.11}, {{2, 3}, 5.1, 0.26, 0.14, 0.61, 0.07}};
+    static const int env = getenv("OB_GEMM3_RT") ? atoi(getenv("OB_GEMM3_RT")) : 0;        // A/B: 8, 7, 6 (256 rows), 4, 3 (128)
+    static const int ks_env = getenv("OB_GEMM3_KSPLIT") ? atoi(getenv("OB_GEMM3_KSPLIT")) : 4;         // A/B: 0 = no slices, 2 .. 4 = that many at most
+    // (the layers of a step ask for the same few shapes; 20 estimates are 0.3 us)
+    struct Key { int64_t N[3], K, T; int np, max_ns, cus; bool operator==(const Key &o) const { return N[0] == o.N[0] && N[1] == o.N[1] && N[2] == o.N[2] && K == o.K && T == o.T && np == o.np && max_ns == o.max_ns && cus == o.cus; } };
+    static thread_local struct { Key key; ObG3Plan plan; } memo[8];
+    static thread_local unsigned next = 0;
+    const Key key = {{N[0], np > 1 ? N[1] : 0, np > 2 ? N[2] : 0}, K, T, np, max_ns, ob_cu_count()};
+    for (const auto &m : memo) if (m.plan.ns && m.key == key) return m.plan;
+    const int quads = (int)(K / (4 * OB_G2_K));
+    max_ns = np == 1 ? std::max(1, std::min(std::min(max_ns, ks_env), quads / 2)) : 1;
+    ObG3Plan best = {};
+    for (const ObG3Cost &c : forms)
+        for (int ns = 1; ns <= max_ns; ++ns) {
+            const double us = ob_g3_us(c, N, np, K, T, ns);
+            if ((best.ns == 0 || us < best.us) && (env == 0 || env == c.f.rt)) best = {c.f, ns, us};
+        }
+    if (best.ns == 0) best = {forms[0].f, 1, ob_g3_us(forms[0], N, np, K, T, 1)};
+    memo[next] = {key, best};
+    next = (next + 1) % 8;
     return best;
 }
-double ob_gemm3_cost(int64_t nb, int64_t T) { return ob_gemm3_tiles_cost(nb, T, ob_gemm3_rt(nb, T)); }
+// From 65 rows on, and 1024 columns of K: fewer are few steps behind a launch's constant, and the 128 x 128 kernel needs no scaled rows
+static bool ob_g3_shape(int64_t T, int64_t K, int64_t N)
+{
+    static const int env3 = getenv("OB_GEMM3") ? atoi(getenv("OB_GEMM3")) : 1;
+    return env3 && T > 64 && K >= 1024 && K % (4 * OB_G2_K) == 0 && N >= 256 && N % 4 == 0 && T * K * 2 < ((int64_t)1 << 32) && N * (K / 8) < ((int64_t)1 << 32);
+}
+static int64_t ob_g3_blocks(int64_t N, int wn) { return (N + ob_g3_rows(wn) - 1) / ob_g3_rows(wn); }
+// go(form as a type): the kernel's instance
+template <typename GO>
+static void ob_gemm3_go(ObG3Form f, GO go)
+{
+    if (f.wn == 2 && f.rt == 3) go(std::integral_constant<int, 3>(), std::integral_constant<int, 2>());
+    else if (f.wn == 2) go(std::integral_constant<int, 4>(), std::integral_constant<int, 2>());
+    else if (f.rt == 6) go(std::integral_constant<int, 6>(), std::integral_constant<int, 4>());
+    else if (f.rt == 7) go(std::integral_constant<int, 7>(), std::integral_constant<int, 4>());
+    else go(std::integral_constant<int, 8>(), std::integral_constant<int, 4>());
+}
 
 // The LDS-DMA GEMM (ob_gemm2.h)
 #ifndef OB_GEMM4_DEFAULT
@@ -347,24 +390,23 @@ static void ob_launch_gemm3(const uint32_t *W, int64_t ldw_words, const _Float16
                             float *zp, int64_t T, int64_t K, int64_t N, hipStream_t s)
 {
     static const int g4_env = getenv("OB_GEMM4") ? atoi(getenv("OB_GEMM4")) : OB_GEMM4_DEFAULT;   // the 32x32x16-MFMA form of the same tiling (ob_gemm4.h)
-    const int nbn = (int)((N + OB_G2_N - 1) / OB_G2_N);
     if (g4_env) {
+        const int nbn = (int)((N + OB_G2_N - 1) / OB_G2_N);
         static bool attr_set[OB_MAX_DEVICES] = {};
         ob_set_max_lds_once(ob_gemm4_f16_kernel<PARTIAL>, attr_set, OB_G4_LDS);
         const int nbt = (int)((T + 127) / 128);
         hipLaunchKernelGGL((ob_gemm4_f16_kernel<PARTIAL>), dim3((unsigned)(nbn * nbt)), dim3(256), OB_G4_LDS, s,
                            W, ldw_words, a, lda, g, u, zp, (int)T, (int)K, (int)N, nbn);
     } else {
-        const int rt = ob_gemm3_rt(nbn, T);
-        const auto go = [&](auto kern, bool (&attr_set)[OB_MAX_DEVICES]) {
-            ob_set_max_lds_once(kern, attr_set, OB_G3_LDS);
-            hipLaunchKernelGGL(kern, dim3((unsigned)(nbn * ((T + 16 * rt - 1) / (16 * rt)))), dim3(256), OB_G3_LDS, s,
-                               W, ldw_words, a, lda, g, u, zp, (int)T, (int)K, (int)N, nbn);
-        };
-        static bool attr_set[3][OB_MAX_DEVICES] = {};
-        if (rt == 6) go(ob_gemm3_f16_kernel<PARTIAL, 6>, attr_set[0]);
-        else if (rt == 7) go(ob_gemm3_f16_kernel<PARTIAL, 7>, attr_set[1]);
-        else go(ob_gemm3_f16_kernel<PARTIAL, 8>, attr_set[2]);
+        const ObG3Form f = ob_g3_plan(&N, 1, K, T, 1).f;
+        ob_gemm3_go(f, [&](auto rt, auto wn) {
+            constexpr int R = decltype(rt)::value, WN = decltype(wn)::value;
+            static bool attr_set[OB_MAX_DEVICES] = {};
+            const int64_t nb = ob_g3_blocks(N, WN);
+            ob_set_max_lds_once(ob_gemm3_f16_kernel<PARTIAL, R, WN>, attr_set, ob_g3_lds(WN, R));
+            hipLaunchKernelGGL((ob_gemm3_f16_kernel<PARTIAL, R, WN>), dim3((unsigned)(nb * ((T + f.tokens() - 1) / f.tokens()))), dim3(256), ob_g3_lds(WN, R), s,
+                               W, ldw_words, a, lda, g, u, zp, (int)T, (int)K, (int)N, (int)nb);
+        });
     }
 }
 
@@ -381,13 +423,10 @@ static void ob_launch_ln_rows(const ObLnRowsArgs &la, int64_t T, hipStream_t s)
 }
 
 static inline size_t ob_align256(size_t b) { return (b + 255) & ~(size_t)255; }
-// shape part of ob_gemm3_ksplit_n's test (pointers unknown: onebit_linear_workspace_bytes)
-static bool ob_ksplit_shape_ok(int64_t T, int64_t K, int64_t N)
+// K slices of onebit_linear_forward's product: rows that ob_ln_rows_kernel adds them in
+static int ob_linear_slices(int64_t T, int64_t K, int64_t N)
 {
-    onebit_proj_t p = {};
-    static const char dummy[16] __attribute__((aligned(16))) = {};
-    p.weight = dummy; p.weight_scale = dummy; p.input_factor = dummy; p.N = N; p.K = K; p.ldw_bytes = K / 8;
-    return K % 128 == 0 && N % 8 == 0 && N <= OB_DEC_MAXV * OB_DEC_THREADS * 8 && ob_gemm3_ksplit_n(p, T) > 0;
+    return ob_g3_shape(T, K, N) && N % 8 == 0 && N <= OB_DEC_MAXV * OB_DEC_THREADS * 8 ? ob_g3_plan(&N, 1, K, T, 4).ns : 1;
 }
 
 static size_t ob_required_workspace(int64_t T, int64_t K, int64_t N, int dtype)
@@ -402,10 +441,11 @@ extern "C" size_t onebit_linear_workspace_bytes(int64_t T, int64_t K, int64_t N,
     if (T <= 0 || N <= 0) return 0;
     // large prefill calls run fastest with room for the pre-scaled activations a = fp16(x * h) (LDS-DMA
     // GEMM); a smaller or absent workspace is accepted and selects the register-staged kernel
-    if (dtype == ONEBIT_F16 && K % 32 == 0 && ob_gemm3_ok(T, K, N)) return (size_t)T * (size_t)K * 2;
-    // a few hundred rows of a projection whose tiles alone leave the chip idle: room for the pre-scaled rows AND the fp32 sums of up to
-    // four K-slices (ob_gemm3_ksplit); without it such a call keeps the register-staged kernel
-    if (dtype == ONEBIT_F16 && ob_ksplit_shape_ok(T, K, N)) return ob_align256((size_t)T * (size_t)K * 2) + 4 * ob_align256((size_t)T * (size_t)N * 4);
+    // -- and, where K slices are faster, their fp32 sums (without room for them: one slice)
+    if (dtype == ONEBIT_F16 && (ob_g3_shape(T, K, N) || (K % 32 == 0 && ob_gemm3_ok(T, K, N)))) {
+        const int ns = ob_linear_slices(T, K, N);
+        return ns == 1 ? (size_t)T * (size_t)K * 2 : ob_align256((size_t)T * (size_t)K * 2) + ns * ob_align256((size_t)T * (size_t)N * 4);
+    }
     // float32: the activations' three bf16 parts and the sums of split K (smaller or absent: ob_simple_kernel)
     if (dtype == ONEBIT_F32 && K > 0 && K % 8 == 0) return ob_f32_workspace(T, K, N);
     return ob_required_workspace(T, K, N, dtype);
@@ -467,33 +507,24 @@ extern "C" int onebit_linear_forward(const void *packed, int64_t ldw_bytes, cons
                 return ob_fail(ONEBIT_E_FLAG, "linear_forward: ONEBIT_FLAG_PRESCALED on a call no pre-scaled kernel takes");
             rc = ob_launch_status("linear_forward(skinny3)");
             if (rc) return rc;
-        } else if (prescaled || (ob_gemm3_ok(T, K, N) && workspace && workspace_bytes >= (size_t)T * (size_t)K * 2 && ob_aligned(workspace, 16) &&
-                                 ldw_bytes % 16 == 0 && ob_aligned(packed, 16) && N * ldw_bytes < ((int64_t)1 << 32))) {
-            // pre-scale once (the fp16 rounding of bitnet.py:113) -- unless the producer of x already did
-            // (ONEBIT_FLAG_PRESCALED) --, then the LDS-DMA GEMM on the scaled rows
-            const _Float16 *a = (const _Float16 *)x;
-            if (!prescaled) {
-                const int64_t nvec = T * K / 8;
-                hipLaunchKernelGGL(ob_scale_rows_kernel, dim3((unsigned)((nvec + 255) / 256)), dim3(256), 0, s, (const _Float16 *)x, K,
-                                   (const _Float16 *)h, (_Float16 *)workspace, T, (int)K);
-                a = (const _Float16 *)workspace;
-            }
-            ob_launch_gemm3<false>((const uint32_t *)packed, ldw_bytes / 4, a, K, (const _Float16 *)g, ubuf, tile_stats, T, K, N, s);
+        } else if (prescaled) {
+            // the producer of x scaled it (ONEBIT_FLAG_PRESCALED)
+            ob_launch_gemm3<false>((const uint32_t *)packed, ldw_bytes / 4, (const _Float16 *)x, K, (const _Float16 *)g, ubuf, tile_stats, T, K, N, s);
             tile_stats_done = tile_stats != nullptr;
             rc = ob_launch_status("linear_forward(gemm3)");
             if (rc) return rc;
-        } else {
-            // K-sliced LDS-DMA GEMM (ob_gemm3_ksplit) when the caller's workspace has room for the pre-scaled rows and the slices' fp32 sums:
-            // scale pass, ns short rounds of workgroups in one launch, then ONE row pass that adds the slices, applies fp16(fp16(.) * g)
-            // and the LayerNorm -- whole call, 512 rows: 11008 -> 4096 132 -> 65 us, 4096 -> 4096 57 -> 44 us (tools/module_T_sweep.py)
+        } else if ((ob_g3_shape(T, K, N) || ob_gemm3_ok(T, K, N)) && workspace && workspace_bytes >= (size_t)T * (size_t)K * 2 && ob_aligned(workspace, 16) &&
+                   ldw_bytes % 16 == 0 && ob_aligned(packed, 16) && N * ldw_bytes < ((int64_t)1 << 32)) {
+            // pre-scale once (the fp16 rounding of bitnet.py:113), then the LDS-DMA GEMM on the scaled rows, whole or in K slices whose sums ONE row pass adds
+            // behind it, with fp16(fp16(.) * g) and the LayerNorm
+            const int64_t nvec = T * K / 8;
+            hipLaunchKernelGGL(ob_scale_rows_kernel, dim3((unsigned)((nvec + 255) / 256)), dim3(256), 0, s, (const _Float16 *)x, K,
+                               (const _Float16 *)h, (_Float16 *)workspace, T, (int)K);
             onebit_proj_t pj = {};
             pj.weight = packed; pj.input_factor = h; pj.weight_scale = g; pj.N = N; pj.K = K; pj.ldw_bytes = ldw_bytes;
-            const int ns = (!tile_stats && N % 8 == 0 && N <= OB_DEC_MAXV * OB_DEC_THREADS * 8 && (!bias || ob_aligned(bias, 16))) ? ob_gemm3_ksplit_n(pj, T) : 0;
+            const int ns = tile_stats || (bias && !ob_aligned(bias, 16)) || ob_linear_slices(T, K, N) == 1 ? 0 : ob_gemm3_ksplit_n(pj, T);
             const size_t a_bytes = ob_align256((size_t)T * (size_t)K * 2), z_bytes = ob_align256((size_t)T * (size_t)N * 4);
-            if (ns > 0 && workspace && ob_aligned(workspace, 256) && workspace_bytes >= a_bytes + (size_t)ns * z_bytes) {
-                const int64_t nvec = T * K / 8;
-                hipLaunchKernelGGL(ob_scale_rows_kernel, dim3((unsigned)((nvec + 255) / 256)), dim3(256), 0, s, (const _Float16 *)x, K,
-                                   (const _Float16 *)h, (_Float16 *)workspace, T, (int)K);
+            if (ns > 0 && workspace_bytes >= a_bytes + (size_t)ns * z_bytes) {
                 float *zs[4] = {nullptr, nullptr, nullptr, nullptr};
                 for (int j = 0; j < ns; ++j) zs[j] = (float *)((char *)workspace + a_bytes + (size_t)j * z_bytes);
                 if ((rc = ob_gemm3_ksplit(pj, workspace, zs, ns, T, s))) return rc;
@@ -513,6 +544,11 @@ extern "C" int onebit_linear_forward(const void *packed, int64_t ldw_bytes, cons
                 }
                 return ob_launch_status("linear_forward(k-sliced)");
             }
+            ob_launch_gemm3<false>((const uint32_t *)packed, ldw_bytes / 4, (const _Float16 *)workspace, K, (const _Float16 *)g, ubuf, tile_stats, T, K, N, s);
+            tile_stats_done = tile_stats != nullptr;
+            rc = ob_launch_status("linear_forward(gemm3)");
+            if (rc) return rc;
+        } else {
             ob_launch_mm16<false>(packed, ldw_bytes, x, K, h, g, ubuf, nullptr, T, K, N, s);
             rc = ob_launch_status("linear_forward(mm16)");
             if (rc) return rc;
@@ -1712,94 +1748,69 @@ int ob_rows_norm(const ObRowsNormCall &c, hipStream_t s)
 
 bool ob_gemm3_group_ok(const onebit_proj_t *const *ps, int np, int64_t T)
 {
-    static const int env = getenv("OB_GEMM3_GROUPED") ? atoi(getenv("OB_GEMM3_GROUPED")) : 1;
-    static const int env3 = getenv("OB_GEMM3") ? atoi(getenv("OB_GEMM3")) : 1;
-    if (!env || !env3 || np < 2 || np > 3) return false;
+    static const int env = getenv("OB_GEMM3_GROUPED") ? atoi(getenv("OB_GEMM3_GROUPED")) : 1;       // A/B: 0 = one launch per projection
+    if (!env || np < 1 || np > 3) return false;
     const int64_t K = ps[0]->K, ldw = ps[0]->ldw_bytes;
-    if (T < 192 || K % (4 * OB_G2_K) != 0 || T * K * 2 >= ((int64_t)1 << 32) || ldw % 16 != 0) return false;
     int64_t tiles = 0;
     for (int i = 0; i < np; ++i) {
         const onebit_proj_t &p = *ps[i];
-        if (!p.weight || !p.weight_scale || p.K != K || p.ldw_bytes != ldw || p.N % 4 != 0 || p.N * (K / 8) >= ((int64_t)1 << 32) ||
-            p.N * ldw >= ((int64_t)1 << 32) || !ob_aligned(p.weight, 16) || !ob_aligned(p.weight_scale, 8))
+        if (!p.weight || !p.weight_scale || !ob_g3_shape(T, p.K, p.N) || p.K != K || p.ldw_bytes != ldw || ldw % 16 != 0 || p.N * ldw >= ((int64_t)1 << 32) ||
+            !ob_aligned(p.weight, 16) || !ob_aligned(p.weight_scale, 8))
             return false;
-        tiles += ((p.N + OB_G2_N - 1) / OB_G2_N) * ((T + 127) / 128);
+        tiles += ob_g3_blocks(p.N, 2) * ((T + 95) / 96);
     }
-    // a GROUP is worth one launch from half a round of workgroups on: the alternative is one launch of the round-1 kernel per member
-    static const int grp_den = getenv("OB_GEMM3_GROUP_DEN") ? atoi(getenv("OB_GEMM3_GROUP_DEN")) : 2;
-    return tiles * std::max(grp_den, 1) >= (int64_t)ob_cu_count() && tiles <= 0x3fffffff;
+    return tiles <= 0x3fffffff;
 }
-
-int64_t ob_gemm3_group_tiles(const onebit_proj_t *const *ps, int np, int64_t T)
+double ob_gemm3_group_us(const onebit_proj_t *const *ps, int np, int64_t T)
 {
-    int64_t tiles = 0;
-    for (int i = 0; i < np; ++i) tiles += ((ps[i]->N + OB_G2_N - 1) / OB_G2_N) * ((T + 127) / 128);
-    return tiles;
+    int64_t N[3];
+    for (int i = 0; i < np; ++i) N[i] = ps[i]->N;
+    return ob_g3_plan(N, np, ps[0]->K, T, 1).us;
 }
-int ob_gemm3_slots() { return 2 * ob_cu_count(); }
 
 int ob_gemm3_grouped(const onebit_proj_t *const *ps, void *const *us, const void *const *as, int np, int64_t T, hipStream_t s)
 {
-    static const int env = getenv("OB_GEMM3_GROUPED") ? atoi(getenv("OB_GEMM3_GROUPED")) : 1;       // A/B: 0 = one launch per projection
-    if (!env || np < 2 || np > 3) return ob_fail(ONEBIT_E_SHAPE, "gemm3_grouped: 2..3 projections");
+    if (!ob_gemm3_group_ok(ps, np, T)) return ob_fail(ONEBIT_E_SHAPE, "gemm3_grouped: not eligible");
     const int64_t K = ps[0]->K, ldw = ps[0]->ldw_bytes;
-    if (T < 192 || K % (4 * OB_G2_K) != 0 || T * K * 2 >= ((int64_t)1 << 32) || ldw % 16 != 0)
-        return ob_fail(ONEBIT_E_SHAPE, "gemm3_grouped: shape not eligible");
     ObG3Group G = {};
-    const int nbt = (int)((T + 127) / 128);
-    int64_t tiles = 0;
+    int64_t N[3];
     for (int i = 0; i < 3; ++i) {
         const int j = i < np ? i : np - 1;
         const onebit_proj_t &p = *ps[j];
-        if (i < np) {
-            if (!p.weight || !p.weight_scale || !us[i] || !as[i] || p.K != K || p.ldw_bytes != ldw || p.N % 4 != 0 || p.N * (K / 8) >= ((int64_t)1 << 32) ||
-                p.N * ldw >= ((int64_t)1 << 32) || !ob_aligned(p.weight, 16) || !ob_aligned(as[i], 16) || !ob_aligned(us[i], 16) || !ob_aligned(p.weight_scale, 8))
-                return ob_fail(ONEBIT_E_SHAPE, "gemm3_grouped: projection %d not eligible", i);
-            G.nbn[i] = (int)((p.N + OB_G2_N - 1) / OB_G2_N);
-            tiles += (int64_t)G.nbn[i] * nbt;
-        } else G.nbn[i] = G.nbn[j];
-        G.W[i] = (const uint32_t *)p.weight; G.a[i] = (const _Float16 *)as[j]; G.g[i] = (const _Float16 *)p.weight_scale; G.u[i] = (_Float16 *)us[j];
-        G.N[i] = (int)p.N; G.tile_end[i] = (int)tiles;
+        if (!us[j] || !as[j] || !ob_aligned(as[j], 16) || !ob_aligned(us[j], 16)) return ob_fail(ONEBIT_E_SHAPE, "gemm3_grouped: projection %d not eligible", j);
+        N[i] = p.N;
+        G.W[i] = (const uint32_t *)p.weight; G.a[i] = (const _Float16 *)as[j]; G.g[i] = (const _Float16 *)p.weight_scale; G.u[i] = (_Float16 *)us[j]; G.N[i] = (int)p.N;
     }
-    if (!ob_gemm3_group_ok(ps, np, T)) return ob_fail(ONEBIT_E_SHAPE, "gemm3_grouped: grid too small / large");
     G.ldw_words = ldw / 4; G.lda = K; G.T = (int)T; G.K = (int)K;
     static const int g4_env = getenv("OB_GEMM4") ? atoi(getenv("OB_GEMM4")) : OB_GEMM4_DEFAULT;
+    const ObG3Form f = g4_env ? ObG3Form{4, 8} : ob_g3_plan(N, np, K, T, 1).f;
+    int end = 0;
+    for (int i = 0; i < 3; ++i) {
+        G.nbn[i] = (int)ob_g3_blocks(G.N[i], f.wn);
+        if (i < np) end += G.nbn[i] * (int)((T + f.tokens() - 1) / f.tokens());
+        G.tile_end[i] = end;
+    }
     if (g4_env) {
         static bool attr_set4[OB_MAX_DEVICES] = {};
         ob_set_max_lds_once(ob_gemm4g_f16_kernel, attr_set4, OB_G4_LDS);
-        hipLaunchKernelGGL(ob_gemm4g_f16_kernel, dim3((unsigned)tiles), dim3(256), OB_G4_LDS, s, G);
+        hipLaunchKernelGGL(ob_gemm4g_f16_kernel, dim3((unsigned)end), dim3(256), OB_G4_LDS, s, G);
         return ob_launch_status("gemm4_grouped");
     }
-    const int64_t nb = tiles / nbt;
-    const int rt = ob_gemm3_rt(nb, T);
-    for (int i = 0; i < 3; ++i) G.tile_end[i] = (int)(G.tile_end[i] / nbt * ((T + 16 * rt - 1) / (16 * rt)));
-    const auto go = [&](auto kern, bool (&attr_set)[OB_MAX_DEVICES]) {
-        ob_set_max_lds_once(kern, attr_set, OB_G3_LDS);
-        hipLaunchKernelGGL(kern, dim3((unsigned)G.tile_end[2]), dim3(256), OB_G3_LDS, s, G);
-    };
-    static bool attr_set[3][OB_MAX_DEVICES] = {};
-    if (rt == 6) go(ob_gemm3g_f16_kernel<6>, attr_set[0]);
-    else if (rt == 7) go(ob_gemm3g_f16_kernel<7>, attr_set[1]);
-    else go(ob_gemm3g_f16_kernel<8>, attr_set[2]);
+    ob_gemm3_go(f, [&](auto rt, auto wn) {
+        constexpr int R = decltype(rt)::value, WN = decltype(wn)::value;
+        static bool attr_set[OB_MAX_DEVICES] = {};
+        ob_set_max_lds_once(ob_gemm3g_f16_kernel<R, WN>, attr_set, ob_g3_lds(WN, R));
+        hipLaunchKernelGGL((ob_gemm3g_f16_kernel<R, WN>), dim3((unsigned)end), dim3(256), ob_g3_lds(WN, R), s, G);
+    });
     return ob_launch_status("gemm3_grouped");
 }
 
 int ob_gemm3_ksplit_n(const onebit_proj_t &p, int64_t T)
 {
-    static const int env = getenv("OB_GEMM3_KSPLIT") ? atoi(getenv("OB_GEMM3_KSPLIT")) : 4;         // A/B: 0 = off, 2 .. 4 = that many slices at most
-    static const int env3 = getenv("OB_GEMM3") ? atoi(getenv("OB_GEMM3")) : 1;
-    // a projection with fewer tiles than this is sliced (default: what the unsliced LDS-DMA GEMM asks for, two thirds of the CUs)
-    static const int tiles_env = getenv("OB_GEMM3_KSPLIT_TILES") ? atoi(getenv("OB_GEMM3_KSPLIT_TILES")) : 0;
-    static const int tmin = getenv("OB_GEMM3_KSPLIT_TMIN") ? atoi(getenv("OB_GEMM3_KSPLIT_TMIN")) : 65;
-    if (env < 2 || !env3 || T < tmin || p.K % (4 * OB_G2_K) != 0 || p.N % 4 != 0 || T * p.K * 2 >= ((int64_t)1 << 32) || p.ldw_bytes % 16 != 0 ||
-        p.N * p.ldw_bytes >= ((int64_t)1 << 32) || !p.weight || !p.weight_scale || !ob_aligned(p.weight, 16) || !ob_aligned(p.weight_scale, 16))
+    if (!ob_g3_shape(T, p.K, p.N) || p.ldw_bytes % 16 != 0 || p.N * p.ldw_bytes >= ((int64_t)1 << 32) || !p.weight || !p.weight_scale ||
+        !ob_aligned(p.weight, 16) || !ob_aligned(p.weight_scale, 16))
         return 0;
-    const int64_t tiles = ((p.N + OB_G2_N - 1) / OB_G2_N) * ((T + 127) / 128);
-    const int64_t cus = ob_cu_count();
-    if (tiles_env ? tiles >= tiles_env : 3 * tiles >= 2 * cus) return 0;      // enough tiles alone
-    // as many slices as leave each at least four quads (1024 columns) of K loop: the shorter the loop, the shorter the one round
-    const int quads = (int)(p.K / (4 * OB_G2_K));
-    const int ns = std::min(std::min(env, 4), quads / 4);
+    const int ns = ob_g3_plan(&p.N, 1, p.K, T, 4).ns;
     return ns >= 2 ? ns : 0;
 }
 
@@ -1813,17 +1824,16 @@ int ob_gemm3_ksplit(const onebit_proj_t &p, const void *a, float *const *z, int 
         if (!G.z[i] || !ob_aligned(G.z[i], 16)) return ob_fail(ONEBIT_E_ALIGN, "gemm3_ksplit: partial sums must be 16-byte aligned");
     }
     G.W = (const uint32_t *)p.weight; G.a = (const _Float16 *)a; G.ldw_words = p.ldw_bytes / 4; G.lda = p.K; G.T = (int)T; G.N = (int)p.N;
-    G.nbn = (int)((p.N + OB_G2_N - 1) / OB_G2_N); G.ns = ns; G.quads = (int)(p.K / (4 * OB_G2_K));
-    const int rt = ob_gemm3_rt((int64_t)G.nbn * ns, T);
-    G.tiles = G.nbn * (int)((T + 16 * rt - 1) / (16 * rt));
-    const auto go = [&](auto kern, bool (&attr_set)[OB_MAX_DEVICES]) {
-        ob_set_max_lds_once(kern, attr_set, OB_G3_LDS);
-        hipLaunchKernelGGL(kern, dim3((unsigned)(ns * G.tiles)), dim3(256), OB_G3_LDS, s, G);
-    };
-    static bool attr_set[3][OB_MAX_DEVICES] = {};
-    if (rt == 6) go(ob_gemm3ks_f16_kernel<6>, attr_set[0]);
-    else if (rt == 7) go(ob_gemm3ks_f16_kernel<7>, attr_set[1]);
-    else go(ob_gemm3ks_f16_kernel<8>, attr_set[2]);
+    G.ns = ns; G.quads = (int)(p.K / (4 * OB_G2_K));
+    const ObG3Form f = ob_g3_plan(&p.N, 1, p.K, T, 4).f;
+    G.nbn = (int)ob_g3_blocks(p.N, f.wn);
+    G.tiles = G.nbn * (int)((T + f.tokens() - 1) / f.tokens());
+    ob_gemm3_go(f, [&](auto rt, auto wn) {
+        constexpr int R = decltype(rt)::value, WN = decltype(wn)::value;
+        static bool attr_set[OB_MAX_DEVICES] = {};
+        ob_set_max_lds_once(ob_gemm3ks_f16_kernel<R, WN>, attr_set, ob_g3_lds(WN, R));
+        hipLaunchKernelGGL((ob_gemm3ks_f16_kernel<R, WN>), dim3((unsigned)(ns * G.tiles)), dim3(256), ob_g3_lds(WN, R), s, G);
+    });
     return ob_launch_status("gemm3_ksplit");
 }
 

@@ -267,10 +267,8 @@ extern "C" int onebit_mixed_step(const onebit_model_t *m, const onebit_mixed_sta
         return onebit_linear_forward(p.weight, p.ldw_bytes, rows, p.input_factor, p.weight_scale, nullptr, u, nullptr, w.gemm_ws, w.gemm_ws_bytes,
                                      T, p.K, p.N, ONEBIT_F16, m->ln_eps, ONEBIT_FLAG_SKIP_LN | (prescaled ? ONEBIT_FLAG_PRESCALED : 0u), s);
     };
-    // 65 .. sk_rows rows: too few for the LDS-DMA GEMM's 256 x 128 tiles to fill the chip even grouped, and the round-1 kernels that took
-    // such calls run a 95-row step at 13B widths in 22.9 ms (a 543-row step: 20.5).  The LDS-DMA skinny GEMM in balanced passes of <= 64 rows
-    // re-reads the packed rows once per pass (40 MB per layer at 13B) and is still 1.5 - 2.7x faster: 95 rows 22.9 -> 8.6 ms, 159 rows 23.2 -> 11.9,
-    // 231 rows 21.8 -> 14.4, 287 rows 18.7 (grouped LDS-DMA GEMM) -> 17.6; 351 rows 18.9 vs 19.1: the grouped GEMM takes over (tools/midt_probe.py).
+    // 65 .. sk_rows rows that the LDS-DMA GEMM does not take, or takes longer for by its estimate: the LDS-DMA skinny GEMM in balanced passes of <= 64 rows, which
+    // re-reads the packed rows once per pass.  A pass: 7.0 us for q | k | v of width 2048, 8.0 gate | up, 13.2 and 18 at width 4096.
     static const int sk_rows = getenv("OB_MIXED_SK_ROWS") ? atoi(getenv("OB_MIXED_SK_ROWS")) : 320;
     bool sk_pass = T > 64 && T <= sk_rows;
     for (int l = 0; sk_pass && l < m->n_layers; ++l) {
@@ -278,6 +276,11 @@ extern "C" int onebit_mixed_step(const onebit_model_t *m, const onebit_mixed_sta
         sk_pass = ob_sk3_proj_ok(L.q) && ob_sk3_proj_ok(L.k) && ob_sk3_proj_ok(L.v) && ob_sk3_proj_ok(L.o) && ob_sk3_proj_ok(L.gate) &&
                   ob_sk3_proj_ok(L.up) && ob_sk3_proj_ok(L.down);
     }
+    auto sk_us = [&](const onebit_proj_t *const *ps, int np, int64_t rows) -> double {
+        double n = 0;
+        for (int i = 0; i < np; ++i) n += (double)ps[i]->N;
+        return (double)((rows + 63) / 64) * (5.4 + 0.145e-6 * n * (double)ps[0]->K);
+    };
     auto sk_passes = [&](const onebit_proj_t *const *ps, void *const *us, const _Float16 *const *as, int np) -> int {
         const int nblk = (T + 63) / 64, rows = (T + nblk - 1) / nblk;
         for (int r0 = 0; r0 < T; r0 += rows) {
@@ -292,36 +295,31 @@ extern "C" int onebit_mixed_step(const onebit_model_t *m, const onebit_mixed_sta
     };
     // up to three projections sharing their input: ONE skinny launch when T <= 64, else one GEMM each
     auto gemm_group = [&](const onebit_proj_t *const *ps, void *const *us, const _Float16 *const *as, int np, bool prescaled) -> int {
-        if (prescaled && T >= 2 && T <= 64) {
+        if (prescaled && np > 1 && T >= 2 && T <= 64) {
             const void *av[3] = {as[0], as[np > 1 ? 1 : 0], as[np > 2 ? 2 : 0]};
             if (ob_sk3_multi(ps, us, av, np, T, s) == 0) return 0;
         }
-        if (prescaled && T >= 192) {             // one grouped launch of the LDS-DMA GEMM: no partly filled last round per projection
+        // one grouped launch of the LDS-DMA GEMM: no partly filled last round per projection
+        if (prescaled && ob_gemm3_group_ok(ps, np, T) && !(sk_pass && sk_us(ps, np, T) < ob_gemm3_group_us(ps, np, T))) {
             const void *av[3] = {as[0], as[np > 1 ? 1 : 0], as[np > 2 ? 2 : 0]};
-            // TAIL: when the last token tile (<= 128 rows) is what pushes the launch into one more round of workgroups (13B gate|up at 543
-            // rows: 540 tiles on 512 slots; a round costs ~100 us whatever its fill), the rows of that tile go through the skinny GEMM
-            // instead (one or two passes, ~30 us each) and the grouped launch covers whole rounds
+            // TAIL: where the last token tile (<= 128 rows) is what pushes the launch into one more round of workgroups (13B gate | up at 543 rows: 540 tiles on 512
+            // slots), the rows of that tile go through the skinny GEMM instead and the grouped launch covers whole rounds
             static const int tail_env = getenv("OB_MIXED_TAIL") ? atoi(getenv("OB_MIXED_TAIL")) : 128;      // A/B: 0 = off; else the most tail rows
             const int nbt = (T + 127) / 128, Tm = 128 * (nbt - 1), tail = T - Tm;
-            if (tail_env > 0 && tail >= 2 && tail <= tail_env && Tm >= 192 && ob_gemm3_group_ok(ps, np, Tm)) {
-                const int64_t slots = ob_gemm3_slots();
-                const int64_t r_all = (ob_gemm3_group_tiles(ps, np, T) + slots - 1) / slots, r_main = (ob_gemm3_group_tiles(ps, np, Tm) + slots - 1) / slots;
-                // (a pass of the skinny GEMM: 30 us next to a round's 105 at K = 4096, 2.4 in ob_gemm3_cost's unit)
-                const int64_t nb = ob_gemm3_group_tiles(ps, np, T) / nbt;
-                bool sk_ok = r_main < r_all && ob_gemm3_cost(nb, Tm) + 2.4 * ((tail + 63) / 64) < ob_gemm3_cost(nb, T);
-                for (int i = 0; sk_ok && i < np; ++i) sk_ok = ob_sk3_proj_ok(*ps[i]);
-                if (sk_ok && ob_gemm3_grouped(ps, us, av, np, Tm, s) == 0) {
-                    const int nblk = (tail + 63) / 64, rows = (tail + nblk - 1) / nblk;
-                    for (int r0 = Tm; r0 < T; r0 += rows) {
-                        const int n = std::min(rows, T - r0);
-                        void *ub[3] = {nullptr, nullptr, nullptr};
-                        const void *ab[3] = {nullptr, nullptr, nullptr};
-                        for (int i = 0; i < np; ++i) { ub[i] = (_Float16 *)us[i] + (size_t)r0 * ps[i]->N; ab[i] = as[i] + (size_t)r0 * ps[i]->K; }
-                        const int rc2 = ob_sk3_multi(ps, ub, ab, np, n, s);           // (n >= 2: tail >= 2, blocks balanced)
-                        if (rc2) return rc2;
-                    }
-                    return 0;
+            bool sk_ok = tail_env > 0 && tail >= 2 && tail <= tail_env && ob_gemm3_group_ok(ps, np, Tm) &&
+                         ob_gemm3_group_us(ps, np, Tm) + sk_us(ps, np, tail) < ob_gemm3_group_us(ps, np, T);
+            for (int i = 0; sk_ok && i < np; ++i) sk_ok = ob_sk3_proj_ok(*ps[i]);
+            if (sk_ok && ob_gemm3_grouped(ps, us, av, np, Tm, s) == 0) {
+                const int nblk = (tail + 63) / 64, rows = (tail + nblk - 1) / nblk;
+                for (int r0 = Tm; r0 < T; r0 += rows) {
+                    const int n = std::min(rows, T - r0);
+                    void *ub[3] = {nullptr, nullptr, nullptr};
+                    const void *ab[3] = {nullptr, nullptr, nullptr};
+                    for (int i = 0; i < np; ++i) { ub[i] = (_Float16 *)us[i] + (size_t)r0 * ps[i]->N; ab[i] = as[i] + (size_t)r0 * ps[i]->K; }
+                    const int rc2 = ob_sk3_multi(ps, ub, ab, np, n, s);           // (n >= 2: tail >= 2, blocks balanced)
+                    if (rc2) return rc2;
                 }
+                return 0;
             }
             if (ob_gemm3_grouped(ps, us, av, np, T, s) == 0) return 0;
         }
@@ -342,18 +340,13 @@ extern "C" int onebit_mixed_step(const onebit_model_t *m, const onebit_mixed_sta
         if ((rc = check(L.q, H, NQ, "q", l)) || (rc = check(L.k, H, NK, "k", l)) || (rc = check(L.v, H, NK, "v", l)) || (rc = check(L.o, NQ, H, "o", l)) ||
             (rc = check(L.gate, H, I, "gate", l)) || (rc = check(L.up, H, I, "up", l)) || (rc = check(L.down, I, H, "down", l)))
             return rc;
-        // pre-scaled rows for a group when every member takes them on its own -- or when the GROUP as one launch fills the chip although a
-        // member alone would not (543 rows at 13B widths: 100 tiles per attention projection, 300 for q|k|v: the grouped LDS-DMA GEMM
-        // instead of three launches of the 128 x 128 kernel)
-        const onebit_proj_t *g_qkv[3] = {&L.q, &L.k, &L.v}, *g_gu[3] = {&L.gate, &L.up, nullptr};
-        const bool grp_qkv = ob_gemm3_group_ok(g_qkv, 3, T), grp_gu = ob_gemm3_group_ok(g_gu, 2, T);
-        // o_proj / down_proj (hidden-width outputs: half the tiles of a q|k|v group) that alone do not fill the chip run as two K-slices of
-        // the same LDS-DMA GEMM; the row kernel that consumes them adds the slices (ks_prev: the previous layer's down_proj went that way)
-        // (0 where the projection alone fills the chip; up to 128 rows two skinny passes are faster: 95 rows 8.6 vs 9.0 ms, 131 rows 11.7 vs 10.9)
-        const bool ks_use = !(sk_pass && T <= 128);
-        const int ks_o = ks_use ? ob_gemm3_ksplit_n(L.o, T) : 0, ks_down = ks_use ? ob_gemm3_ksplit_n(L.down, T) : 0;
-        const bool pres_qkv = (pres_ok(L.q) && pres_ok(L.k) && pres_ok(L.v)) || grp_qkv || sk_pass, pres_o = pres_ok(L.o) || ks_o > 0 || sk_pass;
-        const bool pres_gu = (pres_ok(L.gate) && pres_ok(L.up)) || grp_gu || sk_pass, pres_down = pres_ok(L.down) || ks_down > 0 || sk_pass;
+        // o_proj / down_proj: two to four K slices where those are faster; the row kernel that consumes them adds the slices (ks_prev: the previous layer's
+        // down_proj went that way)
+        const onebit_proj_t *g_qkv[3] = {&L.q, &L.k, &L.v}, *g_gu[3] = {&L.gate, &L.up, nullptr}, *g_o[1] = {&L.o}, *g_down[1] = {&L.down};
+        const bool grp_qkv = ob_gemm3_group_ok(g_qkv, 3, T), grp_gu = ob_gemm3_group_ok(g_gu, 2, T), grp_o = ob_gemm3_group_ok(g_o, 1, T), grp_down = ob_gemm3_group_ok(g_down, 1, T);
+        const int ks_o = ob_gemm3_ksplit_n(L.o, T), ks_down = ob_gemm3_ksplit_n(L.down, T);
+        const bool pres_qkv = (pres_ok(L.q) && pres_ok(L.k) && pres_ok(L.v)) || grp_qkv || sk_pass, pres_o = pres_ok(L.o) || ks_o > 0 || grp_o || sk_pass;
+        const bool pres_gu = (pres_ok(L.gate) && pres_ok(L.up)) || grp_gu || sk_pass, pres_down = pres_ok(L.down) || ks_down > 0 || grp_down || sk_pass;
         // 1. residual (+ LayerNorm of the previous down_proj) + input RMSNorm -> x, or the three consumers' pre-scaled rows
         ObRowsNormCall n1 = {};
         if (l == 0) { n1.embed = m->embed; n1.tokens = st->tokens; }
@@ -387,9 +380,11 @@ extern "C" int onebit_mixed_step(const onebit_model_t *m, const onebit_mixed_sta
             return rc;
         // 5. o_proj
         if (ks_o) { if ((rc = ob_gemm3_ksplit(L.o, w.attn, w.z, ks_o, T, s))) return rc; }
-        else if (sk_pass) { const onebit_proj_t *p1[3] = {&L.o, nullptr, nullptr}; void *u1[3] = {w.uo, nullptr, nullptr}; const _Float16 *a1[3] = {w.attn, nullptr, nullptr};
-                            if ((rc = sk_passes(p1, u1, a1, 1))) return rc; }
-        else if ((rc = gemm(L.o, w.attn, pres_o, w.uo))) return rc;
+        else {
+            void *u1[3] = {w.uo, nullptr, nullptr};
+            const _Float16 *a1[3] = {w.attn, nullptr, nullptr};
+            if ((rc = gemm_group(g_o, u1, a1, 1, pres_o))) return rc;
+        }
         // 6. residual + LayerNorm(u_o) (+ o bias) + post-attention RMSNorm
         ObRowsNormCall n2 = {};
         n2.hres_in = w.hB; n2.bias_prev = L.o_bias;
@@ -410,9 +405,11 @@ extern "C" int onebit_mixed_step(const onebit_model_t *m, const onebit_mixed_sta
         }
         if ((rc = onebit_rows_swiglu(w.ug, w.uu, pres_down ? L.down.input_factor : nullptr, w.act, T, I, m->ln_eps, s))) return rc;
         if (ks_down) { if ((rc = ob_gemm3_ksplit(L.down, w.act, w.z, ks_down, T, s))) return rc; }
-        else if (sk_pass) { const onebit_proj_t *p1[3] = {&L.down, nullptr, nullptr}; void *u1[3] = {w.ud, nullptr, nullptr}; const _Float16 *a1[3] = {w.act, nullptr, nullptr};
-                            if ((rc = sk_passes(p1, u1, a1, 1))) return rc; }
-        else if ((rc = gemm(L.down, w.act, pres_down, w.ud))) return rc;
+        else {
+            void *u1[3] = {w.ud, nullptr, nullptr};
+            const _Float16 *a1[3] = {w.act, nullptr, nullptr};
+            if ((rc = gemm_group(g_down, u1, a1, 1, pres_down))) return rc;
+        }
         ks_prev = ks_down;
     }
     // final norm on the rows that sample, lm_head + greedy token (<= 64 rows per launch)

@@ -41,8 +41,8 @@ class Kernel:
         return [int(v) for v in re.findall(r"L[ib](\d+)E", self.name)]
 
 
-def _kernels(src, tmp):
-    lib, sources = LIBS[src]
+def _kernels(src, tmp, KERNEL=KERNEL):
+    lib, sources = LIBS.get(src, (B.LIB, B.SOURCES))
     if not os.path.exists(B._obj(src)):
         B.build(lib=lib, sources=sources)
     data = open(B._obj(src), "rb").read()
@@ -137,12 +137,12 @@ def _regs(ops, kind="v"):
     return out
 
 
-def test_operands_are_not_written_in_front_of_their_products(kernels):
+def _operands_are_ready(kernels, scratch="scratch_"):
     products = 0
     for k in kernels:
         mf = [i for i, (op, _) in enumerate(k.text) if op.startswith("v_mfma")]
         products += len(mf)
-        assert not any(op.startswith("scratch_") for op, _ in k.text[mf[0]:mf[-1]]), f"{k.name}: a register in scratch between products"
+        assert not any(op.startswith(scratch) for op, _ in k.text[mf[0]:mf[-1]]), f"{k.name}: a register in scratch between products"
         for i in mf:
             parts = re.findall(r"[va]\[\d+:\d+\]", k.text[i][1])
             assert len(parts) == 4 and parts[0] == parts[3] and parts[0][0] == "a" and parts[1][0] == parts[2][0] == "v", (k.name, k.text[i])
@@ -154,4 +154,32 @@ def test_operands_are_not_written_in_front_of_their_products(kernels):
                     assert not _regs(to) & operands and not _regs(to, "a") & sums, f"{k.name}: {op} {ops} in front of {k.text[i]}"
                 states += 1 + (int(ops) if op == "s_nop" else 0)
                 j -= 1
-    assert products > 5000
+    return products
+
+
+def test_operands_are_not_written_in_front_of_their_products(kernels):
+    assert _operands_are_ready(kernels) > 5000
+
+
+@pytest.fixture(scope="module")
+def one_bit(tmp_path_factory):
+    """The 1-bit LDS-DMA product (csrc/ob_gemm2.h, ob_gemm3_body): single, grouped and K-sliced, every tile."""
+    return _kernels("onebit_hip.hip", tmp_path_factory.mktemp("one_bit"), re.compile(r"ob_gemm3(g|ks)?_f16_kernel"))
+
+
+def _tile(k):
+    rt, wn = k.args()[-2:]
+    per = (128 if wn == 4 else 32 * rt) // 32                            # transfers of a wave and step; wn / 2 more for a quad's weights
+    return rt, wn, 2 * per + wn // 2
+
+
+def test_one_bit_products_wait_for_the_tile_they_publish(one_bit):
+    assert len({k.name for k in one_bit}) == 20
+    for k in one_bit:
+        most = _tile(k)[2]
+        late = _late_transfers(k, most)
+        assert late == most, f"{k.name}: {late} transfers on their way behind a barrier, {most} are of later steps"
+
+
+def test_one_bit_operands_are_not_written_in_front_of_their_products(one_bit):
+    assert _operands_are_ready(one_bit, "scratch_load") > 5000             # (the largest tile stores what its epilogue reads, in front of its last steps)
