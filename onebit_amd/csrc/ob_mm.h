@@ -36,22 +36,26 @@ template <bool BF16> __device__ __forceinline__ void ob_mma_acc(ob_float4 &c, ob
 
 // acc[i][j] = sum over nk k steps of w_i a_j.  rw(buf, i), ra(buf, j): operand fragments of the step in LDS buffer `buf`; dma(d, k, buf): transfer d
 // of this wave's PER of step k into `buf` (steps beyond the last are requested too, nobody reads them: dma clamps k).  All waves of the workgroup.
-template <bool BF16, int MN, int MT, int PER, int NST, typename RW, typename RA, typename DMA>
+// CONT: onto the sums that a loop before left in acc.
+template <bool BF16, int MN, int MT, int PER, int NST, bool CONT = false, typename RW, typename RA, typename DMA>
 __device__ __forceinline__ void ob_mm_loop(ob_float4 (&acc)[MN][MT], int nk, RW rw, RA ra, DMA dma)
 {
+    if constexpr (CONT) asm volatile("s_barrier" ::: "memory");         // (everyone is done with the buffers)
     constexpr int H = MN / 2, VM = (NST - 2) * PER, WAIT = (VM & 15) | 0x70 | (VM >> 4 << 14);        // vmcnt(VM), lgkmcnt(0)
     static_assert(MN % 2 == 0 && NST >= 3 && VM < 64, "steps in flight");
 #pragma unroll
     for (int s = 0; s < NST; ++s)
 #pragma unroll
         for (int d = 0; d < PER; ++d) dma(d, s, s);
+    if constexpr (!CONT) {
 #pragma unroll
-    for (int i = 0; i < MN; ++i)
+        for (int i = 0; i < MN; ++i)
 #pragma unroll
-        for (int j = 0; j < MT; ++j) {
-            acc[i][j] = (ob_float4){0.f, 0.f, 0.f, 0.f};
-            asm volatile("" : "+a"(acc[i][j]));
-        }
+            for (int j = 0; j < MT; ++j) {
+                acc[i][j] = (ob_float4){0.f, 0.f, 0.f, 0.f};
+                asm volatile("" : "+a"(acc[i][j]));
+            }
+    }
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" :: "n"((NST - 1) * PER) : "memory");               // (the zeros above are long written)
     ob_u32x4 w[MN], a[MT];
 #pragma unroll
@@ -123,10 +127,11 @@ static inline double ob_wr_cost(int64_t t, int mt, int64_t cus)
 
 // acc[i][j] = sum over nk k steps of direct_i other_j (SWAP: the direct operand is the MFMA's second).  Direct tile i of step k: 16 bytes at wb[i] + 1024 k + wlane.
 // ra(buf, j): operand j of the step in LDS buffer `buf`; dma(d, k, buf): transfer d of this wave's PER of step k < nk into `buf`; dma_next(d, u, buf): the
-// same of step u + NST - 1 behind the turn's first one, in turns one behind the other from the first on.  All waves of the workgroup.
-template <bool BF16, bool SWAP, int MT, int PER, int NST, typename RA, typename DMA, typename DMAN>
+// same of step u + NST - 1 behind the turn's first one, in turns one behind the other from the first on.  All waves of the workgroup.  CONT: as above.
+template <bool BF16, bool SWAP, int MT, int PER, int NST, bool CONT = false, typename RA, typename DMA, typename DMAN>
 __device__ __forceinline__ void ob_wr_loop(ob_float4 (&acc)[4][MT], int nk, const char *const (&wb)[4], uint32_t wlane, RA ra, DMA dma, DMAN dma_next)
 {
+    if constexpr (CONT) asm volatile("s_barrier" ::: "memory");
     constexpr int MN = 4, H = MT / 2, G = MT - H, C = NST / 2, VM = (NST - 2) * (PER + MN), WAIT = (VM & 15) | 0x70 | (VM >> 4 << 14);
     static_assert(VM + 2 * MN < 64 && 2 * PER <= H * MN && 2 * G <= H * MN + 1 && 2 * H <= G * MN + 1, "vmcnt; places behind MFMAs");
     ob_u32x4 w[NST][MN], a[MT];
@@ -140,13 +145,15 @@ __device__ __forceinline__ void ob_wr_loop(ob_float4 (&acc)[4][MT], int nk, cons
 #pragma unroll
         for (int i = 0; i < MN; ++i) wload(i, s, s);
     }
+    if constexpr (!CONT) {
 #pragma unroll
-    for (int i = 0; i < MN; ++i)
+        for (int i = 0; i < MN; ++i)
 #pragma unroll
-        for (int j = 0; j < MT; ++j) {
-            acc[i][j] = (ob_float4){0.f, 0.f, 0.f, 0.f};
-            asm volatile("" : "+a"(acc[i][j]));
-        }
+            for (int j = 0; j < MT; ++j) {
+                acc[i][j] = (ob_float4){0.f, 0.f, 0.f, 0.f};
+                asm volatile("" : "+a"(acc[i][j]));
+            }
+    }
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" :: "n"(VM + 2 * MN) : "memory");                       // (the zeros above are long written)
 #pragma unroll

@@ -4,15 +4,9 @@
 #include "ob_host.h"
 #include "ob_train.h"
 #include "ob_train16.h"
+#include "ob_train32.h"
 
 // onebit_train_forward / onebit_train_backward: bitnet.py:14-28 (SignSTE) and :58-68 (BitLinear.forward)
-template <bool RCA, bool RCB, int TXA, int TXB, int EPI>
-static void ob_launch_tgemm(const ObTGemmArgs &a, hipStream_t s)
-{
-    const dim3 grid((unsigned)((a.N + OB_TG_BN - 1) / OB_TG_BN), (unsigned)((a.M + OB_TG_BM - 1) / OB_TG_BM));
-    hipLaunchKernelGGL((ob_tgemm_kernel<RCA, RCB, TXA, TXB, EPI>), grid, dim3(OB_TG_THREADS), 0, s, a);
-}
-
 static size_t ob_train_align(size_t b) { return (b + 255) & ~(size_t)255; }
 
 // ---- float16 (ob_train16.h) ---------------------------------------------------------------------------------------------
@@ -139,22 +133,122 @@ static int ob_t16_backward(const void *gy, const void *x, const void *w, const v
     return ob_launch_status("train_backward(grad weight)");
 }
 
+// ---- float32 (ob_train32.h) ---------------------------------------------------------------------------------------------
+static void ob_t32_tiles(bool sign, const void *p, const void *vec, char *out, int64_t rows, int64_t cols, hipStream_t s)
+{
+    ObT32Tiles a = {(const float *)p, (const float *)vec, out, ob_t16_bytes(rows, cols), (int)rows, (int)cols, (int)(ob_t16_up32(rows) / 16), (int)(ob_t16_up32(cols) / 32)};
+    const unsigned grid = (unsigned)(((int64_t)a.bands * ((a.ct + 3) / 4) + 3) / 4);
+    if (sign) hipLaunchKernelGGL(ob_t32_tiles_kernel<OB_T16_SIGN>, dim3(grid), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL(ob_t32_tiles_kernel<OB_T16_SCALE>, dim3(grid), dim3(256), 0, s, a);
+}
+
+// the tiles of ob_t16_mm (which states both sides of each line)
+template <int EPI, bool TRW, bool TRA>
+static void ob_t32_mm(const ObT32Mm &a, hipStream_t s)
+{
+    constexpr bool SWAP = TRW, TRL = TRW || TRA;
+    const int64_t cus = ob_cu_count(), narrow = (int64_t)((a.nw + 7) / 8) * ((a.na + 7) / 8), nd = ((SWAP ? a.na : a.nw) + 15) / 16, nl = SWAP ? a.nw : a.na;
+    const auto go = [&](auto kern, int64_t grid, int lds, bool (&attr_set)[OB_MAX_DEVICES]) {
+        ob_set_max_lds_once(kern, attr_set, lds);
+        hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), lds, s, a);
+    };
+    static bool attr_set[3][OB_MAX_DEVICES] = {};
+    const int64_t t8 = nd * ((nl + 7) / 8), t16 = nd * ((nl + 15) / 16);
+    if (narrow <= cus) go(ob_t32_mm_kernel<EPI, TRW, TRA>, narrow, 4 * 16 * 1024, attr_set[0]);
+    else if (ob_wr_cost(t8, 8, cus) <= ob_wr_cost(t16, 16, cus)) go(ob_t32_wr_kernel<EPI, TRL, SWAP, 8>, t8, ob_wr_steps(8) * 8 * 1024, attr_set[1]);
+    else go(ob_t32_wr_kernel<EPI, TRL, SWAP, 16>, t16, ob_wr_steps(16) * 16 * 1024, attr_set[2]);
+}
+
+static void ob_t32_layernorm(const void *z, const void *g, const void *bias, void *y, float *stats, int64_t T, int64_t N, float eps, hipStream_t s)
+{
+#define OB_T32_LN(NV_) hipLaunchKernelGGL(ob_t32_ln_kernel<NV_>, dim3((unsigned)T), dim3(256), 0, s, (const float *)z, (const float *)g, (const float *)bias, \
+                                          (float *)y, stats, (int)N, eps)
+    if (N % 4 != 0 || N > 16384 || !ob_aligned(z, 16) || !ob_aligned(g, 16) || !ob_aligned(y, 16) || (bias && !ob_aligned(bias, 16)))
+        hipLaunchKernelGGL((ob_train_ln_fwd_kernel<float>), dim3((unsigned)T), dim3(256), 0, s, (const float *)z, (const float *)g, (const float *)bias,
+                           (float *)y, stats, (int)N, eps);
+    else if (N <= 1024) OB_T32_LN(1);
+    else if (N <= 4096) OB_T32_LN(4);
+    else if (N <= 8192) OB_T32_LN(8);
+    else if (N <= 12288) OB_T32_LN(12);
+    else OB_T32_LN(16);
+#undef OB_T32_LN
+}
+
+static int64_t ob_t32_portion(int64_t T, int64_t K) { return ob_t16_portion(T, OB_T32_PARTS * K); }
+
+static int ob_t32_forward(const void *x, const void *w, const void *h, const void *g, const void *bias, void *y, void *z, float *stats, char *ws,
+                          int64_t T, int64_t K, int64_t N, float eps, hipStream_t s)
+{
+    char *sg = ws, *a = ws + ob_t16_bytes(N, K);
+    ob_t32_tiles(true, w, nullptr, sg, N, K, s);
+    const int kt = (int)(ob_t16_up32(K) / 32);
+    const int64_t Tp = ob_t32_portion(T, K);
+    for (int64_t t0 = 0; t0 < T; t0 += Tp) {
+        const int64_t n = std::min(Tp, T - t0);
+        ob_t32_tiles(false, (const float *)x + t0 * K, h, a, n, K, s);
+        ObT32Mm m = {sg, a, (int)((N + 15) / 16), (int)((n + 15) / 16), kt, kt, {kt, kt, kt}, {}, {2 * ob_t16_bytes(n, K), ob_t16_bytes(n, K), 0},
+                     (float *)z + t0 * N, (int)n, (int)N};
+        m.vec4 = N % 4 == 0 && ob_aligned(z, 16);
+        ob_t32_mm<OB_T16_Z, false, false>(m, s);
+        if (const int rc = ob_launch_status("train_forward(product)")) return rc;
+    }
+    ob_t32_layernorm(z, g, bias, y, stats, T, N, eps, s);
+    return ob_launch_status("train_forward(layernorm)");
+}
+
+// (the sign matrix and, once the input gradient is formed, the parts of x h in one place)
+static size_t ob_t32_operand_bytes(int64_t T, int64_t K, int64_t N) { return std::max(OB_T32_PARTS * ob_t16_bytes(T, K), ob_t16_bytes(N, K)); }
+
+static int ob_t32_backward(const void *gy, const void *x, const void *w, const void *h, const void *g, const void *z, const float *stats, void *gx, void *gw,
+                           void *gh, void *gg, void *gbias, char *ws, int64_t T, int64_t K, int64_t N, hipStream_t s)
+{
+    char *sg = ws, *a = ws, *gz = ws + ob_t32_operand_bytes(T, K, N);
+    const size_t gzb = ob_t16_bytes(T, N);
+    float *part = (float *)(gz + OB_T32_PARTS * gzb), *rowc = (float *)((char *)part + ob_t16_part_bytes(T, K, N));
+    const int kt = (int)(ob_t16_up32(K) / 32), nt = (int)(ob_t16_up32(N) / 32), tt = (int)(ob_t16_up32(T) / 32), slices = ob_t16_slices(T);
+    ObT32Gz q = {(const float *)gy, (const float *)z, (const float *)g, stats, rowc, part, gz, gzb, (int)T, (int)N, 2 * tt, nt, (2 * tt + slices - 1) / slices};
+    int rc;
+    hipLaunchKernelGGL(ob_t32_rowc_kernel, dim3((unsigned)T), dim3(256), 0, s, q);
+    hipLaunchKernelGGL(ob_t32_gz_kernel, dim3((unsigned)((nt + 3) / 4), (unsigned)slices), dim3(256), 0, s, q);
+    hipLaunchKernelGGL(ob_t32_cols_kernel<2>, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, s, (const float *)part, (float *)gg, (float *)gbias, (int)N, slices);
+    ob_t32_tiles(true, w, nullptr, sg, N, K, s);
+    if ((rc = ob_launch_status("train_backward(layernorm)"))) return rc;
+    // gx [T, K] = (gz S) h;  gh = sum_t (gz S) x
+    ObT32Mm m = {sg, gz, (int)((K + 15) / 16), (int)((T + 15) / 16), kt, nt, {nt, nt, nt}, {}, {2 * gzb, gzb, 0}, (float *)gx, (int)T, (int)K,
+                 (const float *)h, (const float *)x, part};
+    m.vec4 = K % 4 == 0 && ob_aligned(gx, 16) && ob_aligned(x, 16);
+    ob_t32_mm<OB_T16_GX, true, false>(m, s);
+    hipLaunchKernelGGL(ob_t32_cols_kernel<1>, dim3((unsigned)((K + 255) / 256)), dim3(256), 0, s, (const float *)part, (float *)gh, (float *)nullptr, (int)K,
+                       2 * (int)((T + 127) / 128));
+    if ((rc = ob_launch_status("train_backward(grad input)"))) return rc;
+    // gW [N, K] = (gz^T a) (1.001 - tanh(W)^2): a's parts lie lowest first, gz's highest, so that a walk through both meets the pairs of one magnitude
+    ObT32Turn tn = {(const float *)x, (const float *)h, a, (int)T, (int)K, tt, kt};
+    hipLaunchKernelGGL(ob_t32_turn_kernel, dim3((unsigned)(((int64_t)tt * ((kt + 3) / 4) + 3) / 4)), dim3(256), 0, s, tn);
+    ObT32Mm v = {a, gz, (int)((K + 15) / 16), (int)((N + 15) / 16), OB_T32_PARTS * tt, nt, {3 * tt, 2 * tt, tt}, {0, (size_t)tt * 1024, (size_t)tt * 2048}, {},
+                 (float *)gw, (int)N, (int)K, (const float *)w};
+    v.vec4 = K % 4 == 0 && ob_aligned(gw, 16) && ob_aligned(w, 16);
+    ob_t32_mm<OB_T16_GW, false, true>(v, s);
+    return ob_launch_status("train_backward(grad weight)");
+}
+
 // Workspace of the forward pass: a smaller or absent one takes the kernels that transform operands on their way into LDS, and so do small products, where two
-// launches beat four (64 -> 64 up to 2048 rows 10.7 us against 16.3; 128 -> 128, 64 rows 12.9 / 16.1; 256 -> 128 18.0 / 16.4; 64 -> 128, 8192 rows 20.4 / 18.5)
+// launches beat four (float16: 64 -> 64 up to 2048 rows 10.7 us against 16.3; 128 -> 128, 64 rows 12.9 / 16.1; 256 -> 128 18.0 / 16.4; 64 -> 128, 8192 rows 20.4 / 18.5;
+// float32, below 64 M products: 64 rows 512 -> 512 in a trace 30 us / 25, but a call's host time has two launches more, 200 rows 31 / 26; 64 rows 1024 -> 1000, the
+// first that takes it, 65 / 35)
 extern "C" size_t onebit_train_forward_workspace_bytes(int64_t T, int64_t K, int64_t N, int dtype)
 {
-    if (T <= 0 || K <= 0 || N <= 0 || dtype != ONEBIT_F16) return 0;
+    if (T <= 0 || K <= 0 || N <= 0 || (dtype != ONEBIT_F16 && dtype != ONEBIT_F32)) return 0;
     if (K < 512 && (N < 128 || (K < 256 && T < 100000000 / (K * N)))) return 0;
+    if (dtype == ONEBIT_F32) return T * K < 64000000 / N ? 0 : OB_T32_PARTS * ob_t16_bytes(ob_t32_portion(T, K), K) + ob_t16_bytes(N, K);
     return ob_t16_bytes(ob_t16_portion(T, K), K) + ob_t16_bytes(N, K);
 }
 
 extern "C" size_t onebit_train_workspace_bytes(int64_t T, int64_t K, int64_t N, int dtype)
 {
     if (T <= 0 || K <= 0 || N <= 0) return 0;
-    if (dtype != ONEBIT_F32) return std::max(ob_t16_bytes(T, K), ob_t16_bytes(N, K)) + ob_t16_bytes(T, N) + ob_t16_part_bytes(T, K, N) + ob_train_align((size_t)T * 8);
-    const size_t sz = 4;
-    return ob_train_align((size_t)T * N * sz) + ob_train_align((size_t)T * K * sz) + ob_train_align((size_t)T * 2 * sizeof(float)) +
-           ob_train_align((size_t)OB_TC_SLICES * (2 * (size_t)N > (size_t)K ? 2 * (size_t)N : (size_t)K) * sizeof(float));     // column-sum partials
+    const size_t rest = ob_t16_part_bytes(T, K, N) + ob_train_align((size_t)T * 8);
+    if (dtype == ONEBIT_F32) return ob_t32_operand_bytes(T, K, N) + OB_T32_PARTS * ob_t16_bytes(T, N) + rest;
+    return std::max(ob_t16_bytes(T, K), ob_t16_bytes(N, K)) + ob_t16_bytes(T, N) + rest;
 }
 
 static int ob_train_check(const char *what, int64_t T, int64_t K, int64_t N, int dtype)
@@ -178,7 +272,7 @@ static int ob_train_forward_t(const void *x, const void *w, const void *h, const
         ob_set_max_lds_once(ob_tgemm128_f16_kernel, attr_set, OB_TG2_LDS);
         hipLaunchKernelGGL(ob_tgemm128_f16_kernel, dim3((unsigned)((N + OB_TG2_B - 1) / OB_TG2_B), (unsigned)((T + OB_TG2_B - 1) / OB_TG2_B)), dim3(OB_TG_THREADS),
                            OB_TG2_LDS, s, a);
-    } else ob_launch_tgemm<true, true, OB_TX_SCALE_R, OB_TX_SIGN, OB_TE_PLAIN>(a, s);
+    } else hipLaunchKernelGGL(ob_tgemm_kernel, dim3((unsigned)((N + OB_TG_BN - 1) / OB_TG_BN), (unsigned)((T + OB_TG_BM - 1) / OB_TG_BM)), dim3(OB_TG_THREADS), 0, s, a);
     int rc = ob_launch_status("train_forward(gemm)");
     if (rc) return rc;
     hipLaunchKernelGGL((ob_train_ln_fwd_kernel<TI>), dim3((unsigned)T), dim3(256), 0, s, (const TI *)z, (const TI *)g, (const TI *)bias,
@@ -198,7 +292,7 @@ extern "C" int onebit_train_forward_ws(const void *x, const void *w_latent, cons
     hipStream_t s = (hipStream_t)stream;
     const size_t need = onebit_train_forward_workspace_bytes(T, K, N, dtype);
     if (need && workspace && ob_aligned(workspace, 16) && workspace_bytes >= need)
-        return ob_t16_forward(x, w_latent, h, g, bias_or_null, y, z_save, ln_stats, (char *)workspace, T, K, N, ln_eps, s);
+        return (dtype == ONEBIT_F16 ? ob_t16_forward : ob_t32_forward)(x, w_latent, h, g, bias_or_null, y, z_save, ln_stats, (char *)workspace, T, K, N, ln_eps, s);
     return dtype == ONEBIT_F16 ? ob_train_forward_t<_Float16>(x, w_latent, h, g, bias_or_null, y, z_save, ln_stats, T, K, N, ln_eps, s)
                                : ob_train_forward_t<float>(x, w_latent, h, g, bias_or_null, y, z_save, ln_stats, T, K, N, ln_eps, s);
 }
@@ -208,46 +302,6 @@ extern "C" int onebit_train_forward(const void *x, const void *w_latent, const v
                                     float ln_eps, void *stream)
 {
     return onebit_train_forward_ws(x, w_latent, h, g, bias_or_null, y, z_save, ln_stats, nullptr, 0, T, K, N, dtype, ln_eps, stream);
-}
-
-static int ob_train_backward_f32(const void *gy, const void *x, const void *w, const void *h, const void *g, const void *z,
-                                 const float *stats, void *gx, void *gw, void *gh, void *gg, void *gbias, char *ws,
-                                 int64_t T, int64_t K, int64_t N, hipStream_t s)
-{
-    float *gz = (float *)ws;
-    float *ga = (float *)(ws + ob_train_align((size_t)T * N * sizeof(float)));
-    float *rowc = (float *)(ws + ob_train_align((size_t)T * N * sizeof(float)) + ob_train_align((size_t)T * K * sizeof(float)));
-    float *part = (float *)((char *)rowc + ob_train_align((size_t)T * 2 * sizeof(float)));     // [OB_TC_SLICES][2 N | K] column-sum partials
-    int rc;
-    // 1. through the LayerNorm and * g: gz [T, N]; column sums gg, gbias
-    hipLaunchKernelGGL(ob_train_ln_bwd_kernel, dim3((unsigned)T), dim3(256), 0, s, (const float *)gy, (const float *)z, (const float *)g, stats, gz, rowc, (int)N);
-    if ((rc = ob_launch_status("train_backward(layernorm)"))) return rc;
-    hipLaunchKernelGGL(ob_train_cols_ln_kernel, dim3((unsigned)((N + 63) / 64), OB_TC_SLICES), dim3(256), 0, s, (const float *)gy, (const float *)z, (const float *)g, stats,
-                       (const float *)rowc, part, (int)T, (int)N);
-    hipLaunchKernelGGL(ob_train_cols_finish_kernel<2>, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, s, (const float *)part, (float *)gg, (float *)gbias, (int)N);
-    if ((rc = ob_launch_status("train_backward(gg)"))) return rc;
-    // 2. ga [T, K] = gz . sign(W);  gx = ga * h;  gh = sum_t ga * x
-    {
-        ObTGemmArgs a = {};
-        a.A = gz; a.lda = N;                 // A(t, n) = gz[t, n]            (n contiguous)
-        a.B = w; a.ldb = K;                  // B(k, n) = sign(W[n, k])        (k = output index, contiguous)
-        a.C = ga; a.C2 = gx; a.vc = h; a.ldc = K; a.M = (int)T; a.N = (int)K; a.R = (int)N;
-        ob_launch_tgemm<true, false, OB_TX_NONE, OB_TX_SIGN, OB_TE_GX>(a, s);
-        if ((rc = ob_launch_status("train_backward(grad input)"))) return rc;
-        hipLaunchKernelGGL(ob_train_cols_gh_kernel, dim3((unsigned)((K + 63) / 64), OB_TC_SLICES), dim3(256), 0, s, (const float *)ga, (const float *)x, part, (int)T, (int)K);
-        hipLaunchKernelGGL(ob_train_cols_finish_kernel<1>, dim3((unsigned)((K + 255) / 256)), dim3(256), 0, s, (const float *)part, (float *)gh, (float *)nullptr, (int)K);
-        if ((rc = ob_launch_status("train_backward(gh)"))) return rc;
-    }
-    // 3. gW [N, K] = (gz^T . (x * h)) * (1.001 - tanh(W)^2)
-    {
-        ObTGemmArgs a = {};
-        a.A = gz; a.lda = N;                 // A(n, t) = gz[t, n]            (n = output index, contiguous)
-        a.B = x; a.ldb = K; a.vb = h;        // B(k, t) = x[t, k] * h[k]      (k = output index, contiguous)
-        a.C = gw; a.vc = w; a.ldc = K; a.M = (int)N; a.N = (int)K; a.R = (int)T;
-        ob_launch_tgemm<false, false, OB_TX_NONE, OB_TX_SCALE_I, OB_TE_STE>(a, s);
-        if ((rc = ob_launch_status("train_backward(grad weight)"))) return rc;
-    }
-    return 0;
 }
 
 extern "C" int onebit_train_backward(const void *gy, const void *x, const void *w_latent, const void *h, const void *g,
@@ -264,6 +318,6 @@ extern "C" int onebit_train_backward(const void *gy, const void *x, const void *
         return ob_fail(ONEBIT_E_WSPACE, "train_backward: needs %zu bytes of 16-byte aligned workspace", onebit_train_workspace_bytes(T, K, N, dtype));
     hipStream_t s = (hipStream_t)stream;
     return dtype == ONEBIT_F16 ? ob_t16_backward(gy, x, w_latent, h, g, z_save, ln_stats, gx, gw, gh, gg, gbias_or_null, (char *)workspace, T, K, N, s)
-                               : ob_train_backward_f32(gy, x, w_latent, h, g, z_save, ln_stats, gx, gw, gh, gg, gbias_or_null, (char *)workspace, T, K, N, s);
+                               : ob_t32_backward(gy, x, w_latent, h, g, z_save, ln_stats, gx, gw, gh, gg, gbias_or_null, (char *)workspace, T, K, N, s);
 }
 

@@ -5,7 +5,7 @@ constructor, parameter names (``weight`` latent full precision ``[out, in]``, ``
 optional ``bias``) and state-dict keys, so a training checkpoint of the reference loads unchanged and
 ``checkpoint.convert_train_state_dict`` turns it into the packed inference layout.  Forward and backward run
 hand-written HIP kernels through the C ABI (``onebit_train_forward_ws`` / ``onebit_train_backward``,
-``csrc/ob_train.h``, float16 ``csrc/ob_train16.h``): the backward pass applies the reference's straight-through estimator
+``csrc/ob_train.h``, float16 ``csrc/ob_train16.h``, float32 ``csrc/ob_train32.h``): the backward pass applies the reference's straight-through estimator
 ``grad * (1.001 - tanh(w)^2)`` (``SignSTEFunc.backward``, ``:21-23``) in the weight-gradient GEMM's epilogue.
 There is no CPU fallback: CPU tensors raise.  (The torch-ops restatement used to check this lives in
 ``oracle/train_ref.py``, test infrastructure.)

@@ -1,0 +1,97 @@
+"""The float32 train-mode layer on bf16 matrix products (csrc/ob_train32.h) against the same sums in 64 bits: edges of tiles, rows and columns that are no multiples
+of anything, every form of the products, the smallest shapes."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _case(T, K, N, seed, gscale=1.0):
+    from onebit_amd.train import BitLinear
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    m = BitLinear(K, N, bias=True, device=DEV, dtype=torch.float32)
+    r = lambda *s: torch.randn(s, generator=g, device=DEV)
+    with torch.no_grad():
+        m.weight.copy_(0.02 * r(N, K))
+        m.weight[0, :3] = 0.0
+        m.weight_scale.copy_(0.1 * r(N)), m.input_factor.copy_(0.1 * r(K)), m.bias.copy_(r(N))
+    x = r(T, K)
+    x[:, ::512] *= 8
+    return m, x.requires_grad_(True), gscale * r(T, N)
+
+
+def _exact(m, x, gy):
+    w, g, h, x, gy = (t.detach().double() for t in (m.weight, m.weight_scale, m.input_factor, x, gy))
+    s, a = torch.sign(w), x * h
+    z = a @ s.T
+    u = z * g
+    c = u - u.mean(-1, keepdim=True)
+    r = 1 / (c.square().mean(-1, keepdim=True) + 1e-5).sqrt()
+    y = c * r
+    gu = r * (gy - gy.mean(-1, keepdim=True) - y * (gy * y).mean(-1, keepdim=True))
+    gz = gu * g
+    ga = gz @ s
+    return y + m.bias.detach().double(), ga * h, (gz.T @ a) * (1.001 - torch.tanh(w) ** 2), (gu * z).sum(0), (ga * x).sum(0), gy.sum(0)
+
+
+# Norms of the differences: a sum of n float32 terms is off by 2^-24 sqrt(n) / 4 of the terms' norm and less (32 at a time are added for one rounding), n is 13824
+# at most here, and a handful of element-wise roundings precede and follow it; a gradient's terms partly cancel (the LayerNorm takes the mean out), a factor of 4.
+def _check(got, want, n):
+    for name, a, b in zip(("y", "x", "weight", "weight_scale", "input_factor", "bias"), got, want):
+        off = float((a.detach().double() - b).norm() / b.norm().clamp_min(1e-300))
+        assert off <= 2.0 ** -22 * (4 + n ** 0.5 / 4), (name, off)
+
+
+@pytest.mark.parametrize("T,K,N", [(5, 24, 8), (33, 1000, 1000), (64, 1024, 1000), (97, 1027, 1030), (257, 1376, 4100), (300, 2080, 516),      # few tiles
+                                   (129, 13824, 128), (1100, 4096, 2050), (2100, 2049, 3070)])                                              # 128 x 256, 256 x 256 tiles, odd widths
+def test_layer_and_gradients_against_64_bits(T, K, N):
+    m, x, gy = _case(T, K, N, T + K)
+    y = m(x)
+    got = (y, *torch.autograd.grad(y, [x, m.weight, m.weight_scale, m.input_factor, m.bias], gy))
+    _check(got, _exact(m, x, gy), max(T, K, N))
+    y = m(x)
+    again = (y, *torch.autograd.grad(y, [x, m.weight, m.weight_scale, m.input_factor, m.bias], gy))
+    assert all(torch.equal(a, b) for a, b in zip(got, again))
+
+
+def test_gradients_of_any_magnitude():
+    """The parts are exact from 2^-110 on: gradients of 1e-20 and 1e20 are as close as those of 1."""
+    for scale in (1e-20, 1e20):
+        m, x, gy = _case(130, 1024, 1000, 7, scale)
+        y = m(x)
+        _check((y, *torch.autograd.grad(y, [x, m.weight, m.weight_scale, m.input_factor, m.bias], gy)), _exact(m, x, gy), 1024)
+
+
+def test_forward_without_workspace_and_special_values(monkeypatch):
+    """Without memory the forward takes the kernel that needs none; an infinite activation makes its row NaN and no other; NaN weights have no sign."""
+    T, K, N = 200, 1024, 1000
+    m, x, _ = _case(T, K, N, 9)
+    full, empty = m(x.detach()).detach(), torch.empty
+
+    def none_left(*a, dtype=None, **k):
+        if dtype == torch.uint8:
+            raise torch.OutOfMemoryError("full")
+        return empty(*a, dtype=dtype, **k)
+    with monkeypatch.context() as p:
+        p.setattr(torch, "empty", none_left)
+        # (z of the float32 instruction: K / 4 roundings)
+        assert float((m(x.detach()).detach() - full).norm() / full.norm()) <= 2.0 ** -22 * (4 + K ** 0.5)
+    xs = x.detach().clone()
+    xs[17, 5] = float("inf")
+    with torch.no_grad():
+        m.weight[3, 7] = float("nan")
+    y = m(xs).detach()
+    assert torch.isnan(y[17]).all() and torch.isfinite(y[:17]).all() and torch.isfinite(y[18:]).all()
+    with torch.no_grad():
+        m.weight[3, 7] = 0.0
+    assert torch.equal(m(x.detach())[:17], y[:17])
+
+
+def test_workspaces_are_bounded():
+    from onebit_amd import _lib
+    lib, f32 = _lib.load(), _lib.ONEBIT_F32
+    fw, bw = lib.onebit_train_forward_workspace_bytes, lib.onebit_train_workspace_bytes
+    assert fw(60, 1024, 1000, f32) == 0 and fw(64, 1024, 1000, f32) > 0
+    assert fw(400000, 4096, 1000, f32) <= 2 ** 29 + 2 * 1024 * 4096 and fw(4096, 4096, 4096, f32) == (6 + 2) * 4096 * 4096
+    assert bw(4096, 4096, 11008, f32) < 1.05 * 6 * 4096 * (4096 + 11008)

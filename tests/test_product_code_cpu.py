@@ -1,5 +1,5 @@
 """The compiled code of the matrix products whose loops count on instructions that hipcc does not know or may leave out (csrc/ob_mm.h): every
-``ob_dense_wr / mm`` and ``ob_t16_wr / mm`` kernel of the built objects, disassembled.
+``ob_dense_wr / mm``, ``ob_t16_wr / mm`` and ``ob_t32_wr / mm`` kernel of the built objects, disassembled.
 
 - ``ob_wr_loop``'s waits in front of its barriers count the loads of later steps.  hipcc drops a load whose result is never used, and a count that includes it lets the
   barrier pass before a tile has landed.  Along every path through the kernel the waits in front of barriers alone, without the others that hipcc happens to
@@ -17,7 +17,7 @@ import pytest
 from onebit_amd import build as B
 
 LIBS = {"onebit_hybrid.hip": (B.LIB_HYBRID, B.SOURCES_HYBRID), "onebit_train.hip": (B.LIB, B.SOURCES)}
-KERNEL = re.compile(r"ob_(dense|t16)_(wr|mm)_kernel")
+KERNEL = re.compile(r"ob_(dense|t16|t32)_(wr|mm)_kernel")
 
 
 def _objdump():
