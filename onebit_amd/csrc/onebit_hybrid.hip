@@ -72,7 +72,8 @@ static bool lds_ok(const void *f, int bytes)
 // ------------------------------------------------------------------------------------------------------ dense products --
 #define OB_SKINNY_T 64
 #define OB_DEEP_KT 61            // k tiles of a split from which every wave has 16 (the last one 13)
-#define OB_ZROWS 2048           // fp32 rows the partial-sum buffer holds at least: splits * T <= max(OB_ZROWS, T)
+#define OB_ZROWS 2048           // fp32 rows of partial sums that gemm_splits fills at most: splits * T <= max(OB_ZROWS, T)
+#define OB_ZROWS_ALL 8192       // ... that the buffer holds at least, and dense_plan fills
 
 // K splits of an output product: enough workgroups to fill the chip, each with a worthwhile share of k tiles
 static int gemm_splits(int n_tiles, int nkt, int T)
@@ -109,6 +110,43 @@ template <typename F> static int wr_rows(int64_t narrow, int most, F tiles_of)
 // fp32 sums are written while the next tile's products run or not at all; what else a product's output becomes takes a CU's only workgroup 5 us a tile (8
 // prompts' layers of 2048 columns, 9728-19776 columns written: 128 rows 5873 us, 192 6180)
 template <int EPI> constexpr int wr_most() { return EPI == OB_EPI_PART ? 16 : 8; }
+// The tile of a bf16 product (mt as above) and its K splits.  gemm_splits and wr_rows, unless an estimate says that others take 8 % less: F us a launch, and per k tile
+// a + b t / 256 us while t <= 256 workgroups are in flight, A + B (t / 256 - 1) up to 512 (mt > 8: whole rounds of A, one workgroup a CU), c more for each k tile behind
+// the 48th, which weights from HBM no longer keep up with, and 0.38 us a MB of fp32 sums written and read back.
+// Fitted to 9500 products, weights from HBM (70-7000 rows, 1024-19200 k columns, 256-4096 columns, every mt, 1-8 splits; 6-14 % rms): over all shapes 6.7 % faster
+// than the rules alone, between 700 and 3000 rows 1.1-2: 1200 x 9728 x 2048 85 -> 53 us (one split of 128 x 128 tiles, now four of 256 x 160), 2400 x 7680 x 2048 90 ->
+// 67, 850 x 19200 x 4096 171 -> 120, 1200 x 2048 x 256 18.8 -> 8.1.  Below 500 rows gemm_splits' number of splits stands: the estimate does not tell 10 us from 11.  (F of mt > 0: 3 us
+// more than where one kernel repeats; in a model its longer code comes from memory each time, 178 x 768 x 2048 10.3 us with 128 x 128 tiles, 12.7 with 64-row ones.)
+struct DenseCost { int mt; double F, a, b, A, B, c; };
+struct DensePlan { int mt, ns; };
+static double dense_us(const DenseCost &f, int n_tiles, int nkt, int T, int ns)
+{
+    const int64_t kt = cdiv(nkt, ns), n = cdiv(nkt, kt), t = (f.mt ? cdiv(n_tiles, 16) * cdiv(T, 16 * f.mt) : cdiv(n_tiles, 8) * cdiv(T, 128)) * n;
+    const double L = (double)t / cu_count(), per = f.mt > 8 ? 1 : 2, full = (double)(cdiv(t, (int64_t)per * cu_count()) - 1), rem = L - per * full;
+    const double step = rem <= 1 ? f.a + f.b * rem : f.A + f.B * (rem - 1), round = f.mt > 8 ? f.A : f.A + f.B;
+    return f.F + (double)kt * (full * round + step) + (kt > 48 ? (double)(kt - 48) * f.c : 0.0) + 0.38e-6 * 4.0 * 16.0 * (double)n_tiles * (double)T * (double)n;
+}
+// most: rows of a tile in 16s; max_ns: splits (0: ns is given)
+static DensePlan dense_plan(int n_tiles, int nkt, int T, int ns, int most, int max_ns)
+{
+    static const DenseCost forms[] = {{0, 3.9, .222, .05, .43, .05, .011}, {4, 6.9, .177, .12, .44, .08, .115}, {5, 7.4, .21, .095, .51, .095, .115},
+                                      {6, 7.8, .21, .125, .515, .12, .1}, {7, 8.0, .245, .1, .6, .075, .1}, {8, 8.1, .265, .105, .63, .075, .07},
+                                      {10, 8.5, .353, .1, .465, 0, .02}, {12, 9.6, .367, .11, .53, 0, .02}, {14, 10.5, .435, .075, .595, 0, .08},
+                                      {16, 11.3, .47, .07, .67, 0, .1}};
+    const int64_t narrow = cdiv(n_tiles, 8) * cdiv(T, 128) * ns;
+    DensePlan base = {wr_rows(narrow, most, [&](int m) { return cdiv(n_tiles, 16) * cdiv(T, 16 * m) * ns; }), ns}, best = base;
+    if (nkt < 32) return base;                                          // (fewer than were fitted)
+    double base_us = 0, least = 0;
+    for (const DenseCost &f : forms) if (f.mt == base.mt) base_us = least = dense_us(f, n_tiles, nkt, T, ns);
+    for (const DenseCost &f : forms) {
+        if (f.mt > most) break;
+        for (int k = max_ns ? 1 : ns; k <= (max_ns ? max_ns : ns); ++k) {
+            const double us = dense_us(f, n_tiles, nkt, T, k);
+            if (us < least) { best = {f.mt, k}; least = us; }
+        }
+    }
+    return least * 1.08 < base_us ? best : base;
+}
 // the LDS-DMA tiles over `n_tb` blocks of 16 mt rows (wr_rows), of 128 with mt = 0.  Experts' blocks have 128 rows; weights to registers from two rounds of them
 // on (12 prompts of 150 rows, 32 experts: 14041 us for them and 16 tokens each, 14069 always, 14186 never)
 template <typename E, int EPI, int ROWS>
@@ -147,7 +185,7 @@ static int tiles_launch(const typename ObDenseArgsOf<ROWS>::type &a, int64_t n_t
 }
 
 template <typename E, int EPI>
-static int dense_launch(ObDenseArgs a, int n_split, hipStream_t s)
+static int dense_launch(ObDenseArgs a, int n_split, hipStream_t s, int mt = -1)      // mt: dense_plan's
 {
     if (a.T <= 0 || a.n_tiles <= 0) return 0;
     a.kt_split = (int)cdiv(a.nkt, n_split);
@@ -160,8 +198,8 @@ static int dense_launch(ObDenseArgs a, int n_split, hipStream_t s)
         else hipLaunchKernelGGL((ob_dense_skinny_kernel<E, EPI, 4>), grid, dim3(256), 0, s, a);
         return hstatus("dense product");
     }
-    const int64_t narrow = cdiv(a.n_tiles, 8) * cdiv(a.T, 128) * n_split;
-    const int mt = sizeof(E) == 4 ? 0 : wr_rows(narrow, wr_most<EPI>(), [&](int m) { return cdiv(a.n_tiles, 16) * cdiv(a.T, 16 * m) * n_split; });
+    if (sizeof(E) == 4) mt = 0;
+    else if (mt < 0) mt = dense_plan(a.n_tiles, a.nkt, a.T, n_split, wr_most<EPI>(), 0).mt;
     return tiles_launch<E, EPI, OB_ROWS_ALL>(a, cdiv(a.T, mt ? 16 * mt : 128), n_split, mt, "dense product", s);
 }
 
@@ -301,7 +339,7 @@ static int make_plan(const onebit_hmodel_t &m, int64_t rows, int64_t n_out, int 
     P.h = take((size_t)R * m.width_pad * es);
     P.u = take((size_t)R * u * es);
     P.aux = take((size_t)R * aux * 4);
-    P.z = take((size_t)std::max<int64_t>(R, OB_ZROWS) * zc * 4);
+    P.z = take((size_t)std::max<int64_t>(R, OB_ZROWS_ALL) * zc * 4);
     P.hist = take(hist ? (size_t)(m.n_runs + 1) * R * m.width * 4 : 0);
     P.hrm = take(rm ? (size_t)R * m.width_pad * es : 0);
     P.cq = take(cq * es);
@@ -610,8 +648,15 @@ static int part_launch(ObDenseArgs d, float *z, int &n_split, hipStream_t s, int
 {
     d.z = z; d.ldz = 16 * d.n_tiles; d.z_split = (size_t)d.T * d.ldz;
     n_split = std::min(most, gemm_splits(d.n_tiles, d.nkt, d.T));
+    int mt = -1;
+    if (sizeof(E) == 2 && d.T > OB_SKINNY_T) {
+        const DensePlan p = dense_plan(d.n_tiles, d.nkt, d.T, n_split, wr_most<OB_EPI_PART>(),
+                                       d.T < 500 ? 0 : (int)std::min<int64_t>({most, 8, std::max(1, OB_ZROWS_ALL / d.T), std::max(1, d.nkt / 8)}));
+        n_split = p.ns;
+        mt = p.mt;
+    }
     n_split = (int)cdiv(d.nkt, cdiv(d.nkt, n_split));
-    return dense_launch<E, OB_EPI_PART>(d, n_split, s);
+    return dense_launch<E, OB_EPI_PART>(d, n_split, s, mt);
 }
 
 // latent attention up to its heads' outputs, in `act` (the rows of the output product)

@@ -114,6 +114,21 @@ def test_dense_product_tile_heights(T):
         assert float((z.double().sum(0) - a.double() @ w.double().t()).abs().max()) < 2 ** -22 * K + 2 ** -21, (nkt, splits)
 
 
+# tiles by estimate (from 32 k tiles on) where the rounds of workgroups alone choose others, 96 to 256 rows: 128 x 128 tiles of many splits
+@pytest.mark.parametrize("N,T,nkt,splits", [(272, 1450, 96, 8), (528, 1450, 96, 6), (528, 1201, 96, 8), (272, 2401, 96, 8), (1040, 1201, 96, 8), (2064, 701, 96, 8)])
+def test_dense_product_by_estimate(N, T, nkt, splits):
+    test_dense_product_large_tiles(N, T, nkt, splits)
+
+
+# a layer's products whose splits the estimate adds (1201 rows: four and more, of 160 and 192 rows), through the row kernels that add them
+@pytest.mark.parametrize("T", [520, 1201])
+def test_prompt_with_more_splits(T):
+    raw = raw_config([att(heads=4, kv_heads=4, dim=64, vdim=64, scale=0.125, ff=2816)], width=520, vocab=61, max_positions=1300)
+    m, w = build(raw, BF)
+    toks = tokens(T, 61, T)
+    assert err(run(m.step_engine(1, 1300, max_rows=T), 0, 0, toks), R.forward(raw, w, toks)) < TOL[BF]
+
+
 # few rows with eight k tiles in flight per wave (from 61 k tiles a split on), every remainder of a wave's share; the others beside them
 @pytest.mark.parametrize("T", [1, 7, 16, 17])
 @DTYPES
