@@ -72,6 +72,7 @@ struct ObFlashRaggedArgs {
     int nseg;
     int hg;                   // 0: pairs of query blocks; else single blocks, numbered over groups of hg heads (set by ob_fl_number)
     int snake;                // single blocks, all resident at once: the lighter half comes lightest first
+    int levels, per_head;     // nonzero: single blocks numbered by length over all segments, hg = H / 8 heads an XCD: the longest's length in blocks of queries; a head's blocks
     int wg_end[OB_FL_MAXSEG];
     ObFlashSeg seg[OB_FL_MAXSEG];
 };
@@ -116,7 +117,7 @@ struct ObFlSoftmaxBf16 : ObFlSigmoidBf16 {
 #define OB_FL_BN 64
 #define OB_FL_THREADS 256
 
-// Workgroups of a ragged launch on a chip of `cus` CUs: sets wg_end, hg and snake from the segments' row counts; 0 = too many.
+// Workgroups of a ragged launch on a chip of `cus` CUs: sets wg_end (or levels and per_head), hg and snake from the segments' row counts; 0 = too many.
 // Pairs of query blocks are the same work each, but a workgroup is as long as two blocks: where the pairs do not take every slot (two workgroups per
 // CU), some CUs run one (4 waves, the latencies of a block's barriers bare) while others run two, or all run one.  Then the blocks go one by
 // one, heaviest first over the heads that one XCD's share of the launch covers (their keys and values stay in its L2); if all are resident
@@ -127,11 +128,23 @@ struct ObFlSoftmaxBf16 : ObFlSigmoidBf16 {
 //   * else some XCDs get the heavy blocks and others the light ones.  All resident, that is still faster where a pair is a tenth longer than the longest
 //     single block (1.10-1.6x), not where one block far back in its cache is the longest workgroup either way (6 segments x 40 heads: 35 against 45 us)
 //   * not all resident: 3 x 1000 rows x 40 heads 53 against 62 us, half of such launches slower
+// Both leave the segments one after the other: an XCD whose contiguous share holds the long ones is busy long after the others, and pairs of unlike segments
+// are unlike work.  With heads in eighths every XCD gets the same share, H / 8 heads of ALL segments, and the blocks go out longest first over all of them,
+// so that a slot that falls free early takes more of the short ones.  Against the two forms above, 240 random launches (1-20 segments of 1-4096 rows,
+// 8-64 heads of width 64 / 128, with and without past): 0.85x on average, 0.35-0.75x where lengths differ widely (one prompt of 955 rows among 19 short ones
+// 79 -> 31 us; chunks of 512 rows at 4 different depths 243 -> 125 us); softmax-bf16 launches of a prompt batch 101 -> 79 us, sigmoid 124 -> 95 us.
+// Not taken where it cannot help or loses:
+//   * at most one block a CU: the longest block's time either way (1.00-1.09x)
+//   * all segments alike: single blocks grouped as above have the same order already, and blocks or pairs of one length need none (12 x 183 rows x 40 heads
+//     24 -> 26 us)
+//   * many rounds of workgroups: the last one hardly counts, and sweeping all segments of a head at once streams their keys past the L2 (8 x 2853 rows x 64
+//     heads, 12 rounds, 1359 -> 1872 us).  Work over slots, in longest pairs: below 5 where segments differ (4-5: 0.82-0.93x; 5.6: 1.06x), below 2.4
+//     where they are alike (1-2: 0.74-0.97x; 2.6-5: 0.97-1.06x)
 inline int64_t ob_fl_number(ObFlashRaggedArgs &f, int cus)
 {
     const int H = f.a.H;
-    int64_t pairs = 0, single = 0, len1 = 0, len2 = 0;                 // longest single block and pair, in blocks of keys
-    bool equal = true;
+    int64_t pairs = 0, single = 0, work = 0, len1 = 0, len2 = 0;       // longest single block and pair, in blocks of keys
+    bool equal = true, same = true;
     const auto blocks = [&](int i) { return ((int64_t)f.seg[i].n + OB_FL_BM - 1) / OB_FL_BM; };
     for (int i = 0; i < f.nseg; ++i) {
         const int64_t nmb = blocks(i), keys = (int64_t)f.seg[i].past + f.seg[i].n, first = f.seg[i].past + std::min(f.seg[i].n, OB_FL_BM);
@@ -139,6 +152,8 @@ inline int64_t ob_fl_number(ObFlashRaggedArgs &f, int cus)
         single += nmb * H;
         equal = equal && nmb == blocks(0);
         const int64_t top = (keys + OB_FL_BN - 1) / OB_FL_BN;
+        same = equal && same && top == ((int64_t)f.seg[0].past + f.seg[0].n + OB_FL_BN - 1) / OB_FL_BN;
+        work += H * nmb * (top + (first + OB_FL_BN - 1) / OB_FL_BN) / 2;
         len1 = std::max(len1, top);
         len2 = std::max(len2, top + (nmb > 1 ? (first + OB_FL_BN - 1) / OB_FL_BN : 0));
         if (pairs > 0x3fffffffLL) return 0;
@@ -146,6 +161,17 @@ inline int64_t ob_fl_number(ObFlashRaggedArgs &f, int cus)
     const int64_t per_xcd = (int64_t)H * f.nseg / 8;
     const bool whole = equal && (int64_t)H * f.nseg % 8 == 0 && H % per_xcd == 0;
     const bool one = pairs < 2 * cus && (whole || (single <= 2 * cus && 10 * len2 >= 11 * len1));
+    f.levels = f.per_head = 0;
+    if (H % 8 == 0 && single > cus && !(same && (one || blocks(0) <= 2)) && 5 * work < (same ? 12 : 25) * 2 * cus * len2) {
+        for (int i = 0; i < f.nseg; ++i) {
+            f.levels = std::max(f.levels, (int)(((int64_t)f.seg[i].past + f.seg[i].n + OB_FL_BM - 1) / OB_FL_BM));
+            f.per_head += (int)blocks(i);
+        }
+        f.hg = H / 8;
+        const int64_t mine = (int64_t)f.per_head * f.hg;           // of an XCD, with its cus / 8 CUs
+        f.snake = mine > cus / 8 && mine <= cus / 4 ? cus / 8 : 0;
+        return single;
+    }
     f.hg = 0;
     f.snake = one && single <= 2 * cus;
     if (one) for (f.hg = (int)std::min<int64_t>(H, std::max<int64_t>(1, per_xcd)); H % f.hg; --f.hg) ;
@@ -223,21 +249,50 @@ __global__ __launch_bounds__(256, 2) void ob_flash_fwd_kernel(const std::conditi
     int npair, pj, head, b, S, past, nmb;
     int64_t qrow0;                                // first token row of this sequence's queries in q / o
     if constexpr (RAGGED) {
-        // segment of this workgroup: lane l compares with wg_end[l] (one vector load of the kernarg table, one ballot)
-        const int we = lane < AA.nseg ? AA.wg_end[lane] : 0x7fffffff;
-        const int sg = __builtin_popcountll(__builtin_amdgcn_ballot_w64(bid >= we));
-        const int wg0 = sg ? AA.wg_end[sg - 1] : 0;
-        const ObFlashSeg sgd = AA.seg[sg];
-        S = sgd.n; past = sgd.past; b = sgd.slot; qrow0 = sgd.row0;
-        nmb = (S + OB_FL_BM - 1) / OB_FL_BM;
-        npair = (nmb + 1) >> 1;
-        const int loc = bid - wg0;
-        if constexpr (SINGLE) {
-            const int per = nmb * AA.hg, grp = loc / per, r = loc - grp * per;
-            pj = r / AA.hg; head = grp * AA.hg + r - pj * AA.hg;
-            if (AA.snake && pj >= npair) pj = nmb - 1 - (pj - npair);
+        if (SINGLE && AA.levels) {
+            // the r-th longest block of a head: lane l has segment l, whose `cnt` blocks are top, top - 1, .. long (in blocks of queries; all sums exact)
+            int j = orig >> 3;
+            if (AA.snake && j >= AA.snake) j = AA.per_head * AA.hg - 1 - (j - AA.snake);
+            const int r = j / AA.hg;
+            head = xcd * AA.hg + j - r * AA.hg;
+            const ObFlashSeg mine = AA.seg[lane];
+            int sg = 0;
+            pj = r;
+            if (AA.nseg > 1) {
+                const bool has = lane < AA.nseg;
+                const int cnt = has ? (mine.n + OB_FL_BM - 1) / OB_FL_BM : 0, top = has ? (mine.past + mine.n + OB_FL_BM - 1) / OB_FL_BM : 0;
+                const auto longer = [&](int w) { return (int)ob_wave_sum((float)min(max(top - w + 1, 0), cnt)); };      // blocks of length w or more
+                int w = 1, hi = AA.levels + 1;                       // longer(w) > r >= longer(hi)
+                while (hi - w > 1) {
+                    const int mid = (w + hi) >> 1;
+                    if (longer(mid) > r) w = mid; else hi = mid;
+                }
+                uint64_t have = __builtin_amdgcn_ballot_w64(top >= w && top - w < cnt);
+                for (int k = r - longer(w + 1); k > 0; --k) have &= have - 1;
+                sg = __builtin_ctzll(have);
+                pj = __builtin_amdgcn_readlane(top, sg) - w;
+            }
+            S = __builtin_amdgcn_readlane(mine.n, sg); past = __builtin_amdgcn_readlane(mine.past, sg);
+            b = __builtin_amdgcn_readlane(mine.slot, sg); qrow0 = __builtin_amdgcn_readlane(mine.row0, sg);
+            nmb = (S + OB_FL_BM - 1) / OB_FL_BM;
+            npair = (nmb + 1) >> 1;
         } else {
-            pj = loc % npair; head = loc / npair;
+            // segment of this workgroup: lane l compares with wg_end[l] (one vector load of the kernarg table, one ballot)
+            const int we = lane < AA.nseg ? AA.wg_end[lane] : 0x7fffffff;
+            const int sg = __builtin_popcountll(__builtin_amdgcn_ballot_w64(bid >= we));
+            const int wg0 = sg ? AA.wg_end[sg - 1] : 0;
+            const ObFlashSeg sgd = AA.seg[sg];
+            S = sgd.n; past = sgd.past; b = sgd.slot; qrow0 = sgd.row0;
+            nmb = (S + OB_FL_BM - 1) / OB_FL_BM;
+            npair = (nmb + 1) >> 1;
+            const int loc = bid - wg0;
+            if constexpr (SINGLE) {
+                const int per = nmb * AA.hg, grp = loc / per, r = loc - grp * per;
+                pj = r / AA.hg; head = grp * AA.hg + r - pj * AA.hg;
+                if (AA.snake && pj >= npair) pj = nmb - 1 - (pj - npair);
+            } else {
+                pj = loc % npair; head = loc / npair;
+            }
         }
     } else {
         S = A.S; past = A.past; nmb = A.nmb;

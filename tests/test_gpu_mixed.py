@@ -120,6 +120,40 @@ def test_attention_ragged_equals_per_segment_prefill_attention(H, Hkv, D):
                 assert float((o[row0:row0 + n].float() - ref).abs().max()) < 4e-3
 
 
+# Launches whose query blocks go out by length over all segments (more blocks than CUs, heads in eighths): all resident at once and not, one segment in
+# more pairs than slots, ties and lengths that only one segment has, 64 segments of a launch and the next launch's.  The block's arithmetic does not
+# depend on its number: same bits as segment by segment.
+@pytest.mark.parametrize("H,Hkv,D,spec", [
+    (32, 8, 128, [(130, 57), (1, 0), (640, 200), (300, 399), (17, 5)]),
+    (40, 40, 64, [(128, 0), (128, 640), (256, 512), (129, 127), (900, 1), (5, 890)]),
+    (64, 8, 64, [(2305, 0)]),
+    (8, 8, 64, [(1 + 37 * i % 200, 61 * i % 700) for i in range(70)]),
+])
+def test_attention_ragged_longest_blocks_first(H, Hkv, D, spec):
+    L, lib = _lib()
+    dev = torch.device(DEV)
+    g = torch.Generator(device="cpu").manual_seed(H + D)
+    slots, max_len = len(spec), max(n + p for n, p in spec) + 3
+    T = sum(n for n, _ in spec)
+    q = torch.randn(T, H, D, generator=g).half().to(dev)
+    kc = torch.randn(slots, Hkv, max_len, D, generator=g).half().to(dev)
+    vc = torch.randn(slots, Hkv, max_len, D, generator=g).half().to(dev)
+    segs, row = [], 0
+    for i, (n, past) in enumerate(spec):
+        segs.append((row, n, slots - 1 - i, past))
+        row += n
+    o = torch.zeros(T, H, D, dtype=torch.float16, device=dev)
+    L.check(lib.onebit_attention_ragged(q.data_ptr(), kc.data_ptr(), vc.data_ptr(), o.data_ptr(), None,
+                                        ctypes.cast(_segs(segs), ctypes.c_void_p), len(segs), H, Hkv, D, slots, max_len, _sp()), "ragged")
+    for (row0, n, slot, past) in segs:
+        o1 = torch.zeros(1, n, H, D, dtype=torch.float16, device=dev)
+        qs = q[row0:row0 + n].reshape(1, n, H, D).contiguous()
+        L.check(lib.onebit_attention_prefill(qs.data_ptr(), kc[slot:slot + 1].data_ptr(), vc[slot:slot + 1].data_ptr(), o1.data_ptr(),
+                                             None, 1, n, H, Hkv, D, past, max_len, _sp()), "prefill")
+        torch.cuda.synchronize()
+        assert torch.equal(o[row0:row0 + n], o1[0]), (n, slot, past)
+
+
 @pytest.mark.parametrize("H,Hkv,D,chunk", [(4, 4, 64, 64), (8, 2, 128, 128), (40, 40, 128, 256)])
 def test_attention_decode_rows_across_split_boundaries(H, Hkv, D, chunk):
     L, lib = _lib()
