@@ -283,9 +283,9 @@ class BitLinearInf(nn.Module):
             try:
                 ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
             except torch.OutOfMemoryError:
-                if cdt != torch.float32:
+                if cdt != torch.float32 and K % 32:
                     raise
-                ws, ws_bytes = None, 0                         # float32: the general kernel needs none
+                ws, ws_bytes = None, 0                         # the general kernels need none
             rc = lib.onebit_linear_forward(
                 w.data_ptr(), ldw, x.data_ptr(), h.data_ptr(), g.data_ptr(),
                 None if b is None else b.data_ptr(), y.data_ptr(), None,

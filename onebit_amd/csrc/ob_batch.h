@@ -146,9 +146,11 @@ struct ObLnRowsArgs {
     const _Float16 *uin; const float *z[4]; const _Float16 *g, *bias; _Float16 *y;
     int N, skip; float eps;
 };
-template <int NV, bool BIAS, bool ZIN = false>
+// ODD: N % 8 == 4 -- rows start on 8-byte lines, and the last vector of a row is its last four values (the other half takes the shift c0: no part in the sums)
+template <int NV, bool BIAS, bool ZIN = false, bool ODD = false>
 __global__ __launch_bounds__(OB_DEC_THREADS) void ob_ln_rows_kernel(const ObLnRowsArgs A)
 {
+    static_assert(!(ZIN && ODD));
     __shared__ __attribute__((aligned(16))) float red[32];
     const int tid = threadIdx.x, N = A.N;
     const int64_t r0 = (int64_t)blockIdx.x * N;
@@ -174,8 +176,17 @@ __global__ __launch_bounds__(OB_DEC_THREADS) void ob_ln_rows_kernel(const ObLnRo
         const int base = (v * OB_DEC_THREADS + tid) * 8;
         ok[v] = base < N;
         if (ZIN) u[v] = zg8(ok[v] ? base : 0);
+        else if (ODD) {
+            const ob_half4 lo = *reinterpret_cast<const ob_half4 *>(A.uin + r0 + (ok[v] ? base : 0));
+            const ob_half4 hi = *reinterpret_cast<const ob_half4 *>(A.uin + r0 + (base + 8 <= N ? base + 4 : 0));
+            u[v] = (ob_half8){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+            if (base + 4 == N) { const _Float16 c = A.uin[r0]; u[v][4] = u[v][5] = u[v][6] = u[v][7] = c; }
+        }
         else u[v] = *reinterpret_cast<const ob_half8 *>(A.uin + r0 + (ok[v] ? base : 0));
-        if (BIAS) bv[v] = *reinterpret_cast<const ob_half8 *>(A.bias + (ok[v] ? base : 0));
+        if (BIAS && ODD) {
+            const ob_half4 lo = *reinterpret_cast<const ob_half4 *>(A.bias + (ok[v] ? base : 0)), hi = *reinterpret_cast<const ob_half4 *>(A.bias + (base + 8 <= N ? base + 4 : 0));
+            bv[v] = (ob_half8){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        } else if (BIAS) bv[v] = *reinterpret_cast<const ob_half8 *>(A.bias + (ok[v] ? base : 0));
     }
     if (ZIN && A.skip) {                                     // (uniform) the pre-LayerNorm rows themselves
 #pragma unroll
@@ -207,7 +218,10 @@ __global__ __launch_bounds__(OB_DEC_THREADS) void ob_ln_rows_kernel(const ObLnRo
 #pragma unroll
         for (int i = 0; i < 8; ++i) o[i] = ob_ln_apply_h(u[v][i], rstd, nmr);
         if (BIAS) o = o + bv[v];
-        *reinterpret_cast<ob_half8 *>(out + (v * OB_DEC_THREADS + tid) * 8) = o;
+        const int base = (v * OB_DEC_THREADS + tid) * 8;
+        if (ODD && base + 8 > N) *reinterpret_cast<ob_half4 *>(out + base) = (ob_half4){o[0], o[1], o[2], o[3]};
+        else if (ODD) *reinterpret_cast<ob_half8a *>(out + base) = o;
+        else *reinterpret_cast<ob_half8 *>(out + base) = o;
     }
 }
 

@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 typedef _Float16 ob_half8 __attribute__((ext_vector_type(8)));
+typedef ob_half8 ob_half8a __attribute__((aligned(8)));                 // eight halves on an 8-byte line
 typedef _Float16 ob_half4 __attribute__((ext_vector_type(4)));
 typedef _Float16 ob_half2 __attribute__((ext_vector_type(2)));
 typedef float ob_float4 __attribute__((ext_vector_type(4)));

@@ -257,6 +257,31 @@ __global__ __launch_bounds__(256) void ob_scale_rows_kernel(const _Float16 *__re
     *reinterpret_cast<ob_half8 *>(a + i) = xv * hv;                       // fp16(x * h), bitnet.py:113
 }
 
+// The same into a workspace whose rows are `kp` columns apart (a whole number of K-step quads), zeros behind column K, and behind them the packed rows on the same
+// columns (signs beyond K meet zeros).  For K that is no whole number of quads, or packed rows that 16-byte transfers cannot read (K / 8 bytes apart).  One launch:
+// blocks from `xblocks` on copy packed rows, 16 bytes a thread.
+__global__ __launch_bounds__(256) void ob_pad_rows_kernel(const _Float16 *__restrict__ x, int64_t ldx, const _Float16 *__restrict__ h, _Float16 *__restrict__ a, int T,
+                                                          int K, int kp, int xblocks, const uint32_t *__restrict__ W, int64_t ldw_words, uint32_t *__restrict__ wp, int N)
+{
+    if ((int)blockIdx.x < xblocks) {
+        const uint32_t i = blockIdx.x * 256 + threadIdx.x, per = (uint32_t)kp / 8;       // (T * kp * 2 < 4 GB, host-checked)
+        const uint32_t t = i / per, k = (i - t * per) * 8;
+        if (t >= (uint32_t)T) return;
+        ob_half8 v = {};
+        if (k < (uint32_t)K) v = *reinterpret_cast<const ob_half8 *>(x + (int64_t)t * ldx + k) * *reinterpret_cast<const ob_half8 *>(h + k);     // fp16(x * h), bitnet.py:113
+        *reinterpret_cast<ob_half8 *>(a + (int64_t)i * 8) = v;
+        return;
+    }
+    const uint32_t i = (blockIdx.x - xblocks) * 256 + threadIdx.x, per = (uint32_t)kp / 128;
+    const uint32_t n = i / per, w = (i - n * per) * 4, words = (uint32_t)K / 32;         // K % 32 == 0 (host-checked)
+    if (n >= (uint32_t)N) return;
+    const uint32_t *src = W + (int64_t)n * ldw_words;
+    ob_u32x4 v;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = w + j < words ? src[w + j] : 0u;
+    *reinterpret_cast<ob_u32x4 *>(wp + (int64_t)i * 4) = v;
+}
+
 #define OB_G3_BUFS 4
 // A workgroup's tile: WN waves of 64 rows side by side times 4 / WN groups of 16 RT tokens
 __host__ __device__ constexpr int ob_g3_rows(int wn) { return 64 * wn; }
@@ -455,7 +480,9 @@ __device__ __forceinline__ void ob_gemm3_body(
     // of one token -- stored directly that is 8 bytes per lane and 32 contiguous bytes per token row and instruction.
     // Each wave transposes its 64 x 128 tile in its own 18 KB of the (now idle: every read finished before the
     // last barrier) staging memory and writes whole 128-byte row segments, 8 token rows per instruction.
-    if (!PARTIAL && n0 + wn * 64 + 64 <= N && (N & 7) == 0 && (reinterpret_cast<size_t>(u) & 15) == 0) {
+    // (N % 8 == 4: rows 8 bytes off a 16-byte line every other time, which the store allows)
+    if (!PARTIAL && n0 + wn * 64 + 64 <= N && ((N & 7) == 0 || ((N & 3) == 0 && (reinterpret_cast<size_t>(g) & 7) == 0)) &&
+        (reinterpret_cast<size_t>(u) & 15) == 0) {
         constexpr int EP = 144;                                // bytes per token row: 128 + 16 (rows shift by 4 banks)
         char *ep = smem + (size_t)wave * (16 * RT) * EP;
 #pragma unroll
@@ -486,7 +513,7 @@ __device__ __forceinline__ void ob_gemm3_body(
         for (int j = 0; j < 2 * RT; ++j) {
             const int row = j * 8 + (lane >> 3), ch = lane & 7;
             const ob_half8 v = *reinterpret_cast<const ob_half8 *>(ep + row * EP + ch * 16);
-            if (row < trows) *reinterpret_cast<ob_half8 *>(ub + (int64_t)row * N + ch * 8) = v;
+            if (row < trows) *reinterpret_cast<ob_half8a *>(ub + (int64_t)row * N + ch * 8) = v;
             if (tsp) {                                                              // (uniform)
                 float sm = 0.f;
 #pragma unroll

@@ -369,6 +369,14 @@ static bool ob_g3_shape(int64_t T, int64_t K, int64_t N)
     static const int env3 = getenv("OB_GEMM3") ? atoi(getenv("OB_GEMM3")) : 1;
     return env3 && T > 64 && K >= 1024 && K % (4 * OB_G2_K) == 0 && N >= 256 && N % 4 == 0 && T * K * 2 < ((int64_t)1 << 32) && N * (K / 8) < ((int64_t)1 << 32);
 }
+// K that is no whole number of quads of K steps: its next whole number, if the product on rows and signs padded to it (ob_pad_rows_kernel) takes the LDS-DMA GEMM;
+// else 0.  Layer calls, the 128 x 128 kernel -> padded: 4064 -> 1000, 70 rows 49.5 -> 17.8 us, 700 51.4 -> 25.0, 1400 54.2 -> 32.2, 3000 57.8 -> 48.6; 1376 -> 4100,
+// 70 rows 30.6 -> 19.2, 700 35.3 -> 26.5, 16000 326 -> 205 (the epilogue and LayerNorm for N % 8 == 4 among it)
+static int64_t ob_g3_padded(int64_t T, int64_t K, int64_t N)
+{
+    const int64_t kp = (K + 4 * OB_G2_K - 1) / (4 * OB_G2_K) * (4 * OB_G2_K);
+    return K % 32 == 0 && K % (4 * OB_G2_K) != 0 && K >= 1024 && ob_g3_shape(T, kp, N) ? kp : 0;
+}
 static int64_t ob_g3_blocks(int64_t N, int wn) { return (N + ob_g3_rows(wn) - 1) / ob_g3_rows(wn); }
 // go(form as a type): the kernel's instance
 template <typename GO>
@@ -416,6 +424,13 @@ template <bool ZIN>
 static void ob_launch_ln_rows(const ObLnRowsArgs &la, int64_t T, hipStream_t s)
 {
     const int nv = (la.N + OB_DEC_THREADS * 8 - 1) / (OB_DEC_THREADS * 8);
+    if constexpr (!ZIN) if (la.N % 8) {
+#define OB_LN_ROWS(NV_) do { if (la.bias) hipLaunchKernelGGL((ob_ln_rows_kernel<NV_, true, false, true>), dim3((unsigned)T), dim3(OB_DEC_THREADS), 0, s, la); \
+                             else hipLaunchKernelGGL((ob_ln_rows_kernel<NV_, false, false, true>), dim3((unsigned)T), dim3(OB_DEC_THREADS), 0, s, la); } while (0)
+        if (nv == 1) OB_LN_ROWS(1); else if (nv == 2) OB_LN_ROWS(2); else if (nv == 3) OB_LN_ROWS(3); else OB_LN_ROWS(4);
+#undef OB_LN_ROWS
+        return;
+    }
 #define OB_LN_ROWS(NV_) do { if (la.bias) hipLaunchKernelGGL((ob_ln_rows_kernel<NV_, true, ZIN>), dim3((unsigned)T), dim3(OB_DEC_THREADS), 0, s, la); \
                              else hipLaunchKernelGGL((ob_ln_rows_kernel<NV_, false, ZIN>), dim3((unsigned)T), dim3(OB_DEC_THREADS), 0, s, la); } while (0)
     if (nv == 1) OB_LN_ROWS(1); else if (nv == 2) OB_LN_ROWS(2); else if (nv == 3) OB_LN_ROWS(3); else OB_LN_ROWS(4);
@@ -427,6 +442,17 @@ static inline size_t ob_align256(size_t b) { return (b + 255) & ~(size_t)255; }
 static int ob_linear_slices(int64_t T, int64_t K, int64_t N)
 {
     return ob_g3_shape(T, K, N) && N % 8 == 0 && N <= OB_DEC_MAXV * OB_DEC_THREADS * 8 ? ob_g3_plan(&N, 1, K, T, 4).ns : 1;
+}
+
+// The padded rows and packed rows of ob_g3_padded, one behind the other
+static size_t ob_pad_a_bytes(int64_t T, int64_t kp) { return ob_align256((size_t)T * (size_t)kp * 2); }
+static size_t ob_pad_bytes(int64_t T, int64_t kp, int64_t N) { return ob_pad_a_bytes(T, kp) + ob_align256((size_t)N * (size_t)(kp / 8)); }
+static void ob_launch_pad_rows(const void *packed, int64_t ldw_bytes, const void *x, int64_t ldx, const void *h, void *workspace, int64_t T, int64_t K, int64_t kp,
+                               int64_t N, hipStream_t s)
+{
+    const int64_t xb = (T * (kp / 8) + 255) / 256, wb = (N * (kp / 128) + 255) / 256;
+    hipLaunchKernelGGL(ob_pad_rows_kernel, dim3((unsigned)(xb + wb)), dim3(256), 0, s, (const _Float16 *)x, ldx, (const _Float16 *)h, (_Float16 *)workspace, (int)T,
+                       (int)K, (int)kp, (int)xb, (const uint32_t *)packed, ldw_bytes / 4, (uint32_t *)((char *)workspace + ob_pad_a_bytes(T, kp)), (int)N);
 }
 
 static size_t ob_required_workspace(int64_t T, int64_t K, int64_t N, int dtype)
@@ -445,6 +471,10 @@ extern "C" size_t onebit_linear_workspace_bytes(int64_t T, int64_t K, int64_t N,
     if (dtype == ONEBIT_F16 && (ob_g3_shape(T, K, N) || (K % 32 == 0 && ob_gemm3_ok(T, K, N)))) {
         const int ns = ob_linear_slices(T, K, N);
         return ns == 1 ? (size_t)T * (size_t)K * 2 : ob_align256((size_t)T * (size_t)K * 2) + ns * ob_align256((size_t)T * (size_t)N * 4);
+    }
+    if (const int64_t kp = dtype == ONEBIT_F16 ? ob_g3_padded(T, K, N) : 0) {
+        const int ns = ob_linear_slices(T, kp, N);
+        return ob_pad_bytes(T, kp, N) + (ns == 1 ? 0 : ns * ob_align256((size_t)T * (size_t)N * 4));
     }
     // float32: the activations' three bf16 parts and the sums of split K (smaller or absent: ob_simple_kernel)
     if (dtype == ONEBIT_F32 && K > 0 && K % 8 == 0) return ob_f32_workspace(T, K, N);
@@ -485,6 +515,8 @@ extern "C" int onebit_linear_forward(const void *packed, int64_t ldw_bytes, cons
     }
     if (dtype == ONEBIT_F16 && (K == 0 || ob_mfma_ok(packed, ldw_bytes, K, K, dtype))) {
         _Float16 *ubuf = (_Float16 *)(u_or_null ? u_or_null : y);
+        const bool pad = !prescaled && ob_g3_padded(T, K, N) != 0;
+        const int64_t kp = pad ? ob_g3_padded(T, K, N) : K;
         if (K == 0) {
             (void)hipMemsetAsync(ubuf, 0, (size_t)T * N * 2, s);
         } else if (T == 1 && K % 128 == 0 && ldw_bytes % 16 == 0 && ob_aligned(packed, 16) && K <= 16384) {
@@ -513,17 +545,27 @@ extern "C" int onebit_linear_forward(const void *packed, int64_t ldw_bytes, cons
             tile_stats_done = tile_stats != nullptr;
             rc = ob_launch_status("linear_forward(gemm3)");
             if (rc) return rc;
-        } else if ((ob_g3_shape(T, K, N) || ob_gemm3_ok(T, K, N)) && workspace && workspace_bytes >= (size_t)T * (size_t)K * 2 && ob_aligned(workspace, 16) &&
-                   ldw_bytes % 16 == 0 && ob_aligned(packed, 16) && N * ldw_bytes < ((int64_t)1 << 32)) {
+        } else if (workspace && ob_aligned(workspace, 16) &&
+                   (pad ? workspace_bytes >= ob_pad_bytes(T, kp, N)
+                        : (ob_g3_shape(T, K, N) || ob_gemm3_ok(T, K, N)) && workspace_bytes >= (size_t)T * (size_t)K * 2 &&
+                          ldw_bytes % 16 == 0 && ob_aligned(packed, 16) && N * ldw_bytes < ((int64_t)1 << 32))) {
             // pre-scale once (the fp16 rounding of bitnet.py:113), then the LDS-DMA GEMM on the scaled rows, whole or in K slices whose sums ONE row pass adds
             // behind it, with fp16(fp16(.) * g) and the LayerNorm
-            const int64_t nvec = T * K / 8;
-            hipLaunchKernelGGL(ob_scale_rows_kernel, dim3((unsigned)((nvec + 255) / 256)), dim3(256), 0, s, (const _Float16 *)x, K,
-                               (const _Float16 *)h, (_Float16 *)workspace, T, (int)K);
+            const void *W = packed;
+            int64_t ldw = ldw_bytes;
+            if (pad) {
+                ob_launch_pad_rows(packed, ldw_bytes, x, K, h, workspace, T, K, kp, N, s);
+                W = (const char *)workspace + ob_pad_a_bytes(T, kp);
+                ldw = kp / 8;
+            } else {
+                const int64_t nvec = T * K / 8;
+                hipLaunchKernelGGL(ob_scale_rows_kernel, dim3((unsigned)((nvec + 255) / 256)), dim3(256), 0, s, (const _Float16 *)x, K,
+                                   (const _Float16 *)h, (_Float16 *)workspace, T, (int)K);
+            }
             onebit_proj_t pj = {};
-            pj.weight = packed; pj.input_factor = h; pj.weight_scale = g; pj.N = N; pj.K = K; pj.ldw_bytes = ldw_bytes;
-            const int ns = tile_stats || (bias && !ob_aligned(bias, 16)) || ob_linear_slices(T, K, N) == 1 ? 0 : ob_gemm3_ksplit_n(pj, T);
-            const size_t a_bytes = ob_align256((size_t)T * (size_t)K * 2), z_bytes = ob_align256((size_t)T * (size_t)N * 4);
+            pj.weight = W; pj.input_factor = h; pj.weight_scale = g; pj.N = N; pj.K = kp; pj.ldw_bytes = ldw;
+            const int ns = tile_stats || (bias && !ob_aligned(bias, 16)) || ob_linear_slices(T, kp, N) == 1 ? 0 : ob_gemm3_ksplit_n(pj, T);
+            const size_t a_bytes = pad ? ob_pad_bytes(T, kp, N) : ob_align256((size_t)T * (size_t)K * 2), z_bytes = ob_align256((size_t)T * (size_t)N * 4);
             if (ns > 0 && workspace_bytes >= a_bytes + (size_t)ns * z_bytes) {
                 float *zs[4] = {nullptr, nullptr, nullptr, nullptr};
                 for (int j = 0; j < ns; ++j) zs[j] = (float *)((char *)workspace + a_bytes + (size_t)j * z_bytes);
@@ -544,7 +586,7 @@ extern "C" int onebit_linear_forward(const void *packed, int64_t ldw_bytes, cons
                 }
                 return ob_launch_status("linear_forward(k-sliced)");
             }
-            ob_launch_gemm3<false>((const uint32_t *)packed, ldw_bytes / 4, (const _Float16 *)workspace, K, (const _Float16 *)g, ubuf, tile_stats, T, K, N, s);
+            ob_launch_gemm3<false>((const uint32_t *)W, ldw / 4, (const _Float16 *)workspace, kp, (const _Float16 *)g, ubuf, tile_stats, T, kp, N, s);
             tile_stats_done = tile_stats != nullptr;
             rc = ob_launch_status("linear_forward(gemm3)");
             if (rc) return rc;
@@ -558,7 +600,8 @@ extern "C" int onebit_linear_forward(const void *packed, int64_t ldw_bytes, cons
                                           "(workspace for the pre-scaled rows missing?)");
         if (skip && ubuf == y) return 0;
         static const int ln_v3 = getenv("OB_LN_ROWS") ? atoi(getenv("OB_LN_ROWS")) : 1;           // A/B: 0 = ob_layernorm_rows_kernel
-        if (ln_v3 && !skip && T >= 64 && N % 8 == 0 && N <= OB_DEC_MAXV * OB_DEC_THREADS * 8 && ob_aligned(ubuf, 16) && (!bias || ob_aligned(bias, 16))) {
+        // (N % 8 == 4, whatever the rows: else one value a lane and load in three passes; a call of 18 rows 1376 -> 4100 17.2 -> 13.6 us)
+        if (ln_v3 && !skip && ((T >= 64 && N % 8 == 0) || N % 8 == 4) && N <= OB_DEC_MAXV * OB_DEC_THREADS * 8 && ob_aligned(ubuf, 16) && (!bias || ob_aligned(bias, 16))) {
             ObLnRowsArgs la = {};
             la.uin = (const _Float16 *)ubuf; la.bias = (const _Float16 *)bias; la.y = (_Float16 *)y; la.N = (int)N; la.eps = ln_eps;
             ob_launch_ln_rows<false>(la, T, s);
@@ -621,6 +664,10 @@ extern "C" int onebit_matmul_partial_ws(const void *packed, int64_t ldw_bytes, c
         hipLaunchKernelGGL(ob_scale_rows_kernel, dim3((unsigned)((nvec + 255) / 256)), dim3(256), 0, s, (const _Float16 *)x, ldx,
                            (const _Float16 *)h, a, T, (int)K);
         ob_launch_gemm3<true>((const uint32_t *)packed, ldw_bytes / 4, (const _Float16 *)a, K, nullptr, nullptr, zp, T, K, N, s);
+    } else if (const int64_t kp = ob_mfma_ok(packed, ldw_bytes, ldx, K, dtype) ? ob_g3_padded(T, K, N) : 0;
+               kp && workspace && workspace_bytes >= ob_pad_bytes(T, kp, N) && ob_aligned(workspace, 16)) {
+        ob_launch_pad_rows(packed, ldw_bytes, x, ldx, h, workspace, T, K, kp, N, s);
+        ob_launch_gemm3<true>((const uint32_t *)((char *)workspace + ob_pad_a_bytes(T, kp)), kp / 32, (const _Float16 *)workspace, kp, nullptr, nullptr, zp, T, kp, N, s);
     } else if (ob_mfma_ok(packed, ldw_bytes, ldx, K, dtype))
         ob_launch_mm16<true>(packed, ldw_bytes, x, ldx, h, nullptr, nullptr, zp, T, K, N, s);
     else if (dtype == ONEBIT_F16)
