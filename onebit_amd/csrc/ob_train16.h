@@ -108,7 +108,7 @@ __global__ __launch_bounds__(256) void ob_t16_turn_kernel(const ObT16Turn A)
 }
 
 // C[t][n] = sum_r a(t, r) w(n, r).  TRW / TRA: the operand's tiles are reduced over their rows (nw / na count its 16-element groups either way).
-enum { OB_T16_Z = 0, OB_T16_GX = 1, OB_T16_GW = 2 };
+enum { OB_T16_Z = 0, OB_T16_GX = 1, OB_T16_GW = 2, OB_T16_PART = 3 };      // PART: a slice of the steps, its float32 sums to zp
 struct ObT16Mm {
     const char *w, *a;
     int nw, na, wld, ald, nk;      // groups of 16 outputs, tiles per band, steps of 32
@@ -116,7 +116,33 @@ struct ObT16Mm {
     const _Float16 *vec;           // OB_T16_GX: h;  OB_T16_GW: latent W, laid out as C
     const _Float16 *x; float *part;      // OB_T16_GX: [rows][cols]; sums of ga x over half a block's rows, [2 token blocks][cols]
     int vec4;                      // rows of C, vec and x in 8-byte pieces
+    float *zp; size_t zld; int ns; // OB_T16_PART: slice blockIdx.y of ns, its sums from zp + zld * slice on
 };
+// this workgroup's steps [k0, k0 + nk) of A's
+template <int EPI> __device__ __forceinline__ int ob_t16_slice(int nk, int ns, int &k0)
+{
+    if (EPI != OB_T16_PART) { k0 = 0; return nk; }
+    k0 = (int)((int64_t)nk * blockIdx.y / ns);
+    return (int)((int64_t)nk * (blockIdx.y + 1) / ns) - k0;
+}
+template <int MN, int MT, typename ACC>
+__device__ __forceinline__ void ob_t16_part(float *zp, int rows, int cols, int n0, int t0, int lane, ACC acc)
+{
+    const int lr = lane & 15, lg = lane >> 4;
+#pragma unroll
+    for (int i = 0; i < MN; ++i)
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+            const int n = n0 + i * 16 + 4 * lg, t = t0 + j * 16 + lr;
+            if (t >= rows || n >= cols) continue;
+            float *o = zp + (size_t)t * cols + n;
+            if ((cols & 3) == 0) *reinterpret_cast<ob_float4 *>(o) = acc(i, j);
+            else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) if (n + e < cols) o[e] = acc(i, j)[e];
+            }
+        }
+}
 
 // 1.001 - tanh(w)^2 with the tensor ops' roundings (SignSTEFunc.backward, bitnet.py:22-23; ob_train.h); tanh = 1 - 2 / (1 + e^2|w|) from the exp2
 // and reciprocal instructions: 2e-7 absolute before its rounding to 11 bits, and it enters as 1.001 - t^2
@@ -133,6 +159,7 @@ __device__ __forceinline__ float ob_t16_ste(float w)
 template <int EPI, int MN, int MT, typename ACC>
 __device__ __forceinline__ void ob_t16_epilogue(const ObT16Mm &A, int n0, int t0, int half, int lane, ACC acc)
 {
+    if constexpr (EPI == OB_T16_PART) { ob_t16_part<MN, MT>(A.zp + blockIdx.y * A.zld, A.rows, A.cols, n0, t0, lane, acc); return; }
     constexpr int IB = MT >= 16 ? 1 : 16 / MT < MN ? 16 / MT : MN;     // column tiles of a batch
     const int lr = lane & 15, lg = lane >> 4;
     const _Float16 *q = EPI == OB_T16_GX ? A.x : A.vec;
@@ -212,6 +239,8 @@ __global__ __launch_bounds__(256, 2) void ob_t16_mm_kernel(const ObT16Mm A)
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wn = wave & 1, wt = wave >> 1, lr = lane & 15, lg = lane >> 4;
     int nb, tb;
     if (!ob_tile_of(blockIdx.x, (A.nw + NB - 1) / NB, (A.na + TB - 1) / TB, nb, tb)) return;      // (uniform)
+    int k0;
+    const int nk = ob_t16_slice<EPI>(A.nk, A.ns, k0);
     const char *src[PER];
     size_t step[PER];
 #pragma unroll
@@ -222,10 +251,11 @@ __global__ __launch_bounds__(256, 2) void ob_t16_mm_kernel(const ObT16Mm A)
         const char *m = w ? A.w : A.a;
         if (tr) { src[d] = m + ((size_t)(o & 1) * ld + min(b0 / 2 + (o >> 1), ld - 1)) * 1024; step[d] = (size_t)ld * 2048; }
         else { src[d] = m + (size_t)min(b0 + o, n - 1) * ld * 1024; step[d] = 1024; }
+        src[d] += (size_t)k0 * step[d];
     }
     const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) char *)smem;
     const auto dma = [&](int d, int k, int buf) {
-        ob_dma_1k(src[d] + (size_t)min(k, A.nk - 1) * step[d], lane * 16, lds0 + (uint32_t)(buf * TILES + wave * PER + d) * 1024);
+        ob_dma_1k(src[d] + (size_t)min(k, nk - 1) * step[d], lane * 16, lds0 + (uint32_t)(buf * TILES + wave * PER + d) * 1024);
     };
     // operand i of a side whose tiles start at tile t0 of the step's buffer
     const int plain = ob_t16_place(lr, lg);
@@ -235,7 +265,7 @@ __global__ __launch_bounds__(256, 2) void ob_t16_mm_kernel(const ObT16Mm A)
         return ob_t16_turned(base + (i >> 1) * 2048, i & 1, lr, lg);
     };
     ob_float4 acc[MN][MT];
-    ob_mm_loop<false, MN, MT, PER, NST>(acc, A.nk, [&](int buf, int i) { return frag(TRW, buf, 0, wn * MN + i); },
+    ob_mm_loop<false, MN, MT, PER, NST>(acc, nk, [&](int buf, int i) { return frag(TRW, buf, 0, wn * MN + i); },
                                         [&](int buf, int j) { return frag(TRA, buf, NB, wt * MT + j); }, dma);
     ob_t16_epilogue<EPI, MN, MT>(A, (nb * NB + wn * MN) * 16, (tb * TB + wt * MT) * 16, tb * 2 + wt, lane, [&](int i, int j) -> const ob_float4 & { return acc[i][j]; });
 }
@@ -254,6 +284,8 @@ __global__ __launch_bounds__(256, MT > 8 ? 1 : 2) void ob_t16_wr_kernel(const Ob
     int nb, tb;
     if (!ob_tile_of(blockIdx.x, SWAP ? (nl + MT - 1) / MT : (nd + 15) / 16, SWAP ? (nd + 15) / 16 : (nl + MT - 1) / MT, nb, tb)) return;      // (uniform)
     const int d0 = (SWAP ? tb : nb) * 16 + wave * MN, l0 = (SWAP ? nb : tb) * MT;
+    int k0;
+    const int nk = ob_t16_slice<EPI>(A.nk, A.ns, k0);
     const char *src[PER], *nxt[PER], *wb[MN];
     uint32_t ldst[PER];
     const size_t step = TRL ? (size_t)lld * 2048 : 1024;
@@ -261,15 +293,15 @@ __global__ __launch_bounds__(256, MT > 8 ? 1 : 2) void ob_t16_wr_kernel(const Ob
 #pragma unroll
     for (int d = 0; d < PER; ++d) {
         const int o = wave * PER + d;
-        src[d] = lm + (TRL ? (size_t)(o & 1) * lld + min(l0 / 2 + (o >> 1), lld - 1) : (size_t)min(l0 + o, nl - 1) * lld) * 1024;
+        src[d] = lm + (TRL ? (size_t)(o & 1) * lld + min(l0 / 2 + (o >> 1), lld - 1) : (size_t)min(l0 + o, nl - 1) * lld) * 1024 + (size_t)k0 * step;
         nxt[d] = src[d] + (NST - 1) * step;
         ldst[d] = lds0 + (uint32_t)o * 1024;
     }
 #pragma unroll
-    for (int i = 0; i < MN; ++i) wb[i] = dm + (size_t)min(d0 + i, nd - 1) * dld * 1024;
+    for (int i = 0; i < MN; ++i) wb[i] = dm + ((size_t)min(d0 + i, nd - 1) * dld + k0) * 1024;
     const int plain = ob_t16_place(lr, lg);
     ob_float4 acc[MN][MT];
-    ob_wr_loop<false, SWAP, MT, PER, NST>(acc, A.nk, wb, plain,
+    ob_wr_loop<false, SWAP, MT, PER, NST>(acc, nk, wb, plain,
         [&](int buf, int j) -> ob_u32x4 {
             if constexpr (TRL) return ob_t16_turned(smem + (buf * MT + (j & ~1)) * 1024, j & 1, lr, lg);
             else return *reinterpret_cast<const ob_u32x4 *>(smem + (buf * MT + j) * 1024 + plain);
@@ -395,4 +427,89 @@ __global__ __launch_bounds__(256) void ob_t16_cols_kernel(const float *__restric
         for (int s = 0; s < slices; ++s) a += part[((size_t)s * NOUT + j) * C + c];
         o[c] = (_Float16)a;
     }
+}
+
+// The slices' sums put together, in order.  z = fp16(sum), or float32: four values a thread ...
+template <typename T>
+__global__ __launch_bounds__(256) void ob_train_zsum_kernel(const float *__restrict__ zp, size_t zld, int ns, T *__restrict__ z, size_t n, int vec)
+{
+    typedef T T4 __attribute__((ext_vector_type(4)));
+    const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (i + 4 <= n) {
+        ob_float4 a = *reinterpret_cast<const ob_float4 *>(zp + i);
+#pragma unroll 4
+        for (int j = 1; j < ns; ++j) a = a + *reinterpret_cast<const ob_float4 *>(zp + j * zld + i);
+        const T4 o = {(T)a[0], (T)a[1], (T)a[2], (T)a[3]};
+        if (vec) *reinterpret_cast<T4 *>(z + i) = o;
+        else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) z[i + e] = o[e];
+        }
+    } else {
+        for (size_t e = i; e < n; ++e) {
+            float a = zp[e];
+            for (int j = 1; j < ns; ++j) a += zp[j * zld + e];
+            z[e] = (T)a;
+        }
+    }
+}
+// ... and the input gradient's: ga = T(sum), gx = ga h and, over 64 rows, the sums of ga x (the epilogue's rounding points): 64 columns x 64 rows a workgroup, four
+// columns and every 16th row a thread
+template <typename T>
+struct ObTrainGxSum { const float *zp; size_t zld; int ns; const T *h, *x; T *gx; float *part; int rows, cols, vec; };      // vec: x, gx in pieces of four
+template <typename T>
+__global__ __launch_bounds__(256) void ob_train_gxsum_kernel(const ObTrainGxSum<T> A)
+{
+    typedef T T4 __attribute__((ext_vector_type(4)));
+    __shared__ float red[16][64];
+    const int cg = threadIdx.x & 15, rl = threadIdx.x >> 4, n = blockIdx.x * 64 + 4 * cg, left = A.cols - n;
+    T h4[4];
+    float sum[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) h4[e] = e < left ? A.h[n + e] : (T)0.f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int t = blockIdx.y * 64 + r * 16 + rl;
+        if (t >= A.rows || left <= 0) continue;
+        const size_t o = (size_t)t * A.cols + n;
+        float a[4] = {0.f, 0.f, 0.f, 0.f};
+        if ((A.cols & 3) == 0) {
+#pragma unroll 4
+            for (int j = 0; j < A.ns; ++j) {
+                const ob_float4 v = *reinterpret_cast<const ob_float4 *>(A.zp + j * A.zld + o);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) a[e] += v[e];
+            }
+        } else {
+            for (int j = 0; j < A.ns; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) if (e < left) a[e] += A.zp[j * A.zld + o + e];
+        }
+        T4 x4, o4;
+        if (A.vec) x4 = *reinterpret_cast<const T4 *>(A.x + o);
+        else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x4[e] = e < left ? A.x[o + e] : (T)0.f;
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const T c = (T)a[e];
+            if (e < left) sum[e] += (float)(T)(c * x4[e]);
+            o4[e] = c * h4[e];
+        }
+        if (A.vec) *reinterpret_cast<T4 *>(A.gx + o) = o4;
+        else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) if (e < left) A.gx[o + e] = o4[e];
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) red[rl][4 * cg + e] = sum[e];
+    __syncthreads();
+    const int c = threadIdx.x;
+    if (c >= 64 || (int)(blockIdx.x * 64) + c >= A.cols) return;
+    float s = 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s += red[r][c];
+    A.part[(size_t)blockIdx.y * A.cols + blockIdx.x * 64 + c] = s;
 }

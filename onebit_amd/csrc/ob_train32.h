@@ -149,6 +149,7 @@ struct ObT32Mm {
     const float *vec;              // OB_T16_GX: h;  OB_T16_GW: latent W, laid out as C
     const float *x; float *part;   // OB_T16_GX: [rows][cols]; sums of ga x over half a block's rows, [2 token blocks][cols]
     int vec4;                      // rows of C, vec and x in 16-byte pieces
+    float *zp; size_t zld; int ns; // OB_T16_PART: as in ObT16Mm; the parts have as many steps
 };
 
 // 1.001 - tanh(w)^2 (bitnet.py:22-23) as 0.001 + 4 e / (1 + e)^2, e = exp(-2 |w|): nothing cancels, 3e-7 of the value
@@ -162,6 +163,7 @@ __device__ __forceinline__ float ob_t32_ste(float w)
 template <int EPI, int MN, int MT, typename ACC>
 __device__ __forceinline__ void ob_t32_epilogue(const ObT32Mm &A, int n0, int t0, int half, int lane, ACC acc)
 {
+    if constexpr (EPI == OB_T16_PART) { ob_t16_part<MN, MT>(A.zp + blockIdx.y * A.zld, A.rows, A.cols, n0, t0, lane, acc); return; }
     constexpr int JB = MT < 8 ? MT : 8, NB = MN * (MT / JB);           // batches of row tiles of one column tile
     static_assert(MT % JB == 0, "whole batches");
     const int lr = lane & 15, lg = lane >> 4;
@@ -262,10 +264,11 @@ __global__ __launch_bounds__(256, 2) void ob_t32_mm_kernel(const ObT32Mm A)
     };
     ob_float4 acc[MN][MT];
     const auto segment = [&]<bool CONT>(int s) __attribute__((always_inline)) {
-        const int nk = A.nk[s];
+        int k0;
+        const int nk = ob_t16_slice<EPI>(A.nk[s], A.ns, k0);
         const char *at[PER];
 #pragma unroll
-        for (int d = 0; d < PER; ++d) at[d] = src[d] + (isw[d] ? A.wofs[s] : A.aofs[s]);
+        for (int d = 0; d < PER; ++d) at[d] = src[d] + (isw[d] ? A.wofs[s] : A.aofs[s]) + (size_t)k0 * step[d];
         ob_mm_loop<true, MN, MT, PER, NST, CONT>(acc, nk, [&](int buf, int i) { return frag(TRW, buf, 0, wn * MN + i); },
             [&](int buf, int j) { return frag(TRA, buf, NB, wt * MT + j); },
             [&](int d, int k, int buf) { ob_dma_1k(at[d] + (size_t)min(k, nk - 1) * step[d], lane * 16, lds0 + (uint32_t)(buf * TILES + wave * PER + d) * 1024); });
@@ -305,11 +308,13 @@ __global__ __launch_bounds__(256, MT > 8 ? 1 : 2) void ob_t32_wr_kernel(const Ob
     ob_float4 acc[MN][MT];
     const auto segment = [&]<bool CONT>(int s) __attribute__((always_inline)) {
         const char *src[PER], *nxt[PER], *wb[MN];
+        int k0;
+        const int nk = ob_t16_slice<EPI>(A.nk[s], A.ns, k0);
 #pragma unroll
-        for (int d = 0; d < PER; ++d) { src[d] = lsrc[d] + (SWAP ? A.wofs[s] : A.aofs[s]); nxt[d] = src[d] + (NST - 1) * step; }
+        for (int d = 0; d < PER; ++d) { src[d] = lsrc[d] + (SWAP ? A.wofs[s] : A.aofs[s]) + (size_t)k0 * step; nxt[d] = src[d] + (NST - 1) * step; }
 #pragma unroll
-        for (int i = 0; i < MN; ++i) wb[i] = dsrc[i] + (SWAP ? A.aofs[s] : A.wofs[s]);
-        ob_wr_loop<true, SWAP, MT, PER, NST, CONT>(acc, A.nk[s], wb, plain,
+        for (int i = 0; i < MN; ++i) wb[i] = dsrc[i] + (SWAP ? A.aofs[s] : A.wofs[s]) + (size_t)k0 * 1024;
+        ob_wr_loop<true, SWAP, MT, PER, NST, CONT>(acc, nk, wb, plain,
             [&](int buf, int j) -> ob_u32x4 {
                 if constexpr (TRL) return ob_t16_turned(smem + (buf * MT + (j & ~1)) * 1024, j & 1, lr, lg);
                 else return *reinterpret_cast<const ob_u32x4 *>(smem + (buf * MT + j) * 1024 + plain);

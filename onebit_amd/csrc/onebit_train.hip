@@ -20,6 +20,38 @@ static size_t ob_t16_part_bytes(int64_t T, int64_t K, int64_t N)
     return ob_train_align(a > b ? a : b);
 }
 
+// z [T][N] (gx = false) and the input gradient [T][K] of few rows are few tiles with a long sum: their steps of 32 in ns slices, one workgroup a CU, whose float32 sums
+// a pass adds.  128 x 128 outputs a workgroup, beyond 128 rows (wide) 128 x 256.  By what it gives: a step takes 0.26 us (float32: three products, 0.75), the pass 4.5 us
+// and the sums' way out and back at 5 TB/s.  From 600 launches, whole passes, unsliced -> sliced: forward 64 rows 11008 -> 4096 114 -> 56 us, 300 rows 119 -> 74, 700 rows
+// 4096 -> 4096 56 -> 53; backward 64 rows 4096 -> 11008 220 -> 142, 300 rows 258 -> 194, 700 rows 293 -> 255; float32 64 rows 515 -> 280, 700 rows 770 -> 673.  More
+// workgroups than 256, two a CU: 1-4 % either way.  (256: the chip's CUs, as a constant, so that what a workspace was asked for with holds on every device.)
+struct ObTrainPlan { int ns; bool wide; };
+static ObTrainPlan ob_train_plan(int dtype, bool gx, int64_t T, int64_t C, int64_t R)
+{
+    const int nk = (int)std::min<int64_t>(ob_t16_up32(R) / 32, 1 << 26);
+    ObTrainPlan best = {1, T > 128};
+    const int64_t tiles = !best.wide ? (C + 127) / 128 : gx ? ((T + 255) / 256) * ((C + 127) / 128) : ((T + 127) / 128) * ((C + 255) / 256);
+    double most = 0;
+    for (int ns = 2; ns <= 16 && ns * tiles <= 256 && ns * 8 <= nk; ++ns) {
+        const double gain = (dtype == ONEBIT_F16 ? 0.26 : 0.75) * nk * (1.0 - 1.0 / ns) - 4.5 - 8.0 * ns * (double)T * (double)C / 5e6;
+        if (gain > most) { most = gain; best.ns = ns; }
+    }
+    return best;
+}
+static size_t ob_train_zld(int64_t T, int64_t C) { return ob_train_align((size_t)T * C * 4) / 4; }
+static size_t ob_train_slice_bytes(const ObTrainPlan &p, int64_t T, int64_t C) { return p.ns > 1 ? p.ns * ob_train_zld(T, C) * 4 : 0; }
+template <typename T>
+static void ob_train_zsum(const float *zp, size_t zld, int ns, T *z, size_t n, hipStream_t s)
+{
+    hipLaunchKernelGGL(ob_train_zsum_kernel<T>, dim3((unsigned)((n + 1023) / 1024)), dim3(256), 0, s, zp, zld, ns, z, n, ob_aligned(z, 4 * sizeof(T)));
+}
+template <typename T>
+static void ob_train_gxsum(const float *zp, int ns, const void *h, const void *x, void *gx, float *part, int64_t rows, int64_t cols, hipStream_t s)
+{
+    ObTrainGxSum<T> a = {zp, ob_train_zld(rows, cols), ns, (const T *)h, (const T *)x, (T *)gx, part, (int)rows, (int)cols, cols % 4 == 0 && ob_aligned(x, 4 * sizeof(T)) && ob_aligned(gx, 4 * sizeof(T))};
+    hipLaunchKernelGGL(ob_train_gxsum_kernel<T>, dim3((unsigned)((cols + 63) / 64), (unsigned)(2 * ((rows + 127) / 128))), dim3(256), 0, s, a);
+}
+
 static void ob_t16_tiles(bool sign, const void *p, const void *vec, char *out, int64_t rows, int64_t cols, hipStream_t s)
 {
     ObT16Tiles a = {(const _Float16 *)p, (const _Float16 *)vec, out, (int)rows, (int)cols, (int)(ob_t16_up32(rows) / 16), (int)(ob_t16_up32(cols) / 32)};
@@ -40,17 +72,22 @@ static void ob_t16_turn(const void *p, const void *vec, char *out, int64_t rows,
 // Both operands through the LDS -> now, 4096 and 1024 rows: z 343 -> 316, 95 -> 89 us, input gradient 408 -> 282, 131 -> 130 (few tiles: as before), weight
 // gradient 441 -> 376, 163 -> 130.
 template <int EPI, bool TRW, bool TRA>
-static void ob_t16_mm(const ObT16Mm &a, hipStream_t s)
+static void ob_t16_mm(const ObT16Mm &a, const ObTrainPlan &p, hipStream_t s)
 {
     constexpr bool SWAP = TRW, TRL = TRW || TRA;
     static_assert(!(TRW && TRA), "one operand lies as it is reduced");
     const int64_t cus = ob_cu_count(), narrow = (int64_t)((a.nw + 7) / 8) * ((a.na + 7) / 8), nd = ((SWAP ? a.na : a.nw) + 15) / 16, nl = SWAP ? a.nw : a.na;
-    const auto go = [&](auto kern, int64_t grid, int lds, bool (&attr_set)[OB_MAX_DEVICES]) {
+    const auto go = [&](auto kern, int64_t grid, int lds, bool (&attr_set)[OB_MAX_DEVICES], int ns = 1) {
         ob_set_max_lds_once(kern, attr_set, lds);
-        hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), lds, s, a);
+        hipLaunchKernelGGL(kern, dim3((unsigned)grid, (unsigned)ns), dim3(256), lds, s, a);
     };
-    static bool attr_set[4][OB_MAX_DEVICES] = {};
+    static bool attr_set[6][OB_MAX_DEVICES] = {};
     const int64_t t8 = nd * ((nl + 7) / 8), t16 = nd * ((nl + 15) / 16);
+    if constexpr (EPI != OB_T16_GW) if (p.ns > 1) {
+        if (p.wide) go(ob_t16_wr_kernel<OB_T16_PART, TRL, SWAP, 8>, t8, ob_wr_steps(8) * 8 * 1024, attr_set[4], p.ns);
+        else go(ob_t16_mm_kernel<OB_T16_PART, TRW, TRA>, narrow, 4 * 16 * 1024, attr_set[5], p.ns);
+        return;
+    }
     if (narrow <= cus) go(ob_t16_mm_kernel<EPI, TRW, TRA>, narrow, 4 * 16 * 1024, attr_set[0]);
     else if constexpr (EPI == OB_T16_GW) {
         if (a.nk <= 40) go(ob_t16_wr_kernel<EPI, TRL, SWAP, 4>, nd * ((nl + 3) / 4), ob_wr_steps(4) * 4 * 1024, attr_set[3]);
@@ -92,12 +129,16 @@ static int ob_t16_forward(const void *x, const void *w, const void *h, const voi
     ob_t16_tiles(true, w, nullptr, sg, N, K, s);
     const int kt = (int)(ob_t16_up32(K) / 32);
     const int64_t Tp = ob_t16_portion(T, K);
+    const ObTrainPlan p = ob_train_plan(ONEBIT_F16, false, Tp, N, K);
+    float *zp = (float *)(a + ob_t16_bytes(Tp, K));
     for (int64_t t0 = 0; t0 < T; t0 += Tp) {
         const int64_t n = std::min(Tp, T - t0);
         ob_t16_tiles(false, (const _Float16 *)x + t0 * K, h, a, n, K, s);
         ObT16Mm m = {sg, a, (int)((N + 15) / 16), (int)((n + 15) / 16), kt, kt, kt, (_Float16 *)z + t0 * N, (int)n, (int)N};
         m.vec4 = N % 4 == 0 && ob_aligned(z, 8);
-        ob_t16_mm<OB_T16_Z, false, false>(m, s);
+        m.zp = zp; m.zld = ob_train_zld(n, N); m.ns = p.ns;
+        ob_t16_mm<OB_T16_Z, false, false>(m, p, s);
+        if (p.ns > 1) ob_train_zsum<_Float16>(zp, m.zld, p.ns, (_Float16 *)z + t0 * N, (size_t)n * N, s);
         if (const int rc = ob_launch_status("train_forward(product)")) return rc;
     }
     ob_t16_layernorm(z, g, bias, y, stats, T, N, eps, s);
@@ -121,7 +162,10 @@ static int ob_t16_backward(const void *gy, const void *x, const void *w, const v
     // gx [T, K] = fp16(gz S) h;  gh = sum_t fp16(gz S) x
     ObT16Mm m = {sg, gz, (int)((K + 15) / 16), (int)((T + 15) / 16), kt, nt, nt, (_Float16 *)gx, (int)T, (int)K, (const _Float16 *)h, (const _Float16 *)x, part};
     m.vec4 = K % 4 == 0 && ob_aligned(gx, 8) && ob_aligned(x, 8);
-    ob_t16_mm<OB_T16_GX, true, false>(m, s);
+    const ObTrainPlan p = ob_train_plan(ONEBIT_F16, true, T, K, N);
+    m.zp = (float *)((char *)rowc + ob_train_align((size_t)T * 8)); m.zld = ob_train_zld(T, K); m.ns = p.ns;
+    ob_t16_mm<OB_T16_GX, true, false>(m, p, s);
+    if (p.ns > 1) ob_train_gxsum<_Float16>(m.zp, p.ns, h, x, gx, part, T, K, s);
     hipLaunchKernelGGL(ob_t16_cols_kernel<1>, dim3((unsigned)((K + 255) / 256)), dim3(256), 0, s, (const float *)part, (_Float16 *)gh, (_Float16 *)nullptr, (int)K,
                        2 * (int)((T + 127) / 128));
     if ((rc = ob_launch_status("train_backward(grad input)"))) return rc;
@@ -129,7 +173,7 @@ static int ob_t16_backward(const void *gy, const void *x, const void *w, const v
     ob_t16_turn(x, h, a, T, K, s);
     ObT16Mm v = {a, gz, (int)((K + 15) / 16), (int)((N + 15) / 16), tt, nt, tt, (_Float16 *)gw, (int)N, (int)K, (const _Float16 *)w};
     v.vec4 = K % 4 == 0 && ob_aligned(gw, 8) && ob_aligned(w, 8);
-    ob_t16_mm<OB_T16_GW, false, true>(v, s);
+    ob_t16_mm<OB_T16_GW, false, true>(v, {1, false}, s);
     return ob_launch_status("train_backward(grad weight)");
 }
 
@@ -144,16 +188,21 @@ static void ob_t32_tiles(bool sign, const void *p, const void *vec, char *out, i
 
 // the tiles of ob_t16_mm (which states both sides of each line)
 template <int EPI, bool TRW, bool TRA>
-static void ob_t32_mm(const ObT32Mm &a, hipStream_t s)
+static void ob_t32_mm(const ObT32Mm &a, const ObTrainPlan &p, hipStream_t s)
 {
     constexpr bool SWAP = TRW, TRL = TRW || TRA;
     const int64_t cus = ob_cu_count(), narrow = (int64_t)((a.nw + 7) / 8) * ((a.na + 7) / 8), nd = ((SWAP ? a.na : a.nw) + 15) / 16, nl = SWAP ? a.nw : a.na;
-    const auto go = [&](auto kern, int64_t grid, int lds, bool (&attr_set)[OB_MAX_DEVICES]) {
+    const auto go = [&](auto kern, int64_t grid, int lds, bool (&attr_set)[OB_MAX_DEVICES], int ns = 1) {
         ob_set_max_lds_once(kern, attr_set, lds);
-        hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), lds, s, a);
+        hipLaunchKernelGGL(kern, dim3((unsigned)grid, (unsigned)ns), dim3(256), lds, s, a);
     };
-    static bool attr_set[3][OB_MAX_DEVICES] = {};
+    static bool attr_set[5][OB_MAX_DEVICES] = {};
     const int64_t t8 = nd * ((nl + 7) / 8), t16 = nd * ((nl + 15) / 16);
+    if constexpr (EPI != OB_T16_GW) if (p.ns > 1) {
+        if (p.wide) go(ob_t32_wr_kernel<OB_T16_PART, TRL, SWAP, 8>, t8, ob_wr_steps(8) * 8 * 1024, attr_set[3], p.ns);
+        else go(ob_t32_mm_kernel<OB_T16_PART, TRW, TRA>, narrow, 4 * 16 * 1024, attr_set[4], p.ns);
+        return;
+    }
     if (narrow <= cus) go(ob_t32_mm_kernel<EPI, TRW, TRA>, narrow, 4 * 16 * 1024, attr_set[0]);
     else if (ob_wr_cost(t8, 8, cus) <= ob_wr_cost(t16, 16, cus)) go(ob_t32_wr_kernel<EPI, TRL, SWAP, 8>, t8, ob_wr_steps(8) * 8 * 1024, attr_set[1]);
     else go(ob_t32_wr_kernel<EPI, TRL, SWAP, 16>, t16, ob_wr_steps(16) * 16 * 1024, attr_set[2]);
@@ -183,13 +232,17 @@ static int ob_t32_forward(const void *x, const void *w, const void *h, const voi
     ob_t32_tiles(true, w, nullptr, sg, N, K, s);
     const int kt = (int)(ob_t16_up32(K) / 32);
     const int64_t Tp = ob_t32_portion(T, K);
+    const ObTrainPlan p = ob_train_plan(ONEBIT_F32, false, Tp, N, K);
+    float *zp = (float *)(a + OB_T32_PARTS * ob_t16_bytes(Tp, K));
     for (int64_t t0 = 0; t0 < T; t0 += Tp) {
         const int64_t n = std::min(Tp, T - t0);
         ob_t32_tiles(false, (const float *)x + t0 * K, h, a, n, K, s);
         ObT32Mm m = {sg, a, (int)((N + 15) / 16), (int)((n + 15) / 16), kt, kt, {kt, kt, kt}, {}, {2 * ob_t16_bytes(n, K), ob_t16_bytes(n, K), 0},
                      (float *)z + t0 * N, (int)n, (int)N};
         m.vec4 = N % 4 == 0 && ob_aligned(z, 16);
-        ob_t32_mm<OB_T16_Z, false, false>(m, s);
+        m.zp = zp; m.zld = ob_train_zld(n, N); m.ns = p.ns;
+        ob_t32_mm<OB_T16_Z, false, false>(m, p, s);
+        if (p.ns > 1) ob_train_zsum<float>(zp, m.zld, p.ns, (float *)z + t0 * N, (size_t)n * N, s);
         if (const int rc = ob_launch_status("train_forward(product)")) return rc;
     }
     ob_t32_layernorm(z, g, bias, y, stats, T, N, eps, s);
@@ -217,7 +270,10 @@ static int ob_t32_backward(const void *gy, const void *x, const void *w, const v
     ObT32Mm m = {sg, gz, (int)((K + 15) / 16), (int)((T + 15) / 16), kt, nt, {nt, nt, nt}, {}, {2 * gzb, gzb, 0}, (float *)gx, (int)T, (int)K,
                  (const float *)h, (const float *)x, part};
     m.vec4 = K % 4 == 0 && ob_aligned(gx, 16) && ob_aligned(x, 16);
-    ob_t32_mm<OB_T16_GX, true, false>(m, s);
+    const ObTrainPlan p = ob_train_plan(ONEBIT_F32, true, T, K, N);
+    m.zp = (float *)((char *)rowc + ob_train_align((size_t)T * 8)); m.zld = ob_train_zld(T, K); m.ns = p.ns;
+    ob_t32_mm<OB_T16_GX, true, false>(m, p, s);
+    if (p.ns > 1) ob_train_gxsum<float>(m.zp, p.ns, h, x, gx, part, T, K, s);
     hipLaunchKernelGGL(ob_t32_cols_kernel<1>, dim3((unsigned)((K + 255) / 256)), dim3(256), 0, s, (const float *)part, (float *)gh, (float *)nullptr, (int)K,
                        2 * (int)((T + 127) / 128));
     if ((rc = ob_launch_status("train_backward(grad input)"))) return rc;
@@ -227,7 +283,7 @@ static int ob_t32_backward(const void *gy, const void *x, const void *w, const v
     ObT32Mm v = {a, gz, (int)((K + 15) / 16), (int)((N + 15) / 16), OB_T32_PARTS * tt, nt, {3 * tt, 2 * tt, tt}, {0, (size_t)tt * 1024, (size_t)tt * 2048}, {},
                  (float *)gw, (int)N, (int)K, (const float *)w};
     v.vec4 = K % 4 == 0 && ob_aligned(gw, 16) && ob_aligned(w, 16);
-    ob_t32_mm<OB_T16_GW, false, true>(v, s);
+    ob_t32_mm<OB_T16_GW, false, true>(v, {1, false}, s);
     return ob_launch_status("train_backward(grad weight)");
 }
 
@@ -239,14 +295,16 @@ extern "C" size_t onebit_train_forward_workspace_bytes(int64_t T, int64_t K, int
 {
     if (T <= 0 || K <= 0 || N <= 0 || (dtype != ONEBIT_F16 && dtype != ONEBIT_F32)) return 0;
     if (K < 512 && (N < 128 || (K < 256 && T < 100000000 / (K * N)))) return 0;
-    if (dtype == ONEBIT_F32) return T * K < 64000000 / N ? 0 : OB_T32_PARTS * ob_t16_bytes(ob_t32_portion(T, K), K) + ob_t16_bytes(N, K);
-    return ob_t16_bytes(ob_t16_portion(T, K), K) + ob_t16_bytes(N, K);
+    if (dtype == ONEBIT_F32) return T * K < 64000000 / N ? 0 : OB_T32_PARTS * ob_t16_bytes(ob_t32_portion(T, K), K) + ob_t16_bytes(N, K) +
+                                                                      ob_train_slice_bytes(ob_train_plan(dtype, false, ob_t32_portion(T, K), N, K), ob_t32_portion(T, K), N);
+    const int64_t Tp = ob_t16_portion(T, K);
+    return ob_t16_bytes(Tp, K) + ob_t16_bytes(N, K) + ob_train_slice_bytes(ob_train_plan(dtype, false, Tp, N, K), Tp, N);
 }
 
 extern "C" size_t onebit_train_workspace_bytes(int64_t T, int64_t K, int64_t N, int dtype)
 {
     if (T <= 0 || K <= 0 || N <= 0) return 0;
-    const size_t rest = ob_t16_part_bytes(T, K, N) + ob_train_align((size_t)T * 8);
+    const size_t rest = ob_t16_part_bytes(T, K, N) + ob_train_align((size_t)T * 8) + ob_train_slice_bytes(ob_train_plan(dtype, true, T, K, N), T, K);
     if (dtype == ONEBIT_F32) return ob_t32_operand_bytes(T, K, N) + OB_T32_PARTS * ob_t16_bytes(T, N) + rest;
     return std::max(ob_t16_bytes(T, K), ob_t16_bytes(N, K)) + ob_t16_bytes(T, N) + rest;
 }

@@ -146,3 +146,16 @@ def test_sign_and_straight_through_factor_at_special_weights():
     # one float16 ulp of the factor near 1 (2^-11), the roundings of gz and of the products
     assert ((gw.double() - ref).abs() <= 4e-3 * ref.abs() + 4e-3 * ref.abs().mean() * factor).all()
     assert _off(y, gs[0]) <= 4e-3
+
+
+@pytest.mark.parametrize("T,K,N,shift", [(1, 4096, 256, 0), (64, 4096, 1000, 0), (128, 2081, 4100, 1), (129, 8200, 260, 0), (257, 1030, 2050, 3), (600, 4096, 1030, 0),
+                                         (100, 530, 8216, 0)])
+def test_products_in_slices_of_their_steps(T, K, N, shift):
+    """Few output tiles and a long sum (csrc/onebit_train.hip, ob_train_plan): ragged slices, rows and columns, 128 x 128 and 128 x 256 tiles."""
+    from onebit_amd import _lib
+    up = lambda n: -(-n // 32) * 32
+    lib, f16 = _lib.load(), _lib.ONEBIT_F16
+    sliced = (lib.onebit_train_forward_workspace_bytes(T, K, N, f16) > 2 * up(K) * (up(T) + up(N)),
+              lib.onebit_train_workspace_bytes(T, K, N, f16) > 2 * (max(up(T) * up(K), up(K) * up(N)) + up(T) * up(N)) + 4 * T * K)
+    assert any(sliced)
+    test_rows_and_columns_against_64_bits(T, K, N, shift)

@@ -95,3 +95,9 @@ def test_workspaces_are_bounded():
     assert fw(60, 1024, 1000, f32) == 0 and fw(64, 1024, 1000, f32) > 0
     assert fw(400000, 4096, 1000, f32) <= 2 ** 29 + 2 * 1024 * 4096 and fw(4096, 4096, 4096, f32) == (6 + 2) * 4096 * 4096
     assert bw(4096, 4096, 11008, f32) < 1.05 * 6 * 4096 * (4096 + 11008)
+
+
+@pytest.mark.parametrize("T,K,N", [(64, 4096, 1000), (128, 2081, 4100), (129, 8200, 260), (257, 1030, 2050), (600, 4096, 1030), (100, 530, 8216)])
+def test_products_in_slices_of_their_steps(T, K, N):
+    """Few output tiles and a long sum (csrc/onebit_train.hip, ob_train_plan): every slice walks all pairs of parts."""
+    test_layer_and_gradients_against_64_bits(T, K, N)
