@@ -107,6 +107,14 @@ __global__ __launch_bounds__(256) void ob_t16_turn_kernel(const ObT16Turn A)
     }
 }
 
+// The lane's number, made here: the products' loop has no register left for what only stands behind it
+__device__ __forceinline__ int ob_t16_lane()
+{
+    int l;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+    return l;
+}
+
 // C[t][n] = sum_r a(t, r) w(n, r).  TRW / TRA: the operand's tiles are reduced over their rows (nw / na count its 16-element groups either way).
 enum { OB_T16_Z = 0, OB_T16_GX = 1, OB_T16_GW = 2, OB_T16_PART = 3 };      // PART: a slice of the steps, its float32 sums to zp
 struct ObT16Mm {
@@ -230,6 +238,61 @@ __device__ __forceinline__ void ob_t16_epilogue(const ObT16Mm &A, int n0, int t0
     }
 }
 
+// The same for z and the weight gradient where the rows of C (and W) are in 8-byte pieces: a wave's 64 columns x 16 MT rows go through its 9 KB of LDS, 64 rows at a
+// time, so that a load or store is 8 rows of 128 bytes, 16 a lane, instead of 16 of 32; the next 64 rows of W are requested in front of a store.  For waves of a
+// workgroup together (the LDS is the loop's).  The weight gradient of 64 rows, 4096 -> 11008, is 180 MB: 67 -> 39 us (2.7 -> 4.6 TB/s); whole backward, 64 / 300 / 700
+// rows 142 -> 115, 194 -> 160, 255 -> 219.
+#define OB_T16_ROWS_PITCH 144
+#define OB_T16_ROWS_LDS (4 * 64 * OB_T16_ROWS_PITCH)
+template <int EPI, int MT, typename ACC>
+__device__ __forceinline__ void ob_t16_rows(const ObT16Mm &A, int n0, int t0, int lane, char *lds, ACC acc)
+{
+    static_assert(MT % 4 == 0 && (EPI == OB_T16_Z || EPI == OB_T16_GW));
+    const int lr = lane & 15, lg = lane >> 4, n = n0 + (lane & 7) * 8, left = A.cols - n;        // (left % 4 == 0)
+    const int t1 = t0 + (lane >> 3);
+    ob_half8 p[2][8];
+    const auto fetch = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const int t = t1 + c * 64 + q * 8;
+            const _Float16 *w = A.vec + (size_t)t * A.cols + n;
+            ob_half8 v = (ob_half8)(_Float16)0;
+            if (t < A.rows && left >= 8) v = *reinterpret_cast<const ob_half8a *>(w);
+            else if (t < A.rows && left > 0) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = w[e];
+            }
+            p[c & 1][q] = v;
+        }
+    };
+    if (EPI == OB_T16_GW) fetch(0);
+    asm volatile("s_barrier" ::: "memory");                            // (every wave's reads of the loop's buffers have returned)
+#pragma unroll
+    for (int c = 0; c < MT / 4; ++c) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const ob_float4 &z = acc(i, 4 * c + j);
+                *reinterpret_cast<ob_half4 *>(lds + (j * 16 + lr) * OB_T16_ROWS_PITCH + (i * 16 + 4 * lg) * 2) =
+                    (ob_half4){(_Float16)z[0], (_Float16)z[1], (_Float16)z[2], (_Float16)z[3]};
+            }
+        if (EPI == OB_T16_GW && c + 1 < MT / 4) fetch(c + 1);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const int t = t1 + c * 64 + q * 8;
+            ob_half8 v = *reinterpret_cast<const ob_half8 *>(lds + (q * 8 + (lane >> 3)) * OB_T16_ROWS_PITCH + (lane & 7) * 16);
+            if (EPI == OB_T16_GW) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] = (_Float16)((float)v[e] * ob_t16_ste((float)p[c & 1][q][e]));
+            }
+            _Float16 *o = A.C + (size_t)t * A.cols + n;
+            if (t < A.rows && left >= 8) *reinterpret_cast<ob_half8a *>(o) = v;
+            else if (t < A.rows && left > 0) *reinterpret_cast<ob_half4 *>(o) = (ob_half4){v[0], v[1], v[2], v[3]};
+        }
+    }
+}
+
 // both operands through the LDS (ob_mm_loop), 128 x 128 outputs: few tiles
 template <int EPI, bool TRW, bool TRA>
 __global__ __launch_bounds__(256, 2) void ob_t16_mm_kernel(const ObT16Mm A)
@@ -267,6 +330,10 @@ __global__ __launch_bounds__(256, 2) void ob_t16_mm_kernel(const ObT16Mm A)
     ob_float4 acc[MN][MT];
     ob_mm_loop<false, MN, MT, PER, NST>(acc, nk, [&](int buf, int i) { return frag(TRW, buf, 0, wn * MN + i); },
                                         [&](int buf, int j) { return frag(TRA, buf, NB, wt * MT + j); }, dma);
+    if constexpr (EPI == OB_T16_Z || EPI == OB_T16_GW) if (A.vec4) {
+        ob_t16_rows<EPI, MT>(A, (nb * NB + wn * MN) * 16, (tb * TB + wt * MT) * 16, lane, smem + wave * 64 * OB_T16_ROWS_PITCH, [&](int i, int j) -> const ob_float4 & { return acc[i][j]; });
+        return;
+    }
     ob_t16_epilogue<EPI, MN, MT>(A, (nb * NB + wn * MN) * 16, (tb * TB + wt * MT) * 16, tb * 2 + wt, lane, [&](int i, int j) -> const ob_float4 & { return acc[i][j]; });
 }
 
@@ -308,8 +375,13 @@ __global__ __launch_bounds__(256, MT > 8 ? 1 : 2) void ob_t16_wr_kernel(const Ob
         },
         [&](int d, int k, int buf) { ob_dma_1k(src[d] + (size_t)k * step, lane * 16, ldst[d] + buf * MT * 1024); },
         [&](int d, int, int buf) { ob_dma_1k(nxt[d], lane * 16, ldst[d] + buf * MT * 1024); nxt[d] += step; });
-    if constexpr (SWAP) ob_t16_epilogue<EPI, MT, MN>(A, l0 * 16, d0 * 16, tb * 4 + wave, lane, [&](int i, int j) -> const ob_float4 & { return acc[j][i]; });
-    else ob_t16_epilogue<EPI, MN, MT>(A, d0 * 16, l0 * 16, 0, lane, [&](int i, int j) -> const ob_float4 & { return acc[i][j]; });
+    const int le = ob_t16_lane();
+    if constexpr (!SWAP && (EPI == OB_T16_Z || EPI == OB_T16_GW)) if (A.vec4) {
+        ob_t16_rows<EPI, MT>(A, d0 * 16, l0 * 16, le, smem + wave * 64 * OB_T16_ROWS_PITCH, [&](int i, int j) -> const ob_float4 & { return acc[i][j]; });
+        return;
+    }
+    if constexpr (SWAP) ob_t16_epilogue<EPI, MT, MN>(A, l0 * 16, d0 * 16, tb * 4 + wave, le, [&](int i, int j) -> const ob_float4 & { return acc[j][i]; });
+    else ob_t16_epilogue<EPI, MN, MT>(A, d0 * 16, l0 * 16, 0, le, [&](int i, int j) -> const ob_float4 & { return acc[i][j]; });
 }
 
 // LayerNorm of z g, rows up to 16384 wide in registers (N % 8 == 0, 16-byte aligned): ob_train_ln_fwd_kernel's arithmetic, z read once

@@ -66,9 +66,9 @@ static void ob_t16_turn(const void *p, const void *vec, char *out, int64_t rows,
     hipLaunchKernelGGL(ob_t16_turn_kernel, dim3((unsigned)(((int64_t)a.rt * ((a.ct + 3) / 4) + 3) / 4)), dim3(256), 0, s, a);
 }
 
+static int ob_t16_wr_lds(int mt) { return std::max(ob_wr_steps(mt) * mt * 1024, OB_T16_ROWS_LDS); }
 // One operand straight into registers from more 128 x 128 outputs than CUs on, with 128 or 256 of the other operand's, whichever costs less by its rounds.  The
-// weight gradient's epilogue reads W: with 128, whose second workgroup's products run meanwhile (4096 rows, 4096 -> 11008 376 us, 394 with 256), or with 64
-// where it is most of the work, up to 1280 rows (whole step of that layer, 64 / 128: 512 rows 346 / 368 us, 1024 rows 433 / 450, 1500 rows 569 / 563).
+// weight gradient's epilogue reads W: with 128, whose second workgroup's products run meanwhile.
 // Both operands through the LDS -> now, 4096 and 1024 rows: z 343 -> 316, 95 -> 89 us, input gradient 408 -> 282, 131 -> 130 (few tiles: as before), weight
 // gradient 441 -> 376, 163 -> 130.
 template <int EPI, bool TRW, bool TRA>
@@ -81,20 +81,17 @@ static void ob_t16_mm(const ObT16Mm &a, const ObTrainPlan &p, hipStream_t s)
         ob_set_max_lds_once(kern, attr_set, lds);
         hipLaunchKernelGGL(kern, dim3((unsigned)grid, (unsigned)ns), dim3(256), lds, s, a);
     };
-    static bool attr_set[6][OB_MAX_DEVICES] = {};
+    static bool attr_set[5][OB_MAX_DEVICES] = {};
     const int64_t t8 = nd * ((nl + 7) / 8), t16 = nd * ((nl + 15) / 16);
     if constexpr (EPI != OB_T16_GW) if (p.ns > 1) {
-        if (p.wide) go(ob_t16_wr_kernel<OB_T16_PART, TRL, SWAP, 8>, t8, ob_wr_steps(8) * 8 * 1024, attr_set[4], p.ns);
-        else go(ob_t16_mm_kernel<OB_T16_PART, TRW, TRA>, narrow, 4 * 16 * 1024, attr_set[5], p.ns);
+        if (p.wide) go(ob_t16_wr_kernel<OB_T16_PART, TRL, SWAP, 8>, t8, ob_t16_wr_lds(8), attr_set[3], p.ns);
+        else go(ob_t16_mm_kernel<OB_T16_PART, TRW, TRA>, narrow, 4 * 16 * 1024, attr_set[4], p.ns);
         return;
     }
     if (narrow <= cus) go(ob_t16_mm_kernel<EPI, TRW, TRA>, narrow, 4 * 16 * 1024, attr_set[0]);
-    else if constexpr (EPI == OB_T16_GW) {
-        if (a.nk <= 40) go(ob_t16_wr_kernel<EPI, TRL, SWAP, 4>, nd * ((nl + 3) / 4), ob_wr_steps(4) * 4 * 1024, attr_set[3]);
-        else go(ob_t16_wr_kernel<EPI, TRL, SWAP, 8>, t8, ob_wr_steps(8) * 8 * 1024, attr_set[1]);
-    }
-    else if (ob_wr_cost(t8, 8, cus) <= ob_wr_cost(t16, 16, cus)) go(ob_t16_wr_kernel<EPI, TRL, SWAP, 8>, t8, ob_wr_steps(8) * 8 * 1024, attr_set[1]);
-    else go(ob_t16_wr_kernel<EPI, TRL, SWAP, 16>, t16, ob_wr_steps(16) * 16 * 1024, attr_set[2]);
+    else if constexpr (EPI == OB_T16_GW) go(ob_t16_wr_kernel<EPI, TRL, SWAP, 8>, t8, ob_t16_wr_lds(8), attr_set[1]);
+    else if (ob_wr_cost(t8, 8, cus) <= ob_wr_cost(t16, 16, cus)) go(ob_t16_wr_kernel<EPI, TRL, SWAP, 8>, t8, ob_t16_wr_lds(8), attr_set[1]);
+    else go(ob_t16_wr_kernel<EPI, TRL, SWAP, 16>, t16, ob_t16_wr_lds(16), attr_set[2]);
 }
 
 // rows in registers where their width and alignment allow, else ob_train_ln_fwd_kernel
@@ -186,7 +183,8 @@ static void ob_t32_tiles(bool sign, const void *p, const void *vec, char *out, i
     else hipLaunchKernelGGL(ob_t32_tiles_kernel<OB_T16_SCALE>, dim3(grid), dim3(256), 0, s, a);
 }
 
-// the tiles of ob_t16_mm (which states both sides of each line)
+// the tiles of ob_t16_mm (which states both sides of each line); the weight gradient of up to 1280 rows with 128 of the other operand's, whose second workgroup
+// multiplies while an epilogue reads W (whole backward, 256 / 128: 64 rows 4096 -> 11008 279 / 247 us, 300 428 / 389, 700 690 / 650, 1200 1087 / 1058, 2000 1490 / 1493)
 template <int EPI, bool TRW, bool TRA>
 static void ob_t32_mm(const ObT32Mm &a, const ObTrainPlan &p, hipStream_t s)
 {
@@ -204,7 +202,7 @@ static void ob_t32_mm(const ObT32Mm &a, const ObTrainPlan &p, hipStream_t s)
         return;
     }
     if (narrow <= cus) go(ob_t32_mm_kernel<EPI, TRW, TRA>, narrow, 4 * 16 * 1024, attr_set[0]);
-    else if (ob_wr_cost(t8, 8, cus) <= ob_wr_cost(t16, 16, cus)) go(ob_t32_wr_kernel<EPI, TRL, SWAP, 8>, t8, ob_wr_steps(8) * 8 * 1024, attr_set[1]);
+    else if ((EPI == OB_T16_GW && a.nk[2] <= 40) || ob_wr_cost(t8, 8, cus) <= ob_wr_cost(t16, 16, cus)) go(ob_t32_wr_kernel<EPI, TRL, SWAP, 8>, t8, ob_wr_steps(8) * 8 * 1024, attr_set[1]);
     else go(ob_t32_wr_kernel<EPI, TRL, SWAP, 16>, t16, ob_wr_steps(16) * 16 * 1024, attr_set[2]);
 }
 
