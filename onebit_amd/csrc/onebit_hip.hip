@@ -233,7 +233,7 @@ static void ob_launch_mm16(const void *packed, int64_t ldw_bytes, const void *x,
             ka.p[0] = {(const uint32_t *)packed, (long long)(ldw_bytes / 4), (const _Float16 *)h,              \
                        (const _Float16 *)g, (const _Float16 *)x, (_Float16 *)u, zp, (int)N, (int)K,            \
                        (int)((N + 63) / 64)};                                                                  \
-            ka.p[1] = ka.p[0]; ka.p[2] = ka.p[0];                                                              \
+            ka.p[1] = ka.p[0]; ka.p[2] = ka.p[0]; ka.p[3] = ka.p[0];                                           \
             ka.ldx = ldx; ka.T = (int)T;                                                                       \
             ob_launch_skinny<PARTIAL, RT_>(ka, ka.p[0].tile_end, s);                                           \
         } while (0)
@@ -444,6 +444,33 @@ static int ob_linear_slices(int64_t T, int64_t K, int64_t N)
     return ob_g3_shape(T, K, N) && N % 8 == 0 && N <= OB_DEC_MAXV * OB_DEC_THREADS * 8 ? ob_g3_plan(&N, 1, K, T, 4).ns : 1;
 }
 
+// K slices of onebit_linear_forward's product of 2 .. 64 rows: 64 columns a workgroup are few workgroups where N is small, each with a long way through K.  Whole phases
+// of 512 columns of K, up to one workgroup a CU (256, whatever the device: what a workspace was asked for with holds).  From 14 phases on, above 32 rows (a phase takes
+// 1.6 us instead of 0.7) from 8: fewer cost less than the workspace, 2.5 us of a call.  Layer calls, unsliced -> sliced: 11008 -> 4096, 4 / 18 / 40 rows 21.6 -> 16.1,
+// 25.9 -> 16.3, 36.7 -> 17.9 us, 13824 -> 5120 25.3 -> 15.9, 30.4 -> 17.1, 44.0 -> 21.7, 4096 -> 4096, 40 rows 18.8 -> 15.7 (18 rows 14.6, sliced 16.0).
+static int ob_skinny_slices(int64_t T, int64_t K, int64_t N)
+{
+    const int64_t tiles = (N + 63) / 64, phases = (K + 511) / 512;
+    if (T < 2 || T > 64 || K % 128 != 0 || phases < (T > 32 ? 8 : 14) || N % 8 != 0 || N > OB_DEC_MAXV * OB_DEC_THREADS * 8) return 1;
+    return (int)std::max<int64_t>(1, std::min<int64_t>(4, 256 / tiles));
+}
+static void ob_launch_skinny_slices(const void *packed, int64_t ldw_bytes, const void *x, const void *h, float *const *z, int ns, int64_t T, int64_t K, int64_t N,
+                                    hipStream_t s)
+{
+    const int tiles = (int)((N + 63) / 64), phases = (int)((K + 511) / 512);
+    ObSkinnyArgs ka = {};
+    for (int j = 0; j < 4; ++j) {
+        if (j >= ns) { ka.p[j] = ka.p[j - 1]; continue; }
+        const int64_t k0 = (int64_t)(phases * j / ns) * 512, k1 = std::min<int64_t>(K, (int64_t)(phases * (j + 1) / ns) * 512);
+        ka.p[j] = {(const uint32_t *)packed + k0 / 32, (long long)(ldw_bytes / 4), (const _Float16 *)h + k0, nullptr, (const _Float16 *)x + k0, nullptr, z[j], (int)N,
+                   (int)(k1 - k0), tiles * (j + 1)};
+    }
+    ka.ldx = K; ka.T = (int)T;
+    if (T <= 16) ob_launch_skinny<true, 1>(ka, tiles * ns, s);
+    else if (T <= 32) ob_launch_skinny<true, 2>(ka, tiles * ns, s);
+    else ob_launch_skinny<true, 4>(ka, tiles * ns, s);
+}
+
 // The padded rows and packed rows of ob_g3_padded, one behind the other
 static size_t ob_pad_a_bytes(int64_t T, int64_t kp) { return ob_align256((size_t)T * (size_t)kp * 2); }
 static size_t ob_pad_bytes(int64_t T, int64_t kp, int64_t N) { return ob_pad_a_bytes(T, kp) + ob_align256((size_t)N * (size_t)(kp / 8)); }
@@ -472,6 +499,7 @@ extern "C" size_t onebit_linear_workspace_bytes(int64_t T, int64_t K, int64_t N,
         const int ns = ob_linear_slices(T, K, N);
         return ns == 1 ? (size_t)T * (size_t)K * 2 : ob_align256((size_t)T * (size_t)K * 2) + ns * ob_align256((size_t)T * (size_t)N * 4);
     }
+    if (const int ns = dtype == ONEBIT_F16 ? ob_skinny_slices(T, K, N) : 1; ns > 1) return ns * ob_align256((size_t)T * (size_t)N * 4);
     if (const int64_t kp = dtype == ONEBIT_F16 ? ob_g3_padded(T, K, N) : 0) {
         const int ns = ob_linear_slices(T, kp, N);
         return ob_pad_bytes(T, kp, N) + (ns == 1 ? 0 : ns * ob_align256((size_t)T * (size_t)N * 4));
@@ -515,6 +543,24 @@ extern "C" int onebit_linear_forward(const void *packed, int64_t ldw_bytes, cons
     }
     if (dtype == ONEBIT_F16 && (K == 0 || ob_mfma_ok(packed, ldw_bytes, K, K, dtype))) {
         _Float16 *ubuf = (_Float16 *)(u_or_null ? u_or_null : y);
+        // the row pass behind K slices' sums: added, fp16(fp16(.) * g) and the LayerNorm
+        const auto add_slices = [&](float *const *zs, int ns) {
+            ObLnRowsArgs la = {};
+            for (int j = 0; j < ns; ++j) la.z[j] = zs[j];
+            la.g = (const _Float16 *)g; la.bias = skip ? nullptr : (const _Float16 *)bias; la.N = (int)N; la.eps = ln_eps;
+            if (u_or_null && !skip) {                       // both outputs wanted: u first, then y from it
+                la.y = (_Float16 *)u_or_null; la.skip = 1;
+                ob_launch_ln_rows<true>(la, T, s);
+                ObLnRowsArgs lb = {};
+                lb.uin = (const _Float16 *)u_or_null; lb.bias = (const _Float16 *)bias; lb.y = (_Float16 *)y; lb.N = (int)N; lb.eps = ln_eps;
+                ob_launch_ln_rows<false>(lb, T, s);
+            } else {
+                la.y = (_Float16 *)(skip ? ubuf : y); la.skip = skip;
+                ob_launch_ln_rows<true>(la, T, s);
+                if (skip && ubuf != y) (void)hipMemcpyAsync(y, ubuf, (size_t)T * N * 2, hipMemcpyDeviceToDevice, s);
+            }
+        };
+        const int few = !prescaled && !tile_stats && (!bias || ob_aligned(bias, 16)) && ob_aligned(g, 16) && ob_skinny_ok(packed, ldw_bytes, T, K) ? ob_skinny_slices(T, K, N) : 1;
         const bool pad = !prescaled && ob_g3_padded(T, K, N) != 0;
         const int64_t kp = pad ? ob_g3_padded(T, K, N) : K;
         if (K == 0) {
@@ -545,6 +591,13 @@ extern "C" int onebit_linear_forward(const void *packed, int64_t ldw_bytes, cons
             tile_stats_done = tile_stats != nullptr;
             rc = ob_launch_status("linear_forward(gemm3)");
             if (rc) return rc;
+        } else if (few > 1 && workspace && ob_aligned(workspace, 16) && workspace_bytes >= (size_t)few * ob_align256((size_t)T * (size_t)N * 4)) {
+            float *zs[4] = {nullptr, nullptr, nullptr, nullptr};
+            for (int j = 0; j < few; ++j) zs[j] = (float *)((char *)workspace + (size_t)j * ob_align256((size_t)T * (size_t)N * 4));
+            ob_launch_skinny_slices(packed, ldw_bytes, x, h, zs, few, T, K, N, s);
+            if ((rc = ob_launch_status("linear_forward(skinny slices)"))) return rc;
+            add_slices(zs, few);
+            return ob_launch_status("linear_forward(few rows, k-sliced)");
         } else if (workspace && ob_aligned(workspace, 16) &&
                    (pad ? workspace_bytes >= ob_pad_bytes(T, kp, N)
                         : (ob_g3_shape(T, K, N) || ob_gemm3_ok(T, K, N)) && workspace_bytes >= (size_t)T * (size_t)K * 2 &&
@@ -570,20 +623,7 @@ extern "C" int onebit_linear_forward(const void *packed, int64_t ldw_bytes, cons
                 float *zs[4] = {nullptr, nullptr, nullptr, nullptr};
                 for (int j = 0; j < ns; ++j) zs[j] = (float *)((char *)workspace + a_bytes + (size_t)j * z_bytes);
                 if ((rc = ob_gemm3_ksplit(pj, workspace, zs, ns, T, s))) return rc;
-                ObLnRowsArgs la = {};
-                for (int j = 0; j < ns; ++j) la.z[j] = zs[j];
-                la.g = (const _Float16 *)g; la.bias = skip ? nullptr : (const _Float16 *)bias; la.N = (int)N; la.eps = ln_eps;
-                if (u_or_null && !skip) {                       // both outputs wanted: u first, then y from it
-                    la.y = (_Float16 *)u_or_null; la.skip = 1;
-                    ob_launch_ln_rows<true>(la, T, s);
-                    ObLnRowsArgs lb = {};
-                    lb.uin = (const _Float16 *)u_or_null; lb.bias = (const _Float16 *)bias; lb.y = (_Float16 *)y; lb.N = (int)N; lb.eps = ln_eps;
-                    ob_launch_ln_rows<false>(lb, T, s);
-                } else {
-                    la.y = (_Float16 *)(skip ? ubuf : y); la.skip = skip;
-                    ob_launch_ln_rows<true>(la, T, s);
-                    if (skip && ubuf != y) (void)hipMemcpyAsync(y, ubuf, (size_t)T * N * 2, hipMemcpyDeviceToDevice, s);
-                }
+                add_slices(zs, ns);
                 return ob_launch_status("linear_forward(k-sliced)");
             }
             ob_launch_gemm3<false>((const uint32_t *)W, ldw / 4, (const _Float16 *)workspace, kp, (const _Float16 *)g, ubuf, tile_stats, T, kp, N, s);
