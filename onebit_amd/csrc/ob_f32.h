@@ -285,7 +285,8 @@ struct ObF32Ln {
     const float *z, *zt; long long zt_split; int ld_t, S, n_tail;
     const float *g, *bias; float *y, *u; int N, skip; float eps;
 };
-template <int NV, int THREADS>
+// SPLIT: all columns are split ones (the other form keeps twice as many waves on a CU)
+template <int NV, int THREADS, bool SPLIT>
 __global__ __launch_bounds__(THREADS, 4) void ob_f32_ln_kernel(const ObF32Ln A)
 {
     __shared__ float red[2][THREADS / 64];
@@ -296,9 +297,31 @@ __global__ __launch_bounds__(THREADS, 4) void ob_f32_ln_kernel(const ObF32Ln A)
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
         const int n = (v * THREADS + tid) * 4;
-        u[v] = n < A.n_tail && n < A.N ? *reinterpret_cast<const ob_float4 *>(A.z + row + n) : (ob_float4){0.f, 0.f, 0.f, 0.f};
+        u[v] = !SPLIT && n < A.n_tail && n < A.N ? *reinterpret_cast<const ob_float4 *>(A.z + row + n) : (ob_float4){0.f, 0.f, 0.f, 0.f};
     }
-    if (A.n_tail < A.N) {                                              // (uniform)
+    if constexpr (SPLIT) {
+        // the splits in order, G of them in flight for all of a thread's columns (column by column, as below, the way there is made NV S / 4 times: one row of
+        // 11008 columns, five splits 9.8 -> 6.7 us)
+        constexpr int G = NV >= 4 ? 2 : 4;
+        const float *p = A.zt + t * A.ld_t;
+#pragma unroll 1
+        for (int k = 0; k < A.S; k += G) {
+            ob_float4 e[G][NV];
+#pragma unroll
+            for (int i = 0; i < G; ++i)
+#pragma unroll
+                for (int v = 0; v < NV; ++v) {
+                    const int n = (v * THREADS + tid) * 4;
+                    e[i][v] = *reinterpret_cast<const ob_float4 *>(p + min(k + i, A.S - 1) * A.zt_split + (n < A.N ? n : 0));
+                }
+#pragma unroll
+            for (int i = 0; i < G; ++i)
+#pragma unroll
+                for (int v = 0; v < NV; ++v) if (k + i < A.S) u[v] += e[i][v];
+        }
+#pragma unroll
+        for (int v = 0; v < NV; ++v) if ((v * THREADS + tid) * 4 >= A.N) u[v] = (ob_float4){0.f, 0.f, 0.f, 0.f};
+    } else if (A.n_tail < A.N) {                                       // (uniform)
         const float *p = A.zt + t * A.ld_t - A.n_tail;
 #pragma unroll
         for (int v = 0; v < NV; ++v) {

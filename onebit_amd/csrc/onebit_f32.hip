@@ -89,7 +89,8 @@ static void ob_f32_rows(const ObF32Plan &p, const void *packed, int64_t ldw_byte
         return;
     }
     ObF32Ln l = {y, zt, a.zt_split, p.ld_t, p.S, p.nb_full * 128, g, bias, y, u, (int)N, skip, eps};
-#define OB_F32_LN(NV_, TH_) hipLaunchKernelGGL((ob_f32_ln_kernel<NV_, TH_>), dim3((unsigned)T), dim3(TH_), 0, s, l)
+#define OB_F32_LN(NV_, TH_) do { if (p.nb_full == 0) hipLaunchKernelGGL((ob_f32_ln_kernel<NV_, TH_, true>), dim3((unsigned)T), dim3(TH_), 0, s, l); \
+                                 else hipLaunchKernelGGL((ob_f32_ln_kernel<NV_, TH_, false>), dim3((unsigned)T), dim3(TH_), 0, s, l); } while (0)
     if (N <= 1024) OB_F32_LN(1, 256);
     else if (N <= 2048) OB_F32_LN(1, 512);
     else if (N <= 4096) OB_F32_LN(2, 512);
