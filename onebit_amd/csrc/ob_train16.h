@@ -11,8 +11,8 @@
 // conflicts.  Every product has one operand that lies as it is reduced, and goes straight to registers with it: S for z, gz for ga, and for gS a^T, whose tiles
 // their pass turns.  Loops, tile shapes and numbering: ob_mm.h.
 // What bounds it: the chip's power for the products, memory for the passes.  T = 4096, 4096 -> 11008, forward + backward: 1217 us with both operands through the
-// LDS, 1037 now; in a trace the products 343 -> 316 (z), 408 -> 282 (ga) and 441 -> 376 us (gS) = 1.17, 1.31 and 0.98 PFLOP/s, the passes 205 us at 4-5 TB/s.  Each
-// product alone in a loop, at 1.39 kW of the 1.4 that the chip is given: 251 us at 2.08 GHz, 222 at 2.19 and 338 at 1.61 (gS multiplies full-range values by full-range
+// LDS, 1037 with one of them straight to registers, 972 now that outputs go through the LDS; in a trace the products 343 -> 296 (z), 408 -> 286 (ga) and 441 -> 310 us
+// (gS) = 1.25, 1.29 and 1.19 PFLOP/s, the passes 205 us at 4-5 TB/s.  Each product alone in a loop, at 1.39 kW of the 1.4 that the chip is given: 251 us at 2.08 GHz, 222 at 2.19 and 338 at 1.61 (gS multiplies full-range values by full-range
 // values, the others by signs).
 #pragma once
 #include "ob_mm.h"
@@ -293,6 +293,71 @@ __device__ __forceinline__ void ob_t16_rows(const ObT16Mm &A, int n0, int t0, in
     }
 }
 
+// ... and for the input gradient: a wave's 64 rows x 16 CT columns, 64 columns at a time, x likewise; its sums of ga x over the rows end in the lanes of
+// the first row.  Whole backward with it, 2000 rows 4096 -> 11008 399 -> 378 us, 4096 rows 4096 -> 4096 289 -> 268, 11008 -> 4096 764 -> 710.
+template <int CT, typename ACC>
+__device__ __forceinline__ void ob_t16_gx_rows(const ObT16Mm &A, int n0, int t0, int half, int lane, char *lds, ACC acc)
+{
+    static_assert(CT % 4 == 0);
+    const int lr = lane & 15, lg = lane >> 4, t1 = t0 + (lane >> 3), c8 = (lane & 7) * 8;
+    ob_half8 p[2][8], h[2];
+    const auto fetch = [&](int c) __attribute__((always_inline)) {
+        const int n = n0 + c * 64 + c8, left = A.cols - n;                               // (left % 4 == 0)
+        h[c & 1] = (ob_half8)(_Float16)0;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) if (e < left) h[c & 1][e] = A.vec[n + e];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const int t = t1 + q * 8;
+            const _Float16 *x = A.x + (size_t)t * A.cols + n;
+            ob_half8 v = (ob_half8)(_Float16)0;
+            if (t < A.rows && left >= 8) v = *reinterpret_cast<const ob_half8a *>(x);
+            else if (t < A.rows && left > 0) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = x[e];
+            }
+            p[c & 1][q] = v;
+        }
+    };
+    fetch(0);
+    asm volatile("s_barrier" ::: "memory");                            // (every wave's reads of the loop's buffers have returned)
+#pragma unroll
+    for (int c = 0; c < CT / 4; ++c) {
+        const int n = n0 + c * 64 + c8, left = A.cols - n;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const ob_float4 &z = acc(4 * c + i, j);
+                *reinterpret_cast<ob_half4 *>(lds + (j * 16 + lr) * OB_T16_ROWS_PITCH + (i * 16 + 4 * lg) * 2) =
+                    (ob_half4){(_Float16)z[0], (_Float16)z[1], (_Float16)z[2], (_Float16)z[3]};
+            }
+        if (c + 1 < CT / 4) fetch(c + 1);
+        float sum[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sum[e] = 0.f;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const int t = t1 + q * 8;
+            const ob_half8 v = *reinterpret_cast<const ob_half8 *>(lds + (q * 8 + (lane >> 3)) * OB_T16_ROWS_PITCH + c8 * 2);
+            const ob_half8 vx = v * p[c & 1][q], o = v * h[c & 1];
+            if (t >= A.rows) continue;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) sum[e] += (float)vx[e];
+            _Float16 *d = A.C + (size_t)t * A.cols + n;
+            if (left >= 8) *reinterpret_cast<ob_half8a *>(d) = o;
+            else if (left > 0) *reinterpret_cast<ob_half4 *>(d) = (ob_half4){o[0], o[1], o[2], o[3]};
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            sum[e] += OB_DPP_F(sum[e], 0x128, 0xF);                                      // row_ror:8
+            sum[e] += __shfl_xor(sum[e], 16);
+            sum[e] += __shfl_xor(sum[e], 32);
+            if (lane < 8 && e < left && half < 2 * ((A.rows + 127) >> 7)) A.part[(size_t)half * A.cols + n + e] = sum[e];
+        }
+    }
+}
+
 // both operands through the LDS (ob_mm_loop), 128 x 128 outputs: few tiles
 template <int EPI, bool TRW, bool TRA>
 __global__ __launch_bounds__(256, 2) void ob_t16_mm_kernel(const ObT16Mm A)
@@ -332,6 +397,11 @@ __global__ __launch_bounds__(256, 2) void ob_t16_mm_kernel(const ObT16Mm A)
                                         [&](int buf, int j) { return frag(TRA, buf, NB, wt * MT + j); }, dma);
     if constexpr (EPI == OB_T16_Z || EPI == OB_T16_GW) if (A.vec4) {
         ob_t16_rows<EPI, MT>(A, (nb * NB + wn * MN) * 16, (tb * TB + wt * MT) * 16, lane, smem + wave * 64 * OB_T16_ROWS_PITCH, [&](int i, int j) -> const ob_float4 & { return acc[i][j]; });
+        return;
+    }
+    if constexpr (EPI == OB_T16_GX) if (A.vec4) {
+        ob_t16_gx_rows<MN>(A, (nb * NB + wn * MN) * 16, (tb * TB + wt * MT) * 16, tb * 2 + wt, lane, smem + wave * 64 * OB_T16_ROWS_PITCH,
+                           [&](int i, int j) -> const ob_float4 & { return acc[i][j]; });
         return;
     }
     ob_t16_epilogue<EPI, MN, MT>(A, (nb * NB + wn * MN) * 16, (tb * TB + wt * MT) * 16, tb * 2 + wt, lane, [&](int i, int j) -> const ob_float4 & { return acc[i][j]; });
@@ -378,6 +448,10 @@ __global__ __launch_bounds__(256, MT > 8 ? 1 : 2) void ob_t16_wr_kernel(const Ob
     const int le = ob_t16_lane();
     if constexpr (!SWAP && (EPI == OB_T16_Z || EPI == OB_T16_GW)) if (A.vec4) {
         ob_t16_rows<EPI, MT>(A, d0 * 16, l0 * 16, le, smem + wave * 64 * OB_T16_ROWS_PITCH, [&](int i, int j) -> const ob_float4 & { return acc[i][j]; });
+        return;
+    }
+    if constexpr (SWAP && EPI == OB_T16_GX) if (A.vec4) {
+        ob_t16_gx_rows<MT>(A, l0 * 16, d0 * 16, tb * 4 + wave, le, smem + wave * 64 * OB_T16_ROWS_PITCH, [&](int i, int j) -> const ob_float4 & { return acc[j][i]; });
         return;
     }
     if constexpr (SWAP) ob_t16_epilogue<EPI, MT, MN>(A, l0 * 16, d0 * 16, tb * 4 + wave, le, [&](int i, int j) -> const ob_float4 & { return acc[j][i]; });
