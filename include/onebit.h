@@ -91,6 +91,9 @@ int onebit_unpack_signs(const void *packed, void *out, int dtype, int64_t N, int
  *     F16, large calls: the pre-scaled activations fp16(x*h) of the LDS-DMA GEMM;
  *     F16, a few hundred rows: those and the fp32 sums of K slices (256-byte
  *       aligned; 16 bytes selects the register-staged GEMM);
+ *     F16, K % 256 != 0 (K % 32 == 0, from 65 rows on): those and the packed rows,
+ *       both on the next whole number of 256 columns;
+ *     F16, 2 to 64 rows, a long K and few columns: the fp32 sums of K slices;
  *     F32, T*K*N from 24 million on (36 if K % 256 != 0), N % 4 == 0, g / bias /
  *       u (with K % 256 == 0 the packed rows, too) 16-byte aligned: the
  *       activations' three bf16 parts and the sums of split K for the matrix
