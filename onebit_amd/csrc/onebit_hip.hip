@@ -363,11 +363,15 @@ ObG3Plan ob_g3_plan(const int64_t *N, int np, int64_t K, int64_t T, int max_ns)
     next = (next + 1) % 8;
     return best;
 }
-// From 65 rows on, and 1024 columns of K: fewer are few steps behind a launch's constant, and the 128 x 128 kernel needs no scaled rows
+// From 65 rows on, and 1024 columns of K: fewer are few steps behind a launch's constant, and the 128 x 128 kernel needs no scaled rows.  Of fewer than 256 output
+// columns, whose tiles are one beside another at most, from 2048 of K on, where K slices make up for it.  Layer calls of 65 / 700 / 2000 rows, the
+// 128 x 128 kernel -> slices: 2048 -> 128 28.6 / 29.6 / 30.8 -> 11.6 / 14.7 / 22.5 us, 4096 -> 128 48.6 / 50.2 / 51.4 -> 14.1 / 18.7 / 25.6, 11008 -> 200 118 / 122 /
+// 126 -> 23.9 / 30.5 / 42.8; 6000 rows 2048 -> 128 33.9 -> 39.2, 4096 -> 128 56.1 -> 48.6.
 static bool ob_g3_shape(int64_t T, int64_t K, int64_t N)
 {
     static const int env3 = getenv("OB_GEMM3") ? atoi(getenv("OB_GEMM3")) : 1;
-    return env3 && T > 64 && K >= 1024 && K % (4 * OB_G2_K) == 0 && N >= 256 && N % 4 == 0 && T * K * 2 < ((int64_t)1 << 32) && N * (K / 8) < ((int64_t)1 << 32);
+    return env3 && T > 64 && K % (4 * OB_G2_K) == 0 && N % 4 == 0 && (N >= 256 ? K >= 1024 : N % 8 == 0 && K >= 2048) && T * K * 2 < ((int64_t)1 << 32) &&
+           N * (K / 8) < ((int64_t)1 << 32);
 }
 // K that is no whole number of quads of K steps: its next whole number, if the product on rows and signs padded to it (ob_pad_rows_kernel) takes the LDS-DMA GEMM;
 // else 0.  Layer calls, the 128 x 128 kernel -> padded: 4064 -> 1000, 70 rows 49.5 -> 17.8 us, 700 51.4 -> 25.0, 1400 54.2 -> 32.2, 3000 57.8 -> 48.6; 1376 -> 4100,
@@ -375,7 +379,7 @@ static bool ob_g3_shape(int64_t T, int64_t K, int64_t N)
 static int64_t ob_g3_padded(int64_t T, int64_t K, int64_t N)
 {
     const int64_t kp = (K + 4 * OB_G2_K - 1) / (4 * OB_G2_K) * (4 * OB_G2_K);
-    return K % 32 == 0 && K % (4 * OB_G2_K) != 0 && K >= 1024 && ob_g3_shape(T, kp, N) ? kp : 0;
+    return K % 32 == 0 && K % (4 * OB_G2_K) != 0 && K >= 1024 && N >= 256 && ob_g3_shape(T, kp, N) ? kp : 0;
 }
 static int64_t ob_g3_blocks(int64_t N, int wn) { return (N + ob_g3_rows(wn) - 1) / ob_g3_rows(wn); }
 // go(form as a type): the kernel's instance

@@ -93,6 +93,14 @@ def test_argument_errors_without_gpu():
         _lib.check(1, "x")
 
 
+def test_layers_of_few_columns_ask_for_their_slices():
+    """A float16 layer of fewer than 256 columns with a long K runs in K slices: room for its scaled rows and two slices' sums at least."""
+    lib = _lib.load()
+    for T in (65, 300, 2000):
+        for K, N in ((2048, 128), (4096, 8), (4096, 248), (11008, 200)):
+            assert lib.onebit_linear_workspace_bytes(T, K, N, 0) >= T * K * 2 + 2 * T * N * 4, (T, K, N)
+
+
 def test_round6_entry_points_reject_bad_arguments_without_gpu():
     """ABI 9 (ragged rows, key-block decode attention, grouped projections, the mixed step): argument errors come back before any launch."""
     lib = _lib.load()

@@ -37,6 +37,13 @@ def test_one_projection(T, K, N):
     _check(m, x * m.input_factor, m(x))
 
 
+# fewer than 256 columns: K slices from 2048 of K on, the 128 x 128 kernel below
+@pytest.mark.parametrize("K,N", [(2048, 128), (4096, 8), (4096, 248), (11008, 200), (1792, 128), (4096, 124)])
+@pytest.mark.parametrize("T", [65, 96, 97, 129, 300, 2100])
+def test_one_projection_of_few_columns(T, K, N):
+    test_one_projection(T, K, N)
+
+
 @pytest.mark.parametrize("Ns", [(4096, 4096, 4096), (11008, 11008), (5120, 1028, 260)])
 @pytest.mark.parametrize("T", [192, 577, 673, 897, 1025, 1153, 1540])
 def test_grouped_projections(T, Ns):
