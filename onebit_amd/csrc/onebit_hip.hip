@@ -363,15 +363,19 @@ ObG3Plan ob_g3_plan(const int64_t *N, int np, int64_t K, int64_t T, int max_ns)
     next = (next + 1) % 8;
     return best;
 }
+// whole quads of K steps; 32-bit byte offsets from the base pointers inside the kernel
+static bool ob_g3_fits(int64_t T, int64_t K, int64_t N)
+{
+    static const int env3 = getenv("OB_GEMM3") ? atoi(getenv("OB_GEMM3")) : 1;
+    return env3 && K > 0 && K % (4 * OB_G2_K) == 0 && N > 0 && N % 4 == 0 && T * K * 2 < ((int64_t)1 << 32) && N * (K / 8) < ((int64_t)1 << 32);
+}
 // From 65 rows on, and 1024 columns of K: fewer are few steps behind a launch's constant, and the 128 x 128 kernel needs no scaled rows.  Of fewer than 256 output
 // columns, whose tiles are one beside another at most, from 2048 of K on, where K slices make up for it.  Layer calls of 65 / 700 / 2000 rows, the
 // 128 x 128 kernel -> slices: 2048 -> 128 28.6 / 29.6 / 30.8 -> 11.6 / 14.7 / 22.5 us, 4096 -> 128 48.6 / 50.2 / 51.4 -> 14.1 / 18.7 / 25.6, 11008 -> 200 118 / 122 /
 // 126 -> 23.9 / 30.5 / 42.8; 6000 rows 2048 -> 128 33.9 -> 39.2, 4096 -> 128 56.1 -> 48.6.
 static bool ob_g3_shape(int64_t T, int64_t K, int64_t N)
 {
-    static const int env3 = getenv("OB_GEMM3") ? atoi(getenv("OB_GEMM3")) : 1;
-    return env3 && T > 64 && K % (4 * OB_G2_K) == 0 && N % 4 == 0 && (N >= 256 ? K >= 1024 : N % 8 == 0 && K >= 2048) && T * K * 2 < ((int64_t)1 << 32) &&
-           N * (K / 8) < ((int64_t)1 << 32);
+    return ob_g3_fits(T, K, N) && T > 64 && (N >= 256 ? K >= 1024 : N % 8 == 0 && K >= 2048);
 }
 // K that is no whole number of quads of K steps: its next whole number, if the product on rows and signs padded to it (ob_pad_rows_kernel) takes the LDS-DMA GEMM;
 // else 0.  Layer calls, the 128 x 128 kernel -> padded: 4064 -> 1000, 70 rows 49.5 -> 17.8 us, 700 51.4 -> 25.0, 1400 54.2 -> 32.2, 3000 57.8 -> 48.6; 1376 -> 4100,
@@ -1837,20 +1841,27 @@ int ob_rows_norm(const ObRowsNormCall &c, hipStream_t s)
     return ob_launch_status("rows_norm");
 }
 
+// Every member on its own (ob_g3_shape), or, from 192 rows on, as a group that takes half a round of workgroups with 256 x 128 tiles: narrow members ride along, and
+// the few steps of a small K are one launch's constant instead of three.  Mixed steps of four layers, one launch a projection -> a group, 700 / 2000 rows: width
+// 2048 with one key head of 128 776 / 1145 -> 554 / 934 us, 4096 likewise 1539 / 2734 -> 1152 / 2390, 1300 / 2000 rows: width 512 580 / 617 -> 507 / 552, 768 616 / 663 ->
+// 540 / 480.
 bool ob_gemm3_group_ok(const onebit_proj_t *const *ps, int np, int64_t T)
 {
     static const int env = getenv("OB_GEMM3_GROUPED") ? atoi(getenv("OB_GEMM3_GROUPED")) : 1;       // A/B: 0 = one launch per projection
     if (!env || np < 1 || np > 3) return false;
     const int64_t K = ps[0]->K, ldw = ps[0]->ldw_bytes;
-    int64_t tiles = 0;
+    int64_t tiles = 0, large = 0;
+    bool each = true;
     for (int i = 0; i < np; ++i) {
         const onebit_proj_t &p = *ps[i];
-        if (!p.weight || !p.weight_scale || !ob_g3_shape(T, p.K, p.N) || p.K != K || p.ldw_bytes != ldw || ldw % 16 != 0 || p.N * ldw >= ((int64_t)1 << 32) ||
+        if (!p.weight || !p.weight_scale || !ob_g3_fits(T, p.K, p.N) || p.K != K || p.ldw_bytes != ldw || ldw % 16 != 0 || p.N * ldw >= ((int64_t)1 << 32) ||
             !ob_aligned(p.weight, 16) || !ob_aligned(p.weight_scale, 8))
             return false;
+        each = each && ob_g3_shape(T, p.K, p.N);
         tiles += ob_g3_blocks(p.N, 2) * ((T + 95) / 96);
+        large += ob_g3_blocks(p.N, 4) * ((T + 127) / 128);
     }
-    return tiles <= 0x3fffffff;
+    return (each || (np > 1 && T >= 192 && 2 * large >= ob_cu_count())) && tiles <= 0x3fffffff;
 }
 double ob_gemm3_group_us(const onebit_proj_t *const *ps, int np, int64_t T)
 {

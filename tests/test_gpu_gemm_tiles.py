@@ -44,23 +44,43 @@ def test_one_projection_of_few_columns(T, K, N):
     test_one_projection(T, K, N)
 
 
-@pytest.mark.parametrize("Ns", [(4096, 4096, 4096), (11008, 11008), (5120, 1028, 260)])
-@pytest.mark.parametrize("T", [192, 577, 673, 897, 1025, 1153, 1540])
-def test_grouped_projections(T, Ns):
+def _group(T, K, Ns):
+    """(status, layers, rows, outputs) of one grouped launch; a row more than the outputs have is there to see that it stays."""
     from onebit_amd import _lib
     from onebit_amd.bitnet import _stream_ptr
     from onebit_amd.engine import _Proj, _proj
-    K, lib = 1024, _lib.load()
+    lib = _lib.load()
     g = torch.Generator(device=DEV).manual_seed(T)
     ms = [_layer(K, N, g) for N in Ns]
     xs = [torch.randn(T, K, generator=g, device=DEV).half() for _ in ms]
     us = [torch.full((T + 1, N), 7.0, dtype=torch.float16, device=DEV) for N in Ns]
     arr = (_Proj * len(ms))(*[_proj(m) for m in ms])
     up, ap = ((ctypes.c_void_p * 3)(*[t.data_ptr() for t in ts]) for ts in (us, xs))
-    rc = lib.onebit_linear_group_prescaled(ctypes.cast(arr, ctypes.c_void_p), up, ap, len(ms), T, _stream_ptr(xs[0].device))
-    if rc == -2:
-        pytest.skip("too few tiles for one launch")
+    return lib.onebit_linear_group_prescaled(ctypes.cast(arr, ctypes.c_void_p), up, ap, len(ms), T, _stream_ptr(xs[0].device)), ms, xs, us
+
+
+def _check_group(T, K, Ns):
+    rc, ms, xs, us = _group(T, K, Ns)
     assert rc == 0
     for m, x, u in zip(ms, xs, us):
         _check(m, x, u[:T])
         assert (u[T] == 7.0).all()                 # nothing behind the last row
+
+
+@pytest.mark.parametrize("Ns", [(4096, 4096, 4096), (11008, 11008), (5120, 1028, 260)])
+@pytest.mark.parametrize("T", [65, 96, 97, 129, 192, 577, 673, 897, 1025, 1153, 1540])
+def test_grouped_projections(T, Ns):
+    _check_group(T, 1024, Ns)
+
+
+# members of fewer than 256 columns (keys and values of one head) and K below 1024: at any row count from 65 on with K >= 2048, else from half a round of
+# 256 x 128 tiles on
+@pytest.mark.parametrize("T,K,Ns", [(65, 2048, (2048, 128, 128)), (1153, 2048, (2048, 128, 128)), (193, 4096, (4096, 64, 64)), (1540, 1024, (4096, 128, 124)),
+                                    (1540, 512, (1408, 1408)), (2100, 768, (768, 768, 768)), (1025, 256, (4100, 260)), (193, 256, (16384, 8))])
+def test_grouped_projections_of_few_columns(T, K, Ns):
+    _check_group(T, K, Ns)
+
+
+@pytest.mark.parametrize("T,K,Ns", [(200, 512, (512, 512)), (191, 512, (16384, 16384)), (1540, 512, (250, 1408)), (1540, 1056, (4096, 4096))])
+def test_groups_that_are_refused(T, K, Ns):
+    assert _group(T, K, Ns)[0] == -2
