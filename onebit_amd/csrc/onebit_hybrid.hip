@@ -73,7 +73,14 @@ static bool lds_ok(const void *f, int bytes)
 #define OB_SKINNY_T 64
 #define OB_DEEP_KT 61            // k tiles of a split from which every wave has 16 (the last one 13)
 #define OB_ZROWS 2048           // fp32 rows of partial sums that gemm_splits fills at most: splits * T <= max(OB_ZROWS, T)
-#define OB_ZROWS_ALL 8192       // ... that the buffer holds at least, and dense_plan fills
+#define OB_ZROWS_ALL 8192       // ... and dense_plan, from OB_PLAN_T rows on with bf16 weights
+#define OB_PLAN_T 500
+
+// rows of the partial sums' buffer for steps of up to `rows` (width 4096: 34 MB up to 499 rows or in float32, 134 from 1024 on)
+static int64_t z_rows(bool bf16, int64_t rows)
+{
+    return std::max<int64_t>({rup(rows, 256), OB_ZROWS, bf16 && rows >= OB_PLAN_T ? std::min<int64_t>(8 * rows, OB_ZROWS_ALL) : 0});
+}
 
 // K splits of an output product: enough workgroups to fill the chip, each with a worthwhile share of k tiles
 static int gemm_splits(int n_tiles, int nkt, int T)
@@ -339,7 +346,7 @@ static int make_plan(const onebit_hmodel_t &m, int64_t rows, int64_t n_out, int 
     P.h = take((size_t)R * m.width_pad * es);
     P.u = take((size_t)R * u * es);
     P.aux = take((size_t)R * aux * 4);
-    P.z = take((size_t)std::max<int64_t>(R, OB_ZROWS_ALL) * zc * 4);
+    P.z = take((size_t)z_rows(es == 2, rows) * zc * 4);
     P.hist = take(hist ? (size_t)(m.n_runs + 1) * R * m.width * 4 : 0);
     P.hrm = take(rm ? (size_t)R * m.width_pad * es : 0);
     P.cq = take(cq * es);
@@ -651,7 +658,7 @@ static int part_launch(ObDenseArgs d, float *z, int &n_split, hipStream_t s, int
     int mt = -1;
     if (sizeof(E) == 2 && d.T > OB_SKINNY_T) {
         const DensePlan p = dense_plan(d.n_tiles, d.nkt, d.T, n_split, wr_most<OB_EPI_PART>(),
-                                       d.T < 500 ? 0 : (int)std::min<int64_t>({most, 8, std::max(1, OB_ZROWS_ALL / d.T), std::max(1, d.nkt / 8)}));
+                                       d.T < OB_PLAN_T ? 0 : (int)std::min<int64_t>({most, 8, std::max(1, OB_ZROWS_ALL / d.T), std::max(1, d.nkt / 8)}));
         n_split = p.ns;
         mt = p.mt;
     }

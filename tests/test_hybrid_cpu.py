@@ -203,6 +203,18 @@ def _fake_model(a, **kw):
     return m, (L, runs)
 
 
+def test_partial_sums_have_the_room_that_their_plan_can_fill():
+    """2048 rows of float32 sums; bfloat16 steps of 500 rows and more eight splits of each, 8192 at most (48 columns here); else nothing but the rows' own buffers grows."""
+    buf = ctypes.create_string_buffer(4096)
+    def size(rows, dtype):
+        m, keep = _fake_model((ctypes.addressof(buf) + 255) & ~255, dtype=dtype)
+        return _lib.load_hybrid().onebit_hybrid_workspace_bytes(ctypes.byref(m), rows, 8, 3, 4)
+    for dtype, more in ((_lib.HYB_BF16, {256: 2048, 499: 2048, 500: 4000, 768: 6144, 1024: 8192}), (_lib.HYB_F32, {256: 2048, 499: 2048, 500: 2048, 1024: 2048})):
+        row = (size(2048, dtype) - size(1024, dtype)) // 1024
+        for rows, z in more.items():
+            assert size(rows, dtype) - size(256, dtype) == row * (-(-rows // 256) * 256 - 256) + (z - 2048) * 48 * 4, (dtype, rows)
+
+
 def test_native_step_rejects_bad_arguments():
     lib = _lib.load_hybrid()
     E_ARG, E_SHAPE, E_DTYPE, E_WSPACE = -1, -2, -4, -5
