@@ -13,16 +13,21 @@
 #pragma once
 #include "ob_common.h"
 
+enum { OB_TX_NONE = 0, OB_TX_SCALE_R = 1, OB_TX_SCALE_I = 2, OB_TX_SIGN = 3 };
+enum { OB_TE_PLAIN = 0, OB_TE_GX = 1, OB_TE_STE = 2 };
+
 #define OB_TG_BM 64
 #define OB_TG_BN 64
 #define OB_TG_BR 32
 #define OB_TG_THREADS 256
 
 struct ObTGemmArgs {
-    const void *A, *B;        // C[m, n] = sum_r A(m, r) va(r) sign(B(n, r))
+    const void *A, *B;        // C[m, n] = sum_r A(m, r) * B(n, r)
     long long lda, ldb;       // leading dimension of the operand's storage (elements)
-    const void *va;
+    const void *va, *vb;      // transform vectors, or null
     void *C;                  // [M, N] row-major, pitch ldc
+    void *C2;                 // OB_TE_GX: C2 = C * vc[n]
+    const void *vc;           // OB_TE_GX: vector [N];  OB_TE_STE: latent W [M, N] (pitch ldc)
     long long ldc;
     int M, N, R;
 };
@@ -35,29 +40,48 @@ __device__ __forceinline__ TI ob_tg_sign(TI v)
     return (TI)((v > (TI)0) ? 1.0f : ((v < (TI)0) ? -1.0f : 0.0f));      // NaN -> 0, as (v > 0) - (v < 0)
 }
 
-// One 64 x 32 operand tile into LDS as S[i][r], element (i, r) at P[i * ld + r]: times vec[r], or its sign (vec null).  8 contiguous elements per thread, two
-// 16-byte loads when the run is inside the matrix and aligned.
+// One 64 x 32 operand tile into LDS as S[i][r].  RC: the reduction index r is the contiguous one in memory
+// (element (i, r) at P[i * ld + r]); otherwise the output index i is (element at P[r * ld + i]) and the tile is
+// transposed on its way in.  8 contiguous elements per thread, two 16-byte loads when the run is inside the matrix and aligned.  (Forms are compiled in: chosen by
+// whether there is a vec, both transforms are computed, 65 rows 12544 -> 8 877 us instead of 745.)
+template <bool RC, int TX>
 __device__ __forceinline__ void ob_tg_load(float (*S)[OB_TG_PITCH], const float *__restrict__ P, long long ld, const float *__restrict__ vec,
                                            int i0, int r0, int I, int R, int tid)
 {
     float v[8];
-    const int gi = i0 + (tid >> 2), gr = r0 + (tid & 3) * 8;
-    const float *p = P + (long long)gi * ld + gr;
-    if (gi < I && gr + 8 <= R && ((uintptr_t)p % 16) == 0) {
+    int gi, gr;
+    if (RC) { gi = i0 + (tid >> 2); gr = r0 + (tid & 3) * 8; }
+    else { gr = r0 + (tid >> 3); gi = i0 + (tid & 7) * 8; }
+    const float *p = RC ? P + (long long)gi * ld + gr : P + (long long)gr * ld + gi;
+    const bool inside = RC ? (gi < I && gr + 8 <= R) : (gr < R && gi + 8 <= I);
+    if (inside && ((uintptr_t)p % 16) == 0) {
         reinterpret_cast<ob_u32x4 *>(v)[0] = reinterpret_cast<const ob_u32x4 *>(p)[0];
         reinterpret_cast<ob_u32x4 *>(v)[1] = reinterpret_cast<const ob_u32x4 *>(p)[1];
     } else {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = gi < I && gr + e < R ? p[e] : 0.f;
+        for (int e = 0; e < 8; ++e) {
+            const bool ok = RC ? (gi < I && gr + e < R) : (gr < R && gi + e < I);
+            v[e] = ok ? p[e] : 0.f;
+        }
     }
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = !vec ? ob_tg_sign<float>(v[e]) : gi < I && gr + e < R ? v[e] * vec[gr + e] : 0.f;
-    float *d = &S[tid >> 2][(tid & 3) * 8];
-    reinterpret_cast<ob_u32x4 *>(d)[0] = reinterpret_cast<ob_u32x4 *>(v)[0];
-    reinterpret_cast<ob_u32x4 *>(d)[1] = reinterpret_cast<ob_u32x4 *>(v)[1];
+    for (int e = 0; e < 8; ++e) {
+        const int ei = RC ? gi : gi + e, er = RC ? gr + e : gr;
+        if (TX == OB_TX_SIGN) v[e] = ob_tg_sign<float>(v[e]);
+        if (TX == OB_TX_SCALE_R) v[e] = (ei < I && er < R) ? v[e] * vec[er] : 0.f;
+        if (TX == OB_TX_SCALE_I) v[e] = (ei < I && er < R) ? v[e] * vec[ei] : 0.f;
+    }
+    if (RC) {
+        float *d = &S[tid >> 2][(tid & 3) * 8];
+        reinterpret_cast<ob_u32x4 *>(d)[0] = reinterpret_cast<ob_u32x4 *>(v)[0];
+        reinterpret_cast<ob_u32x4 *>(d)[1] = reinterpret_cast<ob_u32x4 *>(v)[1];
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) S[(tid & 7) * 8 + e][tid >> 3] = v[e];
+    }
 }
 
-// float32 product of a forward call without a workspace, or of a small one: 64 x 64 x 32 tiles, v_mfma_f32_16x16x4_f32
+template <bool RCA, bool RCB, int TXA, int TXB, int EPI>
 __global__ __launch_bounds__(OB_TG_THREADS) void ob_tgemm_kernel(const ObTGemmArgs a)
 {
     __shared__ __attribute__((aligned(16))) float As[OB_TG_BM][OB_TG_PITCH];
@@ -73,8 +97,8 @@ __global__ __launch_bounds__(OB_TG_THREADS) void ob_tgemm_kernel(const ObTGemmAr
         for (int y = 0; y < 2; ++y) acc[x][y] = (ob_float4){0.f, 0.f, 0.f, 0.f};
     const float *A = (const float *)a.A, *B = (const float *)a.B;
     for (int r0 = 0; r0 < a.R; r0 += OB_TG_BR) {
-        ob_tg_load(As, A, a.lda, (const float *)a.va, i0, r0, a.M, a.R, tid);
-        ob_tg_load(Bs, B, a.ldb, nullptr, j0, r0, a.N, a.R, tid);
+        ob_tg_load<RCA, TXA>(As, A, a.lda, (const float *)a.va, i0, r0, a.M, a.R, tid);
+        ob_tg_load<RCB, TXB>(Bs, B, a.ldb, (const float *)a.vb, j0, r0, a.N, a.R, tid);
         __syncthreads();
 #pragma unroll
         for (int kk = 0; kk < OB_TG_BR; kk += 4) {
@@ -91,7 +115,8 @@ __global__ __launch_bounds__(OB_TG_THREADS) void ob_tgemm_kernel(const ObTGemmAr
         }
         __syncthreads();
     }
-    float *C = (float *)a.C;
+    float *C = (float *)a.C, *C2 = (float *)a.C2;
+    const float *vc = (const float *)a.vc;
 #pragma unroll
     for (int x = 0; x < 2; ++x) {
         const int m = i0 + wm * 32 + x * 16 + lr;
@@ -100,8 +125,17 @@ __global__ __launch_bounds__(OB_TG_THREADS) void ob_tgemm_kernel(const ObTGemmAr
         for (int y = 0; y < 2; ++y) {
             const int n = j0 + wn * 32 + y * 16 + 4 * lg;
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (n + e < a.N) C[(long long)m * a.ldc + n + e] = acc[x][y][e];
+            for (int e = 0; e < 4; ++e) {
+                if (n + e >= a.N) continue;
+                const long long o = (long long)m * a.ldc + n + e;
+                const float c = acc[x][y][e];
+                if (EPI == OB_TE_PLAIN) C[o] = c;
+                if (EPI == OB_TE_GX) { C[o] = c; C2[o] = c * vc[n + e]; }
+                if (EPI == OB_TE_STE) {                                // SignSTEFunc.backward (bitnet.py:22-23): grad * (1.001 - tanh(w) ** 2)
+                    const float w = tanhf(vc[o]);
+                    C[o] = c * (1.001f - w * w);
+                }
+            }
         }
     }
 }

@@ -328,7 +328,7 @@ static int ob_train_forward_t(const void *x, const void *w, const void *h, const
         ob_set_max_lds_once(ob_tgemm128_f16_kernel, attr_set, OB_TG2_LDS);
         hipLaunchKernelGGL(ob_tgemm128_f16_kernel, dim3((unsigned)((N + OB_TG2_B - 1) / OB_TG2_B), (unsigned)((T + OB_TG2_B - 1) / OB_TG2_B)), dim3(OB_TG_THREADS),
                            OB_TG2_LDS, s, a);
-    } else hipLaunchKernelGGL(ob_tgemm_kernel, dim3((unsigned)((N + OB_TG_BN - 1) / OB_TG_BN), (unsigned)((T + OB_TG_BM - 1) / OB_TG_BM)), dim3(OB_TG_THREADS), 0, s, a);
+    } else hipLaunchKernelGGL((ob_tgemm_kernel<true, true, OB_TX_SCALE_R, OB_TX_SIGN, OB_TE_PLAIN>), dim3((unsigned)((N + OB_TG_BN - 1) / OB_TG_BN), (unsigned)((T + OB_TG_BM - 1) / OB_TG_BM)), dim3(OB_TG_THREADS), 0, s, a);
     int rc = ob_launch_status("train_forward(gemm)");
     if (rc) return rc;
     hipLaunchKernelGGL((ob_train_ln_fwd_kernel<TI>), dim3((unsigned)T), dim3(256), 0, s, (const TI *)z, (const TI *)g, (const TI *)bias,

@@ -183,3 +183,10 @@ def test_one_bit_products_wait_for_the_tile_they_publish(one_bit):
 
 def test_one_bit_operands_are_not_written_in_front_of_their_products(one_bit):
     assert _operands_are_ready(one_bit, "scratch_load") > 5000             # (the largest tile stores what its epilogue reads, in front of its last steps)
+
+
+def test_small_float32_train_product_computes_one_transform_an_operand(tmp_path):
+    """ob_tgemm_kernel's forward instance: the weights' signs are two comparisons of each of a thread's eight elements, the activations' products none."""
+    ks = _kernels("onebit_train.hip", tmp_path, re.compile(r"ob_tgemm_kernel(ILb1ELb1ELi1ELi3|\d)"))
+    assert len(ks) == 1
+    assert sum(bool(re.match(r"v_cmpx?_n?(gt|lt|ge|le)_f32", op)) for op, _ in ks[0].text) == 16
