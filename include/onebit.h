@@ -553,13 +553,17 @@ int onebit_fused_gemv(const onebit_proj_t *projs, void *const *outs, int nproj, 
  *             z_save [T,N] (dtype) receives the GEMM output before * g, ln_stats [T,2] fp32 {mean, rstd}: what the
  *             backward pass reads instead of recomputing the GEMM.
  *   backward  from gy [T,N]: gx [T,K], gw [N,K] = (gz^T . (x*h)) * (1.001 - tanh(W)^2) (the STE, :21-23), gh [K],
- *             gg [N], gbias [N] (optional).  workspace: onebit_train_workspace_bytes(T,K,N,dtype), 16-byte aligned.
- *             forward_ws: the same with scratch memory, onebit_train_forward_workspace_bytes(T,K,N,dtype) of it 16-byte aligned (0 for fp32 and
- *             for products too small to gain;
- *             less or NULL takes the form of onebit_train_forward, half as fast in fp16 at T = 4096, 4096 -> 11008).
+ *             gg [N], gbias [N] (optional).  workspace: onebit_train_workspace_bytes(T,K,N,dtype), 16-byte aligned; onebit_train_least_workspace_bytes
+ *             is required, and less than the former takes slower kernels (fp16: few rows in one slice; fp32: MFMA 16x16x4 f32, 4 times slower at
+ *             T = 3600, 4096 -> 4096).
+ *             forward_ws: the same with scratch memory, onebit_train_forward_workspace_bytes(T,K,N,dtype) of it 16-byte aligned (0 for
+ *             products too small to gain; less or NULL takes the form of onebit_train_forward, half as fast in fp16 at T = 4096, 4096 -> 11008,
+ *             but for the slices of few rows, without whose room the other kernels stay).
  * fp16: MFMA 16x16x32 f16 with fp32 accumulation, every tensor-level op of the reference rounded once to fp16;
- * fp32: MFMA 16x16x4 f32.  Deterministic (no atomics: column sums have a fixed order).                          */
+ * fp32: MFMA 16x16x32 bf16 on three bf16 parts of a number, without the workspace 16x16x4 f32.  Deterministic (no atomics: column sums have a
+ * fixed order).                                                                                                */
 size_t onebit_train_workspace_bytes(int64_t T, int64_t K, int64_t N, int dtype);
+size_t onebit_train_least_workspace_bytes(int64_t T, int64_t K, int64_t N, int dtype);
 size_t onebit_train_forward_workspace_bytes(int64_t T, int64_t K, int64_t N, int dtype);
 int onebit_train_forward_ws(const void *x, const void *w_latent, const void *h, const void *g, const void *bias_or_null,
                             void *y, void *z_save, float *ln_stats, void *workspace, size_t workspace_bytes, int64_t T, int64_t K,

@@ -66,6 +66,7 @@ SYMBOLS = {
     "onebit_debug_fill_lds": (_int, [ctypes.c_uint32, _vp]),
     "onebit_fused_gemv": (_int, [_vp, _vp, _int, _int, _vp, _vp]),
     "onebit_train_workspace_bytes": (ctypes.c_size_t, [_i64, _i64, _i64, _int]),
+    "onebit_train_least_workspace_bytes": (ctypes.c_size_t, [_i64, _i64, _i64, _int]),
     "onebit_train_forward_workspace_bytes": (ctypes.c_size_t, [_i64, _i64, _i64, _int]),
     "onebit_train_forward_ws": (_int, [_vp] * 9 + [ctypes.c_size_t, _i64, _i64, _i64, _int, _f, _vp]),
     "onebit_train_forward": (_int, [_vp] * 8 + [_i64, _i64, _i64, _int, _f, _vp]),

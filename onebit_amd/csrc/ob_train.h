@@ -7,8 +7,9 @@
 //             ga = gz . S;  gx = ga * h;  gh = sum_t ga * x
 //             gS = gz^T . a;  gW = gS * (1.001 - tanh(W)^2)                       (the STE of :21-23)
 //
-// float16: ob_train16.h, float32: ob_train32.h.  Here: the forward passes without a workspace (one product kernel each, whose operand loaders apply x * h and
-// sign(W) on the way into LDS) and the LayerNorm that takes any row.  Accumulation is fp32 in both.  In fp16 every tensor-level op of the reference rounds
+// float16: ob_train16.h, float32: ob_train32.h.  Here: the forward passes without a workspace and the float32 backward pass with as little of one as it can do with (product
+// kernels whose operand loaders apply x * h and sign(W) on the way into LDS and whose epilogues apply what follows: * h for gx, the STE factor for gW), and the
+// LayerNorm that takes any row.  Accumulation is fp32 in both.  In fp16 every tensor-level op of the reference rounds
 // once to fp16 (x * h, z, u, gz, ga, gx, gW), as the torch ops do.
 #pragma once
 #include "ob_common.h"
@@ -259,5 +260,88 @@ __global__ __launch_bounds__(256) void ob_train_ln_fwd_kernel(const TI *__restri
     if (threadIdx.x == 0) { stats[2 * t] = mean; stats[2 * t + 1] = rstd; }
 }
 
-// bands of rows that column sums are taken over by one workgroup each, at most this many; the partial sums are added in order (deterministic)
-#define OB_TC_SLICES 32
+// backward through the LayerNorm and the * g: with uh = (u - mean) * rstd,
+//   gu = rstd * (gy - mean_n(gy) - uh * mean_n(gy * uh));   gz = gu * g
+// rowc[t] = {mean_n(gy), mean_n(gy * uh)} is kept for the column reductions (gg needs gu again).
+__global__ __launch_bounds__(256) void ob_train_ln_bwd_kernel(const float *__restrict__ gy, const float *__restrict__ z, const float *__restrict__ g,
+                                                              const float *__restrict__ stats, float *__restrict__ gz, float *__restrict__ rowc, int N)
+{
+    __shared__ float red[8];
+    const int t = blockIdx.x;
+    const float *zr = z + (long long)t * N, *gr = gy + (long long)t * N;
+    const float mean = stats[2 * t], rstd = stats[2 * t + 1];
+    float s1 = 0.f, s2 = 0.f;
+    for (int n = threadIdx.x; n < N; n += 256) {
+        const float uh = (zr[n] * g[n] - mean) * rstd, d = gr[n];
+        s1 += d; s2 += d * uh;
+    }
+    const float c1 = ob_block_sum(s1, red) / (float)N;
+    const float c2 = ob_block_sum(s2, red) / (float)N;
+    for (int n = threadIdx.x; n < N; n += 256) {
+        const float uh = (zr[n] * g[n] - mean) * rstd;
+        const float gu = rstd * (gr[n] - c1 - uh * c2);
+        gz[(long long)t * N + n] = gu * g[n];
+    }
+    if (threadIdx.x == 0) { rowc[2 * t] = c1; rowc[2 * t + 1] = c2; }
+}
+
+// Column sums over the tokens, in two deterministic stages (one 64-column block walking all T rows took 0.45 / 0.30 ms of a
+// 3.3 ms layer step): stage 1 -- block (column block, token slice s of OB_TC_SLICES) accumulates its rows in fp32 and writes
+// part[s][column]; stage 2 -- one thread per column adds the slices in order.
+//   gg[n] = sum_t gu[t, n] * z[t, n], gbias[n] = sum_t gy[t, n]      (gu: the LayerNorm backward of ob_train_ln_bwd_kernel, recomputed)
+//   gh[k] = sum_t ga[t, k] * x[t, k]
+#define OB_TC_SLICES 32                  // (also: bands of rows of ob_train16.h's and ob_train32.h's column sums, at most)
+__global__ __launch_bounds__(256) void ob_train_cols_ln_kernel(const float *__restrict__ gy, const float *__restrict__ z, const float *__restrict__ g,
+                                                               const float *__restrict__ stats, const float *__restrict__ rowc,
+                                                               float *__restrict__ part, int T, int N)
+{
+    __shared__ float sm[2][4][64];
+    const int c = threadIdx.x & 63, rl = threadIdx.x >> 6, n = blockIdx.x * 64 + c;
+    const int per = (T + OB_TC_SLICES - 1) / OB_TC_SLICES, t0 = blockIdx.y * per, t1 = min(T, t0 + per);
+    float a0 = 0.f, a1 = 0.f;
+    if (n < N) {
+        const float gn = g[n];
+        for (int t = t0 + rl; t < t1; t += 4) {
+            const float mean = stats[2 * t], rstd = stats[2 * t + 1], c1 = rowc[2 * t], c2 = rowc[2 * t + 1];
+            const float zz = z[(long long)t * N + n];
+            const float uh = (zz * gn - mean) * rstd, d = gy[(long long)t * N + n];
+            const float gu = rstd * (d - c1 - uh * c2);
+            a0 += gu * zz;
+            a1 += d;
+        }
+    }
+    sm[0][rl][c] = a0; sm[1][rl][c] = a1;
+    __syncthreads();
+    if (rl == 0 && n < N) {
+        part[((size_t)blockIdx.y * 2 + 0) * N + n] = (sm[0][0][c] + sm[0][1][c]) + (sm[0][2][c] + sm[0][3][c]);
+        part[((size_t)blockIdx.y * 2 + 1) * N + n] = (sm[1][0][c] + sm[1][1][c]) + (sm[1][2][c] + sm[1][3][c]);
+    }
+}
+
+__global__ __launch_bounds__(256) void ob_train_cols_gh_kernel(const float *__restrict__ ga, const float *__restrict__ x, float *__restrict__ part, int T, int K)
+{
+    __shared__ float sm[4][64];
+    const int c = threadIdx.x & 63, rl = threadIdx.x >> 6, k = blockIdx.x * 64 + c;
+    const int per = (T + OB_TC_SLICES - 1) / OB_TC_SLICES, t0 = blockIdx.y * per, t1 = min(T, t0 + per);
+    float a0 = 0.f;
+    if (k < K)
+        for (int t = t0 + rl; t < t1; t += 4) a0 += ga[(long long)t * K + k] * x[(long long)t * K + k];
+    sm[rl][c] = a0;
+    __syncthreads();
+    if (rl == 0 && k < K) part[(size_t)blockIdx.y * K + k] = (sm[0][c] + sm[1][c]) + (sm[2][c] + sm[3][c]);
+}
+
+// stage 2: out_j[c] = sum over slices of part[s][j][c], j < NOUT (out_1 may be null)
+template <int NOUT>
+__global__ __launch_bounds__(256) void ob_train_cols_finish_kernel(const float *__restrict__ part, float *__restrict__ out0, float *__restrict__ out1, int C)
+{
+    const int c = blockIdx.x * 256 + threadIdx.x;
+    if (c >= C) return;
+#pragma unroll
+    for (int j = 0; j < NOUT; ++j) {
+        float a = 0.f;
+        for (int sl = 0; sl < OB_TC_SLICES; ++sl) a += part[((size_t)sl * NOUT + j) * C + c];
+        float *o = j == 0 ? out0 : out1;
+        if (o) o[c] = a;
+    }
+}

@@ -7,6 +7,13 @@
 #include "ob_train32.h"
 
 // onebit_train_forward / onebit_train_backward: bitnet.py:14-28 (SignSTE) and :58-68 (BitLinear.forward)
+template <bool RCA, bool RCB, int TXA, int TXB, int EPI>
+static void ob_launch_tgemm(const ObTGemmArgs &a, hipStream_t s)
+{
+    const dim3 grid((unsigned)((a.N + OB_TG_BN - 1) / OB_TG_BN), (unsigned)((a.M + OB_TG_BM - 1) / OB_TG_BM));
+    hipLaunchKernelGGL((ob_tgemm_kernel<RCA, RCB, TXA, TXB, EPI>), grid, dim3(OB_TG_THREADS), 0, s, a);
+}
+
 static size_t ob_train_align(size_t b) { return (b + 255) & ~(size_t)255; }
 
 // ---- float16 (ob_train16.h) ---------------------------------------------------------------------------------------------
@@ -37,6 +44,12 @@ static ObTrainPlan ob_train_plan(int dtype, bool gx, int64_t T, int64_t C, int64
         if (gain > most) { most = gain; best.ns = ns; }
     }
     return best;
+}
+static ObTrainPlan ob_train_plan(int dtype, bool gx, int64_t T, int64_t C, int64_t R, bool slices)
+{
+    ObTrainPlan p = ob_train_plan(dtype, gx, T, C, R);
+    if (!slices) p.ns = 1;
+    return p;
 }
 static size_t ob_train_zld(int64_t T, int64_t C) { return ob_train_align((size_t)T * C * 4) / 4; }
 static size_t ob_train_slice_bytes(const ObTrainPlan &p, int64_t T, int64_t C) { return p.ns > 1 ? p.ns * ob_train_zld(T, C) * 4 : 0; }
@@ -119,14 +132,14 @@ static int64_t ob_t16_portion(int64_t T, int64_t K)
     return ((T + n - 1) / n + 127) / 128 * 128;
 }
 
-static int ob_t16_forward(const void *x, const void *w, const void *h, const void *g, const void *bias, void *y, void *z, float *stats, char *ws,
+static int ob_t16_forward(const void *x, const void *w, const void *h, const void *g, const void *bias, void *y, void *z, float *stats, char *ws, bool room,
                           int64_t T, int64_t K, int64_t N, float eps, hipStream_t s)
 {
     char *sg = ws, *a = ws + ob_t16_bytes(N, K);
     ob_t16_tiles(true, w, nullptr, sg, N, K, s);
     const int kt = (int)(ob_t16_up32(K) / 32);
     const int64_t Tp = ob_t16_portion(T, K);
-    const ObTrainPlan p = ob_train_plan(ONEBIT_F16, false, Tp, N, K);
+    const ObTrainPlan p = ob_train_plan(ONEBIT_F16, false, Tp, N, K, room);
     float *zp = (float *)(a + ob_t16_bytes(Tp, K));
     for (int64_t t0 = 0; t0 < T; t0 += Tp) {
         const int64_t n = std::min(Tp, T - t0);
@@ -143,7 +156,7 @@ static int ob_t16_forward(const void *x, const void *w, const void *h, const voi
 }
 
 static int ob_t16_backward(const void *gy, const void *x, const void *w, const void *h, const void *g, const void *z, const float *stats, void *gx, void *gw,
-                           void *gh, void *gg, void *gbias, char *ws, int64_t T, int64_t K, int64_t N, hipStream_t s)
+                           void *gh, void *gg, void *gbias, char *ws, bool room, int64_t T, int64_t K, int64_t N, hipStream_t s)
 {
     // (the sign matrix and, once the input gradient is formed, x h in one place)
     char *sg = ws, *a = ws, *gz = ws + std::max(ob_t16_bytes(T, K), ob_t16_bytes(N, K));
@@ -159,7 +172,7 @@ static int ob_t16_backward(const void *gy, const void *x, const void *w, const v
     // gx [T, K] = fp16(gz S) h;  gh = sum_t fp16(gz S) x
     ObT16Mm m = {sg, gz, (int)((K + 15) / 16), (int)((T + 15) / 16), kt, nt, nt, (_Float16 *)gx, (int)T, (int)K, (const _Float16 *)h, (const _Float16 *)x, part};
     m.vec4 = K % 4 == 0 && ob_aligned(gx, 8) && ob_aligned(x, 8);
-    const ObTrainPlan p = ob_train_plan(ONEBIT_F16, true, T, K, N);
+    const ObTrainPlan p = ob_train_plan(ONEBIT_F16, true, T, K, N, room);
     m.zp = (float *)((char *)rowc + ob_train_align((size_t)T * 8)); m.zld = ob_train_zld(T, K); m.ns = p.ns;
     ob_t16_mm<OB_T16_GX, true, false>(m, p, s);
     if (p.ns > 1) ob_train_gxsum<_Float16>(m.zp, p.ns, h, x, gx, part, T, K, s);
@@ -223,14 +236,14 @@ static void ob_t32_layernorm(const void *z, const void *g, const void *bias, voi
 
 static int64_t ob_t32_portion(int64_t T, int64_t K) { return ob_t16_portion(T, OB_T32_PARTS * K); }
 
-static int ob_t32_forward(const void *x, const void *w, const void *h, const void *g, const void *bias, void *y, void *z, float *stats, char *ws,
+static int ob_t32_forward(const void *x, const void *w, const void *h, const void *g, const void *bias, void *y, void *z, float *stats, char *ws, bool room,
                           int64_t T, int64_t K, int64_t N, float eps, hipStream_t s)
 {
     char *sg = ws, *a = ws + ob_t16_bytes(N, K);
     ob_t32_tiles(true, w, nullptr, sg, N, K, s);
     const int kt = (int)(ob_t16_up32(K) / 32);
     const int64_t Tp = ob_t32_portion(T, K);
-    const ObTrainPlan p = ob_train_plan(ONEBIT_F32, false, Tp, N, K);
+    const ObTrainPlan p = ob_train_plan(ONEBIT_F32, false, Tp, N, K, room);
     float *zp = (float *)(a + OB_T32_PARTS * ob_t16_bytes(Tp, K));
     for (int64_t t0 = 0; t0 < T; t0 += Tp) {
         const int64_t n = std::min(Tp, T - t0);
@@ -251,7 +264,7 @@ static int ob_t32_forward(const void *x, const void *w, const void *h, const voi
 static size_t ob_t32_operand_bytes(int64_t T, int64_t K, int64_t N) { return std::max(OB_T32_PARTS * ob_t16_bytes(T, K), ob_t16_bytes(N, K)); }
 
 static int ob_t32_backward(const void *gy, const void *x, const void *w, const void *h, const void *g, const void *z, const float *stats, void *gx, void *gw,
-                           void *gh, void *gg, void *gbias, char *ws, int64_t T, int64_t K, int64_t N, hipStream_t s)
+                           void *gh, void *gg, void *gbias, char *ws, bool room, int64_t T, int64_t K, int64_t N, hipStream_t s)
 {
     char *sg = ws, *a = ws, *gz = ws + ob_t32_operand_bytes(T, K, N);
     const size_t gzb = ob_t16_bytes(T, N);
@@ -268,7 +281,7 @@ static int ob_t32_backward(const void *gy, const void *x, const void *w, const v
     ObT32Mm m = {sg, gz, (int)((K + 15) / 16), (int)((T + 15) / 16), kt, nt, {nt, nt, nt}, {}, {2 * gzb, gzb, 0}, (float *)gx, (int)T, (int)K,
                  (const float *)h, (const float *)x, part};
     m.vec4 = K % 4 == 0 && ob_aligned(gx, 16) && ob_aligned(x, 16);
-    const ObTrainPlan p = ob_train_plan(ONEBIT_F32, true, T, K, N);
+    const ObTrainPlan p = ob_train_plan(ONEBIT_F32, true, T, K, N, room);
     m.zp = (float *)((char *)rowc + ob_train_align((size_t)T * 8)); m.zld = ob_train_zld(T, K); m.ns = p.ns;
     ob_t32_mm<OB_T16_GX, true, false>(m, p, s);
     if (p.ns > 1) ob_train_gxsum<float>(m.zp, p.ns, h, x, gx, part, T, K, s);
@@ -288,23 +301,42 @@ static int ob_t32_backward(const void *gy, const void *x, const void *w, const v
 // Workspace of the forward pass: a smaller or absent one takes the kernels that transform operands on their way into LDS, and so do small products, where two
 // launches beat four (float16: 64 -> 64 up to 2048 rows 10.7 us against 16.3; 128 -> 128, 64 rows 12.9 / 16.1; 256 -> 128 18.0 / 16.4; 64 -> 128, 8192 rows 20.4 / 18.5;
 // float32, below 64 M products: 64 rows 512 -> 512 in a trace 30 us / 25, but a call's host time has two launches more, 200 rows 31 / 26; 64 rows 1024 -> 1000, the
-// first that takes it, 65 / 35)
-extern "C" size_t onebit_train_forward_workspace_bytes(int64_t T, int64_t K, int64_t N, int dtype)
+// first that takes it, 65 / 35).  One without room for slices' sums (ob_train_forward_least) takes products of one slice.
+static size_t ob_train_forward_least(int64_t T, int64_t K, int64_t N, int dtype)
 {
     if (T <= 0 || K <= 0 || N <= 0 || (dtype != ONEBIT_F16 && dtype != ONEBIT_F32)) return 0;
     if (K < 512 && (N < 128 || (K < 256 && T < 100000000 / (K * N)))) return 0;
-    if (dtype == ONEBIT_F32) return T * K < 64000000 / N ? 0 : OB_T32_PARTS * ob_t16_bytes(ob_t32_portion(T, K), K) + ob_t16_bytes(N, K) +
-                                                                      ob_train_slice_bytes(ob_train_plan(dtype, false, ob_t32_portion(T, K), N, K), ob_t32_portion(T, K), N);
-    const int64_t Tp = ob_t16_portion(T, K);
-    return ob_t16_bytes(Tp, K) + ob_t16_bytes(N, K) + ob_train_slice_bytes(ob_train_plan(dtype, false, Tp, N, K), Tp, N);
+    if (dtype == ONEBIT_F32) return T * K < 64000000 / N ? 0 : OB_T32_PARTS * ob_t16_bytes(ob_t32_portion(T, K), K) + ob_t16_bytes(N, K);
+    return ob_t16_bytes(ob_t16_portion(T, K), K) + ob_t16_bytes(N, K);
+}
+extern "C" size_t onebit_train_forward_workspace_bytes(int64_t T, int64_t K, int64_t N, int dtype)
+{
+    const size_t n = ob_train_forward_least(T, K, N, dtype);
+    if (n == 0) return 0;
+    const int64_t Tp = dtype == ONEBIT_F32 ? ob_t32_portion(T, K) : ob_t16_portion(T, K);
+    return n + ob_train_slice_bytes(ob_train_plan(dtype, false, Tp, N, K), Tp, N);
 }
 
+// the backward pass without room for slices' sums; float32 in products of parts (ob_train32.h)
+static size_t ob_train_backward_bytes(int64_t T, int64_t K, int64_t N, int dtype)
+{
+    const size_t rest = ob_t16_part_bytes(T, K, N) + ob_train_align((size_t)T * 8);
+    if (dtype == ONEBIT_F32) return ob_t32_operand_bytes(T, K, N) + OB_T32_PARTS * ob_t16_bytes(T, N) + rest;
+    return std::max(ob_t16_bytes(T, K), ob_t16_bytes(N, K)) + ob_t16_bytes(T, N) + rest;
+}
 extern "C" size_t onebit_train_workspace_bytes(int64_t T, int64_t K, int64_t N, int dtype)
 {
     if (T <= 0 || K <= 0 || N <= 0) return 0;
-    const size_t rest = ob_t16_part_bytes(T, K, N) + ob_train_align((size_t)T * 8) + ob_train_slice_bytes(ob_train_plan(dtype, true, T, K, N), T, K);
-    if (dtype == ONEBIT_F32) return ob_t32_operand_bytes(T, K, N) + OB_T32_PARTS * ob_t16_bytes(T, N) + rest;
-    return std::max(ob_t16_bytes(T, K), ob_t16_bytes(N, K)) + ob_t16_bytes(T, N) + rest;
+    return ob_train_backward_bytes(T, K, N, dtype) + ob_train_slice_bytes(ob_train_plan(dtype, true, T, K, N), T, K);
+}
+extern "C" size_t onebit_train_least_workspace_bytes(int64_t T, int64_t K, int64_t N, int dtype)
+{
+    if (T <= 0 || K <= 0 || N <= 0) return 0;
+    const size_t n = ob_train_backward_bytes(T, K, N, dtype);
+    if (dtype != ONEBIT_F32) return n;
+    return std::min(n,                                                     // (gz, ga, the rows' means, the column sums' partials)
+                    ob_train_align((size_t)T * N * 4) + ob_train_align((size_t)T * K * 4) + ob_train_align((size_t)T * 2 * sizeof(float)) +
+                        ob_train_align((size_t)OB_TC_SLICES * std::max(2 * (size_t)N, (size_t)K) * sizeof(float)));
 }
 
 static int ob_train_check(const char *what, int64_t T, int64_t K, int64_t N, int dtype)
@@ -328,7 +360,7 @@ static int ob_train_forward_t(const void *x, const void *w, const void *h, const
         ob_set_max_lds_once(ob_tgemm128_f16_kernel, attr_set, OB_TG2_LDS);
         hipLaunchKernelGGL(ob_tgemm128_f16_kernel, dim3((unsigned)((N + OB_TG2_B - 1) / OB_TG2_B), (unsigned)((T + OB_TG2_B - 1) / OB_TG2_B)), dim3(OB_TG_THREADS),
                            OB_TG2_LDS, s, a);
-    } else hipLaunchKernelGGL((ob_tgemm_kernel<true, true, OB_TX_SCALE_R, OB_TX_SIGN, OB_TE_PLAIN>), dim3((unsigned)((N + OB_TG_BN - 1) / OB_TG_BN), (unsigned)((T + OB_TG_BM - 1) / OB_TG_BM)), dim3(OB_TG_THREADS), 0, s, a);
+    } else ob_launch_tgemm<true, true, OB_TX_SCALE_R, OB_TX_SIGN, OB_TE_PLAIN>(a, s);
     int rc = ob_launch_status("train_forward(gemm)");
     if (rc) return rc;
     hipLaunchKernelGGL((ob_train_ln_fwd_kernel<TI>), dim3((unsigned)T), dim3(256), 0, s, (const TI *)z, (const TI *)g, (const TI *)bias,
@@ -346,9 +378,10 @@ extern "C" int onebit_train_forward_ws(const void *x, const void *w_latent, cons
     if (K == 0) return ob_fail(ONEBIT_E_SHAPE, "train_forward: in_features = 0");
     if (!x || !w_latent || !h || !g || !y || !z_save || !ln_stats) return ob_fail(ONEBIT_E_ARG, "train_forward: null pointer");
     hipStream_t s = (hipStream_t)stream;
-    const size_t need = onebit_train_forward_workspace_bytes(T, K, N, dtype);
-    if (need && workspace && ob_aligned(workspace, 16) && workspace_bytes >= need)
-        return (dtype == ONEBIT_F16 ? ob_t16_forward : ob_t32_forward)(x, w_latent, h, g, bias_or_null, y, z_save, ln_stats, (char *)workspace, T, K, N, ln_eps, s);
+    const size_t least = ob_train_forward_least(T, K, N, dtype);
+    if (least && workspace && ob_aligned(workspace, 16) && workspace_bytes >= least)
+        return (dtype == ONEBIT_F16 ? ob_t16_forward : ob_t32_forward)(x, w_latent, h, g, bias_or_null, y, z_save, ln_stats, (char *)workspace,
+                                                                       workspace_bytes >= onebit_train_forward_workspace_bytes(T, K, N, dtype), T, K, N, ln_eps, s);
     return dtype == ONEBIT_F16 ? ob_train_forward_t<_Float16>(x, w_latent, h, g, bias_or_null, y, z_save, ln_stats, T, K, N, ln_eps, s)
                                : ob_train_forward_t<float>(x, w_latent, h, g, bias_or_null, y, z_save, ln_stats, T, K, N, ln_eps, s);
 }
@@ -358,6 +391,47 @@ extern "C" int onebit_train_forward(const void *x, const void *w_latent, const v
                                     float ln_eps, void *stream)
 {
     return onebit_train_forward_ws(x, w_latent, h, g, bias_or_null, y, z_save, ln_stats, nullptr, 0, T, K, N, dtype, ln_eps, stream);
+}
+
+// float32 with ob_train_least's workspace: the products on v_mfma_f32_16x16x4_f32, one float32 of gz and of ga each and no sign matrix
+static int ob_train_backward_f32(const void *gy, const void *x, const void *w, const void *h, const void *g, const void *z,
+                                 const float *stats, void *gx, void *gw, void *gh, void *gg, void *gbias, char *ws,
+                                 int64_t T, int64_t K, int64_t N, hipStream_t s)
+{
+    float *gz = (float *)ws;
+    float *ga = (float *)(ws + ob_train_align((size_t)T * N * sizeof(float)));
+    float *rowc = (float *)(ws + ob_train_align((size_t)T * N * sizeof(float)) + ob_train_align((size_t)T * K * sizeof(float)));
+    float *part = (float *)((char *)rowc + ob_train_align((size_t)T * 2 * sizeof(float)));     // [OB_TC_SLICES][2 N | K] column-sum partials
+    int rc;
+    // 1. through the LayerNorm and * g: gz [T, N]; column sums gg, gbias
+    hipLaunchKernelGGL(ob_train_ln_bwd_kernel, dim3((unsigned)T), dim3(256), 0, s, (const float *)gy, (const float *)z, (const float *)g, stats, gz, rowc, (int)N);
+    if ((rc = ob_launch_status("train_backward(layernorm)"))) return rc;
+    hipLaunchKernelGGL(ob_train_cols_ln_kernel, dim3((unsigned)((N + 63) / 64), OB_TC_SLICES), dim3(256), 0, s, (const float *)gy, (const float *)z, (const float *)g, stats,
+                       (const float *)rowc, part, (int)T, (int)N);
+    hipLaunchKernelGGL(ob_train_cols_finish_kernel<2>, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, s, (const float *)part, (float *)gg, (float *)gbias, (int)N);
+    if ((rc = ob_launch_status("train_backward(gg)"))) return rc;
+    // 2. ga [T, K] = gz . sign(W);  gx = ga * h;  gh = sum_t ga * x
+    {
+        ObTGemmArgs a = {};
+        a.A = gz; a.lda = N;                 // A(t, n) = gz[t, n]            (n contiguous)
+        a.B = w; a.ldb = K;                  // B(k, n) = sign(W[n, k])        (k = output index, contiguous)
+        a.C = ga; a.C2 = gx; a.vc = h; a.ldc = K; a.M = (int)T; a.N = (int)K; a.R = (int)N;
+        ob_launch_tgemm<true, false, OB_TX_NONE, OB_TX_SIGN, OB_TE_GX>(a, s);
+        if ((rc = ob_launch_status("train_backward(grad input)"))) return rc;
+        hipLaunchKernelGGL(ob_train_cols_gh_kernel, dim3((unsigned)((K + 63) / 64), OB_TC_SLICES), dim3(256), 0, s, (const float *)ga, (const float *)x, part, (int)T, (int)K);
+        hipLaunchKernelGGL(ob_train_cols_finish_kernel<1>, dim3((unsigned)((K + 255) / 256)), dim3(256), 0, s, (const float *)part, (float *)gh, (float *)nullptr, (int)K);
+        if ((rc = ob_launch_status("train_backward(gh)"))) return rc;
+    }
+    // 3. gW [N, K] = (gz^T . (x * h)) * (1.001 - tanh(W)^2)
+    {
+        ObTGemmArgs a = {};
+        a.A = gz; a.lda = N;                 // A(n, t) = gz[t, n]            (n = output index, contiguous)
+        a.B = x; a.ldb = K; a.vb = h;        // B(k, t) = x[t, k] * h[k]      (k = output index, contiguous)
+        a.C = gw; a.vc = w; a.ldc = K; a.M = (int)N; a.N = (int)K; a.R = (int)T;
+        ob_launch_tgemm<false, false, OB_TX_NONE, OB_TX_SCALE_I, OB_TE_STE>(a, s);
+        if ((rc = ob_launch_status("train_backward(grad weight)"))) return rc;
+    }
+    return 0;
 }
 
 extern "C" int onebit_train_backward(const void *gy, const void *x, const void *w_latent, const void *h, const void *g,
@@ -370,10 +444,13 @@ extern "C" int onebit_train_backward(const void *gy, const void *x, const void *
     if (T == 0 || N == 0 || K == 0) return ob_fail(ONEBIT_E_SHAPE, "train_backward: empty problem");
     if (!gy || !x || !w_latent || !h || !g || !z_save || !ln_stats || !gx || !gw || !gh || !gg)
         return ob_fail(ONEBIT_E_ARG, "train_backward: null pointer");
-    if (!workspace || workspace_bytes < onebit_train_workspace_bytes(T, K, N, dtype) || !ob_aligned(workspace, 16))
-        return ob_fail(ONEBIT_E_WSPACE, "train_backward: needs %zu bytes of 16-byte aligned workspace", onebit_train_workspace_bytes(T, K, N, dtype));
+    const size_t least = onebit_train_least_workspace_bytes(T, K, N, dtype);
+    if (!workspace || workspace_bytes < least || !ob_aligned(workspace, 16))
+        return ob_fail(ONEBIT_E_WSPACE, "train_backward: needs %zu bytes of 16-byte aligned workspace", least);
     hipStream_t s = (hipStream_t)stream;
-    return dtype == ONEBIT_F16 ? ob_t16_backward(gy, x, w_latent, h, g, z_save, ln_stats, gx, gw, gh, gg, gbias_or_null, (char *)workspace, T, K, N, s)
-                               : ob_t32_backward(gy, x, w_latent, h, g, z_save, ln_stats, gx, gw, gh, gg, gbias_or_null, (char *)workspace, T, K, N, s);
+    const bool room = workspace_bytes >= onebit_train_workspace_bytes(T, K, N, dtype);
+    if (dtype == ONEBIT_F16) return ob_t16_backward(gy, x, w_latent, h, g, z_save, ln_stats, gx, gw, gh, gg, gbias_or_null, (char *)workspace, room, T, K, N, s);
+    if (workspace_bytes >= ob_train_backward_bytes(T, K, N, dtype))
+        return ob_t32_backward(gy, x, w_latent, h, g, z_save, ln_stats, gx, gw, gh, gg, gbias_or_null, (char *)workspace, room, T, K, N, s);
+    return ob_train_backward_f32(gy, x, w_latent, h, g, z_save, ln_stats, gx, gw, gh, gg, gbias_or_null, (char *)workspace, T, K, N, s);
 }
-

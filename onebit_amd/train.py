@@ -76,7 +76,11 @@ class _BitLinearFn(torch.autograd.Function):
         gb = torch.empty(N, dtype=dt, device=dev) if ctx.has_bias else None
         lib = _lib.load()
         nws = lib.onebit_train_workspace_bytes(T, K, N, ctx.code)
-        ws = torch.empty(nws, dtype=torch.uint8, device=dev)
+        try:
+            ws = torch.empty(nws, dtype=torch.uint8, device=dev)
+        except torch.OutOfMemoryError:
+            nws = lib.onebit_train_least_workspace_bytes(T, K, N, ctx.code)      # slower kernels
+            ws = torch.empty(nws, dtype=torch.uint8, device=dev)
         with torch.cuda.device(dev):
             rc = lib.onebit_train_backward(gy2.data_ptr(), x2.data_ptr(), w.data_ptr(), h.data_ptr(), g.data_ptr(), z.data_ptr(),
                                            stats.data_ptr(), gx.data_ptr(), gw.data_ptr(), gh.data_ptr(), gg.data_ptr(),

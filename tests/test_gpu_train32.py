@@ -101,3 +101,69 @@ def test_workspaces_are_bounded():
 def test_products_in_slices_of_their_steps(T, K, N):
     """Few output tiles and a long sum (csrc/onebit_train.hip, ob_train_plan): every slice walks all pairs of parts."""
     test_layer_and_gradients_against_64_bits(T, K, N)
+
+
+def _backward(T, K, N, dtype, nbytes, seed=5):
+    """Gradients of the layer of _case(T, K, N, seed) in `dtype` through the C entry with `nbytes` of workspace, between two rows of 7s."""
+    from onebit_amd import _lib
+    lib, code = _lib.load(), _lib.ONEBIT_F32 if dtype == torch.float32 else _lib.ONEBIT_F16
+    m, x, gy = _case(T, K, N, seed)
+    w, h, g, x, gy = (t.detach().to(dtype).contiguous() for t in (m.weight, m.input_factor, m.weight_scale, x, gy))
+    z, y, stats = torch.empty(T, N, dtype=dtype, device=DEV), torch.empty(T, N, dtype=dtype, device=DEV), torch.empty(T, 2, device=DEV)
+    fw = torch.empty(max(1, lib.onebit_train_forward_workspace_bytes(T, K, N, code)), dtype=torch.uint8, device=DEV)
+    out = [torch.empty(s, dtype=dtype, device=DEV) for s in ((T, K), (N, K), (K,), (N,), (N,))]
+    ws = torch.full((nbytes + 512,), 7, dtype=torch.uint8, device=DEV)
+    p, s = (lambda t: t.data_ptr()), torch.cuda.current_stream().cuda_stream
+    _lib.check(lib.onebit_train_forward_ws(p(x), p(w), p(h), p(g), None, p(y), p(z), p(stats), p(fw), fw.numel(), T, K, N, code, 1e-5, s), "forward")
+    _lib.check(lib.onebit_train_backward(p(gy), p(x), p(w), p(h), p(g), p(z), p(stats), *(p(o) for o in (out[0], out[1], out[2], out[3], out[4])),
+                                         p(ws) + 256, nbytes, T, K, N, code, s), "backward")
+    assert (ws[:256] == 7).all() and (ws[256 + nbytes:] == 7).all()
+    gx, gw, gh, gg, gb = (o.float() for o in out)
+    return m, x, gy, (gx, gw, gg, gh, gb)
+
+
+# (the sums of the float32 instruction: a rounding every four terms)
+@pytest.mark.parametrize("T,K,N", [(5, 24, 8), (33, 1000, 1000), (97, 1027, 1030), (257, 1376, 4100), (64, 4096, 1000), (1100, 516, 2050)])
+def test_backward_with_the_least_workspace(T, K, N):
+    from onebit_amd import _lib
+    lib = _lib.load()
+    need, least = (f(T, K, N, _lib.ONEBIT_F32) for f in (lib.onebit_train_workspace_bytes, lib.onebit_train_least_workspace_bytes))
+    assert least < need and least <= 4 * T * (K + N) + 8 * T + 128 * max(2 * N, K) + 1024
+    m, x, gy, got = _backward(T, K, N, torch.float32, least)
+    n = max(T, K, N)
+    for name, a, b in zip(("x", "weight", "weight_scale", "input_factor", "bias"), got, _exact(m, x, gy)[1:]):
+        off = float((a.double() - b).norm() / b.norm().clamp_min(1e-300))
+        assert off <= 2.0 ** -22 * (4 + n ** 0.5), (name, off)
+    assert lib.onebit_train_backward(*[256] * 13, least - 1, T, K, N, _lib.ONEBIT_F32, None) == -5
+
+
+# few rows, whose products run in slices given the room: one slice in what is left without it
+@pytest.mark.parametrize("T,K,N", [(64, 1000, 4096), (129, 260, 8200)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_backward_without_room_for_slices(T, K, N, dtype):
+    from onebit_amd import _lib
+    lib, code = _lib.load(), _lib.ONEBIT_F32 if dtype == torch.float32 else _lib.ONEBIT_F16
+    need = lib.onebit_train_workspace_bytes(T, K, N, code)
+    one = lib.onebit_train_least_workspace_bytes(T, K, N, code) if dtype == torch.float16 else need - 1
+    assert one < need
+    full, less = _backward(T, K, N, dtype, need)[3], _backward(T, K, N, dtype, one)[3]
+    for a, b in zip(full, less):
+        # sums in another order; float16: and the roundings of ga to it
+        assert float((a - b).norm() / b.norm()) <= (2.0 ** -22 * (4 + max(T, K, N) ** 0.5) if dtype == torch.float32 else 2.0 ** -9)
+
+
+def test_backward_without_memory_takes_the_least_workspace(monkeypatch):
+    T, K, N = 97, 1027, 1030
+    from onebit_amd import _lib
+    least = _lib.load().onebit_train_least_workspace_bytes(T, K, N, _lib.ONEBIT_F32)
+    m, x, gy = _case(T, K, N, 6)
+    y, empty = m(x), torch.empty
+
+    def little_left(*a, dtype=None, **k):
+        if dtype == torch.uint8 and a[0] > least:
+            raise torch.OutOfMemoryError("full")
+        return empty(*a, dtype=dtype, **k)
+    monkeypatch.setattr(torch, "empty", little_left)
+    got = torch.autograd.grad(y, [x, m.weight, m.weight_scale, m.input_factor, m.bias], gy)
+    for a, b in zip(got, _exact(m, x, gy)[1:]):
+        assert float((a.double() - b).norm() / b.norm()) <= 2.0 ** -22 * (4 + K ** 0.5)
