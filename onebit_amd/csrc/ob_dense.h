@@ -85,16 +85,6 @@ template <typename E> __device__ __forceinline__ float ob_xielu(float z, float a
     if constexpr (sizeof(E) == 2) em = __builtin_amdgcn_exp2f(1.4426950408889634f * n) - 1.0f; else em = expm1f(n);
     return z > 0.f ? __builtin_fmaf(a * z, z, 0.5f * z) : __builtin_fmaf(b, em - n, 0.5f * z);
 }
-// tanh in float32, within 3 ulp: below 0.8 Lambert's continued fraction cut behind x^2 / 9 (x^10 / 9.8e6 of the value), above 1 - 2 / (1 + e^2|x|) by the exp2 and
-// reciprocal instructions.  No branch and no exact division: 256 rows of 32000 capped logits
-// from 1024 columns 32.0 -> 27.9 us (a thread has 128 of them behind its last product).
-__device__ __forceinline__ float ob_tanh(float x)
-{
-    const float a = fabsf(x), q = x * x;
-    const float lo = a * __builtin_fmaf(q, q + 105.0f, 945.0f) * __builtin_amdgcn_rcpf(__builtin_fmaf(q, __builtin_fmaf(q, 15.0f, 420.0f), 945.0f));
-    const float hi = __builtin_fmaf(-2.0f, __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(2.8853900817779268f * a)), 1.0f);
-    return copysignf(a < 0.8f ? lo : hi, x);
-}
 __device__ __forceinline__ float ob_softplusf(float z) { return fmaxf(z, 0.0f) + log1pf(expf(-fabsf(z))); }
 
 // ---- what a product's output becomes -------------------------------------------------------------------------------------
@@ -191,9 +181,8 @@ __device__ __forceinline__ void ob_dense_epilogue(const ObDenseArgs &A, int nt, 
             ob_float4 v = h ? v1 : v0;
             const int n = (nt + h) * 16 + 4 * g;
             if (A.cap > 0.f) {
-                const float r = 1.0f / A.cap;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = A.cap * (sizeof(E) == 2 ? ob_tanh(v[e] * r) : tanhf(v[e] / A.cap));
+                for (int e = 0; e < 4; ++e) v[e] = A.cap * tanhf(v[e] / A.cap);
             }
             float *o = A.logits + (size_t)t * A.V + n;
             if ((A.V & 3) == 0) {
