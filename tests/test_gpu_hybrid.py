@@ -129,6 +129,23 @@ def test_prompt_with_more_splits(T):
     assert err(run(m.step_engine(1, 1300, max_rows=T), 0, 0, toks), R.forward(raw, w, toks)) < TOL[BF]
 
 
+# cap * tanh(v / cap) from the very sums that the model gives without a cap: half an ulp of a division, one of tanhf, half of a product (measured: 1.76 at most over
+# 1.5 M logits); tiny to saturated, few rows and product tiles
+@pytest.mark.parametrize("T", [5, 70, 300])
+def test_capped_logits_against_64_bits(T):
+    raw = raw_config([att()], width=64, vocab=4099, max_positions=512)
+    toks, v = tokens(T, 4099, T), None
+    for cap in (None, 1e-2, 0.3, 2.0, 30.0, 1e3):
+        m, _ = build(dict(raw, logit_softcap=cap), BF, edit=lambda w: w["head"].mul_(torch.logspace(-6, 2, 4099)[:, None]) if "head" in w else None)
+        got = run(m.step_engine(1, 512, max_rows=T), 0, 0, toks)
+        if cap is None:
+            v = got.double()
+            continue
+        c = float(torch.tensor(cap, dtype=torch.float32))
+        want = c * torch.tanh(v / c)
+        assert bool(((got.double() - want).abs() <= 2.0 * 2.0 ** -23 * want.abs()).all()), (cap, float(((got.double() - want).abs() / want.abs()).max() * 2 ** 23))
+
+
 # few rows with eight k tiles in flight per wave (from 61 k tiles a split on), every remainder of a wave's share; the others beside them
 @pytest.mark.parametrize("T", [1, 7, 16, 17])
 @DTYPES
