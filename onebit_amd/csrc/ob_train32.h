@@ -10,7 +10,7 @@
 // What bounds it: the matrix cores, 3 or 6 products for one, and below some 500 rows the length of the sums that a workgroup takes (the few tiles leave CUs idle).
 // Forward + backward, v_mfma_f32_16x16x4_f32 products (at 84-97 TFLOP/s) -> these: 3600 rows 4096 -> 4096 4336 us -> 1141 (in a trace z 1397 -> 218, ga 1243 -> 250,
 // gS 1562 -> 478), 1000 rows 1371 -> 464, 64 rows 554 -> 327, 512 rows 4096 -> 11008 1995 -> 883, 3600 rows 1376 -> 4100 1774 -> 581, 64 rows 1024 -> 2816 250 -> 170.
-// Off the 64-bit results, norms, before / now: y 1.2e-6 / 9e-8, gx 1.1e-6 / 9e-8, gW 1.1e-6 / 3.8e-7 (3600 rows; 64 rows 1.75e-7 / 1.1e-7), the scales' 1.2e-6 / 1.6e-7.
+// Off the 64-bit results, norms, before / now: y 1.2e-6 / 9e-8, gx 1.1e-6 / 9e-8, gW 1.1e-6 / 3.8e-7 (3600 rows; 64 rows 4096 -> 1000 2.1e-7 / 9.5e-8, 2 rows 1024 -> 1000 1.23e-7 / 1.18e-7), the scales' 1.2e-6 / 1.6e-7.
 #pragma once
 #include "ob_train16.h"
 
@@ -152,11 +152,25 @@ struct ObT32Mm {
     float *zp; size_t zld; int ns; // OB_T16_PART: as in ObT16Mm; the parts have as many steps
 };
 
-// 1.001 - tanh(w)^2 (bitnet.py:22-23) as 0.001 + 4 e / (1 + e)^2, e = exp(-2 |w|): nothing cancels, 3e-7 of the value
+// 1.001 - tanh(w)^2 (bitnet.py:22-23), no farther from 64 bits anywhere than 1.001f - tanhf(w)^2, whose 1.001f alone is 4.7e-8 off: 0.001 is added last.  Below 0.8, with
+// latent weights, 1 - w^2 P(w^2), P fitted to tanh(w)^2 / w^2 (4.3e-9 of 1 left); above 4 e / (1 + e)^2, e = exp(-2 |w|), where nothing cancels.  Root mean square and
+// largest error at |w| in 0-0.02, 0.25-0.5, 0.5-0.8, 0.8-1, 2.5-4: 1.001f - tanhf(w)^2 5.8e-8 / 1.1e-7, 5.2e-8 / 1.2e-7, 6.7e-8 / 2.1e-7, 7.5e-8 / 2.2e-7, 9e-8 / 2.5e-7; the last
+// form everywhere 7.1e-8 / 3.3e-7, 7.1e-8 / 2.8e-7, 6.0e-8 / 2.6e-7, 4.9e-8 / 2.1e-7, 2e-9 / 1e-8; the two 3.9e-8 / 7.7e-8, 2.2e-8 / 5.6e-8, 2.5e-8 / 8.4e-8, as it, as it.
+__device__ __forceinline__ float ob_t32_ste_small(float w)
+{
+    const float q = w * w;
+    float p = __builtin_fmaf(0.00799220707f, q, -0.0359845459f);
+    p = __builtin_fmaf(p, q, 0.0928287283f);
+    p = __builtin_fmaf(p, q, -0.195705429f);
+    p = __builtin_fmaf(p, q, 0.377643019f);
+    p = __builtin_fmaf(p, q, -0.666660547f);
+    p = __builtin_fmaf(p, q, 1.0f);
+    return __builtin_fmaf(-q, p, 1.0f) + 0.001f;
+}
 __device__ __forceinline__ float ob_t32_ste(float w)
 {
-    const float e = __builtin_amdgcn_exp2f(-2.8853900817779268f * fabsf(w)), d = 1.0f + e;
-    return 0.001f + 4.0f * e * __builtin_amdgcn_rcpf(d * d);
+    const float a = fabsf(w), e = __builtin_amdgcn_exp2f(-2.8853900817779268f * a), d = 1.0f + e;
+    return a < 0.8f ? ob_t32_ste_small(w) : 4.0f * e * __builtin_amdgcn_rcpf(d * d) + 0.001f;
 }
 
 // as ob_t16_epilogue; x / W beside an output are requested 8 tiles ahead
@@ -198,6 +212,18 @@ __device__ __forceinline__ void ob_t32_epilogue(const ObT32Mm &A, int n0, int t0
 #pragma unroll
             for (int e = 0; e < 4; ++e) { if (e < left) h4[e] = A.vec[n + e]; if (jb == 0) sum[e] = 0.f; }
         }
+        if (EPI == OB_T16_GW) {                                        // W -> its factors
+            float most = 0.f;
+#pragma unroll
+            for (int j = 0; j < 4 * JB; ++j) most = fmaxf(most, fabsf(p[b & 1][j >> 2][j & 3]));
+            if (__builtin_amdgcn_ballot_w64(most >= 0.8f)) {           // (uniform)
+#pragma unroll
+                for (int j = 0; j < 4 * JB; ++j) p[b & 1][j >> 2][j & 3] = ob_t32_ste(p[b & 1][j >> 2][j & 3]);
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4 * JB; ++j) p[b & 1][j >> 2][j & 3] = ob_t32_ste_small(p[b & 1][j >> 2][j & 3]);
+            }
+        }
 #pragma unroll
         for (int j = 0; j < JB; ++j) {
             const int t = t0 + (jb + j) * 16 + lr;
@@ -210,10 +236,7 @@ __device__ __forceinline__ void ob_t32_epilogue(const ObT32Mm &A, int n0, int t0
                 for (int e = 0; e < 4; ++e) sum[e] += c[e] * d[e];
                 c = c * h4;
             }
-            if (EPI == OB_T16_GW) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) c[e] *= ob_t32_ste(d[e]);
-            }
+            if (EPI == OB_T16_GW) c = c * d;
             if (v4) *reinterpret_cast<ob_float4 *>(A.C + o) = c;
             else {
 #pragma unroll

@@ -167,3 +167,27 @@ def test_backward_without_memory_takes_the_least_workspace(monkeypatch):
     got = torch.autograd.grad(y, [x, m.weight, m.weight_scale, m.input_factor, m.bias], gy)
     for a, b in zip(got, _exact(m, x, gy)[1:]):
         assert float((a.double() - b).norm() / b.norm()) <= 2.0 ** -22 * (4 + K ** 0.5)
+
+
+# the straight-through factor alone: the gradient over that of a layer of the same signs whose weights' factor is 1.001f
+@pytest.mark.parametrize("lo,hi,rms,most", [(0, 0.02, 5.8e-8, 1.1e-7), (0.1, 0.25, 5.0e-8, 1.1e-7), (0.25, 0.5, 5.2e-8, 1.3e-7), (0.5, 0.8, 6.7e-8, 2.1e-7), (0.8, 1.0, 7.5e-8, 2.2e-7),
+                                            (1.0, 2.5, 8.2e-8, 2.4e-7), (2.5, 9.0, 9.1e-8, 2.6e-7)])
+def test_straight_through_factor_against_64_bits(lo, hi, rms, most):
+    """Errors of 1.001f - tanhf(w)^2 (root mean square, largest) are the bounds, and either gradient's rounding (half an ulp at most, 0.42 in the mean square)."""
+    from onebit_amd.train import BitLinear
+    T, K, N = 64, 1024, 1000
+    g = torch.Generator(device=DEV).manual_seed(3)
+    w = lo + (hi - lo) * torch.rand(N, K, generator=g, device=DEV)
+    x, gy = torch.randn(T, K, generator=g, device=DEV), torch.randn(T, N, generator=g, device=DEV)
+    out = []
+    for latent in (w, torch.full_like(w, 1e-30)):                      # the same signs: the same gz and a
+        m = BitLinear(K, N, device=DEV, dtype=torch.float32)
+        with torch.no_grad():
+            m.weight.copy_(latent), m.weight_scale.fill_(1.0), m.input_factor.fill_(1.0)
+        out.append(torch.autograd.grad(m(x), m.weight, gy)[0].double())
+    base = out[1] / float(torch.tensor(1.001, dtype=torch.float32))
+    keep = base.abs() > 1e-3 * base.abs().mean()
+    f = (1.001 - torch.tanh(w.double()) ** 2)[keep]
+    off, room = (out[0] / base)[keep] - f, 2.0 ** -24 * f
+    assert float((off.abs() - 2 * room).max()) <= most, float((off.abs() - 2 * room).max())
+    assert float(off.square().mean().sqrt()) <= (rms ** 2 + 2 * float((0.45 * room).square().mean())) ** 0.5, float(off.square().mean().sqrt())
