@@ -568,7 +568,8 @@ extern "C" int onebit_linear_forward(const void *packed, int64_t ldw_bytes, cons
                 if (skip && ubuf != y) (void)hipMemcpyAsync(y, ubuf, (size_t)T * N * 2, hipMemcpyDeviceToDevice, s);
             }
         };
-        const int few = !prescaled && !tile_stats && (!bias || ob_aligned(bias, 16)) && ob_aligned(g, 16) && ob_skinny_ok(packed, ldw_bytes, T, K) ? ob_skinny_slices(T, K, N) : 1;
+        const bool rows16 = ob_aligned(ubuf, 16) && (!bias || ob_aligned(bias, 16));       // (for ob_ln_rows_kernel's vectors; y is)
+        const int few = !prescaled && !tile_stats && rows16 && ob_aligned(g, 16) && ob_skinny_ok(packed, ldw_bytes, T, K) ? ob_skinny_slices(T, K, N) : 1;
         const bool pad = !prescaled && ob_g3_padded(T, K, N) != 0;
         const int64_t kp = pad ? ob_g3_padded(T, K, N) : K;
         if (K == 0) {
@@ -625,7 +626,7 @@ extern "C" int onebit_linear_forward(const void *packed, int64_t ldw_bytes, cons
             }
             onebit_proj_t pj = {};
             pj.weight = W; pj.input_factor = h; pj.weight_scale = g; pj.N = N; pj.K = kp; pj.ldw_bytes = ldw;
-            const int ns = tile_stats || (bias && !ob_aligned(bias, 16)) || ob_linear_slices(T, kp, N) == 1 ? 0 : ob_gemm3_ksplit_n(pj, T);
+            const int ns = tile_stats || !rows16 || ob_linear_slices(T, kp, N) == 1 ? 0 : ob_gemm3_ksplit_n(pj, T);
             const size_t a_bytes = pad ? ob_pad_bytes(T, kp, N) : ob_align256((size_t)T * (size_t)K * 2), z_bytes = ob_align256((size_t)T * (size_t)N * 4);
             if (ns > 0 && workspace_bytes >= a_bytes + (size_t)ns * z_bytes) {
                 float *zs[4] = {nullptr, nullptr, nullptr, nullptr};

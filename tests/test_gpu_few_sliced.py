@@ -47,3 +47,27 @@ def test_layer(T, K, N, bias):
         assert ((u2.double() - z * gs).abs() <= 2.01 * 2.0 ** -11 * (z * gs).abs() + err * gs.abs() + 2.0 ** -24).all()
         if n:
             assert torch.equal(u2, u) and torch.equal(y2, y)
+
+
+# a second output that no 16-byte store can take, a bias that no 16-byte load can: the kernels that ask for neither, the same layer
+@pytest.mark.parametrize("T,K,N", [(18, 11008, 4096), (100, 11008, 4096), (130, 2816, 1000)])
+@pytest.mark.parametrize("what", ["u", "bias"])
+def test_unaligned_second_output_and_bias(T, K, N, what):
+    g = torch.Generator(device="cuda").manual_seed(T)
+    w = torch.randint(0, 256, (N, K // 8), generator=g, device="cuda", dtype=torch.uint8)
+    h, scale, bias = (0.1 + torch.rand(n, generator=g, device="cuda").half() for n in (K, N, N))
+    x = torch.randn(T, K, generator=g, device="cuda").half()
+    lib, s, p = _lib.load(), torch.cuda.current_stream().cuda_stream, lambda t: t.data_ptr()
+    n = lib.onebit_linear_workspace_bytes(T, K, N, _lib.ONEBIT_F16)
+    ws, res = torch.empty(n, dtype=torch.uint8, device="cuda"), []
+    for off in (0, 1):
+        u, b = torch.full((T * N + 16,), 7.0, dtype=torch.float16, device="cuda"), torch.empty(N + 8, dtype=torch.float16, device="cuda")
+        uo, bo = off if what == "u" else 0, off if what == "bias" else 0
+        b[bo:bo + N] = bias
+        y = torch.empty(T, N, dtype=torch.float16, device="cuda")
+        _lib.check(lib.onebit_linear_forward(p(w), K // 8, p(x), p(h), p(scale), p(b) + 2 * bo, p(y), p(u) + 2 * uo, p(ws), n, T, K, N, _lib.ONEBIT_F16, 1e-5, 0, s), "forward")
+        assert bool((u[:uo] == 7).all()) and bool((u[uo + T * N:] == 7).all())
+        res.append((u[uo:uo + T * N].double(), y.double()))
+    # sums in another order: a rounding to float16 apart here and there
+    for a, b in zip(*res):
+        assert float((a - b).norm() / a.norm()) <= 2.0 ** -10
