@@ -86,6 +86,7 @@ struct ObF32Gemm {
     const char *planes;
     float *z, *zt; long long zt_split; int ld_t;
     int T, N, quads, tb, nb_full, nb_all, S;
+    int columns;                               // whole tiles numbered columns first
 };
 
 template <int WN, int WT, int NW, int TW, int KS, int NST>
@@ -98,17 +99,19 @@ __global__ __launch_bounds__(256, 2) void ob_f32_gemm_kernel(const ObF32Gemm A)
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wn = wave % WN, wt = wave / WN, r = lane & 15, gq = lane >> 4;
     // whole tiles first, then the splits; each part dealt to the 8 XCDs in contiguous ranges.  A column block's packed rows are 1/48 of a token block's parts: the
-    // tiles in flight on an XCD are all the columns of a token block or two.  Up to 8 token blocks (whose parts its range needs anyway), and among
-    // the splits, it is the token blocks that come first, so that an XCD reads its own columns' packed rows alone.  Token blocks first -> as it is, whole call: 5500 rows 4096 -> 4096 750 -> 452 us (2.9 GB
-    // of parts through the L2s, 0.13 now), 16000 rows 1024 -> 2816 453 -> 312, 2000 rows 4096 -> 11008 446 -> 413, 1300 rows 4096 -> 4096 (11 blocks) 141 -> 136;
-    // 731 rows 4096 -> 11008 (6) 152.4 either way, 130 rows (3) 74.0 -> 75.3; splits alone, 1100 rows 1024 -> 2816, 40.4 -> 41.3.
+    // tiles in flight on an XCD are all the columns of a token block or two.  The token blocks come first, so that an XCD reads its own columns' packed rows alone, among
+    // the splits, up to 8 token blocks (whose parts its range needs anyway), and where all tiles run at once and the parts are 9 MB at most, little enough for the L2s.
+    // Token blocks first -> columns first, whole call: 5500 rows 4096 -> 4096 750 -> 452 us (2.9 GB of parts through the L2s, 0.13 now), 16000 rows 1024 -> 2816 453 -> 312,
+    // 2000 rows 4096 -> 11008 446 -> 413, 1300 rows 4096 -> 4096 (11 blocks) 141 -> 136, 9000 rows 64 -> 1024 (568 tiles) 50.4 -> 44.8; 731 rows 4096 -> 11008 (6) 152.4 either
+    // way, 130 rows (3) 74.0 -> 75.3; splits alone, 1100 rows 1024 -> 2816, 40.4 -> 41.3; 2000 rows 64 -> 4096 (512 tiles, 0.8 MB) 38.1 -> 44.0, 2871 rows 256 -> 2048
+    // (368, 4.4 MB) 34.4 -> 37.9, 1409 rows 512 -> 4096 (384, 4.3 MB) 38.7 -> 42.3.
     const int nfull = A.nb_full * A.tb;
     const bool tail = (int)blockIdx.x >= nfull;
     const int nwg = tail ? (int)gridDim.x - nfull : nfull, orig = (int)blockIdx.x - (tail ? nfull : 0);
     const int xcd = orig & 7, q8 = nwg >> 3, rem = nwg & 7;
     int bid = (xcd < rem ? xcd * (q8 + 1) : rem * (q8 + 1) + (xcd - rem) * q8) + (orig >> 3);
     int tblk, nblk, split = 0;
-    if (!tail && A.tb > 8) { nblk = bid % A.nb_full; tblk = bid / A.nb_full; }
+    if (!tail && A.columns) { nblk = bid % A.nb_full; tblk = bid / A.nb_full; }
     else {
         tblk = bid % A.tb;
         bid /= A.tb;

@@ -79,6 +79,7 @@ static void ob_f32_rows(const ObF32Plan &p, const void *packed, int64_t ldw_byte
     a.W = (const char *)packed; a.ldw = ldw_bytes;
     a.planes = planes; a.z = y; a.zt = zt; a.zt_split = (long long)T * p.ld_t; a.ld_t = p.ld_t;
     a.T = (int)T; a.N = (int)N; a.quads = p.quads; a.tb = p.tb; a.nb_full = p.nb_full; a.nb_all = p.nb; a.S = p.S;
+    a.columns = p.tb > 8 && ((int64_t)p.nb * p.tb > 2 * (int64_t)ob_cu_count() || T * K * 6 > 9000000);
     if (p.bt == 16) ob_launch_f32_gemm<4, 1, 2, 1, 4, 4>(a, s);
     else if (p.bt == 32) ob_launch_f32_gemm<4, 1, 2, 2, 2, 4>(a, s);
     else if (p.bt == 64) ob_launch_f32_gemm<2, 2, 4, 2, 1, 4>(a, s);

@@ -51,7 +51,8 @@ def test_rows_against_64_bits(T, K, N):
     _check(m, torch.randn(T, K, generator=g, device="cuda"))
 
 
-# both numberings of the tiles: up to 8 blocks of 128 rows the token blocks come first, beyond it the columns; with and without whole rounds, a split rest in both
+# both numberings of the tiles: the token blocks first up to 8 blocks of 128 rows, beyond it where all tiles run at once on small parts (264 -> 4100), else the columns;
+# with and without whole rounds, a split rest in both
 @pytest.mark.parametrize("T", [1024, 1025, 1409, 2100])
 @pytest.mark.parametrize("K,N", [(264, 4100), (512, 9000), (256, 16388)])
 def test_many_token_blocks_against_64_bits(T, K, N):
