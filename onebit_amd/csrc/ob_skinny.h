@@ -20,8 +20,9 @@
 #pragma once
 #include "ob_common.h"
 
-// Up to 4 projections that share the activations (q|k|v, gate|up) ride in one launch: workgroup b
+// Up to NP = 3 projections that share the activations (q|k|v, gate|up) ride in one launch: workgroup b
 // belongs to the projection whose tile range contains b (entries without a range of their own: copies of the last one).
+// NP = 4: slices of one.  (Four for all would be 1 % of a launch: 13 rows 4096 -> 11008 13.95 -> 14.09 us.)
 // An entry may also be a K-slice of a projection (W, h, x advanced to the slice, K = its length,
 // PARTIAL output): split-K over workgroups for short-and-wide layers (down_proj), summed by the consumer.
 struct ObSkinnyProj {
@@ -35,12 +36,14 @@ struct ObSkinnyProj {
                                   // (ob_decode.h ObTileStats layout), token stride ob_tile_stats_floats(N); N % 16 == 0
 };
 __host__ __device__ __forceinline__ int ob_tile_stats_floats(int n) { return ((n + 4095) >> 12) * 512; }
-struct ObSkinnyArgs {
-    ObSkinnyProj p[4];
+template <int NP>
+struct ObSkinnyArgsOf {
+    ObSkinnyProj p[NP];
     long long ldx;
     int T;
     unsigned long long *dbg;      // -DOB_PROFILE_STAMPS builds: 16 cycle stamps per wave (tools/skinny_phase_probe.py)
 };
+typedef ObSkinnyArgsOf<3> ObSkinnyArgs;
 
 // tokens x k elements of one phase: 16*RT x 512 (42 / 75 / 142 KB of LDS with the packed rows: three,
 // two or one workgroup per CU)
@@ -57,8 +60,8 @@ struct ObSkinnyArgs {
 // ob_skinny3.h is the form without either, for producer-scaled rows.)
 #define OB_SKINNY_LDS2(RT_, RNT_) ((size_t)2 * 16 * (RT_) * (OB_SKINNY_PK(RT_) + 8) * 2 + (size_t)2 * 16 * (RNT_) * (OB_SKINNY_PK(RT_) / 32 + 1) * 4)
 
-template <bool PARTIAL, int RT, int RNT = 4>
-__global__ __launch_bounds__(512) void ob_skinny_f16_kernel(const ObSkinnyArgs A)
+template <bool PARTIAL, int RT, int RNT = 4, int NP = 3>
+__global__ __launch_bounds__(512) void ob_skinny_f16_kernel(const ObSkinnyArgsOf<NP> A)
 {
     constexpr int ROWS = 16 * RNT;
 #ifdef OB_PROFILE_STAMPS
@@ -68,8 +71,8 @@ __global__ __launch_bounds__(512) void ob_skinny_f16_kernel(const ObSkinnyArgs A
 #define OB_SK_STAMP(i) do { } while (0)
 #endif
     OB_SK_STAMP(0);
-    const int pi = (int)blockIdx.x < A.p[0].tile_end ? 0 : ((int)blockIdx.x < A.p[1].tile_end ? 1 : ((int)blockIdx.x < A.p[2].tile_end ? 2 : 3));
-    const ObSkinnyProj P = pi == 0 ? A.p[0] : (pi == 1 ? A.p[1] : (pi == 2 ? A.p[2] : A.p[3]));
+    const int pi = (int)blockIdx.x < A.p[0].tile_end ? 0 : ((int)blockIdx.x < A.p[1].tile_end ? 1 : (NP == 3 || (int)blockIdx.x < A.p[2].tile_end ? 2 : NP - 1));
+    const ObSkinnyProj P = pi == 0 ? A.p[0] : (pi == 1 ? A.p[1] : (NP == 3 || pi == 2 ? A.p[2] : A.p[NP - 1]));
     const uint32_t *__restrict__ W = P.W;
     const int64_t ldw_words = P.ldw_words, ldx = A.ldx;
     const _Float16 *__restrict__ x = P.x, *__restrict__ h = P.h, *__restrict__ g = P.g;
@@ -77,7 +80,7 @@ __global__ __launch_bounds__(512) void ob_skinny_f16_kernel(const ObSkinnyArgs A
     float *__restrict__ zp = P.zp;
     float *__restrict__ stp = P.st;
     const int T = A.T, K = P.K, N = P.N;
-    const int tile0 = pi == 0 ? 0 : (pi == 1 ? A.p[0].tile_end : (pi == 2 ? A.p[1].tile_end : A.p[2].tile_end));
+    const int tile0 = pi == 0 ? 0 : (pi == 1 ? A.p[0].tile_end : (NP == 3 || pi == 2 ? A.p[1].tile_end : A.p[2].tile_end));
     constexpr int PK = OB_SKINNY_PKT(RT) / RT;  // k elements per phase
     constexpr int CPP = PK / 512;               // 512-weight chunks per phase
     constexpr int TT = 16 * RT;                 // tokens of the tile

@@ -190,17 +190,17 @@ static unsigned long long *ob_dbg_buffer()
 }
 #endif
 
-template <bool PARTIAL, int RT, int RNT = 4>
-static void ob_launch_skinny(const ObSkinnyArgs &ka_in, int tiles, hipStream_t s)
+template <bool PARTIAL, int RT, int RNT = 4, int NP = 3>
+static void ob_launch_skinny(const ObSkinnyArgsOf<NP> &ka_in, int tiles, hipStream_t s)
 {
-    ObSkinnyArgs ka = ka_in;
+    ObSkinnyArgsOf<NP> ka = ka_in;
 #ifdef OB_PROFILE_STAMPS
     ka.dbg = ob_dbg_buffer();
 #endif
     const size_t lds = OB_SKINNY_LDS2(RT, RNT) > (size_t)RT * 32768 ? OB_SKINNY_LDS2(RT, RNT) : (size_t)RT * 32768;
     static bool attr_set[OB_MAX_DEVICES] = {};
-    ob_set_max_lds_once(ob_skinny_f16_kernel<PARTIAL, RT, RNT>, attr_set, (int)lds);
-    hipLaunchKernelGGL((ob_skinny_f16_kernel<PARTIAL, RT, RNT>), dim3((unsigned)tiles), dim3(512), lds, s, ka);
+    ob_set_max_lds_once(ob_skinny_f16_kernel<PARTIAL, RT, RNT, NP>, attr_set, (int)lds);
+    hipLaunchKernelGGL((ob_skinny_f16_kernel<PARTIAL, RT, RNT, NP>), dim3((unsigned)tiles), dim3(512), lds, s, ka);
 }
 
 static inline bool ob_skinny_ok(const void *packed, int64_t ldw_bytes, int64_t T, int64_t K)
@@ -233,7 +233,7 @@ static void ob_launch_mm16(const void *packed, int64_t ldw_bytes, const void *x,
             ka.p[0] = {(const uint32_t *)packed, (long long)(ldw_bytes / 4), (const _Float16 *)h,              \
                        (const _Float16 *)g, (const _Float16 *)x, (_Float16 *)u, zp, (int)N, (int)K,            \
                        (int)((N + 63) / 64)};                                                                  \
-            ka.p[1] = ka.p[0]; ka.p[2] = ka.p[0]; ka.p[3] = ka.p[0];                                           \
+            ka.p[1] = ka.p[0]; ka.p[2] = ka.p[0];                                                              \
             ka.ldx = ldx; ka.T = (int)T;                                                                       \
             ob_launch_skinny<PARTIAL, RT_>(ka, ka.p[0].tile_end, s);                                           \
         } while (0)
@@ -466,7 +466,7 @@ static void ob_launch_skinny_slices(const void *packed, int64_t ldw_bytes, const
                                     hipStream_t s)
 {
     const int tiles = (int)((N + 63) / 64), phases = (int)((K + 511) / 512);
-    ObSkinnyArgs ka = {};
+    ObSkinnyArgsOf<4> ka = {};
     for (int j = 0; j < 4; ++j) {
         if (j >= ns) { ka.p[j] = ka.p[j - 1]; continue; }
         const int64_t k0 = (int64_t)(phases * j / ns) * 512, k1 = std::min<int64_t>(K, (int64_t)(phases * (j + 1) / ns) * 512);
