@@ -649,8 +649,9 @@ extern "C" int onebit_linear_forward(const void *packed, int64_t ldw_bytes, cons
                                           "(workspace for the pre-scaled rows missing?)");
         if (skip && ubuf == y) return 0;
         static const int ln_v3 = getenv("OB_LN_ROWS") ? atoi(getenv("OB_LN_ROWS")) : 1;           // A/B: 0 = ob_layernorm_rows_kernel
-        // (N % 8 == 4, whatever the rows: else one value a lane and load in three passes; a call of 18 rows 1376 -> 4100 17.2 -> 13.6 us)
-        if (ln_v3 && !skip && ((T >= 64 && N % 8 == 0) || N % 8 == 4) && N <= OB_DEC_MAXV * OB_DEC_THREADS * 8 && ob_aligned(ubuf, 16) && (!bias || ob_aligned(bias, 16))) {
+        // (N % 8 == 4: else one value a lane and load in three passes; a call of 18 rows 1376 -> 4100 17.2 -> 13.6 us, 8000 rows 128 -> 500 23.6 -> 20.4.  Rows of few values
+        // leave most of a workgroup idle: thousands of them stay there, 4000 / 8000 rows 128 -> 44 12.0 / 14.7 -> 12.8 / 16.3 us, 128 -> 132 13.3 / 17.1 -> 13.2 / 16.9)
+        if (ln_v3 && !skip && ((T >= 64 && N % 8 == 0) || (N % 8 == 4 && (N >= 128 || T <= 1024))) && N <= OB_DEC_MAXV * OB_DEC_THREADS * 8 && ob_aligned(ubuf, 16) && (!bias || ob_aligned(bias, 16))) {
             ObLnRowsArgs la = {};
             la.uin = (const _Float16 *)ubuf; la.bias = (const _Float16 *)bias; la.y = (_Float16 *)y; la.N = (int)N; la.eps = ln_eps;
             ob_launch_ln_rows<false>(la, T, s);

@@ -64,3 +64,11 @@ def test_partial_of_a_slice(T, K, N, pitch):
         _lib.check(lib.onebit_matmul_partial_ws(m.weight.data_ptr(), K // 8, x.data_ptr(), pitch, m.input_factor.data_ptr(), out.data_ptr(),
                                                 None if w is None else w.data_ptr(), 0 if w is None else w.numel(), T, K, N, _lib.ONEBIT_F16, s), "partial")
         assert ((out.double() - z).abs() <= err + 2.0 ** -24).all()
+
+
+# few columns, N % 8 == 4: rows of eight values a load up to 1024 of them and from 128 columns on, beside the other form
+@pytest.mark.parametrize("T", [1024, 1025])
+@pytest.mark.parametrize("N", [12, 124, 132])
+@pytest.mark.parametrize("bias", [False, True])
+def test_rows_of_few_values(T, N, bias):
+    test_layer(T, 128, N, bias)
