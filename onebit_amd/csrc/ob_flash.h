@@ -72,9 +72,10 @@ struct ObFlashRaggedArgs {
     int nseg;
     int hg;                   // 0: pairs of query blocks; else single blocks, numbered over groups of hg heads (set by ob_fl_number)
     int snake;                // single blocks, all resident at once: the lighter half comes lightest first
-    int levels, per_head;     // nonzero: single blocks numbered by length over all segments, hg = H / 8 heads an XCD: the longest's length in blocks of queries; a head's blocks
     int wg_end[OB_FL_MAXSEG];
     ObFlashSeg seg[OB_FL_MAXSEG];
+    int levels, per_head;     // nonzero: single blocks numbered by length over all segments, hg = H / 8 heads an XCD: the longest's length in blocks of queries; a head's blocks
+                              // (behind the tables: in front of them a launch over one segment of 308 rows is 12.4 -> 13.2 us)
 };
 
 // How scores become weights.  The kernel below is written once for all:
@@ -211,14 +212,15 @@ __device__ __forceinline__ float ob_fl_col_sum(float v)
 #endif
 
 // SINGLE: a workgroup has one query block (ObFlashRaggedArgs::hg), no pair -- a kernel of its own: the pairs' loop is 1-4 % slower with the choice in it
-template <int D, bool RAGGED = false, class POL = ObFlSoftmaxF16, bool SINGLE = false>
+// LEVELS: its number by length over all segments (ObFlashRaggedArgs::levels) -- likewise, so that the other numberings' code is what it is without it
+template <int D, bool RAGGED = false, class POL = ObFlSoftmaxF16, bool SINGLE = false, bool LEVELS = false>
 __global__ __launch_bounds__(256, 2) void ob_flash_fwd_kernel(const std::conditional_t<RAGGED, typename POL::RaggedArgs, ObFlashArgs> AA)
 {
     typedef typename POL::H H16;
     typedef typename POL::V8 V8;
     constexpr bool SM = POL::SOFTMAX;
     constexpr bool B16 = POL::BF16;
-    static_assert(RAGGED || !(B16 || SINGLE), "the bf16 forms and single blocks have ragged rows only");
+    static_assert((RAGGED || !(B16 || SINGLE)) && (SINGLE || !LEVELS), "the bf16 forms and single blocks have ragged rows only");
     const ObFlashArgs &A = [&]() -> const ObFlashArgs & { if constexpr (RAGGED) return AA.a; else return AA; }();
     constexpr int DT = D / 16, DK = D / 32;
     constexpr int NPC = D / 8;                  // 16-byte pieces per K / V row
@@ -249,7 +251,7 @@ __global__ __launch_bounds__(256, 2) void ob_flash_fwd_kernel(const std::conditi
     int npair, pj, head, b, S, past, nmb;
     int64_t qrow0;                                // first token row of this sequence's queries in q / o
     if constexpr (RAGGED) {
-        if (SINGLE && AA.levels) {
+        if constexpr (LEVELS) {
             // the r-th longest block of a head: lane l has segment l, whose `cnt` blocks are top, top - 1, .. long (in blocks of queries; all sums exact)
             int j = orig >> 3;
             if (AA.snake && j >= AA.snake) j = AA.per_head * AA.hg - 1 - (j - AA.snake);
@@ -666,6 +668,7 @@ __global__ __launch_bounds__(256, 2) void ob_flash_fwd_kernel(const std::conditi
 template <int D, class POL = ObFlSoftmaxF16>
 inline void ob_fl_launch(const typename POL::RaggedArgs &a, int64_t wgs, hipStream_t s)
 {
-    if (a.hg) hipLaunchKernelGGL((ob_flash_fwd_kernel<D, true, POL, true>), dim3((unsigned)wgs), dim3(OB_FL_THREADS), 0, s, a);
+    if (a.levels) hipLaunchKernelGGL((ob_flash_fwd_kernel<D, true, POL, true, true>), dim3((unsigned)wgs), dim3(OB_FL_THREADS), 0, s, a);
+    else if (a.hg) hipLaunchKernelGGL((ob_flash_fwd_kernel<D, true, POL, true>), dim3((unsigned)wgs), dim3(OB_FL_THREADS), 0, s, a);
     else hipLaunchKernelGGL((ob_flash_fwd_kernel<D, true, POL>), dim3((unsigned)wgs), dim3(OB_FL_THREADS), 0, s, a);
 }
