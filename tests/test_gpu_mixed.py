@@ -299,18 +299,21 @@ def test_mixed_step_at_13b_widths_chunked_prompts_next_to_decoding_slots():
         assert out[rid] == ref or _near_tie(model, p, ref, out[rid], dev), rid
 
 
-@pytest.mark.parametrize("hidden,inter,heads,rows", [(5120, 13824, 40, 543), (5120, 13824, 40, 700), (4096, 11008, 32, 700),
-                                                     (5120, 13824, 40, 95), (5120, 13824, 40, 200), (4096, 11008, 32, 131), (4096, 11008, 32, 65)])
-def test_mixed_step_mid_size_routes(hidden, inter, heads, rows):
-    """A few hundred rows at 13B / 7B widths (7B down_proj: K = 11008 splits into 5632 + 5376): q|k|v and gate|up take pre-scaled rows because the GROUP fills the chip (ob_gemm3_group_ok),
-    o_proj / down_proj run as two K-slices whose fp32 sums the next row kernel adds (ob_gemm3_ksplit2); 65 .. 320 rows: every projection
-    as balanced passes of <= 64 rows through the LDS-DMA skinny GEMM.  Logits of the prompt's last row and of the decode rows against
-    the module path."""
+@pytest.mark.parametrize("hidden,inter,heads,kv,rows", [
+    (5120, 13824, 40, 40, 543), (5120, 13824, 40, 40, 700), (4096, 11008, 32, 32, 700), (5120, 13824, 40, 40, 95), (5120, 13824, 40, 40, 200), (4096, 11008, 32, 32, 131),
+    (4096, 11008, 32, 32, 65), (4096, 11008, 32, 32, 100), (4096, 11008, 32, 32, 128), (5120, 13824, 40, 40, 113), (768, 2048, 12, 12, 130), (512, 1408, 8, 8, 250),
+    (2048, 5632, 16, 1, 300), (4096, 11008, 32, 1, 700), (512, 2816, 8, 8, 780)])
+def test_mixed_step_mid_size_routes(hidden, inter, heads, kv, rows):
+    """What a few hundred rows' products run as, by the estimates of their times (onebit_mixed.hip, gemm_group).  Width 4096 and 5120: gate | up in one LDS-DMA launch, o and
+    down in two to four K slices that the next row kernel adds (o of 700 rows whole); q | k | v in one launch, at 97 to 128 rows in passes of at most 64 rows of the
+    skinny product, at 543 and 700 rows the last few by such a pass.  Width 768 and 512: passes for everything up to 320 rows but the long down projection's slices; 780
+    rows: gate | up as a group of half a round of workgroups, the others one launch each.  One key head of 128 columns: it rides in the group of q.  Logits of the
+    prompt's last row and of the decode rows against the module path."""
     from onebit_amd.llama import OneBitLlamaConfig, build_synthetic_model
     from onebit_amd.engine import MixedStep
     dev = torch.device(DEV)
     cfg = OneBitLlamaConfig(vocab_size=512, hidden_size=hidden, intermediate_size=inter, num_hidden_layers=2,
-                            num_attention_heads=heads, max_position_embeddings=1024)
+                            num_attention_heads=heads, num_key_value_heads=kv, max_position_embeddings=1024)
     model = build_synthetic_model(cfg, seed=29, device=dev)
     slots, max_len, n_dec = 4, 800, 3
     shape = (slots, cfg.num_key_value_heads, max_len, cfg.head_dim)
