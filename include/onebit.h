@@ -88,12 +88,14 @@ int onebit_unpack_signs(const void *packed, void *out, int dtype, int64_t N, int
  *   onebit_linear_workspace_bytes() bytes, 16-byte aligned.  Required only for
  *   F16 with K % 32 != 0 (fp32 z).  Otherwise optional; smaller or NULL selects
  *   a slower kernel, with the same results up to the order of fp32 sums:
- *     F16, large calls: the pre-scaled activations fp16(x*h) of the LDS-DMA GEMM;
- *     F16, a few hundred rows: those and the fp32 sums of K slices (256-byte
- *       aligned; 16 bytes selects the register-staged GEMM);
+ *     F16, from 65 rows on, K % 256 == 0: the pre-scaled activations fp16(x*h) of
+ *       the LDS-DMA GEMM, and behind them, where K slices are faster, their fp32
+ *       sums (without room for these, or with u or bias not 16-byte aligned: one
+ *       slice);
  *     F16, K % 256 != 0 (K % 32 == 0, from 65 rows on): those and the packed rows,
  *       both on the next whole number of 256 columns;
- *     F16, 2 to 64 rows, a long K and few columns: the fp32 sums of K slices;
+ *     F16, 2 to 64 rows, a long K and few columns: the fp32 sums of K slices (g, u
+ *       and bias 16-byte aligned);
  *     F32, T*K*N from 24 million on (36 if K % 256 != 0), N % 4 == 0, g / bias /
  *       u (with K % 256 == 0 the packed rows, too) 16-byte aligned: the
  *       activations' three bf16 parts and the sums of split K for the matrix
@@ -426,7 +428,9 @@ int onebit_decode_step_ksharded(const onebit_model_t *model, const onebit_kshard
  * u[i] [T, N_i] = fp16(fp16(W_i . a_i) * g_i), the pre-LayerNorm output (ONEBIT_FLAG_SKIP_LN | ONEBIT_FLAG_PRESCALED semantics of
  * onebit_linear_forward, bit-identical to it).  One launch instead of three keeps the workgroup rounds full (T = 2048, 7B: three
  * launches of 256 tiles each on 512 workgroup slots vs one of 768).  2 <= T <= 64: the LDS-DMA skinny GEMM; larger T: the LDS-DMA
- * GEMM.  Returns ONEBIT_E_SHAPE when the group is not eligible (the caller then issues one onebit_linear_forward per projection). */
+ * GEMM, for two or three projections with K % 256 == 0 and N_i % 4 == 0, 16-byte aligned rows of packed signs, if every one has K >= 1024 and
+ * N_i >= 256 (or K >= 2048 and N_i % 8 == 0), or, from T = 192 on, if together they have half as many tiles of 256 x 128 outputs as the chip has
+ * CUs.  Returns ONEBIT_E_SHAPE when the group is not eligible (the caller then issues one onebit_linear_forward per projection). */
 int onebit_linear_group_prescaled(const onebit_proj_t *projs, void *const *u, const void *const *a, int32_t n_proj, int64_t T, void *stream);
 
 /* ---- ragged token rows: several sequences in one call (continuous batching, BASELINE config 5; ABI 9) -----------------
