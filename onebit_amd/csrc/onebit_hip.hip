@@ -370,13 +370,16 @@ static bool ob_g3_fits(int64_t T, int64_t K, int64_t N)
     return env3 && K > 0 && K % (4 * OB_G2_K) == 0 && N > 0 && N % 4 == 0 && T * K * 2 < ((int64_t)1 << 32) && N * (K / 8) < ((int64_t)1 << 32);
 }
 // From 65 rows on, and 1024 columns of K: fewer are few steps behind a launch's constant, and the 128 x 128 kernel needs no scaled rows.  Of fewer than 256 output
-// columns, whose tiles are one beside another at most, from 2048 of K on, where K slices make up for it.  Layer calls of 65 / 700 / 2000 rows, the
-// 128 x 128 kernel -> slices: 2048 -> 128 28.6 / 29.6 / 30.8 -> 11.6 / 14.7 / 22.5 us, 4096 -> 128 48.6 / 50.2 / 51.4 -> 14.1 / 18.7 / 25.6, 11008 -> 200 118 / 122 /
-// 126 -> 23.9 / 30.5 / 42.8; 6000 rows 2048 -> 128 33.9 -> 39.2, 4096 -> 128 56.1 -> 48.6.
+// columns, whose tiles are one beside another at most, from 2048 of K on, where K slices make up for it.
 static bool ob_g3_shape(int64_t T, int64_t K, int64_t N)
 {
     return ob_g3_fits(T, K, N) && T > 64 && (N >= 256 ? K >= 1024 : N % 8 == 0 && K >= 2048);
 }
+// A layer call, which scales its rows first.  Fewer than 256 columns: the 128 x 128 kernel goes through K once whatever the rows (to 128 a CU), the scaled rows and the
+// slices' sums grow with them.  128 x 128 kernel -> slices: 65 / 700 / 2000 rows 2048 -> 128 28.6 / 29.6 / 30.8 -> 11.6 / 14.7 / 22.5 us, 11008 -> 200 118 / 122 / 126 ->
+// 23.9 / 30.5 / 42.8; 3000 / 5000 rows 2048 -> 64 31.3 / 32.5 -> 26.9 / 34.9, 6000 / 8000 rows 3584 -> 64 50.6 / 52.0 -> 46.4 / 53.6, 8000 / 10000 / 20000 rows 11008 -> 64
+// 131 / 133 / 166 -> 120 / 148 / 303.
+static bool ob_g3_layer(int64_t T, int64_t K, int64_t N) { return ob_g3_shape(T, K, N) && (N >= 256 || (T <= 8192 && 4 * T <= 7 * K)); }
 // K that is no whole number of quads of K steps: its next whole number, if the product on rows and signs padded to it (ob_pad_rows_kernel) takes the LDS-DMA GEMM;
 // else 0.  Layer calls, the 128 x 128 kernel -> padded: 4064 -> 1000, 70 rows 49.5 -> 17.8 us, 700 51.4 -> 25.0, 1400 54.2 -> 32.2, 3000 57.8 -> 48.6; 1376 -> 4100,
 // 70 rows 30.6 -> 19.2, 700 35.3 -> 26.5, 16000 326 -> 205 (the epilogue and LayerNorm for N % 8 == 4 among it)
@@ -449,7 +452,7 @@ static inline size_t ob_align256(size_t b) { return (b + 255) & ~(size_t)255; }
 // K slices of onebit_linear_forward's product: rows that ob_ln_rows_kernel adds them in
 static int ob_linear_slices(int64_t T, int64_t K, int64_t N)
 {
-    return ob_g3_shape(T, K, N) && N % 8 == 0 && N <= OB_DEC_MAXV * OB_DEC_THREADS * 8 ? ob_g3_plan(&N, 1, K, T, 4).ns : 1;
+    return ob_g3_layer(T, K, N) && N % 8 == 0 && N <= OB_DEC_MAXV * OB_DEC_THREADS * 8 ? ob_g3_plan(&N, 1, K, T, 4).ns : 1;
 }
 
 // K slices of onebit_linear_forward's product of 2 .. 64 rows: 64 columns a workgroup are few workgroups where N is small, each with a long way through K.  Whole phases
@@ -503,7 +506,7 @@ extern "C" size_t onebit_linear_workspace_bytes(int64_t T, int64_t K, int64_t N,
     // large prefill calls run fastest with room for the pre-scaled activations a = fp16(x * h) (LDS-DMA
     // GEMM); a smaller or absent workspace is accepted and selects the register-staged kernel
     // -- and, where K slices are faster, their fp32 sums (without room for them: one slice)
-    if (dtype == ONEBIT_F16 && (ob_g3_shape(T, K, N) || (K % 32 == 0 && ob_gemm3_ok(T, K, N)))) {
+    if (dtype == ONEBIT_F16 && (ob_g3_layer(T, K, N) || (K % 32 == 0 && ob_gemm3_ok(T, K, N)))) {
         const int ns = ob_linear_slices(T, K, N);
         return ns == 1 ? (size_t)T * (size_t)K * 2 : ob_align256((size_t)T * (size_t)K * 2) + ns * ob_align256((size_t)T * (size_t)N * 4);
     }
@@ -609,7 +612,7 @@ extern "C" int onebit_linear_forward(const void *packed, int64_t ldw_bytes, cons
             return ob_launch_status("linear_forward(few rows, k-sliced)");
         } else if (workspace && ob_aligned(workspace, 16) &&
                    (pad ? workspace_bytes >= ob_pad_bytes(T, kp, N)
-                        : (ob_g3_shape(T, K, N) || ob_gemm3_ok(T, K, N)) && workspace_bytes >= (size_t)T * (size_t)K * 2 &&
+                        : (ob_g3_layer(T, K, N) || ob_gemm3_ok(T, K, N)) && workspace_bytes >= (size_t)T * (size_t)K * 2 &&
                           ldw_bytes % 16 == 0 && ob_aligned(packed, 16) && N * ldw_bytes < ((int64_t)1 << 32))) {
             // pre-scale once (the fp16 rounding of bitnet.py:113), then the LDS-DMA GEMM on the scaled rows, whole or in K slices whose sums ONE row pass adds
             // behind it, with fp16(fp16(.) * g) and the LayerNorm

@@ -99,6 +99,9 @@ def test_layers_of_few_columns_ask_for_their_slices():
     for T in (65, 300, 2000):
         for K, N in ((2048, 128), (4096, 8), (4096, 248), (11008, 200)):
             assert lib.onebit_linear_workspace_bytes(T, K, N, 0) >= T * K * 2 + 2 * T * N * 4, (T, K, N)
+    # many rows: the 128 x 128 kernel, which needs none
+    for T, K, N in ((6000, 2048, 128), (8193, 4096, 8), (12000, 4096, 248), (20000, 11008, 200)):
+        assert lib.onebit_linear_workspace_bytes(T, K, N, 0) == 0, (T, K, N)
 
 
 def test_round6_entry_points_reject_bad_arguments_without_gpu():
