@@ -94,6 +94,7 @@ int onebit_unpack_signs(const void *packed, void *out, int dtype, int64_t N, int
  *       slice);
  *     F16, K % 256 != 0 (K % 32 == 0, from 65 rows on): those and the packed rows,
  *       both on the next whole number of 256 columns;
+ *       (N <= 768 and some thousand rows: 0 where a kernel that takes none is faster)
  *     F16, 2 to 64 rows, a long K and few columns: the fp32 sums of K slices (g, u
  *       and bias 16-byte aligned);
  *     F32, T*K*N from 24 million on (36 if K % 256 != 0), N % 4 == 0, g / bias /

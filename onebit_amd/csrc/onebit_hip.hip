@@ -375,18 +375,28 @@ static bool ob_g3_shape(int64_t T, int64_t K, int64_t N)
 {
     return ob_g3_fits(T, K, N) && T > 64 && (N >= 256 ? K >= 1024 : N % 8 == 0 && K >= 2048);
 }
-// A layer call, which scales its rows first.  Fewer than 256 columns: the 128 x 128 kernel goes through K once whatever the rows (to 128 a CU), the scaled rows and the
-// slices' sums grow with them.  128 x 128 kernel -> slices: 65 / 700 / 2000 rows 2048 -> 128 28.6 / 29.6 / 30.8 -> 11.6 / 14.7 / 22.5 us, 11008 -> 200 118 / 122 / 126 ->
-// 23.9 / 30.5 / 42.8; 3000 / 5000 rows 2048 -> 64 31.3 / 32.5 -> 26.9 / 34.9, 6000 / 8000 rows 3584 -> 64 50.6 / 52.0 -> 46.4 / 53.6, 8000 / 10000 / 20000 rows 11008 -> 64
-// 131 / 133 / 166 -> 120 / 148 / 303.
-static bool ob_g3_layer(int64_t T, int64_t K, int64_t N) { return ob_g3_shape(T, K, N) && (N >= 256 || (T <= 8192 && 4 * T <= 7 * K)); }
+// Layer calls of up to 768 columns: whether the 128 x 128 kernel is slower.  It reads rows as they are and goes through K once for up to a tile a CU, half as long again for
+// two; scaled rows and slices' sums grow with the rows.  Estimates of a call's time, LayerNorm included (fitted to 750 and 970 calls, 65 .. 34000 rows, K 1024 ..
+// 13824; 3 and 5 % rms), which choose 0.3 % worse than the better of the two.  128 x 128 kernel -> LDS-DMA: 2000 rows 2048 -> 128 30.8 -> 22.5 us, 11008 -> 200
+// 126 -> 42.8, 6000 / 8000 rows 3584 -> 64 50.6 / 52.0 -> 46.4 / 53.6, 20000 rows 11008 -> 64 166 -> 303; 3000 / 9000 rows 1024 -> 256 22.4 / 28.6 -> 22.9 / 33.5, 1376 -> 320
+// 26.1 / 33.6 -> 26.7 / 38.0, 9000 / 20000 rows 4064 -> 320 61.5 / 93.9 -> 63.3 / 144.
+static bool ob_g3_faster(int64_t T, int64_t K, int64_t N, int64_t kp)
+{
+    if (N > 768 || T <= 2048) return true;                     // (2000 rows 1024 -> 320 21.0 -> 19.6 us, the least of the gains there)
+    const ObG3Plan p = ob_g3_plan(&N, 1, kp, T, N % 8 == 0 ? 4 : 1);
+    const double t = 1e-3 * (double)T, k = 1e-3 * (double)K, n = 1e-3 * (double)N, mb = 2e-3 * t * (double)kp;          // (MB of scaled rows)
+    const double L = (double)(((N + 127) / 128) * ((T + 127) / 128)) / ob_cu_count(), full = floor(0.5 * L), rem = L - 2 * full;
+    const double tiles = 8.7 + k * (16.6 * full + (rem <= 0 ? 0.0 : rem <= 1 ? 10.2 + 1.3 * rem : 16.6)) + t * (0.7 + 0.82 * n);
+    return 10.0 + 0.72 * p.us + 0.31 * mb + 0.2 * std::max(0.0, mb - 100.0) + t * ((p.ns > 1 ? 1.67 : 0.58) + 0.58 * n) <= tiles;
+}
+static bool ob_g3_layer(int64_t T, int64_t K, int64_t N) { return ob_g3_shape(T, K, N) && (ob_gemm3_ok(T, K, N) ? N >= 256 : ob_g3_faster(T, K, N, K)); }
 // K that is no whole number of quads of K steps: its next whole number, if the product on rows and signs padded to it (ob_pad_rows_kernel) takes the LDS-DMA GEMM;
 // else 0.  Layer calls, the 128 x 128 kernel -> padded: 4064 -> 1000, 70 rows 49.5 -> 17.8 us, 700 51.4 -> 25.0, 1400 54.2 -> 32.2, 3000 57.8 -> 48.6; 1376 -> 4100,
 // 70 rows 30.6 -> 19.2, 700 35.3 -> 26.5, 16000 326 -> 205 (the epilogue and LayerNorm for N % 8 == 4 among it)
 static int64_t ob_g3_padded(int64_t T, int64_t K, int64_t N)
 {
     const int64_t kp = (K + 4 * OB_G2_K - 1) / (4 * OB_G2_K) * (4 * OB_G2_K);
-    return K % 32 == 0 && K % (4 * OB_G2_K) != 0 && K >= 1024 && N >= 256 && ob_g3_shape(T, kp, N) ? kp : 0;
+    return K % 32 == 0 && K % (4 * OB_G2_K) != 0 && K >= 1024 && N >= 256 && ob_g3_shape(T, kp, N) && ob_g3_faster(T, K, N, kp) ? kp : 0;
 }
 static int64_t ob_g3_blocks(int64_t N, int wn) { return (N + ob_g3_rows(wn) - 1) / ob_g3_rows(wn); }
 // go(form as a type): the kernel's instance
@@ -449,10 +459,10 @@ static void ob_launch_ln_rows(const ObLnRowsArgs &la, int64_t T, hipStream_t s)
 }
 
 static inline size_t ob_align256(size_t b) { return (b + 255) & ~(size_t)255; }
-// K slices of onebit_linear_forward's product: rows that ob_ln_rows_kernel adds them in
+// K slices of onebit_linear_forward's LDS-DMA product: rows that ob_ln_rows_kernel adds them in
 static int ob_linear_slices(int64_t T, int64_t K, int64_t N)
 {
-    return ob_g3_layer(T, K, N) && N % 8 == 0 && N <= OB_DEC_MAXV * OB_DEC_THREADS * 8 ? ob_g3_plan(&N, 1, K, T, 4).ns : 1;
+    return ob_g3_shape(T, K, N) && (N >= 256 || !ob_gemm3_ok(T, K, N)) && N % 8 == 0 && N <= OB_DEC_MAXV * OB_DEC_THREADS * 8 ? ob_g3_plan(&N, 1, K, T, 4).ns : 1;
 }
 
 // K slices of onebit_linear_forward's product of 2 .. 64 rows: 64 columns a workgroup are few workgroups where N is small, each with a long way through K.  Whole phases

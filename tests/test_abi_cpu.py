@@ -99,9 +99,18 @@ def test_layers_of_few_columns_ask_for_their_slices():
     for T in (65, 300, 2000):
         for K, N in ((2048, 128), (4096, 8), (4096, 248), (11008, 200)):
             assert lib.onebit_linear_workspace_bytes(T, K, N, 0) >= T * K * 2 + 2 * T * N * 4, (T, K, N)
-    # many rows: the 128 x 128 kernel, which needs none
-    for T, K, N in ((6000, 2048, 128), (8193, 4096, 8), (12000, 4096, 248), (20000, 11008, 200)):
-        assert lib.onebit_linear_workspace_bytes(T, K, N, 0) == 0, (T, K, N)
+
+
+def test_layers_of_few_columns_and_many_rows_ask_for_nothing():
+    """Up to some hundred columns the 128 x 128 kernel, which reads the rows as they are, is the faster one from some thousand rows on; K of whole 256 or not."""
+    lib = _lib.load()
+    for K, N, few, many in ((2048, 128, 2000, 8000), (4096, 8, 4000, 12000), (4096, 248, 4000, 12000), (11008, 200, 6000, 20000), (1024, 256, 1500, 9000), (1024, 320, 1500, 9000),
+                            (1376, 320, 1500, 9000), (4064, 320, 4000, 20000), (8224, 512, 4000, 14000)):
+        assert lib.onebit_linear_workspace_bytes(few, K, N, 0) >= few * K * 2, (few, K, N)
+        assert lib.onebit_linear_workspace_bytes(many, K, N, 0) == 0, (many, K, N)
+    # beyond 768 columns, and where whole K leaves both many tiles: the LDS-DMA product
+    for T, K, N in ((9000, 1376, 1000), (12000, 4064, 1000), (12000, 4096, 512), (30000, 1024, 256)):
+        assert lib.onebit_linear_workspace_bytes(T, K, N, 0) >= T * K * 2, (T, K, N)
 
 
 def test_round6_entry_points_reject_bad_arguments_without_gpu():
