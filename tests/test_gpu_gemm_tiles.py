@@ -44,6 +44,12 @@ def test_one_projection_of_few_columns(T, K, N):
     test_one_projection(T, K, N)
 
 
+# up to 768 columns, either side of the rows from which on the 128 x 128 kernel is the faster one; K that is padded, and not
+@pytest.mark.parametrize("T,K,N", [(2049, 1024, 260), (8001, 2048, 136), (3001, 2048, 136), (9000, 1376, 320), (2100, 1376, 320), (20001, 4064, 260), (4001, 4064, 768)])
+def test_many_rows_of_few_columns(T, K, N):
+    test_one_projection(T, K, N)
+
+
 def _group(T, K, Ns):
     """(status, layers, rows, outputs) of one grouped launch; a row more than the outputs have is there to see that it stays."""
     from onebit_amd import _lib
